@@ -11,6 +11,7 @@ import torch  # noqa: F401  (must be loaded before the HIP library, see module d
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libao_amd.so")
+HOST_PATH = os.path.join(_HERE, "lib", "ao_amd_host.so")
 
 F32, BF16, F16, I32, I64, I8, U8 = 0, 1, 2, 3, 4, 5, 6
 MAP_SYMMETRIC, MAP_ASYMMETRIC = 0, 1
@@ -111,6 +112,32 @@ def lib():
             fn.argtypes, fn.restype = argtypes, restype
         _lib = handle
     return _lib
+
+
+class _NoHost:
+    """Stands in for the native host module in a tree that is not built: no call is served, so that the operator's
+    torch.library route reports the missing library."""
+
+    def __getattr__(self, name):
+        return lambda *args: NotImplemented
+
+
+def _load_host():
+    import importlib.machinery
+    import importlib.util
+
+    if not os.path.exists(HOST_PATH):
+        if os.path.exists(LIB_PATH):
+            raise ImportError(f"{HOST_PATH} is missing while {LIB_PATH} is there: run `python -m ao_amd._build`")
+        return _NoHost()
+    loader = importlib.machinery.ExtensionFileLoader("ao_amd_host", HOST_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("ao_amd_host", loader))
+    loader.exec_module(module)
+    return module
+
+
+# Native host path of the eager operators (csrc/host): each function serves the plain case or returns NotImplemented
+host = _load_host()
 
 
 def check(rc: int) -> None:

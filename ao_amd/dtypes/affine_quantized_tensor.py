@@ -173,6 +173,10 @@ class AffineQuantizedTensor(torch.Tensor):
 
     @classmethod
     def __torch_function__(cls, func, types, args=(), kwargs=None):
+        if func is _F_LINEAR and cls is AffineQuantizedTensor and not kwargs:
+            out = _linear_on_host_path(*args)
+            if out is not NotImplemented:
+                return out
         kwargs = {} if kwargs is None else kwargs
         handler = _ATEN_OP_OR_TORCH_FN_TABLE[cls].get(func)
         if handler is not None:
@@ -343,6 +347,32 @@ class Gfx950WaveTiledAQTLayout(AQTLayout):
 
 # the reference's class name, for code that imports it
 TensorCoreTiledAQTLayout = Gfx950WaveTiledAQTLayout
+
+
+_F_LINEAR = torch.nn.functional.linear
+
+
+def _linear_on_host_path(x, weight, bias=None):
+    """F.linear through the native host path under the same conditions as `_quantized_linear_op`, or NotImplemented.
+    Properties of a tensor subclass (shape, dtype, ...) cost a trip through __torch_function__ each: only plain attributes
+    are looked at here, the host path reads dtype and sizes off the tensor itself."""
+    if type(weight) is not AffineQuantizedTensor or type(x) is not torch.Tensor or torch.compiler.is_dynamo_compiling():
+        return NotImplemented
+    layout, block = weight.layout_tensor, weight.block_size
+    if len(block) != 2 or block[0] != 1:
+        return NotImplemented
+    if type(layout) is Gfx950WaveTiledAQTLayout:
+        if layout.transposed or not _is_uint4(weight) or weight.zero_point_domain is not ZeroPointDomain.FLOAT \
+                or ops.int4wo_two_pass(x.numel() // layout.K, layout.N, layout.K):
+            return NotImplemented
+        return ops.host.int4wo_linear(x, layout.packed_weight, layout.scale_and_zero, layout.group_size, layout.N, layout.K,
+                                      bias, weight)
+    if type(layout) is PlainAQTLayout and weight.zero_point_domain is ZeroPointDomain.INT:
+        N, K = layout.int_data.shape
+        if block[1] != K or ops.int8wo_two_pass(x.numel() // K, N, K):
+            return NotImplemented
+        return ops.host.int8wo_linear(x, layout.int_data, layout.scale, bias, weight)
+    return NotImplemented
 
 
 def _quantized_linear_op(input_tensor, weight_qtensor, bias):

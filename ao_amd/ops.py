@@ -14,7 +14,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from ._lib import BF16, DTYPE_CODE, F16, F32, check, current_stream, lib, require_cuda
+from ._lib import BF16, DTYPE_CODE, F16, F32, check, current_stream, host, lib, require_cuda
 
 __all__ = [
     "quant_llm_linear",
@@ -1030,6 +1030,12 @@ def _(ebits, mbits, x, native, scale):
 
 
 # ------------------------------------------------------------------------------------ python wrappers
+#
+# Eager calls with plain GPU tensors go through the native host path (csrc/host), which answers NotImplemented for every
+# other case; dynamo traces the torch.library operator.
+
+_tracing = torch.compiler.is_dynamo_compiling
+
 
 def quant_llm_linear(EXPONENT: int, MANTISSA: int, _in_feats: Tensor, _weights: Tensor, _scales: Tensor,
                      splitK: int = 1) -> Tensor:
@@ -1057,6 +1063,10 @@ def fp6_repack(fpx_data: Tensor, nbits: int = 6) -> Tensor:
 
 def fp6_linear_native(ebits: int, mbits: int, x: Tensor, native: Tensor, scale: Tensor) -> Tensor:
     """x fp16 [M,K] @ W^T with W given in the native tile order -> fp16 [M,N]."""
+    if not _tracing() and x.dim() == 2 and not fp6_two_pass(x.shape[0], scale.shape[0], x.shape[1]):
+        y = host.fp6_linear(ebits, mbits, x, native, scale)
+        if y is not NotImplemented:
+            return y
     return torch.ops.torchao.fp6_linear_native.default(ebits, mbits, x, native, scale)
 
 
@@ -1121,6 +1131,10 @@ def int4wo_swiglu_interleaved(x, packed_pair, qparams_pair, group_size, N, norm_
 
 def int8wo_linear(x: Tensor, w_int8: Tensor, scale: Tensor, bias=None, fp32_out: bool = False) -> Tensor:
     """bf16(bf16(x @ w_int8^T) * scale) (+ bias): x bf16 [M,K], w_int8 int8 [N,K] (plain layout), scale bf16 [N]."""
+    if not _tracing() and not fp32_out and x.dim() == 2 and not int8wo_two_pass(x.shape[0], scale.numel(), x.shape[1]):
+        y = host.int8wo_linear(x, w_int8, scale, bias, None)
+        if y is not NotImplemented:
+            return y
     return torch.ops.torchao.int8wo_linear.default(x, w_int8, scale, bias, fp32_out)
 
 
@@ -1133,6 +1147,10 @@ def hqq_mixed_mm_mfma(a: Tensor, packed_2xint4: Tensor, scales: Tensor, zeros: T
                       transposed: bool = False) -> Tensor:
     """a [M <= 64, K] @ W, or a [M <= 64, N] @ W^T when `transposed`, with W = (q - zero) * scale [K, N] dequantized
     inside the matrix-core kernel."""
+    if not _tracing():
+        y = host.hqq_mixed_mm(a, packed_2xint4, scales, zeros, group_size, transposed)
+        if y is not NotImplemented:
+            return y
     return torch.ops.torchao.hqq_mixed_mm_mfma.default(a, packed_2xint4, scales, zeros, group_size, transposed)
 
 
@@ -1201,4 +1219,8 @@ def int4wo_dequantize(packed: Tensor, qparams: Tensor, N: int, K: int, group_siz
 def int4wo_linear(x: Tensor, packed: Tensor, qparams: Tensor, group_size: int, N: int, bias=None,
                   fp32_out: bool = False) -> Tensor:
     """x [M,K] bf16 @ dequant(W)[N,K]^T (+bias) -> [M,N] bf16 (fp32 when fp32_out)."""
+    if not _tracing() and not fp32_out and x.dim() == 2 and not int4wo_two_pass(x.shape[0], N, x.shape[1]):
+        y = host.int4wo_linear(x, packed, qparams, group_size, N, x.shape[1], bias, None)
+        if y is not NotImplemented:
+            return y
     return torch.ops.torchao.int4wo_linear.default(x, packed, qparams, group_size, N, bias, fp32_out)

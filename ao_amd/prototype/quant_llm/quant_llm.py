@@ -90,6 +90,14 @@ def _fpx_linear(act, weight, bias=None):
     split-K factor comes from a table tuned for NVIDIA SM counts, :212-345, while the gfx950 kernel sizes its own K
     split from the shape)."""
     assert isinstance(weight, QuantLlmLinearWeight)
+    if type(act) is Tensor and not torch.compiler.is_dynamo_compiling():
+        N, K = weight.fpx_data.shape[0], act.shape[-1]
+        if not ops.fp6_two_pass(act.numel() // max(K, 1), N, K):
+            out = ops.host.fp6_linear(weight.ebits, weight.mbits, act, weight.native(), weight.scale)
+            if out is not NotImplemented:
+                if bias is not None:
+                    out += bias
+                return out
     out_features, in_features = weight.shape
     rows = act.reshape(-1, in_features).to(torch.float16)
     out = ops.fp6_linear_native(weight.ebits, weight.mbits, rows, weight.native(), weight.scale)
