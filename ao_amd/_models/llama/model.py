@@ -214,8 +214,11 @@ class Transformer(nn.Module):
         self.causal_mask = torch.tril(torch.ones(max_seq_length, max_seq_length, dtype=torch.bool, device=device))
 
     def _decode_linears(self):
-        return [self.output] + [m for b in self.layers for m in (b.attention.wqkv, b.attention.wo, b.feed_forward.w1,
-                                                                 b.feed_forward.w3, b.feed_forward.w2)]
+        linears = [self._modules["output"]]
+        for b in self.layers:
+            att, ff = b._modules["attention"]._modules, b._modules["feed_forward"]._modules
+            linears += (att["wqkv"], att["wo"], ff["w1"], ff["w3"], ff["w2"])
+        return linears
 
     def fused_decode_kind(self) -> Optional[str]:
         """"int4" / "int8" / "fp6" when a batch-1 single-token step can run on the HIP decode path, else None.  int4:
@@ -235,10 +238,12 @@ class Transformer(nn.Module):
         for lin in self._decode_linears():
             if not isinstance(lin, nn.Linear):  # module-swapped layers (WeightOnlyInt4Linear, ...) run as modules
                 return None
-            w = lin.weight
-            if lin.bias is not None or not isinstance(w, AffineQuantizedTensor) or w.dtype is not torch.bfloat16 \
-                    or not w.is_cuda:
+            w = lin._parameters["weight"]
+            if lin._parameters["bias"] is not None or not isinstance(w, AffineQuantizedTensor):
                 return None
+            with torch._C.DisableTorchFunctionSubclass():  # properties without a trip through __torch_function__ each
+                if w.dtype is not torch.bfloat16 or not w.is_cuda:
+                    return None
             lay = w.layout_tensor
             if isinstance(lay, Gfx950WaveTiledAQTLayout) and not lay.transposed:
                 kinds.add("int4")
@@ -264,6 +269,52 @@ class Transformer(nn.Module):
 
     def fused_decode_ready(self) -> bool:
         return self.fused_decode_kind() is not None
+
+    def _modules_are_watched(self) -> bool:
+        """Whether a hook wants to see the calls of single modules, which the native pass does not make."""
+        hooks = torch.nn.modules.module
+        if hooks._global_forward_hooks or hooks._global_forward_pre_hooks:
+            return True
+        return any(m._forward_hooks or m._forward_pre_hooks for m in self.modules() if m is not self)
+
+    def _host_plan(self, kind: str, rows: int) -> tuple:
+        """The model as csrc/host/llama.cpp reads it: nested tuples of the tensors that a pass of `rows` tokens needs.  Made
+        for every pass, so that replaced weights, caches and norms are seen; plain dictionary lookups keep that at a few us a
+        layer (an attribute of a module or a property of a tensor subclass costs several times that)."""
+        from ... import ops
+
+        cfg = self.config
+        ebits = mbits = group = 0
+
+        def linear(lin):
+            nonlocal ebits, mbits, group
+            w = lin._parameters["weight"]
+            if kind == "int4":
+                lay = w.layout_tensor
+                group, N, K = lay.group_size, lay.N, lay.K
+                return lay.packed_weight, lay.scale_and_zero, N, K, rows > 1 and ops.int4wo_two_pass(rows, N, K)
+            if kind == "int8":
+                lay = w.layout_tensor
+                N, K = lay.int_data.shape
+                return lay.int_data, lay.scale, N, K, rows > 1 and ops.int8wo_two_pass(rows, N, K)
+            ebits, mbits = w.ebits, w.mbits
+            N, K = w.fpx_data.shape[0], w.fpx_data.shape[1] // w.nbits * 8
+            return w.native(), w.scale, N, K, rows > 1 and ops.fp6_two_pass(rows, N, K)
+
+        layers = []
+        for b in self.layers:
+            att, ff = b._modules["attention"], b._modules["feed_forward"]
+            an, fn, kv = b._modules["attention_norm"], b._modules["ffn_norm"], att.kv_cache
+            m, f = att._modules, ff._modules
+            pair, pair_q = self._gate_up_pair(ff)[:2] if kind == "int4" and rows == 1 else (None, None)
+            layers.append((an._parameters["weight"], an.eps, linear(m["wqkv"]), linear(m["wo"]), kv._buffers["k_cache"],
+                           kv._buffers["v_cache"], fn._parameters["weight"], fn.eps, linear(f["w1"]), linear(f["w3"]),
+                           linear(f["w2"]), pair, pair_q))
+        output = linear(self.output)
+        ksplit = self.qkv_ksplit((cfg.n_head + 2 * cfg.n_local_heads) * cfg.head_dim)
+        return (("int4", "int8", "fp6").index(kind), ebits, mbits, group, cfg.n_head, cfg.n_local_heads, ksplit,
+                self.tok_embeddings.weight, self.freqs_cis, tuple(layers), self.norm.weight, self.norm.eps, output,
+                self.max_seq_length)
 
     @staticmethod
     def qkv_ksplit(n_rows: int, n_cu: int = 256) -> int:
@@ -394,7 +445,18 @@ class Transformer(nn.Module):
         return lin(x, self.output, norm=self.norm).view(1, 1, cfg.vocab_size)
 
     def forward(self, idx: Tensor, input_pos: Optional[Tensor] = None) -> Tensor:
+        from ... import ops
+
         assert self.freqs_cis is not None, "Caches must be initialized first"
+        if self.use_fused_decode and input_pos is not None and idx.dim() == 2 and idx.shape[0] == 1 \
+                and not torch.compiler.is_dynamo_compiling():
+            # every launch of the pass from one native call; it declines what it does not take before it launches anything
+            kind = self.fused_decode_kind()
+            if kind is not None and (idx.numel() == 1 or not self._modules_are_watched()):
+                pos = input_pos.to(torch.int32) if idx.numel() == 1 and input_pos.dtype is not torch.int32 else input_pos
+                logits = ops.host.llama_forward(self._host_plan(kind, idx.numel()), idx, pos)
+                if logits is not NotImplemented:
+                    return logits
         if self.use_fused_decode and idx.numel() == 1 and input_pos is not None and input_pos.numel() == 1:
             kind = self.fused_decode_kind()
             if kind == "int4":

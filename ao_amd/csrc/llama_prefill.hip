@@ -1,0 +1,426 @@
+// Prompt-sized work of the Llama harness between the quantized linears (batch 1, head_dim 128):
+//
+//   rope + cache write   torchao/_models/llama/model.py:196-203  (keys rotated and stored at input_pos, values stored)
+//   attention            torchao/_models/llama/model.py:205-210  (query row i over the cache positions 0 .. input_pos[i])
+//   residual + RMSNorm   torchao/_models/llama/model.py:162-165, 232-244
+//   SiLU(gate) * up      torchao/_models/llama/model.py:229
+//
+// Module by module these were some 30 launches a layer over fp32 temporaries and an attention that walked the whole cache
+// under a boolean mask: 4 layers of Llama-3-8B widths at 1000 positions spent 2.1 of 4.8 ms in them.
+#include "llama_elem.h"
+
+namespace ao {
+
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+
+// 32x32x16 product, 8 elements of a 16-bit type per lane and operand
+template <class E> struct Mfma32;
+template <> struct Mfma32<ElemBf16> {
+    typedef __bf16 x8 __attribute__((ext_vector_type(8)));
+    static __device__ __forceinline__ f32x16_t mul(uint4 a, uint4 b, f32x16_t c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(x8, a), __builtin_bit_cast(x8, b), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ uint32_t pack(float lo, float hi) { return hw_bf16_pack(lo, hi); }
+};
+template <> struct Mfma32<ElemF16> {
+    typedef _Float16 x8 __attribute__((ext_vector_type(8)));
+    static __device__ __forceinline__ f32x16_t mul(uint4 a, uint4 b, f32x16_t c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(x8, a), __builtin_bit_cast(x8, b), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ uint32_t pack(float lo, float hi) {
+        return (uint32_t)f32_to_f16_bits(lo) | ((uint32_t)f32_to_f16_bits(hi) << 16);
+    }
+};
+
+__device__ __forceinline__ int64_t position(const void* pos, int pos_is_i64, int64_t i) {
+    return pos_is_i64 ? ((const int64_t*)pos)[i] : (int64_t)((const int32_t*)pos)[i];
+}
+
+// Rotates the consecutive pairs (2i, 2i+1) of 8 elements d .. d+7 of a head: fp32 products rounded one by one, the result
+// rounded to the element type, as the module does.  `cs` holds the four (cos, sin) pairs.
+template <class E>
+__device__ __forceinline__ uint4 rotate8(uint4 x, uint4 cs) {
+    const uint32_t u[4] = {x.x, x.y, x.z, x.w}, f[4] = {cs.x, cs.y, cs.z, cs.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float x0 = E::lo(u[j]), x1 = E::hi(u[j]), c = E::lo(f[j]), s = E::hi(f[j]);
+        o[j] = (uint32_t)E::to_bits(x0 * c - x1 * s) | ((uint32_t)E::to_bits(x1 * c + x0 * s) << 16);
+    }
+    return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// Keys rotated and values as they are, into row input_pos[t] of the caches.  One thread per 8 elements; a row outside the
+// cache is not written.
+template <class E>
+__global__ __launch_bounds__(256) void prefill_cache_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ freqs,
+                                                            const void* __restrict__ pos, int pos_is_i64, int T, int n_head,
+                                                            int n_kv, int64_t S, uint16_t* __restrict__ k_cache,
+                                                            uint16_t* __restrict__ v_cache) {
+    const int per_row = 2 * n_kv * 16;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int t = (int)(i / per_row), c = (int)(i % per_row);
+    if (t >= T) return;
+    const int64_t p = position(pos, pos_is_i64, t);
+    if (p < 0 || p >= S) return;
+    const int head = c >> 4, d = (c & 15) * 8;
+    const uint4 x = *(const uint4*)(qkv + ((int64_t)t * (n_head + 2 * n_kv) + n_head + head) * 128 + d);
+    if (head < n_kv)
+        *(uint4*)(k_cache + ((int64_t)head * S + p) * 128 + d) = rotate8<E>(x, *(const uint4*)(freqs + p * 128 + d));
+    else
+        *(uint4*)(v_cache + ((int64_t)(head - n_kv) * S + p) * 128 + d) = x;
+}
+
+// Causal attention of T query rows over the cache, flash style.
+//
+// A workgroup of 4 waves walks the cache in tiles of 64 positions; a wave owns 32 query rows of one head.  HEADS: the four
+// waves are four query heads of one KV head (grouped-query models: one K / V tile serves four heads); otherwise they are
+// four consecutive 32-row blocks of one head.
+//
+// Both products are 32x32x16 matrix instructions with the query on the column side: S^T = K Q^T leaves a lane with 16 scores
+// of ONE query row per 32 positions, so the softmax statistics are lane-local up to one exchange between the wave's
+// halves, the rescaling of O^T = V^T P^T is one multiply per accumulator, and the 8 probabilities a lane already holds are
+// its operand of the second product: that product may take positions in any order as long as both operands agree, so V^T is
+// stored in LDS in the order the first product leaves them in (lane half h of step s: positions 16 s + 4 h + 0..3 and
+// 16 s + 8 + 4 h + 0..3).  V is turned on its way into LDS: a lane loads 2 columns of 8 positions and writes two 16-byte runs.
+// LDS rows are XOR-swizzled in 16-byte chunks (fragment reads of 16 lanes cover all banks).  Tiles are double-buffered
+// through registers, one barrier per tile.
+//
+// Bound by its LDS fragment reads (32 reads of 1 KB per 32 matrix instructions and wave).  Llama-3-8B widths, 1000
+// positions: see the figures beside prefill_attention below.
+template <class E, bool HEADS>
+__global__ __launch_bounds__(256) void prefill_attention_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ freqs,
+                                                                const void* __restrict__ pos, int pos_is_i64, int T, int n_head,
+                                                                int n_kv, int64_t S, const uint16_t* __restrict__ k_cache,
+                                                                const uint16_t* __restrict__ v_cache, uint16_t* __restrict__ out) {
+    typedef Mfma32<E> MM;
+    __shared__ uint4 ks[2][64 * 16];   // [key][chunk of 8 d], chunk ^ (key & 15)
+    __shared__ uint4 vs[2][64 * 16];   // [d / 2][(d & 1) * 8 + (chunk of 8 keys ^ (d / 2 & 7))]
+    __shared__ int wave_last[4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 31, half = lane >> 5;
+    const int tile = gridDim.y - 1 - blockIdx.y;   // the rows that see most positions start first
+    int head, row0;
+    if (HEADS) {
+        head = blockIdx.x * 4 + wave;
+        row0 = tile * 32;
+    } else {
+        head = blockIdx.x;
+        row0 = tile * 128 + wave * 32;
+    }
+    const int kv = head / (n_head / n_kv);
+    const uint16_t* kc = k_cache + (int64_t)kv * S * 128;
+    const uint16_t* vc = v_cache + (int64_t)kv * S * 128;
+
+    // this lane's query row: position, rotated fragments
+    const int row = row0 + col;
+    const int srow = row < T ? row : T - 1;
+    int last = -1;                                  // last position the row sees; -1: none
+    {
+        const int64_t p = position(pos, pos_is_i64, srow);
+        if (p >= 0 && p < S && row < T) last = (int)p;
+    }
+    uint4 q[8];
+    const int64_t frow = last < 0 ? 0 : last;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const int d = 16 * s + 8 * half;
+        q[s] = rotate8<E>(*(const uint4*)(qkv + ((int64_t)srow * (n_head + 2 * n_kv) + head) * 128 + d),
+                          *(const uint4*)(freqs + frow * 128 + d));
+    }
+    int hi = last, lo = last;
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1) {
+        hi = max(hi, __shfl_xor(hi, o, 64));
+        lo = min(lo, __shfl_xor(lo, o, 64));
+    }
+    hi = __builtin_amdgcn_readfirstlane(hi);
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    if (lane == 0) wave_last[wave] = hi;
+    __syncthreads();
+    const int ntile = (max(max(wave_last[0], wave_last[1]), max(wave_last[2], wave_last[3])) + 64) / 64;
+
+    uint4 kr[4];
+    uint32_t vr[16];
+    const int smax = (int)S - 1;
+    auto fetch = [&](int t) {
+        const int base = t * 64;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int key = min(base + i * 16 + (tid >> 4), smax);
+            kr[i] = *(const uint4*)(kc + (int64_t)key * 128 + (tid & 15) * 8);
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const int c = wave * 2 + g;             // (step, half) of the 8 positions
+            const int kb = base + 16 * (c >> 1) + 4 * (c & 1);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int key = min(kb + (j & 3) + 8 * (j >> 2), smax);
+                vr[g * 8 + j] = *(const uint32_t*)(vc + (int64_t)key * 128 + 2 * lane);
+            }
+        }
+    };
+    auto stash = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int key = i * 16 + (tid >> 4);
+            ks[b][key * 16 + ((tid & 15) ^ (key & 15))] = kr[i];
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+            const int c = wave * 2 + g;
+            uint32_t even[4], odd[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                even[j] = __builtin_amdgcn_perm(vr[g * 8 + 2 * j + 1], vr[g * 8 + 2 * j], 0x05040100u);
+                odd[j] = __builtin_amdgcn_perm(vr[g * 8 + 2 * j + 1], vr[g * 8 + 2 * j], 0x07060302u);
+            }
+            vs[b][lane * 16 + (c ^ (lane & 7))] = make_uint4(even[0], even[1], even[2], even[3]);
+            vs[b][lane * 16 + 8 + (c ^ (lane & 7))] = make_uint4(odd[0], odd[1], odd[2], odd[3]);
+        }
+    };
+
+    f32x16_t o[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[b][r] = 0.f;
+    float m = -INFINITY, sum = 0.f;                 // running maximum and (this lane's share of the) sum, base 2
+    const float scale = 0.08838834764831845f * 1.4426950408889634f;  // 1 / sqrt(128), log2(e)
+
+    if (ntile > 0) {
+        fetch(0);
+        stash(0);
+    }
+    for (int t = 0; t < ntile; ++t) {
+        const int b = t & 1;
+        if (t + 1 < ntile) fetch(t + 1);
+        __syncthreads();                            // tile t is in LDS; everybody is done with the other buffer
+        if (t * 64 <= hi) {
+            f32x16_t s2[2];
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s2[kb][r] = 0.f;
+                const int key = kb * 32 + col;
+#pragma unroll
+                for (int s = 0; s < 8; ++s) s2[kb] = MM::mul(ks[b][key * 16 + ((2 * s + half) ^ (key & 15))], q[s], s2[kb]);
+            }
+            float tmax = -INFINITY;
+            const bool masked = t * 64 + 63 > lo;
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float v = s2[kb][r] * scale;
+                    if (masked && t * 64 + kb * 32 + 8 * (r >> 2) + 4 * half + (r & 3) > last) v = -INFINITY;
+                    s2[kb][r] = v;
+                    tmax = fmaxf(tmax, v);
+                }
+            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+            const float m2 = fmaxf(m, tmax), base = m2 == -INFINITY ? 0.f : m2;
+            const float alpha = __builtin_amdgcn_exp2f(m - base);
+            m = m2;
+            sum *= alpha;
+#pragma unroll
+            for (int bb = 0; bb < 4; ++bb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[bb][r] *= alpha;
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    s2[kb][r] = __builtin_amdgcn_exp2f(s2[kb][r] - base);
+                    sum += s2[kb][r];
+                }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const f32x16_t& p = s2[s >> 1];
+                const int r = 8 * (s & 1);
+                const uint4 pb = make_uint4(MM::pack(p[r], p[r + 1]), MM::pack(p[r + 2], p[r + 3]), MM::pack(p[r + 4], p[r + 5]),
+                                            MM::pack(p[r + 6], p[r + 7]));
+#pragma unroll
+                for (int db = 0; db < 4; ++db) {
+                    const int d = db * 32 + col;
+                    o[db] = MM::mul(vs[b][(d >> 1) * 16 + (d & 1) * 8 + ((2 * s + half) ^ ((d >> 1) & 7))], pb, o[db]);
+                }
+            }
+        }
+        if (t + 1 < ntile) stash(b ^ 1);
+    }
+    sum += __shfl_xor(sum, 32, 64);
+    const float inv = 1.0f / sum;                   // a row that sees nothing (a position outside the cache) becomes NaN
+    if (row < T) {
+        uint16_t* dst = out + ((int64_t)row * n_head + head) * 128;
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4)
+                *(uint2*)(dst + db * 32 + 8 * (r >> 2) + 4 * half) =
+                    make_uint2(MM::pack(o[db][r] * inv, o[db][r + 1] * inv), MM::pack(o[db][r + 2] * inv, o[db][r + 3] * inv));
+    }
+}
+
+// h = x + y, n = rmsnorm(h) * w: one workgroup per row, the row in registers (dim a multiple of 8, at most 8192).
+template <class E>
+__global__ __launch_bounds__(256) void add_rmsnorm_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ y,
+                                                          const uint16_t* __restrict__ w, int dim, float eps,
+                                                          uint16_t* __restrict__ h, uint16_t* __restrict__ n) {
+    constexpr int MAXC = 4;
+    __shared__ float part[4];
+    const int64_t row = blockIdx.x;
+    const int nchunk = dim / 8;
+    uint32_t v[MAXC][4];
+    uint4 g[MAXC];
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) {
+        const int i = threadIdx.x + c * 256;
+        if (i < nchunk) {
+            const uint4 a4 = ((const uint4*)(x + row * dim))[i], b4 = ((const uint4*)(y + row * dim))[i];
+            g[c] = ((const uint4*)w)[i];
+            const uint32_t a[4] = {a4.x, a4.y, a4.z, a4.w}, b[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[c][j] = (uint32_t)E::to_bits(E::lo(a[j]) + E::lo(b[j])) | ((uint32_t)E::to_bits(E::hi(a[j]) + E::hi(b[j])) << 16);
+                const float lo = E::lo(v[c][j]), hi = E::hi(v[c][j]);
+                ss += lo * lo + hi * hi;
+            }
+        }
+    }
+    ss = wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    const float r = rsqrtf((part[0] + part[1] + part[2] + part[3]) / (float)dim + eps);
+#pragma unroll
+    for (int c = 0; c < MAXC; ++c) {
+        const int i = threadIdx.x + c * 256;
+        if (i < nchunk) {
+            const uint32_t gg[4] = {g[c].x, g[c].y, g[c].z, g[c].w};
+            uint32_t o[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                o[j] = (uint32_t)E::to_bits(E::rne(E::lo(v[c][j]) * r) * E::lo(gg[j])) |
+                       ((uint32_t)E::to_bits(E::rne(E::hi(v[c][j]) * r) * E::hi(gg[j])) << 16);
+            ((uint4*)(h + row * dim))[i] = make_uint4(v[c][0], v[c][1], v[c][2], v[c][3]);
+            ((uint4*)(n + row * dim))[i] = make_uint4(o[0], o[1], o[2], o[3]);
+        }
+    }
+}
+
+// out = silu(gate) * up, 8 elements per thread; silu is rounded to the element type before the product, as F.silu leaves it
+template <class E>
+__global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* gate, const uint16_t* __restrict__ up, int64_t n8,
+                                                       uint16_t* out) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    const uint4 a4 = ((const uint4*)gate)[i], b4 = ((const uint4*)up)[i];
+    const uint32_t a[4] = {a4.x, a4.y, a4.z, a4.w}, b[4] = {b4.x, b4.y, b4.z, b4.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float x0 = E::lo(a[j]), x1 = E::hi(a[j]);
+        const float s0 = E::rne(x0 / (1.0f + expf(-x0))), s1 = E::rne(x1 / (1.0f + expf(-x1)));
+        o[j] = (uint32_t)E::to_bits(s0 * E::lo(b[j])) | ((uint32_t)E::to_bits(s1 * E::hi(b[j])) << 16);
+    }
+    ((uint4*)out)[i] = make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// Rows of the embedding table.  A token outside the table leaves a row of NaN (both 16-bit types: all bits set).
+__global__ __launch_bounds__(256) void embed_kernel(const void* __restrict__ tokens, int is_i64, const uint4* __restrict__ table,
+                                                    int64_t vocab, int row16, uint4* __restrict__ out) {
+    const int64_t t = blockIdx.x, tok = position(tokens, is_i64, t);
+    const bool ok = tok >= 0 && tok < vocab;
+    for (int i = blockIdx.y * 256 + threadIdx.x; i < row16; i += gridDim.y * 256)
+        out[t * row16 + i] = ok ? table[tok * row16 + i] : make_uint4(~0u, ~0u, ~0u, ~0u);
+}
+
+static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// Llama-3-8B widths (32 query heads over 8 KV heads), 1000 positions of a 1128-position cache.
+template <class E>
+static void prefill_attention(const uint16_t* qkv, const uint16_t* freqs, const void* pos, int pos_is_i64, int T, int n_head, int n_kv,
+                              int64_t S, uint16_t* kc, uint16_t* vc, uint16_t* out, hipStream_t st) {
+    const int64_t chunks = (int64_t)T * 2 * n_kv * 16;
+    hipLaunchKernelGGL(prefill_cache_kernel<E>, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, qkv, freqs, pos, pos_is_i64, T,
+                       n_head, n_kv, S, kc, vc);
+    if (n_head / n_kv % 4 == 0)
+        hipLaunchKernelGGL((prefill_attention_kernel<E, true>), dim3(n_head / 4, (T + 31) / 32), dim3(256), 0, st, qkv, freqs, pos,
+                           pos_is_i64, T, n_head, n_kv, S, kc, vc, out);
+    else
+        hipLaunchKernelGGL((prefill_attention_kernel<E, false>), dim3(n_head, (T + 127) / 128), dim3(256), 0, st, qkv, freqs, pos,
+                           pos_is_i64, T, n_head, n_kv, S, kc, vc, out);
+}
+
+}  // namespace ao
+
+using namespace ao;
+
+extern "C" int ao_amd_llama_prefill_attention(const void* qkv, int is_f16, const void* freqs_cis, const void* positions, int pos_is_i64,
+                                              int64_t T, void* k_cache, void* v_cache, int n_head, int n_kv, int head_dim,
+                                              int64_t max_seq, void* out, void* stream) {
+    AO_REQUIRE(qkv && freqs_cis && positions && k_cache && v_cache && out, "null pointer argument");
+    AO_REQUIRE(head_dim == 128, "prefill attention is built for head_dim 128, got %d", head_dim);
+    AO_REQUIRE(n_kv > 0 && n_head > 0 && n_head % n_kv == 0, "n_head=%d must be a multiple of n_kv=%d", n_head, n_kv);
+    AO_REQUIRE(n_head <= 65535 && T >= 0 && T <= 1 << 20 && max_seq > 0 && max_seq <= 1 << 20, "T=%lld, max_seq=%lld out of range",
+               (long long)T, (long long)max_seq);
+    AO_REQUIRE(aligned16(qkv) && aligned16(freqs_cis) && aligned16(k_cache) && aligned16(v_cache) && aligned16(out),
+               "16-byte aligned tensors needed");
+    if (T == 0) return 0;
+    if (is_f16)
+        prefill_attention<ElemF16>((const uint16_t*)qkv, (const uint16_t*)freqs_cis, positions, pos_is_i64, (int)T, n_head, n_kv, max_seq,
+                                   (uint16_t*)k_cache, (uint16_t*)v_cache, (uint16_t*)out, (hipStream_t)stream);
+    else
+        prefill_attention<ElemBf16>((const uint16_t*)qkv, (const uint16_t*)freqs_cis, positions, pos_is_i64, (int)T, n_head, n_kv, max_seq,
+                                    (uint16_t*)k_cache, (uint16_t*)v_cache, (uint16_t*)out, (hipStream_t)stream);
+    AO_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int ao_amd_add_rmsnorm(const void* x, const void* y, const void* weight, int is_f16, int64_t rows, int64_t dim, float eps,
+                                  void* sum, void* normed, void* stream) {
+    AO_REQUIRE(x && y && weight && sum && normed, "null pointer argument");
+    AO_REQUIRE(rows >= 0 && rows <= INT32_MAX && dim > 0 && dim <= 8192 && dim % 8 == 0, "rows=%lld, dim=%lld: dim must be a multiple of 8, at most 8192",
+               (long long)rows, (long long)dim);
+    AO_REQUIRE(aligned16(x) && aligned16(y) && aligned16(weight) && aligned16(sum) && aligned16(normed), "16-byte aligned tensors needed");
+    if (rows == 0) return 0;
+    if (is_f16)
+        hipLaunchKernelGGL(add_rmsnorm_kernel<ElemF16>, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)x,
+                           (const uint16_t*)y, (const uint16_t*)weight, (int)dim, eps, (uint16_t*)sum, (uint16_t*)normed);
+    else
+        hipLaunchKernelGGL(add_rmsnorm_kernel<ElemBf16>, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)x,
+                           (const uint16_t*)y, (const uint16_t*)weight, (int)dim, eps, (uint16_t*)sum, (uint16_t*)normed);
+    AO_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int ao_amd_silu_mul(const void* gate, const void* up, int is_f16, int64_t n, void* out, void* stream) {
+    AO_REQUIRE(gate && up && out, "null pointer argument");
+    AO_REQUIRE(n >= 0 && n % 8 == 0 && n / 8 / 256 < INT32_MAX, "n=%lld must be a multiple of 8", (long long)n);
+    AO_REQUIRE(aligned16(gate) && aligned16(up) && aligned16(out), "16-byte aligned tensors needed");
+    if (n == 0) return 0;
+    const dim3 grid((unsigned)((n / 8 + 255) / 256));
+    if (is_f16)
+        hipLaunchKernelGGL(silu_mul_kernel<ElemF16>, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)gate, (const uint16_t*)up,
+                           n / 8, (uint16_t*)out);
+    else
+        hipLaunchKernelGGL(silu_mul_kernel<ElemBf16>, grid, dim3(256), 0, (hipStream_t)stream, (const uint16_t*)gate, (const uint16_t*)up,
+                           n / 8, (uint16_t*)out);
+    AO_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int ao_amd_llama_embed(const void* tokens, int is_i64, int64_t T, const void* table, int64_t vocab, int64_t dim, void* out,
+                                  void* stream) {
+    AO_REQUIRE(tokens && table && out, "null pointer argument");
+    AO_REQUIRE(T >= 0 && T <= INT32_MAX && vocab > 0 && dim > 0 && dim % 8 == 0, "T=%lld, dim=%lld: dim must be a multiple of 8",
+               (long long)T, (long long)dim);
+    AO_REQUIRE(aligned16(table) && aligned16(out), "16-byte aligned tensors needed");
+    if (T == 0) return 0;
+    // one row: spread over a few workgroups, many rows: one each
+    const dim3 grid((unsigned)T, T >= 64 ? 1u : (unsigned)((dim / 8 + 255) / 256));
+    hipLaunchKernelGGL(embed_kernel, grid, dim3(256), 0, (hipStream_t)stream, tokens, is_i64, (const uint4*)table, vocab, (int)(dim / 8),
+                       (uint4*)out);
+    AO_LAUNCH_CHECK();
+    return 0;
+}
