@@ -77,6 +77,9 @@ _SIGNATURES = {
     "ao_amd_int4wo_interleave_pair": ([_p, _p, _p, _p, _i64, _i64, _i64, _p, _p, _p], _int),
     "ao_amd_int4wo_swiglu_interleaved": ([_p, _i64, _i64, _i64, _p, ctypes.c_float, _p, _p, _i64, _i64, _p, _i64, _p], _int),
     "ao_amd_int8wo_linear": ([_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _int, _i64, _p], _int),
+    "ao_amd_int8wo_linear_plan": ([_i64, _i64, _i64, ctypes.c_char_p, _i64], _int),
+    "ao_amd_int8wo_linear_ws_bytes": ([_i64, _i64, _i64, _i64p], _int),
+    "ao_amd_int8wo_linear_ws": ([_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _int, _i64, _p, _i64, _p], _int),
     "ao_amd_int8wo_linear_residual": ([_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p], _int),
     "ao_amd_int8wo_linear_gated": ([_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p], _int),
     "ao_amd_int8wo_rmsnorm_linear": ([_p, _i64, _i64, _i64, _p, ctypes.c_float, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p], _int),

@@ -44,20 +44,23 @@ PyObject* int4wo_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     });
 }
 
-// (x, w_int8, scale, bias, weight or None): bf16(bf16(x @ w^T) * scale) (+ bias) on the streaming kernels
+// (x, w_int8, scale, bias, weight or None): bf16(bf16(x @ w^T) * scale) (+ bias)
 PyObject* int8wo_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     AO_NEED(5);
     const Tensor &x = a.tensor(0, at::kBFloat16), &w = a.tensor(1, at::kChar), &scale = a.tensor(2, at::kBFloat16);
     const Tensor& bias = a.tensor(3, at::kBFloat16, true);
     AO_WANT(a.ok && current(a.device));
     const Rows r(x);
-    AO_WANT(r.ok && w.dim() == 2 && w.size(1) == r.K && w.stride(1) == 1 && w.stride(0) % 16 == 0 && r.K % 128 == 0);
+    AO_WANT(r.ok && w.dim() == 2 && w.size(1) == r.K && w.stride(1) == 1 && w.stride(0) % 16 == 0 && r.K % 64 == 0);
     const int64_t N = w.size(0);
     AO_WANT(stands_for_bf16_matrix(v[4], N, r.K) && scale.numel() == N && scale.is_contiguous() && bias_ok(bias, N));
     return guarded([&]() -> PyObject* {
-        Tensor y = empty_rows(x, N, at::kBFloat16);
-        AO_CALL(ao_amd_int8wo_linear(ptr(x), r.M, r.K, r.ld, ptr(w), w.stride(0), ptr(scale), N, ptr(bias), y.data_ptr(), AO_BF16, N,
-                                     stream_of(a.device)));
+        Tensor y = empty_rows(x, N, at::kBFloat16), ws;
+        int64_t need = 0;
+        AO_CALL(ao_amd_int8wo_linear_ws_bytes(r.M, r.K, N, &need));
+        if (need) ws = workspace(need, a.device);
+        AO_CALL(ao_amd_int8wo_linear_ws(ptr(x), r.M, r.K, r.ld, ptr(w), w.stride(0), ptr(scale), N, ptr(bias), y.data_ptr(), AO_BF16, N,
+                                        need ? ws.data_ptr() : nullptr, need, stream_of(a.device)));
         return THPVariable_Wrap(std::move(y));
     });
 }

@@ -174,10 +174,10 @@ struct Pass {
             return true;
         }
         y = alloc(M, l.N);
-        if (m.kind == INT8)
-            return ao_amd_int8wo_linear(ptr(x), M, l.K, l.K, ptr(l.codes), l.K, ptr(l.scales), l.N, nullptr, y.data_ptr(), AO_BF16, l.N, st) == 0;
         int64_t need = 0;
-        if (M >= 16 && M <= 256) {
+        if (m.kind == INT8) {
+            AO_TRY(ao_amd_int8wo_linear_ws_bytes(M, l.K, l.N, &need));
+        } else if (M >= 16 && M <= 256) {
             if (m.kind == INT4)
                 AO_TRY(ao_amd_int4wo_linear_ws_bytes(M, l.K, l.N, m.group, &need));
             else
@@ -185,6 +185,9 @@ struct Pass {
         }
         Tensor ws;
         if (need) ws = workspace(need, device);
+        if (m.kind == INT8)
+            return ao_amd_int8wo_linear_ws(ptr(x), M, l.K, l.K, ptr(l.codes), l.K, ptr(l.scales), l.N, nullptr, y.data_ptr(), AO_BF16, l.N,
+                                           need ? ws.data_ptr() : nullptr, need, st) == 0;
         if (m.kind == INT4)
             return ao_amd_int4wo_linear_ws(ptr(x), M, l.K, l.K, ptr(l.codes), ptr(l.scales), l.N, m.group, nullptr, y.data_ptr(), AO_BF16,
                                            l.N, need ? ws.data_ptr() : nullptr, need, st) == 0;

@@ -1,0 +1,122 @@
+// int8 weight-only linear for batches beyond the streaming kernels (int8wo_linear.hip): y = bf16(bf16(x @ W^T) * scale) (+ bias),
+// torchao/dtypes/affine_quantized_tensor.py:641-665, on the tiled product of tile_gemm.h.  The plain [N, K] int8 rows are
+// copied into LDS as they are and converted by the multiplying wave (an int8 is exact in bf16: two byte conversions and a
+// pack per pair), where the earlier route wrote the whole weight as bf16, called the library GEMM and scaled the
+// result in a third pass.  11008 x 4096 at 333 rows: 22 + 43 + 6 us -> 44.
+#include "int8wo_gemm.h"
+#include "int4wo_linear.h"
+
+namespace ao {
+
+typedef __bf16 i8_bf16x8 __attribute__((ext_vector_type(8)));
+
+struct Int8Tile {
+    static constexpr int STEP_BYTES = 64;   // of one weight row per 64-wide K step
+    struct Row {};
+    struct Raw { uint4 v[2]; };             // 32 consecutive k of one row
+    struct Cols { float scale[4], bias[4]; bool has_bias; };
+
+    // request j of a tile: 16 rows x 64 bytes; slot (row, p) holds 16-byte chunk p ^ (row / 4 % 4): conflict-free reads
+    static __device__ __forceinline__ uint32_t request_offset(const TileGemmArgs& a, int64_t n0, int j, int lane) {
+        const int row = j * 16 + (lane >> 2);
+        const int64_t rel = (n0 + row < a.N ? n0 + row : a.N - 1) - n0;   // rows past N repeat the last one
+        return (uint32_t)(rel * a.ldw) + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
+    }
+    static __device__ __forceinline__ const uint8_t* tile_base(const TileGemmArgs& a, int64_t n0) { return a.w + n0 * a.ldw; }
+    static __device__ __forceinline__ const uint8_t* step_base(const TileGemmArgs&, const uint8_t* base, int s) { return base + (int64_t)s * 64; }
+    static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) { return Row(); }
+    static __device__ __forceinline__ Raw read(const uint8_t* B, int n, int half) {
+        Raw r;
+        r.v[0] = *(const uint4*)(B + n * 64 + (((2 * half) ^ ((n >> 2) & 3)) << 4));
+        r.v[1] = *(const uint4*)(B + n * 64 + (((2 * half + 1) ^ ((n >> 2) & 3)) << 4));
+        return r;
+    }
+    // dword d (k = 8 s + 2 d, + 1) of slice s
+    static __device__ __forceinline__ uint32_t piece(const Raw& r, int s, int d, const Row&) {
+        const uint4 v = r.v[s >> 1];
+        const uint32_t w = s & 1 ? (d < 2 ? v.z : v.w) : (d < 2 ? v.x : v.y);
+        float f0, f1;
+        if (d & 1)
+            asm("v_cvt_f32_i32_sdwa %0, sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2\n\t"
+                "v_cvt_f32_i32_sdwa %1, sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3" : "=&v"(f0), "=&v"(f1) : "v"(w));
+        else
+            asm("v_cvt_f32_i32_sdwa %0, sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0\n\t"
+                "v_cvt_f32_i32_sdwa %1, sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=&v"(f0), "=&v"(f1) : "v"(w));
+        return hw_bf16_pack(f0, f1);
+    }
+    static __device__ __forceinline__ tg_f32x16 mul(uint4 w, uint4 x, tg_f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(i8_bf16x8, w), __builtin_bit_cast(i8_bf16x8, x), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ Cols columns(const TileGemmArgs& a, int64_t n) {
+        Cols c;
+        c.has_bias = a.bias != nullptr;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int64_t i = n + v < a.N ? n + v : a.N - 1;
+            c.scale[v] = bf16_bits_to_f32(a.scale[i]);
+            c.bias[v] = a.bias ? bf16_bits_to_f32(a.bias[i]) : 0.f;
+        }
+        return c;
+    }
+    static __device__ __forceinline__ uint16_t finish(float acc, const Cols& c, int v) {
+        const float y = rne_bf16(acc) * c.scale[v];
+        return f32_to_bf16_bits(c.has_bias ? rne_bf16(y) + c.bias[v] : y);
+    }
+    // the residual and gated epilogues of the streaming kernels, on the rounded result
+    static __device__ __forceinline__ void combine(const TileGemmArgs& a, int64_t m, int64_t n, uint16_t (&o)[4]) {
+        if (!a.residual && !a.gate) return;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            if (n + v >= a.N) break;
+            const float y = bf16_bits_to_f32(o[v]);
+            o[v] = f32_to_bf16_bits(a.residual ? y + bf16_bits_to_f32(a.residual[m * a.ldres + n + v])
+                                               : silu_bf16(bf16_bits_to_f32(a.gate[m * a.ldgate + n + v])) * y);
+        }
+    }
+};
+
+// us at K = 4096 with one and two workgroups on a CU (14336 and 11008 columns at 64 - 512 rows)
+static const TileShape kInt8Shapes[] = {
+    {64, 128, 25.5, 0.0},    // two groups of 4 waves along K
+    {96, 128, 32.0, 47.5},
+    {128, 128, 38.0, 0.0},
+    {192, 128, 46.0, 0.0},
+    {128, 256, 54.0, 0.0},   // 128 x 64 a wave
+};
+
+TilePlan int8wo_gemm_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
+    return tile_plan(kInt8Shapes, (int)(sizeof(kInt8Shapes) / sizeof(kInt8Shapes[0])), M, N, K, max_parts);
+}
+
+void int8wo_gemm_describe(const TilePlan& p, char* out, size_t cap) {
+    snprintf(out, cap, "tile %dx%d parts=%d", kInt8Shapes[p.shape].bm, kInt8Shapes[p.shape].bn, p.parts);
+}
+
+template <int WN, int KW, int MT, int NT>
+static void launch(const TileGemmArgs& a, int parts, hipStream_t st) {
+    hipEvent_t ev0 = g_prof_start, ev1 = g_prof_stop;
+    g_prof_start = g_prof_stop = nullptr;
+    hipExtLaunchKernelGGL((tile_gemm_kernel<Int8Tile, WN, KW, MT, NT>), dim3((unsigned)(a.per_xcd * 8), (unsigned)parts), dim3(64 * WN * KW), 0,
+                          st, ev0, ev1, 0, a);
+}
+
+void launch_int8wo_gemm(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
+    const TileShape& s = kInt8Shapes[p.shape];
+    a.tiles_n = (int)((a.N + s.bn - 1) / s.bn);
+    a.tiles = a.tiles_n * (int)((a.M + s.bm - 1) / s.bm);
+    a.per_xcd = (a.tiles + 7) / 8;
+    if (p.parts == 1) a.parts = nullptr;
+    switch (p.shape) {
+        case 0: launch<4, 2, 2, 1>(a, p.parts, st); break;
+        case 1: launch<4, 1, 3, 1>(a, p.parts, st); break;
+        case 2: launch<4, 1, 4, 1>(a, p.parts, st); break;
+        case 3: launch<4, 1, 6, 1>(a, p.parts, st); break;
+        default: launch<4, 1, 4, 2>(a, p.parts, st); break;
+    }
+    if (p.parts > 1) {
+        const int64_t n = a.M * ((a.N + 3) / 4);
+        hipLaunchKernelGGL(tile_finish_kernel<Int8Tile>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, p.parts);
+    }
+}
+
+}  // namespace ao

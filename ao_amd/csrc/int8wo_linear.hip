@@ -9,7 +9,7 @@
 // byte select) and a pack to bf16: 12 VALU instructions per 8 weights, an eighth of the int4 path's cost per byte.
 // The scale is applied once per output element in the epilogue, after the bf16 rounding of the matmul result,
 // as the reference's module chain does.
-#include "common.h"
+#include "int8wo_gemm.h"
 
 namespace ao {
 
@@ -561,17 +561,87 @@ static int int8wo_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
     return 0;
 }
 
+// Where the tiled product serves instead of the streaming kernels above, which read the weight once per 16 or 32 rows.
+static bool tiled(int64_t M, int64_t N, int64_t K) {
+    static const int forced = [] { const char* e = knob("AO_AMD_INT8_TILED"); return e ? atoi(e) : -1; }();
+    if (forced >= 0) return forced != 0 && M > 0;
+    // The streaming kernels hold on where the weight is small enough to be read again per 32 rows, and where a launch of
+    // tiles would not fill the chip.  Measured, us streaming / tiled: 4096 x 14336 at 17 rows 38 / 22, 14336 x 4096 at 24 / 40
+    // rows 22 / 22, 39 / 23; 4096 x 4096 at 32 / 40 rows 14.7 / 15.0, 18.9 / 15.9; 1024 x 4096 at 128 / 192 rows 13.8 / 14.0,
+    // 19.1 / 15.5; 640 x 1024 at 512 / 1024 rows 8.4 / 10.7, 15.2 / 10.9.
+    // In_features that are a multiple of 64 but not of 128 run on tiles whatever the rows: the streaming kernels walk 128-wide
+    // tiles of K.
+    const int64_t weight = N * K;
+    return K % 128 != 0 || M > (weight >= (32 << 20) ? 16 : weight >= (12 << 20) ? 32 : weight >= (3 << 20) ? 128 : 768);
+}
+
+static int int8wo_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* w_int8, int64_t ldw, const void* scale_bf16,
+                        int64_t N, const void* bias_bf16, void* y, int64_t ldy, const void* residual, int64_t ldres, const void* gate,
+                        int64_t ldgate, float* workspace, int64_t workspace_bytes, void* stream) {
+    AO_REQUIRE((!residual || ldres >= N) && (!gate || ldgate >= N), "epilogue operand rows shorter than N=%lld", (long long)N);
+    AO_REQUIRE(x_bf16 && w_int8 && scale_bf16 && y, "null pointer argument");
+    AO_REQUIRE(M >= 0 && N > 0 && K > 0 && K % 64 == 0, "int8 weight-only linear needs in_features to be a multiple of 64, got %lld", (long long)K);
+    if (M == 0) return 0;
+    AO_REQUIRE(ldx >= K && ldw >= K && ldy >= N, "row strides (ldx=%lld, ldw=%lld, ldy=%lld) smaller than the rows",
+               (long long)ldx, (long long)ldw, (long long)ldy);
+    AO_REQUIRE((((uintptr_t)x_bf16) & 15) == 0 && (ldx & 7) == 0 && (((uintptr_t)w_int8) & 15) == 0 && (ldw & 15) == 0,
+               "activation and weight rows must be 16-byte aligned");
+    // per-lane offsets within a tile are 32 bits wide
+    AO_REQUIRE(192 * ldx * 2 < ((int64_t)1 << 32) && 256 * ldw < ((int64_t)1 << 32) && M * N < ((int64_t)1 << 40), "operands too large");
+    TilePlan p = int8wo_gemm_plan(M, N, K, 8);
+    if (p.parts > 1 && (!workspace || workspace_bytes < p.parts * M * N * (int64_t)sizeof(float))) p = int8wo_gemm_plan(M, N, K, 1);
+    launch_int8wo_gemm(TileGemmArgs{(const uint16_t*)x_bf16, M, K, ldx, (const uint8_t*)w_int8, ldw, (const uint16_t*)scale_bf16,
+                                    (const uint16_t*)bias_bf16, N, (uint16_t*)y, ldy, 0, 0, 0, (const uint16_t*)residual, ldres,
+                                    (const uint16_t*)gate, ldgate, workspace},
+                       p, (hipStream_t)stream);
+    AO_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int ao_amd_int8wo_linear_ws_bytes(int64_t M, int64_t K, int64_t N, int64_t* bytes) {
+    AO_REQUIRE(bytes, "null pointer argument");
+    AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
+    *bytes = 0;
+    if (M > 0 && K % 64 == 0 && tiled(M, N, K)) {
+        const TilePlan p = int8wo_gemm_plan(M, N, K, 8);
+        if (p.parts > 1) *bytes = p.parts * M * N * (int64_t)sizeof(float);
+    }
+    return 0;
+}
+
+extern "C" int ao_amd_int8wo_linear_plan(int64_t M, int64_t K, int64_t N, char* out, int64_t out_cap) {
+    AO_REQUIRE(out && out_cap > 0 && M > 0 && N > 0 && K > 0 && K % 64 == 0, "need positive M and N, K a multiple of 64, and a buffer");
+    if (!tiled(M, N, K)) {
+        snprintf(out, (size_t)out_cap, "streaming");
+        return 0;
+    }
+    int8wo_gemm_describe(int8wo_gemm_plan(M, N, K, 8), out, (size_t)out_cap);
+    return 0;
+}
+
+extern "C" int ao_amd_int8wo_linear_ws(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* w_int8, int64_t ldw,
+                                       const void* scale_bf16, int64_t N, const void* bias_bf16, void* y, int y_dtype, int64_t ldy,
+                                       void* workspace, int64_t workspace_bytes, void* stream) {
+    AO_REQUIRE(!workspace || (((uintptr_t)workspace) & 15) == 0, "the workspace must be 16-byte aligned");
+    if (y_dtype == AO_BF16 && K % 64 == 0 && tiled(M, N, K))
+        return int8wo_tiled(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, ldy, nullptr, 0, nullptr, 0, (float*)workspace, workspace_bytes, stream);
+    return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, y_dtype, ldy, nullptr, 0, nullptr, 0, stream);
+}
+
 extern "C" int ao_amd_int8wo_linear(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* w_int8, int64_t ldw,
                                     const void* scale_bf16, int64_t N, const void* bias_bf16, void* y, int y_dtype,
                                     int64_t ldy, void* stream) {
-    return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, y_dtype, ldy, nullptr, 0, nullptr, 0,
-                           stream);
+    AO_REQUIRE(K % 128 == 0, "int8 weight-only linear needs in_features to be a multiple of 128, got %lld", (long long)K);
+    return ao_amd_int8wo_linear_ws(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, y_dtype, ldy, nullptr, 0, stream);
 }
 
 extern "C" int ao_amd_int8wo_linear_residual(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* w_int8,
                                              int64_t ldw, const void* scale_bf16, int64_t N, const void* residual_bf16,
                                              int64_t ldres, void* y_bf16, int64_t ldy, void* stream) {
     AO_REQUIRE(residual_bf16, "null pointer argument");
+    if (K % 128 == 0 && tiled(M, N, K))
+        return int8wo_tiled(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, ldy, residual_bf16, ldres, nullptr, 0, nullptr, 0,
+                            stream);
     return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, AO_BF16, ldy, residual_bf16, ldres,
                            nullptr, 0, stream);
 }
@@ -580,6 +650,9 @@ extern "C" int ao_amd_int8wo_linear_gated(const void* x_bf16, int64_t M, int64_t
                                           int64_t ldw, const void* scale_bf16, int64_t N, const void* gate_bf16,
                                           int64_t ldgate, void* y_bf16, int64_t ldy, void* stream) {
     AO_REQUIRE(gate_bf16, "null pointer argument");
+    if (K % 128 == 0 && tiled(M, N, K))
+        return int8wo_tiled(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, ldy, nullptr, 0, gate_bf16, ldgate, nullptr, 0,
+                            stream);
     return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, AO_BF16, ldy, nullptr, 0, gate_bf16,
                            ldgate, stream);
 }

@@ -1,0 +1,287 @@
+// Tiled product y[M,N] = x[M,K] @ dequant(W[N,K])^T for batches beyond the streaming kernels, generic over the weight format.
+//
+// A workgroup of WN x KW waves computes a tile of 32 MT activation rows x 32 NT WN weight rows; a wave owns MT x NT blocks of
+// 32x32x16 matrix instructions over all rows of the tile, so every weight is dequantized once per tile, and with KW > 1 the
+// groups of WN waves take the 64-wide K steps round-robin and add their accumulators through LDS at the end.  Both
+// operands of a step come into LDS by direct loads (no registers, no LDS store instructions) through a ring of STAGES
+// buffers with one barrier per step.  Weights are stored in LDS as they are in memory and dequantized by the wave that
+// multiplies them, in registers, on the way into the matrix instruction.
+//
+// The weight is the row operand of the matrix instruction: a lane of the result holds 4 consecutive outputs of one
+// activation row (8-byte stores), and the order of the 64 reduction indices within a step is free as long as both
+// operands agree, so a lane half takes 32 consecutive k of its rows: a format's natural contiguous run.
+//
+// What bounds it (ablations on 14336 x 4096 int8, 64 - 256 rows): with one wave per SIMD nothing overlaps inside the wave, so
+// LDS reads, conversion and requests add to the matrix time; and a step's data takes 0.7 us from the last-level cache, so
+// the bytes in flight per CU set the pace of small tiles.  Requests three steps ahead instead of two took 128 x 128 tiles
+// at 256 rows from 51 to 38 us; two groups along K (two waves per SIMD) took 64 x 128 tiles from 29 to 24 us.
+#pragma once
+#include "common.h"
+
+namespace ao {
+
+typedef float tg_f32x16 __attribute__((ext_vector_type(16)));
+
+struct TileGemmArgs {
+    const uint16_t* x; int64_t M, K, ldx;
+    const uint8_t* w; int64_t ldw;      // weight and its row (or row-block) stride in bytes
+    const uint16_t* scale;
+    const uint16_t* bias;               // or null
+    int64_t N;
+    uint16_t* y; int64_t ldy;
+    int tiles_n, tiles, per_xcd;
+    const uint16_t* residual; int64_t ldres;   // y += residual, or null
+    const uint16_t* gate; int64_t ldgate;      // y = silu(gate) * y, or null
+    float* parts;                       // K split over blockIdx.y: fp32 partial products [gridDim.y][M][N], or null
+};
+
+// 16 bytes per lane, global -> LDS: lane L of the wave lands at lds + 16 L.  Scalar base + 32-bit byte offset per lane.
+__device__ __forceinline__ void tg_dma(uint32_t lds, const void* base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void tg_wait_barrier() {
+    // lgkmcnt: this wave's reads of the buffer that the next requests overwrite have returned
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+template <class F, int WN, int KW, int MT, int NT>
+__global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmArgs a) {
+    constexpr int STAGES = 4, G = WN, BM = 32 * MT, BN = 32 * NT * WN;
+    constexpr int ABYTES = BM * 128, BBYTES = BN * F::STEP_BYTES, STAGE = ABYTES + BBYTES;
+    constexpr int AREQ = ABYTES / 1024 / G, BREQ = BBYTES / 1024 / G, REQ = AREQ + BREQ;
+    static_assert(AREQ * G * 1024 == ABYTES && BREQ * G * 1024 == BBYTES, "every wave issues the same number of requests");
+    constexpr int ACC = MT * NT * 4096;   // bytes of one wave's accumulators
+    constexpr int LDS = KW * STAGES * STAGE > (KW - 1) * G * ACC ? KW * STAGES * STAGE : (KW - 1) * G * ACC;
+    __shared__ __align__(1024) uint8_t lds[LDS];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = wave / G, gw = wave % G;
+    // consecutive tiles of one XCD share an activation slice
+    const int tile = (int)(blockIdx.x & 7) * a.per_xcd + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= a.per_xcd || tile >= a.tiles) return;
+    const int64_t m0 = (int64_t)(tile / a.tiles_n) * BM, n0 = (int64_t)(tile % a.tiles_n) * BN;
+    // this workgroup's run of 64-wide K steps: all of them, or the blockIdx.y-th of gridDim.y equal parts
+    const int all = (int)(a.K / 64), per = (all + (int)gridDim.y - 1) / (int)gridDim.y, first = per * (int)blockIdx.y;
+    const int KS = min(per, all - first), nst = (KS + KW - 1) / KW;
+
+    // Activation request j of a wave: 8 rows x 128 bytes, slot (row, p) holds k chunk p ^ (row / 2 % 8), so that the fragment
+    // reads below (16 rows, one chunk) cover all banks.  Rows past M repeat the last one; their outputs are not stored.
+    uint32_t aoff[AREQ], boff[BREQ];
+#pragma unroll
+    for (int j = 0; j < AREQ; ++j) {
+        const int row = (gw * AREQ + j) * 8 + (lane >> 3);
+        const int64_t rel = (m0 + row < a.M ? m0 + row : a.M - 1) - m0;
+        aoff[j] = (uint32_t)(rel * a.ldx * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+    }
+#pragma unroll
+    for (int j = 0; j < BREQ; ++j) boff[j] = F::request_offset(a, n0, gw * BREQ + j, lane);
+    const uint16_t* const abase = a.x + m0 * a.ldx;
+    const uint8_t* const bbase = F::tile_base(a, n0);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + group * STAGES * STAGE;
+    auto request = [&](int r, int t, int buf) __attribute__((always_inline)) {
+        int s = t * KW + group;
+        s = first + (s < KS ? s : KS - 1);   // a step past the end repeats the last one and is not multiplied
+        const uint32_t at = lds0 + buf * STAGE;
+        if (r < AREQ)
+            tg_dma(at + (gw * AREQ + r) * 1024, abase + (int64_t)s * 64, aoff[r]);
+        else
+            tg_dma(at + ABYTES + (gw * BREQ + r - AREQ) * 1024, F::step_base(a, bbase, s), boff[r - AREQ]);
+    };
+
+    tg_f32x16 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    const int r32 = lane & 31, half = lane >> 5;
+    typename F::Row row_const[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) row_const[j] = F::row(a, n0 + (gw * NT + j) * 32 + r32);
+
+    // Steps 0 .. 2 are requested; from then on step t multiplies buffer t, whose first fragments were read before its
+    // barrier, requests step t + 3 into the buffer that step t - 1 has left, and reads ahead: the barrier in front of step t
+    // has seen step t + 1 arrive, so the last slice of a step reads the first fragments of the next one and no wave starts a
+    // step by waiting for LDS.  A slice is MT x NT slots of one matrix instruction each; its share of the conversion, the
+    // LDS reads and the requests are dealt out over the slots.
+    constexpr int SLOTS = MT * NT, PIECES = NT * 4;
+#pragma unroll
+    for (int t = 0; t < STAGES - 1; ++t)
+#pragma unroll
+        for (int r = 0; r < REQ; ++r) request(r, t, t);
+    auto a_at = [&](int buf) { return lds + (group * STAGES + buf) * STAGE; };
+    auto b_at = [&](int buf) { return lds + (group * STAGES + buf) * STAGE + ABYTES; };
+    auto read_a = [&](const uint8_t* A, int i, int s) __attribute__((always_inline)) {
+        return *(const uint4*)(A + (i * 32 + r32) * 128 + (((4 * half + s) ^ ((r32 >> 1) & 7)) << 4));
+    };
+    union Frag { uint32_t u[4]; uint4 q; };
+    Frag fa[2][MT], fb[2][NT];
+    typename F::Raw raw[NT], raw_next[NT];
+    tg_wait_barrier<(STAGES - 3) * REQ>();
+#pragma unroll
+    for (int j = 0; j < NT; ++j) raw[j] = F::read(b_at(0), (gw * NT + j) * 32 + r32, half);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) fa[0][i].q = read_a(a_at(0), i, 0);
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) fb[0][j].u[d] = F::piece(raw[j], 0, d, row_const[j]);
+    int buf = 0;
+    for (int t = 0; t < nst; ++t) {
+        const int next = buf + 1 == STAGES ? 0 : buf + 1, ahead = buf == 0 ? STAGES - 1 : buf - 1;
+        const bool live = KW == 1 || t * KW + group < KS;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int cur = s & 1, nxt = cur ^ 1;
+#pragma unroll
+            for (int q = 0; q < SLOTS; ++q) {
+                const int i = q % MT, j = q / MT;
+                if (live) acc[i][j] = F::mul(fb[cur][j].q, fa[cur][i].q, acc[i][j]);
+                if (q < MT) fa[nxt][q].q = s < 3 ? read_a(a_at(buf), q, s + 1) : read_a(a_at(next), q, 0);
+                if (s == 2 && q < NT) raw_next[q] = F::read(b_at(next), (gw * NT + q) * 32 + r32, half);
+#pragma unroll
+                for (int p = q * PIECES / SLOTS; p < (q + 1) * PIECES / SLOTS; ++p)
+                    fb[nxt][p / 4].u[p % 4] = F::piece(s < 3 ? raw[p / 4] : raw_next[p / 4], (s + 1) & 3, p % 4, row_const[p / 4]);
+                if (s < 2)
+#pragma unroll
+                    for (int r = (s * SLOTS + q) * REQ / (2 * SLOTS); r < (s * SLOTS + q + 1) * REQ / (2 * SLOTS); ++r) request(r, t + STAGES - 1, ahead);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) raw[j] = raw_next[j];
+        tg_wait_barrier<(STAGES - 3) * REQ>();
+        buf = next;
+    }
+    // requests past the end have landed before LDS is used again or the workgroup ends
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    if (KW > 1) {
+        __syncthreads();
+        float* mine = (float*)(lds + ((group > 0 ? group - 1 : 0) * G + gw) * ACC) + lane * 4;
+        if (group > 0)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; e += 4)
+                        *(float4*)(mine + ((i * NT + j) * 4 + e / 4) * 256) =
+                            make_float4(acc[i][j][e], acc[i][j][e + 1], acc[i][j][e + 2], acc[i][j][e + 3]);
+        __syncthreads();
+        if (group > 0) return;
+#pragma unroll
+        for (int g = 0; g < KW - 1; ++g)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; e += 4) {
+                        const float4 v = *(const float4*)((const float*)(lds + (g * G + gw) * ACC) + lane * 4 + ((i * NT + j) * 4 + e / 4) * 256);
+                        acc[i][j][e] += v.x; acc[i][j][e + 1] += v.y; acc[i][j][e + 2] += v.z; acc[i][j][e + 3] += v.w;
+                    }
+    }
+    // acc[i][j][e]: output row m = 32 i + lane % 32, column n = 32 j + 8 (e / 4) + 4 (lane / 32) + e % 4
+    const bool wide = (a.ldy & 3) == 0 && ((uintptr_t)a.y & 7) == 0;
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; e += 4) {
+            const int64_t n = n0 + (gw * NT + j) * 32 + 8 * (e >> 2) + 4 * half;
+            const typename F::Cols cols = F::columns(a, n);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const int64_t m = m0 + i * 32 + r32;
+                if (m >= a.M) continue;
+                if (a.parts) {
+                    float* dst = a.parts + ((int64_t)blockIdx.y * a.M + m) * a.N + n;
+                    if ((a.N & 3) == 0 && n + 3 < a.N)
+                        *(float4*)dst = make_float4(acc[i][j][e], acc[i][j][e + 1], acc[i][j][e + 2], acc[i][j][e + 3]);
+                    else
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            if (n + v < a.N) dst[v] = acc[i][j][e + v];
+                    continue;
+                }
+                uint16_t o[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) o[v] = F::finish(acc[i][j][e + v], cols, v);
+                F::combine(a, m, n, o);
+                uint16_t* dst = a.y + m * a.ldy + n;
+                if (wide && n + 3 < a.N) {
+                    *(uint2*)dst = make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        if (n + v < a.N) dst[v] = o[v];
+                }
+            }
+        }
+}
+
+// Adds the K parts of a tile_gemm_kernel and finishes as that kernel does: 4 columns a thread.
+template <class F>
+__global__ __launch_bounds__(256) void tile_finish_kernel(const TileGemmArgs a, int nparts) {
+    const int64_t per_row = (a.N + 3) / 4, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t m = i / per_row, n = (i - m * per_row) * 4;
+    if (m >= a.M) return;
+    const bool quad = (a.N & 3) == 0;
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < nparts; ++p) {
+        const float* src = a.parts + ((int64_t)p * a.M + m) * a.N + n;
+        if (quad) {
+            const float4 v = *(const float4*)src;
+            sum[0] += v.x; sum[1] += v.y; sum[2] += v.z; sum[3] += v.w;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if (n + v < a.N) sum[v] += src[v];
+        }
+    }
+    const typename F::Cols cols = F::columns(a, n);
+    uint16_t o[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) o[v] = F::finish(sum[v], cols, v);
+    uint16_t* dst = a.y + m * a.ldy + n;
+    if (quad && (a.ldy & 3) == 0 && ((uintptr_t)a.y & 7) == 0) {
+        *(uint2*)dst = make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
+    } else {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            if (n + v < a.N) dst[v] = o[v];
+    }
+}
+
+// Tile shape and K parts for M x N x K: the cheapest by a measured model.  A shape costs `one` us for a wave of workgroups
+// over 4096 of K with one workgroup on a CU and `two` with two (0: only one fits), 6 us of it whatever K is; K parts add a
+// second launch and 8 bytes of fp32 per output and part.
+struct TileShape {
+    int bm, bn;
+    double one, two;
+};
+struct TilePlan {
+    int shape, parts;
+    double us;
+};
+inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64_t N, int64_t K, int max_parts) {
+    TilePlan best{-1, 1, 1e30};
+    const int64_t steps = K / 64;
+    for (int i = 0; i < nshapes; ++i)
+        for (int z = 1; z <= max_parts; z *= 2) {
+            const int64_t per = (steps + z - 1) / z;
+            if (z > 1 && (per < 8 || (z - 1) * per >= steps)) break;
+            const int64_t wgs = (M + shapes[i].bm - 1) / shapes[i].bm * ((N + shapes[i].bn - 1) / shapes[i].bn) * z;
+            const int64_t fit = shapes[i].two > 0 ? 512 : 256, full = wgs / fit, rest = wgs % fit;
+            auto us = [&](double t) { return 6.0 + (t - 6.0) * (double)per / 64.0; };
+            const double wave = us(shapes[i].two > 0 ? shapes[i].two : shapes[i].one);
+            double t = full * wave + (rest == 0 ? 0.0 : rest <= 256 ? us(shapes[i].one) : wave);
+            if (z > 1) t += 3.0 + 8e-6 * (double)(M * N * z) / 4.0;
+            if (t < best.us) best = TilePlan{i, z, t};
+        }
+    return best;
+}
+
+}  // namespace ao

@@ -83,16 +83,16 @@ TWO_PASS_MIN_M = 4096
 
 
 # int8 and FPx: the same choice.  The conversion pass costs the same whatever the row count, so the narrower the weight
-# the later it pays (fused / two-pass in us, int8: 14336 x 4096 at 96 / 128 / 256 rows 57 / 58, 73 / 61, 128 / 76;
-# 4096 x 4096 at 128 / 256 / 384 rows 22 / 42, 40 / 42, 53 / 41; 4096 x 14336 at 128 / 192 / 256 rows 64 / 93, 125 / 113,
-# 125 / 80; 1024 x 4096 at 512 / 1536 rows 22 / 37, 51 / 38.  FP6: 14336 x 4096 at 768 / 1024 rows 115 / 126, 142 / 134;
-# 4096 x 4096 at 1024 / 1536 / 3072 rows 50 / 54, 71 / 66, 113 / 96; 1024 x 4096 at 2048 / 3072 rows 32 / 36, 46 / 41).
+# the later it pays.  int8, fused (tiled kernel) / two-pass in us: 14336 x 4096 at 1024 / 1536 / 2048 rows 140 / 138, 202 / 198,
+# 271 / 226; 28672 x 8192 at 1024 / 1536 / 2048 rows 482 / 518, 693 / 657, 912 / 818; 4096 x 14336 at 2048 rows 211 / 229;
+# 4096 x 4096 at 2048 rows 71 / 82.  FP6: 14336 x 4096 at 768 / 1024 rows 115 / 126, 142 / 134; 4096 x 4096 at 1024 / 1536 /
+# 3072 rows 50 / 54, 71 / 66, 113 / 96; 1024 x 4096 at 2048 / 3072 rows 32 / 36, 46 / 41.
 INT8_TWO_PASS_MIN_M = 128
 FP6_TWO_PASS_MIN_M = 1024
 
 
 def int8wo_two_pass(M: int, N: int, K: int) -> bool:
-    return M >= INT8_TWO_PASS_MIN_M and (M * N >= 1500000 or (K >= 8192 and M * N >= 700000))
+    return M >= INT8_TWO_PASS_MIN_M * (12 if N >= 8192 else 32)
 
 
 def fp6_two_pass(M: int, N: int, K: int) -> bool:
@@ -268,16 +268,19 @@ def _int8wo_linear_cuda(x, w_int8, scale, bias, fp32_out):
         bias = bias.contiguous()
     if int8wo_two_pass(M, N, K) and not fp32_out and K % 16 == 0:
         # prefill-sized batch: bf16 copy of the codes (HIP kernel), library bf16 GEMM, scale, bias: the reference's
-        # `torch.mm(x, w_int8.t().to(x.dtype)) * scale` (+ bias) op by op.  The streaming kernel below re-reads the
-        # weight for every 16 activation rows and falls behind from about 128 rows on.
+        # `torch.mm(x, w_int8.t().to(x.dtype)) * scale` (+ bias) op by op
         wb = torch.empty((N, K), dtype=torch.bfloat16, device=x.device)
         check(lib().ao_amd_int8_to_bf16(w_int8.data_ptr(), N, K, w_int8.stride(0), wb.data_ptr(), current_stream(x.device)))
         y = torch.nn.functional.linear(x, wb) * scale
         return y if bias is None else y + bias
     y = torch.empty((M, N), dtype=torch.float32 if fp32_out else torch.bfloat16, device=x.device)
-    check(lib().ao_amd_int8wo_linear(x.data_ptr(), M, K, x.stride(0) if M > 0 else K, w_int8.data_ptr(),
-                                     w_int8.stride(0), scale.data_ptr(), N, None if bias is None else bias.data_ptr(),
-                                     y.data_ptr(), F32 if fp32_out else BF16, N, current_stream(x.device)))
+    need = ctypes.c_int64(0)
+    check(lib().ao_amd_int8wo_linear_ws_bytes(M, K, N, ctypes.byref(need)))
+    ws = torch.empty((need.value // 4,), dtype=torch.float32, device=x.device) if need.value else None
+    check(lib().ao_amd_int8wo_linear_ws(x.data_ptr(), M, K, x.stride(0) if M > 0 else K, w_int8.data_ptr(),
+                                        w_int8.stride(0), scale.data_ptr(), N, None if bias is None else bias.data_ptr(),
+                                        y.data_ptr(), F32 if fp32_out else BF16, N, None if ws is None else ws.data_ptr(),
+                                        need.value, current_stream(x.device)))
     return y
 
 

@@ -1,0 +1,62 @@
+"""The tiled product (tile_gemm.h) at the sizes where it can go wrong: rows and columns around the edges of every tile shape,
+fewer K steps than the prefetch distance or than the wave groups along K, K parts with a short last part, strided
+activations, odd output widths."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (M, N, K): every tile shape of the int8 table, with and without K parts (checked below)
+CASES = [
+    (17, 4100, 8320), (33, 4096, 8192), (64, 3072, 4224), (65, 5121, 6528), (96, 8200, 4096), (97, 16400, 4096), (129, 1100, 4096),
+    (191, 16400, 2048), (192, 24600, 2048), (193, 15000, 2176), (255, 14336, 1024), (256, 14336, 1024), (257, 21000, 1024), (384, 12416, 2048),
+    (769, 130, 128), (770, 127, 256), (1000, 600, 1024), (1025, 14336, 512), (513, 28672, 640),
+    (1, 300, 64), (5, 2000, 192), (40, 4096, 8256),  # in_features not a multiple of 128: any row count
+]
+
+
+def _plan(M, N, K):
+    from ao_amd import _lib
+
+    out = ctypes.create_string_buffer(64)
+    _lib.check(_lib.lib().ao_amd_int8wo_linear_plan(M, K, N, out, 64))
+    return out.value.decode()
+
+
+def _run(M, N, K, bias=False, pad=0):
+    from ao_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w = torch.randint(-128, 128, (N, K), device="cuda", dtype=torch.int8, generator=g)
+    x = torch.randn(M, K + pad, device="cuda", generator=g).bfloat16()[:, :K]
+    s = (torch.rand(N, device="cuda", generator=g) * 0.01 + 0.001).bfloat16()
+    b = torch.randn(N, device="cuda", generator=g).bfloat16() if bias else None
+    y = ops.int8wo_linear(x, w, s, b)
+    acc = x.float() @ w.float().t()
+    want = (acc.bfloat16().float() * s.float()).bfloat16()
+    if bias:
+        want = (want.float() + b.float()).bfloat16()
+    rel = ((y.float() - want.float()).norm() / want.float().norm()).item()
+    # exact products; sums of K <= 8320 of them in fp32 differ by their order in about 1e-6 relative, which moves a rounding
+    # of the result (relative step 2^-8) now and then: few elements, by one step of the value (or of the sum before the
+    # bias, which can cancel)
+    assert (y != want).float().mean() <= 0.01 and rel <= 1e-3, (M, N, K, rel)
+
+
+def test_cases_cover_every_tile_shape():
+    plans = {c: _plan(*c) for c in CASES}
+    shapes = {p.split()[1] for p in plans.values() if p != "streaming"}
+    assert shapes == {"64x128", "96x128", "128x128", "192x128", "128x256"}, plans
+    assert any(p.endswith("parts=1") for p in plans.values()) and any(not p.endswith("parts=1") for p in plans.values())
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_int8_tiles(case):
+    _run(*case)
+
+
+@pytest.mark.parametrize("case", [(65, 5121, 6528), (257, 21000, 1024), (129, 1100, 4096)])
+def test_int8_tiles_bias_and_row_stride(case):
+    _run(*case, bias=True, pad=72)
