@@ -8,6 +8,8 @@
 // product over K, x @ W^T for the transposed product over N that the backward pass of a fine-tuning run needs):
 // the packed layout is N-major, so a thread that takes 16 consecutive bytes of one k2 row produces two 32-byte
 // runs of the output rows 2*k2 and 2*k2 + 1, and neighbouring threads continue those rows.
+#include <type_traits>
+
 #include "common.h"
 
 namespace ao {
@@ -234,21 +236,32 @@ __device__ __forceinline__ hqq_f32x4_t hqq_mfma(const u32x4_t a, const uint32_t 
     }
 }
 
-// two codes (unsigned nibbles u0, u1; sign-extended when SIGNED) with the (scale, zero) pairs sz0, sz1 (each one dword:
-// two 16-bit values of the storage dtype, scale low / zero high is NOT assumed: s2 and z2 are dwords holding the pair
-// (value for code 0, value for code 1)) -> the two weights (q - z) * s packed in one dword
-template <bool BF16, bool SIGNED>
-__device__ __forceinline__ uint32_t hqq_weight_pair(uint32_t u0, uint32_t u1, uint32_t s2, uint32_t z2) {
+// The eight codes of a dword of four byte rows or columns -> low and high nibbles as one byte each: the byte-to-float
+// conversions and byte permutes below then take them in place (shifting every code down to bit 0 first cost a third of the
+// kernel's instructions).  The sign bit of a signed nibble is flipped: code = byte - 8.
+template <bool SIGNED>
+__device__ __forceinline__ void hqq_nibbles(uint32_t w, uint32_t& lo, uint32_t& hi) {
+    lo = w & 0x0f0f0f0fu;
+    hi = (w >> 4) & 0x0f0f0f0fu;
+    if (SIGNED) {
+        lo ^= 0x08080808u;
+        hi ^= 0x08080808u;
+    }
+}
+// codes in bytes B0 of `a` and B1 of `b` -> the weight pair (q - z) * s, each operation rounded to the storage type; scales
+// and zeros as a packed pair (fp16) or as fp32 values (bf16)
+template <bool BF16, bool SIGNED, int B0, int B1>
+__device__ __forceinline__ uint32_t hqq_pair(uint32_t a, uint32_t b, uint32_t s2, uint32_t z2, float s0, float s1, float z0, float z1) {
     if (BF16) {
-        const float q0 = SIGNED ? (float)((int)(u0 ^ 8u) - 8) : (float)u0;
-        const float q1 = SIGNED ? (float)((int)(u1 ^ 8u) - 8) : (float)u1;
-        const float z0 = __uint_as_float(z2 << 16), z1 = __uint_as_float(z2 & 0xffff0000u);
-        const float s0 = __uint_as_float(s2 << 16), s1 = __uint_as_float(s2 & 0xffff0000u);
+        float q0 = (float)((a >> (8 * B0)) & 0xffu), q1 = (float)((b >> (8 * B1)) & 0xffu);
+        if (SIGNED) {
+            q0 -= 8.0f;   // exact
+            q1 -= 8.0f;
+        }
         return hw_bf16_pack(hw_rne_bf16(q0 - z0) * s0, hw_rne_bf16(q1 - z1) * s1);
     } else {
-        // 0x6400 | u is the fp16 value 1024 + u, exactly; subtracting 1024 (or 1032 with the nibble's sign bit flipped)
-        // leaves the code as an fp16 value without a conversion
-        const uint32_t m = (SIGNED ? ((u0 ^ 8u) | ((u1 ^ 8u) << 16)) : (u0 | (u1 << 16))) | 0x64006400u;
+        // 0x6400 | u is the fp16 value 1024 + u, exactly: one byte permute builds the pair without a conversion
+        const uint32_t m = __builtin_amdgcn_perm(b, a, 0x0c000c00u | B0 | ((4u + B1) << 16)) | 0x64006400u;
         hqq_f16x2_t q, s, z;
         __builtin_memcpy(&q, &m, 4);
         __builtin_memcpy(&s, &s2, 4);
@@ -262,18 +275,48 @@ __device__ __forceinline__ uint32_t hqq_weight_pair(uint32_t u0, uint32_t u1, ui
     }
 }
 
-template <bool BF16, bool SIGNED, bool TRANSPOSED, int MB>
-__global__ __launch_bounds__(256) void hqq_mm_mfma_kernel(const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scales,
+// One wave's run of steps, loaded one ahead into two fragment sets that are used in turn (a copy from the one to the other was
+// a seventh of the loop).  COPY: where the two halves together need more registers than they save time.
+template <class Frag, bool COPY, class Load, class Compute>
+__device__ __forceinline__ void hqq_run(int s0, int s1, const Load& load, const Compute& compute) {
+    Frag fa, fb;
+    load(s0, fa);
+    if (COPY) {
+        for (int s = s0; s < s1; ++s) {
+            load(s + 1, fb);
+            compute(s, fa);
+            fa = fb;
+        }
+        return;
+    }
+    for (int s = s0; s < s1; s += 2) {
+        load(s + 1, fb);
+        compute(s, fa);
+        if (s + 1 >= s1) break;
+        load(s + 2, fa);
+        compute(s + 1, fb);
+    }
+}
+
+// Waves of a workgroup: each takes a run of the reduction, and they add up in LDS.  A step's loads take a microsecond and a
+// wave keeps one step ahead in flight, so the runs are kept short (2 - 4 steps) and the waves many; eight of them to a
+// workgroup keep the number of fp32 partial sums in memory where four waves with runs of eight steps had it.
+
+// RB (transposed product): blocks of 16 byte rows per wave.  With two of them in one quantization group the activation
+// fragments and the scales and zeros, 128 bytes a lane and step, serve 32 bytes of codes instead of 16.
+template <bool BF16, bool SIGNED, bool TRANSPOSED, int MB, int RB, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* __restrict__ packed, const uint16_t* __restrict__ scales,
                                                           const uint16_t* __restrict__ zeros, const uint16_t* __restrict__ a,
                                                           int64_t lda, int M, int64_t K, int64_t N, int64_t group,
                                                           int steps, int steps_per_wave, float* __restrict__ part) {
-    constexpr int NACC = TRANSPOSED ? 2 : 4;   // accumulators per block of 16 activation rows
-    __shared__ float red[4][NACC * 4][64];
+    static_assert(TRANSPOSED || RB == 1, "the forward product takes one block of columns per wave");
+    constexpr int NACC = TRANSPOSED ? 2 * RB : 4;   // accumulators per block of 16 activation rows
+    __shared__ float red[WAVES][NACC * 4][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 15, q4 = lane >> 4;
     const int64_t K2 = K / 2;
-    const int s0 = ((int)blockIdx.y * 4 + wave) * steps_per_wave;
+    const int s0 = ((int)blockIdx.y * WAVES + wave) * steps_per_wave;
     const int s1 = s0 + steps_per_wave < steps ? s0 + steps_per_wave : steps;
     hqq_f32x4_t acc[MB][NACC];
 #pragma unroll
@@ -294,7 +337,8 @@ __global__ __launch_bounds__(256) void hqq_mm_mfma_kernel(const uint8_t* __restr
         const bool live = n0 < N;   // N is a multiple of 4
         struct Frag { uint32_t d[4]; u32x4_t x[MB]; };
         int64_t g_cur = -1;
-        uint32_t sv[2] = {0u, 0u}, zv[2] = {0u, 0u};   // (col 0, col 1), (col 2, col 3)
+        uint32_t sv[4] = {0u, 0u, 0u, 0u}, zv[4] = {0u, 0u, 0u, 0u};   // a column's value twice
+        float sf[4] = {0.f, 0.f, 0.f, 0.f}, zf[4] = {0.f, 0.f, 0.f, 0.f};
         auto load = [&](int s, Frag& f) {
             const int64_t k2 = (int64_t)s * 16 + 4 * q4;
             const bool ok = s < s1 && k2 < K2;   // K is a multiple of 8: the lane's 4 byte rows exist together
@@ -307,92 +351,108 @@ __global__ __launch_bounds__(256) void hqq_mm_mfma_kernel(const uint8_t* __restr
         auto compute = [&](int s, const Frag& f) {
             const int64_t k2 = (int64_t)s * 16 + 4 * q4;
             const int64_t g = (2 * k2) / group;   // group is a multiple of 8: one group for the lane's 8 k
-            if (g != g_cur && live && k2 < K2) {
+            if (g != g_cur && live && s < s1 && k2 < K2) {
                 g_cur = g;
                 const uint2 s2 = *reinterpret_cast<const uint2*>(scales + g * N + n0);
                 const uint2 z2 = *reinterpret_cast<const uint2*>(zeros + g * N + n0);
-                sv[0] = s2.x; sv[1] = s2.y; zv[0] = z2.x; zv[1] = z2.y;
-            }
+                const uint32_t ss[2] = {s2.x, s2.y}, zz[2] = {z2.x, z2.y};
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                // both nibbles of a byte belong to column c: the pair's scale and zero are the same value twice
-                const uint32_t s16 = (c & 1) ? (sv[c >> 1] >> 16) : (sv[c >> 1] & 0xffffu);
-                const uint32_t z16 = (c & 1) ? (zv[c >> 1] >> 16) : (zv[c >> 1] & 0xffffu);
-                const uint32_t s2 = s16 | (s16 << 16), z2 = z16 | (z16 << 16);
-                uint32_t b[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const uint32_t byte = (f.d[r] >> (8 * c)) & 0xffu;
-                    b[r] = hqq_weight_pair<BF16, SIGNED>(byte & 15u, byte >> 4, s2, z2);
+                for (int c = 0; c < 4; ++c) {
+                    const uint32_t sh = (c & 1) ? ss[c >> 1] >> 16 : ss[c >> 1] & 0xffffu, zh = (c & 1) ? zz[c >> 1] >> 16 : zz[c >> 1] & 0xffffu;
+                    sv[c] = sh | (sh << 16);
+                    zv[c] = zh | (zh << 16);
+                    sf[c] = __uint_as_float(sh << 16);
+                    zf[c] = __uint_as_float(zh << 16);
                 }
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb) acc[mb][c] = hqq_mfma<BF16>(f.x[mb], b, acc[mb][c]);
             }
+            uint32_t lo[4], hi[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) hqq_nibbles<SIGNED>(f.d[r], lo[r], hi[r]);
+            // both nibbles of byte c belong to column c
+            auto column = [&](auto c_c) {
+                constexpr int c = decltype(c_c)::value;
+                uint32_t w[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) w[r] = hqq_pair<BF16, SIGNED, c, c>(lo[r], hi[r], sv[c], zv[c], sf[c], sf[c], zf[c], zf[c]);
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) acc[mb][c] = hqq_mfma<BF16>(f.x[mb], w, acc[mb][c]);
+            };
+            column(std::integral_constant<int, 0>());
+            column(std::integral_constant<int, 1>());
+            column(std::integral_constant<int, 2>());
+            column(std::integral_constant<int, 3>());
         };
-        Frag cur, nxt;
-        load(s0, cur);
-        for (int s = s0; s < s1; ++s) {
-            load(s + 1, nxt);
-            compute(s, cur);
-            cur = nxt;
-        }
+        hqq_run<Frag, (MB >= 2)>(s0, s1, load, compute);
     } else {
-        const int64_t k2 = (int64_t)blockIdx.x * 16 + j;
-        const bool live = k2 < K2;
-        const int64_t g = live ? (2 * k2) / group : 0;
+        int64_t k2[RB];
+        bool live[RB];
+        const uint8_t* prow[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            k2[rb] = (int64_t)blockIdx.x * 16 * RB + 16 * rb + j;
+            live[rb] = k2[rb] < K2;
+            prow[rb] = packed + (live[rb] ? k2[rb] : 0) * N;
+        }
+        const int64_t g = live[0] ? (2 * k2[0]) / group : 0;   // RB == 2: the host has checked that both blocks share it
         const uint16_t* srow = scales + g * N;
         const uint16_t* zrow = zeros + g * N;
-        const uint8_t* prow = packed + (live ? k2 : 0) * N;
-        struct Frag { u32x4_t d, s[2], z[2], x[MB][2]; };
+        struct Frag { u32x4_t d[RB], s[2], z[2], x[MB][2]; };
         auto load = [&](int s, Frag& f) {
             const int64_t n = (int64_t)s * 64 + 16 * q4;
             const bool ok = s < s1 && n < N;   // N is a multiple of 16
-            const bool w = ok && live;
-            f.d = w ? *reinterpret_cast<const u32x4_t*>(prow + n) : zero4;
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) f.d[rb] = ok && live[rb] ? *reinterpret_cast<const u32x4_t*>(prow[rb] + n) : zero4;
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                f.s[h] = w ? *reinterpret_cast<const u32x4_t*>(srow + n + 8 * h) : zero4;
-                f.z[h] = w ? *reinterpret_cast<const u32x4_t*>(zrow + n + 8 * h) : zero4;
+                f.s[h] = ok ? *reinterpret_cast<const u32x4_t*>(srow + n + 8 * h) : zero4;
+                f.z[h] = ok ? *reinterpret_cast<const u32x4_t*>(zrow + n + 8 * h) : zero4;
 #pragma unroll
                 for (int mb = 0; mb < MB; ++mb)
                     f.x[mb][h] = ok ? *reinterpret_cast<const u32x4_t*>(arow[mb] + n + 8 * h) : zero4;
             }
         };
-        auto compute = [&](const Frag& f) {
-            const uint32_t dd[4] = {f.d.x, f.d.y, f.d.z, f.d.w};
+        auto compute = [&](int, const Frag& f) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const uint32_t ss[4] = {f.s[h].x, f.s[h].y, f.s[h].z, f.s[h].w};
                 const uint32_t zz[4] = {f.z[h].x, f.z[h].y, f.z[h].z, f.z[h].w};
-                uint32_t lo[4], hi[4];
+                float sl[4], sh[4], zl[4], zh[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    // reduction indices 8 h + 2 i, 8 h + 2 i + 1: bytes 2 i and 2 i + 1 of dword pair h
-                    const uint32_t two = (dd[2 * h + (i >> 1)] >> (16 * (i & 1))) & 0xffffu;
-                    const uint32_t b0 = two & 0xffu, b1 = two >> 8;
-                    lo[i] = hqq_weight_pair<BF16, SIGNED>(b0 & 15u, b1 & 15u, ss[i], zz[i]);
-                    hi[i] = hqq_weight_pair<BF16, SIGNED>(b0 >> 4, b1 >> 4, ss[i], zz[i]);
+                    sl[i] = __uint_as_float(ss[i] << 16);
+                    sh[i] = __uint_as_float(ss[i] & 0xffff0000u);
+                    zl[i] = __uint_as_float(zz[i] << 16);
+                    zh[i] = __uint_as_float(zz[i] & 0xffff0000u);
                 }
 #pragma unroll
-                for (int mb = 0; mb < MB; ++mb) {
-                    acc[mb][0] = hqq_mfma<BF16>(f.x[mb][h], lo, acc[mb][0]);
-                    acc[mb][1] = hqq_mfma<BF16>(f.x[mb][h], hi, acc[mb][1]);
+                for (int rb = 0; rb < RB; ++rb) {
+                    const uint32_t dd[4] = {f.d[rb].x, f.d[rb].y, f.d[rb].z, f.d[rb].w};
+                    uint32_t lo[4], hi[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i += 2) {
+                        // reduction indices 8 h + 2 i .. + 3: the four bytes of dword 2 h + i / 2
+                        uint32_t nl, nh;
+                        hqq_nibbles<SIGNED>(dd[2 * h + (i >> 1)], nl, nh);
+                        lo[i] = hqq_pair<BF16, SIGNED, 0, 1>(nl, nl, ss[i], zz[i], sl[i], sh[i], zl[i], zh[i]);
+                        hi[i] = hqq_pair<BF16, SIGNED, 0, 1>(nh, nh, ss[i], zz[i], sl[i], sh[i], zl[i], zh[i]);
+                        lo[i + 1] = hqq_pair<BF16, SIGNED, 2, 3>(nl, nl, ss[i + 1], zz[i + 1], sl[i + 1], sh[i + 1], zl[i + 1], zh[i + 1]);
+                        hi[i + 1] = hqq_pair<BF16, SIGNED, 2, 3>(nh, nh, ss[i + 1], zz[i + 1], sl[i + 1], sh[i + 1], zl[i + 1], zh[i + 1]);
+                    }
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb) {
+                        acc[mb][2 * rb] = hqq_mfma<BF16>(f.x[mb][h], lo, acc[mb][2 * rb]);
+                        acc[mb][2 * rb + 1] = hqq_mfma<BF16>(f.x[mb][h], hi, acc[mb][2 * rb + 1]);
+                    }
                 }
             }
         };
-        Frag cur, nxt;
-        load(s0, cur);
-        for (int s = s0; s < s1; ++s) {
-            load(s + 1, nxt);
-            compute(cur);
-            cur = nxt;
-        }
+        hqq_run<Frag, MB == 4>(s0, s1, load, compute);
     }
 
-    // the four waves of the workgroup add up, one block of 16 rows at a time: thread (wave w, lane) sums element r = w
-    // of every accumulator, which is output row 4 (lane / 16) + w of the block and NACC adjacent columns
+    // the waves of the workgroup add up, one block of 16 rows at a time: thread (wave w < 4, lane) sums element r = w of
+    // every accumulator, which is output row 4 (lane / 16) + w of the block and NACC adjacent columns
     const int64_t cols = TRANSPOSED ? K : N;
-    const int64_t col0 = TRANSPOSED ? 2 * ((int64_t)blockIdx.x * 16 + j) : (int64_t)blockIdx.x * 64 + 4 * j;
+    const int64_t col0 = TRANSPOSED ? 2 * ((int64_t)blockIdx.x * 16 * RB + j) : (int64_t)blockIdx.x * 64 + 4 * j;
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
         if (mb) __syncthreads();
@@ -401,34 +461,54 @@ __global__ __launch_bounds__(256) void hqq_mm_mfma_kernel(const uint8_t* __restr
 #pragma unroll
             for (int r = 0; r < 4; ++r) red[wave][c * 4 + r][lane] = acc[mb][c][r];
         __syncthreads();
+        if (wave >= 4) continue;
         const int m = mb * 16 + 4 * q4 + wave;
         float v[NACC];
 #pragma unroll
-        for (int c = 0; c < NACC; ++c)
-            v[c] = red[0][c * 4 + wave][lane] + red[1][c * 4 + wave][lane] + red[2][c * 4 + wave][lane] + red[3][c * 4 + wave][lane];
-        if (m < M && col0 < cols) {
-            float* o = part + ((int64_t)blockIdx.y * M + m) * cols + col0;
-            if (TRANSPOSED) *reinterpret_cast<float2*>(o) = float2{v[0], v[1]};
-            else *reinterpret_cast<float4*>(o) = float4{v[0], v[1], v[NACC - 2], v[NACC - 1]};
+        for (int c = 0; c < NACC; ++c) {
+            v[c] = red[0][c * 4 + wave][lane];
+#pragma unroll
+            for (int w = 1; w < WAVES; ++w) v[c] += red[w][c * 4 + wave][lane];
+        }
+        float* o = part + ((int64_t)blockIdx.y * M + m) * cols + col0;
+        if (TRANSPOSED) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+                if (m < M && col0 + 32 * rb < cols) *reinterpret_cast<float2*>(o + 32 * rb) = float2{v[2 * rb], v[2 * rb + 1]};
+        } else if (m < M && col0 < cols) {
+            *reinterpret_cast<float4*>(o) = float4{v[0], v[1], v[NACC - 2], v[NACC - 1]};
         }
     }
 }
 
-// reduction steps (32 k forward, 64 n transposed), output tiles and the slices of the reduction over workgroups: about
-// 8 steps per wave while that still gives every CU a workgroup, fewer slices for more rows (the partial sums grow with
-// both)
-struct HqqMfmaPlan { int tiles, steps, slices, steps_per_wave; };
-static HqqMfmaPlan hqq_mfma_plan(int64_t M, int64_t K, int64_t N, bool transposed) {
-    HqqMfmaPlan p;
-    p.tiles = (int)(transposed ? (K / 2 + 15) / 16 : (N + 63) / 64);
+// reduction steps (32 k forward, 64 n transposed), output tiles and the slices of the reduction over workgroups
+struct HqqMfmaPlan { int waves, rb, tiles, steps, slices, steps_per_wave; };
+static HqqMfmaPlan hqq_mfma_plan(int64_t M, int64_t K, int64_t N, bool transposed, int64_t group) {
+    HqqMfmaPlan p{};
     p.steps = (int)(transposed ? (N + 63) / 64 : (K + 31) / 32);
-    int per_wave = 8;
-    int slices = (p.steps + 4 * per_wave - 1) / (4 * per_wave);
-    const int cap = M <= 16 ? 16 : M <= 32 ? 8 : 4;
-    if (slices > cap) slices = cap;
-    if (slices < 1) slices = 1;
-    p.steps_per_wave = (p.steps + slices * 4 - 1) / (slices * 4);
-    p.slices = (p.steps + p.steps_per_wave * 4 - 1) / (p.steps_per_wave * 4);
+    // Cheapest by a measured model (in us, 1 to 64 rows, 4096 and 11008 wide): a CU takes 0.15 us for a kilobyte of codes with
+    // all its waves together, eight at least (a step of one wave alone lasts 1.2), plus the start of each run, and its
+    // workgroups come in whole rounds; a slice costs its fp32 partial sums, written and read.
+    // Two blocks of 16 byte rows (64 values of k) per wave in the transposed product where they share their group.
+    const int most_slices = M <= 16 ? 16 : 8;
+    double best = 1e30;
+    for (int rb = 1; rb <= (transposed && group % 64 == 0 ? 2 : 1); ++rb) {
+        const int tiles = (int)(transposed ? (K / 2 + 16 * rb - 1) / (16 * rb) : (N + 63) / 64);
+        for (int waves = 8; waves >= 4 * rb; waves -= 4)   // (four waves of block pairs do not fit the registers twice)
+            for (int slices = 1; slices <= most_slices; ++slices) {
+                if (slices > 1 && p.steps < 2 * waves * slices) break;   // runs of at least two steps
+                const int per = (p.steps + slices * waves - 1) / (slices * waves), z = (p.steps + per * waves - 1) / (per * waves);
+                if (z != slices) continue;
+                // (a block pair reads scales, zeros and activations once for both)
+                const int64_t on_cu = ((int64_t)tiles * z + 255) / 256 * waves;
+                const double us = 0.15 * (rb == 2 ? 1.6 : 1.0) * (double)(on_cu > 8 ? on_cu : 8) * (per + 0.7) +
+                                  2e-6 * (double)(M * (transposed ? K : N)) * z;
+                if (us < best) {
+                    best = us;
+                    p = HqqMfmaPlan{waves, rb, tiles, p.steps, z, per};
+                }
+            }
+    }
     return p;
 }
 
@@ -526,8 +606,9 @@ extern "C" int ao_amd_hqq_mixed_mm_mfma_workspace(int64_t M, int64_t K, int64_t 
     AO_REQUIRE(bytes, "null pointer argument");
     AO_REQUIRE(M >= 1 && M <= 64 && K > 0 && N > 0 && K % 2 == 0, "need 1 <= M <= 64, K even, got M=%lld K=%lld N=%lld",
                (long long)M, (long long)K, (long long)N);
-    const HqqMfmaPlan p = hqq_mfma_plan(M, K, N, transposed != 0);
-    *bytes = (int64_t)p.slices * M * (transposed ? K : N) * (int64_t)sizeof(float);
+    // whatever the group size: the plan depends on whether it is a multiple of 64
+    const int a = hqq_mfma_plan(M, K, N, transposed != 0, 64).slices, b = hqq_mfma_plan(M, K, N, transposed != 0, 2).slices;
+    *bytes = (int64_t)(a > b ? a : b) * M * (transposed ? K : N) * (int64_t)sizeof(float);
     return 0;
 }
 
@@ -558,25 +639,28 @@ extern "C" int ao_amd_hqq_mixed_mm_mfma(const void* a, int64_t M, int64_t lda, c
     if (int rc = ao_amd_hqq_mixed_mm_mfma_workspace(M, K, N, transposed, &need)) return rc;
     AO_REQUIRE(workspace_bytes >= need && (((uintptr_t)workspace) & 15) == 0, "16-byte aligned workspace of %lld bytes needed, got %lld",
                (long long)need, (long long)workspace_bytes);
-    const HqqMfmaPlan p = hqq_mfma_plan(M, K, N, transposed != 0);
+    const HqqMfmaPlan p = hqq_mfma_plan(M, K, N, transposed != 0, group_size);
     const dim3 grid((unsigned)p.tiles, (unsigned)p.slices);
     hipStream_t st = (hipStream_t)stream;
     const uint8_t* pk = (const uint8_t*)packed_2xint4;
     const uint16_t *s = (const uint16_t*)scales, *z = (const uint16_t*)zeros, *av = (const uint16_t*)a;
     float* part = (float*)workspace;
-#define AO_HQQ_MFMA(BF, SG, TR, MBV)                                                                                       \
-    hipLaunchKernelGGL((hqq_mm_mfma_kernel<BF, SG, TR, MBV>), grid, dim3(256), 0, st, pk, s, z, av, lda, (int)M, K, N, \
+#define AO_HQQ_MFMA(BF, SG, TR, MBV, RBV)                                                                                       \
+    if (p.waves == 8 || RBV == 2) hipLaunchKernelGGL((hqq_mm_mfma_kernel<BF, SG, TR, MBV, RBV, 8>), grid, dim3(512), 0, st, pk, s, z, av, lda, (int)M, K, N, \
+                       group_size, p.steps, p.steps_per_wave, part); \
+    else hipLaunchKernelGGL((hqq_mm_mfma_kernel<BF, SG, TR, MBV, 1, 4>), grid, dim3(256), 0, st, pk, s, z, av, lda, (int)M, K, N, \
                        group_size, p.steps, p.steps_per_wave, part)
-#define AO_HQQ_MFMA_M(BF, SG, TR)                    \
-    do {                                             \
-        if (M <= 16) AO_HQQ_MFMA(BF, SG, TR, 1);     \
-        else if (M <= 32) AO_HQQ_MFMA(BF, SG, TR, 2); \
-        else AO_HQQ_MFMA(BF, SG, TR, 4);             \
+#define AO_HQQ_MFMA_M(BF, SG, TR, RBV)                     \
+    do {                                                   \
+        if (M <= 16) { AO_HQQ_MFMA(BF, SG, TR, 1, RBV); }      \
+        else if (M <= 32) { AO_HQQ_MFMA(BF, SG, TR, 2, RBV); } \
+        else { AO_HQQ_MFMA(BF, SG, TR, 4, RBV); }              \
     } while (0)
-#define AO_HQQ_MFMA_T(BF, SG)                         \
-    do {                                              \
-        if (transposed) AO_HQQ_MFMA_M(BF, SG, true);  \
-        else AO_HQQ_MFMA_M(BF, SG, false);            \
+#define AO_HQQ_MFMA_T(BF, SG)                                            \
+    do {                                                                 \
+        if (transposed && p.rb == 2) AO_HQQ_MFMA_M(BF, SG, true, 2);     \
+        else if (transposed) AO_HQQ_MFMA_M(BF, SG, true, 1);             \
+        else AO_HQQ_MFMA_M(BF, SG, false, 1);                            \
     } while (0)
     if (dtype == AO_BF16) {
         if (is_signed) AO_HQQ_MFMA_T(true, true); else AO_HQQ_MFMA_T(true, false);

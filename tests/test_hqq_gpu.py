@@ -271,3 +271,24 @@ def test_matrix_core_product_limits():
     assert ops.hqq_mixed_mm_mfma(torch.randn(4, 128, dtype=torch.float16, device=dev), b, s, z, 64, False).shape == (4, 40)
     with pytest.raises(RuntimeError, match="multiple of 16"):
         ops.hqq_mixed_mm_mfma(torch.randn(4, 40, dtype=torch.float16, device=dev), b, s, z, 64, True)
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("N,K,g", [(2048, 6336, 64), (11008, 1088, 64), (4096, 4160, 32), (208, 14336, 128), (5200, 192, 64)])
+def test_matrix_core_product_over_its_plans(M, N, K, g, transposed):
+    """Workgroups of 4 and 8 waves, one and two byte-row blocks per wave (groups of 64 and more, transposed; K / 64 odd
+    leaves the last block pair half empty), runs of an odd number of steps, waves without a step.  Products of bf16
+    values summed in fp32 in any order and rounded once: 1.5e-3 relative L2, as above."""
+    from ao_amd import ops
+    from ao_amd.prototype.hqq.mixed_mm import pack_2xint4
+
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    q = torch.randint(0, 16, (K, N), dtype=torch.uint8, device="cuda", generator=gen)
+    s = (torch.rand(K // g, N, device="cuda", generator=gen) * 0.02 + 1e-3).bfloat16()
+    z = (torch.rand(K // g, N, device="cuda", generator=gen) * 6 + 5).bfloat16()
+    w = ((q.bfloat16().reshape(K // g, g, N) - z[:, None]) * s[:, None]).reshape(K, N).double()
+    x = torch.randn(M, N if transposed else K, device="cuda", generator=gen).bfloat16()
+    got = ops.hqq_mixed_mm_mfma(x, pack_2xint4(q), s, z, g, transposed)
+    want = (x.double() @ (w.t() if transposed else w)).bfloat16()
+    assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 1.5e-3
