@@ -11,28 +11,32 @@ namespace ao {
 typedef __bf16 i8_bf16x8 __attribute__((ext_vector_type(8)));
 
 struct Int8Tile {
-    static constexpr int STEP_BYTES = 64;   // of one weight row per 64-wide K step
+    static constexpr int REQ = 2, BLOCK_BYTES = 2048;   // 32 rows x 64 bytes
     struct Row {};
     struct Raw { uint4 v[2]; };             // 32 consecutive k of one row
+    typedef Raw Ready;
     struct Cols { float scale[4], bias[4]; bool has_bias; };
 
-    // request j of a tile: 16 rows x 64 bytes; slot (row, p) holds 16-byte chunk p ^ (row / 4 % 4): conflict-free reads
-    static __device__ __forceinline__ uint32_t request_offset(const TileGemmArgs& a, int64_t n0, int j, int lane) {
-        const int row = j * 16 + (lane >> 2);
-        const int64_t rel = (n0 + row < a.N ? n0 + row : a.N - 1) - n0;   // rows past N repeat the last one
+    // request r: 16 rows x 64 bytes; slot (row, p) holds 16-byte chunk p ^ (row / 4 % 4): conflict-free reads
+    static __device__ __forceinline__ uint32_t lane_offset(const TileGemmArgs& a, int64_t n0, int64_t n, int r, int lane) {
+        const int row = r * 16 + (lane >> 2);
+        const int64_t rel = (n + row < a.N ? n + row : a.N - 1) - n0;   // rows past N repeat the last one
         return (uint32_t)(rel * a.ldw) + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
     }
-    static __device__ __forceinline__ const uint8_t* tile_base(const TileGemmArgs& a, int64_t n0) { return a.w + n0 * a.ldw; }
-    static __device__ __forceinline__ const uint8_t* step_base(const TileGemmArgs&, const uint8_t* base, int s) { return base + (int64_t)s * 64; }
+    static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, uint32_t off) {
+        tg_dma(lds + r * 1024, a.w + n0 * a.ldw + (int64_t)s * 64, off);
+    }
     static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) { return Row(); }
-    static __device__ __forceinline__ Raw read(const uint8_t* B, int n, int half) {
+    static __device__ __forceinline__ Raw read(const uint8_t* block, int lane) {
+        const int n = lane & 31, half = lane >> 5;
         Raw r;
-        r.v[0] = *(const uint4*)(B + n * 64 + (((2 * half) ^ ((n >> 2) & 3)) << 4));
-        r.v[1] = *(const uint4*)(B + n * 64 + (((2 * half + 1) ^ ((n >> 2) & 3)) << 4));
+        r.v[0] = *(const uint4*)(block + n * 64 + (((2 * half) ^ ((n >> 2) & 3)) << 4));
+        r.v[1] = *(const uint4*)(block + n * 64 + (((2 * half + 1) ^ ((n >> 2) & 3)) << 4));
         return r;
     }
+    static __device__ __forceinline__ Ready prepare(const Raw& r, const Row&) { return r; }
     // dword d (k = 8 s + 2 d, + 1) of slice s
-    static __device__ __forceinline__ uint32_t piece(const Raw& r, int s, int d, const Row&) {
+    static __device__ __forceinline__ uint32_t piece(const Ready& r, int s, int d) {
         const uint4 v = r.v[s >> 1];
         const uint32_t w = s & 1 ? (d < 2 ? v.z : v.w) : (d < 2 ? v.x : v.y);
         float f0, f1;
@@ -53,7 +57,7 @@ struct Int8Tile {
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             const int64_t i = n + v < a.N ? n + v : a.N - 1;
-            c.scale[v] = bf16_bits_to_f32(a.scale[i]);
+            c.scale[v] = bf16_bits_to_f32(((const uint16_t*)a.scale)[i]);
             c.bias[v] = a.bias ? bf16_bits_to_f32(a.bias[i]) : 0.f;
         }
         return c;

@@ -509,7 +509,12 @@ static int int8wo_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
         while (waves < 16 && xbytes > (int64_t)waves * 16 * 1024) waves *= 2;
     // staging costs a pass over the rows and a barrier: it pays once a wave has 4 or more K tiles to stream
     // (the staged path addresses the weight with 32-bit per-lane offsets)
-    const bool fits = xbytes <= 64 * 1024 && xbytes <= (int64_t)waves * 16 * 1024 && N * ldw < ((int64_t)1 << 32);
+    // ... or 140 KB, one workgroup to a CU, where the row blocks are no more than the CUs and there is nothing to share a CU
+    // with: the unstaged kernel's activation loads return in order with its weight loads and hold back the requests for
+    // weights (4096 x 14336 at 3 / 4 / 5 rows 19.4 / 20.0 / 20.3 -> 16.8 / 17.2 / 17.3 us, 4096 x 11008 at 6 rows 16.1 ->
+    // 15.3)
+    const bool one_each = !need_lds && xbytes <= 140 * 1024 && waves == 16 && RB * mchunks <= 256;
+    const bool fits = ((xbytes <= 64 * 1024 && xbytes <= (int64_t)waves * 16 * 1024) || one_each) && N * ldw < ((int64_t)1 << 32);
     // ... and, from three rows on, only where the kernel with four row blocks per workgroup below does not apply: it
     // needs no staging pass (14336 x 4096 at 3 / 4 / 5 / 8 rows: 17.2 / 17.7 / 21.9 / 23.3 us staged, 16.6 / 16.9 / 17.2 /
     // 17.4 us not; at 2 rows the staged kernel is as fast or faster everywhere: 28672 x 4096 25.9 against 30.6 us)
@@ -562,7 +567,7 @@ static int int8wo_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
 }
 
 // Where the tiled product serves instead of the streaming kernels above, which read the weight once per 16 or 32 rows.
-static bool tiled(int64_t M, int64_t N, int64_t K) {
+static bool tiled(int64_t M, int64_t N, int64_t K, bool workspace) {
     static const int forced = [] { const char* e = knob("AO_AMD_INT8_TILED"); return e ? atoi(e) : -1; }();
     if (forced >= 0) return forced != 0 && M > 0;
     // The streaming kernels hold on where the weight is small enough to be read again per 32 rows, and where a launch of
@@ -572,7 +577,14 @@ static bool tiled(int64_t M, int64_t N, int64_t K) {
     // In_features that are a multiple of 64 but not of 128 run on tiles whatever the rows: the streaming kernels walk 128-wide
     // tiles of K.
     const int64_t weight = N * K;
-    return K % 128 != 0 || M > (weight >= (32 << 20) ? 16 : weight >= (12 << 20) ? 32 : weight >= (3 << 20) ? 128 : 768);
+    if (K % 128 != 0) return M > 0;
+    if (weight < (32 << 20)) return M > (weight >= (12 << 20) ? 32 : weight >= (3 << 20) ? 128 : 768);
+    // Long rows: every 16 or 64 rows of W read all of x again (8192 x 28672 at 3 / 8 / 16 rows 62 / 72 / 87 us streaming, 54 /
+    // 54 / 57 tiled; 8192 x 8192 at 8 / 16 rows 23.5 / 26.6, 22.2 / 22.7; 28672 x 8192 at 12 / 16 rows 66 / 69, 61 / 62; but
+    // 14336 x 8192 at 12 / 16 rows, one even pass of four-block workgroups, 35 / 37 and 37 / 38).
+    // At so few rows the tiles fill the chip only with K split over workgroups, which takes a workspace.
+    if (workspace && K >= 16384 && N <= 16384) return M > 2;
+    return M > (workspace && K >= 8192 && (N <= 8192 || N >= 24576) ? 8 : 16);
 }
 
 static int int8wo_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* w_int8, int64_t ldw, const void* scale_bf16,
@@ -590,9 +602,9 @@ static int int8wo_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, c
     AO_REQUIRE(192 * ldx * 2 < ((int64_t)1 << 32) && 256 * ldw < ((int64_t)1 << 32) && M * N < ((int64_t)1 << 40), "operands too large");
     TilePlan p = int8wo_gemm_plan(M, N, K, 8);
     if (p.parts > 1 && (!workspace || workspace_bytes < p.parts * M * N * (int64_t)sizeof(float))) p = int8wo_gemm_plan(M, N, K, 1);
-    launch_int8wo_gemm(TileGemmArgs{(const uint16_t*)x_bf16, M, K, ldx, (const uint8_t*)w_int8, ldw, (const uint16_t*)scale_bf16,
+    launch_int8wo_gemm(TileGemmArgs{(const uint16_t*)x_bf16, M, K, ldx, (const uint8_t*)w_int8, ldw, scale_bf16,
                                     (const uint16_t*)bias_bf16, N, (uint16_t*)y, ldy, 0, 0, 0, (const uint16_t*)residual, ldres,
-                                    (const uint16_t*)gate, ldgate, workspace},
+                                    (const uint16_t*)gate, ldgate, 0, workspace},
                        p, (hipStream_t)stream);
     AO_LAUNCH_CHECK();
     return 0;
@@ -602,7 +614,7 @@ extern "C" int ao_amd_int8wo_linear_ws_bytes(int64_t M, int64_t K, int64_t N, in
     AO_REQUIRE(bytes, "null pointer argument");
     AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
     *bytes = 0;
-    if (M > 0 && K % 64 == 0 && tiled(M, N, K)) {
+    if (M > 0 && K % 64 == 0 && tiled(M, N, K, true)) {
         const TilePlan p = int8wo_gemm_plan(M, N, K, 8);
         if (p.parts > 1) *bytes = p.parts * M * N * (int64_t)sizeof(float);
     }
@@ -611,7 +623,7 @@ extern "C" int ao_amd_int8wo_linear_ws_bytes(int64_t M, int64_t K, int64_t N, in
 
 extern "C" int ao_amd_int8wo_linear_plan(int64_t M, int64_t K, int64_t N, char* out, int64_t out_cap) {
     AO_REQUIRE(out && out_cap > 0 && M > 0 && N > 0 && K > 0 && K % 64 == 0, "need positive M and N, K a multiple of 64, and a buffer");
-    if (!tiled(M, N, K)) {
+    if (!tiled(M, N, K, true)) {
         snprintf(out, (size_t)out_cap, "streaming");
         return 0;
     }
@@ -623,7 +635,7 @@ extern "C" int ao_amd_int8wo_linear_ws(const void* x_bf16, int64_t M, int64_t K,
                                        const void* scale_bf16, int64_t N, const void* bias_bf16, void* y, int y_dtype, int64_t ldy,
                                        void* workspace, int64_t workspace_bytes, void* stream) {
     AO_REQUIRE(!workspace || (((uintptr_t)workspace) & 15) == 0, "the workspace must be 16-byte aligned");
-    if (y_dtype == AO_BF16 && K % 64 == 0 && tiled(M, N, K))
+    if (y_dtype == AO_BF16 && K % 64 == 0 && tiled(M, N, K, workspace != nullptr))
         return int8wo_tiled(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, ldy, nullptr, 0, nullptr, 0, (float*)workspace, workspace_bytes, stream);
     return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, y_dtype, ldy, nullptr, 0, nullptr, 0, stream);
 }
@@ -639,7 +651,7 @@ extern "C" int ao_amd_int8wo_linear_residual(const void* x_bf16, int64_t M, int6
                                              int64_t ldw, const void* scale_bf16, int64_t N, const void* residual_bf16,
                                              int64_t ldres, void* y_bf16, int64_t ldy, void* stream) {
     AO_REQUIRE(residual_bf16, "null pointer argument");
-    if (K % 128 == 0 && tiled(M, N, K))
+    if (K % 128 == 0 && tiled(M, N, K, false))
         return int8wo_tiled(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, ldy, residual_bf16, ldres, nullptr, 0, nullptr, 0,
                             stream);
     return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, AO_BF16, ldy, residual_bf16, ldres,
@@ -650,7 +662,7 @@ extern "C" int ao_amd_int8wo_linear_gated(const void* x_bf16, int64_t M, int64_t
                                           int64_t ldw, const void* scale_bf16, int64_t N, const void* gate_bf16,
                                           int64_t ldgate, void* y_bf16, int64_t ldy, void* stream) {
     AO_REQUIRE(gate_bf16, "null pointer argument");
-    if (K % 128 == 0 && tiled(M, N, K))
+    if (K % 128 == 0 && tiled(M, N, K, false))
         return int8wo_tiled(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, ldy, nullptr, 0, gate_bf16, ldgate, nullptr, 0,
                             stream);
     return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, AO_BF16, ldy, nullptr, 0, gate_bf16,

@@ -24,14 +24,15 @@ typedef float tg_f32x16 __attribute__((ext_vector_type(16)));
 
 struct TileGemmArgs {
     const uint16_t* x; int64_t M, K, ldx;
-    const uint8_t* w; int64_t ldw;      // weight and its row (or row-block) stride in bytes
-    const uint16_t* scale;
+    const uint8_t* w; int64_t ldw;      // weight and its row (or 16-row block) stride in bytes
+    const void* scale;                  // bf16 / fp16 row scales, or the int4 (scale, zero) words
     const uint16_t* bias;               // or null
     int64_t N;
     uint16_t* y; int64_t ldy;
     int tiles_n, tiles, per_xcd;
     const uint16_t* residual; int64_t ldres;   // y += residual, or null
     const uint16_t* gate; int64_t ldgate;      // y = silu(gate) * y, or null
+    int group_shift;                    // int4: log2 of the group size
     float* parts;                       // K split over blockIdx.y: fp32 partial products [gridDim.y][M][N], or null
 };
 
@@ -45,12 +46,26 @@ __device__ __forceinline__ void tg_wait_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// 4 bytes per lane
+__device__ __forceinline__ void tg_dma4(uint32_t lds, const void* base, uint32_t off) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+}
+
+// A weight format F describes a block of 32 weight rows of one 64-wide K step:
+//   REQ, BLOCK_BYTES      requests that bring it into LDS, and its bytes there
+//   lane_offset(a, n0, n, r, lane)   this lane's offset of request r from the tile's base, rows n ..
+//   request(a, n0, s, r, lds, off)   issues request r of step s for a block at `lds`
+//   Raw read(block, lane)            a lane's share: row lane % 32, the 32 k of half lane / 32
+//   Ready prepare(raw, row)          whatever is computed once per step
+//   uint32_t piece(ready, s, d)      two dequantized weights: dword d of the 8 k of slice s
+//   mul, columns, finish, combine    the matrix instruction and the epilogue
 template <class F, int WN, int KW, int MT, int NT>
 __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmArgs a) {
-    constexpr int STAGES = 4, G = WN, BM = 32 * MT, BN = 32 * NT * WN;
-    constexpr int ABYTES = BM * 128, BBYTES = BN * F::STEP_BYTES, STAGE = ABYTES + BBYTES;
-    constexpr int AREQ = ABYTES / 1024 / G, BREQ = BBYTES / 1024 / G, REQ = AREQ + BREQ;
-    static_assert(AREQ * G * 1024 == ABYTES && BREQ * G * 1024 == BBYTES, "every wave issues the same number of requests");
+    constexpr int G = WN, BM = 32 * MT, BN = 32 * NT * WN;
+    constexpr int ABYTES = BM * 128, STAGE = ABYTES + WN * NT * F::BLOCK_BYTES;
+    constexpr int STAGES = KW * 4 * STAGE <= 160 * 1024 ? 4 : 3;
+    constexpr int AREQ = ABYTES / 1024 / G, BREQ = NT * F::REQ, REQ = AREQ + BREQ;
+    static_assert(AREQ * G * 1024 == ABYTES, "every wave issues the same number of requests");
     constexpr int ACC = MT * NT * 4096;   // bytes of one wave's accumulators
     constexpr int LDS = KW * STAGES * STAGE > (KW - 1) * G * ACC ? KW * STAGES * STAGE : (KW - 1) * G * ACC;
     __shared__ __align__(1024) uint8_t lds[LDS];
@@ -76,9 +91,8 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
         aoff[j] = (uint32_t)(rel * a.ldx * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
     }
 #pragma unroll
-    for (int j = 0; j < BREQ; ++j) boff[j] = F::request_offset(a, n0, gw * BREQ + j, lane);
+    for (int j = 0; j < BREQ; ++j) boff[j] = F::lane_offset(a, n0, n0 + (gw * NT + j / F::REQ) * 32, j % F::REQ, lane);
     const uint16_t* const abase = a.x + m0 * a.ldx;
-    const uint8_t* const bbase = F::tile_base(a, n0);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + group * STAGES * STAGE;
     auto request = [&](int r, int t, int buf) __attribute__((always_inline)) {
         int s = t * KW + group;
@@ -87,7 +101,7 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
         if (r < AREQ)
             tg_dma(at + (gw * AREQ + r) * 1024, abase + (int64_t)s * 64, aoff[r]);
         else
-            tg_dma(at + ABYTES + (gw * BREQ + r - AREQ) * 1024, F::step_base(a, bbase, s), boff[r - AREQ]);
+            F::request(a, n0, s, (r - AREQ) % F::REQ, at + ABYTES + (gw * NT + (r - AREQ) / F::REQ) * F::BLOCK_BYTES, boff[r - AREQ]);
     };
 
     tg_f32x16 acc[MT][NT];
@@ -113,22 +127,23 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
 #pragma unroll
         for (int r = 0; r < REQ; ++r) request(r, t, t);
     auto a_at = [&](int buf) { return lds + (group * STAGES + buf) * STAGE; };
-    auto b_at = [&](int buf) { return lds + (group * STAGES + buf) * STAGE + ABYTES; };
+    auto b_at = [&](int buf, int j) { return lds + (group * STAGES + buf) * STAGE + ABYTES + (gw * NT + j) * F::BLOCK_BYTES; };
     auto read_a = [&](const uint8_t* A, int i, int s) __attribute__((always_inline)) {
         return *(const uint4*)(A + (i * 32 + r32) * 128 + (((4 * half + s) ^ ((r32 >> 1) & 7)) << 4));
     };
     union Frag { uint32_t u[4]; uint4 q; };
     Frag fa[2][MT], fb[2][NT];
-    typename F::Raw raw[NT], raw_next[NT];
+    typename F::Raw raw[NT];
+    typename F::Ready ready[NT];
     tg_wait_barrier<(STAGES - 3) * REQ>();
 #pragma unroll
-    for (int j = 0; j < NT; ++j) raw[j] = F::read(b_at(0), (gw * NT + j) * 32 + r32, half);
+    for (int j = 0; j < NT; ++j) ready[j] = F::prepare(F::read(b_at(0, j), lane), row_const[j]);
 #pragma unroll
     for (int i = 0; i < MT; ++i) fa[0][i].q = read_a(a_at(0), i, 0);
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int d = 0; d < 4; ++d) fb[0][j].u[d] = F::piece(raw[j], 0, d, row_const[j]);
+        for (int d = 0; d < 4; ++d) fb[0][j].u[d] = F::piece(ready[j], 0, d);
     int buf = 0;
     for (int t = 0; t < nst; ++t) {
         const int next = buf + 1 == STAGES ? 0 : buf + 1, ahead = buf == 0 ? STAGES - 1 : buf - 1;
@@ -141,18 +156,19 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
                 const int i = q % MT, j = q / MT;
                 if (live) acc[i][j] = F::mul(fb[cur][j].q, fa[cur][i].q, acc[i][j]);
                 if (q < MT) fa[nxt][q].q = s < 3 ? read_a(a_at(buf), q, s + 1) : read_a(a_at(next), q, 0);
-                if (s == 2 && q < NT) raw_next[q] = F::read(b_at(next), (gw * NT + q) * 32 + r32, half);
+                if (s == 2 && q < NT) raw[q] = F::read(b_at(next, q), lane);
+                if (s == 3 && q == 0)   // slice 2 has made the last pieces of this step
+#pragma unroll
+                    for (int j2 = 0; j2 < NT; ++j2) ready[j2] = F::prepare(raw[j2], row_const[j2]);
 #pragma unroll
                 for (int p = q * PIECES / SLOTS; p < (q + 1) * PIECES / SLOTS; ++p)
-                    fb[nxt][p / 4].u[p % 4] = F::piece(s < 3 ? raw[p / 4] : raw_next[p / 4], (s + 1) & 3, p % 4, row_const[p / 4]);
+                    fb[nxt][p / 4].u[p % 4] = F::piece(ready[p / 4], (s + 1) & 3, p % 4);
                 if (s < 2)
 #pragma unroll
                     for (int r = (s * SLOTS + q) * REQ / (2 * SLOTS); r < (s * SLOTS + q + 1) * REQ / (2 * SLOTS); ++r) request(r, t + STAGES - 1, ahead);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-#pragma unroll
-        for (int j = 0; j < NT; ++j) raw[j] = raw_next[j];
         tg_wait_barrier<(STAGES - 3) * REQ>();
         buf = next;
     }

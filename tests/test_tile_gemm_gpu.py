@@ -60,3 +60,15 @@ def test_int8_tiles(case):
 @pytest.mark.parametrize("case", [(65, 5121, 6528), (257, 21000, 1024), (129, 1100, 4096)])
 def test_int8_tiles_bias_and_row_stride(case):
     _run(*case, bias=True, pad=72)
+
+
+@pytest.mark.parametrize("case,tiles", [
+    ((3, 4096, 14336), False), ((5, 4090, 14336), False), ((6, 2064, 11008), False), ((2, 4096, 28672), False),  # rows staged in 65 to 140 KB
+    ((6, 4096, 14336), False),                                                                                # just past that
+    ((3, 2048, 16512), True), ((9, 4104, 8320), True), ((8, 4104, 8320), False), ((9, 24592, 8192), True),
+])
+def test_int8_few_rows(case, tiles):
+    assert (_plan(*case) != "streaming") == tiles
+    # the bound of _run holds here too: the sums are at most 3.5 times as long, and their order moves them by about
+    # sqrt(K) 2^-24 of their size, 1e-5 at most, against the 2^-8 steps of the result
+    _run(*case)
