@@ -1,0 +1,158 @@
+// FP6 weight-only linear on the tiled product of tile_gemm.h: native tiles (fp6.hip: 16 rows x 128 k in 1536 bytes) come into
+// LDS as they are, one conversion instruction per lane and 64-wide K step makes 32 fp16 values, and a packed fp16 multiply per
+// pair applies the row's scale with the one rounding of the reference kernel, fp16(fp6 * scale): 17 VALU instructions for 32
+// weights, so the tiles are bounded by what tile_gemm.h names, the bytes in flight and the LDS reads of the activations.  The
+// kernels of fp6.hip at these row counts move the activations through registers and convert the weight in every wave.
+#include "tile_gemm.h"
+
+namespace ao {
+
+typedef _Float16 ft_f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 ft_f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 ft_f16x32 __attribute__((ext_vector_type(32)));
+typedef uint32_t ft_u32x6 __attribute__((ext_vector_type(6)));
+
+template <bool E3M2>
+struct Fp6Tile {
+    static constexpr int REQ = 2, BLOCK_BYTES = 2048;   // 1 KB of first dwords, 512 bytes of last dwords and their repetition
+    struct Row { ft_f16x2 scale; };
+    struct Raw { uint4 lo; uint2 hi; };     // 32 codes of 6 bits
+    struct Ready { ft_f16x32 v; ft_f16x2 scale; };
+    struct Cols {};
+
+    static __device__ __forceinline__ uint32_t lane_offset(const TileGemmArgs& a, int64_t n0, int64_t n, int r, int lane) {
+        const int64_t nblocks = a.N / 16;
+        // first dwords: 32 lanes of 16 bytes a row block; last dwords: 16 lanes (8 bytes a weight row and k half)
+        int64_t nb = n / 16 + (r == 0 ? lane >> 5 : (lane >> 4) & 1);
+        if (nb >= nblocks) nb = nblocks - 1;   // a row block past N repeats the last one; its columns are not stored
+        return (uint32_t)((nb - n0 / 16) * a.ldw) + (r == 0 ? lane & 31 : lane & 15) * 16;
+    }
+    static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, uint32_t off) {
+        const uint8_t* const tile = a.w + (n0 / 16) * a.ldw + (int64_t)(s >> 1) * 1536;
+        tg_dma(lds + r * 1024, tile + (r == 0 ? (s & 1) * 512 : 1024 + (s & 1) * 256), off);
+    }
+    static __device__ __forceinline__ Row row(const TileGemmArgs& a, int64_t n) {
+        const _Float16 s = __builtin_bit_cast(_Float16, ((const uint16_t*)a.scale)[n < a.N ? n : a.N - 1]);
+        return Row{{s, s}};
+    }
+    static __device__ __forceinline__ Raw read(const uint8_t* block, int lane) {
+        const int slot = ((lane & 16) << 1) + (lane >> 5) * 16 + (lane & 15);   // row lane % 32, half lane / 32
+        return Raw{*(const uint4*)(block + slot * 16), *(const uint2*)(block + 1024 + slot * 8)};
+    }
+    static __device__ __forceinline__ Ready prepare(const Raw& r, const Row& row) {
+        const ft_u32x6 p = {r.lo.x, r.lo.y, r.lo.z, r.lo.w, r.hi.x, r.hi.y};
+        Ready out;
+        out.v = E3M2 ? __builtin_amdgcn_cvt_scalef32_pk32_f16_bf6(p, 1.0f) : __builtin_amdgcn_cvt_scalef32_pk32_f16_fp6(p, 1.0f);
+        out.scale = row.scale;
+        return out;
+    }
+    static __device__ __forceinline__ uint32_t piece(const Ready& r, int s, int d) {
+        const ft_f16x2 v = {r.v[8 * s + 2 * d], r.v[8 * s + 2 * d + 1]};
+        return __builtin_bit_cast(uint32_t, v * r.scale);
+    }
+    static __device__ __forceinline__ tg_f32x16 mul(uint4 w, uint4 x, tg_f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(ft_f16x8, w), __builtin_bit_cast(ft_f16x8, x), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ Cols columns(const TileGemmArgs&, int64_t) { return Cols(); }
+    static __device__ __forceinline__ uint16_t finish(float acc, const Cols&, int) { return f32_to_f16_bits(acc); }
+    static __device__ __forceinline__ void combine(const TileGemmArgs&, int64_t, int64_t, uint16_t (&)[4]) {}
+};
+
+// us at K = 4096, 192 to 256 workgroups (14336, 6144 and 4096 columns)
+static const TileShape kFp6Shapes[] = {
+    {64, 64, 19.0, 0.0},     // four groups along K
+    {64, 128, 24.6, 0.0},    // two groups
+    {96, 128, 30.5, 0.0},    // two groups
+    {128, 128, 40.8, 0.0},   // two groups
+    {192, 128, 49.8, 0.0},
+    {128, 256, 62.0, 0.0},   // 128 x 64 a wave
+    {192, 256, 90.0, 0.0},   // eight waves
+};
+
+template <bool E3M2>
+static void launch_shape(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
+    typedef Fp6Tile<E3M2> F;
+    tile_grid(a, kFp6Shapes[p.shape], p.parts);
+    switch (p.shape) {
+        case 0: tile_launch<F, 2, 4, 2, 1>(a, p.parts, st); break;
+        case 1: tile_launch<F, 4, 2, 2, 1>(a, p.parts, st); break;
+        case 2: tile_launch<F, 4, 2, 3, 1>(a, p.parts, st); break;
+        case 3: tile_launch<F, 4, 2, 4, 1>(a, p.parts, st); break;
+        case 4: tile_launch<F, 4, 1, 6, 1>(a, p.parts, st); break;
+        case 5: tile_launch<F, 4, 1, 4, 2>(a, p.parts, st); break;
+        default: tile_launch<F, 8, 1, 6, 1>(a, p.parts, st); break;
+    }
+    tile_finish<F>(a, p.parts, st);
+}
+
+static TilePlan fp6_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
+    return tile_plan(kFp6Shapes, (int)(sizeof(kFp6Shapes) / sizeof(kFp6Shapes[0])), M, N, K, max_parts);
+}
+
+// Whether the tiled product is the faster one.  The kernels of fp6.hip cost, by measurement at 33 to 1000 rows on 16 weights from
+// 768 x 1024 to 28672 x 8192: 32 x 64 tiles 4 us and 8 us per round over the CUs and 4096 of K, 64 x 64 tiles 4 and 14, and
+// 128 x 128 tiles 50 for one round and 37 for each of several.  us, those /
+// tiled: 14336 x 4096 at 65 / 160 / 256 / 384 / 768 rows 30 / 24, 44 / 30, 56 / 40, 68 / 49, 114 / 88; 4096 x 14336 at 160 / 512 / 1000 rows
+// 57 / 35, 97 / 74, 169 / 120; 4096 x 4096 at 128 / 384 / 1000 rows 12.3 / 15.0, 27 / 21, 50 / 39; 5120 x 5120 at 96 / 384 rows 14.4 /
+// 18.0, 34 / 32; 1024 x 4096 at 512 / 640 rows 12.6 / 15.4, 17.8 / 16.8.  Up to 64 rows the streaming kernels and small tiles
+// hold on except on the largest weights (28672 x 8192 at 33 / 48 rows 56 / 44, 59 / 45), and where those split K over workgroups
+// (fp6.hip: fp6_ws_parts) they are kept.
+static bool fp6_tiled(int64_t M, int64_t N, int64_t K) {
+    if (K % 64 != 0 || N % 16 != 0 || M <= 32 || M * N >= ((int64_t)1 << 40) || 192 * K * 2 >= ((int64_t)1 << 32)) return false;
+    if (ao_amd_fp6_linear_ws_parts(M, K, N) != 1) return false;
+    const double tile_us = fp6_tile_plan(M, N, K, 8).us;
+    // streamed once per 16 rows there (14336 x 4032 at 33 / 128 / 1000 rows 22 / 50 / 305 us, tiled 20 / 24 / 119; 4096 x 4160 at 65 / 128 /
+    // 1000 rows 14 / 17 / 96, tiled 16 / 16 / 41)
+    if (K % 128 != 0) return tile_us < 5.0 + 8.5e-8 * (double)(N * K) * (double)((M + 15) / 16);
+    if (M <= 64) return N * K >= ((int64_t)1 << 27);
+    const int64_t big = (N + 127) / 128 * ((M + 127) / 128), mid = (N + 63) / 64 * ((M + 63) / 64), small = (N + 63) / 64 * ((M + 31) / 32);
+    const double k = (double)K / 4096.0;
+    const double us = big >= 256 ? k * (big > 256 ? 37.0 * (double)((big + 255) / 256) : 50.0)
+                      : mid >= 192 ? 4.0 + 14.0 * k * (double)((mid + 255) / 256)
+                                   : 4.0 + 8.0 * k * (double)((small + 255) / 256);
+    return tile_us < (big >= 256 ? 0.9 : 1.0) * us;
+}
+
+}  // namespace ao
+
+using namespace ao;
+
+extern "C" int ao_amd_fp6_linear_tiled_bytes(int64_t M, int64_t K, int64_t N, int64_t* bytes) {
+    AO_REQUIRE(bytes, "null pointer argument");
+    AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
+    *bytes = -1;
+    if (!fp6_tiled(M, N, K)) return 0;
+    const TilePlan p = fp6_tile_plan(M, N, K, 8);
+    *bytes = p.parts > 1 ? p.parts * M * N * (int64_t)sizeof(float) : 0;
+    return 0;
+}
+
+extern "C" int ao_amd_fp6_linear_tiled_plan(int64_t M, int64_t K, int64_t N, char* out, int64_t out_cap) {
+    AO_REQUIRE(out && out_cap > 0 && M > 0 && N > 0 && K > 0 && K % 64 == 0, "need positive M and N, K a multiple of 64, and a buffer");
+    const TilePlan p = fp6_tile_plan(M, N, K, 8);
+    snprintf(out, (size_t)out_cap, "tile %dx%d parts=%d", kFp6Shapes[p.shape].bm, kFp6Shapes[p.shape].bn, p.parts);
+    return 0;
+}
+
+extern "C" int ao_amd_fp6_linear_tiled(const void* x_f16, int64_t M, int64_t K, const void* weights_native, const void* scale_f16, int64_t N,
+                                       int ebits, int mbits, void* out_f16, void* workspace, int64_t workspace_bytes, void* stream) {
+    AO_REQUIRE(x_f16 && weights_native && scale_f16 && out_f16, "null pointer argument");
+    AO_REQUIRE((ebits == 3 && (mbits == 1 || mbits == 2)) || (ebits == 2 && (mbits == 2 || mbits == 3)),
+               "native tiles hold e3m2, e2m3, e2m2 and e3m1, got e%dm%d", ebits, mbits);   // 5-bit codes in their 6-bit form
+    AO_REQUIRE(K > 0 && K % 64 == 0, "Expected in_features to be a multiple of 64, but received %lld", (long long)K);
+    AO_REQUIRE(N > 0 && N % 16 == 0, "out_features must be a positive multiple of 16, got %lld", (long long)N);
+    AO_REQUIRE(M >= 0, "negative batch");
+    AO_REQUIRE((((uintptr_t)x_f16) & 15) == 0 && (((uintptr_t)weights_native) & 15) == 0 && (((uintptr_t)workspace) & 15) == 0,
+               "buffers must be 16-byte aligned");
+    // per-lane offsets within a tile are 32 bits wide
+    AO_REQUIRE(192 * K * 2 < ((int64_t)1 << 32) && M * N < ((int64_t)1 << 40), "operands too large");
+    if (M == 0) return 0;
+    TilePlan p = fp6_tile_plan(M, N, K, 8);
+    if (p.parts > 1 && (!workspace || workspace_bytes < p.parts * M * N * (int64_t)sizeof(float))) p = fp6_tile_plan(M, N, K, 1);
+    const TileGemmArgs a{(const uint16_t*)x_f16, M, K, K, (const uint8_t*)weights_native, round_up(K, 128) / 128 * 1536, scale_f16, nullptr, N,
+                         (uint16_t*)out_f16, N, 0, 0, 0, nullptr, 0, nullptr, 0, 0, (float*)workspace};
+    if (ebits == 3) launch_shape<true>(a, p, (hipStream_t)stream);
+    else launch_shape<false>(a, p, (hipStream_t)stream);
+    AO_LAUNCH_CHECK();
+    return 0;
+}

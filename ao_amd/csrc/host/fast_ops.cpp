@@ -29,11 +29,11 @@ PyObject* int4wo_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     return guarded([&]() -> PyObject* {
         Tensor y = empty_rows(x, N, at::kBFloat16), ws;
         int64_t need = 0;
+        hipStream_t st = stream_of(a.device);
         if (r.M >= 16 && r.M <= 256) {
             AO_CALL(ao_amd_int4wo_linear_ws_bytes(r.M, K, N, g, &need));
             if (need) ws = workspace(need, a.device);
         }
-        hipStream_t st = stream_of(a.device);
         if (need) {
             AO_CALL(ao_amd_int4wo_linear_ws(ptr(x), r.M, K, r.ld, ptr(packed), ptr(qparams), N, g, ptr(bias), y.data_ptr(), AO_BF16,
                                             N, ws.data_ptr(), need, st));
@@ -77,12 +77,20 @@ PyObject* fp6_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     AO_WANT(native.numel() == fp6_native_words(N, r.K));
     return guarded([&]() -> PyObject* {
         Tensor y = empty_rows(x, N, at::kHalf), ws;
-        int64_t need = 0;
+        int64_t need = -1;
+        hipStream_t st = stream_of(a.device);
+        if (r.M > 32) AO_CALL(ao_amd_fp6_linear_tiled_bytes(r.M, r.K, N, &need));
+        if (need >= 0) {
+            if (need) ws = workspace(need, a.device);
+            AO_CALL(ao_amd_fp6_linear_tiled(ptr(x), r.M, r.K, ptr(native), ptr(scale), N, (int)e, (int)m, y.data_ptr(),
+                                            need ? ws.data_ptr() : nullptr, need, st));
+            return THPVariable_Wrap(std::move(y));
+        }
+        need = 0;
         if (r.M >= 16 && r.M <= 256) {
             AO_CALL(ao_amd_fp6_linear_ws_bytes(r.M, r.K, N, &need));
             if (need) ws = workspace(need, a.device);
         }
-        hipStream_t st = stream_of(a.device);
         if (need) {
             AO_CALL(ao_amd_fp6_linear_ws(ptr(x), r.M, r.K, ptr(native), ptr(scale), N, (int)e, (int)m, y.data_ptr(), ws.data_ptr(), need, st));
         } else {

@@ -174,7 +174,15 @@ struct Pass {
             return true;
         }
         y = alloc(M, l.N);
-        int64_t need = 0;
+        int64_t need = -1;
+        if (m.kind == FP6 && M > 32) AO_TRY(ao_amd_fp6_linear_tiled_bytes(M, l.K, l.N, &need));
+        if (need >= 0) {
+            Tensor ws;
+            if (need) ws = workspace(need, device);
+            void* w = need ? ws.data_ptr() : nullptr;
+            return ao_amd_fp6_linear_tiled(ptr(x), M, l.K, ptr(l.codes), ptr(l.scales), l.N, m.ebits, m.mbits, y.data_ptr(), w, need, st) == 0;
+        }
+        need = 0;
         if (m.kind == INT8) {
             AO_TRY(ao_amd_int8wo_linear_ws_bytes(M, l.K, l.N, &need));
         } else if (M >= 16 && M <= 256) {

@@ -96,31 +96,16 @@ void int8wo_gemm_describe(const TilePlan& p, char* out, size_t cap) {
     snprintf(out, cap, "tile %dx%d parts=%d", kInt8Shapes[p.shape].bm, kInt8Shapes[p.shape].bn, p.parts);
 }
 
-template <int WN, int KW, int MT, int NT>
-static void launch(const TileGemmArgs& a, int parts, hipStream_t st) {
-    hipEvent_t ev0 = g_prof_start, ev1 = g_prof_stop;
-    g_prof_start = g_prof_stop = nullptr;
-    hipExtLaunchKernelGGL((tile_gemm_kernel<Int8Tile, WN, KW, MT, NT>), dim3((unsigned)(a.per_xcd * 8), (unsigned)parts), dim3(64 * WN * KW), 0,
-                          st, ev0, ev1, 0, a);
-}
-
 void launch_int8wo_gemm(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
-    const TileShape& s = kInt8Shapes[p.shape];
-    a.tiles_n = (int)((a.N + s.bn - 1) / s.bn);
-    a.tiles = a.tiles_n * (int)((a.M + s.bm - 1) / s.bm);
-    a.per_xcd = (a.tiles + 7) / 8;
-    if (p.parts == 1) a.parts = nullptr;
+    tile_grid(a, kInt8Shapes[p.shape], p.parts);
     switch (p.shape) {
-        case 0: launch<4, 2, 2, 1>(a, p.parts, st); break;
-        case 1: launch<4, 1, 3, 1>(a, p.parts, st); break;
-        case 2: launch<4, 1, 4, 1>(a, p.parts, st); break;
-        case 3: launch<4, 1, 6, 1>(a, p.parts, st); break;
-        default: launch<4, 1, 4, 2>(a, p.parts, st); break;
+        case 0: tile_launch<Int8Tile, 4, 2, 2, 1>(a, p.parts, st); break;
+        case 1: tile_launch<Int8Tile, 4, 1, 3, 1>(a, p.parts, st); break;
+        case 2: tile_launch<Int8Tile, 4, 1, 4, 1>(a, p.parts, st); break;
+        case 3: tile_launch<Int8Tile, 4, 1, 6, 1>(a, p.parts, st); break;
+        default: tile_launch<Int8Tile, 4, 1, 4, 2>(a, p.parts, st); break;
     }
-    if (p.parts > 1) {
-        const int64_t n = a.M * ((a.N + 3) / 4);
-        hipLaunchKernelGGL(tile_finish_kernel<Int8Tile>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, p.parts);
-    }
+    tile_finish<Int8Tile>(a, p.parts, st);
 }
 
 }  // namespace ao

@@ -300,4 +300,25 @@ inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64
     return best;
 }
 
+// The launches of a plan: tile_grid once, tile_launch with the shape's constants, tile_finish.
+inline void tile_grid(TileGemmArgs& a, const TileShape& s, int parts) {
+    a.tiles_n = (int)((a.N + s.bn - 1) / s.bn);
+    a.tiles = a.tiles_n * (int)((a.M + s.bm - 1) / s.bm);
+    a.per_xcd = (a.tiles + 7) / 8;
+    if (parts == 1) a.parts = nullptr;
+}
+template <class F, int WN, int KW, int MT, int NT>
+void tile_launch(const TileGemmArgs& a, int parts, hipStream_t st) {
+    hipEvent_t ev0 = g_prof_start, ev1 = g_prof_stop;
+    g_prof_start = g_prof_stop = nullptr;
+    hipExtLaunchKernelGGL((tile_gemm_kernel<F, WN, KW, MT, NT>), dim3((unsigned)(a.per_xcd * 8), (unsigned)parts), dim3(64 * WN * KW), 0, st,
+                          ev0, ev1, 0, a);
+}
+template <class F>
+void tile_finish(const TileGemmArgs& a, int parts, hipStream_t st) {
+    if (parts == 1) return;
+    const int64_t n = a.M * ((a.N + 3) / 4);
+    hipLaunchKernelGGL(tile_finish_kernel<F>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, parts);
+}
+
 }  // namespace ao

@@ -401,6 +401,14 @@ int ao_amd_fp6_linear_ws_bytes(int64_t M, int64_t K, int64_t N, int64_t* bytes);
 int ao_amd_fp6_linear_ws_parts(int64_t M, int64_t K, int64_t N);
 int ao_amd_fp6_linear_ws(const void* x_f16, int64_t M, int64_t K, const void* weights_native, const void* scale_f16, int64_t N,
                          int ebits, int mbits, void* out_f16, void* workspace, int64_t workspace_bytes, void* stream);
+/* The same product on LDS-staged tiles whose K may be split over workgroups, for batches beyond the streaming kernels: K a
+ * multiple of 64, N of 16.  ao_amd_fp6_linear_tiled_bytes gives the workspace for a shape, or -1 where ao_amd_fp6_linear (or
+ * ao_amd_fp6_linear_ws) is as fast; with less (or none) K is not split.  ao_amd_fp6_linear_tiled_plan writes
+ * "tile <rows>x<columns> parts=<K parts>". */
+int ao_amd_fp6_linear_tiled_bytes(int64_t M, int64_t K, int64_t N, int64_t* bytes);
+int ao_amd_fp6_linear_tiled_plan(int64_t M, int64_t K, int64_t N, char* out, int64_t out_cap);
+int ao_amd_fp6_linear_tiled(const void* x_f16, int64_t M, int64_t K, const void* weights_native, const void* scale_f16, int64_t N,
+                            int ebits, int mbits, void* out_f16, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Which kernel instantiation the FPx linear entry points run for a problem, without launching anything: writes a name
  * such as "fp6_gemm_kernel<1,1,4,4,4>" (e3m2 flag, then the tile variant) or "fp6_gemv_kernel<8,1,0>" to `out`.  The

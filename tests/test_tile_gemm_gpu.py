@@ -72,3 +72,72 @@ def test_int8_few_rows(case, tiles):
     # the bound of _run holds here too: the sums are at most 3.5 times as long, and their order moves them by about
     # sqrt(K) 2^-24 of their size, 1e-5 at most, against the 2^-8 steps of the result
     _run(*case)
+
+
+def _tiled_plan(fmt, M, N, K):
+    from ao_amd import _lib
+
+    out = ctypes.create_string_buffer(64)
+    _lib.check(getattr(_lib.lib(), f"ao_amd_{fmt}_linear_tiled_plan")(M, K, N, out, 64))
+    return out.value.decode()
+
+
+def _tiled_bytes(fmt, M, N, K, *group):
+    from ao_amd import _lib
+
+    need = ctypes.c_int64(0)
+    _lib.check(getattr(_lib.lib(), f"ao_amd_{fmt}_linear_tiled_bytes")(M, K, N, *group, ctypes.byref(need)))
+    return need.value
+
+
+# (M, N, K): every tile shape of the FP6 table, with and without K parts, K a multiple of 64 but not of 128, one K step
+FP6_TILES = [
+    (1, 64, 64), (33, 4160, 4096), (65, 1088, 192), (65, 14336, 1024), (96, 4096, 8192), (97, 14400, 512), (129, 14336, 1024), (200, 14336, 1024),
+    (257, 14336, 1024), (192, 24640, 512), (512, 14336, 512), (640, 14400, 512), (769, 4096, 2112), (1000, 4096, 3072), (100, 8192, 8192),
+]
+
+
+def _fp6_tiles(M, N, K, ebits, mbits):
+    from ao_amd import _lib, ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w = (torch.randn(N, K, device="cuda", generator=g) * 0.05).half()
+    tc, scale = ops.fp6_quantize_pack(w, ebits, mbits)
+    native = ops.fp6_repack(tc, 1 + ebits + mbits)
+    x = torch.randn(M, K, device="cuda", generator=g).half()
+    wd = ops.fp6_dequantize(tc, scale, ebits, mbits).half()    # the kernels multiply fp16(value * scale)
+    want = (x.float() @ wd.float().t()).half()
+    ws = torch.empty(8 * M * N, device="cuda")
+    for size in (ws.numel() * 4, 0):                           # with the plan's K parts, and without room for them
+        y = torch.full((M, N), float("nan"), device="cuda").half()
+        _lib.check(_lib.lib().ao_amd_fp6_linear_tiled(x.data_ptr(), M, K, native.data_ptr(), scale.data_ptr(), N, ebits, mbits, y.data_ptr(),
+                                                      ws.data_ptr() if size else None, size, torch.cuda.current_stream().cuda_stream))
+        # the products are exact in fp32 and sums of K <= 8192 of them differ by their order in about 1e-6 relative, which moves
+        # a rounding of the result (relative step 2^-11) now and then
+        rel = ((y.float() - want.float()).norm() / want.float().norm()).item()
+        assert rel <= 1e-4, (M, N, K, rel)
+    return x, native, scale, y
+
+
+@pytest.mark.parametrize("case", FP6_TILES)
+def test_fp6_tiles(case):
+    _fp6_tiles(*case, 3, 2)
+
+
+@pytest.mark.parametrize("ebits,mbits", [(2, 3), (2, 2), (3, 1)])
+def test_fp6_tiles_other_formats(ebits, mbits):
+    _fp6_tiles(129, 4160, 1088, ebits, mbits)
+
+
+def test_fp6_tiles_cover_every_shape_and_the_operator_takes_them():
+    from ao_amd import ops
+
+    plans = {c: _tiled_plan("fp6", *c) for c in FP6_TILES}
+    assert {p.split()[1] for p in plans.values()} == {"64x64", "64x128", "96x128", "128x128", "192x128", "128x256", "192x256"}, plans
+    assert any(p.endswith("parts=1") for p in plans.values()) and any(not p.endswith("parts=1") for p in plans.values())
+    assert _tiled_bytes("fp6", 64, 14336, 4096) == -1 and _tiled_bytes("fp6", 65, 14336, 4096) >= 0 and _tiled_bytes("fp6", 65, 1024, 4096) == -1
+    assert _tiled_bytes("fp6", 33, 28672, 8192) >= 0 and _tiled_bytes("fp6", 512, 2112, 2112) == 0
+    for M, N, K in ((160, 4096, 8192), (129, 14336, 1024), (512, 2112, 2112)):
+        x, native, scale, _ = _fp6_tiles(M, N, K, 3, 2)
+        eager = ops.fp6_linear_native(3, 2, x, native, scale)
+        assert torch.equal(eager, torch.ops.torchao.fp6_linear_native.default(3, 2, x, native, scale))   # both host paths
