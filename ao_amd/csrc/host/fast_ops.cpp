@@ -28,8 +28,16 @@ PyObject* int4wo_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     AO_WANT(r.ok && r.K == K && int4_weight_ok(packed, qparams, N, K, g) && bias_ok(bias, N));
     return guarded([&]() -> PyObject* {
         Tensor y = empty_rows(x, N, at::kBFloat16), ws;
-        int64_t need = 0;
+        int64_t need = -1;
         hipStream_t st = stream_of(a.device);
+        if (r.M > 32 && r.ld % 8 == 0 && (uintptr_t)ptr(x) % 16 == 0) AO_CALL(ao_amd_int4wo_linear_tiled_bytes(r.M, K, N, g, &need));
+        if (need >= 0) {
+            if (need) ws = workspace(need, a.device);
+            AO_CALL(ao_amd_int4wo_linear_tiled(ptr(x), r.M, K, r.ld, ptr(packed), ptr(qparams), N, g, ptr(bias), y.data_ptr(), N,
+                                               need ? ws.data_ptr() : nullptr, need, st));
+            return THPVariable_Wrap(std::move(y));
+        }
+        need = 0;
         if (r.M >= 16 && r.M <= 256) {
             AO_CALL(ao_amd_int4wo_linear_ws_bytes(r.M, K, N, g, &need));
             if (need) ws = workspace(need, a.device);

@@ -175,11 +175,15 @@ struct Pass {
         }
         y = alloc(M, l.N);
         int64_t need = -1;
+        if (m.kind == INT4 && M > 32) AO_TRY(ao_amd_int4wo_linear_tiled_bytes(M, l.K, l.N, m.group, &need));
         if (m.kind == FP6 && M > 32) AO_TRY(ao_amd_fp6_linear_tiled_bytes(M, l.K, l.N, &need));
         if (need >= 0) {
             Tensor ws;
             if (need) ws = workspace(need, device);
             void* w = need ? ws.data_ptr() : nullptr;
+            if (m.kind == INT4)
+                return ao_amd_int4wo_linear_tiled(ptr(x), M, l.K, l.K, ptr(l.codes), ptr(l.scales), l.N, m.group, nullptr, y.data_ptr(), l.N, w,
+                                                  need, st) == 0;
             return ao_amd_fp6_linear_tiled(ptr(x), M, l.K, ptr(l.codes), ptr(l.scales), l.N, m.ebits, m.mbits, y.data_ptr(), w, need, st) == 0;
         }
         need = 0;

@@ -1,0 +1,178 @@
+// int4 weight-only linear between the streaming kernels and the prefill kernels, on the tiled product of tile_gemm.h:
+// y[M, N] = x[M, K] . dequant(W)[N, K]^T, torchao/dtypes/affine_quantized_tensor.py:600-640.  The packed codes of 32 weight
+// rows and one 64-wide K step are one request of 1 KB (two runs of 512 bytes), their (scale, zero) words a second one.
+//
+// What bounds it: the exact two-rounding dequantization, 34 VALU instructions per 8 weights, against MT matrix instructions
+// (MT = rows of the tile / 32).  Two waves per SIMD (two groups along K) overlap one wave's dequantization with the other's
+// matrix instructions: 96 x 128 tiles of 14336 x 4096 at 160 rows take 36 us, where the 128 x 64 tiles of int4wo_gemm.hip, one
+// wave per SIMD and a second round, take 45.
+#include "int4wo_linear.h"
+#include "tile_gemm.h"
+
+namespace ao {
+
+struct Int4Tile {
+    static constexpr int REQ = 2, BLOCK_BYTES = 1024 + 256;
+    struct Row {};
+    struct Raw { uint4 codes; uint32_t qp; };   // 32 consecutive k of one row, the scale and zero of their group
+    struct Ready { uint32_t w[4]; float s, c, s16, c16, z; };   // c = -1032 s, s16 = s / 16, c16 = -72 s
+    struct Cols { float bias[4]; };
+
+    // in_features as packed, a multiple of max(128, group); the K steps end at in_features, a multiple of 64
+    static __device__ __forceinline__ int64_t padded_k(const TileGemmArgs& a) { return a.ldw >> 3; }
+    // this lane's row within the block, its k half within the step: (lane % 16 + 16 * block half, lane / 16 % 2)
+    static __device__ __forceinline__ uint32_t lane_offset(const TileGemmArgs& a, int64_t n0, int64_t n, int r, int lane) {
+        const int64_t nblocks = (a.N + 15) / 16;
+        int64_t nb = n / 16 + (lane >> 5);
+        if (nb >= nblocks) nb = nblocks - 1;   // a row block past N repeats the last one; its columns are not stored
+        const int64_t rel = nb - n0 / 16;
+        const int half = (lane >> 4) & 1, row = lane & 15;
+        if (r == 0) return (uint32_t)(rel * a.ldw) + (half * 16 + row) * 16;
+        // one word per row and group: a 64-wide step has two groups of 32 or lies within one
+        return (uint32_t)(rel * (padded_k(a) >> a.group_shift) * 64) + (a.group_shift == 5 ? half * 64 : 0) + row * 4;
+    }
+    static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, uint32_t off) {
+        if (r == 0)
+            tg_dma(lds, a.w + (n0 / 16) * a.ldw + (int64_t)s * 512, off);
+        else
+            tg_dma4(lds + 1024, (const uint8_t*)a.scale + (n0 / 16) * (padded_k(a) >> a.group_shift) * 64 + (((int64_t)s * 64) >> a.group_shift) * 64, off);
+    }
+    static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) { return Row(); }
+    static __device__ __forceinline__ Raw read(const uint8_t* block, int lane) {
+        const int slot = ((lane & 16) << 1) + (lane >> 5) * 16 + (lane & 15);   // row lane % 32, half lane / 32
+        return Raw{*(const uint4*)(block + slot * 16), *(const uint32_t*)(block + 1024 + slot * 4)};
+    }
+    static __device__ __forceinline__ Ready prepare(const Raw& r, const Row&) {
+        const float s = __uint_as_float(r.qp << 16);
+        return Ready{{r.codes.x, r.codes.y, r.codes.z, r.codes.w}, s, -1032.0f * s, 0.0625f * s, -72.0f * s, __uint_as_float(r.qp & 0xffff0000u)};
+    }
+    // Codes 2 d and 2 d + 1 of dword s as dequantize_affine rounds them: t = bf16((q - 8) * scale), w = bf16(t + zero).  The
+    // pairs sit at bits (0, 16), (4, 20), (8, 24), (12, 28): masked and or'ed into the fp16 pair 1024 + q (1024 + 16 q for odd
+    // pairs, whose factor goes into the scale), widened and scaled by one mixed fma each, exact in fp32.
+    static __device__ __forceinline__ uint32_t piece(const Ready& r, int s, int d) {
+        const uint32_t w = d < 2 ? r.w[s] : r.w[s] >> 8;
+        const uint32_t p = (w & (d & 1 ? 0x00F000F0u : 0x000F000Fu)) | 0x64006400u;
+        const float sc = d & 1 ? r.s16 : r.s, c = d & 1 ? r.c16 : r.c;
+        float t0, t1;
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(t0) : "v"(p), "v"(sc), "v"(c));
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(t1) : "v"(p), "v"(sc), "v"(c));
+        // a zero low operand: the rounded value lands in the high half, where it is an fp32 again
+        asm("v_cvt_pk_bf16_f32 %0, 0, %0" : "+v"(t0));
+        asm("v_cvt_pk_bf16_f32 %0, 0, %0" : "+v"(t1));
+        return hw_bf16_pack(t0 + r.z, t1 + r.z);
+    }
+    static __device__ __forceinline__ tg_f32x16 mul(uint4 w, uint4 x, tg_f32x16 c) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ Cols columns(const TileGemmArgs& a, int64_t n) {
+        Cols c;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) c.bias[v] = a.bias ? bf16_bits_to_f32(a.bias[n + v < a.N ? n + v : a.N - 1]) : 0.f;
+        return c;
+    }
+    static __device__ __forceinline__ uint16_t finish(float acc, const Cols& c, int v) { return f32_to_bf16_bits(acc + c.bias[v]); }
+    static __device__ __forceinline__ void combine(const TileGemmArgs&, int64_t, int64_t, uint16_t (&)[4]) {}
+};
+
+// us at K = 4096, 192 to 256 workgroups (14336, 6144 and 4096 columns)
+static const TileShape kInt4Shapes[] = {
+    {64, 64, 19.4, 0.0},     // four groups along K
+    {64, 128, 31.0, 0.0},    // two groups
+    {96, 128, 36.4, 0.0},    // two groups
+    {128, 128, 41.8, 0.0},   // two groups
+    {192, 128, 57.0, 0.0},
+    {256, 128, 66.0, 0.0},
+};
+
+static TilePlan int4wo_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
+    return tile_plan(kInt4Shapes, (int)(sizeof(kInt4Shapes) / sizeof(kInt4Shapes[0])), M, N, K, max_parts);
+}
+
+// us of the kernel that ao_amd_int4wo_linear(_ws) runs, by measurement at 33 to 1000 rows on 16 weights from 768 x 1024 to 28672 x
+// 8192; 0 where it is not one of the tile kernels (few rows: the weight is streamed).
+static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
+    char name[96] = "";
+    if (ao_amd_int4wo_linear_plan(M, K, N, g, 1, 0, 0, 0, 0, 1, AO_BF16, name, sizeof(name)) != 0) return 0.0;
+    const double k = (double)K / 4096.0;
+    auto rounds = [&](int bm, int bn) { return (double)((M + bm - 1) / bm * ((N + bn - 1) / bn)) / 256.0; };
+    auto up = [](double r) { return (double)(int64_t)(r + 255.0 / 256.0); };
+    if (!strncmp(name, "int4wo_gemm_lds_kernel", 22)) {
+        const bool wide = strstr(name, ",2>") != nullptr;
+        if (wide) return 6.0 + 98.0 * k * up(rounds(256, 256));
+        const double r = rounds(256, 128), full = (double)(int64_t)r, rest = r - full;
+        return 14.0 + k * (52.5 * full + (rest == 0.0 ? 0.0 : full > 0.0 && rest <= 0.5 ? 28.0 : 52.5));
+    }
+    if (!strncmp(name, "int4wo_gemm_kwave_kernel", 24)) {
+        const double r = up(rounds(128, 64));
+        return 6.0 + (r > 1.0 ? 20.0 : 18.5) * k * r;
+    }
+    if (strncmp(name, "int4wo_gemm_", 12)) return 0.0;
+    if (ao_amd_int4wo_linear_ws_parts(M, K, N, g) > 1) return M <= 64 ? 0.0 : 4.0 + 8.0 * k;
+    if (strstr(name, ",2,8>")) return 90.0 * k * rounds(128, 128) / 2.0;
+    if (rounds(64, 64) >= 0.75) return 5.0 + (K >= 8192 ? 14.0 : 18.0) * k * up(rounds(64, 64));
+    return 4.0 + 10.4 * k * up(rounds(32, 64));
+}
+
+// Whether the tiled product is the faster one.  us, the others / tiled: 14336 x 4096 at 64 / 128 / 160 / 256 / 384 / 512 rows 23.8 / 21.3,
+// 24.4 / 31.3, 44.8 / 37.4, 46.9 / 42.5, 62.9 / 57.3, 63.8 / 67.2; 4096 x 14336 at 96 / 160 / 640 / 1000 rows 32.7 / 26.8, 53.9 / 39.5, 124 /
+// 108, 141 / 135; 4096 x 4096 at 128 / 256 / 512 / 768 rows 14.7 / 15.9, 23.5 / 19.6, 24.6 / 31.6, 44.1 / 37.6; 11008 x 4096 at 48 / 96 / 384
+// rows 26.2 / 18.5, 35.1 / 25.2, 66.1 / 56.5; 8192 x 28672 at 96 rows 114 / 74.  The estimates hold to some 10 %: a lead of 5 % is asked for.
+static bool int4wo_tiled(int64_t M, int64_t N, int64_t K, int64_t g) {
+    if (!valid_group(g) || K % 64 != 0 || M <= 32 || M * N >= ((int64_t)1 << 40)) return false;
+    // in_features that were padded to whole tiles of the packed layout: the others take activations copied to that width first
+    const int64_t Kp = round_up(K, g > 128 ? g : 128);
+    const double other = int4wo_other_us(M, N, Kp, g);
+    return other > 0.0 && int4wo_tile_plan(M, N, K, 8).us < (Kp == K ? 0.95 * other : other + 4.0);
+}
+
+}  // namespace ao
+
+using namespace ao;
+
+extern "C" int ao_amd_int4wo_linear_tiled_bytes(int64_t M, int64_t K, int64_t N, int64_t g, int64_t* bytes) {
+    AO_REQUIRE(bytes, "null pointer argument");
+    AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
+    *bytes = -1;
+    if (!int4wo_tiled(M, N, K, g)) return 0;
+    const TilePlan p = int4wo_tile_plan(M, N, K, 8);
+    *bytes = p.parts > 1 ? p.parts * M * N * (int64_t)sizeof(float) : 0;
+    return 0;
+}
+
+extern "C" int ao_amd_int4wo_linear_tiled_plan(int64_t M, int64_t K, int64_t N, char* out, int64_t out_cap) {
+    AO_REQUIRE(out && out_cap > 0 && M > 0 && N > 0 && K > 0 && K % 64 == 0, "need positive M and N, K a multiple of 64, and a buffer");
+    const TilePlan p = int4wo_tile_plan(M, N, K, 8);
+    snprintf(out, (size_t)out_cap, "tile %dx%d parts=%d", kInt4Shapes[p.shape].bm, kInt4Shapes[p.shape].bn, p.parts);
+    return 0;
+}
+
+extern "C" int ao_amd_int4wo_linear_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams,
+                                          int64_t N, int64_t g, const void* bias_bf16, void* y_bf16, int64_t ldy, void* workspace,
+                                          int64_t workspace_bytes, void* stream) {
+    AO_REQUIRE(x_bf16 && packed && qparams && y_bf16, "null pointer argument");
+    AO_REQUIRE(valid_group(g), "group size must be 32, 64, 128 or 256, got %lld", (long long)g);
+    AO_REQUIRE(M >= 0 && N > 0 && K > 0 && K % 64 == 0, "the tiled int4 product needs in_features to be a multiple of 64, got %lld", (long long)K);
+    if (M == 0) return 0;
+    AO_REQUIRE(ldx >= K && ldy >= N, "row strides (ldx=%lld, ldy=%lld) smaller than the rows", (long long)ldx, (long long)ldy);
+    AO_REQUIRE((((uintptr_t)x_bf16) & 15) == 0 && (ldx & 7) == 0 && (((uintptr_t)packed) & 15) == 0 && (((uintptr_t)workspace) & 15) == 0,
+               "activation rows, packed codes and workspace must be 16-byte aligned");
+    // per-lane offsets within a tile are 32 bits wide
+    AO_REQUIRE(256 * ldx * 2 < ((int64_t)1 << 32) && M * N < ((int64_t)1 << 40), "operands too large");
+    TilePlan p = int4wo_tile_plan(M, N, K, 8);
+    if (p.parts > 1 && (!workspace || workspace_bytes < p.parts * M * N * (int64_t)sizeof(float))) p = int4wo_tile_plan(M, N, K, 1);
+    TileGemmArgs a{(const uint16_t*)x_bf16, M, K, ldx, (const uint8_t*)packed, round_up(K, g > 128 ? g : 128) * 8, qparams, (const uint16_t*)bias_bf16, N,
+                   (uint16_t*)y_bf16, ldy, 0, 0, 0, nullptr, 0, nullptr, 0, g == 32 ? 5 : g == 64 ? 6 : g == 128 ? 7 : 8, (float*)workspace};
+    hipStream_t st = (hipStream_t)stream;
+    tile_grid(a, kInt4Shapes[p.shape], p.parts);
+    switch (p.shape) {
+        case 0: tile_launch<Int4Tile, 2, 4, 2, 1>(a, p.parts, st); break;
+        case 1: tile_launch<Int4Tile, 4, 2, 2, 1>(a, p.parts, st); break;
+        case 2: tile_launch<Int4Tile, 4, 2, 3, 1>(a, p.parts, st); break;
+        case 3: tile_launch<Int4Tile, 4, 2, 4, 1>(a, p.parts, st); break;
+        case 4: tile_launch<Int4Tile, 4, 1, 6, 1>(a, p.parts, st); break;
+        default: tile_launch<Int4Tile, 4, 1, 8, 1>(a, p.parts, st); break;
+    }
+    tile_finish<Int4Tile>(a, p.parts, st);
+    AO_LAUNCH_CHECK();
+    return 0;
+}

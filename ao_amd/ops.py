@@ -199,6 +199,16 @@ def _linear_cuda(x: Tensor, packed: Tensor, qparams: Tensor, group_size: int, N:
         # definition of the result: dequantize, then F.linear.
         return torch.nn.functional.linear(x, _dequantize_cuda(packed, qparams, N, K, group_size), bias)
     y = torch.empty((M, N), dtype=torch.float32 if fp32_out else torch.bfloat16, device=x.device)
+    if M > 32 and not fp32_out and x.stride(0) % 8 == 0 and x.stride(0) < 1 << 23 and x.data_ptr() % 16 == 0:
+        # batches between the streaming and the prefill kernels
+        need = ctypes.c_int64(-1)
+        check(lib().ao_amd_int4wo_linear_tiled_bytes(M, K, N, group_size, ctypes.byref(need)))
+        if need.value >= 0:
+            ws = torch.empty((need.value // 4,), dtype=torch.float32, device=x.device) if need.value else None
+            check(lib().ao_amd_int4wo_linear_tiled(x.data_ptr(), M, K, x.stride(0), packed.data_ptr(), qparams.data_ptr(), N, group_size,
+                                                   None if bias is None else bias.data_ptr(), y.data_ptr(), N,
+                                                   None if ws is None else ws.data_ptr(), need.value, current_stream(x.device)))
+            return y
     if 16 <= M <= 256:
         # the row counts at which the library may split K over workgroups through a workspace (narrow weights, long K)
         need = ctypes.c_int64(0)

@@ -156,6 +156,15 @@ int ao_amd_int4wo_linear_ws_parts(int64_t M, int64_t K, int64_t N, int64_t g);
 int ao_amd_int4wo_linear_ws(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams,
                             int64_t N, int64_t g, const void* bias_bf16, void* y, int y_dtype, int64_t ldy, void* workspace,
                             int64_t workspace_bytes, void* stream);
+/* The same product with bf16 output on LDS-staged tiles whose K may be split over workgroups, for batches between the streaming
+ * and the prefill kernels: K a multiple of 64, x and packed 16-byte aligned, ldx a multiple of 8.
+ * ao_amd_int4wo_linear_tiled_bytes gives the workspace for a shape, or -1 where ao_amd_int4wo_linear is as fast; with less (or
+ * none) K is not split.  ao_amd_int4wo_linear_tiled_plan writes "tile <rows>x<columns> parts=<K parts>". */
+int ao_amd_int4wo_linear_tiled_bytes(int64_t M, int64_t K, int64_t N, int64_t g, int64_t* bytes);
+int ao_amd_int4wo_linear_tiled_plan(int64_t M, int64_t K, int64_t N, char* out, int64_t out_cap);
+int ao_amd_int4wo_linear_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams,
+                               int64_t N, int64_t g, const void* bias_bf16, void* y_bf16, int64_t ldy, void* workspace,
+                               int64_t workspace_bytes, void* stream);
 
 /* Linear with the K range split over `ksplit` (1..8) groups of workgroups, for weights whose row-block count does not fill
  * the CUs evenly (Llama-3-8B wqkv: 384 row blocks on 256 CUs): y_f32_parts[z][M][ldy] = sum over the z-th run of K tiles

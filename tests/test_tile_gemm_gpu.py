@@ -141,3 +141,74 @@ def test_fp6_tiles_cover_every_shape_and_the_operator_takes_them():
         x, native, scale, _ = _fp6_tiles(M, N, K, 3, 2)
         eager = ops.fp6_linear_native(3, 2, x, native, scale)
         assert torch.equal(eager, torch.ops.torchao.fp6_linear_native.default(3, 2, x, native, scale))   # both host paths
+
+
+# (M, N, K, group): every tile shape of the int4 table, groups below, at and beyond a K step, widths with part of a row block,
+# in_features that the packed layout pads (to a multiple of 128 or of the group)
+INT4_TILES = [
+    (1, 20, 128, 32), (33, 4100, 4096, 64), (65, 1040, 256, 256), (65, 14330, 1024, 128), (96, 4096, 8192, 32), (97, 14336, 512, 64),
+    (129, 14336, 1024, 128), (200, 14337, 1024, 256), (257, 14336, 1024, 64), (512, 14336, 512, 32), (640, 4096, 14336, 64), (769, 4096, 2048, 128),
+    (1000, 4099, 2048, 64), (100, 8192, 4096, 256), (34, 1030, 64, 128), (70, 4096, 4032, 256), (130, 4099, 1088, 64), (40, 2048, 8256, 32),
+]
+
+
+def _int4_tiles(M, N, K, group, bias=False, pad=0):
+    from ao_amd import _lib, ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    packed, qp = ops.int4wo_quantize_pack((torch.randn(N, K, device="cuda", generator=g) * 0.02).bfloat16(), group)
+    dq = ops.int4wo_dequantize(packed, qp, N, K, group)
+    x = torch.randn(M, K + pad, device="cuda", generator=g).bfloat16()[:, :K]
+    b = torch.randn(N, device="cuda", generator=g).bfloat16() if bias else None
+    want = x.float() @ dq.float().t()
+    want = (want + b.float() if bias else want).bfloat16()
+    ws = torch.empty(8 * M * N, device="cuda")
+    for size in (ws.numel() * 4, 0):
+        y = torch.full((M, N), float("nan"), device="cuda").bfloat16()
+        _lib.check(_lib.lib().ao_amd_int4wo_linear_tiled(x.data_ptr(), M, K, x.stride(0), packed.data_ptr(), qp.data_ptr(), N, group,
+                                                         b.data_ptr() if bias else None, y.data_ptr(), N, ws.data_ptr() if size else None, size,
+                                                         torch.cuda.current_stream().cuda_stream))
+        # as above; the result's step is 2^-8
+        rel = ((y.float() - want.float()).norm() / want.float().norm()).item()
+        assert rel <= 1e-3 and (y != want).float().mean() <= 0.01, (M, N, K, rel)
+    return x, packed, qp, b
+
+
+@pytest.mark.parametrize("case", INT4_TILES)
+def test_int4_tiles(case):
+    _int4_tiles(*case)
+
+
+@pytest.mark.parametrize("case", [(97, 4099, 1024, 64), (129, 4100, 8192, 32)])
+def test_int4_tiles_bias_and_row_stride(case):
+    _int4_tiles(*case, bias=True, pad=72)
+
+
+def test_int4_tiles_read_the_weight_bit_for_bit():
+    """One-hot rows return columns of the dequantized weight."""
+    from ao_amd import _lib, ops
+
+    M, N, K, group = 200, 1030, 1024, 32
+    packed, qp = ops.int4wo_quantize_pack((torch.randn(N, K, device="cuda") * 0.02).bfloat16(), group)
+    at = torch.arange(M, device="cuda") * 5 + 3
+    x = torch.zeros(M, K, device="cuda").bfloat16()
+    x[torch.arange(M, device="cuda"), at] = 1.0
+    y = torch.empty(M, N, device="cuda").bfloat16()
+    _lib.check(_lib.lib().ao_amd_int4wo_linear_tiled(x.data_ptr(), M, K, K, packed.data_ptr(), qp.data_ptr(), N, group, None, y.data_ptr(), N, None,
+                                                     0, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(y, ops.int4wo_dequantize(packed, qp, N, K, group)[:, at].t())
+
+
+def test_int4_tiles_cover_every_shape_and_the_operator_takes_them():
+    from ao_amd import ops
+
+    plans = {c: _tiled_plan("int4wo", *c[:3]) for c in INT4_TILES}
+    assert {p.split()[1] for p in plans.values()} == {"64x64", "64x128", "96x128", "128x128", "192x128", "256x128"}, plans
+    assert any(p.endswith("parts=1") for p in plans.values()) and any(not p.endswith("parts=1") for p in plans.values())
+    for rows, taken in ((32, False), (48, False), (128, False), (160, True), (256, True), (384, True), (768, False)):
+        assert (_tiled_bytes("int4wo", rows, 14336, 4096, 64) >= 0) == taken, rows
+    for case in ((160, 14336, 1024, 64), (96, 4096, 14336, 128), (130, 4099, 1088, 64)):
+        for bias in (False, True):
+            x, packed, qp, b = _int4_tiles(*case, bias=bias, pad=8)
+            eager = ops.int4wo_linear(x, packed, qp, case[3], case[1], b)
+            assert torch.equal(eager, torch.ops.torchao.int4wo_linear.default(x, packed, qp, case[3], case[1], b, False))
