@@ -38,15 +38,19 @@ PyObject* int4wo_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
             return THPVariable_Wrap(std::move(y));
         }
         need = 0;
+        const void* rows = ptr(x);
+        int64_t k = K, ld = r.ld;
+        Tensor copy;
+        AO_WANT(pad_int4_rows(rows, r.M, k, ld, N, g, copy, a.device, st));
         if (r.M >= 16 && r.M <= 256) {
-            AO_CALL(ao_amd_int4wo_linear_ws_bytes(r.M, K, N, g, &need));
+            AO_CALL(ao_amd_int4wo_linear_ws_bytes(r.M, k, N, g, &need));
             if (need) ws = workspace(need, a.device);
         }
         if (need) {
-            AO_CALL(ao_amd_int4wo_linear_ws(ptr(x), r.M, K, r.ld, ptr(packed), ptr(qparams), N, g, ptr(bias), y.data_ptr(), AO_BF16,
+            AO_CALL(ao_amd_int4wo_linear_ws(rows, r.M, k, ld, ptr(packed), ptr(qparams), N, g, ptr(bias), y.data_ptr(), AO_BF16,
                                             N, ws.data_ptr(), need, st));
         } else {
-            AO_CALL(ao_amd_int4wo_linear(ptr(x), r.M, K, r.ld, ptr(packed), ptr(qparams), N, g, ptr(bias), y.data_ptr(), AO_BF16, N, st));
+            AO_CALL(ao_amd_int4wo_linear(rows, r.M, k, ld, ptr(packed), ptr(qparams), N, g, ptr(bias), y.data_ptr(), AO_BF16, N, st));
         }
         return THPVariable_Wrap(std::move(y));
     });

@@ -125,6 +125,27 @@ static bool int4wo_tiled(int64_t M, int64_t N, int64_t K, int64_t g) {
     return other > 0.0 && int4wo_tile_plan(M, N, K, 8).us < (Kp == K ? 0.95 * other : other + 4.0);
 }
 
+// x [M, K] with row stride ldx -> y [M, Kp], zeros beyond K, 8 elements a thread: activations whose rows are not 16-byte aligned
+// or end before the packed width.  The kernel that reads such rows as they are does it element by element, for every 16 weight
+// rows again; a copy is 2 to 3 us and the launch's gap.
+__global__ __launch_bounds__(256) void pad_rows_kernel(const uint16_t* __restrict__ x, int64_t M, int64_t K, int64_t ldx, int64_t Kp,
+                                                       bool vec, uint16_t* __restrict__ y) {
+    const int64_t per_row = Kp / 8, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t m = i / per_row, k = (i - m * per_row) * 8;
+    if (m >= M) return;
+    const uint16_t* src = x + m * ldx + k;
+    uint4 out;
+    if (vec && k + 8 <= K) {
+        out = *(const uint4*)src;
+    } else {
+        uint32_t v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = k + e < K ? src[e] : 0u;
+        out = make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
+    }
+    *(uint4*)(y + m * Kp + k) = out;
+}
+
 }  // namespace ao
 
 using namespace ao;
@@ -173,6 +194,19 @@ extern "C" int ao_amd_int4wo_linear_tiled(const void* x_bf16, int64_t M, int64_t
         default: tile_launch<Int4Tile, 4, 1, 8, 1>(a, p.parts, st); break;
     }
     tile_finish<Int4Tile>(a, p.parts, st);
+    AO_LAUNCH_CHECK();
+    return 0;
+}
+
+extern "C" int ao_amd_pad_rows(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t Kp, void* y, void* stream) {
+    AO_REQUIRE(x && y, "null pointer argument");
+    AO_REQUIRE(M >= 0 && K > 0 && ldx >= K && Kp >= K && Kp % 8 == 0, "need M >= 0, ldx >= K > 0 and Kp >= K a multiple of 8");
+    AO_REQUIRE((((uintptr_t)y) & 15) == 0, "output must be 16-byte aligned");
+    const int64_t blocks = (M * (Kp / 8) + 255) / 256;
+    AO_REQUIRE(blocks < ((int64_t)1 << 31), "operand too large");
+    if (M == 0) return 0;
+    const bool vec = (((uintptr_t)x) & 15) == 0 && (ldx & 7) == 0;
+    hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)x, M, K, ldx, Kp, vec, (uint16_t*)y);
     AO_LAUNCH_CHECK();
     return 0;
 }

@@ -209,6 +209,14 @@ def _linear_cuda(x: Tensor, packed: Tensor, qparams: Tensor, group_size: int, N:
                                                    None if bias is None else bias.data_ptr(), y.data_ptr(), N,
                                                    None if ws is None else ws.data_ptr(), need.value, current_stream(x.device)))
             return y
+    q = max(128, group_size)
+    Kp = (K + q - 1) // q * q
+    if (K != Kp or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0) \
+            and (N * K * (M + 4) >= 50000000 or K * (13 if M == 1 else min(M, 16) + 4) >= 18000):
+        # rows that the fast kernels cannot read, copied to the packed width (csrc/host/host.h: pad_int4_rows)
+        padded = torch.empty((M, Kp), dtype=x.dtype, device=x.device)
+        check(lib().ao_amd_pad_rows(x.data_ptr(), M, K, x.stride(0), Kp, padded.data_ptr(), current_stream(x.device)))
+        x, K = padded, Kp
     if 16 <= M <= 256:
         # the row counts at which the library may split K over workgroups through a workspace (narrow weights, long K)
         need = ctypes.c_int64(0)

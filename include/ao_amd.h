@@ -165,6 +165,8 @@ int ao_amd_int4wo_linear_tiled_plan(int64_t M, int64_t K, int64_t N, char* out, 
 int ao_amd_int4wo_linear_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams,
                                int64_t N, int64_t g, const void* bias_bf16, void* y_bf16, int64_t ldy, void* workspace,
                                int64_t workspace_bytes, void* stream);
+/* 16-bit rows x [M, K] (row stride ldx, any alignment) -> y [M, Kp] with zeros beyond K; Kp a multiple of 8, y 16-byte aligned. */
+int ao_amd_pad_rows(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t Kp, void* y, void* stream);
 
 /* Linear with the K range split over `ksplit` (1..8) groups of workgroups, for weights whose row-block count does not fill
  * the CUs evenly (Llama-3-8B wqkv: 384 row blocks on 256 CUs): y_f32_parts[z][M][ldy] = sum over the z-th run of K tiles

@@ -212,3 +212,26 @@ def test_int4_tiles_cover_every_shape_and_the_operator_takes_them():
             x, packed, qp, b = _int4_tiles(*case, bias=bias, pad=8)
             eager = ops.int4wo_linear(x, packed, qp, case[3], case[1], b)
             assert torch.equal(eager, torch.ops.torchao.int4wo_linear.default(x, packed, qp, case[3], case[1], b, False))
+
+
+@pytest.mark.parametrize("M,N,K,group,shift", [
+    (1, 14336, 4032, 64, 0), (1, 8192, 4100, 128, 0), (3, 4099, 4160, 32, 0), (16, 4096, 4041, 256, 0), (17, 4096, 4032, 256, 0), (33, 4100, 4160, 64, 0),
+    (300, 4096, 4100, 64, 0), (600, 14336, 1090, 128, 0),                    # rows that end before the packed width
+    (1, 14336, 4096, 64, 1), (9, 4096, 4096, 128, 3), (200, 4096, 4096, 64, 1),  # rows that are not 16-byte aligned
+    (2, 64, 192, 64, 0), (1, 1024, 704, 64, 1),                              # too small for the copy to pay
+])
+def test_int4_rows_that_are_copied_to_the_packed_width(M, N, K, group, shift):
+    from ao_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    packed, qp = ops.int4wo_quantize_pack((torch.randn(N, K, device="cuda", generator=g) * 0.02).bfloat16(), group)
+    dq = ops.int4wo_dequantize(packed, qp, N, K, group)
+    x = torch.randn(M, K + 2 * shift, device="cuda", generator=g).bfloat16()[:, shift:K + shift]
+    want = (x.float() @ dq.float().t()).bfloat16()
+    for y in (ops.int4wo_linear(x, packed, qp, group, N), torch.ops.torchao.int4wo_linear.default(x, packed, qp, group, N, None, False)):
+        rel = ((y.float() - want.float()).norm() / want.float().norm()).item()   # as for the tiles
+        assert rel <= 1e-3, (M, N, K, rel)
+    y32 = ops.int4wo_linear(x, packed, qp, group, N, fp32_out=True)
+    want = x.double() @ dq.double().t()
+    # sums of K <= 4160 exact products in fp32: sqrt(K) roundings of 2^-24 of the partial sum, about 4e-6, times the cancellation in it
+    assert ((y32.double() - want).norm() / want.norm()).item() <= 2e-5
