@@ -156,3 +156,22 @@ def test_row_stride_larger_than_k_through_the_c_abi(N, K, bK):
             got.append((s.view(torch.int16), z.view(torch.int16) if zdt == BF16 else z, q))
         for a, b in zip(*got):
             assert torch.equal(a, b), (name, N, K, bK)
+
+
+@pytest.mark.parametrize("N,K", [(1, 8), (3, 520), (17, 512), (5, 1032), (130, 4160), (64, 4096)])
+@pytest.mark.parametrize("zero_point", [None, 0, 3])
+def test_int8_rows_dequantize(N, K, zero_point):
+    """One scale per row in bf16, the int8 weight-only recipe: every code, scales that are infinite, NaN, subnormal and huge."""
+    from ao_amd.quantization.quant_primitives import dequantize_affine
+
+    g = torch.Generator().manual_seed(N + K)
+    q = torch.randint(-128, 128, (N, K), dtype=torch.int8, generator=g)
+    s = (torch.rand(N, generator=g) * 0.01 + 1e-3).bfloat16()
+    for i, v in enumerate((float("inf"), float("nan"), 1e-40, 3e38)):
+        if N > 16:
+            s[3 * i] = v
+    zp = None if zero_point is None else torch.full((N,), zero_point, dtype=torch.int64)
+    out = dequantize_affine(q.cuda(), (1, K), s.cuda(), None if zp is None else zp.cuda(), torch.int8, -128, 127, output_dtype=torch.bfloat16)
+    want = (q.int() - (zero_point or 0)).bfloat16() * s[:, None]
+    assert np.array_equal(bits16(out)[~want.isnan().numpy()], bits16(want)[~want.isnan().numpy()])
+    assert (bits16(out)[want.isnan().numpy()] == 0x7FC0).all()
