@@ -51,6 +51,7 @@ _SIGNATURES = {
     "ao_amd_fp6_repack": ([_p, _i64, _i64, _int, _p, _p], _int),
     "ao_amd_fp6_linear": ([_p, _i64, _i64, _p, _p, _i64, _int, _int, _p, _p], _int),
     "ao_amd_fp6_linear_ws_bytes": ([_i64, _i64, _i64, ctypes.POINTER(ctypes.c_int64)], _int),
+    "ao_amd_fp6_dequantize_to": ([_p, _p, _i64, _i64, _int, _int, _p, _int, _p], _int),
     "ao_amd_fp6_linear_tiled_bytes": ([_i64, _i64, _i64, _i64p], _int),
     "ao_amd_fp6_linear_tiled_plan": ([_i64, _i64, _i64, ctypes.c_char_p, _i64], _int),
     "ao_amd_fp6_linear_tiled": ([_p, _i64, _i64, _p, _p, _i64, _int, _int, _p, _p, _i64, _p], _int),

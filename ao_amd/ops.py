@@ -65,7 +65,7 @@ _LIB.define("llama_decode_attention(Tensor qkv, Tensor freqs_cis, Tensor input_p
 # schema of the reference op, verbatim (torchao/csrc/fp6_llm.cpp:7)
 _LIB.define("quant_llm_linear(int EXPONENT, int MANTISSA, Tensor _in_feats, Tensor _weights, Tensor _scales, int splitK) -> Tensor")
 _LIB.define("fp6_quantize_pack(Tensor w, int ebits, int mbits) -> (Tensor, Tensor)")
-_LIB.define("fp6_dequantize(Tensor fpx_data, Tensor? scale, int ebits, int mbits) -> Tensor")
+_LIB.define("fp6_dequantize(Tensor fpx_data, Tensor? scale, int ebits, int mbits, ScalarType? dtype=None) -> Tensor")
 _LIB.define("fp6_repack(Tensor fpx_data, int nbits=6) -> Tensor")
 _LIB.define("fp6_linear_native(int ebits, int mbits, Tensor x, Tensor native, Tensor scale) -> Tensor")
 _LIB.define("fp6_rmsnorm_linear(int ebits, int mbits, Tensor x, Tensor norm_weight, float eps, Tensor native, Tensor scale) -> Tensor")
@@ -689,7 +689,7 @@ def _fp6_quantize_pack_cuda(w, ebits, mbits):
     return data, scale
 
 
-def _fp6_dequantize_cuda(fpx_data, scale, ebits, mbits):
+def _fp6_dequantize_cuda(fpx_data, scale, ebits, mbits, dtype=None):
     require_cuda(fpx_data, scale)
     _check_fp6_format(ebits, mbits)
     torch._check(fpx_data.dim() == 2 and fpx_data.dtype is torch.uint8, lambda: "fpx_data must be a 2d uint8 tensor")
@@ -697,10 +697,14 @@ def _fp6_dequantize_cuda(fpx_data, scale, ebits, mbits):
     if scale is not None:
         torch._check(scale.dtype is torch.float16 and scale.numel() == N, lambda: "scale must be float16 of size N")
         scale = scale.contiguous()
-    out = torch.empty((N, K), dtype=torch.float32, device=fpx_data.device)
-    check(lib().ao_amd_fp6_dequantize(fpx_data.contiguous().data_ptr(), None if scale is None else scale.data_ptr(), N, K,
-                                      ebits, mbits, out.data_ptr(), current_stream(fpx_data.device)))
-    return out
+    fpx_data = fpx_data.contiguous()
+    # 16-bit outputs in one pass for 6-bit codes; any other type is converted from fp32
+    direct = dtype in (torch.float16, torch.bfloat16) and ebits + mbits == 5 and fpx_data.data_ptr() % 16 == 0
+    out = torch.empty((N, K), dtype=dtype if direct else torch.float32, device=fpx_data.device)
+    check(lib().ao_amd_fp6_dequantize_to(fpx_data.data_ptr(), None if scale is None else scale.data_ptr(), N, K, ebits, mbits,
+                                         out.data_ptr(), {torch.float16: F16, torch.bfloat16: BF16}[dtype] if direct else F32,
+                                         current_stream(fpx_data.device)))
+    return out if dtype is None else out.to(dtype)
 
 
 def _fp6_repack_cuda(fpx_data, nbits=6):
@@ -1031,8 +1035,8 @@ def _(w, ebits, mbits):
 
 
 @torch.library.register_fake("torchao::fp6_dequantize")
-def _(fpx_data, scale, ebits, mbits):
-    return fpx_data.new_empty((fpx_data.shape[0], fpx_data.shape[1] // (1 + ebits + mbits) * 8), dtype=torch.float32)
+def _(fpx_data, scale, ebits, mbits, dtype=None):
+    return fpx_data.new_empty((fpx_data.shape[0], fpx_data.shape[1] // (1 + ebits + mbits) * 8), dtype=dtype or torch.float32)
 
 
 @torch.library.register_fake("torchao::fp6_repack")
@@ -1082,9 +1086,9 @@ def fp6_quantize_pack(w: Tensor, ebits: int, mbits: int):
     return torch.ops.torchao.fp6_quantize_pack.default(w, ebits, mbits)
 
 
-def fp6_dequantize(fpx_data: Tensor, scale, ebits: int, mbits: int) -> Tensor:
-    """TC-FPx bytes (+ optional fp16 row scales) -> fp32 [N,K]."""
-    return torch.ops.torchao.fp6_dequantize.default(fpx_data, scale, ebits, mbits)
+def fp6_dequantize(fpx_data: Tensor, scale, ebits: int, mbits: int, dtype=None) -> Tensor:
+    """TC-FPx bytes (+ optional fp16 row scales) -> fp32 [N,K], or that rounded to `dtype`."""
+    return torch.ops.torchao.fp6_dequantize.default(fpx_data, scale, ebits, mbits, dtype)
 
 
 def fp6_repack(fpx_data: Tensor, nbits: int = 6) -> Tensor:

@@ -76,8 +76,8 @@ class QuantLlmLinearWeight(PackedWeightBase):
         return cls(*to_scaled_tc_fpx(input_float, ebits, mbits), ebits, mbits)
 
     def dequantize(self, output_dtype=None):
-        values = from_scaled_tc_fpx(self.fpx_data, self.ebits, self.mbits, self.scale)
-        return values.to(torch.get_default_dtype() if output_dtype is None else output_dtype)
+        dtype = torch.get_default_dtype() if output_dtype is None else output_dtype
+        return ops.fp6_dequantize(self.fpx_data, self.scale, self.ebits, self.mbits, dtype)
 
     def __repr__(self):
         return (f"{type(self).__name__}(dtype=fp{self.nbits}_e{self.ebits}m{self.mbits}, shape={tuple(self.shape)}, "

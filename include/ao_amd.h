@@ -382,6 +382,9 @@ int ao_amd_fp6_quantize_pack(const void* w, int w_dtype, int64_t N, int64_t K, i
  * out fp32 [N,K] = fpx_to_f32(unpack(tc)) * float(scale) (scale may be NULL). */
 int ao_amd_fp6_dequantize(const void* tc, const void* scale_f16, int64_t N, int64_t K, int ebits, int mbits,
                           float* out, void* stream);
+/* ... into out_dtype: AO_F32, or AO_F16 / AO_BF16 (rounded once) for 6-bit codes in 16-byte aligned buffers. */
+int ao_amd_fp6_dequantize_to(const void* tc, const void* scale_f16, int64_t N, int64_t K, int ebits, int mbits, void* out,
+                             int out_dtype, void* stream);
 
 /* One-time device repack of the TC-FPx bytes (nbits = 5 or 6) into the kernel's wave64 order (no counterpart in the
  * reference, whose kernel reads the TC bytes directly with 32-lane fragment loads).  A 5-bit code is stored as the

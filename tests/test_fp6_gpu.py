@@ -83,6 +83,28 @@ def test_quantize_pack_16_bit_rows_bit_exact_on_edge_cases(oracle, shape, fmt, d
     assert np.array_equal(data.cpu().numpy(), packed_ref)
 
 
+@pytest.mark.parametrize("N,K", [(64, 64), (128, 192), (192, 4160), (320, 1024)])
+@pytest.mark.parametrize("ebits,mbits", [(3, 2), (2, 3), (2, 2)])
+def test_dequantize_into_16_bits_is_the_fp32_value_rounded_once(oracle, N, K, ebits, mbits):
+    from ao_amd import ops
+
+    dev = _dev()
+    rng = np.random.default_rng(N + K)
+    nbits = 1 + ebits + mbits
+    tc = torch.from_numpy(rng.integers(0, 256, (N, K * nbits // 8), dtype=np.uint8)).to(dev)
+    scale = torch.from_numpy((rng.random(N) * 0.01 + 1e-3).astype(np.float16)).to(dev)
+    scale[:4] = torch.tensor([float("inf"), float("nan"), 0.0, 6e-8])
+    for s in (scale, None):
+        full = ops.fp6_dequantize(tc, s, ebits, mbits)
+        assert full.dtype is torch.float32
+        for dtype in (torch.float16, torch.bfloat16, torch.float32, torch.float64):
+            out = ops.fp6_dequantize(tc, s, ebits, mbits, dtype)
+            assert out.dtype is dtype and torch.equal(out.nan_to_num(nan=-777.0), full.to(dtype).nan_to_num(nan=-777.0))
+    if nbits == 6:   # the fp32 values themselves, per element from the codes
+        codes = oracle.unpack_tc_fp6(tc.cpu().numpy(), N, K)
+        assert np.array_equal(ops.fp6_dequantize(tc, None, ebits, mbits).cpu().numpy(), oracle.fpx_to_f32(codes, ebits, mbits))
+
+
 def test_dequantize_and_repack_round_trip(oracle):
     from ao_amd import ops
 
