@@ -86,6 +86,8 @@ static const TileShape kInt8Shapes[] = {
     {128, 128, 38.0, 0.0},
     {192, 128, 46.0, 0.0},
     {128, 256, 54.0, 0.0},   // 128 x 64 a wave
+    {64, 64, 20.0, 0.0},     // four groups along K
+    {192, 256, 90.0, 0.0},   // eight waves
 };
 
 TilePlan int8wo_gemm_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
@@ -103,7 +105,9 @@ void launch_int8wo_gemm(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
         case 1: tile_launch<Int8Tile, 4, 1, 3, 1>(a, p.parts, st); break;
         case 2: tile_launch<Int8Tile, 4, 1, 4, 1>(a, p.parts, st); break;
         case 3: tile_launch<Int8Tile, 4, 1, 6, 1>(a, p.parts, st); break;
-        default: tile_launch<Int8Tile, 4, 1, 4, 2>(a, p.parts, st); break;
+        case 4: tile_launch<Int8Tile, 4, 1, 4, 2>(a, p.parts, st); break;
+        case 5: tile_launch<Int8Tile, 2, 4, 2, 1>(a, p.parts, st); break;
+        default: tile_launch<Int8Tile, 8, 1, 6, 1>(a, p.parts, st); break;
     }
     tile_finish<Int8Tile>(a, p.parts, st);
 }

@@ -578,7 +578,14 @@ static bool tiled(int64_t M, int64_t N, int64_t K, bool workspace) {
     // tiles of K.
     const int64_t weight = N * K;
     if (K % 128 != 0) return M > 0;
-    if (weight < (32 << 20)) return M > (weight >= (12 << 20) ? 32 : weight >= (3 << 20) ? 128 : 768);
+    // With K parts over workgroups, 64 x 64 tiles serve the smaller weights earlier: 4096 x 4096 at 17 / 24 / 32 rows 11.9 / 13.3 / 14.4
+    // streaming, 12.4 / 12.7 / 12.9 tiled; 6144 x 4096 and 5120 x 5120 at 24 rows 19.0 / 14.5, 25.8 / 15.6; 1024 x 4096 at 64 / 128 rows
+    // 8.6 / 12.1, 13.9 / 12.7; 1001 x 2048 at 128 / 160 / 512 rows 9.6 / 13.5, 17.2 / 13.2, 27.8 / 13.8.
+    if (weight < (32 << 20)) {
+        if (weight >= (12 << 20)) return M > (!workspace ? 32 : weight >= (24 << 20) ? 16 : 20);
+        if (weight >= (3 << 20)) return M > (workspace && weight >= (4 << 20) && K >= 4096 ? 64 : 128);
+        return M > (weight >= 1500000 ? 128 : 768);
+    }
     // Long rows: every 16 or 64 rows of W read all of x again (8192 x 28672 at 3 / 8 / 16 rows 62 / 72 / 87 us streaming, 54 /
     // 54 / 57 tiled; 8192 x 8192 at 8 / 16 rows 23.5 / 26.6, 22.2 / 22.7; 28672 x 8192 at 12 / 16 rows 66 / 69, 61 / 62; but
     // 14336 x 8192 at 12 / 16 rows, one even pass of four-block workgroups, 35 / 37 and 37 / 38).

@@ -273,7 +273,7 @@ __global__ __launch_bounds__(256) void tile_finish_kernel(const TileGemmArgs a, 
 
 // Tile shape and K parts for M x N x K: the cheapest by a measured model.  A shape costs `one` us for a wave of workgroups
 // over 4096 of K with one workgroup on a CU and `two` with two (0: only one fits), 6 us of it whatever K is; K parts add a
-// second launch and 8 bytes of fp32 per output and part.
+// second launch, 1 us with each doubling and 8 bytes of fp32 per output and part.
 struct TileShape {
     int bm, bn;
     double one, two;
@@ -294,7 +294,7 @@ inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64
             auto us = [&](double t) { return 6.0 + (t - 6.0) * (double)per / 64.0; };
             const double wave = us(shapes[i].two > 0 ? shapes[i].two : shapes[i].one);
             double t = full * wave + (rest == 0 ? 0.0 : rest <= 256 ? us(shapes[i].one) : wave);
-            if (z > 1) t += 3.0 + 8e-6 * (double)(M * N * z) / 4.0;
+            if (z > 1) t += 1.5 + (z == 2 ? 1.0 : z == 4 ? 2.0 : 3.0) + 8e-6 * (double)(M * N * z) / 4.0;
             if (t < best.us) best = TilePlan{i, z, t};
         }
     return best;

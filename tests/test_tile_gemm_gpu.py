@@ -13,6 +13,7 @@ CASES = [
     (17, 4100, 8320), (33, 4096, 8192), (64, 3072, 4224), (65, 5121, 6528), (96, 8200, 4096), (97, 16400, 4096), (129, 1100, 4096),
     (191, 16400, 2048), (192, 24600, 2048), (193, 15000, 2176), (255, 14336, 1024), (256, 14336, 1024), (257, 21000, 1024), (384, 12416, 2048),
     (769, 130, 128), (770, 127, 256), (1000, 600, 1024), (1025, 14336, 512), (513, 28672, 640),
+    (70, 1028, 4096), (24, 4100, 4096), (160, 1001, 2048), (640, 14337, 512),
     (1, 300, 64), (5, 2000, 192), (40, 4096, 8256),  # in_features not a multiple of 128: any row count
 ]
 
@@ -48,7 +49,7 @@ def _run(M, N, K, bias=False, pad=0):
 def test_cases_cover_every_tile_shape():
     plans = {c: _plan(*c) for c in CASES}
     shapes = {p.split()[1] for p in plans.values() if p != "streaming"}
-    assert shapes == {"64x128", "96x128", "128x128", "192x128", "128x256"}, plans
+    assert shapes == {"64x64", "64x128", "96x128", "128x128", "192x128", "128x256", "192x256"}, plans
     assert any(p.endswith("parts=1") for p in plans.values()) and any(not p.endswith("parts=1") for p in plans.values())
 
 
