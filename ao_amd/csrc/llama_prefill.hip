@@ -12,6 +12,7 @@
 namespace ao {
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x4p_t __attribute__((ext_vector_type(4)));   // loads that wait in registers: a uint4 struct is kept in scratch
 
 // 32x32x16 product, 8 elements of a 16-bit type per lane and operand
 template <class E> struct Mfma32;
@@ -73,9 +74,10 @@ __global__ __launch_bounds__(256) void prefill_cache_kernel(const uint16_t* __re
 
 // Causal attention of T query rows over the cache, flash style.
 //
-// A workgroup of 4 waves walks the cache in tiles of 64 positions; a wave owns 32 query rows of one head.  HEADS: the four
-// waves are four query heads of one KV head (grouped-query models: one K / V tile serves four heads); otherwise they are
-// four consecutive 32-row blocks of one head.
+// Two groups of 4 waves walk the cache in tiles of 64 positions, one the even and one the odd tiles; a wave owns 32 query rows of
+// one head, the same ones in both groups, whose maxima, sums and accumulators meet at the end.  HEADS: the four waves are four
+// query heads of one KV head (grouped-query models: one K / V tile serves four heads); otherwise they are four consecutive
+// 32-row blocks of one head.
 //
 // Both products are 32x32x16 matrix instructions with the query on the column side: S^T = K Q^T leaves a lane with 16 scores
 // of ONE query row per 32 positions, so the softmax statistics are lane-local up to one exchange between the wave's
@@ -86,18 +88,21 @@ __global__ __launch_bounds__(256) void prefill_cache_kernel(const uint16_t* __re
 // LDS rows are XOR-swizzled in 16-byte chunks (fragment reads of 16 lanes cover all banks).  Tiles are double-buffered
 // through registers, one barrier per tile.
 //
-// Bound by its LDS fragment reads (32 reads of 1 KB per 32 matrix instructions and wave).  Llama-3-8B widths, 1000
-// positions: see the figures beside prefill_attention below.
+// Bound by the latency of a tile's chain (scores, maximum, exponentials, second product), which a second wave per SIMD half
+// hides: with one group (and the fetched keys kept in scratch memory, as structs) the rows of the last tiles took 3.5 us per tile.
+// Llama-3-8B widths, 1000 positions: 56 -> 35 us.
 template <class E, bool HEADS>
-__global__ __launch_bounds__(256) void prefill_attention_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ freqs,
+__global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ freqs,
                                                                 const void* __restrict__ pos, int pos_is_i64, int T, int n_head,
                                                                 int n_kv, int64_t S, const uint16_t* __restrict__ k_cache,
                                                                 const uint16_t* __restrict__ v_cache, uint16_t* __restrict__ out) {
     typedef Mfma32<E> MM;
-    __shared__ uint4 ks[2][64 * 16];   // [key][chunk of 8 d], chunk ^ (key & 15)
-    __shared__ uint4 vs[2][64 * 16];   // [d / 2][(d & 1) * 8 + (chunk of 8 keys ^ (d / 2 & 7))]
+    __shared__ uint4 lds[2][2][2][64 * 16];   // [group][K / V][buffer]
     __shared__ int wave_last[4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 31, half = lane >> 5;
+    const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    uint4 (*const ks)[64 * 16] = lds[group][0];   // [key][chunk of 8 d], chunk ^ (key & 15)
+    uint4 (*const vs)[64 * 16] = lds[group][1];   // [d / 2][(d & 1) * 8 + (chunk of 8 keys ^ (d / 2 & 7))]
+    const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, col = lane & 31, half = lane >> 5;
     const int tile = gridDim.y - 1 - blockIdx.y;   // the rows that see most positions start first
     int head, row0;
     if (HEADS) {
@@ -139,7 +144,7 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(const uint16_t* 
     __syncthreads();
     const int ntile = (max(max(wave_last[0], wave_last[1]), max(wave_last[2], wave_last[3])) + 64) / 64;
 
-    uint4 kr[4];
+    u32x4p_t kr[4];
     uint32_t vr[16];
     const int smax = (int)S - 1;
     auto fetch = [&](int t) {
@@ -147,7 +152,7 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(const uint16_t* 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int key = min(base + i * 16 + (tid >> 4), smax);
-            kr[i] = *(const uint4*)(kc + (int64_t)key * 128 + (tid & 15) * 8);
+            kr[i] = *(const u32x4p_t*)(kc + (int64_t)key * 128 + (tid & 15) * 8);
         }
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
@@ -164,7 +169,7 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(const uint16_t* 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int key = i * 16 + (tid >> 4);
-            ks[b][key * 16 + ((tid & 15) ^ (key & 15))] = kr[i];
+            *(u32x4p_t*)&ks[b][key * 16 + ((tid & 15) ^ (key & 15))] = kr[i];
         }
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
@@ -188,15 +193,15 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(const uint16_t* 
     float m = -INFINITY, sum = 0.f;                 // running maximum and (this lane's share of the) sum, base 2
     const float scale = 0.08838834764831845f * 1.4426950408889634f;  // 1 / sqrt(128), log2(e)
 
-    if (ntile > 0) {
-        fetch(0);
+    if (group < ntile) {
+        fetch(group);
         stash(0);
     }
-    for (int t = 0; t < ntile; ++t) {
-        const int b = t & 1;
-        if (t + 1 < ntile) fetch(t + 1);
+    for (int t = group; t < ntile + group; t += 2) {   // as many passes in both groups: they share the barrier
+        const int b = (t >> 1) & 1;
+        if (t + 2 < ntile) fetch(t + 2);
         __syncthreads();                            // tile t is in LDS; everybody is done with the other buffer
-        if (t * 64 <= hi) {
+        if (t < ntile && t * 64 <= hi) {
             f32x16_t s2[2];
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
@@ -246,7 +251,36 @@ __global__ __launch_bounds__(256) void prefill_attention_kernel(const uint16_t* 
                 }
             }
         }
-        if (t + 1 < ntile) stash(b ^ 1);
+        if (t + 2 < ntile) stash(b ^ 1);
+    }
+    // the second group's maximum, sum and accumulators join the first's
+    __syncthreads();
+    float* const part = (float*)lds + (wave * 64 + lane) * 4;   // [64 / 4 + 1][4 waves * 64 lanes][4]
+    if (group) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4)
+                *(float4*)(part + (b * 4 + r / 4) * 1024) = make_float4(o[b][r], o[b][r + 1], o[b][r + 2], o[b][r + 3]);
+        *(float2*)(part + 16 * 1024) = make_float2(m, sum);
+    }
+    __syncthreads();
+    if (group) return;
+    {
+        const float2 ms = *(const float2*)(part + 16 * 1024);
+        const float m2 = fmaxf(m, ms.x), base = m2 == -INFINITY ? 0.f : m2;
+        const float a0 = __builtin_amdgcn_exp2f(m - base), a1 = __builtin_amdgcn_exp2f(ms.x - base);
+        sum = sum * a0 + ms.y * a1;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) {
+                const float4 v = *(const float4*)(part + (b * 4 + r / 4) * 1024);
+                o[b][r] = o[b][r] * a0 + v.x * a1;
+                o[b][r + 1] = o[b][r + 1] * a0 + v.y * a1;
+                o[b][r + 2] = o[b][r + 2] * a0 + v.z * a1;
+                o[b][r + 3] = o[b][r + 3] * a0 + v.w * a1;
+            }
     }
     sum += __shfl_xor(sum, 32, 64);
     const float inv = 1.0f / sum;                   // a row that sees nothing (a position outside the cache) becomes NaN
@@ -345,10 +379,10 @@ static void prefill_attention(const uint16_t* qkv, const uint16_t* freqs, const 
     hipLaunchKernelGGL(prefill_cache_kernel<E>, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, qkv, freqs, pos, pos_is_i64, T,
                        n_head, n_kv, S, kc, vc);
     if (n_head / n_kv % 4 == 0)
-        hipLaunchKernelGGL((prefill_attention_kernel<E, true>), dim3(n_head / 4, (T + 31) / 32), dim3(256), 0, st, qkv, freqs, pos,
+        hipLaunchKernelGGL((prefill_attention_kernel<E, true>), dim3(n_head / 4, (T + 31) / 32), dim3(512), 0, st, qkv, freqs, pos,
                            pos_is_i64, T, n_head, n_kv, S, kc, vc, out);
     else
-        hipLaunchKernelGGL((prefill_attention_kernel<E, false>), dim3(n_head, (T + 127) / 128), dim3(256), 0, st, qkv, freqs, pos,
+        hipLaunchKernelGGL((prefill_attention_kernel<E, false>), dim3(n_head, (T + 127) / 128), dim3(512), 0, st, qkv, freqs, pos,
                            pos_is_i64, T, n_head, n_kv, S, kc, vc, out);
 }
 
