@@ -152,6 +152,9 @@ __device__ __forceinline__ const T* uniform_ptr(const T* p) {
 // registers, in the shadow of the matrix instructions.  The activation slice (256 x 64 bf16) is shared through LDS,
 // double buffered, one barrier per K step.
 //
+// K may be split over blockIdx.y (launch_int4wo_gemm_lds_parts) where the tiles of a narrow weight leave CUs idle: 4096 x 14336 at
+// 1000 rows, 128 tiles of 256 x 128 in two parts each, 123 us against 137 of the 128-row kernel's 512 workgroups.
+//
 // One K step = 4 sub-steps ks of 16 slots; a slot is one matrix instruction followed by the work that runs in its
 // shadow.  Entering step s, fragment set 0 holds sub-step 0 of both operands.
 //   every ks:  slots 0-7 read the activation fragments of the next sub-step (ks 3: sub-step 0 of step s + 1, from the
@@ -176,7 +179,10 @@ __global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a
     if ((int)(blockIdx.x >> 3) >= tiles_per_xcd || tile >= tiles_total) return;
     const int tile_m = tile / tiles_n, tile_n = tile - tile_m * tiles_n;
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
-    const int KS = (int)(a.Kp / 64);
+    // the 64-wide K steps of this workgroup: all of them, or with a.ksplit > 1 the blockIdx.y-th run of an even number of them,
+    // whose fp32 products go to part blockIdx.y of a.y [ksplit][M][ldy]
+    const int KA = (int)(a.Kp / 64), per = ((KA + a.ksplit - 1) / a.ksplit + 1) & ~1, first = per * (int)blockIdx.y;
+    const int KS = KA - first < per ? KA - first : per;
     const int KB = (int)(a.Kp / 128);
     const int64_t nblocks = (a.N + 15) / 16;
     const uint32_t magic = 0x64006400u;  // the fp16 pair (1024, 1024)
@@ -194,7 +200,7 @@ __global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a
         const int64_t rel = (m0 + row < a.M ? m0 + row : a.M - 1) - m0;
         xoff[j] = (uint32_t)(rel * a.ldx * 2) + ((xp ^ (row & 7)) << 4);
     }
-    const uint16_t* const xbase = uniform_ptr(a.x + m0 * a.ldx);
+    const uint16_t* const xbase = uniform_ptr(a.x + m0 * a.ldx + (int64_t)first * 64);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&lds[0][0];
     auto dma_x1 = [&](int j, int s) __attribute__((always_inline)) {
         s = s < KS ? s : KS - 1;   // steps past the end repeat the last one and are never used
@@ -214,7 +220,7 @@ __global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a
         woff[j] = (uint32_t)((nb - nb0) * KB * 1024) + kq * 256 + (frow & 15) * 16;
         qoff[j] = (uint32_t)((nb - nb0) * (a.Kp / G) * 64) + (G == 32 ? kq * 64 : 0) + (frow & 15) * 4;
     }
-    const uint4* const wbase = uniform_ptr(a.packed + nb0 * KB * 64);
+    const uint4* const wbase = uniform_ptr(a.packed + nb0 * KB * 64 + (int64_t)(first >> 1) * 64);
     const uint32_t* const qbase = uniform_ptr(a.qparams + nb0 * (a.Kp / G) * 16);
     // All loads of the loop are asm statements with explicit waits (the compiler does not count them): per step, in
     // this order, 8 activation requests and then 4 weight requests.
@@ -225,7 +231,7 @@ __global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
             wr[set][j] = asm_load_b128(wbase + (int64_t)(s >> 1) * 64 + (s & 1) * 32, woff[j]);
-            qr[set][j] = asm_load_b32(qbase + (int64_t)((s * 64) / G) * 16, qoff[j]);
+            qr[set][j] = asm_load_b32(qbase + (int64_t)(((first + s) * 64) / G) * 16, qoff[j]);
         }
     };
 
@@ -390,7 +396,7 @@ __global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a
                 const int64_t m = m0 + i * 32 + 8 * (e >> 2) + 4 * kq + (e & 3);
                 if (m < a.M) {
                     const float v = acc_read(acc[i][j][e]) + bv;
-                    if (a.y_is_f32) ((float*)a.y)[m * a.ldy + n] = v;
+                    if (a.y_is_f32) ((float*)a.y)[((int64_t)blockIdx.y * a.M + m) * a.ldy + n] = v;
                     else ((uint16_t*)a.y)[m * a.ldy + n] = f32_to_bf16_bits(v);
                 }
             }
@@ -705,7 +711,7 @@ static void launch_gemm_kwave(const LinearArgs& a, int64_t g, const GemmLdsPlan&
 template <int NT>
 static void launch_gemm_lds_nt(const LinearArgs& a, int64_t g, const GemmLdsPlan& p, hipStream_t st) {
     const int total = p.tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
-    const dim3 grid((unsigned)(per_xcd * 8)), block(256);
+    const dim3 grid((unsigned)(per_xcd * 8), (unsigned)a.ksplit), block(256);
     auto go = [&](auto kernel) {
         if (g_prof_start && g_prof_stop) {
             hipExtLaunchKernelGGL(kernel, grid, block, 0, st, g_prof_start, g_prof_stop, 0, a, p.tiles_n, total, per_xcd);
@@ -720,6 +726,12 @@ static void launch_gemm_lds_nt(const LinearArgs& a, int64_t g, const GemmLdsPlan
         case 128: go(int4wo_gemm_lds_kernel<128, NT>); break;
         default: go(int4wo_gemm_lds_kernel<256, NT>); break;
     }
+}
+
+void launch_int4wo_gemm_lds_parts(const LinearArgs& a, int64_t g, int nt, hipStream_t st) {
+    const GemmLdsPlan p{nt, (int)((a.M + 255) / 256), (int)((a.N + 128 * nt - 1) / (128 * nt))};
+    if (nt == 1) launch_gemm_lds_nt<1>(a, g, p, st);
+    else launch_gemm_lds_nt<2>(a, g, p, st);
 }
 
 bool launch_int4wo_gemm_lds(const LinearArgs& a, int64_t g, hipStream_t st) {

@@ -153,5 +153,8 @@ bool int4wo_gemv2_plan(const LinearArgs& a, int64_t g, int64_t RB, char* out, si
 // Prefill GEMM with the weight tile dequantized once per workgroup into LDS (int4wo_gemm.hip); same contract as above.
 bool launch_int4wo_gemm_lds(const LinearArgs& a, int64_t g, hipStream_t st);
 bool int4wo_gemm_lds_plan(const LinearArgs& a, int64_t g, char* out, size_t cap);
+// Its 256 x 128 nt tiles with K split over a.ksplit workgroups: a.y takes fp32 parts [ksplit][M][ldy], no bias.  K is the packed
+// width, every part has at least 8 of the 64-wide steps and a.ksplit is at most 4 (no part is empty then).
+void launch_int4wo_gemm_lds_parts(const LinearArgs& a, int64_t g, int nt, hipStream_t st);
 
 }  // namespace ao

@@ -82,10 +82,14 @@ static const TileShape kInt4Shapes[] = {
     {128, 128, 41.8, 0.0},   // two groups
     {192, 128, 57.0, 0.0},
     {256, 128, 66.0, 0.0},
+    // the kernels of int4wo_gemm.hip, which have no K parts of their own: in_features of the packed width only
+    {256, 128, 64.0, 0.0, 4},
+    {256, 256, 104.0, 0.0, 4},
 };
+static constexpr int kInt4Own = 6, kInt4All = 8;
 
 static TilePlan int4wo_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
-    return tile_plan(kInt4Shapes, (int)(sizeof(kInt4Shapes) / sizeof(kInt4Shapes[0])), M, N, K, max_parts);
+    return tile_plan(kInt4Shapes, K % 256 == 0 && M >= 128 ? kInt4All : kInt4Own, M, N, K, max_parts);
 }
 
 // us of the kernel that ao_amd_int4wo_linear(_ws) runs, by measurement at 33 to 1000 rows on 16 weights from 768 x 1024 to 28672 x
@@ -98,7 +102,8 @@ static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
     auto up = [](double r) { return (double)(int64_t)(r + 255.0 / 256.0); };
     if (!strncmp(name, "int4wo_gemm_lds_kernel", 22)) {
         const bool wide = strstr(name, ",2>") != nullptr;
-        if (wide) return 6.0 + 98.0 * k * up(rounds(256, 256));
+        const double rw = rounds(256, 256);
+        if (wide) return 6.0 + 100.0 * k * (rw < 1.0 ? 0.4 + 0.6 * rw : up(rw));   // CUs that run at once slow each other down
         const double r = rounds(256, 128), full = (double)(int64_t)r, rest = r - full;
         return 14.0 + k * (52.5 * full + (rest == 0.0 ? 0.0 : full > 0.0 && rest <= 0.5 ? 28.0 : 52.5));
     }
@@ -115,7 +120,7 @@ static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
 
 // Whether the tiled product is the faster one.  us, the others / tiled: 14336 x 4096 at 64 / 128 / 160 / 256 / 384 / 512 rows 23.8 / 21.3,
 // 24.4 / 31.3, 44.8 / 37.4, 46.9 / 42.5, 62.9 / 57.3, 63.8 / 67.2; 4096 x 14336 at 96 / 160 / 640 / 1000 rows 32.7 / 26.8, 53.9 / 39.5, 124 /
-// 108, 141 / 135; 4096 x 4096 at 128 / 256 / 512 / 768 rows 14.7 / 15.9, 23.5 / 19.6, 24.6 / 31.6, 44.1 / 37.6; 11008 x 4096 at 48 / 96 / 384
+// 108, 137 / 123; 8192 x 28672 at 448 rows 275 / 207; 4096 x 4096 at 128 / 256 / 512 / 768 rows 14.7 / 15.9, 23.5 / 19.6, 24.6 / 31.6, 44.1 / 37.6; 11008 x 4096 at 48 / 96 / 384
 // rows 26.2 / 18.5, 35.1 / 25.2, 66.1 / 56.5; 8192 x 28672 at 96 rows 114 / 74.  The estimates hold to some 10 %: a lead of 5 % is asked for.
 static bool int4wo_tiled(int64_t M, int64_t N, int64_t K, int64_t g) {
     if (!valid_group(g) || K % 64 != 0 || M <= 32 || M * N >= ((int64_t)1 << 40)) return false;
@@ -191,7 +196,19 @@ extern "C" int ao_amd_int4wo_linear_tiled(const void* x_bf16, int64_t M, int64_t
         case 2: tile_launch<Int4Tile, 4, 2, 3, 1>(a, p.parts, st); break;
         case 3: tile_launch<Int4Tile, 4, 2, 4, 1>(a, p.parts, st); break;
         case 4: tile_launch<Int4Tile, 4, 1, 6, 1>(a, p.parts, st); break;
-        default: tile_launch<Int4Tile, 4, 1, 8, 1>(a, p.parts, st); break;
+        case 5: tile_launch<Int4Tile, 4, 1, 8, 1>(a, p.parts, st); break;
+        default: {
+            LinearArgs l{};
+            l.x = a.x; l.M = M; l.K = l.Kp = K; l.ldx = ldx;
+            l.packed = (const uint4*)packed; l.qparams = (const uint32_t*)qparams; l.N = N;
+            l.ksplit = p.parts;
+            if (p.parts == 1) {
+                l.bias = a.bias; l.y = a.y; l.ldy = ldy;
+            } else {
+                l.y = a.parts; l.y_is_f32 = 1; l.ldy = N;
+            }
+            launch_int4wo_gemm_lds_parts(l, g, p.shape - kInt4Own + 1, st);
+        }
     }
     tile_finish<Int4Tile>(a, p.parts, st);
     AO_LAUNCH_CHECK();

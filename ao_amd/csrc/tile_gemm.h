@@ -277,6 +277,7 @@ __global__ __launch_bounds__(256) void tile_finish_kernel(const TileGemmArgs a, 
 struct TileShape {
     int bm, bn;
     double one, two;
+    int max_parts = 8;
 };
 struct TilePlan {
     int shape, parts;
@@ -286,7 +287,7 @@ inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64
     TilePlan best{-1, 1, 1e30};
     const int64_t steps = K / 64;
     for (int i = 0; i < nshapes; ++i)
-        for (int z = 1; z <= max_parts; z *= 2) {
+        for (int z = 1; z <= (max_parts < shapes[i].max_parts ? max_parts : shapes[i].max_parts); z *= 2) {
             const int64_t per = (steps + z - 1) / z;
             if (z > 1 && (per < 8 || (z - 1) * per >= steps)) break;
             const int64_t wgs = (M + shapes[i].bm - 1) / shapes[i].bm * ((N + shapes[i].bn - 1) / shapes[i].bn) * z;

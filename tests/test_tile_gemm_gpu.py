@@ -149,7 +149,10 @@ def test_fp6_tiles_cover_every_shape_and_the_operator_takes_them():
 INT4_TILES = [
     (1, 20, 128, 32), (33, 4100, 4096, 64), (65, 1040, 256, 256), (65, 14330, 1024, 128), (96, 4096, 8192, 32), (97, 14336, 512, 64),
     (129, 14336, 1024, 128), (200, 14337, 1024, 256), (257, 14336, 1024, 64), (512, 14336, 512, 32), (640, 4096, 14336, 64), (769, 4096, 2048, 128),
-    (1000, 4099, 2048, 64), (100, 8192, 4096, 256), (34, 1030, 64, 128), (70, 4096, 4032, 256), (130, 4099, 1088, 64), (40, 2048, 8256, 32),
+    (1000, 4099, 2048, 64), (100, 8192, 4096, 256),
+    # the prefill kernel's tiles with K parts: two and four of them, part lengths rounded up to an even number of steps, short last part
+    (400, 4096, 9984, 256), (400, 4090, 12544, 32), (512, 6144, 12544, 128), (200, 11008, 8192, 64), (400, 11000, 14336, 64), (900, 4096, 14336, 64),
+    (34, 1030, 64, 128), (70, 4096, 4032, 256), (130, 4099, 1088, 64), (40, 2048, 8256, 32),
 ]
 
 
@@ -204,7 +207,8 @@ def test_int4_tiles_cover_every_shape_and_the_operator_takes_them():
     from ao_amd import ops
 
     plans = {c: _tiled_plan("int4wo", *c[:3]) for c in INT4_TILES}
-    assert {p.split()[1] for p in plans.values()} == {"64x64", "64x128", "96x128", "128x128", "192x128", "256x128"}, plans
+    assert {p.split()[1] for p in plans.values()} == {"64x64", "64x128", "96x128", "128x128", "192x128", "256x128", "256x256"}, plans
+    assert {f"tile 256x{n} parts={z}" for n, z in ((128, 2), (128, 4), (256, 2), (256, 4))} <= set(plans.values()), plans
     assert any(p.endswith("parts=1") for p in plans.values()) and any(not p.endswith("parts=1") for p in plans.values())
     for rows, taken in ((32, False), (48, False), (128, False), (160, True), (256, True), (384, True), (768, False)):
         assert (_tiled_bytes("int4wo", rows, 14336, 4096, 64) >= 0) == taken, rows
