@@ -34,6 +34,7 @@ _SIGNATURES = {
     "ao_amd_abi_version": ([], _int),
     "ao_amd_last_error": ([], ctypes.c_char_p),
     "ao_amd_choose_qparams_affine": ([_p, _int, _i64, _i64, _i64, _i64, _i64, _int, _i64, _i64, _dbl, _int, _int, _int, _int, _p, _p, _p], _int),
+    "ao_amd_int8wo_quantize": ([_p, _i64, _i64, _i64, _i64, _i64, ctypes.c_double, _p, _p, _p, _p], _int),
     "ao_amd_quantize_affine": ([_p, _int, _i64, _i64, _i64, _i64, _i64, _p, _int, _p, _int, _i64, _i64, _int, _p, _int, _p], _int),
     "ao_amd_dequantize_affine": ([_p, _int, _i64, _i64, _i64, _i64, _p, _int, _p, _int, _i64, _i64, _int, _p, _int, _p], _int),
     "ao_amd_int4wo_packed_shape": ([_i64, _i64, _i64, _i64p, _i64p, _i64p, _i64p], _int),

@@ -17,6 +17,7 @@ from ..quantization.quant_primitives import (
     ZeroPointDomain,
     choose_qparams_affine,
     dequantize_affine,
+    int8wo_quantize,
     quantize_affine,
 )
 from .utils import (
@@ -157,11 +158,20 @@ class AffineQuantizedTensor(torch.Tensor):
                 pad_k = (-input_float.shape[-1]) % g
                 if pad_k:
                     input_float = torch.nn.functional.pad(input_float, (0, pad_k))
-            scale, zero_point = choose_qparams_affine(input_float, mapping_type, block_size, target_dtype, quant_min,
-                                                      quant_max, eps, scale_dtype, zero_point_dtype, preserve_zero,
-                                                      zero_point_domain)
-            int_data = quantize_affine(input_float, block_size, scale, zero_point, target_dtype, quant_min, quant_max,
-                                       zero_point_domain)
+            int8_recipe = (
+                mapping_type == MappingType.SYMMETRIC and target_dtype is torch.int8 and scale_dtype in (None, torch.bfloat16)
+                and zero_point_dtype is torch.int64 and preserve_zero and zero_point_domain == ZeroPointDomain.INT
+                and input_float.dim() == 2 and tuple(block_size) == (1, input_float.shape[1])
+            )
+            one_pass = int8wo_quantize(input_float, quant_min, quant_max, eps) if int8_recipe else None
+            if one_pass is not None:
+                int_data, scale, zero_point = one_pass
+            else:
+                scale, zero_point = choose_qparams_affine(input_float, mapping_type, block_size, target_dtype, quant_min,
+                                                          quant_max, eps, scale_dtype, zero_point_dtype, preserve_zero,
+                                                          zero_point_domain)
+                int_data = quantize_affine(input_float, block_size, scale, zero_point, target_dtype, quant_min, quant_max,
+                                           zero_point_domain)
             ctor = get_layout_tensor_constructor(extended_layout)
             if tiled:
                 layout_tensor = ctor(int_data, scale, zero_point, inner_k_tiles)

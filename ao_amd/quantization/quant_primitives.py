@@ -205,6 +205,25 @@ def quantize_affine(
     return out
 
 
+def int8wo_quantize(w: torch.Tensor, quant_min: Optional[int], quant_max: Optional[int], eps: Optional[float]):
+    """choose_qparams_affine and quantize_affine of int8_weight_only's call (one symmetric scale per row) in one pass over the
+    weight -> (codes, scale, zero point), the same bits; None where the kernel does not take the weight."""
+    N, K = w.shape
+    if w.dtype is not torch.bfloat16 or not w.is_cuda or N < 1 or K < 8 or K % 8 or K > 16384 or w.stride(1) != 1 or w.stride(0) % 8 \
+            or w.stride(0) < K or w.data_ptr() % 16:
+        return None
+    quant_min, quant_max = _get_and_check_qmin_qmax(torch.int8, quant_min, quant_max)
+    if quant_max <= quant_min:
+        return None
+    codes = torch.empty((N, K), dtype=torch.int8, device=w.device)
+    scale = torch.empty((N,), dtype=torch.bfloat16, device=w.device)
+    zero_point = torch.empty((N,), dtype=torch.int64, device=w.device)
+    require_cuda(w)
+    check(lib().ao_amd_int8wo_quantize(w.data_ptr(), N, K, w.stride(0), quant_min, quant_max, -1.0 if eps is None else float(eps),
+                                       codes.data_ptr(), scale.data_ptr(), zero_point.data_ptr(), current_stream(w.device)))
+    return codes, scale, zero_point
+
+
 def dequantize_affine(
     input: torch.Tensor,
     block_size: Tuple[int, ...],

@@ -50,6 +50,11 @@ int ao_amd_choose_qparams_affine(const void* in, int in_dtype, int64_t N, int64_
                                  int zp_domain, int scale_dtype, int zp_dtype, void* scale, void* zero_point,
                                  void* stream);
 
+/* choose_qparams_affine and quantize_affine of int8_weight_only's call (torchao/quantization/quant_api.py:390-405) in one pass:
+ * bf16 rows [N, K] (row stride ld, K and ld multiples of 8, K at most 16384) -> int8 codes [N, K], one bf16 scale and int64 zero
+ * point per row; symmetric mapping, eps < 0: the type's.  Bit for bit what the two calls give. */
+int ao_amd_int8wo_quantize(const void* w_bf16, int64_t N, int64_t K, int64_t ld, int64_t qmin, int64_t qmax, double eps,
+                           void* out_int8, void* scale_bf16, void* zero_point_i64, void* stream);
 /* replaces quantize_affine, torchao/quantization/quant_primitives.py:134-206
  * zero_point may be NULL in the INT domain.  out: contiguous [N,K] of out_dtype (AO_I32/I64/I8/U8). */
 int ao_amd_quantize_affine(const void* in, int in_dtype, int64_t N, int64_t K, int64_t ld, int64_t bN, int64_t bK,

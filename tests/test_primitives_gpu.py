@@ -175,3 +175,30 @@ def test_int8_rows_dequantize(N, K, zero_point):
     want = (q.int() - (zero_point or 0)).bfloat16() * s[:, None]
     assert np.array_equal(bits16(out)[~want.isnan().numpy()], bits16(want)[~want.isnan().numpy()])
     assert (bits16(out)[want.isnan().numpy()] == 0x7FC0).all()
+
+
+@pytest.mark.parametrize("N,K", [(1, 8), (3, 520), (17, 2048), (9, 2056), (130, 4096), (6, 4104), (5, 8192), (4, 8200), (2, 6144), (2, 10248), (2, 12288), (2, 14336), (3, 16384)])
+@pytest.mark.parametrize("pad", [0, 24])
+def test_int8_quantization_in_one_pass_is_the_two_calls(N, K, pad):
+    from ao_amd import int8_weight_only
+    from ao_amd.quantization.quant_primitives import MappingType, choose_qparams_affine, int8wo_quantize, quantize_affine
+
+    w = torch.zeros(N, K + pad, dtype=torch.bfloat16)
+    w[:, :K] = _weight(N, K, torch.bfloat16, N + K)
+    if N > 8:
+        w[3, 5], w[4, 1], w[5, K - 1] = float("inf"), float("nan"), -float("inf")
+        w[6] *= 1e-38
+        w[7] *= 3e38
+        w[8] = -w[8].abs()
+    w = w.cuda()[:, :K]
+    for lo, hi, eps in ((None, None, torch.finfo(torch.float32).eps), (-127, 127, None), (-100, 90, 1e-3)):
+        s, z = choose_qparams_affine(w, MappingType.SYMMETRIC, (1, K), torch.int8, lo, hi, eps, None, torch.int64)
+        q = quantize_affine(w, (1, K), s, z, torch.int8, lo, hi)
+        got = int8wo_quantize(w, lo, hi, eps)
+        assert torch.equal(got[0], q) and np.array_equal(bits16(got[1]), bits16(s)) and torch.equal(got[2], z)
+    layout = int8_weight_only()(w).layout_tensor
+    s, z = choose_qparams_affine(w, MappingType.SYMMETRIC, (1, K), torch.int8, eps=torch.finfo(torch.float32).eps, zero_point_dtype=torch.int64)
+    assert torch.equal(layout.int_data, quantize_affine(w, (1, K), s, z, torch.int8)) and layout.int_data.is_contiguous()
+    assert np.array_equal(bits16(layout.scale), bits16(s)) and torch.equal(layout.zero_point, z) and layout.scale.shape == s.shape
+    for other in (w.half(), w[:, : K - 4] if K > 8 else w.float(), torch.zeros(2, 16392, dtype=torch.bfloat16, device="cuda")):
+        assert int8wo_quantize(other, None, None, None) is None
