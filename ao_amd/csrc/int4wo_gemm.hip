@@ -412,13 +412,17 @@ __global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a
 // step) and waits for them with its own counters.  The weights are dequantized once per workgroup, as in the 256-row
 // kernel, but a 128-row tile has only 4 matrix instructions per weight dword, so the 33 VALU instructions of the
 // dequantization bound the loop (8 per matrix instruction): about 60 cycles per matrix instruction instead of 32.
-// Slot schedule of a step: as in the 256-row kernel with 8 slots per sub-step; the DMA requests of step t + 2 go one
+// Slot schedule of a step: as in the 256-row kernel with 2 MT slots per sub-step; the DMA requests of step t + 2 go one
 // per slot into sub-step 3 (after a wait for the LDS reads of the buffer they overwrite) and sub-step 0 of step t + 1.
-template <int G>
-__global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs a, int tiles_n, int tiles_total,
-                                                                 int tiles_per_xcd) {
-    constexpr int BM = 128, BN = 64, MT = 4, NT = 2, XCH = 16, SLOTS = MT * NT;
-    __shared__ __align__(16) uint8_t lds[4][2][BM * 128];
+// MT = 3: 96-row tiles where there are no more of them than 128-row ones.  The activations come from L2 once per 64 columns, 11
+// TB/s at 77 rows, and a quarter of that is rows past M; and three slices fit the LDS, so a step's requests (sub-steps 0 to 2,
+// for the step after next, into the slice that the step before has left) have a whole step to arrive.  13824 x 5120 at 77 rows
+// 31.0 us on 128-row tiles, 27.9 on 96-row tiles with two slices, 24.7 with three.
+template <int G, int MT>
+__device__ __forceinline__ void gemm_kwave(const LinearArgs& a, int tiles_n, int tiles_total, int tiles_per_xcd) {
+    constexpr int BM = 32 * MT, BN = 64, NT = 2, XCH = 4 * MT, SLOTS = MT * NT;
+    constexpr int NB = MT == 3 ? 3 : 2, BUF = BM * 128;   // activation slices of a wave in LDS: as many as 160 KB hold
+    __shared__ __align__(16) uint8_t lds[4][NB][BUF];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -445,10 +449,10 @@ __global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs
     const uint16_t* const xbase = uniform_ptr(a.x + m0 * a.ldx);
     uint8_t* const Lw = &lds[wave][0][0];
     const uint32_t ldsw = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)Lw;
-    auto dma_x1 = [&](int j, int t) __attribute__((always_inline)) {
+    auto dma_x1 = [&](int j, int t, int b) __attribute__((always_inline)) {
         const int tc = t < nst ? t : nst - 1;   // steps past the end repeat the last one and are never used
         const int s = wave + 4 * tc;
-        const uint32_t m0v = ldsw + (t & 1) * (BM * 128) + j * 1024;
+        const uint32_t m0v = ldsw + b * BUF + j * 1024;
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                      :: "v"(xoff[j]), "s"(xbase + (int64_t)s * 64), "s"(m0v) : "memory");
     };
@@ -489,20 +493,29 @@ __global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs
 
     Frag fa[2][MT], fb[2][NT];
 #pragma unroll
-    for (int j = 0; j < XCH; ++j) dma_x1(j, 0);
+    for (int j = 0; j < XCH; ++j) dma_x1(j, 0, 0);
     load_w(0, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    load_w(1, 1);
+    if constexpr (NB == 2) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        load_w(1, 1);
 #pragma unroll
-    for (int j = 0; j < XCH / 2; ++j) dma_x1(j, 1);
+        for (int j = 0; j < XCH / 2; ++j) dma_x1(j, 1, 1);
+    } else {
+#pragma unroll
+        for (int j = 0; j < XCH; ++j) dma_x1(j, 1, 1);
+        load_w(1, 1);
+        // everything of step 0; the targets as operands, so that nothing reads them in front of the wait
+        asm volatile("s_waitcnt vmcnt(%4)" : "+v"(wr[0][0]), "+v"(wr[0][1]), "+v"(qr[0][0]), "+v"(qr[0][1]) : "n"(XCH + 2 * NT) : "memory");
+    }
 #pragma unroll
     for (int j = 0; j < NT; ++j) fb[0][j].q = dq8_all(wr[0][j].x, make_group_f32(qr[0][j]), magic);
 #pragma unroll
     for (int i = 0; i < MT; ++i) fa[0][i].q = *reinterpret_cast<const u32x4_t*>(Lw + afrag0 + i * 4096);
 
-    auto step = [&](int t, const int set) __attribute__((always_inline)) {
-        const uint8_t* As = Lw + (t & 1) * (BM * 128);
-        const uint8_t* An = Lw + ((t + 1) & 1) * (BM * 128);
+    auto step = [&](int t, const int set, const int b) __attribute__((always_inline)) {
+        const int next = b + 1 == NB ? 0 : b + 1, ahead = b == 0 ? NB - 1 : b - 1;   // ahead: step t + 2's of three slices
+        const uint8_t* As = Lw + b * BUF;
+        const uint8_t* An = Lw + next * BUF;
         GroupF32 gc[NT];
 #pragma unroll
         for (int j = 0; j < NT; ++j) gc[j] = make_group_f32(qr[set][j]);
@@ -525,7 +538,7 @@ __global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs
                     gc[j] = make_group_f32(qr[set ^ 1][j]);
                 }
                 // the LDS reads of this step's buffer have returned before the requests below overwrite it
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                if constexpr (NB == 2) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             }
             __builtin_amdgcn_sched_barrier(0);
             static_for<0, SLOTS>([&](auto q_c) __attribute__((always_inline)) {
@@ -542,20 +555,25 @@ __global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs
                     else fa[nxt][q].q = *reinterpret_cast<const u32x4_t*>(An + afrag0 + q * 4096);
                 }
                 if constexpr (ks == 3 && q == 0) load_w(set, t + 2);
-                if constexpr (ks == 3) dma_x1(q, t + 2);
-                if constexpr (ks == 0) dma_x1(8 + q, t + 1);
+                if constexpr (NB == 2 && ks == 3) dma_x1(q, t + 2, b);
+                if constexpr (NB == 2 && ks == 0) dma_x1(XCH / 2 + q, t + 1, next);
+                if constexpr (NB == 3 && ks < 3 && q % 3 != 2) dma_x1(ks * 4 + q - q / 3, t + 2, ahead);
                 __builtin_amdgcn_sched_barrier(0);
             });
             if constexpr (ks == 2) {
-                // the wave's activation slice of step t + 1 has landed, and the weights requested before its second half
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                // the wave's activation slice of step t + 1 has landed, and its weights (two slices: requested before the second
+                // half of the activations; three: before this step's requests, which stay in flight)
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NB == 2 ? 0 : XCH) : "memory");
             }
         });
     };
+    int b = 0;
     for (int t = 0; t < nst; t += 2) {
-        step(t, 0);
+        step(t, 0, b);
+        b = b + 1 == NB ? 0 : b + 1;
         if (t + 1 >= nst) break;
-        step(t + 1, 1);
+        step(t + 1, 1, b);
+        b = b + 1 == NB ? 0 : b + 1;
     }
     // a matrix instruction's result may be read 18 issue slots after it at the earliest; the epilogue reads the
     // accumulators through acc_read, volatile asm statements that stay behind this one
@@ -569,9 +587,9 @@ __global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs
                    "+v"(qr[1][0]), "+v"(qr[1][1])
                  :: "memory");
 
-    // Sum of the four waves' partial tiles: every wave leaves its own in its 32 KB of LDS as fp32 [128][64] (the column
+    // Sum of the four waves' partial tiles: every wave leaves its own in its 8 MT KB of LDS as fp32 [BM][64] (the column
     // index flipped by 32 in rows whose bit 2 is set: the two half-waves write rows 4 apart, 1024 bytes, the same
-    // banks otherwise), then wave w adds up rows 32 w .. 32 w + 31 of the four and stores them, 4 columns a lane.
+    // banks otherwise), then wave w adds up a quarter of the rows of the four and stores them, 4 columns a lane.
     // acc[i][j][e] = C[m = m0 + 32 i + 8 (e / 4) + 4 kq + e % 4][n = n0 + 32 j + frow]
 #pragma unroll
     for (int i = 0; i < MT; ++i)
@@ -594,8 +612,8 @@ __global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs
     }
     const bool wide = n + 3 < a.N && (a.ldy & 3) == 0 && ((uintptr_t)a.y & 15) == 0;
 #pragma unroll
-    for (int pass = 0; pass < 8; ++pass) {
-        const int row = 32 * wave + 4 * pass + r;
+    for (int pass = 0; pass < 2 * MT; ++pass) {
+        const int row = 8 * MT * wave + 4 * pass + r;
         const int pc = (c4 * 4) ^ (((row >> 2) & 1) << 5);
         f32x4_t sum = *reinterpret_cast<const f32x4_t*>(&lds[0][0][0] + (row * 64 + pc) * 4);
 #pragma unroll
@@ -623,6 +641,15 @@ __global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs
                 }
         }
     }
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs a, int tiles_n, int tiles_total, int tiles_per_xcd) {
+    gemm_kwave<G, 4>(a, tiles_n, tiles_total, tiles_per_xcd);
+}
+template <int G>
+__global__ __launch_bounds__(256) void int4wo_gemm_kwave96_kernel(const LinearArgs a, int tiles_n, int tiles_total, int tiles_per_xcd) {
+    gemm_kwave<G, 3>(a, tiles_n, tiles_total, tiles_per_xcd);
 }
 
 struct GemmLdsPlan {
@@ -690,6 +717,7 @@ bool int4wo_gemm_lds_plan(const LinearArgs& a, int64_t g, char* out, size_t cap)
 }
 
 static void launch_gemm_kwave(const LinearArgs& a, int64_t g, const GemmLdsPlan& p, hipStream_t st) {
+    const bool three = (a.M + 95) / 96 == p.tiles_m;   // 96-row tiles where they are no more
     const int total = p.tiles_m * p.tiles_n, per_xcd = (total + 7) / 8;
     const dim3 grid((unsigned)(per_xcd * 8)), block(256);
     auto go = [&](auto kernel) {
@@ -701,10 +729,10 @@ static void launch_gemm_kwave(const LinearArgs& a, int64_t g, const GemmLdsPlan&
         }
     };
     switch (g) {
-        case 32: go(int4wo_gemm_kwave_kernel<32>); break;
-        case 64: go(int4wo_gemm_kwave_kernel<64>); break;
-        case 128: go(int4wo_gemm_kwave_kernel<128>); break;
-        default: go(int4wo_gemm_kwave_kernel<256>); break;
+        case 32: three ? go(int4wo_gemm_kwave96_kernel<32>) : go(int4wo_gemm_kwave_kernel<32>); break;
+        case 64: three ? go(int4wo_gemm_kwave96_kernel<64>) : go(int4wo_gemm_kwave_kernel<64>); break;
+        case 128: three ? go(int4wo_gemm_kwave96_kernel<128>) : go(int4wo_gemm_kwave_kernel<128>); break;
+        default: three ? go(int4wo_gemm_kwave96_kernel<256>) : go(int4wo_gemm_kwave_kernel<256>); break;
     }
 }
 

@@ -109,7 +109,8 @@ static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
     }
     if (!strncmp(name, "int4wo_gemm_kwave_kernel", 24)) {
         const double r = up(rounds(128, 64));
-        return 6.0 + (r > 1.0 ? 20.0 : 18.5) * k * r;
+        const bool three = (M + 95) / 96 == (M + 127) / 128;   // its 96-row tiles
+        return 6.0 + (three ? (r > 1.0 ? 17.5 : 16.5) : r > 1.0 ? 20.0 : 18.5) * k * r;
     }
     if (strncmp(name, "int4wo_gemm_", 12)) return 0.0;
     if (ao_amd_int4wo_linear_ws_parts(M, K, N, g) > 1) return M <= 64 ? 0.0 : 4.0 + 8.0 * k;

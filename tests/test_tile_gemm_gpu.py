@@ -240,3 +240,26 @@ def test_int4_rows_that_are_copied_to_the_packed_width(M, N, K, group, shift):
     want = x.double() @ dq.double().t()
     # sums of K <= 4160 exact products in fp32: sqrt(K) roundings of 2^-24 of the partial sum, about 4e-6, times the cancellation in it
     assert ((y32.double() - want).norm() / want.norm()).item() <= 2e-5
+
+
+@pytest.mark.parametrize("M,N,K,group", [(65, 12300, 1024, 64), (96, 12288, 1152, 32), (97, 12288, 1152, 64), (130, 6150, 1280, 256), (192, 6144, 2176, 128),
+                                         (257, 4100, 1024, 64), (288, 4096, 1408, 128), (289, 4096, 1024, 64)])
+def test_int4_kwave_tiles_of_96_and_128_rows(M, N, K, group):
+    """Edges of the 96-row tiles (up to 96, 192 and 288 rows; one more takes 128-row ones), K steps that leave the waves unequal and
+    odd counts, against the fp32 product and, one-hot, the weight bit for bit."""
+    from ao_amd import _lib, ops
+
+    assert _lib.int4wo_linear_plan(M, K, N, group).startswith("int4wo_gemm_kwave_kernel")
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    packed, qp = ops.int4wo_quantize_pack((torch.randn(N, K, device="cuda", generator=g) * 0.02).bfloat16(), group)
+    dq = ops.int4wo_dequantize(packed, qp, N, K, group)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    hot = torch.zeros(M, K, device="cuda").bfloat16()
+    at = (torch.arange(M, device="cuda") * 37 + 5) % K
+    hot[torch.arange(M, device="cuda"), at] = 1.0
+    for rows, want in ((x, (x.float() @ dq.float().t()).bfloat16()), (hot, dq[:, at].t())):
+        y = torch.full((M, N), float("nan"), device="cuda").bfloat16()
+        _lib.check(_lib.lib().ao_amd_int4wo_linear(rows.data_ptr(), M, K, K, packed.data_ptr(), qp.data_ptr(), N, group, None, y.data_ptr(),
+                                                   _lib.BF16, N, torch.cuda.current_stream().cuda_stream))
+        rel = ((y.float() - want.float()).norm() / want.float().norm()).item()   # as for the tiles; one-hot rows are exact
+        assert rel <= (1e-3 if rows is x else 0.0), (M, N, K, rel)
