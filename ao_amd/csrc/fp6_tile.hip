@@ -105,6 +105,8 @@ static bool fp6_tiled(int64_t M, int64_t N, int64_t K) {
     // 1000 rows 14 / 17 / 96, tiled 16 / 16 / 41)
     if (K % 128 != 0) return tile_us < 5.0 + 8.5e-8 * (double)(N * K) * (double)((M + 15) / 16);
     if (M <= 64) return N * K >= ((int64_t)1 << 27);
+    // (the 128 x 128 tiles of fp6.hip were never ahead there: 14336 x 4096 at 1200 / 1500 rows 169 / 178 tiled)
+    if (M >= 1024 && N >= 2048) return true;
     const int64_t big = (N + 127) / 128 * ((M + 127) / 128), mid = (N + 63) / 64 * ((M + 63) / 64), small = (N + 63) / 64 * ((M + 31) / 32);
     const double k = (double)K / 4096.0;
     const double us = big >= 256 ? k * (big > 256 ? 37.0 * (double)((big + 255) / 256) : 50.0)

@@ -85,10 +85,12 @@ TWO_PASS_MIN_M = 4096
 # int8 and FPx: the same choice.  The conversion pass costs the same whatever the row count, so the narrower the weight
 # the later it pays.  int8, fused (tiled kernel) / two-pass in us: 14336 x 4096 at 1024 / 1536 / 2048 rows 140 / 138, 202 / 198,
 # 271 / 226; 28672 x 8192 at 1024 / 1536 / 2048 rows 482 / 518, 693 / 657, 912 / 818; 4096 x 14336 at 2048 rows 211 / 229;
-# 4096 x 4096 at 2048 rows 71 / 82.  FP6: 14336 x 4096 at 768 / 1024 rows 115 / 126, 142 / 134; 4096 x 4096 at 1024 / 1536 /
-# 3072 rows 50 / 54, 71 / 66, 113 / 96; 1024 x 4096 at 2048 / 3072 rows 32 / 36, 46 / 41.
+# 4096 x 4096 at 2048 rows 71 / 82.  FP6: 14336 x 4096 at 1024 / 1500 / 1800 rows 142 / 139, 178 / 197, 243 / 220; 28672 x 8192 at
+# 1024 / 1500 / 2048 rows 465 / 552, 683 / 684, 860 / 850; 6144 x 4096 at 1500 / 1800 / 2048 rows 80 / 99, 92 / 102, 115 / 107; 4096 x
+# 4096 at 1536 / 2048 / 2500 / 3000 rows 54 / 70, 67 / 80, 88 / 89, 97 / 101, 4096 x 14336 at 2048 / 2500 rows 208 / 242, 277 / 274; 1024 x
+# 4096 at 2048 / 3072 rows 32 / 36, 46 / 41.
 INT8_TWO_PASS_MIN_M = 128
-FP6_TWO_PASS_MIN_M = 1024
+FP6_TWO_PASS_MIN_M = 1537
 
 
 def int8wo_two_pass(M: int, N: int, K: int) -> bool:
@@ -96,7 +98,7 @@ def int8wo_two_pass(M: int, N: int, K: int) -> bool:
 
 
 def fp6_two_pass(M: int, N: int, K: int) -> bool:
-    return M >= (3 * FP6_TWO_PASS_MIN_M if N < 2048 else (3 * FP6_TWO_PASS_MIN_M // 2 if N <= 4096 else FP6_TWO_PASS_MIN_M))
+    return M >= (3072 if N < 2048 else 2432 if N <= 4096 else 1920 if N < 8192 else FP6_TWO_PASS_MIN_M)
 
 
 def int4wo_two_pass(M: int, N: int, K: int) -> bool:
@@ -730,7 +732,7 @@ def _fp6_linear_native_cuda(ebits, mbits, x, native, scale):
     if fp6_two_pass(M, N, K):
         # prefill-sized batch: the weight as an fp16 matrix (HIP kernel, the same fp16(fpx * scale) values the fused
         # kernel multiplies) and the library fp16 GEMM; the fused kernel tops out near 0.95 PFLOP/s, the library GEMM
-        # at 1.3-1.5, and the conversion costs about as much as 300 activation rows
+        # at 1.3-1.5, and the conversion costs about as much as 300 activation rows (rule: fp6_two_pass)
         w16 = torch.empty((N, K), dtype=torch.float16, device=x.device)
         check(lib().ao_amd_fp6_native_to_f16(native.data_ptr(), scale.contiguous().data_ptr(), N, K, ebits, mbits,
                                              w16.data_ptr(), current_stream(x.device)))
