@@ -105,6 +105,26 @@ def test_dequantize_into_16_bits_is_the_fp32_value_rounded_once(oracle, N, K, eb
         assert np.array_equal(ops.fp6_dequantize(tc, None, ebits, mbits).cpu().numpy(), oracle.fpx_to_f32(codes, ebits, mbits))
 
 
+@pytest.mark.parametrize("N,K", [(64, 64), (128, 192), (192, 4160), (320, 1024)])
+def test_repack_from_aligned_and_unaligned_bytes(oracle, N, K):
+    """The 16-byte path against the byte-wise one (which takes bytes at an odd address) and the codes themselves."""
+    from ao_amd import ops
+
+    raw = torch.from_numpy(np.random.default_rng(N * K).integers(0, 256, N * K * 6 // 8 + 1, dtype=np.uint8)).to(_dev())
+    odd = raw[1:].view(N, K * 6 // 8)
+    even = odd.clone()
+    assert odd.data_ptr() % 16 and even.data_ptr() % 16 == 0
+    native = ops.fp6_repack(even)
+    assert torch.equal(native, ops.fp6_repack(odd))
+    codes = oracle.unpack_tc_fp6(even.cpu().numpy(), N, K)
+    tiles = native.cpu().numpy().view(np.uint32).reshape(N // 16, (K + 127) // 128, 384)
+    lanes = np.concatenate([tiles[:, :, :256].reshape(*tiles.shape[:2], 64, 4), tiles[:, :, 256:].reshape(*tiles.shape[:2], 64, 2)], -1)
+    bits = np.unpackbits(lanes.astype("<u4").view(np.uint8).reshape(*tiles.shape[:2], 64, 24), axis=-1, bitorder="little")
+    got = np.packbits(bits.reshape(*tiles.shape[:2], 64, 32, 6), axis=-1, bitorder="little")[..., 0]     # [rb, kb, lane, 32]
+    got = got.reshape(*tiles.shape[:2], 4, 16, 32).transpose(0, 3, 1, 2, 4).reshape(N, -1)
+    assert np.array_equal(got[:, :K], codes) and not got[:, K:].any()
+
+
 def test_dequantize_and_repack_round_trip(oracle):
     from ao_amd import ops
 
