@@ -4,6 +4,7 @@
 //
 // The caller describes the model as nested tuples of tensors and numbers (Transformer._host_plan); they are checked
 // completely before the first launch.
+#include <ATen/autocast_mode.h>
 #include <ATen/ops/linear.h>
 #include <ATen/ops/mul.h>
 
@@ -323,6 +324,9 @@ PyObject* llama_forward(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     const int64_t T = tokens.numel();
     AO_WANT(T >= 1 && tokens.dim() == 2 && tokens.size(0) == 1 && tokens.is_contiguous() && pos.dim() == 1 && pos.numel() == T &&
             pos.is_contiguous() && (T > 1 || pos.scalar_type() == at::kInt));
+    // Autocast changes the types between the modules of a prompt (it clears a key that is excluded otherwise, so nothing_watches()
+    // does not see it); a decode step is made of operators that it leaves alone.
+    AO_WANT(T == 1 || !at::autocast::is_autocast_enabled(at::kCUDA));
     return guarded([&]() -> PyObject* {
         const Model m = read_model(a, v[0]);
         AO_WANT(a.ok);

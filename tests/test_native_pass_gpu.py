@@ -1,0 +1,59 @@
+"""The native pass of the Llama model (csrc/host/llama.cpp) against the module chain that it stands for: where the modules would
+give something else it has to leave the prompt to them, bit for bit."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+RECIPES = ("int4", "int8", "fp6")
+
+
+def _model(fmt, layers=2, intermediate=1024, positions=160, block_size=512, seed=0):
+    from ao_amd import fp6_llm_weight_only, int4_weight_only, int8_weight_only, quantize_
+    from ao_amd._models.llama.generate import random_init_
+    from ao_amd._models.llama.model import ModelArgs, Transformer
+
+    args = ModelArgs(block_size=block_size, n_layer=layers, n_head=4, n_local_heads=2, dim=512, intermediate_size=intermediate,
+                     vocab_size=1024)
+    with torch.device("cuda"):
+        model = Transformer(args).to(torch.bfloat16)
+    random_init_(model, seed=seed)
+    model = model.eval().to(torch.float16 if fmt == "fp6" else torch.bfloat16)
+    quantize_(model, {"int4": lambda: int4_weight_only(64), "int8": int8_weight_only, "fp6": fp6_llm_weight_only}[fmt]())
+    model.setup_caches(1, positions)
+    return model
+
+
+def _prompt(model, T, seed=1):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randint(0, model.config.vocab_size, (1, T), device="cuda", generator=g), torch.arange(T, device="cuda")
+
+
+def _caches(model):
+    return [c for b in model.layers for c in (b.attention.kv_cache.k_cache, b.attention.kv_cache.v_cache)]
+
+
+def _both(model, tokens, pos):
+    """(logits, caches) of the call as it is, and of the module chain."""
+    runs = []
+    for fused in (True, False):
+        for c in _caches(model):
+            c.zero_()
+        model.use_fused_decode = fused
+        with torch.no_grad():
+            runs.append([model(tokens, pos)] + [c.clone() for c in _caches(model)])
+    model.use_fused_decode = True
+    return runs
+
+
+def _same(got, want):
+    return all(a.dtype is b.dtype and torch.equal(a, b) for a, b in zip(got, want))
+
+
+# 1536 and 1537 rows: w1 and w3 go through a 16-bit copy of the weight and the library product, which autocast would cast
+@pytest.mark.parametrize("fmt,T,intermediate", [(f, 17, 1024) for f in RECIPES] + [("int8", 1536, 8192), ("fp6", 1537, 8192)])
+def test_autocast_prompts_run_as_modules(fmt, T, intermediate):
+    model = _model(fmt, 1, intermediate, T, 2048)
+    with torch.autocast("cuda", dtype=torch.bfloat16 if fmt == "fp6" else torch.float16):
+        got, want = _both(model, *_prompt(model, T))
+    assert _same(got, want) and not want[0].isnan().any()
