@@ -174,6 +174,24 @@ class TransformerBlock(nn.Module):
         return h + self.feed_forward(self.ffn_norm(h))
 
 
+def _chain_functions():
+    return nn.Module.__call__, KVCache.update, apply_rotary_emb, F.scaled_dot_product_attention, F.silu
+
+
+# What the native pass of a prompt stands for: these classes with their own forward, over these functions
+_CHAIN_FORWARDS = {c: c.forward for c in (nn.Linear, RMSNorm, Attention, FeedForward, TransformerBlock, KVCache)}
+_CHAIN_FUNCTIONS = _chain_functions()
+
+
+def _is_plain(m) -> bool:
+    """m's call runs the forward of its class, one of those above, and nobody has hooked or replaced it."""
+    forward = _CHAIN_FORWARDS.get(type(m))
+    if forward is None or forward is not type(m).forward:
+        return False
+    d = m.__dict__
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d or "update" in d or d.get("_compiled_call_impl"))
+
+
 class Transformer(nn.Module):
     def __init__(self, config: ModelArgs):
         super().__init__()
@@ -270,12 +288,28 @@ class Transformer(nn.Module):
     def fused_decode_ready(self) -> bool:
         return self.fused_decode_kind() is not None
 
-    def _modules_are_watched(self) -> bool:
-        """Whether a hook wants to see the calls of single modules, which the native pass does not make."""
-        hooks = torch.nn.modules.module
-        if hooks._global_forward_hooks or hooks._global_forward_pre_hooks:
-            return True
-        return any(m._forward_hooks or m._forward_pre_hooks for m in self.modules() if m is not self)
+    def _prompt_is_the_module_chain(self) -> bool:
+        """Whether calling module after module would compute what the native pass of a prompt computes: the modules and
+        functions of this file, none subclassed (an adapter's linear), replaced (another norm or block), patched or watched by a
+        hook.  Read anew for every prompt, some 5 us a layer."""
+        hooks, cfg = torch.nn.modules.module, self.config
+        if hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _chain_functions() != _CHAIN_FUNCTIONS:
+            return False
+        if not (_is_plain(self.norm) and _is_plain(self.output)):
+            return False
+        heads = (cfg.n_head, cfg.n_local_heads, cfg.head_dim, cfg.dim)
+        for b in self.layers:
+            if not _is_plain(b):
+                return False
+            parts = b._modules
+            att, ff = parts.get("attention"), parts.get("feed_forward")
+            if not (_is_plain(att) and _is_plain(ff) and (att.n_head, att.n_local_heads, att.head_dim, att.dim) == heads):
+                return False
+            a, f = att._modules, ff._modules
+            if not all(map(_is_plain, (parts.get("attention_norm"), parts.get("ffn_norm"), a.get("kv_cache"), a.get("wqkv"), a.get("wo"),
+                                       f.get("w1"), f.get("w3"), f.get("w2")))):
+                return False
+        return True
 
     def _host_plan(self, kind: str, rows: int) -> tuple:
         """The model as csrc/host/llama.cpp reads it: nested tuples of the tensors that a pass of `rows` tokens needs.  Made
@@ -451,8 +485,8 @@ class Transformer(nn.Module):
         if self.use_fused_decode and input_pos is not None and idx.dim() == 2 and idx.shape[0] == 1 \
                 and not torch.compiler.is_dynamo_compiling():
             # every launch of the pass from one native call; it declines what it does not take before it launches anything
-            kind = self.fused_decode_kind()
-            if kind is not None and (idx.numel() == 1 or not self._modules_are_watched()):
+            kind = self.fused_decode_kind() if idx.numel() == 1 or self._prompt_is_the_module_chain() else None
+            if kind is not None:
                 pos = input_pos.to(torch.int32) if idx.numel() == 1 and input_pos.dtype is not torch.int32 else input_pos
                 logits = ops.host.llama_forward(self._host_plan(kind, idx.numel()), idx, pos)
                 if logits is not NotImplemented:

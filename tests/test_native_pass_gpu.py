@@ -57,3 +57,80 @@ def test_autocast_prompts_run_as_modules(fmt, T, intermediate):
     with torch.autocast("cuda", dtype=torch.bfloat16 if fmt == "fp6" else torch.float16):
         got, want = _both(model, *_prompt(model, T))
     assert _same(got, want) and not want[0].isnan().any()
+
+
+class _Adapter(torch.nn.Linear):
+    def forward(self, x):
+        return super().forward(x) + x.mean(-1, keepdim=True)
+
+
+class _Block(torch.nn.Module):
+    def forward(self, x, input_pos, freqs_cis, mask):
+        return x * 2
+
+
+class _Cache(torch.nn.Module):
+    """A cache of its own that stores halved values."""
+
+    def __init__(self, like):
+        super().__init__()
+        self.k_cache, self.v_cache = like.k_cache, like.v_cache
+
+    def update(self, input_pos, k, v):
+        self.k_cache[:, :, input_pos], self.v_cache[:, :, input_pos] = k / 2, v / 2
+        return self.k_cache, self.v_cache
+
+
+def _adapt(linear):
+    linear.__class__ = _Adapter
+
+
+def _patch(module):
+    forward = module.forward
+    module.forward = lambda *a: forward(*a) * 2
+
+
+def _layer_norm(module, name):
+    setattr(module, name, torch.nn.LayerNorm(512, device="cuda", dtype=torch.bfloat16))
+
+
+CHANGES = {
+    "adapter in wqkv": lambda m, mp: _adapt(m.layers[1].attention.wqkv),
+    "adapter in w2": lambda m, mp: _adapt(m.layers[0].feed_forward.w2),
+    "adapter in output": lambda m, mp: _adapt(m.output),
+    "patched linear": lambda m, mp: _patch(m.layers[0].feed_forward.w1),
+    "patched feed-forward": lambda m, mp: _patch(m.layers[1].feed_forward),
+    "patched class": lambda m, mp: mp.setattr(type(m.norm), "forward", lambda self, x: x * 2),
+    "patched attention function": lambda m, mp: mp.setattr(torch.nn.functional, "scaled_dot_product_attention", lambda q, k, v, **kw: q * 2),
+    "other norm in a block": lambda m, mp: _layer_norm(m.layers[0], "ffn_norm"),
+    "other norm at the end": lambda m, mp: _layer_norm(m, "norm"),
+    "other block": lambda m, mp: m.layers.__setitem__(0, _Block()),
+    "other cache": lambda m, mp: setattr(m.layers[0].attention, "kv_cache", _Cache(m.layers[0].attention.kv_cache)),
+}
+
+
+@pytest.mark.parametrize("change", list(CHANGES))
+def test_changed_modules_run_as_modules(change, monkeypatch):
+    """A module that is not the plain one is called: the prompt gives what the module chain gives."""
+    model = _model("int4")
+    CHANGES[change](model, monkeypatch)
+    if change == "other block":  # the first block holds no cache any more
+        with torch.no_grad():
+            got = [model(*_prompt(model, 17))]
+            model.use_fused_decode = False
+            want = [model(*_prompt(model, 17))]
+    else:
+        got, want = _both(model, *_prompt(model, 17))
+    assert _same(got, want)
+
+
+@pytest.mark.parametrize("fmt", RECIPES)
+def test_plain_prompts_take_the_native_pass(fmt, monkeypatch):
+    from ao_amd import ops
+
+    seen, native = [], ops.host.llama_forward
+    monkeypatch.setattr(ops.host, "llama_forward", lambda *a: seen.append(native(*a)) or seen[-1])
+    model = _model(fmt)
+    with torch.no_grad():
+        out = model(*_prompt(model, 17))
+    assert len(seen) == 1 and seen[0] is out
