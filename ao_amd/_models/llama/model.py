@@ -202,6 +202,7 @@ class Transformer(nn.Module):
         self.output = nn.Linear(config.dim, config.vocab_size, bias=False)
         self.freqs_cis: Optional[Tensor] = None
         self.causal_mask: Optional[Tensor] = None
+        self._own_mask = None, 0  # the mask that setup_caches made, and its version then
         self.max_batch_size = -1
         self.max_seq_length = -1
         # single-token batch-1 steps go through the fused HIP decode path whenever the model qualifies
@@ -229,7 +230,9 @@ class Transformer(nn.Module):
                                            self.config.head_dim, dtype, device)
         self.freqs_cis = precompute_freqs_cis(self.config.block_size, self.config.head_dim, self.config.rope_base,
                                               dtype, device)
-        self.causal_mask = torch.tril(torch.ones(max_seq_length, max_seq_length, dtype=torch.bool, device=device))
+        with torch.inference_mode(False):  # an inference tensor has no version to compare
+            self.causal_mask = torch.tril(torch.ones(max_seq_length, max_seq_length, dtype=torch.bool, device=device))
+        self._own_mask = self.causal_mask, self.causal_mask._version
 
     def _decode_linears(self):
         linears = [self._modules["output"]]
@@ -291,9 +294,12 @@ class Transformer(nn.Module):
     def _prompt_is_the_module_chain(self) -> bool:
         """Whether calling module after module would compute what the native pass of a prompt computes: the modules and
         functions of this file, none subclassed (an adapter's linear), replaced (another norm or block), patched or watched by a
-        hook.  Read anew for every prompt, some 5 us a layer."""
+        hook, under the causal mask that setup_caches made.  Read anew for every prompt, some 5 us a layer."""
         hooks, cfg = torch.nn.modules.module, self.config
         if hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _chain_functions() != _CHAIN_FUNCTIONS:
+            return False
+        mask, version = self.__dict__.get("_own_mask", (None, 0))  # a model pickled by an earlier version has none
+        if mask is None or self.causal_mask is not mask or mask._version != version:
             return False
         if not (_is_plain(self.norm) and _is_plain(self.output)):
             return False

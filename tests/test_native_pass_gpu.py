@@ -104,6 +104,8 @@ CHANGES = {
     "patched attention function": lambda m, mp: mp.setattr(torch.nn.functional, "scaled_dot_product_attention", lambda q, k, v, **kw: q * 2),
     "other norm in a block": lambda m, mp: _layer_norm(m.layers[0], "ffn_norm"),
     "other norm at the end": lambda m, mp: _layer_norm(m, "norm"),
+    "other mask": lambda m, mp: setattr(m, "causal_mask", torch.ones_like(m.causal_mask)),
+    "mask changed in place": lambda m, mp: m.causal_mask.fill_(True),
     "other block": lambda m, mp: m.layers.__setitem__(0, _Block()),
     "other cache": lambda m, mp: setattr(m.layers[0].attention, "kv_cache", _Cache(m.layers[0].attention.kv_cache)),
 }
@@ -134,3 +136,18 @@ def test_plain_prompts_take_the_native_pass(fmt, monkeypatch):
     with torch.no_grad():
         out = model(*_prompt(model, 17))
     assert len(seen) == 1 and seen[0] is out
+
+
+def test_caches_made_in_inference_mode_take_the_native_pass(monkeypatch):
+    from ao_amd import ops
+
+    model = _model("int4", positions=32)
+    seen, native = [], ops.host.llama_forward
+    monkeypatch.setattr(ops.host, "llama_forward", lambda *a: seen.append(native(*a)) or seen[-1])
+    with torch.inference_mode():
+        model.setup_caches(1, 160)
+        model(*_prompt(model, 17))
+        assert torch.is_tensor(seen[-1])
+        model.causal_mask[3, 9] = True
+        model(*_prompt(model, 17))
+    assert len(seen) == 1
