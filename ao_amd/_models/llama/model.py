@@ -174,6 +174,18 @@ class TransformerBlock(nn.Module):
         return h + self.feed_forward(self.ffn_norm(h))
 
 
+# m.<name> without the cost of a module's attribute lookup where it is an ordinary parameter or child; a pruned or parametrized
+# module computes the attribute instead
+def _parameter(m: nn.Module, name: str):
+    p = m._parameters
+    return p[name] if name in p else getattr(m, name)
+
+
+def _child(m: nn.Module, name: str):
+    c = m._modules
+    return c[name] if name in c else getattr(m, name)
+
+
 def _chain_functions():
     return nn.Module.__call__, KVCache.update, apply_rotary_emb, F.scaled_dot_product_attention, F.silu
 
@@ -235,10 +247,10 @@ class Transformer(nn.Module):
         self._own_mask = self.causal_mask, self.causal_mask._version
 
     def _decode_linears(self):
-        linears = [self._modules["output"]]
+        linears = [_child(self, "output")]
         for b in self.layers:
-            att, ff = b._modules["attention"]._modules, b._modules["feed_forward"]._modules
-            linears += (att["wqkv"], att["wo"], ff["w1"], ff["w3"], ff["w2"])
+            att, ff = _child(b, "attention"), _child(b, "feed_forward")
+            linears += (_child(att, "wqkv"), _child(att, "wo"), _child(ff, "w1"), _child(ff, "w3"), _child(ff, "w2"))
         return linears
 
     def fused_decode_kind(self) -> Optional[str]:
@@ -259,8 +271,8 @@ class Transformer(nn.Module):
         for lin in self._decode_linears():
             if not isinstance(lin, nn.Linear):  # module-swapped layers (WeightOnlyInt4Linear, ...) run as modules
                 return None
-            w = lin._parameters["weight"]
-            if lin._parameters["bias"] is not None or not isinstance(w, AffineQuantizedTensor):
+            w = _parameter(lin, "weight")
+            if _parameter(lin, "bias") is not None or not isinstance(w, AffineQuantizedTensor):
                 return None
             with torch._C.DisableTorchFunctionSubclass():  # properties without a trip through __torch_function__ each
                 if w.dtype is not torch.bfloat16 or not w.is_cuda:
@@ -319,8 +331,7 @@ class Transformer(nn.Module):
 
     def _host_plan(self, kind: str, rows: int) -> tuple:
         """The model as csrc/host/llama.cpp reads it: nested tuples of the tensors that a pass of `rows` tokens needs.  Made
-        for every pass, so that replaced weights, caches and norms are seen; plain dictionary lookups keep that at a few us a
-        layer (an attribute of a module or a property of a tensor subclass costs several times that)."""
+        for every pass, so that replaced weights, caches and norms are seen."""
         from ... import ops
 
         cfg = self.config
@@ -328,7 +339,7 @@ class Transformer(nn.Module):
 
         def linear(lin):
             nonlocal ebits, mbits, group
-            w = lin._parameters["weight"]
+            w = _parameter(lin, "weight")
             if kind == "int4":
                 lay = w.layout_tensor
                 group, N, K = lay.group_size, lay.N, lay.K
@@ -343,13 +354,12 @@ class Transformer(nn.Module):
 
         layers = []
         for b in self.layers:
-            att, ff = b._modules["attention"], b._modules["feed_forward"]
-            an, fn, kv = b._modules["attention_norm"], b._modules["ffn_norm"], att.kv_cache
-            m, f = att._modules, ff._modules
+            att, ff = _child(b, "attention"), _child(b, "feed_forward")
+            an, fn, kv = _child(b, "attention_norm"), _child(b, "ffn_norm"), _child(att, "kv_cache")
             pair, pair_q = self._gate_up_pair(ff)[:2] if kind == "int4" and rows == 1 else (None, None)
-            layers.append((an._parameters["weight"], an.eps, linear(m["wqkv"]), linear(m["wo"]), kv._buffers["k_cache"],
-                           kv._buffers["v_cache"], fn._parameters["weight"], fn.eps, linear(f["w1"]), linear(f["w3"]),
-                           linear(f["w2"]), pair, pair_q))
+            layers.append((_parameter(an, "weight"), an.eps, linear(_child(att, "wqkv")), linear(_child(att, "wo")), kv.k_cache,
+                           kv.v_cache, _parameter(fn, "weight"), fn.eps, linear(_child(ff, "w1")), linear(_child(ff, "w3")),
+                           linear(_child(ff, "w2")), pair, pair_q))
         output = linear(self.output)
         ksplit = self.qkv_ksplit((cfg.n_head + 2 * cfg.n_local_heads) * cfg.head_dim)
         return (("int4", "int8", "fp6").index(kind), ebits, mbits, group, cfg.n_head, cfg.n_local_heads, ksplit,

@@ -290,3 +290,20 @@ def test_torchao_alias_package_resolves_to_this_library():
         if name.startswith("torchao.") and mod is not None:
             twin = sys.modules.get("ao_amd." + name[len("torchao."):])
             assert twin is None or twin is mod, name
+
+
+def test_pruned_and_parametrized_linears_run():
+    """Their weight is no entry of _parameters: prompts and decode steps run as modules."""
+    from torch.nn import utils
+    from torch.nn.utils import prune
+
+    from ao_amd._models.llama.model import Transformer
+
+    for change in (lambda lin: prune.l1_unstructured(lin, "weight", 0.2), utils.parametrizations.weight_norm):
+        model = Transformer.from_name("tiny128").bfloat16()
+        model.setup_caches(1, 32)
+        change(model.output)
+        change(model.layers[0].attention.wo)
+        with torch.no_grad():
+            for n in (3, 1):
+                assert model(torch.zeros(1, n, dtype=torch.int64), torch.arange(n)).shape == (1, n, 1024)

@@ -151,3 +151,20 @@ def test_caches_made_in_inference_mode_take_the_native_pass(monkeypatch):
         model.causal_mask[3, 9] = True
         model(*_prompt(model, 17))
     assert len(seen) == 1
+
+
+@pytest.mark.parametrize("fmt", ["int4", "int8"])
+def test_parametrized_weights_run(fmt):
+    """Weights that are no entries of _parameters any more: plain tensors that a parametrization puts together again."""
+    from ao_amd.utils import unwrap_tensor_subclass
+
+    model, plain = _model(fmt), _model(fmt)
+    unwrap_tensor_subclass(model)
+    assert "weight" not in model.output._parameters
+    assert _same(*_both(model, *_prompt(model, 17)))
+    step = torch.tensor([[3]], device="cuda"), torch.tensor([17], device="cuda")
+    with torch.no_grad():
+        for m in (model, plain):
+            for c in _caches(m):
+                c.fill_(0.5)
+        assert torch.equal(model(*step), plain(*step))
