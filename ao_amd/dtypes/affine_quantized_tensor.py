@@ -431,7 +431,7 @@ def _quantized_linear_op(input_tensor, weight_qtensor, bias):
             orig_dtype is torch.bfloat16
             and weight_qtensor.dtype is torch.bfloat16
             and layout.int_data.is_cuda
-            and weight_qtensor.shape[1] % 64 == 0
+            and weight_qtensor.shape[1] % 128 == 0
             and layout.int_data.stride(1) == 1 and layout.int_data.stride(0) % 16 == 0
         ):
             act = input_tensor.reshape(-1, orig_shape[-1])
@@ -441,8 +441,9 @@ def _quantized_linear_op(input_tensor, weight_qtensor, bias):
             if bias is not None and fused_bias is None:
                 y = y + bias
             return y.to(orig_dtype)
-        # other activation dtypes (the product is formed in the activation's dtype there) and in_features that are
-        # not a multiple of 64: the reference's own op sequence
+        # other activation dtypes (the product is formed in the activation's dtype there) and in_features that are not a
+        # multiple of 128: the reference's own op sequence, which takes empty batches and rows of any alignment and records a
+        # gradient.  Plain calls with in_features in multiples of 64 were served by _linear_on_host_path.
         y = torch.mm(input_tensor.reshape(-1, orig_shape[-1]), layout.int_data.t().to(orig_dtype)) * layout.scale
         y = y.reshape(*orig_shape[:-1], y.shape[-1])
         if bias is not None:

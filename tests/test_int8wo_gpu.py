@@ -296,3 +296,39 @@ def test_four_row_blocks_per_workgroup_kernel(M, N, K, bias):
     got = ops.int8wo_linear_gated(x, q, s, other).float().cpu().numpy()
     want = (torch.nn.functional.silu(other) * y).float().cpu().numpy()
     assert same_residual and np.count_nonzero(got != want) <= 0.002 * got.size + 1 and rel_l2(got, want) <= 1e-3
+
+
+def _linear_and_mm(K, N=48, bias=False):
+    """An int8 linear and the plain operator sequence it stands for."""
+    import ao_amd
+
+    lin = torch.nn.Linear(K, N, bias=bias, device="cuda", dtype=torch.bfloat16)
+    ao_amd.quantize_(lin, ao_amd.int8_weight_only())
+    lay = lin.weight.layout_tensor
+
+    def mm(x):
+        return (torch.mm(x.reshape(-1, K), lay.int_data.t().to(x.dtype)) * lay.scale).reshape(*x.shape[:-1], N)
+
+    return lin, mm
+
+
+@pytest.mark.parametrize("K", [64, 192])
+def test_half_tile_in_features_take_every_call(K):
+    """in_features that are an odd multiple of 64 ran torch.mm before the tiled kernel took the plain calls: empty batches, rows that
+    are not 16-byte aligned and gradients still do."""
+    lin, mm = _linear_and_mm(K)
+
+    def rows(n):
+        return torch.randn(n, device="cuda", dtype=torch.bfloat16)
+
+    with torch.no_grad():
+        assert lin(rows(0).view(0, K)).shape == (0, 48) and lin(rows(0).view(2, 0, K)).shape == (2, 0, 48)
+        for x in (rows(5 * K + 1)[1:].view(5, K), rows(5 * (K + 4)).view(5, K + 4)[:, :K], rows(5 * K).view(K, 5).t()):
+            assert torch.equal(lin(x), mm(x))
+    x, y = rows(5 * K).view(5, K), rows(5 * 48).view(5, 48)
+    grads = []
+    for f in (lin, mm):
+        xi = x.clone().requires_grad_()
+        f(xi).backward(y)
+        grads.append(xi.grad)
+    assert torch.equal(*grads)
