@@ -6,7 +6,7 @@
 // the other ran at the host's pace (4096 -> 1024, one row: 21.8 us a call for a 5.2 us kernel).
 //
 // Contract of every function here: it serves the plain case (exact torch.Tensor or Parameter arguments on one GPU,
-// dtypes, shapes and strides as the kernels take them, no gradient to record, no mode, transform or trace active) and
+// dtypes, shapes and strides as the kernels take them, no gradient or tangent to record, no mode, transform or trace active) and
 // returns NotImplemented for everything else *before* it does anything.  The caller then takes the torch.library route,
 // which reports errors, records for torch.compile, and covers the rare layouts.  Nothing is raised here.
 #pragma once
@@ -60,7 +60,8 @@ struct Args {
         const Tensor& t = THPVariable_Unpack(obj);
         if (!t.defined() || t.scalar_type() != dtype || !only(t.key_set(), plain) || !t.is_cuda()) return fail(none);
         if (device < 0) device = t.get_device();
-        if (t.get_device() != device || (grad && t.requires_grad())) return fail(none);
+        // a tangent of forward-mode differentiation is recorded whatever the gradient mode
+        if (t.get_device() != device || (grad && t.requires_grad()) || t._fw_grad(0).defined()) return fail(none);
         return t;
     }
     // Tensor of one of two 16-bit types

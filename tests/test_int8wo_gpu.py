@@ -332,3 +332,15 @@ def test_half_tile_in_features_take_every_call(K):
         f(xi).backward(y)
         grads.append(xi.grad)
     assert torch.equal(*grads)
+
+
+@pytest.mark.parametrize("grad_mode", [True, False])
+def test_half_tile_in_features_keep_forward_mode(grad_mode):
+    """The plain calls are declined where an argument carries a tangent."""
+    from torch.autograd import forward_ad
+
+    lin, mm = _linear_and_mm(192)
+    x, t = (torch.randn(5, 192, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    with torch.set_grad_enabled(grad_mode), forward_ad.dual_level():
+        got, want = (forward_ad.unpack_dual(f(forward_ad.make_dual(x, t))) for f in (lin, mm))
+    assert torch.equal(got.primal, want.primal) and torch.equal(got.tangent, want.tangent)
