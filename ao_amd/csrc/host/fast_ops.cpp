@@ -1,4 +1,6 @@
 // The quantized linears and the HQQ product on the native host path (contract and reasons: host.h).
+#include <ATen/autocast_mode.h>
+
 #include "host.h"
 
 using namespace ao_host;
@@ -65,6 +67,8 @@ PyObject* int8wo_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     const Rows r(x);
     AO_WANT(r.ok && w.dim() == 2 && w.size(1) == r.K && w.stride(1) == 1 && w.stride(0) % 16 == 0 && r.K % 64 == 0);
     const int64_t N = w.size(0);
+    // without the kernel an odd multiple of 64 runs torch.mm, which autocast casts; the operator of the others it leaves alone
+    AO_WANT(r.K % 128 == 0 || !at::autocast::is_autocast_enabled(at::kCUDA));
     AO_WANT(stands_for_bf16_matrix(v[4], N, r.K) && scale.numel() == N && scale.is_contiguous() && bias_ok(bias, N));
     return guarded([&]() -> PyObject* {
         Tensor y = empty_rows(x, N, at::kBFloat16), ws;

@@ -344,3 +344,12 @@ def test_half_tile_in_features_keep_forward_mode(grad_mode):
     with torch.set_grad_enabled(grad_mode), forward_ad.dual_level():
         got, want = (forward_ad.unpack_dual(f(forward_ad.make_dual(x, t))) for f in (lin, mm))
     assert torch.equal(got.primal, want.primal) and torch.equal(got.tangent, want.tangent)
+
+
+def test_half_tile_in_features_under_autocast():
+    """torch.mm casts there (fp16 product, fp32 after the scale); the result comes back in the activation's type."""
+    lin, mm = _linear_and_mm(192)
+    x = torch.randn(5, 192, device="cuda", dtype=torch.bfloat16)
+    with torch.no_grad(), torch.autocast("cuda"):
+        want = mm(x)
+        assert want.dtype is torch.float32 and torch.equal(lin(x), want.to(x.dtype))
