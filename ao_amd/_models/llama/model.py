@@ -263,9 +263,10 @@ class Transformer(nn.Module):
         if self.freqs_cis is None or self.max_batch_size != 1 or self.config.head_dim != 128 \
                 or self.max_seq_length > 16384:
             return None
-        if self.tok_embeddings.weight.dtype is torch.float16:
+        dtype = getattr(getattr(self.tok_embeddings, "weight", None), "dtype", None)  # an embedding of another kind may have none
+        if dtype is torch.float16:
             return "fp6" if self._fp6_decode_ready() else None
-        if self.tok_embeddings.weight.dtype is not torch.bfloat16:
+        if dtype is not torch.bfloat16:
             return None
         kinds, groups = set(), set()
         for lin in self._decode_linears():
@@ -363,7 +364,7 @@ class Transformer(nn.Module):
         output = linear(self.output)
         ksplit = self.qkv_ksplit((cfg.n_head + 2 * cfg.n_local_heads) * cfg.head_dim)
         return (("int4", "int8", "fp6").index(kind), ebits, mbits, group, cfg.n_head, cfg.n_local_heads, ksplit,
-                self.tok_embeddings.weight, self.freqs_cis, tuple(layers), self.norm.weight, self.norm.eps, output,
+                self.freqs_cis, tuple(layers), self.norm.weight, self.norm.eps, output,
                 self.max_seq_length)
 
     @staticmethod
@@ -419,13 +420,13 @@ class Transformer(nn.Module):
         ff = ops.int4wo_swiglu_interleaved(h, pair, pair_q, group, n_ff, b.ffn_norm.weight, b.ffn_norm.eps)
         return lin(ff, b.feed_forward.w2, h)
 
-    def _fused_decode(self, idx: Tensor, input_pos: Tensor) -> Tensor:
+    def _fused_decode(self, x: Tensor, input_pos: Tensor) -> Tensor:
         """One token, batch 1: five launches per layer, then norm + head.  Same roundings as the module-by-module
         path."""
         from ... import ops
 
         cfg = self.config
-        x = self.tok_embeddings(idx).view(1, cfg.dim)
+        x = x.view(1, cfg.dim)
         pos = input_pos.to(torch.int32) if input_pos.dtype is not torch.int32 else input_pos
         for b in self.layers:
             x = self._fused_layer(b, x, pos)
@@ -434,7 +435,7 @@ class Transformer(nn.Module):
                                            ow.group_size, ow.N)
         return logits.view(1, 1, cfg.vocab_size)
 
-    def _fused_decode_int8(self, idx: Tensor, input_pos: Tensor) -> Tensor:
+    def _fused_decode_int8(self, x: Tensor, input_pos: Tensor) -> Tensor:
         """The same step over int8 weight-only linears: the streaming int8 kernel per linear and the decode attention
         kernel, with each RMSNorm fused into the linears it feeds and the residual add and the SiLU(gate) * up product
         fused into the linear that precedes them; w1 and w3 stream in one launch (5 launches per layer)."""
@@ -452,7 +453,7 @@ class Transformer(nn.Module):
                 return ops.int8wo_linear_gated(x, lay.int_data, lay.scale.reshape(-1), gate)
             return ops.int8wo_linear(x, lay.int_data, lay.scale.reshape(-1))
 
-        x = self.tok_embeddings(idx).view(1, cfg.dim)
+        x = x.view(1, cfg.dim)
         pos = input_pos.to(torch.int32) if input_pos.dtype is not torch.int32 else input_pos
         for b in self.layers:
             att, ffn = b.attention, b.feed_forward
@@ -466,7 +467,7 @@ class Transformer(nn.Module):
             x = lin(act, ffn.w2, residual=h)
         return lin(x, self.output, norm=self.norm).view(1, 1, cfg.vocab_size)
 
-    def _fused_decode_fp6(self, idx: Tensor, input_pos: Tensor) -> Tensor:
+    def _fused_decode_fp6(self, x: Tensor, input_pos: Tensor) -> Tensor:
         """The same step over FPx weights on an fp16 model: the fp6 GEMV per linear with each RMSNorm fused into the
         staging of the linear it feeds, the residual add in the epilogue, w1 and w3 in one launch with the
         SiLU(gate) * up product, and the fp16 instance of the decode attention kernel (5 launches per layer)."""
@@ -480,7 +481,7 @@ class Transformer(nn.Module):
                 return ops.fp6_rmsnorm_linear(w.ebits, w.mbits, x, norm.weight, norm.eps, w.native(), w.scale)
             return ops.fp6_linear_native_fused(w.ebits, w.mbits, x, w.native(), w.scale, residual, False)
 
-        x = self.tok_embeddings(idx).view(1, cfg.dim)
+        x = x.view(1, cfg.dim)
         pos = input_pos.to(torch.int32) if input_pos.dtype is not torch.int32 else input_pos
         for b in self.layers:
             att, ffn = b.attention, b.feed_forward
@@ -498,26 +499,26 @@ class Transformer(nn.Module):
         from ... import ops
 
         assert self.freqs_cis is not None, "Caches must be initialized first"
+        x = self.tok_embeddings(idx)
         if self.use_fused_decode and input_pos is not None and idx.dim() == 2 and idx.shape[0] == 1 \
                 and not torch.compiler.is_dynamo_compiling():
             # every launch of the pass from one native call; it declines what it does not take before it launches anything
             kind = self.fused_decode_kind() if idx.numel() == 1 or self._prompt_is_the_module_chain() else None
             if kind is not None:
                 pos = input_pos.to(torch.int32) if idx.numel() == 1 and input_pos.dtype is not torch.int32 else input_pos
-                logits = ops.host.llama_forward(self._host_plan(kind, idx.numel()), idx, pos)
+                logits = ops.host.llama_forward(self._host_plan(kind, idx.numel()), x, pos)
                 if logits is not NotImplemented:
                     return logits
         if self.use_fused_decode and idx.numel() == 1 and input_pos is not None and input_pos.numel() == 1:
             kind = self.fused_decode_kind()
             if kind == "int4":
-                return self._fused_decode(idx, input_pos)
+                return self._fused_decode(x, input_pos)
             if kind == "int8":
-                return self._fused_decode_int8(idx, input_pos)
+                return self._fused_decode_int8(x, input_pos)
             if kind == "fp6":
-                return self._fused_decode_fp6(idx, input_pos)
+                return self._fused_decode_fp6(x, input_pos)
         mask = self.causal_mask[None, None, input_pos]
         freqs_cis = self.freqs_cis[input_pos]
-        x = self.tok_embeddings(idx)
         for layer in self.layers:
             x = layer(x, input_pos, freqs_cis, mask)
         return self.output(self.norm(x))

@@ -35,7 +35,7 @@ struct Model {
     int kind = INT4, ebits = 0, mbits = 0;
     int64_t group = 0, n_head = 0, n_kv = 0, dim = 0, max_seq = 0, ksplit = 1;
     at::ScalarType dtype = at::kBFloat16;
-    Tensor embeddings, freqs, norm;
+    Tensor freqs, norm;
     double eps = 0;
     Linear output;
     std::vector<Layer> layers;
@@ -129,24 +129,23 @@ Model read_model(Args& a, PyObject* tuple) {
     m.n_kv = r.integer();
     m.ksplit = r.integer();
     if (m.kind == FP6) m.dtype = at::kHalf;
-    m.embeddings = r.tensor(m.dtype);
     m.freqs = r.tensor(m.dtype);
     PyObject* layers = r.next();
     m.norm = r.tensor(m.dtype);
     m.eps = r.real();
     PyObject* output = r.next();
     m.max_seq = r.integer();
-    if (!a.ok || m.kind > FP6 || m.n_kv < 1 || m.n_head % m.n_kv || m.embeddings.dim() != 2 || !m.embeddings.is_contiguous() ||
-        m.freqs.dim() != 3 || m.freqs.size(0) < m.max_seq || m.freqs.size(1) != 64 || m.freqs.size(2) != 2 || !m.freqs.is_contiguous()) {
+    if (!a.ok || m.kind > FP6 || m.n_kv < 1 || m.n_head % m.n_kv || m.freqs.dim() != 3 || m.freqs.size(0) < m.max_seq ||
+        m.freqs.size(1) != 64 || m.freqs.size(2) != 2 || !m.freqs.is_contiguous()) {
         a.ok = false;
         return m;
     }
-    m.dim = m.embeddings.size(1);
     m.output = read_linear(m, a, output);
+    m.dim = m.output.K;
     Reader ls(a, layers);
     m.layers.reserve(ls.n);
     for (Py_ssize_t i = 0; i < ls.n && a.ok; ++i) m.layers.push_back(read_layer(m, a, ls.next()));
-    a.ok = a.ok && m.dim % 8 == 0 && m.dim <= 8192 && is_row(m.norm, m.dim) && m.output.K == m.dim;
+    a.ok = a.ok && m.dim % 8 == 0 && m.dim <= 8192 && is_row(m.norm, m.dim);
     return m;
 }
 
@@ -313,27 +312,26 @@ struct Pass {
 
 }  // namespace
 
-// (plan, tokens int32 or int64 [1, T], positions [T]: int32 for T = 1, else int32 or int64) -> logits [1, T, vocab]
+// (plan, embedded tokens [1, T, dim], positions [T]: int32 for T = 1, else int32 or int64) -> logits [1, T, vocab].  The caller looks
+// the tokens up through the model's embedding module: it may be another one, and its kernel refuses a token outside the table.
 PyObject* llama_forward(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     AO_NEED(3);
-    auto index_dtype = [&](PyObject* o) {
-        return THPVariable_CheckExact(o) && THPVariable_Unpack(o).defined() && THPVariable_Unpack(o).scalar_type() == at::kLong ? at::kLong : at::kInt;
-    };
-    const Tensor &tokens = a.tensor(1, index_dtype(v[1])), &pos = a.tensor(2, index_dtype(v[2]));
-    AO_WANT(a.ok && current(a.device));
-    const int64_t T = tokens.numel();
-    AO_WANT(T >= 1 && tokens.dim() == 2 && tokens.size(0) == 1 && tokens.is_contiguous() && pos.dim() == 1 && pos.numel() == T &&
-            pos.is_contiguous() && (T > 1 || pos.scalar_type() == at::kInt));
+    at::ScalarType dtype;
+    const Tensor& x = a.tensor16(1, dtype);
+    const bool is_long = THPVariable_CheckExact(v[2]) && THPVariable_Unpack(v[2]).defined() && THPVariable_Unpack(v[2]).scalar_type() == at::kLong;
+    const Tensor& pos = a.tensor(2, is_long ? at::kLong : at::kInt);
+    AO_WANT(a.ok && current(a.device) && x.dim() == 3 && x.size(0) == 1 && x.is_contiguous() &&
+            (uintptr_t)ptr(x) % 16 == 0);
+    const int64_t T = x.size(1);
+    AO_WANT(T >= 1 && pos.dim() == 1 && pos.numel() == T && pos.is_contiguous() && (T > 1 || pos.scalar_type() == at::kInt));
     // Autocast changes the types between the modules of a prompt (it clears a key that is excluded otherwise, so nothing_watches()
     // does not see it); a decode step is made of operators that it leaves alone.
     AO_WANT(T == 1 || !at::autocast::is_autocast_enabled(at::kCUDA));
     return guarded([&]() -> PyObject* {
         const Model m = read_model(a, v[0]);
-        AO_WANT(a.ok);
+        AO_WANT(a.ok && dtype == m.dtype && x.size(2) == m.dim);
         Pass p{m, a.device, stream_of(a.device)};
-        Tensor x = p.alloc(T, m.dim), logits;
-        AO_CALL(ao_amd_llama_embed(ptr(tokens), tokens.scalar_type() == at::kLong, T, ptr(m.embeddings), m.embeddings.size(0), m.dim,
-                                   x.data_ptr(), p.st));
+        Tensor logits;
         AO_WANT(T == 1 ? p.decode(x, pos, logits) : p.prefill(x, pos, T, logits));
         return THPVariable_Wrap(logits.view({1, T, m.output.N}));
     });

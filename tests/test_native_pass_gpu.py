@@ -168,3 +168,35 @@ def test_parametrized_weights_run(fmt):
             for c in _caches(m):
                 c.fill_(0.5)
         assert torch.equal(model(*step), plain(*step))
+
+
+class _Table(torch.nn.Module):
+    def __init__(self, like):
+        super().__init__()
+        self.table, self.calls = like.weight, 0
+
+    def forward(self, idx):
+        self.calls += 1
+        return torch.nn.functional.embedding(idx, self.table) * 2
+
+
+@pytest.mark.parametrize("fmt", RECIPES)
+@pytest.mark.parametrize("kind", ["hook", "weight", "no weight"])
+def test_the_embedding_module_is_called(fmt, kind):
+    """Once for a prompt or a decode step, whatever module it is: it refuses tokens outside its table."""
+    model, plain = _model(fmt), _model(fmt)
+    with torch.no_grad():
+        plain.tok_embeddings.weight.mul_(2)
+    seen = []
+    if kind == "hook":
+        model.tok_embeddings.register_forward_hook(lambda m, i, o: seen.append(1) or o * 2)
+    else:
+        model.tok_embeddings = table = _Table(model.tok_embeddings)
+        if kind == "weight":
+            table.weight = table.table
+    with torch.no_grad():
+        for call in (_prompt(model, 17), (torch.tensor([[3]], device="cuda"), torch.tensor([17], device="cuda"))):
+            if kind == "no weight":  # nothing says the type of the model: modules
+                plain.use_fused_decode = False
+            assert torch.equal(model(*call), plain(*call))
+    assert (len(seen) if kind == "hook" else table.calls) == 2
