@@ -114,12 +114,12 @@ class AoAmdError(RuntimeError):
 
 
 def lib():
-    """The loaded C-ABI library.  Raises if it has not been built (python -m ao_amd._build)."""
+    """The loaded C-ABI library.  Raises if it has not been built (python ao_amd/_build.py)."""
     global _lib
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise ImportError(
-                f"{LIB_PATH} is missing: the HIP kernels are not built. Run `python -m ao_amd._build` "
+                f"{LIB_PATH} is missing: the HIP kernels are not built. Run `python ao_amd/_build.py` "
                 "(hipcc, gfx950). ao_amd has no CPU or eager fallback."
             )
         handle = ctypes.CDLL(LIB_PATH)
@@ -144,7 +144,7 @@ def _load_host():
 
     if not os.path.exists(HOST_PATH):
         if os.path.exists(LIB_PATH):
-            raise ImportError(f"{HOST_PATH} is missing while {LIB_PATH} is there: run `python -m ao_amd._build`")
+            raise ImportError(f"{HOST_PATH} is missing while {LIB_PATH} is there: run `python ao_amd/_build.py`")
         return _NoHost()
     loader = importlib.machinery.ExtensionFileLoader("ao_amd_host", HOST_PATH)
     module = importlib.util.module_from_spec(importlib.util.spec_from_loader("ao_amd_host", loader))

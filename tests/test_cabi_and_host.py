@@ -307,3 +307,19 @@ def test_pruned_and_parametrized_linears_run():
         with torch.no_grad():
             for n in (3, 1):
                 assert model(torch.zeros(1, n, dtype=torch.int64), torch.arange(n)).shape == (1, n, 1024)
+
+
+def test_build_runs_in_a_tree_with_the_libraries_of_an_earlier_build(tmp_path):
+    """Such a tree may not import (here the host module is missing): building must not need the package."""
+    import shutil
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    shutil.copytree(os.path.join(root, "ao_amd"), tmp_path / "ao_amd", ignore=shutil.ignore_patterns("lib", "csrc", "__pycache__"))
+    shutil.copy(os.path.join(root, "__graft_entry__.py"), tmp_path)
+    (tmp_path / "ao_amd" / "lib").mkdir()
+    (tmp_path / "ao_amd" / "lib" / "libao_amd.so").touch()
+    (tmp_path / "ao_amd" / "_build.py").write_text("def build(verbose):\n    raise SystemExit(7)\n")
+    run = subprocess.run([sys.executable, "-c", "import __graft_entry__ as g; g.build()"], cwd=tmp_path, capture_output=True, text=True)
+    assert run.returncode == 7, run.stderr
