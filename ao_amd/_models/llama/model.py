@@ -215,6 +215,7 @@ class Transformer(nn.Module):
         self.freqs_cis: Optional[Tensor] = None
         self.causal_mask: Optional[Tensor] = None
         self._own_mask = None, 0  # the mask that setup_caches made, and its version then
+        self._cache_rows: Optional[Tensor] = None  # 0 .. max_seq_length - 1
         self.max_batch_size = -1
         self.max_seq_length = -1
         # single-token batch-1 steps go through the fused HIP decode path whenever the model qualifies
@@ -245,6 +246,7 @@ class Transformer(nn.Module):
         with torch.inference_mode(False):  # an inference tensor has no version to compare
             self.causal_mask = torch.tril(torch.ones(max_seq_length, max_seq_length, dtype=torch.bool, device=device))
         self._own_mask = self.causal_mask, self.causal_mask._version
+        self._cache_rows = torch.arange(max_seq_length, dtype=torch.int32, device=device)
 
     def _decode_linears(self):
         linears = [_child(self, "output")]
@@ -365,7 +367,7 @@ class Transformer(nn.Module):
         ksplit = self.qkv_ksplit((cfg.n_head + 2 * cfg.n_local_heads) * cfg.head_dim)
         return (("int4", "int8", "fp6").index(kind), ebits, mbits, group, cfg.n_head, cfg.n_local_heads, ksplit,
                 self.freqs_cis, tuple(layers), self.norm.weight, self.norm.eps, output,
-                self.max_seq_length)
+                self.max_seq_length, self.__dict__.get("_cache_rows"))
 
     @staticmethod
     def qkv_ksplit(n_rows: int, n_cu: int = 256) -> int:

@@ -5,6 +5,7 @@
 // The caller describes the model as nested tuples of tensors and numbers (Transformer._host_plan); they are checked
 // completely before the first launch.
 #include <ATen/autocast_mode.h>
+#include <ATen/ops/index.h>
 #include <ATen/ops/linear.h>
 #include <ATen/ops/mul.h>
 
@@ -35,7 +36,7 @@ struct Model {
     int kind = INT4, ebits = 0, mbits = 0;
     int64_t group = 0, n_head = 0, n_kv = 0, dim = 0, max_seq = 0, ksplit = 1;
     at::ScalarType dtype = at::kBFloat16;
-    Tensor freqs, norm;
+    Tensor freqs, norm, cache_rows;
     double eps = 0;
     Linear output;
     std::vector<Layer> layers;
@@ -135,8 +136,10 @@ Model read_model(Args& a, PyObject* tuple) {
     m.eps = r.real();
     PyObject* output = r.next();
     m.max_seq = r.integer();
+    m.cache_rows = r.tensor(at::kInt);
     if (!a.ok || m.kind > FP6 || m.n_kv < 1 || m.n_head % m.n_kv || m.freqs.dim() != 3 || m.freqs.size(0) < m.max_seq ||
-        m.freqs.size(1) != 64 || m.freqs.size(2) != 2 || !m.freqs.is_contiguous()) {
+        m.freqs.size(1) != 64 || m.freqs.size(2) != 2 || !m.freqs.is_contiguous() || m.cache_rows.dim() != 1 ||
+        m.cache_rows.size(0) != m.max_seq) {
         a.ok = false;
         return m;
     }
@@ -279,7 +282,11 @@ struct Pass {
     }
 
     // ---- several rows
-    bool prefill(Tensor x, const Tensor& pos, int64_t T, Tensor& logits) {
+    bool prefill(Tensor x, const Tensor& input_pos, int64_t T, Tensor& logits) {
+        // torch's indexing, as in the module chain: it refuses a position outside the cache or the rotary table and counts a negative
+        // one from the end of each
+        const c10::List<std::optional<Tensor>> at_pos({std::optional<Tensor>(input_pos)});
+        const Tensor pos = at::index(m.cache_rows, at_pos), freqs = at::index(m.freqs, at_pos);
         Tensor n = alloc(T, m.dim);
         const Layer* first = m.layers.empty() ? nullptr : &m.layers[0];
         const Tensor& w0 = first ? first->attn_norm : m.norm;
@@ -293,9 +300,8 @@ struct Pass {
             const float next_eps = (float)(end ? m.eps : m.layers[i + 1].attn_eps);
             Tensor qkv, y = alloc(T, m.n_head * 128), o, gate, up, down;
             if (!linear(l.wqkv, n, T, qkv)) return false;
-            AO_TRY(ao_amd_llama_prefill_attention(ptr(qkv), f16, ptr(m.freqs), ptr(pos), pos.scalar_type() == at::kLong, T,
-                                                  l.k_cache.data_ptr(), l.v_cache.data_ptr(), (int)m.n_head, (int)m.n_kv, 128, m.max_seq,
-                                                  y.data_ptr(), st));
+            AO_TRY(ao_amd_llama_prefill_attention_rows(ptr(qkv), f16, ptr(freqs), ptr(pos), 0, T, l.k_cache.data_ptr(), l.v_cache.data_ptr(),
+                                                       (int)m.n_head, (int)m.n_kv, 128, m.max_seq, y.data_ptr(), st));
             if (!linear(l.wo, y, T, o)) return false;
             Tensor h = alloc(T, m.dim), hn = alloc(T, m.dim);
             AO_TRY(ao_amd_add_rmsnorm(ptr(x), ptr(o), ptr(l.ffn_norm), f16, T, m.dim, (float)l.ffn_eps, h.data_ptr(), hn.data_ptr(), st));

@@ -52,11 +52,11 @@ __device__ __forceinline__ uint4 rotate8(uint4 x, uint4 cs) {
 }
 
 // Keys rotated and values as they are, into row input_pos[t] of the caches.  One thread per 8 elements; a row outside the
-// cache is not written.
+// cache is not written.  The (cos, sin) pairs are rows of the whole table, or already gathered, one row a token.
 template <class E>
 __global__ __launch_bounds__(256) void prefill_cache_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ freqs,
-                                                            const void* __restrict__ pos, int pos_is_i64, int T, int n_head,
-                                                            int n_kv, int64_t S, uint16_t* __restrict__ k_cache,
+                                                            bool freqs_by_row, const void* __restrict__ pos, int pos_is_i64, int T,
+                                                            int n_head, int n_kv, int64_t S, uint16_t* __restrict__ k_cache,
                                                             uint16_t* __restrict__ v_cache) {
     const int per_row = 2 * n_kv * 16;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(256) void prefill_cache_kernel(const uint16_t* __re
     const int head = c >> 4, d = (c & 15) * 8;
     const uint4 x = *(const uint4*)(qkv + ((int64_t)t * (n_head + 2 * n_kv) + n_head + head) * 128 + d);
     if (head < n_kv)
-        *(uint4*)(k_cache + ((int64_t)head * S + p) * 128 + d) = rotate8<E>(x, *(const uint4*)(freqs + p * 128 + d));
+        *(uint4*)(k_cache + ((int64_t)head * S + p) * 128 + d) = rotate8<E>(x, *(const uint4*)(freqs + (freqs_by_row ? t : p) * 128 + d));
     else
         *(uint4*)(v_cache + ((int64_t)(head - n_kv) * S + p) * 128 + d) = x;
 }
@@ -93,8 +93,8 @@ __global__ __launch_bounds__(256) void prefill_cache_kernel(const uint16_t* __re
 // Llama-3-8B widths, 1000 positions: 56 -> 35 us.
 template <class E, bool HEADS>
 __global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ freqs,
-                                                                const void* __restrict__ pos, int pos_is_i64, int T, int n_head,
-                                                                int n_kv, int64_t S, const uint16_t* __restrict__ k_cache,
+                                                                bool freqs_by_row, const void* __restrict__ pos, int pos_is_i64,
+                                                                int T, int n_head, int n_kv, int64_t S, const uint16_t* __restrict__ k_cache,
                                                                 const uint16_t* __restrict__ v_cache, uint16_t* __restrict__ out) {
     typedef Mfma32<E> MM;
     __shared__ uint4 lds[2][2][2][64 * 16];   // [group][K / V][buffer]
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* 
         if (p >= 0 && p < S && row < T) last = (int)p;
     }
     uint4 q[8];
-    const int64_t frow = last < 0 ? 0 : last;
+    const int64_t frow = freqs_by_row ? srow : last < 0 ? 0 : last;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
         const int d = 16 * s + 8 * half;
@@ -371,19 +371,47 @@ __global__ __launch_bounds__(256) void embed_kernel(const void* __restrict__ tok
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-// Llama-3-8B widths (32 query heads over 8 KV heads), 1000 positions of a 1128-position cache.
+struct PrefillAttention {
+    const uint16_t *qkv, *freqs;
+    bool freqs_by_row;
+    const void* pos;
+    int pos_is_i64;
+    int64_t T;
+    uint16_t *k_cache, *v_cache;
+    int n_head, n_kv;
+    int64_t S;
+    uint16_t* out;
+};
+
 template <class E>
-static void prefill_attention(const uint16_t* qkv, const uint16_t* freqs, const void* pos, int pos_is_i64, int T, int n_head, int n_kv,
-                              int64_t S, uint16_t* kc, uint16_t* vc, uint16_t* out, hipStream_t st) {
-    const int64_t chunks = (int64_t)T * 2 * n_kv * 16;
-    hipLaunchKernelGGL(prefill_cache_kernel<E>, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, qkv, freqs, pos, pos_is_i64, T,
-                       n_head, n_kv, S, kc, vc);
-    if (n_head / n_kv % 4 == 0)
-        hipLaunchKernelGGL((prefill_attention_kernel<E, true>), dim3(n_head / 4, (T + 31) / 32), dim3(512), 0, st, qkv, freqs, pos,
-                           pos_is_i64, T, n_head, n_kv, S, kc, vc, out);
+static void prefill_attention(const PrefillAttention& a, hipStream_t st) {
+    const int T = (int)a.T;
+    const int64_t chunks = a.T * 2 * a.n_kv * 16;
+    hipLaunchKernelGGL(prefill_cache_kernel<E>, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, a.qkv, a.freqs, a.freqs_by_row,
+                       a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache);
+    if (a.n_head / a.n_kv % 4 == 0)
+        hipLaunchKernelGGL((prefill_attention_kernel<E, true>), dim3(a.n_head / 4, (T + 31) / 32), dim3(512), 0, st, a.qkv, a.freqs,
+                           a.freqs_by_row, a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache, a.out);
     else
-        hipLaunchKernelGGL((prefill_attention_kernel<E, false>), dim3(n_head, (T + 127) / 128), dim3(512), 0, st, qkv, freqs, pos,
-                           pos_is_i64, T, n_head, n_kv, S, kc, vc, out);
+        hipLaunchKernelGGL((prefill_attention_kernel<E, false>), dim3(a.n_head, (T + 127) / 128), dim3(512), 0, st, a.qkv, a.freqs,
+                           a.freqs_by_row, a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache, a.out);
+}
+
+static int prefill_attention_entry(const PrefillAttention& a, int is_f16, int head_dim, void* stream) {
+    AO_REQUIRE(a.qkv && a.freqs && a.pos && a.k_cache && a.v_cache && a.out, "null pointer argument");
+    AO_REQUIRE(head_dim == 128, "prefill attention is built for head_dim 128, got %d", head_dim);
+    AO_REQUIRE(a.n_kv > 0 && a.n_head > 0 && a.n_head % a.n_kv == 0, "n_head=%d must be a multiple of n_kv=%d", a.n_head, a.n_kv);
+    AO_REQUIRE(a.n_head <= 65535 && a.T >= 0 && a.T <= 1 << 20 && a.S > 0 && a.S <= 1 << 20, "T=%lld, max_seq=%lld out of range",
+               (long long)a.T, (long long)a.S);
+    AO_REQUIRE(aligned16(a.qkv) && aligned16(a.freqs) && aligned16(a.k_cache) && aligned16(a.v_cache) && aligned16(a.out),
+               "16-byte aligned tensors needed");
+    if (a.T == 0) return 0;
+    if (is_f16)
+        prefill_attention<ElemF16>(a, (hipStream_t)stream);
+    else
+        prefill_attention<ElemBf16>(a, (hipStream_t)stream);
+    AO_LAUNCH_CHECK();
+    return 0;
 }
 
 }  // namespace ao
@@ -393,22 +421,15 @@ using namespace ao;
 extern "C" int ao_amd_llama_prefill_attention(const void* qkv, int is_f16, const void* freqs_cis, const void* positions, int pos_is_i64,
                                               int64_t T, void* k_cache, void* v_cache, int n_head, int n_kv, int head_dim,
                                               int64_t max_seq, void* out, void* stream) {
-    AO_REQUIRE(qkv && freqs_cis && positions && k_cache && v_cache && out, "null pointer argument");
-    AO_REQUIRE(head_dim == 128, "prefill attention is built for head_dim 128, got %d", head_dim);
-    AO_REQUIRE(n_kv > 0 && n_head > 0 && n_head % n_kv == 0, "n_head=%d must be a multiple of n_kv=%d", n_head, n_kv);
-    AO_REQUIRE(n_head <= 65535 && T >= 0 && T <= 1 << 20 && max_seq > 0 && max_seq <= 1 << 20, "T=%lld, max_seq=%lld out of range",
-               (long long)T, (long long)max_seq);
-    AO_REQUIRE(aligned16(qkv) && aligned16(freqs_cis) && aligned16(k_cache) && aligned16(v_cache) && aligned16(out),
-               "16-byte aligned tensors needed");
-    if (T == 0) return 0;
-    if (is_f16)
-        prefill_attention<ElemF16>((const uint16_t*)qkv, (const uint16_t*)freqs_cis, positions, pos_is_i64, (int)T, n_head, n_kv, max_seq,
-                                   (uint16_t*)k_cache, (uint16_t*)v_cache, (uint16_t*)out, (hipStream_t)stream);
-    else
-        prefill_attention<ElemBf16>((const uint16_t*)qkv, (const uint16_t*)freqs_cis, positions, pos_is_i64, (int)T, n_head, n_kv, max_seq,
-                                    (uint16_t*)k_cache, (uint16_t*)v_cache, (uint16_t*)out, (hipStream_t)stream);
-    AO_LAUNCH_CHECK();
-    return 0;
+    return prefill_attention_entry({(const uint16_t*)qkv, (const uint16_t*)freqs_cis, false, positions, pos_is_i64, T, (uint16_t*)k_cache,
+                                    (uint16_t*)v_cache, n_head, n_kv, max_seq, (uint16_t*)out}, is_f16, head_dim, stream);
+}
+
+extern "C" int ao_amd_llama_prefill_attention_rows(const void* qkv, int is_f16, const void* freqs_rows, const void* positions,
+                                                   int pos_is_i64, int64_t T, void* k_cache, void* v_cache, int n_head, int n_kv,
+                                                   int head_dim, int64_t max_seq, void* out, void* stream) {
+    return prefill_attention_entry({(const uint16_t*)qkv, (const uint16_t*)freqs_rows, true, positions, pos_is_i64, T, (uint16_t*)k_cache,
+                                    (uint16_t*)v_cache, n_head, n_kv, max_seq, (uint16_t*)out}, is_f16, head_dim, stream);
 }
 
 extern "C" int ao_amd_add_rmsnorm(const void* x, const void* y, const void* weight, int is_f16, int64_t rows, int64_t dim, float eps,

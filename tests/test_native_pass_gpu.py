@@ -200,3 +200,27 @@ def test_the_embedding_module_is_called(fmt, kind):
                 plain.use_fused_decode = False
             assert torch.equal(model(*call), plain(*call))
     assert (len(seen) if kind == "hook" else table.calls) == 2
+
+
+@pytest.mark.parametrize("fmt", ["int4", "fp6"])
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_negative_positions_count_from_the_end(fmt, dtype):
+    """As indexing has it: from the end of the cache for the row, from the end of the rotary table for the angle.  Both paths take the
+    same steps with sums in another order (3e-2 as for the decode steps; the caches of the first layer see one linear: 2^-8)."""
+    model = _model(fmt)
+    tokens, _ = _prompt(model, 5)
+    got, want = _both(model, tokens, torch.tensor([3, -1, 7, -160, 159 - 64], device="cuda", dtype=dtype))
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert (a.float() - b.float()).norm() <= (3e-2 if i in (0, 3, 4) else 2 ** -8) * b.float().norm()
+        assert torch.equal(a == 0, b == 0) if i in (1, 2) else not a.isnan().any()
+
+
+def test_prompts_pass_the_range_checks_of_indexing():
+    """Tokens go through torch's embedding kernel and positions through its indexing, which refuse what is out of range."""
+    model = _model("int8")
+    call = _prompt(model, 9)
+    with torch.no_grad(), torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        model(*call)
+    count = {e.key: e.count for e in prof.key_averages()}
+    assert count.get("aten::embedding") == 1 and count.get("aten::index") == 2
+    assert not any(k.startswith("torchao::") for k in count)  # the native pass, not the modules

@@ -144,3 +144,25 @@ def test_native_pass_is_the_module_chain(quantization, T):
     model.use_fused_decode = False
     for a, b in zip(got, both()):
         assert a.shape == b.shape and a.dtype is b.dtype and _rel(a, b) <= 3e-2
+
+
+@pytest.mark.parametrize("T", [1, 33, 130])
+@pytest.mark.parametrize("heads", [(4, 1), (3, 3)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_attention_with_gathered_rotary_rows(T, heads, dtype):
+    """The entry that takes one rotary row a token: bit for bit the other one on the gathered rows; a position outside the cache
+    reads its row and no other."""
+    from ao_amd._models.llama.model import precompute_freqs_cis
+
+    n_head, n_kv = heads
+    S = 160
+    qkv = _qkv(T, n_head, n_kv, dtype)
+    freqs = precompute_freqs_cis(S, 128, dtype=dtype, device="cuda")
+    pos = torch.randperm(S, device="cuda", generator=torch.Generator(device="cuda").manual_seed(T))[:T]
+    results = []
+    for name, f in (("ao_amd_llama_prefill_attention", freqs), ("ao_amd_llama_prefill_attention_rows", freqs[pos])):
+        kc, vc = (torch.ones(n_kv, S, 128, device="cuda", dtype=dtype) for _ in range(2))
+        out = torch.full((T, n_head * 128), 7.0, device="cuda", dtype=dtype)
+        _call(name, qkv, int(dtype is torch.float16), f, pos, 1, T, kc, vc, n_head, n_kv, 128, S, out)
+        results.append((out, kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*results)) and not results[0][0].isnan().any()
