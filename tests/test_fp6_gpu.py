@@ -308,3 +308,17 @@ def test_native_to_fp16_is_the_scaled_weight_and_feeds_the_two_pass_linear(oracl
     monkeypatch.setattr(ops, "fp6_two_pass", lambda M, N, K: False)
     y_small = ops.fp6_linear_native(e, m, x[:64], native, scale).float().cpu().numpy()   # fused kernel, same rows
     assert rel_l2(y[:64], y_small) <= 1e-3
+
+
+@pytest.mark.parametrize("K,other", [(256, 192), (192, 256), (128, 64)])
+def test_activations_of_another_width_are_refused(K, other):
+    """Also where both widths fill the same number of 128-column tiles."""
+    import ao_amd
+
+    lin = torch.nn.Linear(K, 256, bias=False, device="cuda", dtype=torch.float16)
+    ao_amd.quantize_(lin, ao_amd.fp6_llm_weight_only())
+    with torch.no_grad():
+        assert lin(torch.randn(4, K, device="cuda", dtype=torch.float16)).shape == (4, 256)
+        for shape in ((5, other), ()):
+            with pytest.raises(RuntimeError):
+                lin(torch.randn(shape, device="cuda", dtype=torch.float16))
