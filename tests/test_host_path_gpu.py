@@ -89,3 +89,75 @@ def test_calls_that_others_have_to_see_are_declined():
     assert call(packed=packed[:2]) is NotImplemented      # fewer row blocks than N asks for
     assert call(bias=torch.zeros(n - 1, device="cuda", dtype=torch.bfloat16)) is NotImplemented
     assert torch.func.vmap(lambda r: torch.tensor(call(x=r[None]) is NotImplemented))(x).all()
+
+
+def _plain_calls():
+    """(function, arguments, index of the activations) of a call that each function serves."""
+    import ao_amd
+    from ao_amd import ops
+    from ao_amd._models.llama.generate import build_random_model
+    from ao_amd.prototype.hqq.mixed_mm import pack_2xint4
+
+    def weight(recipe, dtype):
+        lin = torch.nn.Linear(256, 256, bias=False, device="cuda", dtype=dtype)
+        ao_amd.quantize_(lin, recipe)
+        return lin.weight
+
+    def x(dtype):
+        return torch.randn(2, 256, device="cuda", dtype=dtype)
+
+    w8, w6 = weight(ao_amd.int8_weight_only(), torch.bfloat16), weight(ao_amd.fp6_llm_weight_only(), torch.float16)
+    codes = pack_2xint4(torch.randint(0, 16, (256, 256), dtype=torch.uint8, device="cuda"))
+    q = [torch.rand(4, 256, device="cuda", dtype=torch.bfloat16) for _ in range(2)]
+    model = build_random_model("tiny128", torch.device("cuda"), "int4wo-64")
+    model.setup_caches(1, 64)
+    rows = torch.randn(1, 5, 512, device="cuda", dtype=torch.bfloat16)
+    packed, qparams = _int4(64, 256)
+    return {
+        "int4wo_linear": ([x(torch.bfloat16), packed, qparams, 64, 64, 256, None, None], 0),
+        "int8wo_linear": ([x(torch.bfloat16), w8.layout_tensor.int_data, w8.layout_tensor.scale, None, None], 0),
+        "fp6_linear": ([3, 2, x(torch.float16), w6.native(), w6.scale], 2),
+        "hqq_mixed_mm": ([x(torch.bfloat16), codes, *q, 64, False], 0),
+        "llama_forward": ([model._host_plan("int4", 5), rows, torch.arange(5, device="cuda")], 1),
+    }
+
+
+@pytest.mark.parametrize("name", ["int4wo_linear", "int8wo_linear", "fp6_linear", "hqq_mixed_mm", "llama_forward"])
+def test_every_function_declines_what_others_have_to_see(name):
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from ao_amd import ops
+
+    args, i = _plain_calls()[name]
+
+    def call(x=args[i]):
+        return getattr(ops.host, name)(*args[:i], x, *args[i + 1:])
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatches(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Subclass(torch.Tensor):
+        pass
+
+    with torch.no_grad():
+        assert torch.is_tensor(call())
+        for mode in (Functions(), Dispatches(), FakeTensorMode()):
+            with mode:
+                assert call() is NotImplemented
+        x = args[i]
+        with forward_ad.dual_level():
+            assert call(forward_ad.make_dual(x, x)) is NotImplemented
+        assert torch.func.vmap(lambda r: torch.tensor(call(r) is NotImplemented))(x[None]).all()
+        for other in (x.cpu(), x.float(), x.transpose(-1, -2), x.as_subclass(Subclass), x[..., :128], None, 3):
+            assert call(other) is NotImplemented
+    if name != "llama_forward":  # its norms are parameters that ask for a gradient
+        assert torch.is_tensor(call())
+    assert call(x.clone().requires_grad_()) is NotImplemented

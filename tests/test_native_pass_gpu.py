@@ -8,18 +8,18 @@ pytestmark = pytest.mark.gpu
 RECIPES = ("int4", "int8", "fp6")
 
 
-def _model(fmt, layers=2, intermediate=1024, positions=160, block_size=512, seed=0):
+def _model(fmt, layers=2, intermediate=1024, positions=160, block_size=512, seed=0, heads=(4, 2), group=64):
     from ao_amd import fp6_llm_weight_only, int4_weight_only, int8_weight_only, quantize_
     from ao_amd._models.llama.generate import random_init_
     from ao_amd._models.llama.model import ModelArgs, Transformer
 
-    args = ModelArgs(block_size=block_size, n_layer=layers, n_head=4, n_local_heads=2, dim=512, intermediate_size=intermediate,
-                     vocab_size=1024)
+    args = ModelArgs(block_size=block_size, n_layer=layers, n_head=heads[0], n_local_heads=heads[1], dim=128 * heads[0],
+                     intermediate_size=intermediate, vocab_size=1024)
     with torch.device("cuda"):
         model = Transformer(args).to(torch.bfloat16)
     random_init_(model, seed=seed)
     model = model.eval().to(torch.float16 if fmt == "fp6" else torch.bfloat16)
-    quantize_(model, {"int4": lambda: int4_weight_only(64), "int8": int8_weight_only, "fp6": fp6_llm_weight_only}[fmt]())
+    quantize_(model, {"int4": lambda: int4_weight_only(group), "int8": int8_weight_only, "fp6": fp6_llm_weight_only}[fmt]())
     model.setup_caches(1, positions)
     return model
 
@@ -224,3 +224,66 @@ def test_prompts_pass_the_range_checks_of_indexing():
     count = {e.key: e.count for e in prof.key_averages()}
     assert count.get("aten::embedding") == 1 and count.get("aten::index") == 2
     assert not any(k.startswith("torchao::") for k in count)  # the native pass, not the modules
+
+
+def _call(name, *args):
+    from ao_amd import _lib
+
+    args = [a.data_ptr() if torch.is_tensor(a) else a for a in args]
+    _lib.check(getattr(_lib.lib(), name)(*args, _lib.current_stream(torch.device("cuda"))))
+
+
+def _linear(lin, x):
+    w, op = lin.weight, torch.ops.torchao
+    if hasattr(w, "fpx_data"):
+        return op.fp6_linear_native.default(w.ebits, w.mbits, x, w.native(), w.scale)
+    lay = w.layout_tensor
+    if hasattr(lay, "packed_weight"):
+        return op.int4wo_linear.default(x, lay.packed_weight, lay.scale_and_zero, lay.group_size, lay.N, None, False)
+    return op.int8wo_linear.default(x, lay.int_data, lay.scale, None, False)
+
+
+def _composed(model, tokens, pos):
+    """The prompt kernel by kernel: logits and caches."""
+    cfg, T = model.config, tokens.numel()
+    f16 = int(model.freqs_cis.dtype is torch.float16)
+    x = model.tok_embeddings(tokens).view(T, -1)
+    n = torch.empty_like(x)
+    blocks = list(model.layers)
+    _call("ao_amd_rmsnorm_f16" if f16 else "ao_amd_rmsnorm_bf16", x, blocks[0].attention_norm.weight, T, cfg.dim, cfg.norm_eps, n)
+    for b, after in zip(blocks, [b.attention_norm for b in blocks[1:]] + [model.norm]):
+        kv, y = b.attention.kv_cache, torch.empty_like(x)
+        _call("ao_amd_llama_prefill_attention", _linear(b.attention.wqkv, n), f16, model.freqs_cis, pos, 1, T, kv.k_cache, kv.v_cache,
+              cfg.n_head, cfg.n_local_heads, 128, model.max_seq_length, y)
+        h, hn = torch.empty_like(x), torch.empty_like(x)
+        _call("ao_amd_add_rmsnorm", x, _linear(b.attention.wo, y), b.ffn_norm.weight, f16, T, cfg.dim, cfg.norm_eps, h, hn)
+        gate, up = _linear(b.feed_forward.w1, hn), _linear(b.feed_forward.w3, hn)
+        _call("ao_amd_silu_mul", gate, up, f16, gate.numel(), gate)
+        x, n = torch.empty_like(x), torch.empty_like(x)
+        _call("ao_amd_add_rmsnorm", h, _linear(b.feed_forward.w2, gate), after.weight, f16, T, cfg.dim, cfg.norm_eps, x, n)
+    return [_linear(model.output, n).view(1, T, -1)] + [c.clone() for c in _caches(model)]
+
+
+# Short prompts on every kind of product, and the lengths at which the weight goes through a 16-bit copy and the library product.
+# 1088 and 2112 in_features, and 640 in groups of 256, end before the packed width.
+@pytest.mark.parametrize("fmt,T,intermediate,heads,group", [(f, T, 1024, (4, 2), 64) for f in RECIPES for T in (2, 17, 33, 130)] +
+                         [("int4", T, 1088, (4, 1), 64) for T in (17, 130)] +
+                         [("int4", 4096, 2048, (4, 2), 64), ("int4", 4096, 2112, (5, 1), 256), ("int8", 1536, 8192, (4, 2), 0),
+                          ("fp6", 1537, 8192, (4, 2), 0)])
+def test_native_pass_is_its_kernels(fmt, T, intermediate, heads, group, monkeypatch):
+    """Bit for bit the operators and kernels it is made of, each of which has a test of its own: no rounding, operand or route differs."""
+    from ao_amd import ops
+
+    model = _model(fmt, 2, intermediate, max(T, 160), 4096, 0, heads, group)
+    tokens, pos = _prompt(model, T)
+    seen, native = [], ops.host.llama_forward
+    monkeypatch.setattr(ops.host, "llama_forward", lambda plan, *a: seen.append(plan) or native(plan, *a))
+    with torch.no_grad():
+        got = [model(tokens, pos)] + [c.clone() for c in _caches(model)]
+        for c in _caches(model):
+            c.zero_()
+        want = _composed(model, tokens, pos)
+    assert _same(got, want) and not want[0].isnan().any()
+    (plan,) = seen
+    two_pass = [lin[4] for layer in plan[8] for lin in layer if isinstance(lin, tuple)]
+    assert any(two_pass) == (T >= 1536)

@@ -166,3 +166,25 @@ def test_attention_with_gathered_rotary_rows(T, heads, dtype):
         _call(name, qkv, int(dtype is torch.float16), f, pos, 1, T, kc, vc, n_head, n_kv, 128, S, out)
         results.append((out, kc, vc))
     assert all(torch.equal(a, b) for a, b in zip(*results)) and not results[0][0].isnan().any()
+
+
+@pytest.mark.parametrize("T,heads", [(1025, (8, 2)), (4096, (4, 1)), (2049, (3, 3))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_long_attention_matches_fp32(T, heads, dtype):
+    """As test_attention_matches_fp32, over 17 to 65 tiles of positions; one query head at a time in fp32."""
+    from ao_amd._models.llama.model import apply_rotary_emb, precompute_freqs_cis
+
+    n_head, n_kv = heads
+    qkv = _qkv(T, n_head, n_kv, dtype)
+    freqs = precompute_freqs_cis(T, 128, dtype=dtype, device="cuda")
+    pos = torch.arange(T, device="cuda")
+    kc, vc = (torch.zeros(n_kv, T, 128, device="cuda", dtype=dtype) for _ in range(2))
+    out = torch.empty(T, n_head * 128, device="cuda", dtype=dtype)
+    _call("ao_amd_llama_prefill_attention", qkv, int(dtype is torch.float16), freqs, pos, 1, T, kc, vc, n_head, n_kv, 128, T, out)
+    q = apply_rotary_emb(qkv.view(1, T, -1, 128)[:, :, :n_head], freqs)[0].float()
+    later = torch.ones(T, T, device="cuda", dtype=torch.bool).triu(1)
+    for h in range(n_head):
+        kv = h * n_kv // n_head
+        s = (q[:, h] @ kc[kv].float().t().contiguous() / math.sqrt(128)).masked_fill_(later, float("-inf"))
+        want = s.softmax(-1) @ vc[kv].float()
+        assert _rel(out.view(T, n_head, 128)[:, h], want) <= (2 ** -8 if dtype is torch.bfloat16 else 2 ** -11)
