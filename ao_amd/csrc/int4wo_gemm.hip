@@ -703,14 +703,18 @@ static bool gemm_kwave_plan(const LinearArgs& a, int64_t g, GemmLdsPlan* p) {
     return tiles >= 192 && tiles <= 1024;
 }
 
-bool int4wo_gemm_lds_plan(const LinearArgs& a, int64_t g, char* out, size_t cap) {
+// Fills the plan and returns true where one of this file's kernels takes the problem; the name of the one whose waves split K
+// stands for its 96- and its 128-row tiles
+bool int4wo_gemm_lds_plan(const LinearArgs& a, int64_t g, Int4Plan* plan) {
     GemmLdsPlan p;
     if (gemm_lds_plan(a, g, &p)) {
-        snprintf(out, cap, "int4wo_gemm_lds_kernel<%lld,%d>", (long long)g, p.nt);
+        plan->kernel = p.nt == 1 ? Int4Kernel::lds_256x128 : Int4Kernel::lds_256x256;
+        if (plan->name) snprintf(plan->name, plan->cap, "int4wo_gemm_lds_kernel<%lld,%d>", (long long)g, p.nt);
         return true;
     }
     if (gemm_kwave_plan(a, g, &p)) {
-        snprintf(out, cap, "int4wo_gemm_kwave_kernel<%lld>", (long long)g);
+        plan->kernel = Int4Kernel::kwave;
+        if (plan->name) snprintf(plan->name, plan->cap, "int4wo_gemm_kwave_kernel<%lld>", (long long)g);
         return true;
     }
     return false;

@@ -138,6 +138,18 @@ inline void launch_timed(Kernel kernel, dim3 grid, dim3 block, size_t smem, hipS
     hipLaunchKernelGGL(kernel, grid, block, smem, st, a);
 }
 
+// What the linear's dispatch decides for a problem: the kernel as the rules know it (int4wo_tile.hip prices it against its own
+// tiles) and, where `name` is not null, its instantiation in words (ao_amd_int4wo_linear_plan).
+enum class Int4Kernel { streaming, tiles, tiles_128x128, kwave, lds_256x128, lds_256x256 };
+struct Int4Plan {
+    Int4Kernel kernel;
+    char* name;
+    size_t cap;
+};
+// For plain operands: aligned rows of the packed width, bf16 output, no fused operand.  Answers without a launch; false for a
+// problem that the dispatch refuses.
+bool int4wo_plain_kernel(int64_t M, int64_t K, int64_t N, int64_t g, Int4Kernel* kernel);
+
 // Single-row GEMV on the 4x4x4 matrix instructions (int4wo_gemv1.hip).  Returns true when it took the launch;
 // false when the shape is outside what it handles (the caller then uses the general kernels).
 bool launch_int4wo_gemv1(const LinearArgs& a, int64_t g, int64_t RB, hipStream_t st);
@@ -152,7 +164,7 @@ bool int4wo_gemv2_plan(const LinearArgs& a, int64_t g, int64_t RB, char* out, si
 
 // Prefill GEMM with the weight tile dequantized once per workgroup into LDS (int4wo_gemm.hip); same contract as above.
 bool launch_int4wo_gemm_lds(const LinearArgs& a, int64_t g, hipStream_t st);
-bool int4wo_gemm_lds_plan(const LinearArgs& a, int64_t g, char* out, size_t cap);
+bool int4wo_gemm_lds_plan(const LinearArgs& a, int64_t g, Int4Plan* plan);
 // Its 256 x 128 nt tiles with K split over a.ksplit workgroups: a.y takes fp32 parts [ksplit][M][ldy], no bias.  K is the packed
 // width, every part has at least 8 of the 64-wide steps and a.ksplit is at most 4 (no part is empty then).
 void launch_int4wo_gemm_lds_parts(const LinearArgs& a, int64_t g, int nt, hipStream_t st);

@@ -1141,12 +1141,13 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
                            const void* packed2, const void* qparams2, int64_t N, int64_t g, const void* bias_bf16,
                            const void* residual_bf16, int64_t ldres, void* y, int y_dtype, int64_t ldy, void* stream,
                            const void* norm_weight_bf16 = nullptr, float norm_eps = 0.f, bool pair8 = false,
-                           int ksplit = 1, char* plan_out = nullptr, size_t plan_cap = 0) {
-    // plan_out: do not launch; write the name of the kernel the arguments select (ao_amd_int4wo_linear_plan)
-#define AO_PLAN(...)                                    \
-    if (plan_out) {                                     \
-        snprintf(plan_out, plan_cap, __VA_ARGS__);      \
-        return 0;                                       \
+                           int ksplit = 1, Int4Plan* plan = nullptr) {
+    // plan: do not launch; say which kernel the arguments select
+#define AO_PLAN(which, ...)                                             \
+    if (plan) {                                                         \
+        plan->kernel = which;                                           \
+        if (plan->name) snprintf(plan->name, plan->cap, __VA_ARGS__);   \
+        return 0;                                                       \
     }
     // pair8: `packed` / `qparams` hold 2 * N rows (gate and up rows interleaved in eights), the output has N columns
     const int64_t n_out = N;
@@ -1245,10 +1246,8 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
     if ((M > 16 || ws_tiles) && aligned && !dual && !residual_bf16 && !norm_weight_bf16 &&
         (ws_tiles || (!gemm_starved && !rb4_two_blocks))) {
         if (!ws_tiles) {
-            char name[96];
-            if (int4wo_gemm_lds_plan(a, g, name, sizeof(name))) {
-                AO_PLAN("%s", name);
-                launch_int4wo_gemm_lds(a, g, st);
+            if (plan && int4wo_gemm_lds_plan(a, g, plan)) return 0;
+            if (!plan && launch_int4wo_gemm_lds(a, g, st)) {
                 AO_LAUNCH_CHECK();
                 return 0;
             }
@@ -1266,7 +1265,8 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
         // each group has 2 or more K tiles; the 64-row tiles (192 or more workgroups, which already overlap each other)
         // from 64 K tiles on (K = 14336, 512 rows: -4 %; K = 4096: +4 % and therefore not split)
         const bool ksplit_tiles = ws_tiles || (!big && KB_all >= (tiny ? 8 : 64));
-        AO_PLAN("%s<%lld,%d,%d>", (!big && ksplit_tiles) ? "int4wo_gemm_ksplit_kernel" : "int4wo_gemm_kernel", (long long)g,
+        AO_PLAN(big ? Int4Kernel::tiles_128x128 : Int4Kernel::tiles, "%s<%lld,%d,%d>",
+                (!big && ksplit_tiles) ? "int4wo_gemm_ksplit_kernel" : "int4wo_gemm_kernel", (long long)g,
                 big ? 2 : (tiny && ksplit_tiles ? 2 : (tiny ? 1 : (ksplit_tiles ? 4 : 1))),
                 big ? 8 : (tiny && ksplit_tiles ? 4 : (tiny ? 2 : 4)));
 #define AO_GEMM_LAUNCH(GG)                                                                                     \
@@ -1289,13 +1289,13 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
     if (M == 1 && aligned && !dual) {
         char name[96];
         if (int4wo_gemv2_plan(a, g, RB, name, sizeof(name))) {
-            AO_PLAN("%s", name);
+            AO_PLAN(Int4Kernel::streaming, "%s", name);
             if (!launch_int4wo_gemv2(a, g, RB, st)) return -2;
             AO_LAUNCH_CHECK();
             return 0;
         }
         if (int4wo_gemv1_plan(a, g, RB, name, sizeof(name))) {
-            AO_PLAN("%s", name);
+            AO_PLAN(Int4Kernel::streaming, "%s", name);
             launch_int4wo_gemv1(a, g, RB, st);
             AO_LAUNCH_CHECK();
             return 0;
@@ -1319,8 +1319,8 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
             // two activation blocks (140 registers): beyond one workgroup per CU, three 4-wave workgroups share a CU
             // where 8-wave ones would queue (28672 x 4096 at 24-32 rows: 32 -> 25.5 us)
             if (mb >= 2 && wgs > 256) w4 = 4;
-            if (mb == 1) AO_PLAN("int4wo_linear_rb4_kernel<%lld,%d>", (long long)g, w4);
-            AO_PLAN("int4wo_linear_rb4_kernel<%lld,%d,%d>", (long long)g, w4, mb);
+            if (mb == 1) AO_PLAN(Int4Kernel::streaming, "int4wo_linear_rb4_kernel<%lld,%d>", (long long)g, w4);
+            AO_PLAN(Int4Kernel::streaming, "int4wo_linear_rb4_kernel<%lld,%d,%d>", (long long)g, w4, mb);
             const dim3 grid4((unsigned)(RB / 4), (unsigned)mch);
             auto go = [&](auto kernel, int nw) {
                 if (g_prof_start && g_prof_stop) {
@@ -1349,7 +1349,7 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
             return 0;
         }
     }
-    AO_PLAN("%s<%lld,%d,%s%d>", xmode == X_LDS ? "int4wo_gemv_kernel" : "int4wo_linear_kernel", (long long)g, waves,
+    AO_PLAN(Int4Kernel::streaming, "%s<%lld,%d,%s%d>", xmode == X_LDS ? "int4wo_gemv_kernel" : "int4wo_linear_kernel", (long long)g, waves,
             xmode == X_LDS ? "" : (xmode == X_GLOBAL ? "X_GLOBAL," : "X_CHECKED,"), dual ? 1 : 0);
 #undef AO_PLAN
     dim3 grid((unsigned)RB, (unsigned)mchunks, (unsigned)ksplit);
@@ -1365,6 +1365,17 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
     }
     AO_LAUNCH_CHECK();
     return 0;
+}
+
+bool int4wo_plain_kernel(int64_t M, int64_t K, int64_t N, int64_t g, Int4Kernel* kernel) {
+    // aligned addresses that are never dereferenced
+    const void* p = reinterpret_cast<const void*>((uintptr_t)8192);
+    Int4Plan plan{Int4Kernel::streaming, nullptr, 0};
+    if (linear_dispatch(p, M, K, K, p, p, nullptr, nullptr, N, g, nullptr, nullptr, 0, const_cast<void*>(p), AO_BF16, N, nullptr, nullptr, 0.f,
+                        false, 1, &plan) != 0)
+        return false;
+    *kernel = plan.kernel;
+    return true;
 }
 
 }  // namespace ao
@@ -1385,9 +1396,10 @@ extern "C" int ao_amd_int4wo_linear_plan(int64_t M, int64_t K, int64_t N, int64_
     const void* p = reinterpret_cast<const void*>(aligned ? (uintptr_t)4096 : (uintptr_t)4098);
     const void* w = reinterpret_cast<const void*>((uintptr_t)8192);
     out[0] = 0;
+    Int4Plan plan{Int4Kernel::streaming, out, (size_t)out_cap};
     return linear_dispatch(p, M, K, K, w, w, dual ? w : nullptr, dual ? w : nullptr, N, g, nullptr, has_residual ? w : nullptr,
                            pair8 ? 2 * N : N, const_cast<void*>(w), y_dtype, N, nullptr, has_norm ? w : nullptr, 1e-5f,
-                           pair8 != 0, ksplit, out, (size_t)out_cap);
+                           pair8 != 0, ksplit, &plan);
 }
 
 extern "C" int ao_amd_int4wo_linear(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed,

@@ -95,26 +95,24 @@ static TilePlan int4wo_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts)
 // us of the kernel that ao_amd_int4wo_linear(_ws) runs, by measurement at 33 to 1000 rows on 16 weights from 768 x 1024 to 28672 x
 // 8192; 0 where it is not one of the tile kernels (few rows: the weight is streamed).
 static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
-    char name[96] = "";
-    if (ao_amd_int4wo_linear_plan(M, K, N, g, 1, 0, 0, 0, 0, 1, AO_BF16, name, sizeof(name)) != 0) return 0.0;
+    Int4Kernel kernel;
+    if (!int4wo_plain_kernel(M, K, N, g, &kernel) || kernel == Int4Kernel::streaming) return 0.0;
     const double k = (double)K / 4096.0;
     auto rounds = [&](int bm, int bn) { return (double)((M + bm - 1) / bm * ((N + bn - 1) / bn)) / 256.0; };
     auto up = [](double r) { return (double)(int64_t)(r + 255.0 / 256.0); };
-    if (!strncmp(name, "int4wo_gemm_lds_kernel", 22)) {
-        const bool wide = strstr(name, ",2>") != nullptr;
+    if (kernel == Int4Kernel::lds_256x256 || kernel == Int4Kernel::lds_256x128) {
         const double rw = rounds(256, 256);
-        if (wide) return 6.0 + 100.0 * k * (rw < 1.0 ? 0.4 + 0.6 * rw : up(rw));   // CUs that run at once slow each other down
+        if (kernel == Int4Kernel::lds_256x256) return 6.0 + 100.0 * k * (rw < 1.0 ? 0.4 + 0.6 * rw : up(rw));   // CUs that run at once slow each other down
         const double r = rounds(256, 128), full = (double)(int64_t)r, rest = r - full;
         return 14.0 + k * (52.5 * full + (rest == 0.0 ? 0.0 : full > 0.0 && rest <= 0.5 ? 28.0 : 52.5));
     }
-    if (!strncmp(name, "int4wo_gemm_kwave_kernel", 24)) {
+    if (kernel == Int4Kernel::kwave) {
         const double r = up(rounds(128, 64));
         const bool three = (M + 95) / 96 == (M + 127) / 128;   // its 96-row tiles
         return 6.0 + (three ? (r > 1.0 ? 17.5 : 16.5) : r > 1.0 ? 20.0 : 18.5) * k * r;
     }
-    if (strncmp(name, "int4wo_gemm_", 12)) return 0.0;
     if (ao_amd_int4wo_linear_ws_parts(M, K, N, g) > 1) return M <= 64 ? 0.0 : 4.0 + 8.0 * k;
-    if (strstr(name, ",2,8>")) return 90.0 * k * rounds(128, 128) / 2.0;
+    if (kernel == Int4Kernel::tiles_128x128) return 90.0 * k * rounds(128, 128) / 2.0;
     if (rounds(64, 64) >= 0.75) return 5.0 + (K >= 8192 ? 14.0 : 18.0) * k * up(rounds(64, 64));
     return 4.0 + 10.4 * k * up(rounds(32, 64));
 }

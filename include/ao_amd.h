@@ -141,7 +141,8 @@ int ao_amd_int4wo_rmsnorm_swiglu(const void* x_bf16, int64_t M, int64_t K, int64
                                  const void* qparams_up, int64_t N, int64_t g, void* y_bf16, int64_t ldy, void* stream);
 
 /* Which kernel instantiation the int4 linear entry points above run for a problem, without launching anything: writes a
- * name such as "int4wo_gemm_ksplit_kernel<64,4,4>" or "int4wo_gemv1_kernel<4,2,0> wpr=4" to `out`.  `aligned`: K is a
+ * name such as "int4wo_gemm_ksplit_kernel<64,4,4>" or "int4wo_gemv1_kernel<4,2,0> wpr=4" to `out` ("int4wo_gemm_kwave_kernel"
+ * stands for its 96- and its 128-row tiles).  `aligned`: K is a
  * multiple of max(128, g) and the activation rows are 16-byte aligned; the other flags say which fused variant is meant
  * (residual epilogue, RMSNorm on the activations, two weights, interleaved gate/up weight, K split).  The test suite walks
  * the dispatch with it so that no instantiation ships without a test that reaches it.  No counterpart in the reference

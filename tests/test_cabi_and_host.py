@@ -323,3 +323,23 @@ def test_build_runs_in_a_tree_with_the_libraries_of_an_earlier_build(tmp_path):
     (tmp_path / "ao_amd" / "_build.py").write_text("def build(verbose):\n    raise SystemExit(7)\n")
     run = subprocess.run([sys.executable, "-c", "import __graft_entry__ as g; g.build()"], cwd=tmp_path, capture_output=True, text=True)
     assert run.returncode == 7, run.stderr
+
+
+def test_int4_tiled_product_is_priced_against_every_tile_kernel(cabi):
+    """One shape per kernel it competes with at which it is the faster one, and the ones at which it is not; the rule reads the
+    dispatch's decision, no kernel's name."""
+
+    def offered(M, K, N):
+        need = ctypes.c_int64(-2)
+        cabi.check(cabi.lib().ao_amd_int4wo_linear_tiled_bytes(M, K, N, 64, ctypes.byref(need)))
+        return need.value >= 0
+
+    for shape, rival in (((160, 4096, 14336), "int4wo_gemm_kwave_kernel<64>"), ((384, 4096, 14336), "int4wo_gemm_lds_kernel<64,1>"),
+                         ((256, 4096, 4096), "int4wo_gemm_kernel<64,1,4>"), ((48, 4096, 11008), "int4wo_gemm_ksplit_kernel<64,2,4>"),
+                         ((96, 28672, 8192), "int4wo_gemm_ksplit_kernel<64,4,4>")):
+        M, K, N = shape
+        assert cabi.int4wo_linear_plan(M, K, N, 64) == rival and offered(*shape), shape
+    for shape in ((32, 4096, 14336), (128, 4096, 14336), (1000, 4096, 14336), (900, 8192, 8192)):
+        assert not offered(*shape), shape
+    with open(os.path.join(os.path.dirname(cabi.__file__), "csrc", "int4wo_tile.hip")) as f:
+        assert not re.search(r"\bstr(n?cmp|str)\b", f.read())
