@@ -594,6 +594,11 @@ static bool tiled(int64_t M, int64_t N, int64_t K, bool workspace) {
     return M > (workspace && K >= 8192 && (N <= 8192 || N >= 24576) ? 8 : 16);
 }
 
+// Per-lane offsets within a tile are 32 bits wide: rows further apart than that keep the streaming kernels.
+static bool tiles_reach(int64_t M, int64_t N, int64_t ldx, int64_t ldw) {
+    return 192 * ldx * 2 < ((int64_t)1 << 32) && 256 * ldw < ((int64_t)1 << 32) && M * N < ((int64_t)1 << 40);
+}
+
 static int int8wo_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* w_int8, int64_t ldw, const void* scale_bf16,
                         int64_t N, const void* bias_bf16, void* y, int64_t ldy, const void* residual, int64_t ldres, const void* gate,
                         int64_t ldgate, float* workspace, int64_t workspace_bytes, void* stream) {
@@ -605,8 +610,7 @@ static int int8wo_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, c
                (long long)ldx, (long long)ldw, (long long)ldy);
     AO_REQUIRE((((uintptr_t)x_bf16) & 15) == 0 && (ldx & 7) == 0 && (((uintptr_t)w_int8) & 15) == 0 && (ldw & 15) == 0,
                "activation and weight rows must be 16-byte aligned");
-    // per-lane offsets within a tile are 32 bits wide
-    AO_REQUIRE(192 * ldx * 2 < ((int64_t)1 << 32) && 256 * ldw < ((int64_t)1 << 32) && M * N < ((int64_t)1 << 40), "operands too large");
+    AO_REQUIRE(tiles_reach(M, N, ldx, ldw), "operands too large");
     TilePlan p = int8wo_gemm_plan(M, N, K, 8);
     if (p.parts > 1 && (!workspace || workspace_bytes < p.parts * M * N * (int64_t)sizeof(float))) p = int8wo_gemm_plan(M, N, K, 1);
     launch_int8wo_gemm(TileGemmArgs{(const uint16_t*)x_bf16, M, K, ldx, (const uint8_t*)w_int8, ldw, scale_bf16,
@@ -642,7 +646,8 @@ extern "C" int ao_amd_int8wo_linear_ws(const void* x_bf16, int64_t M, int64_t K,
                                        const void* scale_bf16, int64_t N, const void* bias_bf16, void* y, int y_dtype, int64_t ldy,
                                        void* workspace, int64_t workspace_bytes, void* stream) {
     AO_REQUIRE(!workspace || (((uintptr_t)workspace) & 15) == 0, "the workspace must be 16-byte aligned");
-    if (y_dtype == AO_BF16 && K % 64 == 0 && tiled(M, N, K, workspace != nullptr))
+    // (in_features that are an odd multiple of 64 have no other kernel)
+    if (y_dtype == AO_BF16 && K % 64 == 0 && tiled(M, N, K, workspace != nullptr) && (K % 128 != 0 || tiles_reach(M, N, ldx, ldw)))
         return int8wo_tiled(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, ldy, nullptr, 0, nullptr, 0, (float*)workspace, workspace_bytes, stream);
     return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, y_dtype, ldy, nullptr, 0, nullptr, 0, stream);
 }
@@ -658,7 +663,7 @@ extern "C" int ao_amd_int8wo_linear_residual(const void* x_bf16, int64_t M, int6
                                              int64_t ldw, const void* scale_bf16, int64_t N, const void* residual_bf16,
                                              int64_t ldres, void* y_bf16, int64_t ldy, void* stream) {
     AO_REQUIRE(residual_bf16, "null pointer argument");
-    if (K % 128 == 0 && tiled(M, N, K, false))
+    if (K % 128 == 0 && tiled(M, N, K, false) && tiles_reach(M, N, ldx, ldw))
         return int8wo_tiled(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, ldy, residual_bf16, ldres, nullptr, 0, nullptr, 0,
                             stream);
     return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, AO_BF16, ldy, residual_bf16, ldres,
@@ -669,7 +674,7 @@ extern "C" int ao_amd_int8wo_linear_gated(const void* x_bf16, int64_t M, int64_t
                                           int64_t ldw, const void* scale_bf16, int64_t N, const void* gate_bf16,
                                           int64_t ldgate, void* y_bf16, int64_t ldy, void* stream) {
     AO_REQUIRE(gate_bf16, "null pointer argument");
-    if (K % 128 == 0 && tiled(M, N, K, false))
+    if (K % 128 == 0 && tiled(M, N, K, false) && tiles_reach(M, N, ldx, ldw))
         return int8wo_tiled(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, ldy, nullptr, 0, gate_bf16, ldgate, nullptr, 0,
                             stream);
     return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, nullptr, y_bf16, AO_BF16, ldy, nullptr, 0, gate_bf16,

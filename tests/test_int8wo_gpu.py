@@ -353,3 +353,20 @@ def test_half_tile_in_features_under_autocast():
     with torch.no_grad(), torch.autocast("cuda"):
         want = mm(x)
         assert want.dtype is torch.float32 and torch.equal(lin(x), want.to(x.dtype))
+
+
+def test_rows_that_are_far_apart():
+    """A row stride beyond the 32-bit offsets of the tiles (22 MB) is streamed, as every batch was before there were tiles."""
+    from ao_amd import ops
+
+    M, N, K, stride = 36, 4096, 4096, 11184816
+    g = torch.Generator(device="cuda").manual_seed(5)
+    w = torch.randint(-128, 128, (N, K), device="cuda", dtype=torch.int8, generator=g)
+    scale = torch.rand(N, device="cuda", generator=g).bfloat16()
+    x = torch.empty((M - 1) * stride + K, device="cuda", dtype=torch.bfloat16).as_strided((M, K), (stride, 1))
+    x.normal_(generator=g)
+    other = torch.randn(M, N, device="cuda", generator=g).bfloat16()
+    want = (x.float() @ w.float().t().contiguous()).bfloat16() * scale
+    # each side sums exact products in fp32 and rounds twice to bf16: within a step (2^-8) each
+    for got, ref in ((ops.int8wo_linear(x, w, scale), want), (ops.int8wo_linear_residual(x, w, scale, other), want + other)):
+        assert (got.float() - ref.float()).norm() <= 2 ** -7 * ref.float().norm()
