@@ -56,6 +56,8 @@ _SIGNATURES = {
     "ao_amd_fp6_linear_tiled_bytes": ([_i64, _i64, _i64, _i64p], _int),
     "ao_amd_fp6_linear_tiled_plan": ([_i64, _i64, _i64, ctypes.c_char_p, _i64], _int),
     "ao_amd_fp6_linear_tiled": ([_p, _i64, _i64, _p, _p, _i64, _int, _int, _p, _p, _i64, _p], _int),
+    "ao_amd_fp6_linear_auto_bytes": ([_i64, _i64, _i64, _i64p], _int),
+    "ao_amd_fp6_linear_auto": ([_p, _i64, _i64, _p, _p, _i64, _int, _int, _p, _p, _i64, _p], _int),
     "ao_amd_fp6_linear_ws_parts": ([_i64, _i64, _i64], _int),
     "ao_amd_fp6_linear_ws": ([_p, _i64, _i64, _p, _p, _i64, _int, _int, _p, _p, _i64, _p], _int),
     "ao_amd_fp6_rmsnorm_linear": ([_p, _i64, _i64, _p, ctypes.c_float, _p, _p, _i64, _int, _int, _p, _p], _int),
@@ -77,6 +79,8 @@ _SIGNATURES = {
     "ao_amd_int4wo_linear_tiled_bytes": ([_i64, _i64, _i64, _i64, _i64p], _int),
     "ao_amd_int4wo_linear_tiled_plan": ([_i64, _i64, _i64, ctypes.c_char_p, _i64], _int),
     "ao_amd_int4wo_linear_tiled": ([_p, _i64, _i64, _i64, _p, _p, _i64, _i64, _p, _p, _i64, _p, _i64, _p], _int),
+    "ao_amd_int4wo_linear_auto_bytes": ([_p, _i64, _i64, _i64, _i64, _i64, _int, _i64p], _int),
+    "ao_amd_int4wo_linear_auto": ([_p, _i64, _i64, _i64, _p, _p, _i64, _i64, _p, _p, _int, _i64, _p, _i64, _p], _int),
     "ao_amd_pad_rows": ([_p, _i64, _i64, _i64, _i64, _p, _p], _int),
     "ao_amd_int4wo_linear_ws_parts": ([_i64, _i64, _i64, _i64], _int),
     "ao_amd_int4wo_linear_ws": ([_p, _i64, _i64, _i64, _p, _p, _i64, _i64, _p, _p, _int, _i64, _p, _i64, _p], _int),

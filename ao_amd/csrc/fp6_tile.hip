@@ -158,3 +158,16 @@ extern "C" int ao_amd_fp6_linear_tiled(const void* x_f16, int64_t M, int64_t K, 
     AO_LAUNCH_CHECK();
     return 0;
 }
+
+extern "C" int ao_amd_fp6_linear_auto_bytes(int64_t M, int64_t K, int64_t N, int64_t* bytes) {
+    if (int rc = ao_amd_fp6_linear_tiled_bytes(M, K, N, bytes)) return rc;
+    return *bytes >= 0 ? 0 : ao_amd_fp6_linear_ws_bytes(M, K, N, bytes);
+}
+
+extern "C" int ao_amd_fp6_linear_auto(const void* x_f16, int64_t M, int64_t K, const void* weights_native, const void* scale_f16, int64_t N,
+                                      int ebits, int mbits, void* out_f16, void* workspace, int64_t workspace_bytes, void* stream) {
+    AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
+    if (fp6_tiled(M, N, K))
+        return ao_amd_fp6_linear_tiled(x_f16, M, K, weights_native, scale_f16, N, ebits, mbits, out_f16, workspace, workspace_bytes, stream);
+    return ao_amd_fp6_linear_ws(x_f16, M, K, weights_native, scale_f16, N, ebits, mbits, out_f16, workspace, workspace_bytes, stream);
+}

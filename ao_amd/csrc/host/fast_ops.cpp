@@ -30,30 +30,11 @@ PyObject* int4wo_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     AO_WANT(r.ok && r.K == K && int4_weight_ok(packed, qparams, N, K, g) && bias_ok(bias, N));
     return guarded([&]() -> PyObject* {
         Tensor y = empty_rows(x, N, at::kBFloat16), ws;
-        int64_t need = -1;
-        hipStream_t st = stream_of(a.device);
-        if (r.M > 32 && r.ld % 8 == 0 && (uintptr_t)ptr(x) % 16 == 0) AO_CALL(ao_amd_int4wo_linear_tiled_bytes(r.M, K, N, g, &need));
-        if (need >= 0) {
-            if (need) ws = workspace(need, a.device);
-            AO_CALL(ao_amd_int4wo_linear_tiled(ptr(x), r.M, K, r.ld, ptr(packed), ptr(qparams), N, g, ptr(bias), y.data_ptr(), N,
-                                               need ? ws.data_ptr() : nullptr, need, st));
-            return THPVariable_Wrap(std::move(y));
-        }
-        need = 0;
-        const void* rows = ptr(x);
-        int64_t k = K, ld = r.ld;
-        Tensor copy;
-        AO_WANT(pad_int4_rows(rows, r.M, k, ld, N, g, copy, a.device, st));
-        if (r.M >= 16 && r.M <= 256) {
-            AO_CALL(ao_amd_int4wo_linear_ws_bytes(r.M, k, N, g, &need));
-            if (need) ws = workspace(need, a.device);
-        }
-        if (need) {
-            AO_CALL(ao_amd_int4wo_linear_ws(rows, r.M, k, ld, ptr(packed), ptr(qparams), N, g, ptr(bias), y.data_ptr(), AO_BF16,
-                                            N, ws.data_ptr(), need, st));
-        } else {
-            AO_CALL(ao_amd_int4wo_linear(rows, r.M, k, ld, ptr(packed), ptr(qparams), N, g, ptr(bias), y.data_ptr(), AO_BF16, N, st));
-        }
+        int64_t need = 0;
+        AO_CALL(ao_amd_int4wo_linear_auto_bytes(ptr(x), r.M, K, r.ld, N, g, AO_BF16, &need));
+        if (need) ws = workspace(need, a.device);
+        AO_CALL(ao_amd_int4wo_linear_auto(ptr(x), r.M, K, r.ld, ptr(packed), ptr(qparams), N, g, ptr(bias), y.data_ptr(), AO_BF16, N,
+                                          need ? ws.data_ptr() : nullptr, need, stream_of(a.device)));
         return THPVariable_Wrap(std::move(y));
     });
 }
@@ -93,25 +74,11 @@ PyObject* fp6_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     AO_WANT(native.numel() == fp6_native_words(N, r.K));
     return guarded([&]() -> PyObject* {
         Tensor y = empty_rows(x, N, at::kHalf), ws;
-        int64_t need = -1;
-        hipStream_t st = stream_of(a.device);
-        if (r.M > 32) AO_CALL(ao_amd_fp6_linear_tiled_bytes(r.M, r.K, N, &need));
-        if (need >= 0) {
-            if (need) ws = workspace(need, a.device);
-            AO_CALL(ao_amd_fp6_linear_tiled(ptr(x), r.M, r.K, ptr(native), ptr(scale), N, (int)e, (int)m, y.data_ptr(),
-                                            need ? ws.data_ptr() : nullptr, need, st));
-            return THPVariable_Wrap(std::move(y));
-        }
-        need = 0;
-        if (r.M >= 16 && r.M <= 256) {
-            AO_CALL(ao_amd_fp6_linear_ws_bytes(r.M, r.K, N, &need));
-            if (need) ws = workspace(need, a.device);
-        }
-        if (need) {
-            AO_CALL(ao_amd_fp6_linear_ws(ptr(x), r.M, r.K, ptr(native), ptr(scale), N, (int)e, (int)m, y.data_ptr(), ws.data_ptr(), need, st));
-        } else {
-            AO_CALL(ao_amd_fp6_linear(ptr(x), r.M, r.K, ptr(native), ptr(scale), N, (int)e, (int)m, y.data_ptr(), st));
-        }
+        int64_t need = 0;
+        AO_CALL(ao_amd_fp6_linear_auto_bytes(r.M, r.K, N, &need));
+        if (need) ws = workspace(need, a.device);
+        AO_CALL(ao_amd_fp6_linear_auto(ptr(x), r.M, r.K, ptr(native), ptr(scale), N, (int)e, (int)m, y.data_ptr(),
+                                       need ? ws.data_ptr() : nullptr, need, stream_of(a.device)));
         return THPVariable_Wrap(std::move(y));
     });
 }

@@ -161,25 +161,6 @@ inline bool int4_weight_ok(const Tensor& packed, const Tensor& qparams, int64_t 
            qparams.size(2) == 16 && qparams.is_contiguous();
 }
 
-// Activations of an int4 linear whose rows the fast kernels cannot read (not 16-byte aligned, or shorter than the packed width):
-// copied to that width, where the copy (2 to 3 us with its launch) costs less than the element-wise kernel loses, whose time
-// follows the length of the rows, or the whole product where the weight is large.  us a call as they are / copied: 4096 x 4160 at 1 / 6 /
-// 16 / 64 rows 15.5 / 18 / 35 / 121, 10.5 / 10.0 / 10.5 / 16.4; 14336 x 4032 at 1 / 16 rows 30 / 114, 13.5 / 15.5; 1024 x 2112 at 1 / 2 / 8 /
-// 16 rows 13.9 / 8.9 / 12.9 / 19.8, about 9.5; 1024 x 704 up to 64 rows 7 to 9, about 9.
-inline bool pad_int4_rows(const void*& x, int64_t M, int64_t& K, int64_t& ld, int64_t N, int64_t g, Tensor& copy, c10::DeviceIndex device,
-                          hipStream_t st) {
-    const int64_t q = g > 128 ? g : 128, Kp = (K + q - 1) / q * q;
-    const int64_t rows = M < 16 ? M : 16;
-    if ((K == Kp && ld % 8 == 0 && (uintptr_t)x % 16 == 0) ||
-        (N * K * (M + 4) < 50000000 && K * (M == 1 ? 13 : rows + 4) < 18000))
-        return true;
-    copy = empty({M, Kp}, at::kBFloat16, device);
-    if (ao_amd_pad_rows(x, M, K, ld, Kp, copy.data_ptr(), st) != 0) return false;
-    x = copy.const_data_ptr();
-    K = ld = Kp;
-    return true;
-}
-
 inline int64_t fp6_native_words(int64_t N, int64_t K) { return N / 16 * ((K + 127) / 128) * 384; }
 
 // llama.cpp

@@ -177,41 +177,23 @@ struct Pass {
             return true;
         }
         y = alloc(M, l.N);
-        int64_t need = -1;
-        if (m.kind == INT4 && M > 32) AO_TRY(ao_amd_int4wo_linear_tiled_bytes(M, l.K, l.N, m.group, &need));
-        if (m.kind == FP6 && M > 32) AO_TRY(ao_amd_fp6_linear_tiled_bytes(M, l.K, l.N, &need));
-        if (need >= 0) {
-            Tensor ws;
-            if (need) ws = workspace(need, device);
-            void* w = need ? ws.data_ptr() : nullptr;
-            if (m.kind == INT4)
-                return ao_amd_int4wo_linear_tiled(ptr(x), M, l.K, l.K, ptr(l.codes), ptr(l.scales), l.N, m.group, nullptr, y.data_ptr(), l.N, w,
-                                                  need, st) == 0;
-            return ao_amd_fp6_linear_tiled(ptr(x), M, l.K, ptr(l.codes), ptr(l.scales), l.N, m.ebits, m.mbits, y.data_ptr(), w, need, st) == 0;
-        }
-        need = 0;
-        const void* rows = ptr(x);
-        int64_t K = l.K, ld = l.K;
-        Tensor copy;
-        if (m.kind == INT4 && !pad_int4_rows(rows, M, K, ld, l.N, m.group, copy, device, st)) return false;
-        if (m.kind == INT8) {
+        int64_t need = 0;
+        if (m.kind == INT4)
+            AO_TRY(ao_amd_int4wo_linear_auto_bytes(ptr(x), M, l.K, l.K, l.N, m.group, AO_BF16, &need));
+        else if (m.kind == INT8)
             AO_TRY(ao_amd_int8wo_linear_ws_bytes(M, l.K, l.N, &need));
-        } else if (M >= 16 && M <= 256) {
-            if (m.kind == INT4)
-                AO_TRY(ao_amd_int4wo_linear_ws_bytes(M, K, l.N, m.group, &need));
-            else
-                AO_TRY(ao_amd_fp6_linear_ws_bytes(M, l.K, l.N, &need));
-        }
+        else
+            AO_TRY(ao_amd_fp6_linear_auto_bytes(M, l.K, l.N, &need));
         Tensor ws;
         if (need) ws = workspace(need, device);
-        if (m.kind == INT8)
-            return ao_amd_int8wo_linear_ws(ptr(x), M, l.K, l.K, ptr(l.codes), l.K, ptr(l.scales), l.N, nullptr, y.data_ptr(), AO_BF16, l.N,
-                                           need ? ws.data_ptr() : nullptr, need, st) == 0;
+        void* w = need ? ws.data_ptr() : nullptr;
         if (m.kind == INT4)
-            return ao_amd_int4wo_linear_ws(rows, M, K, ld, ptr(l.codes), ptr(l.scales), l.N, m.group, nullptr, y.data_ptr(), AO_BF16,
-                                           l.N, need ? ws.data_ptr() : nullptr, need, st) == 0;
-        return ao_amd_fp6_linear_ws(ptr(x), M, l.K, ptr(l.codes), ptr(l.scales), l.N, m.ebits, m.mbits, y.data_ptr(),
-                                    need ? ws.data_ptr() : nullptr, need, st) == 0;
+            return ao_amd_int4wo_linear_auto(ptr(x), M, l.K, l.K, ptr(l.codes), ptr(l.scales), l.N, m.group, nullptr, y.data_ptr(), AO_BF16,
+                                             l.N, w, need, st) == 0;
+        if (m.kind == INT8)
+            return ao_amd_int8wo_linear_ws(ptr(x), M, l.K, l.K, ptr(l.codes), l.K, ptr(l.scales), l.N, nullptr, y.data_ptr(), AO_BF16, l.N, w,
+                                           need, st) == 0;
+        return ao_amd_fp6_linear_auto(ptr(x), M, l.K, ptr(l.codes), ptr(l.scales), l.N, m.ebits, m.mbits, y.data_ptr(), w, need, st) == 0;
     }
 
     // ---- one row: the norm, the residual and the gated product ride in the linears

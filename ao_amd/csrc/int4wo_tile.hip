@@ -150,6 +150,39 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const uint16_t* __restric
     *(uint4*)(y + m * Kp + k) = out;
 }
 
+// Which route a plain linear takes and what its workspace holds: the copied rows first, then the K parts.
+struct Int4Auto {
+    bool tiled;
+    int64_t Kp;           // the width of the copied rows, 0: read as they are
+    int64_t copy, parts;  // bytes
+};
+static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t N, int64_t g, int y_dtype, Int4Auto* r) {
+    *r = Int4Auto{false, 0, 0, 0};
+    const bool aligned = (ldx & 7) == 0 && (((uintptr_t)x) & 15) == 0;
+    if (M > 32 && y_dtype == AO_BF16 && aligned && 256 * ldx * 2 < ((int64_t)1 << 32)) {
+        int64_t need = -1;
+        if (int rc = ao_amd_int4wo_linear_tiled_bytes(M, K, N, g, &need)) return rc;
+        if (need >= 0) {
+            r->tiled = true;
+            r->parts = need;
+            return 0;
+        }
+    }
+    // Rows that the fast kernels cannot read are copied to the packed width where the copy (2 to 3 us with its launch) costs less than the
+    // element-wise kernel loses, whose time follows the length of the rows, or the whole product where the weight is large.  us a call
+    // as they are / copied: 4096 x 4160 at 1 / 6 / 16 / 64 rows 15.5 / 18 / 35 / 121, 10.5 / 10.0 / 10.5 / 16.4; 14336 x 4032 at 1 / 16
+    // rows 30 / 114, 13.5 / 15.5; 1024 x 2112 at 1 / 2 / 8 / 16 rows 13.9 / 8.9 / 12.9 / 19.8, about 9.5; 1024 x 704 up to 64 rows 7
+    // to 9, about 9.
+    int64_t Np, Kp;
+    if (int rc = ao_amd_int4wo_packed_shape(N, K, g, &Np, &Kp, nullptr, nullptr)) return rc;
+    const int64_t rows = M < 16 ? M : 16;
+    if (M > 0 && (K != Kp || !aligned) && (N * K * (M + 4) >= 50000000 || K * (M == 1 ? 13 : rows + 4) >= 18000)) {
+        r->Kp = Kp;
+        r->copy = M * Kp * 2;
+    }
+    return ao_amd_int4wo_linear_ws_bytes(M, r->Kp ? Kp : K, N, g, &r->parts);
+}
+
 }  // namespace ao
 
 using namespace ao;
@@ -225,4 +258,35 @@ extern "C" int ao_amd_pad_rows(const void* x, int64_t M, int64_t K, int64_t ldx,
     hipLaunchKernelGGL(pad_rows_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream, (const uint16_t*)x, M, K, ldx, Kp, vec, (uint16_t*)y);
     AO_LAUNCH_CHECK();
     return 0;
+}
+
+extern "C" int ao_amd_int4wo_linear_auto_bytes(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, int64_t N, int64_t g, int y_dtype,
+                                               int64_t* bytes) {
+    AO_REQUIRE(bytes, "null pointer argument");
+    AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
+    Int4Auto r;
+    if (int rc = int4wo_auto(x_bf16, M, K, ldx, N, g, y_dtype, &r)) return rc;
+    *bytes = r.copy + r.parts;
+    return 0;
+}
+
+extern "C" int ao_amd_int4wo_linear_auto(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams,
+                                         int64_t N, int64_t g, const void* bias_bf16, void* y, int y_dtype, int64_t ldy, void* workspace,
+                                         int64_t workspace_bytes, void* stream) {
+    AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
+    AO_REQUIRE(ldx >= K, "row stride ldx=%lld smaller than the rows", (long long)ldx);
+    Int4Auto r;
+    if (int rc = int4wo_auto(x_bf16, M, K, ldx, N, g, y_dtype, &r)) return rc;
+    AO_REQUIRE(r.copy + r.parts == 0 || (workspace && workspace_bytes >= r.copy + r.parts && (((uintptr_t)workspace) & 15) == 0),
+               "16-byte aligned workspace of %lld bytes needed (ao_amd_int4wo_linear_auto_bytes), got %lld", (long long)(r.copy + r.parts),
+               (long long)workspace_bytes);
+    if (r.tiled)
+        return ao_amd_int4wo_linear_tiled(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, ldy, workspace, r.parts, stream);
+    if (r.Kp) {
+        if (int rc = ao_amd_pad_rows(x_bf16, M, K, ldx, r.Kp, workspace, stream)) return rc;
+        x_bf16 = workspace;
+        K = ldx = r.Kp;
+    }
+    return ao_amd_int4wo_linear_ws(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy,
+                                   r.parts ? (uint8_t*)workspace + r.copy : nullptr, r.parts, stream);
 }

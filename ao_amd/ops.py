@@ -201,38 +201,13 @@ def _linear_cuda(x: Tensor, packed: Tensor, qparams: Tensor, group_size: int, N:
         # definition of the result: dequantize, then F.linear.
         return torch.nn.functional.linear(x, _dequantize_cuda(packed, qparams, N, K, group_size), bias)
     y = torch.empty((M, N), dtype=torch.float32 if fp32_out else torch.bfloat16, device=x.device)
-    if M > 32 and not fp32_out and x.stride(0) % 8 == 0 and x.stride(0) < 1 << 23 and x.data_ptr() % 16 == 0:
-        # batches between the streaming and the prefill kernels
-        need = ctypes.c_int64(-1)
-        check(lib().ao_amd_int4wo_linear_tiled_bytes(M, K, N, group_size, ctypes.byref(need)))
-        if need.value >= 0:
-            ws = torch.empty((need.value // 4,), dtype=torch.float32, device=x.device) if need.value else None
-            check(lib().ao_amd_int4wo_linear_tiled(x.data_ptr(), M, K, x.stride(0), packed.data_ptr(), qparams.data_ptr(), N, group_size,
-                                                   None if bias is None else bias.data_ptr(), y.data_ptr(), N,
-                                                   None if ws is None else ws.data_ptr(), need.value, current_stream(x.device)))
-            return y
-    q = max(128, group_size)
-    Kp = (K + q - 1) // q * q
-    if (K != Kp or x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0) \
-            and (N * K * (M + 4) >= 50000000 or K * (13 if M == 1 else min(M, 16) + 4) >= 18000):
-        # rows that the fast kernels cannot read, copied to the packed width (csrc/host/host.h: pad_int4_rows)
-        padded = torch.empty((M, Kp), dtype=x.dtype, device=x.device)
-        check(lib().ao_amd_pad_rows(x.data_ptr(), M, K, x.stride(0), Kp, padded.data_ptr(), current_stream(x.device)))
-        x, K = padded, Kp
-    if 16 <= M <= 256:
-        # the row counts at which the library may split K over workgroups through a workspace (narrow weights, long K)
-        need = ctypes.c_int64(0)
-        check(lib().ao_amd_int4wo_linear_ws_bytes(M, K, N, group_size, ctypes.byref(need)))
-        if need.value:
-            ws = torch.empty((need.value // 4,), dtype=torch.float32, device=x.device)
-            check(lib().ao_amd_int4wo_linear_ws(x.data_ptr(), M, K, x.stride(0), packed.data_ptr(), qparams.data_ptr(), N,
-                                                group_size, None if bias is None else bias.data_ptr(), y.data_ptr(),
-                                                F32 if fp32_out else BF16, N, ws.data_ptr(), need.value,
-                                                current_stream(x.device)))
-            return y
-    check(lib().ao_amd_int4wo_linear(x.data_ptr(), M, K, x.stride(0) if M > 0 else K, packed.data_ptr(),
-                                     qparams.data_ptr(), N, group_size, None if bias is None else bias.data_ptr(),
-                                     y.data_ptr(), F32 if fp32_out else BF16, N, current_stream(x.device)))
+    # the library picks the kernel by the shape and the alignment of the rows, and may split K over workgroups or copy the rows
+    ld, y_dtype, need = x.stride(0) if M > 0 else K, F32 if fp32_out else BF16, ctypes.c_int64(0)
+    check(lib().ao_amd_int4wo_linear_auto_bytes(x.data_ptr(), M, K, ld, N, group_size, y_dtype, ctypes.byref(need)))
+    ws = torch.empty(((need.value + 3) // 4,), dtype=torch.float32, device=x.device) if need.value else None
+    check(lib().ao_amd_int4wo_linear_auto(x.data_ptr(), M, K, ld, packed.data_ptr(), qparams.data_ptr(), N, group_size,
+                                          None if bias is None else bias.data_ptr(), y.data_ptr(), y_dtype, N,
+                                          None if ws is None else ws.data_ptr(), need.value, current_stream(x.device)))
     return y
 
 
@@ -738,29 +713,13 @@ def _fp6_linear_native_cuda(ebits, mbits, x, native, scale):
                                              w16.data_ptr(), current_stream(x.device)))
         return torch.nn.functional.linear(x, w16)
     out = torch.empty((M, N), dtype=torch.float16, device=x.device)
-    if M > 32:
-        # batches beyond the streaming kernels and the small tiles
-        need = ctypes.c_int64(-1)
-        check(lib().ao_amd_fp6_linear_tiled_bytes(M, K, N, ctypes.byref(need)))
-        if need.value >= 0:
-            ws = torch.empty((need.value // 4,), dtype=torch.float32, device=x.device) if need.value else None
-            check(lib().ao_amd_fp6_linear_tiled(x.contiguous().data_ptr(), M, K, native.data_ptr(), scale.contiguous().data_ptr(), N, ebits,
-                                                mbits, out.data_ptr(), None if ws is None else ws.data_ptr(), need.value,
-                                                current_stream(x.device)))
-            return out
-    if 16 <= M <= 256:
-        # the row counts at which the library may split K over workgroups through a workspace, as the reference's
-        # operator does with its `splitK` argument (here the library picks the part count)
-        need = ctypes.c_int64(0)
-        check(lib().ao_amd_fp6_linear_ws_bytes(M, K, N, ctypes.byref(need)))
-        if need.value:
-            ws = torch.empty((need.value // 4,), dtype=torch.float32, device=x.device)
-            check(lib().ao_amd_fp6_linear_ws(x.contiguous().data_ptr(), M, K, native.data_ptr(), scale.contiguous().data_ptr(),
-                                             N, ebits, mbits, out.data_ptr(), ws.data_ptr(), need.value,
-                                             current_stream(x.device)))
-            return out
-    check(lib().ao_amd_fp6_linear(x.contiguous().data_ptr(), M, K, native.data_ptr(), scale.contiguous().data_ptr(), N,
-                                  ebits, mbits, out.data_ptr(), current_stream(x.device)))
+    # the library picks the kernel and may split K over workgroups through a workspace, as the reference's operator does with
+    # its `splitK` argument
+    x, scale, need = x.contiguous(), scale.contiguous(), ctypes.c_int64(0)
+    check(lib().ao_amd_fp6_linear_auto_bytes(M, K, N, ctypes.byref(need)))
+    ws = torch.empty((need.value // 4,), dtype=torch.float32, device=x.device) if need.value else None
+    check(lib().ao_amd_fp6_linear_auto(x.data_ptr(), M, K, native.data_ptr(), scale.data_ptr(), N, ebits, mbits, out.data_ptr(),
+                                       None if ws is None else ws.data_ptr(), need.value, current_stream(x.device)))
     return out
 
 

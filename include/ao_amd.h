@@ -171,6 +171,14 @@ int ao_amd_int4wo_linear_tiled_plan(int64_t M, int64_t K, int64_t N, char* out, 
 int ao_amd_int4wo_linear_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams,
                                int64_t N, int64_t g, const void* bias_bf16, void* y_bf16, int64_t ldy, void* workspace,
                                int64_t workspace_bytes, void* stream);
+/* The linear on whichever of the routes above is the fastest for the shape and for the alignment of the rows: one call for the
+ * workspace (x is not read), one for the product.  The workspace holds the K parts and, where the rows are not 16-byte aligned or end
+ * before the packed width and it pays, their copy; the second call needs all of it. */
+int ao_amd_int4wo_linear_auto_bytes(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, int64_t N, int64_t g, int y_dtype,
+                                    int64_t* bytes);
+int ao_amd_int4wo_linear_auto(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams,
+                              int64_t N, int64_t g, const void* bias_bf16, void* y, int y_dtype, int64_t ldy, void* workspace,
+                              int64_t workspace_bytes, void* stream);
 /* 16-bit rows x [M, K] (row stride ldx, any alignment) -> y [M, Kp] with zeros beyond K; Kp a multiple of 8, y 16-byte aligned. */
 int ao_amd_pad_rows(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t Kp, void* y, void* stream);
 
@@ -433,6 +441,11 @@ int ao_amd_fp6_linear_tiled_bytes(int64_t M, int64_t K, int64_t N, int64_t* byte
 int ao_amd_fp6_linear_tiled_plan(int64_t M, int64_t K, int64_t N, char* out, int64_t out_cap);
 int ao_amd_fp6_linear_tiled(const void* x_f16, int64_t M, int64_t K, const void* weights_native, const void* scale_f16, int64_t N,
                             int ebits, int mbits, void* out_f16, void* workspace, int64_t workspace_bytes, void* stream);
+
+/* The linear on whichever of the routes above is the fastest for the shape: one call for the workspace, one for the product. */
+int ao_amd_fp6_linear_auto_bytes(int64_t M, int64_t K, int64_t N, int64_t* bytes);
+int ao_amd_fp6_linear_auto(const void* x_f16, int64_t M, int64_t K, const void* weights_native, const void* scale_f16, int64_t N,
+                           int ebits, int mbits, void* out_f16, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* Which kernel instantiation the FPx linear entry points run for a problem, without launching anything: writes a name
  * such as "fp6_gemm_kernel<1,1,4,4,4>" (e3m2 flag, then the tile variant) or "fp6_gemv_kernel<8,1,0>" to `out`.  The

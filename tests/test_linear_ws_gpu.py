@@ -170,3 +170,71 @@ def test_fp6_workspace_linear(N, K, M, parts, ebits, mbits):
     yh = run(xh.to(dev))
     exact = bool(torch.equal(yh, wd[:, ks.to(dev)].t().contiguous()))
     assert exact
+
+
+def _empty_ws(nbytes):
+    return torch.empty(max(nbytes, 16), dtype=torch.uint8, device="cuda")
+
+
+# (N, K, group, M, offset of the rows in elements, route)
+@pytest.mark.parametrize("N,K,g,M,shift,route", [
+    (4096, 4096, 64, 1, 0, "ws"), (4096, 14336, 64, 32, 0, "ws"), (256, 200, 64, 3, 4, "ws"), (1024, 704, 128, 33, 0, "ws"),
+    (4096, 4096, 64, 160, 0, "tiled"), (4096, 14336, 64, 160, 0, "tiled"), (4096, 4160, 64, 6, 0, "copied"),
+    (4096, 4096, 64, 6, 1, "copied"), (4096, 14208, 256, 32, 0, "copied")])
+@pytest.mark.parametrize("fp32", [False, True])
+def test_the_one_entry_picks_these_routes(N, K, g, M, shift, route, fp32):
+    """ao_amd_int4wo_linear_auto is bit for bit the entry that its rule names, with a workspace of exactly the bytes it asks for."""
+    from ao_amd import _lib
+
+    L, code, st = _lib.lib(), _lib.F32 if fp32 else _lib.BF16, torch.cuda.current_stream().cuda_stream
+    packed, qp, _ = _setup(N, K, g, 3)
+    x = torch.randn(M * K + shift, device="cuda").bfloat16()[shift:].view(M, K)
+    bias = torch.randn(N, device="cuda").bfloat16()
+    need = ctypes.c_int64(-1)
+
+    def call(name, x, nbytes, ws, *y_dtype):
+        y = torch.zeros(M, N, device="cuda", dtype=torch.float32 if fp32 else torch.bfloat16)
+        return getattr(L, name)(x.data_ptr(), M, x.shape[1], x.shape[1], packed.data_ptr(), qp.data_ptr(), N, g, bias.data_ptr(), y.data_ptr(),
+                                *y_dtype, N, ws, nbytes, st), y
+
+    _lib.check(L.ao_amd_int4wo_linear_auto_bytes(x.data_ptr(), M, K, K, N, g, code, ctypes.byref(need)))
+    total, ws = need.value, _empty_ws(need.value)
+    rc, got = call("ao_amd_int4wo_linear_auto", x, total, ws.data_ptr() if total else None, code)
+    _lib.check(rc)
+    if total:
+        assert call("ao_amd_int4wo_linear_auto", x, total, None, code)[0] and call("ao_amd_int4wo_linear_auto", x, total - 1, ws.data_ptr(), code)[0]
+    if route == "tiled" and not fp32:   # its output is bf16
+        _lib.check(L.ao_amd_int4wo_linear_tiled_bytes(M, K, N, g, ctypes.byref(need)))
+        assert need.value == total
+        rc, want = call("ao_amd_int4wo_linear_tiled", x, total, ws.data_ptr())
+    else:
+        if route == "copied":
+            q = max(128, g)
+            x = torch.nn.functional.pad(x, (0, -K % q)).clone()
+            assert x.data_ptr() % 16 == 0
+        _lib.check(L.ao_amd_int4wo_linear_ws_bytes(M, x.shape[1], N, g, ctypes.byref(need)))
+        assert total == need.value + (2 * x.numel() if route == "copied" else 0)
+        ws = _empty_ws(need.value)
+        rc, want = call("ao_amd_int4wo_linear_ws", x, need.value, ws.data_ptr(), code)
+    _lib.check(rc)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("N,K,M,route", [(4096, 4096, 2, "ws"), (4096, 14336, 32, "ws"), (4096, 14336, 160, "tiled"), (14336, 4032, 33, "tiled")])
+def test_the_one_fp6_entry_picks_these_routes(N, K, M, route):
+    from ao_amd import _lib, ops
+
+    L, st = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    data, scale = ops.fp6_quantize_pack((torch.randn(N, K, device="cuda") * 0.02).half(), 3, 2)
+    native = ops.fp6_repack(data, 6)
+    x = torch.randn(M, K, device="cuda").half()
+    got, want = torch.zeros(M, N, device="cuda").half(), torch.ones(M, N, device="cuda").half()
+    need, part = ctypes.c_int64(-1), ctypes.c_int64(-1)
+    _lib.check(L.ao_amd_fp6_linear_auto_bytes(M, K, N, ctypes.byref(need)))
+    _lib.check(getattr(L, f"ao_amd_fp6_linear_{route}_bytes")(M, K, N, ctypes.byref(part)))
+    assert need.value == part.value >= 0
+    ws = _empty_ws(need.value)
+    for name, y in (("auto", got), (route, want)):
+        _lib.check(getattr(L, f"ao_amd_fp6_linear_{name}")(x.data_ptr(), M, K, native.data_ptr(), scale.data_ptr(), N, 3, 2, y.data_ptr(),
+                                                           ws.data_ptr(), need.value, st))
+    assert torch.equal(got, want)
