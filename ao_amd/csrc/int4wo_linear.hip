@@ -1419,14 +1419,15 @@ extern "C" int ao_amd_int4wo_linear(const void* x_bf16, int64_t M, int64_t K, in
 // those); 14336 x 4096: slower at every row count (224 workgroups already).  Below 16 rows the streaming kernels win
 // everywhere (4096 x 14336 at 8 rows 14.3 / 16.6).
 static int ws_parts(int64_t M, int64_t K, int64_t N, int64_t g) {
+    static const int forced = [] { const char* e = knob("AO_AMD_WS_PARTS"); return e ? atoi(e) : 0; }();
+    if (forced <= 0 && (M < 16 || M > 256)) return 1;
     int64_t Np, Kp;
     if (ao_amd_int4wo_packed_shape(N, K, g, &Np, &Kp, nullptr, nullptr)) return 1;
-    static const int forced = [] { const char* e = knob("AO_AMD_WS_PARTS"); return e ? atoi(e) : 0; }();
     const int64_t KB = Kp / 128, RB = Np / 16;
     int z = 1;
     if (forced > 0) {
         z = forced;
-    } else if (M >= 16 && M <= 256 && (RB >= 256 || M > 64)) {
+    } else if (RB >= 256 || M > 64) {
         const int64_t wgs = ((RB + 3) / 4) * (M <= 32 ? 1 : (M + 63) / 64);
         // parts while the grid stays within the CUs, at least 8 K tiles (2 per group of waves) each
         while (z < 4 && wgs * z * 2 <= 256 && KB / (z * 2) >= 8) z *= 2;

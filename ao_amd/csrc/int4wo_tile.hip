@@ -173,9 +173,8 @@ static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t
     // as they are / copied: 4096 x 4160 at 1 / 6 / 16 / 64 rows 15.5 / 18 / 35 / 121, 10.5 / 10.0 / 10.5 / 16.4; 14336 x 4032 at 1 / 16
     // rows 30 / 114, 13.5 / 15.5; 1024 x 2112 at 1 / 2 / 8 / 16 rows 13.9 / 8.9 / 12.9 / 19.8, about 9.5; 1024 x 704 up to 64 rows 7
     // to 9, about 9.
-    int64_t Np, Kp;
-    if (int rc = ao_amd_int4wo_packed_shape(N, K, g, &Np, &Kp, nullptr, nullptr)) return rc;
-    const int64_t rows = M < 16 ? M : 16;
+    AO_REQUIRE(valid_group(g), "group size must be 32, 64, 128 or 256, got %lld", (long long)g);
+    const int64_t Kp = round_up(K, g > 128 ? g : 128), rows = M < 16 ? M : 16;
     if (M > 0 && (K != Kp || !aligned) && (N * K * (M + 4) >= 50000000 || K * (M == 1 ? 13 : rows + 4) >= 18000)) {
         r->Kp = Kp;
         r->copy = M * Kp * 2;
@@ -287,6 +286,7 @@ extern "C" int ao_amd_int4wo_linear_auto(const void* x_bf16, int64_t M, int64_t 
         x_bf16 = workspace;
         K = ldx = r.Kp;
     }
-    return ao_amd_int4wo_linear_ws(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy,
-                                   r.parts ? (uint8_t*)workspace + r.copy : nullptr, r.parts, stream);
+    if (!r.parts) return ao_amd_int4wo_linear(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, stream);
+    return ao_amd_int4wo_linear_ws(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, (uint8_t*)workspace + r.copy,
+                                   r.parts, stream);
 }
