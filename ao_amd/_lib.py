@@ -66,7 +66,7 @@ _SIGNATURES = {
     "ao_amd_fp6_linear_fused": ([_p, _i64, _i64, _p, _p, _i64, _int, _int, _p, _p, _p, _p], _int),
     "ao_amd_llama_embed": ([_p, _int, _i64, _p, _i64, _i64, _p, _p], _int),
     "ao_amd_llama_prefill_attention": ([_p, _int, _p, _p, _int, _i64, _p, _p, _int, _int, _int, _i64, _p, _p], _int),
-    "ao_amd_llama_prefill_attention_rows": ([_p, _int, _p, _p, _int, _i64, _p, _p, _int, _int, _int, _i64, _p, _p], _int),
+    "ao_amd_llama_prefill_attention_wrap": ([_p, _int, _p, _i64, _p, _int, _i64, _p, _p, _int, _int, _int, _i64, _p, _p], _int),
     "ao_amd_add_rmsnorm": ([_p, _p, _p, _int, _i64, _i64, ctypes.c_float, _p, _p, _p], _int),
     "ao_amd_silu_mul": ([_p, _p, _int, _i64, _p, _p], _int),
     "ao_amd_rmsnorm_f16": ([_p, _p, _i64, _i64, ctypes.c_float, _p, _p], _int),

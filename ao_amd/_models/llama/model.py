@@ -187,11 +187,12 @@ def _child(m: nn.Module, name: str):
 
 
 def _chain_functions():
-    return nn.Module.__call__, KVCache.update, apply_rotary_emb, F.scaled_dot_product_attention, F.silu
+    return nn.Module.__call__, KVCache.update, apply_rotary_emb, F.scaled_dot_product_attention, F.silu, F.embedding
 
 
 # What the native pass of a prompt stands for: these classes with their own forward, over these functions
-_CHAIN_FORWARDS = {c: c.forward for c in (nn.Linear, RMSNorm, Attention, FeedForward, TransformerBlock, KVCache)}
+_CHAIN_FORWARDS = {c: c.forward for c in (nn.Linear, RMSNorm, Attention, FeedForward, TransformerBlock, KVCache,
+                                                       nn.Embedding)}
 _CHAIN_FUNCTIONS = _chain_functions()
 
 
@@ -306,13 +307,23 @@ class Transformer(nn.Module):
     def fused_decode_ready(self) -> bool:
         return self.fused_decode_kind() is not None
 
+    def _calls_are_watched(self) -> bool:
+        """Whether somebody wants to see the calls of every module, or replaced a function that the modules call."""
+        hooks = torch.nn.modules.module
+        return bool(hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _chain_functions() != _CHAIN_FUNCTIONS)
+
+    def _embedding_is_plain(self) -> bool:
+        """Whether calling the embedding module does no more than look the rows up in its table."""
+        e = _child(self, "tok_embeddings")
+        return _is_plain(e) and e.max_norm is None and not self._calls_are_watched()
+
     def _prompt_is_the_module_chain(self) -> bool:
         """Whether calling module after module would compute what the native pass of a prompt computes: the modules and
         functions of this file, none subclassed (an adapter's linear), replaced (another norm or block), patched or watched by a
         hook, under the causal mask that setup_caches made.  Read anew for every prompt, some 5 us a layer."""
-        hooks, cfg = torch.nn.modules.module, self.config
-        if hooks._global_forward_hooks or hooks._global_forward_pre_hooks or _chain_functions() != _CHAIN_FUNCTIONS:
+        if self._calls_are_watched():
             return False
+        cfg = self.config
         mask, version = self.__dict__.get("_own_mask", (None, 0))  # a model pickled by an earlier version has none
         if mask is None or self.causal_mask is not mask or mask._version != version:
             return False
@@ -501,16 +512,20 @@ class Transformer(nn.Module):
         from ... import ops
 
         assert self.freqs_cis is not None, "Caches must be initialized first"
-        x = self.tok_embeddings(idx)
+        x = None
         if self.use_fused_decode and input_pos is not None and idx.dim() == 2 and idx.shape[0] == 1 \
                 and not torch.compiler.is_dynamo_compiling():
             # every launch of the pass from one native call; it declines what it does not take before it launches anything
             kind = self.fused_decode_kind() if idx.numel() == 1 or self._prompt_is_the_module_chain() else None
             if kind is not None:
                 pos = input_pos.to(torch.int32) if idx.numel() == 1 and input_pos.dtype is not torch.int32 else input_pos
-                logits = ops.host.llama_forward(self._host_plan(kind, idx.numel()), x, pos)
+                table = self.tok_embeddings.weight if self._embedding_is_plain() else None
+                x = None if table is not None else self.tok_embeddings(idx)
+                logits = ops.host.llama_forward(self._host_plan(kind, idx.numel()), x if table is None else idx, table, pos)
                 if logits is not NotImplemented:
                     return logits
+        if x is None:
+            x = self.tok_embeddings(idx)
         if self.use_fused_decode and idx.numel() == 1 and input_pos is not None and input_pos.numel() == 1:
             kind = self.fused_decode_kind()
             if kind == "int4":

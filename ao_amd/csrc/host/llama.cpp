@@ -5,6 +5,8 @@
 // The caller describes the model as nested tuples of tensors and numbers (Transformer._host_plan); they are checked
 // completely before the first launch.
 #include <ATen/autocast_mode.h>
+#include <ATen/core/LegacyTypeDispatch.h>
+#include <ATen/ops/embedding.h>
 #include <ATen/ops/index.h>
 #include <ATen/ops/linear.h>
 #include <ATen/ops/mul.h>
@@ -264,11 +266,10 @@ struct Pass {
     }
 
     // ---- several rows
-    bool prefill(Tensor x, const Tensor& input_pos, int64_t T, Tensor& logits) {
-        // torch's indexing, as in the module chain: it refuses a position outside the cache or the rotary table and counts a negative
-        // one from the end of each
-        const c10::List<std::optional<Tensor>> at_pos({std::optional<Tensor>(input_pos)});
-        const Tensor pos = at::index(m.cache_rows, at_pos), freqs = at::index(m.freqs, at_pos);
+    bool prefill(Tensor x, const Tensor& pos, int64_t T, Tensor& logits) {
+        // torch's indexing, as in the module chain, for its refusal of a position outside the cache (and the rotary table, which is no
+        // shorter).  The attention finds the rows of the others itself: negative ones count from the end, as they do there.
+        (void)at::index(m.cache_rows, {std::optional<Tensor>(pos)});
         Tensor n = alloc(T, m.dim);
         const Layer* first = m.layers.empty() ? nullptr : &m.layers[0];
         const Tensor& w0 = first ? first->attn_norm : m.norm;
@@ -282,8 +283,9 @@ struct Pass {
             const float next_eps = (float)(end ? m.eps : m.layers[i + 1].attn_eps);
             Tensor qkv, y = alloc(T, m.n_head * 128), o, gate, up, down;
             if (!linear(l.wqkv, n, T, qkv)) return false;
-            AO_TRY(ao_amd_llama_prefill_attention_rows(ptr(qkv), f16, ptr(freqs), ptr(pos), 0, T, l.k_cache.data_ptr(), l.v_cache.data_ptr(),
-                                                       (int)m.n_head, (int)m.n_kv, 128, m.max_seq, y.data_ptr(), st));
+            AO_TRY(ao_amd_llama_prefill_attention_wrap(ptr(qkv), f16, ptr(m.freqs), m.freqs.size(0), ptr(pos), pos.scalar_type() == at::kLong, T,
+                                                       l.k_cache.data_ptr(), l.v_cache.data_ptr(), (int)m.n_head, (int)m.n_kv, 128, m.max_seq,
+                                                       y.data_ptr(), st));
             if (!linear(l.wo, y, T, o)) return false;
             Tensor h = alloc(T, m.dim), hn = alloc(T, m.dim);
             AO_TRY(ao_amd_add_rmsnorm(ptr(x), ptr(o), ptr(l.ffn_norm), f16, T, m.dim, (float)l.ffn_eps, h.data_ptr(), hn.data_ptr(), st));
@@ -300,24 +302,31 @@ struct Pass {
 
 }  // namespace
 
-// (plan, embedded tokens [1, T, dim], positions [T]: int32 for T = 1, else int32 or int64) -> logits [1, T, vocab].  The caller looks
-// the tokens up through the model's embedding module: it may be another one, and its kernel refuses a token outside the table.
+// (plan, tokens int32 or int64 [1, T] and the embedding table, or embedded tokens [1, T, dim] and None, positions [T]: int32 for T = 1,
+// else int32 or int64) -> logits [1, T, vocab].  Tokens are looked up by torch's embedding, which refuses one outside the table; the
+// caller calls an embedding module that does more itself.
 PyObject* llama_forward(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
-    AO_NEED(3);
+    AO_NEED(4);
+    auto index = [&](int i) -> const Tensor& {
+        const bool is_long = THPVariable_CheckExact(v[i]) && THPVariable_Unpack(v[i]).defined() && THPVariable_Unpack(v[i]).scalar_type() == at::kLong;
+        return a.tensor(i, is_long ? at::kLong : at::kInt);
+    };
     at::ScalarType dtype;
-    const Tensor& x = a.tensor16(1, dtype);
-    const bool is_long = THPVariable_CheckExact(v[2]) && THPVariable_Unpack(v[2]).defined() && THPVariable_Unpack(v[2]).scalar_type() == at::kLong;
-    const Tensor& pos = a.tensor(2, is_long ? at::kLong : at::kInt);
-    AO_WANT(a.ok && current(a.device) && x.dim() == 3 && x.size(0) == 1 && x.is_contiguous() &&
-            (uintptr_t)ptr(x) % 16 == 0);
-    const int64_t T = x.size(1);
+    const bool embedded = v[2] == Py_None;
+    const Tensor &rows = embedded ? a.tensor16(1, dtype) : index(1), &pos = index(3);
+    const Tensor* table = embedded ? nullptr : &a.tensor16(2, dtype);
+    AO_WANT(a.ok && current(a.device) && rows.dim() == (embedded ? 3 : 2) && rows.size(0) == 1 && (embedded || table->dim() == 2));
+    const int64_t T = rows.size(1);
     AO_WANT(T >= 1 && pos.dim() == 1 && pos.numel() == T && pos.is_contiguous() && (T > 1 || pos.scalar_type() == at::kInt));
     // Autocast changes the types between the modules of a prompt (it clears a key that is excluded otherwise, so nothing_watches()
     // does not see it); a decode step is made of operators that it leaves alone.
     AO_WANT(T == 1 || !at::autocast::is_autocast_enabled(at::kCUDA));
     return guarded([&]() -> PyObject* {
         const Model m = read_model(a, v[0]);
-        AO_WANT(a.ok && dtype == m.dtype && x.size(2) == m.dim);
+        at::AutoDispatchBelowADInplaceOrView below;   // no gradient is recorded here: the arguments were looked at for one
+        AO_WANT(a.ok && dtype == m.dtype && (embedded ? rows.size(2) : table->size(1)) == m.dim);
+        const Tensor x = embedded ? rows : at::embedding(*table, rows);
+        AO_WANT(x.is_contiguous() && (uintptr_t)ptr(x) % 16 == 0);
         Pass p{m, a.device, stream_of(a.device)};
         Tensor logits;
         AO_WANT(T == 1 ? p.decode(x, pos, logits) : p.prefill(x, pos, T, logits));

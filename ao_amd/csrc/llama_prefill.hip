@@ -37,6 +37,18 @@ __device__ __forceinline__ int64_t position(const void* pos, int pos_is_i64, int
     return pos_is_i64 ? ((const int64_t*)pos)[i] : (int64_t)((const int32_t*)pos)[i];
 }
 
+// The cache row of a position and its row of the rotary table.  With wrap, the rows of that table (at least S), a negative position
+// counts from the end of either.  row -1: outside the cache.
+struct Position {
+    int64_t row, freq;
+};
+__device__ __forceinline__ Position locate(const void* pos, int pos_is_i64, int64_t i, int64_t S, int64_t wrap) {
+    const int64_t p = position(pos, pos_is_i64, i);
+    const bool behind = wrap > 0 && p < 0;
+    const int64_t row = behind ? p + S : p;
+    return row >= 0 && row < S ? Position{row, behind ? p + wrap : p} : Position{-1, 0};
+}
+
 // Rotates the consecutive pairs (2i, 2i+1) of 8 elements d .. d+7 of a head: fp32 products rounded one by one, the result
 // rounded to the element type, as the module does.  `cs` holds the four (cos, sin) pairs.
 template <class E>
@@ -52,24 +64,24 @@ __device__ __forceinline__ uint4 rotate8(uint4 x, uint4 cs) {
 }
 
 // Keys rotated and values as they are, into row input_pos[t] of the caches.  One thread per 8 elements; a row outside the
-// cache is not written.  The (cos, sin) pairs are rows of the whole table, or already gathered, one row a token.
+// cache is not written.
 template <class E>
 __global__ __launch_bounds__(256) void prefill_cache_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ freqs,
-                                                            bool freqs_by_row, const void* __restrict__ pos, int pos_is_i64, int T,
+                                                            int64_t wrap, const void* __restrict__ pos, int pos_is_i64, int T,
                                                             int n_head, int n_kv, int64_t S, uint16_t* __restrict__ k_cache,
                                                             uint16_t* __restrict__ v_cache) {
     const int per_row = 2 * n_kv * 16;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int t = (int)(i / per_row), c = (int)(i % per_row);
     if (t >= T) return;
-    const int64_t p = position(pos, pos_is_i64, t);
-    if (p < 0 || p >= S) return;
+    const Position p = locate(pos, pos_is_i64, t, S, wrap);
+    if (p.row < 0) return;
     const int head = c >> 4, d = (c & 15) * 8;
     const uint4 x = *(const uint4*)(qkv + ((int64_t)t * (n_head + 2 * n_kv) + n_head + head) * 128 + d);
     if (head < n_kv)
-        *(uint4*)(k_cache + ((int64_t)head * S + p) * 128 + d) = rotate8<E>(x, *(const uint4*)(freqs + (freqs_by_row ? t : p) * 128 + d));
+        *(uint4*)(k_cache + ((int64_t)head * S + p.row) * 128 + d) = rotate8<E>(x, *(const uint4*)(freqs + p.freq * 128 + d));
     else
-        *(uint4*)(v_cache + ((int64_t)(head - n_kv) * S + p) * 128 + d) = x;
+        *(uint4*)(v_cache + ((int64_t)(head - n_kv) * S + p.row) * 128 + d) = x;
 }
 
 // Causal attention of T query rows over the cache, flash style.
@@ -93,7 +105,7 @@ __global__ __launch_bounds__(256) void prefill_cache_kernel(const uint16_t* __re
 // Llama-3-8B widths, 1000 positions: 56 -> 35 us.
 template <class E, bool HEADS>
 __global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ freqs,
-                                                                bool freqs_by_row, const void* __restrict__ pos, int pos_is_i64,
+                                                                int64_t wrap, const void* __restrict__ pos, int pos_is_i64,
                                                                 int T, int n_head, int n_kv, int64_t S, const uint16_t* __restrict__ k_cache,
                                                                 const uint16_t* __restrict__ v_cache, uint16_t* __restrict__ out) {
     typedef Mfma32<E> MM;
@@ -119,18 +131,14 @@ __global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* 
     // this lane's query row: position, rotated fragments
     const int row = row0 + col;
     const int srow = row < T ? row : T - 1;
-    int last = -1;                                  // last position the row sees; -1: none
-    {
-        const int64_t p = position(pos, pos_is_i64, srow);
-        if (p >= 0 && p < S && row < T) last = (int)p;
-    }
+    const Position p = locate(pos, pos_is_i64, srow, S, wrap);
+    const int last = row < T ? (int)p.row : -1;     // last position the row sees; -1: none
     uint4 q[8];
-    const int64_t frow = freqs_by_row ? srow : last < 0 ? 0 : last;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
         const int d = 16 * s + 8 * half;
         q[s] = rotate8<E>(*(const uint4*)(qkv + ((int64_t)srow * (n_head + 2 * n_kv) + head) * 128 + d),
-                          *(const uint4*)(freqs + frow * 128 + d));
+                          *(const uint4*)(freqs + p.freq * 128 + d));
     }
     int hi = last, lo = last;
 #pragma unroll
@@ -373,7 +381,7 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 struct PrefillAttention {
     const uint16_t *qkv, *freqs;
-    bool freqs_by_row;
+    int64_t wrap;   // rows of freqs from whose end negative positions count, 0: they are outside
     const void* pos;
     int pos_is_i64;
     int64_t T;
@@ -387,14 +395,14 @@ template <class E>
 static void prefill_attention(const PrefillAttention& a, hipStream_t st) {
     const int T = (int)a.T;
     const int64_t chunks = a.T * 2 * a.n_kv * 16;
-    hipLaunchKernelGGL(prefill_cache_kernel<E>, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, a.qkv, a.freqs, a.freqs_by_row,
+    hipLaunchKernelGGL(prefill_cache_kernel<E>, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, a.qkv, a.freqs, a.wrap,
                        a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache);
     if (a.n_head / a.n_kv % 4 == 0)
         hipLaunchKernelGGL((prefill_attention_kernel<E, true>), dim3(a.n_head / 4, (T + 31) / 32), dim3(512), 0, st, a.qkv, a.freqs,
-                           a.freqs_by_row, a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache, a.out);
+                           a.wrap, a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache, a.out);
     else
         hipLaunchKernelGGL((prefill_attention_kernel<E, false>), dim3(a.n_head, (T + 127) / 128), dim3(512), 0, st, a.qkv, a.freqs,
-                           a.freqs_by_row, a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache, a.out);
+                           a.wrap, a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache, a.out);
 }
 
 static int prefill_attention_entry(const PrefillAttention& a, int is_f16, int head_dim, void* stream) {
@@ -403,6 +411,7 @@ static int prefill_attention_entry(const PrefillAttention& a, int is_f16, int he
     AO_REQUIRE(a.n_kv > 0 && a.n_head > 0 && a.n_head % a.n_kv == 0, "n_head=%d must be a multiple of n_kv=%d", a.n_head, a.n_kv);
     AO_REQUIRE(a.n_head <= 65535 && a.T >= 0 && a.T <= 1 << 20 && a.S > 0 && a.S <= 1 << 20, "T=%lld, max_seq=%lld out of range",
                (long long)a.T, (long long)a.S);
+    AO_REQUIRE(a.wrap == 0 || a.wrap >= a.S, "freqs_cis has %lld rows for a cache of %lld positions", (long long)a.wrap, (long long)a.S);
     AO_REQUIRE(aligned16(a.qkv) && aligned16(a.freqs) && aligned16(a.k_cache) && aligned16(a.v_cache) && aligned16(a.out),
                "16-byte aligned tensors needed");
     if (a.T == 0) return 0;
@@ -421,14 +430,15 @@ using namespace ao;
 extern "C" int ao_amd_llama_prefill_attention(const void* qkv, int is_f16, const void* freqs_cis, const void* positions, int pos_is_i64,
                                               int64_t T, void* k_cache, void* v_cache, int n_head, int n_kv, int head_dim,
                                               int64_t max_seq, void* out, void* stream) {
-    return prefill_attention_entry({(const uint16_t*)qkv, (const uint16_t*)freqs_cis, false, positions, pos_is_i64, T, (uint16_t*)k_cache,
+    return prefill_attention_entry({(const uint16_t*)qkv, (const uint16_t*)freqs_cis, 0, positions, pos_is_i64, T, (uint16_t*)k_cache,
                                     (uint16_t*)v_cache, n_head, n_kv, max_seq, (uint16_t*)out}, is_f16, head_dim, stream);
 }
 
-extern "C" int ao_amd_llama_prefill_attention_rows(const void* qkv, int is_f16, const void* freqs_rows, const void* positions,
-                                                   int pos_is_i64, int64_t T, void* k_cache, void* v_cache, int n_head, int n_kv,
-                                                   int head_dim, int64_t max_seq, void* out, void* stream) {
-    return prefill_attention_entry({(const uint16_t*)qkv, (const uint16_t*)freqs_rows, true, positions, pos_is_i64, T, (uint16_t*)k_cache,
+extern "C" int ao_amd_llama_prefill_attention_wrap(const void* qkv, int is_f16, const void* freqs_cis, int64_t freqs_len,
+                                                   const void* positions, int pos_is_i64, int64_t T, void* k_cache, void* v_cache,
+                                                   int n_head, int n_kv, int head_dim, int64_t max_seq, void* out, void* stream) {
+    AO_REQUIRE(freqs_len > 0, "freqs_len=%lld must be positive", (long long)freqs_len);
+    return prefill_attention_entry({(const uint16_t*)qkv, (const uint16_t*)freqs_cis, freqs_len, positions, pos_is_i64, T, (uint16_t*)k_cache,
                                     (uint16_t*)v_cache, n_head, n_kv, max_seq, (uint16_t*)out}, is_f16, head_dim, stream);
 }
 

@@ -344,8 +344,8 @@ int ao_amd_llama_decode_attention_split_static(const void* qkv_bf16, const void*
  *   llama_prefill_attention  rotary embedding of the queries and keys of qkv [T, (n_head + 2 n_kv) * 128], keys and values
  *                            into cache rows positions[t] ([n_kv, max_seq, 128]), query row t over cache positions
  *                            0 .. positions[t] -> out [T, n_head * 128] (a position outside the cache: no cache row is
- *                            written, the output row is NaN).  freqs_cis [>= max_seq, 64, 2]; `_rows`: the rows of the
- *                            T tokens [T, 64, 2]
+ *                            written, the output row is NaN).  freqs_cis [>= max_seq, 64, 2].  `_wrap`: of freqs_len rows; a
+ *                            negative position counts from the end of the cache and from the end of freqs_cis
  *   add_rmsnorm              sum = x + y, normed = rmsnorm(sum) * weight; dim a multiple of 8 up to 8192
  *   silu_mul                 out = silu(gate) * up over n elements, n a multiple of 8; out may be gate
  * Every operation rounds to the element type where the module chain does (torchao/_models/llama/model.py:162-244). */
@@ -354,9 +354,9 @@ int ao_amd_llama_embed(const void* tokens, int is_i64, int64_t T, const void* ta
 int ao_amd_llama_prefill_attention(const void* qkv, int is_f16, const void* freqs_cis, const void* positions, int pos_is_i64,
                                    int64_t T, void* k_cache, void* v_cache, int n_head, int n_kv, int head_dim,
                                    int64_t max_seq, void* out, void* stream);
-int ao_amd_llama_prefill_attention_rows(const void* qkv, int is_f16, const void* freqs_rows, const void* positions,
-                                        int pos_is_i64, int64_t T, void* k_cache, void* v_cache, int n_head, int n_kv,
-                                        int head_dim, int64_t max_seq, void* out, void* stream);
+int ao_amd_llama_prefill_attention_wrap(const void* qkv, int is_f16, const void* freqs_cis, int64_t freqs_len,
+                                        const void* positions, int pos_is_i64, int64_t T, void* k_cache, void* v_cache,
+                                        int n_head, int n_kv, int head_dim, int64_t max_seq, void* out, void* stream);
 int ao_amd_add_rmsnorm(const void* x, const void* y, const void* weight, int is_f16, int64_t rows, int64_t dim, float eps,
                        void* sum, void* normed, void* stream);
 int ao_amd_silu_mul(const void* gate, const void* up, int is_f16, int64_t n, void* out, void* stream);

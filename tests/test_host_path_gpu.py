@@ -118,7 +118,7 @@ def _plain_calls():
         "int8wo_linear": ([x(torch.bfloat16), w8.layout_tensor.int_data, w8.layout_tensor.scale, None, None], 0),
         "fp6_linear": ([3, 2, x(torch.float16), w6.native(), w6.scale], 2),
         "hqq_mixed_mm": ([x(torch.bfloat16), codes, *q, 64, False], 0),
-        "llama_forward": ([model._host_plan("int4", 5), rows, torch.arange(5, device="cuda")], 1),
+        "llama_forward": ([model._host_plan("int4", 5), rows, None, torch.arange(5, device="cuda")], 1),
     }
 
 

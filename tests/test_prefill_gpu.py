@@ -149,23 +149,36 @@ def test_native_pass_is_the_module_chain(quantization, T):
 @pytest.mark.parametrize("T", [1, 33, 130])
 @pytest.mark.parametrize("heads", [(4, 1), (3, 3)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_attention_with_gathered_rotary_rows(T, heads, dtype):
-    """The entry that takes one rotary row a token: bit for bit the other one on the gathered rows; a position outside the cache
-    reads its row and no other."""
+@pytest.mark.parametrize("long", [False, True])
+def test_attention_with_negative_positions(T, heads, dtype, long):
+    """Counted from the end: bit for bit the other entry at the rows they mean, whose rotary rows stand at those rows in a table of
+    its own; a position beyond either end writes no cache row and leaves a NaN row."""
     from ao_amd._models.llama.model import precompute_freqs_cis
 
     n_head, n_kv = heads
-    S = 160
+    S, F = 160, 200
     qkv = _qkv(T, n_head, n_kv, dtype)
-    freqs = precompute_freqs_cis(S, 128, dtype=dtype, device="cuda")
-    pos = torch.randperm(S, device="cuda", generator=torch.Generator(device="cuda").manual_seed(T))[:T]
+    freqs = precompute_freqs_cis(F, 128, dtype=dtype, device="cuda")
+    rows = torch.randperm(S, device="cuda", generator=torch.Generator(device="cuda").manual_seed(T))[:T]
+    negative = torch.arange(T, device="cuda") % 3 == 0
+    pos = torch.where(negative, rows - S, rows)
+    if T > 1:
+        pos[-1], rows[-1], pos[-2], rows[-2] = -S - 1, S, S, S
+    own = torch.zeros(S + 1, 64, 2, device="cuda", dtype=dtype)
+    own[rows] = freqs[pos.clamp(-F, F - 1)]
     results = []
-    for name, f in (("ao_amd_llama_prefill_attention", freqs), ("ao_amd_llama_prefill_attention_rows", freqs[pos])):
+    for wrap in (True, False):
         kc, vc = (torch.ones(n_kv, S, 128, device="cuda", dtype=dtype) for _ in range(2))
         out = torch.full((T, n_head * 128), 7.0, device="cuda", dtype=dtype)
-        _call(name, qkv, int(dtype is torch.float16), f, pos, 1, T, kc, vc, n_head, n_kv, 128, S, out)
+        p = pos if wrap else rows
+        p = p if long else p.int()
+        _call("ao_amd_llama_prefill_attention" + ("_wrap" if wrap else ""), qkv, int(dtype is torch.float16), freqs if wrap else own,
+              *([F] if wrap else []), p, int(long), T, kc, vc, n_head, n_kv, 128, S, out)
         results.append((out, kc, vc))
-    assert all(torch.equal(a, b) for a, b in zip(*results)) and not results[0][0].isnan().any()
+    bad = 2 if T > 1 else 0
+    for a, b in zip(*results):
+        assert torch.equal(a.nan_to_num(9.0), b.nan_to_num(9.0))
+    assert results[0][0].isnan().all(1).sum() == bad == results[0][0].isnan().any(1).sum()
 
 
 @pytest.mark.parametrize("T,heads", [(1025, (8, 2)), (4096, (4, 1)), (2049, (3, 3))])
