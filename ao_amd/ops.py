@@ -89,12 +89,12 @@ TWO_PASS_MIN_M = 4096
 # 1024 / 1500 / 2048 rows 465 / 552, 683 / 684, 860 / 850; 6144 x 4096 at 1500 / 1800 / 2048 rows 80 / 99, 92 / 102, 115 / 107; 4096 x
 # 4096 at 1536 / 2048 / 2500 / 3000 rows 54 / 70, 67 / 80, 88 / 89, 97 / 101, 4096 x 14336 at 2048 / 2500 rows 208 / 242, 277 / 274; 1024 x
 # 4096 at 2048 / 3072 rows 32 / 36, 46 / 41.
-INT8_TWO_PASS_MIN_M = 128
+INT8_TWO_PASS_MIN_M = 1536
 FP6_TWO_PASS_MIN_M = 1537
 
 
 def int8wo_two_pass(M: int, N: int, K: int) -> bool:
-    return M >= INT8_TWO_PASS_MIN_M * (12 if N >= 8192 else 32)
+    return M >= (INT8_TWO_PASS_MIN_M if N >= 8192 else 4096)
 
 
 def fp6_two_pass(M: int, N: int, K: int) -> bool:

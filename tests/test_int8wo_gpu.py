@@ -47,7 +47,7 @@ def test_quantize_bit_exact(oracle, shape):
     assert np.array_equal(zero.cpu().numpy().reshape(-1), z.reshape(-1))
 
 
-@pytest.mark.parametrize("M", [1, 4, 16, 33, 130, 300])  # from 128 rows on the two-pass path is checked as well
+@pytest.mark.parametrize("M", [1, 4, 16, 33, 130, 300])  # at 130 and 300 rows the two-pass path is checked as well
 @pytest.mark.parametrize("shape", [(256, 1024), (48, 256), (1000, 4096)])
 def test_linear_matches_oracle(oracle, shape, M, monkeypatch):
     from ao_amd import ops
@@ -75,8 +75,8 @@ def test_linear_matches_oracle(oracle, shape, M, monkeypatch):
     assert rel_l2(y32, pre) <= 1e-3
     assert rel_l2(y16, expect) <= 1e-3
     assert np.count_nonzero(y16 != expect) <= 0.02 * y16.size + 1
-    if M >= ops.INT8_TWO_PASS_MIN_M:
-        # large weights take the bf16 copy of the codes + the library GEMM from here on (ops.int8wo_two_pass): same bar
+    if M >= 128:
+        # the bf16 copy of the codes + the library GEMM, which prompts take (ops.int8wo_two_pass): same bar
         monkeypatch.setattr(ops, "int8wo_two_pass", lambda M, N, K: True)
         y2p = ops.int8wo_linear(x.to(dev), qd, sd, bd, False).float().cpu().numpy()
         assert rel_l2(y2p, expect) <= 1e-3
