@@ -287,3 +287,34 @@ def test_native_pass_is_its_kernels(fmt, T, intermediate, heads, group, monkeypa
     (plan,) = seen
     two_pass = [lin[4] for layer in plan[8] for lin in layer if isinstance(lin, tuple)]
     assert any(two_pass) == (T >= 1536)
+
+
+@pytest.mark.parametrize("fmt", RECIPES)
+def test_prompts_in_a_captured_graph(fmt):
+    """Replays on other tokens and positions, eager work in between, against eager calls."""
+    model = _model(fmt)
+    tokens, pos = _prompt(model, 33)
+    static = tokens.clone(), pos.clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), torch.no_grad():
+        model(*static)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.no_grad(), torch.cuda.graph(graph):
+        logits = model(*static)
+    for i in range(4):
+        tokens, _ = _prompt(model, 33, 10 + i)
+        with torch.no_grad():
+            want = model(tokens, pos + 20 * i).clone()
+            caches = [c.clone() for c in _caches(model)]
+            for c in _caches(model):
+                c.zero_()
+            model(*_prompt(model, 20 * i)) if i else None
+        static[0].copy_(tokens)
+        static[1].copy_(pos + 20 * i)
+        for c, w in zip(_caches(model), caches):
+            c.copy_(w)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(logits, want) and all(map(torch.equal, _caches(model), caches))
