@@ -5,10 +5,11 @@
 // torch.ops -> Python implementation -> ctypes took 18-26 us of host time, so a program that launches linears one after
 // the other ran at the host's pace (4096 -> 1024, one row: 21.8 us a call for a 5.2 us kernel).
 //
-// Contract of every function here: it serves the plain case (exact torch.Tensor or Parameter arguments on one GPU,
-// dtypes, shapes and strides as the kernels take them, no gradient or tangent to record, no mode, transform or trace active) and
-// returns NotImplemented for everything else *before* it does anything.  The caller then takes the torch.library route,
-// which reports errors, records for torch.compile, and covers the rare layouts.  Nothing is raised here.
+// Contract of every function here: it serves the plain case (exact torch.Tensor or Parameter arguments on one GPU, dtypes, shapes
+// and strides as the kernels take them, no gradient or tangent to record, no mode, transform or trace active) and returns
+// NotImplemented for everything else *before* it launches anything; only a pass of the model may find a shape that a kernel refuses
+// later, and is then run again from its start by another route.  The caller takes the torch.library route, which reports errors,
+// records for torch.compile, and covers the rare layouts.  Nothing is raised here.
 #pragma once
 #include <Python.h>
 
