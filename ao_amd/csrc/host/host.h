@@ -88,7 +88,11 @@ struct Args {
         }
         return r;
     }
-    bool truth(int i) { return v[i] == Py_True; }
+    bool truth(int i) { return truth_of(v[i]); }
+    bool truth_of(PyObject* obj) {
+        if (obj != Py_True && obj != Py_False) ok = false;
+        return obj == Py_True;
+    }
 
  private:
     const Tensor& fail(const Tensor& none) {

@@ -69,7 +69,7 @@ struct Reader {
     Tensor tensor(at::ScalarType t, bool optional = false) { return a.tensor_of(next(), t, optional); }
     int64_t integer() { return a.integer_of(next()); }
     double real() { return a.real_of(next()); }
-    bool truth() { return next() == Py_True; }
+    bool truth() { return a.truth_of(next()); }
 };
 
 Linear read_linear(const Model& m, Args& a, PyObject* tuple) {

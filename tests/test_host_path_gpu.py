@@ -161,3 +161,14 @@ def test_every_function_declines_what_others_have_to_see(name):
     if name != "llama_forward":  # its norms are parameters that ask for a gradient
         assert torch.is_tensor(call())
     assert call(x.clone().requires_grad_()) is NotImplemented
+
+
+def test_hqq_flag_that_is_not_a_bool():
+    """The operator takes a number for `transposed`; on a square weight the other product has the same shape."""
+    from ao_amd import ops
+
+    (x, codes, scales, zeros, group, _), _ = _plain_calls()["hqq_mixed_mm"]
+    want = [ops.hqq_mixed_mm_mfma(x, codes, scales, zeros, group, t) for t in (False, True)]
+    assert not torch.equal(*want)
+    for flag in (0, 1):
+        assert torch.equal(ops.hqq_mixed_mm_mfma(x, codes, scales, zeros, group, flag), want[flag])
