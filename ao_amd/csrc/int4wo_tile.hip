@@ -273,7 +273,8 @@ extern "C" int ao_amd_int4wo_linear_auto(const void* x_bf16, int64_t M, int64_t 
                                          int64_t N, int64_t g, const void* bias_bf16, void* y, int y_dtype, int64_t ldy, void* workspace,
                                          int64_t workspace_bytes, void* stream) {
     AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
-    AO_REQUIRE(ldx >= K, "row stride ldx=%lld smaller than the rows", (long long)ldx);
+    AO_REQUIRE(ldx >= K && ldy >= N, "row strides (ldx=%lld, ldy=%lld) smaller than the rows (K=%lld, N=%lld)", (long long)ldx, (long long)ldy,
+               (long long)K, (long long)N);
     Int4Auto r;
     if (int rc = int4wo_auto(x_bf16, M, K, ldx, N, g, y_dtype, &r)) return rc;
     AO_REQUIRE(r.copy + r.parts == 0 || (workspace && workspace_bytes >= r.copy + r.parts && (((uintptr_t)workspace) & 15) == 0),
