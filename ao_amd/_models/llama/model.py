@@ -307,6 +307,20 @@ class Transformer(nn.Module):
     def fused_decode_ready(self) -> bool:
         return self.fused_decode_kind() is not None
 
+    def _mask_is_own(self) -> bool:
+        """Whether the causal mask is the one that setup_caches made, unchanged."""
+        mask, version = self.__dict__.get("_own_mask", (None, 0))  # a model pickled by an earlier version has none
+        return mask is not None and self.causal_mask is mask and mask._version == version
+
+    # a copy's mask starts with a version of its own
+    def __getstate__(self):
+        return self.__dict__ if self._mask_is_own() else {**self.__dict__, "_own_mask": (None, 0)}
+
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        mask, _ = self.__dict__.get("_own_mask", (None, 0))
+        self._own_mask = (None, 0) if mask is None or mask.is_inference() else (mask, mask._version)
+
     def _calls_are_watched(self) -> bool:
         """Whether somebody wants to see the calls of every module, or replaced a function that the modules call."""
         hooks = torch.nn.modules.module
@@ -324,8 +338,7 @@ class Transformer(nn.Module):
         if self._calls_are_watched():
             return False
         cfg = self.config
-        mask, version = self.__dict__.get("_own_mask", (None, 0))  # a model pickled by an earlier version has none
-        if mask is None or self.causal_mask is not mask or mask._version != version:
+        if not self._mask_is_own():
             return False
         if not (_is_plain(self.norm) and _is_plain(self.output)):
             return False

@@ -318,3 +318,25 @@ def test_prompts_in_a_captured_graph(fmt):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(logits, want) and all(map(torch.equal, _caches(model), caches))
+
+
+@pytest.mark.parametrize("how", ["deepcopy", "file"])
+def test_copies_of_a_model_take_the_native_pass(how, monkeypatch, tmp_path):
+    """Unless their mask had been changed before."""
+    import copy
+
+    from ao_amd import ops
+
+    def copied(model):
+        if how == "deepcopy":
+            return copy.deepcopy(model)
+        torch.save(model, tmp_path / "model.pt")
+        return torch.load(tmp_path / "model.pt", weights_only=False)
+
+    model = _model("int8")
+    seen, native = [], ops.host.llama_forward
+    monkeypatch.setattr(ops.host, "llama_forward", lambda *a: seen.append(native(*a)) or seen[-1])
+    want = _both(model, *_prompt(model, 17))[0]
+    assert _same(_both(copied(model), *_prompt(model, 17))[0], want) and len(seen) == 2 and all(map(torch.is_tensor, seen))
+    model.causal_mask.fill_(True)
+    assert _same(*_both(copied(model), *_prompt(model, 17))) and len(seen) == 2
