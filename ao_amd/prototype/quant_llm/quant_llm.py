@@ -91,11 +91,11 @@ def _fpx_linear(act, weight, bias=None):
     split from the shape)."""
     assert isinstance(weight, QuantLlmLinearWeight)
     if type(act) is Tensor and not torch.compiler.is_dynamo_compiling():
-        N, row_bytes = weight.fpx_data.shape
-        K = row_bytes // weight.nbits * 8
-        # the rows are compared here: the kernel's tile order is padded to 128 columns and does not say where they end
-        if act.dim() > 0 and act.shape[-1] == K and not ops.fp6_two_pass(act.numel() // max(K, 1), N, K):
-            out = ops.host.fp6_linear(weight.ebits, weight.mbits, act, weight.native(), weight.scale)
+        ebits, mbits, shape, (N, row_bytes) = weight.ebits, weight.mbits, act.shape, weight.fpx_data.shape
+        # the widths are compared here: the kernel's tile order is padded to 128 columns and does not say where the rows end
+        K = shape[-1] if shape else 0
+        if K and K * (1 + ebits + mbits) == 8 * row_bytes and not ops.fp6_two_pass(act.numel() // K, N, K):
+            out = ops.host.fp6_linear(ebits, mbits, act, weight.native(), weight.scale)
             if out is not NotImplemented:
                 if bias is not None:
                     out += bias
