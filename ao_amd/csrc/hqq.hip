@@ -3,14 +3,12 @@
 // The reference's Triton kernel (torchao/prototype/hqq/kernels.py:200-380) multiplies activations with a weight kept
 // as `pack_2xint4(W_q.T)`: uint8 [K/2, N], byte (k2, n) = W_q[n][2*k2] | W_q[n][2*k2 + 1] << 4
 // (torchao/prototype/hqq/mixed_mm.py:13-35), with scales and zeros of shape [K/group, N] in the activation dtype, and
-// dequantizes in that dtype, op by op: w = (q - zero) * scale (kernels.py:358).  Here the dequantization is a pass of
-// its own into a [K, N] matrix of the activation dtype, followed by a plain library GEMM (x @ W for the forward
-// product over K, x @ W^T for the transposed product over N that the backward pass of a fine-tuning run needs):
-// the packed layout is N-major, so a thread that takes 16 consecutive bytes of one k2 row produces two 32-byte
+// dequantizes in that dtype, op by op: w = (q - zero) * scale (kernels.py:358).  The products of few rows (x @ W over K, and x @ W^T over N,
+// which the backward pass of a fine-tuning run needs) are fused below.  For the others the dequantization is a pass of its own into a [K, N] matrix of the activation dtype, followed by a plain library GEMM: the packed layout is N-major, so a thread that takes 16 consecutive bytes of one k2 row produces two 32-byte
 // runs of the output rows 2*k2 and 2*k2 + 1, and neighbouring threads continue those rows.
 #include <type_traits>
 
-#include "common.h"
+#include "hqq_format.h"
 
 namespace ao {
 
@@ -173,19 +171,30 @@ __global__ __launch_bounds__(256) void hqq_mm_small_kernel(const uint8_t* __rest
     }
 }
 
+// four sums a thread; N is a multiple of 4
 template <bool BF16>
 __global__ __launch_bounds__(256) void hqq_mm_finish_kernel(const float* __restrict__ part, int slices, int64_t MN,
                                                             uint16_t* __restrict__ y) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= MN) return;
-    float s = 0.f;
-    for (int z = 0; z < slices; ++z) s += part[(int64_t)z * MN + i];
-    if (BF16) {
-        y[i] = hw_bf16_bits(s);
-    } else {
-        const _Float16 h = (_Float16)s;
-        __builtin_memcpy(&y[i], &h, 2);
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int z = 0; z < slices; ++z) {
+        const float4 v = *reinterpret_cast<const float4*>(part + (int64_t)z * MN + i);
+        s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
     }
+    uint16_t o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = BF16 ? hw_bf16_bits(s[e]) : f32_to_f16_bits(s[e]);
+    if (((uintptr_t)y & 7) == 0)
+        *reinterpret_cast<uint2*>(y + i) = make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
+    else
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[i + e] = o[e];
+}
+void launch_hqq_finish(const float* part, int slices, int64_t count, bool bf16, uint16_t* y, hipStream_t st) {
+    const dim3 grid((unsigned)((count / 4 + 255) / 256));
+    if (bf16) hipLaunchKernelGGL(hqq_mm_finish_kernel<true>, grid, dim3(256), 0, st, part, slices, count, y);
+    else hipLaunchKernelGGL(hqq_mm_finish_kernel<false>, grid, dim3(256), 0, st, part, slices, count, y);
 }
 
 // K slices of the small-M product: enough waves to occupy the chip, at least 8 byte rows per wave
@@ -218,7 +227,6 @@ static int hqq_mm_slices(int64_t K, int64_t N) {
 // is rounded twice to the storage dtype, exactly as hqq_dequantize_kernel rounds it.
 typedef __bf16 hqq_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 hqq_f16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 hqq_f16x2_t __attribute__((ext_vector_type(2)));
 typedef float hqq_f32x4_t __attribute__((ext_vector_type(4)));
 
 template <bool BF16>
@@ -233,45 +241,6 @@ __device__ __forceinline__ hqq_f32x4_t hqq_mfma(const u32x4_t a, const uint32_t 
         xa.q = a;
         xb.q = u32x4_t{b[0], b[1], b[2], b[3]};
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(xa.v, xb.v, c, 0, 0, 0);
-    }
-}
-
-// The eight codes of a dword of four byte rows or columns -> low and high nibbles as one byte each: the byte-to-float
-// conversions and byte permutes below then take them in place (shifting every code down to bit 0 first cost a third of the
-// kernel's instructions).  The sign bit of a signed nibble is flipped: code = byte - 8.
-template <bool SIGNED>
-__device__ __forceinline__ void hqq_nibbles(uint32_t w, uint32_t& lo, uint32_t& hi) {
-    lo = w & 0x0f0f0f0fu;
-    hi = (w >> 4) & 0x0f0f0f0fu;
-    if (SIGNED) {
-        lo ^= 0x08080808u;
-        hi ^= 0x08080808u;
-    }
-}
-// codes in bytes B0 of `a` and B1 of `b` -> the weight pair (q - z) * s, each operation rounded to the storage type; scales
-// and zeros as a packed pair (fp16) or as fp32 values (bf16)
-template <bool BF16, bool SIGNED, int B0, int B1>
-__device__ __forceinline__ uint32_t hqq_pair(uint32_t a, uint32_t b, uint32_t s2, uint32_t z2, float s0, float s1, float z0, float z1) {
-    if (BF16) {
-        float q0 = (float)((a >> (8 * B0)) & 0xffu), q1 = (float)((b >> (8 * B1)) & 0xffu);
-        if (SIGNED) {
-            q0 -= 8.0f;   // exact
-            q1 -= 8.0f;
-        }
-        return hw_bf16_pack(hw_rne_bf16(q0 - z0) * s0, hw_rne_bf16(q1 - z1) * s1);
-    } else {
-        // 0x6400 | u is the fp16 value 1024 + u, exactly: one byte permute builds the pair without a conversion
-        const uint32_t m = __builtin_amdgcn_perm(b, a, 0x0c000c00u | B0 | ((4u + B1) << 16)) | 0x64006400u;
-        hqq_f16x2_t q, s, z;
-        __builtin_memcpy(&q, &m, 4);
-        __builtin_memcpy(&s, &s2, 4);
-        __builtin_memcpy(&z, &z2, 4);
-        const _Float16 off = SIGNED ? (_Float16)1032.0f : (_Float16)1024.0f;
-        q = q - hqq_f16x2_t{off, off};                 // exact
-        const hqq_f16x2_t w = (q - z) * s;             // each op rounds to fp16
-        uint32_t r;
-        __builtin_memcpy(&r, &w, 4);
-        return r;
     }
 }
 
@@ -365,17 +334,20 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
                     zf[c] = __uint_as_float(zh << 16);
                 }
             }
-            uint32_t lo[4], hi[4];
+            uint32_t lo[4], hi[4], w[4][4];   // w: [column][byte row]
 #pragma unroll
-            for (int r = 0; r < 4; ++r) hqq_nibbles<SIGNED>(f.d[r], lo[r], hi[r]);
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (BF16) hqq_columns<SIGNED>(f.d[r], zf, sf, w[0][r], w[1][r], w[2][r], w[3][r]);
+                else hqq_nibbles<SIGNED>(f.d[r], lo[r], hi[r]);
+            }
             // both nibbles of byte c belong to column c
             auto column = [&](auto c_c) {
                 constexpr int c = decltype(c_c)::value;
-                uint32_t w[4];
+                if constexpr (!BF16)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) w[r] = hqq_pair<BF16, SIGNED, c, c>(lo[r], hi[r], sv[c], zv[c], sf[c], sf[c], zf[c], zf[c]);
+                    for (int r = 0; r < 4; ++r) w[c][r] = hqq_pair<SIGNED, c, c>(lo[r], hi[r], sv[c], zv[c]);
 #pragma unroll
-                for (int mb = 0; mb < MB; ++mb) acc[mb][c] = hqq_mfma<BF16>(f.x[mb], w, acc[mb][c]);
+                for (int mb = 0; mb < MB; ++mb) acc[mb][c] = hqq_mfma<BF16>(f.x[mb], w[c], acc[mb][c]);
             };
             column(std::integral_constant<int, 0>());
             column(std::integral_constant<int, 1>());
@@ -416,13 +388,13 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
             for (int h = 0; h < 2; ++h) {
                 const uint32_t ss[4] = {f.s[h].x, f.s[h].y, f.s[h].z, f.s[h].w};
                 const uint32_t zz[4] = {f.z[h].x, f.z[h].y, f.z[h].z, f.z[h].w};
-                float sl[4], sh[4], zl[4], zh[4];
+                float sf[8], zf[8];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    sl[i] = __uint_as_float(ss[i] << 16);
-                    sh[i] = __uint_as_float(ss[i] & 0xffff0000u);
-                    zl[i] = __uint_as_float(zz[i] << 16);
-                    zh[i] = __uint_as_float(zz[i] & 0xffff0000u);
+                    sf[2 * i] = __uint_as_float(ss[i] << 16);
+                    sf[2 * i + 1] = __uint_as_float(ss[i] & 0xffff0000u);
+                    zf[2 * i] = __uint_as_float(zz[i] << 16);
+                    zf[2 * i + 1] = __uint_as_float(zz[i] & 0xffff0000u);
                 }
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb) {
@@ -431,12 +403,18 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
 #pragma unroll
                     for (int i = 0; i < 4; i += 2) {
                         // reduction indices 8 h + 2 i .. + 3: the four bytes of dword 2 h + i / 2
-                        uint32_t nl, nh;
-                        hqq_nibbles<SIGNED>(dd[2 * h + (i >> 1)], nl, nh);
-                        lo[i] = hqq_pair<BF16, SIGNED, 0, 1>(nl, nl, ss[i], zz[i], sl[i], sh[i], zl[i], zh[i]);
-                        hi[i] = hqq_pair<BF16, SIGNED, 0, 1>(nh, nh, ss[i], zz[i], sl[i], sh[i], zl[i], zh[i]);
-                        lo[i + 1] = hqq_pair<BF16, SIGNED, 2, 3>(nl, nl, ss[i + 1], zz[i + 1], sl[i + 1], sh[i + 1], zl[i + 1], zh[i + 1]);
-                        hi[i + 1] = hqq_pair<BF16, SIGNED, 2, 3>(nh, nh, ss[i + 1], zz[i + 1], sl[i + 1], sh[i + 1], zl[i + 1], zh[i + 1]);
+                        const uint32_t d = dd[2 * h + (i >> 1)];
+                        if constexpr (BF16) {
+                            hqq_row<SIGNED, false>(d, zf + 2 * i, sf + 2 * i, lo[i], lo[i + 1]);
+                            hqq_row<SIGNED, true>(d, zf + 2 * i, sf + 2 * i, hi[i], hi[i + 1]);
+                        } else {
+                            uint32_t nl, nh;
+                            hqq_nibbles<SIGNED>(d, nl, nh);
+                            lo[i] = hqq_pair<SIGNED, 0, 1>(nl, nl, ss[i], zz[i]);
+                            hi[i] = hqq_pair<SIGNED, 0, 1>(nh, nh, ss[i], zz[i]);
+                            lo[i + 1] = hqq_pair<SIGNED, 2, 3>(nl, nl, ss[i + 1], zz[i + 1]);
+                            hi[i + 1] = hqq_pair<SIGNED, 2, 3>(nh, nh, ss[i + 1], zz[i + 1]);
+                        }
                     }
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb) {
@@ -564,11 +542,7 @@ extern "C" int ao_amd_hqq_mixed_mm(const void* a, int64_t M, int64_t K, int64_t 
 #undef AO_HQQ_MM_M
 #undef AO_HQQ_MM
     AO_LAUNCH_CHECK();
-    const int64_t MN = M * N;
-    if (dtype == AO_BF16)
-        hipLaunchKernelGGL(hqq_mm_finish_kernel<true>, dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, st, part, slices, MN, (uint16_t*)y);
-    else
-        hipLaunchKernelGGL(hqq_mm_finish_kernel<false>, dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, st, part, slices, MN, (uint16_t*)y);
+    launch_hqq_finish(part, slices, M * N, dtype == AO_BF16, (uint16_t*)y, st);
     AO_LAUNCH_CHECK();
     return 0;
 }
@@ -671,11 +645,7 @@ extern "C" int ao_amd_hqq_mixed_mm_mfma(const void* a, int64_t M, int64_t lda, c
 #undef AO_HQQ_MFMA_M
 #undef AO_HQQ_MFMA
     AO_LAUNCH_CHECK();
-    const int64_t MC = M * (transposed ? K : N);
-    if (dtype == AO_BF16)
-        hipLaunchKernelGGL(hqq_mm_finish_kernel<true>, dim3((unsigned)((MC + 255) / 256)), dim3(256), 0, st, part, p.slices, MC, (uint16_t*)y);
-    else
-        hipLaunchKernelGGL(hqq_mm_finish_kernel<false>, dim3((unsigned)((MC + 255) / 256)), dim3(256), 0, st, part, p.slices, MC, (uint16_t*)y);
+    launch_hqq_finish(part, p.slices, M * (transposed ? K : N), dtype == AO_BF16, (uint16_t*)y, st);
     AO_LAUNCH_CHECK();
     return 0;
 }

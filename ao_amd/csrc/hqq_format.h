@@ -1,0 +1,89 @@
+// HQQ two-per-byte codes in registers: for the kernels of hqq.hip.
+#pragma once
+#include "common.h"
+
+namespace ao {
+
+typedef _Float16 hqq_f16x2_t __attribute__((ext_vector_type(2)));
+
+// The eight codes of a dword of four byte rows or columns -> low and high nibbles as one byte each: the byte-to-float
+// conversions and byte permutes below then take them in place (shifting every code down to bit 0 first cost a third of the
+// kernel's instructions).  The sign bit of a signed nibble is flipped: code = byte - 8.
+template <bool SIGNED>
+__device__ __forceinline__ void hqq_nibbles(uint32_t w, uint32_t& lo, uint32_t& hi) {
+    lo = w & 0x0f0f0f0fu;
+    hi = (w >> 4) & 0x0f0f0f0fu;
+    if (SIGNED) {
+        lo ^= 0x08080808u;
+        hi ^= 0x08080808u;
+    }
+}
+// fp16: codes in bytes B0 of `a` and B1 of `b` -> the weight pair (q - z) * s, each operation rounded
+template <bool SIGNED, int B0, int B1>
+__device__ __forceinline__ uint32_t hqq_pair(uint32_t a, uint32_t b, uint32_t s2, uint32_t z2) {
+    // 0x6400 | u is the fp16 value 1024 + u, exactly: one byte permute builds the pair without a conversion
+    const uint32_t m = __builtin_amdgcn_perm(b, a, 0x0c000c00u | B0 | ((4u + B1) << 16)) | 0x64006400u;
+    hqq_f16x2_t q, s, z;
+    __builtin_memcpy(&q, &m, 4);
+    __builtin_memcpy(&s, &s2, 4);
+    __builtin_memcpy(&z, &z2, 4);
+    const _Float16 off = SIGNED ? (_Float16)1032.0f : (_Float16)1024.0f;
+    q = q - hqq_f16x2_t{off, off};                 // exact
+    const hqq_f16x2_t w = (q - z) * s;             // each op rounds to fp16
+    uint32_t r;
+    __builtin_memcpy(&r, &w, 4);
+    return r;
+}
+
+// bf16: the weights of the nibbles at bits (0, 16) or, ODD, (4, 20) of p, as fp32 products that the caller rounds to bf16.  The masked
+// nibble is the fp16 subnormal q 2^-24 (q 2^-20), which a mixed fma turns into q - z with the one rounding of the subtraction;
+// with a zero low operand the conversion leaves bf16(q - z) in the high half, an fp32 again.  33 instructions for 8
+// weights, where a byte conversion and a subtraction for each took 39.  SIGNED: p has its sign bits flipped, code = nibble - 8.
+template <bool SIGNED, bool ODD>
+__device__ __forceinline__ void hqq_products(uint32_t p, float z0, float z1, float s0, float s1, float& w0, float& w1) {
+    p &= ODD ? 0x00F000F0u : 0x000F000Fu;
+    const float up = ODD ? 0x1p20f : 0x1p24f;
+    float t0, t1;
+    if (SIGNED) {   // - 8 is exact
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(t0) : "v"(p), "s"(up), "v"(-8.0f));
+        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(t1) : "v"(p), "s"(up), "v"(-8.0f));
+        t0 -= z0;
+        t1 -= z1;
+    } else {
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[1,0,0]" : "=v"(t0) : "v"(p), "s"(up), "v"(z0));
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(t1) : "v"(p), "s"(up), "v"(z1));
+    }
+    w0 = hw_rne_bf16(t0) * s0;
+    w1 = hw_rne_bf16(t1) * s1;
+}
+// a dword of four bytes along n.  Columns: the (low, high) pair of bytes O and O + 2, whose columns' zeros and scales are z[O], z[O + 2] ..
+template <bool SIGNED, int O>
+__device__ __forceinline__ void hqq_columns2(uint32_t d, const float* z, const float* s, uint32_t& c0, uint32_t& c2) {
+    if (SIGNED) d ^= 0x88888888u;
+    if (O) d >>= 8;
+    float l0, l2, h0, h2;
+    hqq_products<SIGNED, false>(d, z[O], z[O + 2], s[O], s[O + 2], l0, l2);
+    hqq_products<SIGNED, true>(d, z[O], z[O + 2], s[O], s[O + 2], h0, h2);
+    c0 = hw_bf16_pack(l0, h0);
+    c2 = hw_bf16_pack(l2, h2);
+}
+template <bool SIGNED>
+__device__ __forceinline__ void hqq_columns(uint32_t d, const float* z, const float* s, uint32_t& c0, uint32_t& c1, uint32_t& c2, uint32_t& c3) {
+    hqq_columns2<SIGNED, 0>(d, z, s, c0, c2);
+    hqq_columns2<SIGNED, 1>(d, z, s, c1, c3);
+}
+// .. Row: the four low or, HIGH, high nibbles as two pairs
+template <bool SIGNED, bool HIGH>
+__device__ __forceinline__ void hqq_row(uint32_t d, const float* z, const float* s, uint32_t& p0, uint32_t& p1) {
+    if (SIGNED) d ^= 0x88888888u;
+    float w0, w1, w2, w3;
+    hqq_products<SIGNED, HIGH>(d, z[0], z[2], s[0], s[2], w0, w2);
+    hqq_products<SIGNED, HIGH>(d >> 8, z[1], z[3], s[1], s[3], w1, w3);
+    p0 = hw_bf16_pack(w0, w1);
+    p1 = hw_bf16_pack(w2, w3);
+}
+
+// fp32 partial sums [slices][rows x columns], a multiple of 4 of them, added and rounded to bf16 or fp16
+void launch_hqq_finish(const float* part, int slices, int64_t count, bool bf16, uint16_t* y, hipStream_t st);
+
+}  // namespace ao
