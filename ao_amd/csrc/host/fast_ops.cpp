@@ -83,8 +83,10 @@ PyObject* fp6_linear(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     });
 }
 
-// (a, codes, scales, zeros, group_size, transposed): the fused matrix-core product over HQQ codes
-PyObject* hqq_mixed_mm(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
+// (a, codes, scales, zeros, group_size, transposed): the fused products over HQQ codes, of up to 64 rows or, MANY, of more by its tiles where
+// they are faster than the dequantized weight and torch.matmul, which autocast casts
+template <bool MANY>
+PyObject* hqq_product(PyObject* const* v, Py_ssize_t nargs) {
     AO_NEED(6);
     at::ScalarType dtype;
     const Tensor& x = a.tensor16(0, dtype);
@@ -97,19 +99,35 @@ PyObject* hqq_mixed_mm(PyObject*, PyObject* const* v, Py_ssize_t nargs) {
     AO_WANT(g > 0 && x.dim() == 2 && b.dim() == 2 && b.is_contiguous() && scales.dim() == 2 && scales.is_contiguous() && zeros.is_contiguous() &&
             scales.sizes() == zeros.sizes());
     const int64_t M = x.size(0), K = 2 * b.size(0), N = b.size(1), R = transposed ? N : K;
-    AO_WANT(x.size(1) == R && x.stride(1) == 1 && x.stride(0) % 8 == 0 && (uintptr_t)ptr(x) % 16 == 0 && M >= 1 && M <= 64 &&
+    AO_WANT(x.size(1) == R && x.stride(1) == 1 && x.stride(0) % 8 == 0 && (uintptr_t)ptr(x) % 16 == 0 && M >= 1 && MANY == (M > 64) &&
             scales.size(0) * g == K && scales.size(1) == N);
     AO_WANT(transposed ? N % 16 == 0 && g % 2 == 0 : K % 8 == 0 && g % 8 == 0 && N % 4 == 0);
+    const int code = dtype == at::kBFloat16 ? AO_BF16 : AO_F16;
+    if (MANY) {
+        AO_WANT(!at::autocast::is_autocast_enabled(at::kCUDA) && x.stride(0) < ((int64_t)1 << 24));
+        int64_t need = -1;
+        AO_CALL(ao_amd_hqq_mixed_mm_tiled_bytes(M, K, N, g, code, transposed, &need));
+        AO_WANT(need >= 0);
+        return guarded([&]() -> PyObject* {
+            Tensor y = empty({M, transposed ? K : N}, dtype, a.device), ws;
+            if (need) ws = workspace(need, a.device);
+            AO_CALL(ao_amd_hqq_mixed_mm_tiled(ptr(x), M, x.stride(0), ptr(b), is_signed, K, N, ptr(scales), ptr(zeros), g, code, transposed,
+                                              need ? ws.data_ptr() : nullptr, need, y.data_ptr(), stream_of(a.device)));
+            return THPVariable_Wrap(std::move(y));
+        });
+    }
     return guarded([&]() -> PyObject* {
         int64_t need = 0;
         AO_CALL(ao_amd_hqq_mixed_mm_mfma_workspace(M, K, N, transposed, &need));
         Tensor y = empty({M, transposed ? K : N}, dtype, a.device), ws = workspace(need, a.device);
-        AO_CALL(ao_amd_hqq_mixed_mm_mfma(ptr(x), M, x.stride(0), ptr(b), is_signed, K, N, ptr(scales), ptr(zeros), g,
-                                         dtype == at::kBFloat16 ? AO_BF16 : AO_F16, transposed, ws.data_ptr(), need, y.data_ptr(),
-                                         stream_of(a.device)));
+        AO_CALL(ao_amd_hqq_mixed_mm_mfma(ptr(x), M, x.stride(0), ptr(b), is_signed, K, N, ptr(scales), ptr(zeros), g, code,
+                                         transposed, ws.data_ptr(), need, y.data_ptr(), stream_of(a.device)));
         return THPVariable_Wrap(std::move(y));
     });
 }
+
+PyObject* hqq_mixed_mm(PyObject*, PyObject* const* v, Py_ssize_t nargs) { return hqq_product<false>(v, nargs); }
+PyObject* hqq_mixed_mm_many(PyObject*, PyObject* const* v, Py_ssize_t nargs) { return hqq_product<true>(v, nargs); }
 
 #define AO_METHOD(f) {#f, (PyCFunction)(void (*)(void))f, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
@@ -117,6 +135,7 @@ PyMethodDef methods[] = {
     AO_METHOD(int8wo_linear),
     AO_METHOD(fp6_linear),
     AO_METHOD(hqq_mixed_mm),
+    AO_METHOD(hqq_mixed_mm_many),
     {"llama_forward", (PyCFunction)(void (*)(void))llama_forward, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

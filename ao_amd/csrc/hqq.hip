@@ -3,8 +3,9 @@
 // The reference's Triton kernel (torchao/prototype/hqq/kernels.py:200-380) multiplies activations with a weight kept
 // as `pack_2xint4(W_q.T)`: uint8 [K/2, N], byte (k2, n) = W_q[n][2*k2] | W_q[n][2*k2 + 1] << 4
 // (torchao/prototype/hqq/mixed_mm.py:13-35), with scales and zeros of shape [K/group, N] in the activation dtype, and
-// dequantizes in that dtype, op by op: w = (q - zero) * scale (kernels.py:358).  The products of few rows (x @ W over K, and x @ W^T over N,
-// which the backward pass of a fine-tuning run needs) are fused below.  For the others the dequantization is a pass of its own into a [K, N] matrix of the activation dtype, followed by a plain library GEMM: the packed layout is N-major, so a thread that takes 16 consecutive bytes of one k2 row produces two 32-byte
+// dequantizes in that dtype, op by op: w = (q - zero) * scale (kernels.py:358).  The products (x @ W over K, and x @ W^T over N,
+// which the backward pass of a fine-tuning run needs) are fused below and in hqq_tile.hip.  For what those do not take the
+// dequantization is a pass of its own into a [K, N] matrix of the activation dtype, followed by a plain library GEMM: the packed layout is N-major, so a thread that takes 16 consecutive bytes of one k2 row produces two 32-byte
 // runs of the output rows 2*k2 and 2*k2 + 1, and neighbouring threads continue those rows.
 #include <type_traits>
 
@@ -580,9 +581,14 @@ extern "C" int ao_amd_hqq_mixed_mm_mfma_workspace(int64_t M, int64_t K, int64_t 
     AO_REQUIRE(bytes, "null pointer argument");
     AO_REQUIRE(M >= 1 && M <= 64 && K > 0 && N > 0 && K % 2 == 0, "need 1 <= M <= 64, K even, got M=%lld K=%lld N=%lld",
                (long long)M, (long long)K, (long long)N);
-    // whatever the group size: the plan depends on whether it is a multiple of 64
+    // whatever the group size and the type: the plans depend on whether it is a multiple of 64, and on the type
     const int a = hqq_mfma_plan(M, K, N, transposed != 0, 64).slices, b = hqq_mfma_plan(M, K, N, transposed != 0, 2).slices;
-    *bytes = (int64_t)(a > b ? a : b) * M * (transposed ? K : N) * (int64_t)sizeof(float);
+    int most = a > b ? a : b;
+    for (int bf16 = 0; bf16 < 2; ++bf16) {
+        const HqqTilePlan t = hqq_tile_plan(M, K, N, 64, transposed != 0, bf16 != 0);
+        if (hqq_tiled(t, M, K, N, transposed != 0, bf16 != 0) && t.parts > most) most = t.parts;
+    }
+    *bytes = (int64_t)most * M * (transposed ? K : N) * (int64_t)sizeof(float);
     return 0;
 }
 
@@ -613,6 +619,13 @@ extern "C" int ao_amd_hqq_mixed_mm_mfma(const void* a, int64_t M, int64_t lda, c
     if (int rc = ao_amd_hqq_mixed_mm_mfma_workspace(M, K, N, transposed, &need)) return rc;
     AO_REQUIRE(workspace_bytes >= need && (((uintptr_t)workspace) & 15) == 0, "16-byte aligned workspace of %lld bytes needed, got %lld",
                (long long)need, (long long)workspace_bytes);
+    const HqqTilePlan t = hqq_tile_plan(M, K, N, group_size, transposed != 0, dtype == AO_BF16);
+    if (hqq_tiled(t, M, K, N, transposed != 0, dtype == AO_BF16) && (((uintptr_t)y) & 15) == 0 && lda < (1 << 24)) {
+        launch_hqq_tile(t, (const uint8_t*)packed_2xint4, (const uint16_t*)scales, (const uint16_t*)zeros, (const uint16_t*)a, lda, M, K, N, group_size,
+                        is_signed != 0, dtype == AO_BF16, transposed != 0, (float*)workspace, (uint16_t*)y, (hipStream_t)stream);
+        AO_LAUNCH_CHECK();
+        return 0;
+    }
     const HqqMfmaPlan p = hqq_mfma_plan(M, K, N, transposed != 0, group_size);
     const dim3 grid((unsigned)p.tiles, (unsigned)p.slices);
     hipStream_t st = (hipStream_t)stream;

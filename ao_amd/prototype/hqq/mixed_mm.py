@@ -1,9 +1,10 @@
 """Mixed matmul over HQQ-format int4 weights (reference torchao/prototype/hqq/mixed_mm.py).
 
-The reference fuses the dequantization into a Triton GEMM.  Here both products (forward over K, transposed over N) of up
-to 64 activation rows run a fused matrix-core HIP kernel that streams the packed codes once and dequantizes them in
-registers; more rows dequantize the weight with a HIP kernel into a matrix of the activation dtype, op by op as the
-reference's kernel does ((q - zero) * scale, kernels.py:318-358), and call the vendor GEMM on it.
+The reference fuses the dequantization into a Triton GEMM.  Here both products (forward over K, transposed over N) run fused
+matrix-core HIP kernels that dequantize the packed codes in registers: streaming kernels and tiles up to 64 activation rows, tiles
+beyond.  Calls of more rows that the tiles do not take (gradients, traces, other groupings) or where they are slower (some hundreds of
+rows on large weights) dequantize the weight with a HIP kernel into a matrix of the activation dtype, op by op as the reference's
+kernel does ((q - zero) * scale, kernels.py:318-358), and call the vendor GEMM on it.
 """
 import torch
 
@@ -53,6 +54,10 @@ def mixed_mm(a, b, scales, zeros, group_size, transposed=False, acc_dtype=None, 
             return ops.hqq_mixed_mm_mfma(a, b, scales, zeros, group_size, False)
     if not transposed and 1 <= M <= FUSED_MAX_ROWS and N % 4 == 0:
         return ops.hqq_mixed_mm_small(a, b, scales, zeros, group_size)
+    if M > MFMA_MAX_ROWS and scales.shape[0] * group_size == 2 * K2:
+        y = ops.host.hqq_mixed_mm_many(a, b, scales, zeros, group_size, transposed)
+        if y is not NotImplemented:
+            return y
     w = ops.hqq_dequantize(b, scales, zeros, group_size)  # [K, N]
     return torch.matmul(a, w.t() if transposed else w)
 

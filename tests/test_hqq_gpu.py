@@ -292,3 +292,94 @@ def test_matrix_core_product_over_its_plans(M, N, K, g, transposed):
     got = ops.hqq_mixed_mm_mfma(x, pack_2xint4(q), s, z, g, transposed)
     want = (x.double() @ (w.t() if transposed else w)).bfloat16()
     assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 1.5e-3
+
+
+def _tiled(x, packed, s, z, g, transposed, workspace=True):
+    """ao_amd_hqq_mixed_mm_tiled itself, with room for 16 parts or without a workspace (the reduction is then not split)."""
+    from ao_amd._lib import BF16, F16, check, current_stream, lib
+
+    M, (K2, N) = x.shape[0], packed.shape
+    y = torch.empty(M, 2 * K2 if transposed else N, dtype=x.dtype, device=x.device)
+    ws = torch.empty(16 * y.numel() if workspace else 4, dtype=torch.float32, device=x.device)
+    check(lib().ao_amd_hqq_mixed_mm_tiled(x.data_ptr(), M, x.stride(0), packed.data_ptr(), int(packed.dtype is torch.int8), 2 * K2, N,
+                                          s.data_ptr(), z.data_ptr(), g, BF16 if x.dtype is torch.bfloat16 else F16, int(transposed),
+                                          ws.data_ptr(), ws.numel() * 4 if workspace else 0, y.data_ptr(), current_stream(x.device)))
+    return y
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("dtype,signed", [(torch.bfloat16, False), (torch.bfloat16, True), (torch.float16, False), (torch.float16, True)])
+@pytest.mark.parametrize("M,N,K,g", [(1, 16, 64, 64), (32, 80, 192, 64), (33, 272, 1088, 64), (64, 2960, 128, 128), (65, 144, 4224, 128),
+                                     (96, 1040, 640, 128), (97, 4080, 512, 256), (193, 48, 576, 192)])
+def test_tiled_product(M, N, K, g, dtype, signed, transposed):
+    """Tiles of 32, 64 and 96 rows with full and ragged last tiles, column tiles that end early, reductions that end inside a step
+    (N = 16, 80, 272 .. transposed), waves without a step, split reductions.  Reference: the float64 product with the dequantized
+    weight, rounded once; products summed in fp32 in any order stay within 1.5e-3 (bf16) and 3e-4 (fp16) of it.  One-hot rows give
+    single weights back bit for bit.  What lies behind the rows' ends is NaN and must not be read into a product."""
+    from ao_amd import ops
+    from ao_amd.prototype.hqq import pack_2xint4
+
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    q = torch.randint(-8 if signed else 0, 8 if signed else 16, (K, N), dtype=torch.int8 if signed else torch.uint8, device="cuda", generator=gen)
+    s = (torch.rand(K // g, N, device="cuda", generator=gen) * 0.02 + 1e-3).to(dtype)
+    z = (torch.rand(K // g, N, device="cuda", generator=gen) * 6 - (3 if signed else -5)).to(dtype)
+    packed = pack_2xint4(q)
+    w = ops.hqq_dequantize(packed, s, z, g)
+    R = N if transposed else K
+    xp = torch.full((M + 1, R + 8), float("nan"), dtype=dtype, device="cuda")
+    x = xp[:M, :R]
+    x.copy_(torch.randn(M, R, device="cuda", generator=gen).to(dtype))
+    want = (x.double() @ (w.t() if transposed else w).double()).to(dtype).double()
+    for workspace in (True, False):
+        got = _tiled(x, packed, s, z, g, transposed, workspace).double()
+        assert ((got - want).norm() / want.norm()).item() <= (1.5e-3 if dtype is torch.bfloat16 else 3e-4)
+    at = torch.randint(0, R, (M,), device="cuda", generator=gen)
+    at[0], at[-1] = 0, R - 1
+    x.zero_()
+    x[torch.arange(M, device="cuda"), at] = 1.0
+    assert torch.equal(_tiled(x, packed, s, z, g, transposed), (w.t() if transposed else w)[at].contiguous())
+
+
+def test_tiled_product_refusals():
+    x = torch.zeros(70, 128, dtype=torch.bfloat16, device="cuda")
+    q = torch.zeros(64, 128, dtype=torch.uint8, device="cuda")
+    for g, n in ((32, 128), (64, 120)):
+        sz = torch.zeros(128 // g, n, dtype=torch.bfloat16, device="cuda")
+        with pytest.raises(RuntimeError, match="multiple"):
+            _tiled(x, q[:, :n].contiguous(), sz, sz, g, False)
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+def test_mixed_mm_of_many_rows_keeps_its_other_routes(transposed):
+    """Beyond 64 rows plain calls take the tiles; gradients, autocast, other layouts of the activations and groupings that the tiles
+    refuse run the dequantized weight and torch.matmul as before."""
+    from ao_amd import ops
+    from ao_amd.prototype.hqq.mixed_mm import mixed_mm, pack_2xint4
+
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    K, N, M = 1024, 2048, 100
+
+    def case(g):
+        s = (torch.rand(K // g, N, device="cuda", generator=gen) * 0.02 + 1e-3).bfloat16()
+        z = (torch.rand(K // g, N, device="cuda", generator=gen) * 6 + 5).bfloat16()
+        return pack_2xint4(torch.randint(0, 16, (K, N), dtype=torch.uint8, device="cuda", generator=gen)), s, z, g
+
+    x = torch.randn(M, N if transposed else K, device="cuda", generator=gen).bfloat16()
+    b, s, z, g = case(64)
+    w = ops.hqq_dequantize(b, s, z, g)
+    two_pass = torch.matmul(x, w.t() if transposed else w)
+    tiles = mixed_mm(x, b, s, z, g, transposed=transposed)
+    assert torch.equal(tiles, _tiled(x, b, s, z, g, transposed))
+    assert ((tiles.double() - two_pass.double()).norm() / two_pass.double().norm()).item() <= 3e-3
+    xg = x.clone().requires_grad_()
+    y = mixed_mm(xg, b, s, z, g, transposed=transposed)
+    assert torch.equal(y, two_pass)
+    y.backward(torch.ones_like(y))
+    assert xg.grad is not None
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert mixed_mm(x, b, s, z, g, transposed=transposed).dtype is torch.float16
+    strided = torch.empty(M, x.shape[1] + 3, dtype=x.dtype, device="cuda")[:, 1:-2].copy_(x)   # rows that are not 16-byte aligned
+    assert torch.equal(mixed_mm(strided, b, s, z, g, transposed=transposed), torch.matmul(strided, w.t() if transposed else w))
+    b, s, z, g = case(32)
+    w = ops.hqq_dequantize(b, s, z, g)
+    assert torch.equal(mixed_mm(x, b, s, z, g, transposed=transposed), torch.matmul(x, w.t() if transposed else w))
