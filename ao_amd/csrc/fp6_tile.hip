@@ -60,13 +60,13 @@ struct Fp6Tile {
 
 // us at K = 4096, 192 to 256 workgroups (14336, 6144 and 4096 columns)
 static const TileShape kFp6Shapes[] = {
-    {64, 64, 19.0, 0.0},     // four groups along K
+    {64, 64, 17.4, 0.0},     // four groups along K
     {64, 128, 24.6, 0.0},    // two groups
     {96, 128, 30.5, 0.0},    // two groups
-    {128, 128, 40.8, 0.0},   // two groups
+    {128, 128, 35.9, 0.0},   // two groups
     {192, 128, 49.8, 0.0},
     {128, 256, 62.0, 0.0},   // 128 x 64 a wave
-    {192, 256, 90.0, 0.0},   // eight waves
+    {192, 256, 87.0, 0.0},   // eight waves
 };
 
 template <bool E3M2>

@@ -79,15 +79,15 @@ struct Int8Tile {
     }
 };
 
-// us at K = 4096 with one and two workgroups on a CU (14336 and 11008 columns at 64 - 512 rows)
+// us at K = 4096 with one and two workgroups on a CU (14336 columns, 224 workgroups, 448 for the second figure)
 static const TileShape kInt8Shapes[] = {
-    {64, 128, 25.5, 0.0},    // two groups of 4 waves along K
-    {96, 128, 32.0, 47.5},
-    {128, 128, 38.0, 0.0},
-    {192, 128, 46.0, 0.0},
-    {128, 256, 54.0, 0.0},   // 128 x 64 a wave
+    {64, 128, 26.4, 0.0},    // two groups of 4 waves along K
+    {96, 128, 32.0, 52.7},
+    {128, 128, 35.2, 0.0},   // two groups; 14336 of K 115 us, one group of four waves 122
+    {192, 128, 47.4, 0.0},
+    {128, 256, 57.0, 0.0},   // eight waves; four of 128 x 64 each are 7 % slower
     {64, 64, 20.0, 0.0},     // four groups along K
-    {192, 256, 90.0, 0.0},   // eight waves
+    {192, 256, 77.8, 0.0},   // eight waves
 };
 
 TilePlan int8wo_gemm_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
@@ -103,9 +103,9 @@ void launch_int8wo_gemm(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
     switch (p.shape) {
         case 0: tile_launch<Int8Tile, 4, 2, 2, 1>(a, p.parts, st); break;
         case 1: tile_launch<Int8Tile, 4, 1, 3, 1>(a, p.parts, st); break;
-        case 2: tile_launch<Int8Tile, 4, 1, 4, 1>(a, p.parts, st); break;
+        case 2: tile_launch<Int8Tile, 4, 2, 4, 1>(a, p.parts, st); break;
         case 3: tile_launch<Int8Tile, 4, 1, 6, 1>(a, p.parts, st); break;
-        case 4: tile_launch<Int8Tile, 4, 1, 4, 2>(a, p.parts, st); break;
+        case 4: tile_launch<Int8Tile, 8, 1, 4, 1>(a, p.parts, st); break;
         case 5: tile_launch<Int8Tile, 2, 4, 2, 1>(a, p.parts, st); break;
         default: tile_launch<Int8Tile, 8, 1, 6, 1>(a, p.parts, st); break;
     }

@@ -14,7 +14,10 @@
 // What bounds it (ablations on 14336 x 4096 int8, 64 - 256 rows): with one wave per SIMD nothing overlaps inside the wave, so
 // LDS reads, conversion and requests add to the matrix time; and a step's data takes 0.7 us from the last-level cache, so
 // the bytes in flight per CU set the pace of small tiles.  Requests three steps ahead instead of two took 128 x 128 tiles
-// at 256 rows from 51 to 38 us; two groups along K (two waves per SIMD) took 64 x 128 tiles from 29 to 24 us.
+// at 256 rows from 51 to 38 us; two groups along K (two waves per SIMD) took 64 x 128 tiles from 29 to 24 us.  A CU takes 125
+// bytes a nanosecond from its XCD's L2, but only 55 to 70 while the weights come from memory: requests return in order, so
+// those behind a weight wait with it.  More buffers than four change nothing then (six measured), and neither do wider
+// tiles for a wave (64 columns, half the LDS reads).
 #pragma once
 #include "common.h"
 
@@ -96,7 +99,7 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + group * STAGES * STAGE;
     auto request = [&](int r, int t, int buf) __attribute__((always_inline)) {
         int s = t * KW + group;
-        s = first + (s < KS ? s : KS - 1);   // a step past the end repeats the last one and is not multiplied
+        s = first + (s < KS ? s : KS - 1);   // a request past the end repeats the last step's and is not used
         const uint32_t at = lds0 + buf * STAGE;
         if (r < AREQ)
             tg_dma(at + (gw * AREQ + r) * 1024, abase + (int64_t)s * 64, aoff[r]);
@@ -116,11 +119,13 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
 #pragma unroll
     for (int j = 0; j < NT; ++j) row_const[j] = F::row(a, n0 + (gw * NT + j) * 32 + r32);
 
-    // Steps 0 .. 2 are requested; from then on step t multiplies buffer t, whose first fragments were read before its
-    // barrier, requests step t + 3 into the buffer that step t - 1 has left, and reads ahead: the barrier in front of step t
-    // has seen step t + 1 arrive, so the last slice of a step reads the first fragments of the next one and no wave starts a
-    // step by waiting for LDS.  A slice is MT x NT slots of one matrix instruction each; its share of the conversion, the
-    // LDS reads and the requests are dealt out over the slots.
+    // Steps 0 .. STAGES - 2 are requested; from then on step t multiplies buffer t and requests step t + STAGES - 1 into the buffer
+    // that step t - 1 has left.  The step's barrier stands in front of its last slice, where every wave has read what it needs of
+    // buffer t and step t + 1 has to have landed: the last slice reads the first fragments of the next step, so no wave starts
+    // a step by waiting for LDS, and a request has STAGES - 2 steps and three quarters to arrive.  (With the barrier at the end of a
+    // step, which then had to see step t + 2 arrive, the three-buffer shapes had less than one: 64 x 64 tiles of int8 at 106
+    // rows, 4888 x 3456, 18.4 -> 14.4 us.)  A slice is MT x NT slots of one matrix instruction each; its share of the
+    // conversion, the LDS reads and the requests are dealt out over the slots.
     constexpr int SLOTS = MT * NT, PIECES = NT * 4;
 #pragma unroll
     for (int t = 0; t < STAGES - 1; ++t)
@@ -135,7 +140,7 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
     Frag fa[2][MT], fb[2][NT];
     typename F::Raw raw[NT];
     typename F::Ready ready[NT];
-    tg_wait_barrier<(STAGES - 3) * REQ>();
+    tg_wait_barrier<(STAGES - 2) * REQ>();
 #pragma unroll
     for (int j = 0; j < NT; ++j) ready[j] = F::prepare(F::read(b_at(0, j), lane), row_const[j]);
 #pragma unroll
@@ -145,33 +150,40 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
 #pragma unroll
         for (int d = 0; d < 4; ++d) fb[0][j].u[d] = F::piece(ready[j], 0, d);
     int buf = 0;
-    for (int t = 0; t < nst; ++t) {
+    // (a group that has one step less runs one less; a test around every matrix instruction of that step cost 2 to 5 %)
+    const int own = (KS - group + KW - 1) / KW;
+    for (int t = 0; t < own; ++t) {
         const int next = buf + 1 == STAGES ? 0 : buf + 1, ahead = buf == 0 ? STAGES - 1 : buf - 1;
-        const bool live = KW == 1 || t * KW + group < KS;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const int cur = s & 1, nxt = cur ^ 1;
+            if (s == 3) {
+                tg_wait_barrier<(STAGES - 2) * REQ>();
+#pragma unroll
+                for (int j = 0; j < NT; ++j) raw[j] = F::read(b_at(next, j), lane);
+            }
 #pragma unroll
             for (int q = 0; q < SLOTS; ++q) {
                 const int i = q % MT, j = q / MT;
-                if (live) acc[i][j] = F::mul(fb[cur][j].q, fa[cur][i].q, acc[i][j]);
+                acc[i][j] = F::mul(fb[cur][j].q, fa[cur][i].q, acc[i][j]);
                 if (q < MT) fa[nxt][q].q = s < 3 ? read_a(a_at(buf), q, s + 1) : read_a(a_at(next), q, 0);
-                if (s == 2 && q < NT) raw[q] = F::read(b_at(next, q), lane);
-                if (s == 3 && q == 0)   // slice 2 has made the last pieces of this step
+                if (s == 3 && q == 1)
 #pragma unroll
                     for (int j2 = 0; j2 < NT; ++j2) ready[j2] = F::prepare(raw[j2], row_const[j2]);
+                // (the last slice's pieces are the next step's first, whose codes arrive in its first slot)
+                const int p0 = s < 3 ? q * PIECES / SLOTS : q == 0 ? 0 : (q - 1) * PIECES / (SLOTS - 1);
+                const int p1 = s < 3 ? (q + 1) * PIECES / SLOTS : q * PIECES / (SLOTS - 1);
 #pragma unroll
-                for (int p = q * PIECES / SLOTS; p < (q + 1) * PIECES / SLOTS; ++p)
-                    fb[nxt][p / 4].u[p % 4] = F::piece(ready[p / 4], (s + 1) & 3, p % 4);
+                for (int p = p0; p < p1; ++p) fb[nxt][p / 4].u[p % 4] = F::piece(ready[p / 4], (s + 1) & 3, p % 4);
                 if (s < 2)
 #pragma unroll
                     for (int r = (s * SLOTS + q) * REQ / (2 * SLOTS); r < (s * SLOTS + q + 1) * REQ / (2 * SLOTS); ++r) request(r, t + STAGES - 1, ahead);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        tg_wait_barrier<(STAGES - 3) * REQ>();
         buf = next;
     }
+    if (KW > 1 && own < nst) tg_wait_barrier<0>();   // the barrier of the step that this group does not have
     // requests past the end have landed before LDS is used again or the workgroup ends
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     if (KW > 1) {
