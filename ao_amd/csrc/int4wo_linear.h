@@ -149,6 +149,8 @@ struct Int4Plan {
 // For plain operands: aligned rows of the packed width, bf16 output, no fused operand.  Answers without a launch; false for a
 // problem that the dispatch refuses.
 bool int4wo_plain_kernel(int64_t M, int64_t K, int64_t N, int64_t g, Int4Kernel* kernel);
+// Whether the dispatch reads activation rows of a multiple of 8 elements that end before the packed width as they are
+bool int4wo_takes_short_rows(int64_t M, int64_t N, int64_t g);
 
 // Single-row GEMV on the 4x4x4 matrix instructions (int4wo_gemv1.hip).  Returns true when it took the launch;
 // false when the shape is outside what it handles (the caller then uses the general kernels).

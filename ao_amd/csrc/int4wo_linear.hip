@@ -115,9 +115,27 @@ __device__ __forceinline__ uint4 load_x8_checked(const uint16_t* __restrict__ x,
     return r.q;
 }
 
+// A lane's 32 activations of K tile kb, four 16-byte loads from its row at `xp` (+ 32 qd).  SHORT: a tile that K ends in (K a multiple of
+// 8) gets zeros beyond: its codes there stand for padded weights, whose products must be zero whatever they are.
+template <bool SHORT>
+__device__ __forceinline__ void load_x_tile(uint4 (&x)[4], const uint16_t* xp, int kb, int qd, int64_t K) {
+    const uint4* xv = reinterpret_cast<const uint4*>(xp + (int64_t)kb * 128);
+    if (!SHORT || (int64_t)(kb + 1) * 128 <= K) {
+#pragma unroll
+        for (int sl = 0; sl < 4; ++sl) x[sl] = xv[sl];
+    } else {
+#pragma unroll
+        for (int sl = 0; sl < 4; ++sl) {
+            x[sl] = make_uint4(0, 0, 0, 0);
+            if ((int64_t)kb * 128 + qd * 32 + sl * 8 < K) x[sl] = xv[sl];
+        }
+    }
+}
+
 // How a wave gets its activation fragments (MFMA A operand: row m = lane%16, 8 consecutive k):
-constexpr int X_GLOBAL = 0;   // 16-byte global loads, prefetched with the weight tile (K % 128 == 0, aligned rows)
+constexpr int X_GLOBAL = 0;   // 16-byte global loads, prefetched with the weight tile (K of the packed width, aligned rows)
 constexpr int X_CHECKED = 1;  // element-wise global loads with bounds checks (any K, any alignment)
+constexpr int X_SHORT = 3;    // X_GLOBAL with rows of a multiple of 8 elements that end before the packed width
 constexpr int X_LDS = 2;      // the workgroup stages its <= 16 activation rows in LDS once (small M x K)
 
 template <int XMODE, bool DUAL>
@@ -184,7 +202,7 @@ __device__ __forceinline__ GroupRegs make_group_asm(uint32_t qp) {
 // Epilogue order for the single-weight form: y = bf16(acc + bias), then y = bf16(y + residual).
 template <int G, int WAVES, int XMODE, bool DUAL>
 __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_kernel(const LinearArgs a) {
-    static_assert(XMODE == X_GLOBAL || XMODE == X_CHECKED, "the LDS-staged path is int4wo_gemv_kernel");
+    static_assert(XMODE == X_GLOBAL || XMODE == X_CHECKED || XMODE == X_SHORT, "the LDS-staged path is int4wo_gemv_kernel");
     constexpr int D = 2;
     constexpr int NRED = DUAL ? 2 : 1;
     __shared__ float red[NRED][WAVES][4][64];
@@ -193,7 +211,7 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_kernel(const LinearA
     const int r = lane & 15, qd = lane >> 4;
     const int64_t rb = blockIdx.x;
     const int64_t m0 = (int64_t)blockIdx.y * 16;
-    const int KB = (int)(a.Kp / 128);
+    const int KB = XMODE == X_SHORT ? (int)((a.K + 127) / 128) : (int)(a.Kp / 128);   // (g = 256: the packed row may go on)
     const uint32_t magic = 0x43004300u, one_lo = 0x00003F80u, one_hi = 0x3F800000u;
     // selection matrices of stage 2 as A operands: lane (i = lane%16, qd) holds kk = 8*qd + e; the single 1.0 of
     // row i sits at kk = 8*(i/4) + i%4 (sel_a) or + 4 (sel_b), i.e. only in the lanes with qd == i/4
@@ -204,7 +222,7 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_kernel(const LinearA
     const u32x4_t sel_a = {s_even, s_odd, 0u, 0u};
     const u32x4_t sel_b = {0u, 0u, s_even, s_odd};
 
-    const int64_t woff = rb * KB * 64 + lane;
+    const int64_t woff = rb * (XMODE == X_SHORT ? a.Kp / 128 : KB) * 64 + lane;
     const int64_t qoff = rb * (a.Kp / G) * 16 + r;
     const bool xact = (m0 + r) < a.M;
     const uint16_t* xp = a.x + (xact ? (m0 + r) : 0) * a.ldx + qd * 32;
@@ -224,12 +242,8 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_kernel(const LinearA
             b.w2 = load_w(a.packed2, kb);
             b.q2 = load_q(a.qparams2, gidx);
         }
-        if (XMODE == X_GLOBAL) {
-            if (xact) {
-                const uint4* xv = reinterpret_cast<const uint4*>(xp + (int64_t)kb * 128);
-#pragma unroll
-                for (int sl = 0; sl < 4; ++sl) b.x[sl] = xv[sl];
-            }
+        if (XMODE == X_GLOBAL || XMODE == X_SHORT) {
+            if (xact) load_x_tile<XMODE == X_SHORT>(b.x, xp, kb, qd, a.K);
         } else if (XMODE == X_CHECKED) {
 #pragma unroll
             for (int sl = 0; sl < 4; ++sl)
@@ -342,7 +356,9 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_kernel(const LinearA
 // four times the bytes of its weights at 16 rows (896 workgroups x 128 KB on 14336 x 4096), and the fill rate of a
 // CU's L1 (about 20 bytes per cycle), not memory, sets the time.  Here a wave loads the activation fragments of a K
 // tile once and runs them against the tiles of four row blocks: a quarter of the activation traffic, four accumulators.
-template <int G, int WAVES, int MB>
+// EDGE: activation rows that end before the packed width, and row blocks that are no multiple of four (the tests of both cost the
+// others 2 to 5 %).
+template <int G, int WAVES, int MB, bool EDGE>
 __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const LinearArgs a) {
     // MB 16-row blocks of activations per workgroup (17 to 32 rows with MB = 2): every dequantized dword then feeds MB
     // matrix instructions, and the dequantization, which bounds the kernel, is done once for all of them
@@ -354,7 +370,12 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
     const int r = lane & 15, qd = lane >> 4;
     const int64_t rb0 = (int64_t)blockIdx.x * RBW;
     const int64_t m0 = (int64_t)blockIdx.y * (16 * MB);
-    const int KB = (int)(a.Kp / 128);
+    const int KP = (int)(a.Kp / 128), KB = EDGE ? (int)((a.K + 127) / 128) : KP;   // (g = 256: the packed row may go on)
+    // a row block past the end repeats the last one and is not stored
+    auto row_block = [&](int j) __attribute__((always_inline)) {
+        const int64_t last = (a.N + 15) / 16 - 1;
+        return EDGE && rb0 + j > last ? last : rb0 + j;
+    };
     const uint32_t magic = 0x43004300u;
     const bool sel_lane = qd == (r >> 2);
     const uint32_t one_bits = (r & 1) ? 0x3F800000u : 0x00003F80u;
@@ -385,16 +406,12 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
         const int gidx = ((kb * 128 + qd * 32) / G) * 16;
 #pragma unroll
         for (int j = 0; j < RBW; ++j) {
-            b.w[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(a.packed + ((rb0 + j) * KB + kb) * 64 + lane));
-            b.q[j] = a.qparams[(rb0 + j) * (a.Kp / G) * 16 + r + gidx];
+            b.w[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(a.packed + (row_block(j) * KP + kb) * 64 + lane));
+            b.q[j] = a.qparams[row_block(j) * (a.Kp / G) * 16 + r + gidx];
         }
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
-            if (xact[mb]) {
-                const uint4* xv = reinterpret_cast<const uint4*>(xp[mb] + (int64_t)kb * 128);
-#pragma unroll
-                for (int sl = 0; sl < 4; ++sl) b.x[mb][sl] = xv[sl];
-            }
+            if (xact[mb]) load_x_tile<EDGE>(b.x[mb], xp[mb], kb, qd, a.K);
     };
     u32x4_t tcur = {0, 0, 0, 0};
     // one tile = 16 dwords per lane (4 row blocks x 4); the three dequantization stages run as in int4wo_linear_kernel
@@ -1137,6 +1154,18 @@ static void launch_group(int64_t g, int waves, dim3 grid, size_t smem, hipStream
     }
 }
 
+// 17 and more rows on int4wo_linear_rb4_kernel: from 768 row blocks on, up to this many
+static int64_t int4wo_rb4_max_rows(int64_t RB) { return RB >= 4096 ? 64 : 48; }
+// Rows that end before the packed width: the single-row kernel and the two whose lanes load their own activation fragments fill up
+// with zeros.  The other kernels take rows that were copied to that width first (int4wo_tile.hip), 4 us more: 9316 x 5312 at 1 row
+// 12.3 -> 10.4 us, 10768 x 704 at 2 rows 8.8 -> 4.8,
+// 28000 x 1088 at 12 rows 12.2 -> 8.7, 23576 x 7552 at 5 rows 39.3 -> 31.6 (also for its 1474 row blocks, no multiple of four).
+bool int4wo_takes_short_rows(int64_t M, int64_t N, int64_t g) {
+    if (M == 1) return g >= 64;
+    const int64_t RB = (N + 15) / 16;
+    return M < 16 || (RB >= 768 && M <= int4wo_rb4_max_rows(RB));
+}
+
 static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams,
                            const void* packed2, const void* qparams2, int64_t N, int64_t g, const void* bias_bf16,
                            const void* residual_bf16, int64_t ldres, void* y, int y_dtype, int64_t ldy, void* stream,
@@ -1182,7 +1211,10 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
     // ... but not with fewer than 4 K tiles per wave while the row still fits two chunks per thread
     if (M == 1)
         while (waves > 4 && KB < 4 * waves && (int64_t)(waves / 2) * 128 >= Kp / 8) waves /= 2;
-    const bool aligned = (K == Kp) && ((ldx & 7) == 0) && ((((uintptr_t)x_bf16) & 15) == 0);
+    const bool aligned_rows = (K & 7) == 0 && ((ldx & 7) == 0) && ((((uintptr_t)x_bf16) & 15) == 0);
+    const bool aligned = K == Kp && aligned_rows;
+    // rows that end before the packed width: the single-row kernel and the two whose lanes load their own fragments fill up with zeros
+    const bool short_rows = K != Kp && aligned_rows && int4wo_takes_short_rows(M, N, g) && !dual && !norm_weight_bf16 && !pair8 && ksplit == 1;
     const int64_t rows = M < 16 ? M : 16;
     const size_t xbytes = (size_t)rows * (size_t)Kp * 2;
     // the fused RMSNorm and the interleaved gate/up epilogue exist on the LDS-staged path only: use workgroups
@@ -1199,7 +1231,7 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
     // 8 / 16 rows: 7.0 / 5.8, 7.7 / 6.3, 8.2 / 6.5, 9.9 / 7.9; 6144 x 4096 at 2 / 4 / 10 rows: 9.1 / 7.8, 9.6 / 8.2, 14.8 / 9.5;
     // 4096 x 14336 at 2 / 4 rows: 13.2 / 12.5, 14.0 / 12.6; 14336 x 4096 at 2 rows 13.6 / 13.6; 28672 x 4096 at 2 rows 21.2 / 23.1).
     const bool want_lds = M == 1 || norm_weight_bf16 || pair8 || packed2 != nullptr || ksplit > 1 || (M == 2 && RB >= 1536);
-    int xmode = aligned ? (lds_ok && want_lds ? X_LDS : X_GLOBAL) : X_CHECKED;
+    int xmode = aligned ? (lds_ok && want_lds ? X_LDS : X_GLOBAL) : short_rows ? X_SHORT : X_CHECKED;
     LinearArgs a{(const uint16_t*)x_bf16, M, K, ldx, (const uint4*)packed, (const uint32_t*)qparams,
                  (const uint4*)packed2, (const uint32_t*)qparams2, n_out, Kp, (const uint16_t*)bias_bf16,
                  (const uint16_t*)residual_bf16, ldres, y, y_dtype == AO_F32, ldy,
@@ -1231,8 +1263,8 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
     // ... and 33 to 48 rows (to 64 on weights with 4096 or more row blocks) with four activation blocks, which fit the
     // registers since the kernel keeps one tile buffer: 14336 x 4096 at 33-48 rows 25.5 -> 20.4-21.0 us, 28672 x 4096 38 ->
     // 32-33.5, the head at 33-64 rows 164-167 -> 115-145 (at 56-64 rows the tiles are as fast or faster on the others)
-    const int64_t rb4_max_m = RB / 4 >= 1024 ? 64 : 48;
-    const bool rb4_two_blocks = !rb4_off && M > 16 && M <= rb4_max_m && RB % 4 == 0 && RB / 4 >= 192 && a.K == a.Kp;
+    const int64_t rb4_max_m = int4wo_rb4_max_rows(RB);
+    const bool rb4_two_blocks = !rb4_off && M > 16 && M <= rb4_max_m && RB >= 768 && (aligned || short_rows);
     // K split over workgroups from 17 rows on: the 32- and 64-row tiles whose K loop is already split over four groups of waves
     // (and below that when the rows do not fit the LDS staging of the streaming kernel)
     const bool ws_tiles = ksplit > 1 && (M > 16 || !(aligned && lds_ok));
@@ -1286,7 +1318,7 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
         return 0;
     }
     // one activation row: the kernel built on the 4x4x4 matrix instructions (group size 64 and up, K up to 16384)
-    if (M == 1 && aligned && !dual) {
+    if (M == 1 && (aligned || short_rows) && !dual) {
         char name[96];
         if (int4wo_gemv2_plan(a, g, RB, name, sizeof(name))) {
             AO_PLAN(Int4Kernel::streaming, "%s", name);
@@ -1305,14 +1337,13 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
     // workgroups (see int4wo_linear_rb4_kernel).  Measured on 14336 x 4096, us at 2 / 3 / 4 / 5 / 8 / 12 / 16 rows: 13.1 /
     // 13.9 / 13.5 / 13.6 / 13.7 / 13.7 / 14.1 against 12.8 / 14.0 / 14.2 / 16.4 / 14.8 / 18.2 / 20.6 of the kernels below
     // (LDS-staged up to 5 rows there); the vocabulary head at 16 rows 85 against 129.
-    if ((xmode == X_GLOBAL || (xmode == X_LDS && !norm_weight_bf16 && !pair8)) && !dual && ksplit == 1 && M >= 4 &&
-        RB % 4 == 0 && a.K == a.Kp) {
+    if ((xmode == X_GLOBAL || xmode == X_SHORT || (xmode == X_LDS && !norm_weight_bf16 && !pair8)) && !dual && ksplit == 1 && M >= 4) {
         static const bool rb4_disabled = [] { const char* e = knob("AO_AMD_RB4"); return e && e[0] == '0'; }();
         // two 16-row activation blocks per workgroup from 17 rows on: the dequantized dword feeds both (four of them
         // do not fit the registers)
         const int mb = M > 32 && M <= rb4_max_m ? 4 : (M > 16 ? 2 : 1);
         const int64_t mch = (M + 16 * mb - 1) / (16 * mb);
-        const int64_t wgs = (RB / 4) * mch;
+        const int64_t wgs = (RB + 3) / 4 * mch;
         if (!rb4_disabled && wgs >= 192) {
             int w4 = 4;   // at least four waves: wave j finishes row block j
             while (w4 < 8 && wgs * w4 * 2 <= 4096 + wgs && w4 * 2 <= a.Kp / 128) w4 *= 2;
@@ -1321,7 +1352,7 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
             if (mb >= 2 && wgs > 256) w4 = 4;
             if (mb == 1) AO_PLAN(Int4Kernel::streaming, "int4wo_linear_rb4_kernel<%lld,%d>", (long long)g, w4);
             AO_PLAN(Int4Kernel::streaming, "int4wo_linear_rb4_kernel<%lld,%d,%d>", (long long)g, w4, mb);
-            const dim3 grid4((unsigned)(RB / 4), (unsigned)mch);
+            const dim3 grid4((unsigned)((RB + 3) / 4), (unsigned)mch);
             auto go = [&](auto kernel, int nw) {
                 if (g_prof_start && g_prof_stop) {
                     hipExtLaunchKernelGGL(kernel, grid4, dim3(nw * 64), 0, st, g_prof_start, g_prof_stop, 0, a);
@@ -1330,9 +1361,12 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
                     hipLaunchKernelGGL(kernel, grid4, dim3(nw * 64), 0, st, a);
                 }
             };
+            const bool edge = short_rows || RB % 4 != 0;
 #define AO_RB4_MB(GG, MBV)                                                 \
-    if (w4 == 4) go(int4wo_linear_rb4_kernel<GG, 4, MBV>, 4);              \
-    else go(int4wo_linear_rb4_kernel<GG, 8, MBV>, 8)
+    if (w4 == 4 && !edge) go(int4wo_linear_rb4_kernel<GG, 4, MBV, false>, 4); \
+    else if (w4 == 4) go(int4wo_linear_rb4_kernel<GG, 4, MBV, true>, 4);   \
+    else if (!edge) go(int4wo_linear_rb4_kernel<GG, 8, MBV, false>, 8);    \
+    else go(int4wo_linear_rb4_kernel<GG, 8, MBV, true>, 8)
 #define AO_RB4(GG)                                                         \
     if (mb == 1) { AO_RB4_MB(GG, 1); }                                     \
     else if (mb == 2) { AO_RB4_MB(GG, 2); }                                \
@@ -1350,7 +1384,7 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
         }
     }
     AO_PLAN(Int4Kernel::streaming, "%s<%lld,%d,%s%d>", xmode == X_LDS ? "int4wo_gemv_kernel" : "int4wo_linear_kernel", (long long)g, waves,
-            xmode == X_LDS ? "" : (xmode == X_GLOBAL ? "X_GLOBAL," : "X_CHECKED,"), dual ? 1 : 0);
+            xmode == X_LDS ? "" : (xmode == X_GLOBAL ? "X_GLOBAL," : xmode == X_SHORT ? "X_SHORT," : "X_CHECKED,"), dual ? 1 : 0);
 #undef AO_PLAN
     dim3 grid((unsigned)RB, (unsigned)mchunks, (unsigned)ksplit);
     const size_t smem = xmode == X_LDS ? xbytes : 0;
@@ -1361,6 +1395,7 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
     } else {
         if (xmode == X_LDS) launch_gemv<false>(g, waves, grid, smem, st, a);
         else if (xmode == X_GLOBAL) launch_group<X_GLOBAL, false>(g, waves, grid, smem, st, a);
+        else if (xmode == X_SHORT) launch_group<X_SHORT, false>(g, waves, grid, smem, st, a);
         else launch_group<X_CHECKED, false>(g, waves, grid, smem, st, a);
     }
     AO_LAUNCH_CHECK();

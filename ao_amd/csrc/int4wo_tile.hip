@@ -153,11 +153,12 @@ __global__ __launch_bounds__(256) void pad_rows_kernel(const uint16_t* __restric
 // Which route a plain linear takes and what its workspace holds: the copied rows first, then the K parts.
 struct Int4Auto {
     bool tiled;
+    bool as_is;           // the plain kernel reads the rows itself: nothing is copied (the workspace keeps the size that callers know)
     int64_t Kp;           // the width of the copied rows, 0: read as they are
     int64_t copy, parts;  // bytes
 };
 static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t N, int64_t g, int y_dtype, Int4Auto* r) {
-    *r = Int4Auto{false, 0, 0, 0};
+    *r = Int4Auto{false, false, 0, 0, 0};
     const bool aligned = (ldx & 7) == 0 && (((uintptr_t)x) & 15) == 0;
     if (M > 32 && y_dtype == AO_BF16 && aligned && 256 * ldx * 2 < ((int64_t)1 << 32)) {
         int64_t need = -1;
@@ -168,7 +169,7 @@ static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t
             return 0;
         }
     }
-    // Rows that the fast kernels cannot read are copied to the packed width where the copy (2 to 3 us with its launch) costs less than the
+    // Rows that the kernel cannot read (int4wo_takes_short_rows) are copied to the packed width where the copy (2 to 3 us with its launch) costs less than the
     // element-wise kernel loses, whose time follows the length of the rows, or the whole product where the weight is large.  us a call
     // as they are / copied: 4096 x 4160 at 1 / 6 / 16 / 64 rows 15.5 / 18 / 35 / 121, 10.5 / 10.0 / 10.5 / 16.4; 14336 x 4032 at 1 / 16
     // rows 30 / 114, 13.5 / 15.5; 1024 x 2112 at 1 / 2 / 8 / 16 rows 13.9 / 8.9 / 12.9 / 19.8, about 9.5; 1024 x 704 up to 64 rows 7
@@ -178,6 +179,7 @@ static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t
     if (M > 0 && (K != Kp || !aligned) && (N * K * (M + 4) >= 50000000 || K * (M == 1 ? 13 : rows + 4) >= 18000)) {
         r->Kp = Kp;
         r->copy = M * Kp * 2;
+        r->as_is = aligned && K % 8 == 0 && int4wo_takes_short_rows(M, N, g);
     }
     return ao_amd_int4wo_linear_ws_bytes(M, r->Kp ? Kp : K, N, g, &r->parts);
 }
@@ -282,6 +284,7 @@ extern "C" int ao_amd_int4wo_linear_auto(const void* x_bf16, int64_t M, int64_t 
                (long long)workspace_bytes);
     if (r.tiled)
         return ao_amd_int4wo_linear_tiled(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, ldy, workspace, r.parts, stream);
+    if (r.as_is) return ao_amd_int4wo_linear(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, stream);
     if (r.Kp) {
         if (int rc = ao_amd_pad_rows(x_bf16, M, K, ldx, r.Kp, workspace, stream)) return rc;
         x_bf16 = workspace;

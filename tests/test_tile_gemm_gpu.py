@@ -263,3 +263,35 @@ def test_int4_kwave_tiles_of_96_and_128_rows(M, N, K, group):
                                                    _lib.BF16, N, torch.cuda.current_stream().cuda_stream))
         rel = ((y.float() - want.float()).norm() / want.float().norm()).item()   # as for the tiles; one-hot rows are exact
         assert rel <= (1e-3 if rows is x else 0.0), (M, N, K, rel)
+
+
+@pytest.mark.parametrize("M,N,K,group,name", [
+    (1, 14336, 4032, 64, "int4wo_gemv1_short_kernel"), (1, 560, 1856, 64, "int4wo_gemv1_short_kernel"), (1, 9316, 5312, 128, "int4wo_gemv1_short_kernel"),
+    (1, 2288, 9736, 256, "int4wo_gemv1_short_kernel"), (1, 4096, 16136, 256, "int4wo_gemv1_short_kernel"), (1, 30000, 1032, 128, "int4wo_gemv1_short_kernel"),
+    (2, 4099, 4160, 32, "int4wo_linear_kernel"), (15, 4096, 8072, 256, "int4wo_linear_kernel"), (3, 70, 136, 64, "int4wo_linear_kernel"),
+    (4, 12290, 1096, 64, "int4wo_linear_rb4_kernel"), (16, 12336, 7552, 256, "int4wo_linear_rb4_kernel"), (17, 14344, 4040, 128, "int4wo_linear_rb4_kernel"),
+    (48, 12300, 1160, 32, "int4wo_linear_rb4_kernel"), (64, 65552, 264, 64, "int4wo_linear_rb4_kernel"),
+    (5, 12304, 1024, 64, "int4wo_linear_rb4_kernel"), (33, 14360, 2048, 128, "int4wo_linear_rb4_kernel"),   # row blocks that are no multiple of four
+])
+def test_int4_rows_that_are_read_as_they_end(M, N, K, group, name):
+    """Rows of a multiple of 8 elements that end before the packed width, and row blocks that are no multiple of four, on the kernels that
+    take them without a copy: the fp32 product (as for the tiles), single weights bit for bit, and nothing of what lies behind a row's
+    end (NaN here) in the result."""
+    from ao_amd import _lib, ops
+
+    assert _lib.int4wo_linear_plan(M, K, N, group).startswith(name)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    packed, qp = ops.int4wo_quantize_pack((torch.randn(N, K, device="cuda", generator=g) * 0.02).bfloat16(), group)
+    dq = ops.int4wo_dequantize(packed, qp, N, K, group)
+    rows = torch.full((M + 1, K + 264), float("nan"), device="cuda").bfloat16()
+    x = rows[:M, :K]
+    x.copy_(torch.randn(M, K, device="cuda", generator=g))
+    y = ops.int4wo_linear(x, packed, qp, group, N)
+    want = (x.float() @ dq.float().t()).bfloat16()
+    rel = ((y.float() - want.float()).norm() / want.float().norm()).item()
+    assert rel <= 1e-3 and (y != want).float().mean() <= 0.01, rel
+    at = torch.arange(M, device="cuda") * 37 % K
+    at[-1] = K - 1
+    x.zero_()
+    x[torch.arange(M, device="cuda"), at] = 1.0
+    assert torch.equal(ops.int4wo_linear(x, packed, qp, group, N), dq[:, at].t())
