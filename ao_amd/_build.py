@@ -22,6 +22,8 @@ HIPCC_FLAGS = [
     "-ffp-contract=off",
     # hipcc may not form packed fp32 math on this target
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # leading scalar and pointer arguments of a kernel arrive in registers: a launch starts without waiting for their load
+    "-mllvm", "-amdgpu-kernarg-preload-count=14",
     "-Wno-unused-command-line-argument",
 ]
 
