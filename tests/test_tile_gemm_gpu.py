@@ -144,6 +144,21 @@ def test_fp6_tiles_cover_every_shape_and_the_operator_takes_them():
         assert torch.equal(eager, torch.ops.torchao.fp6_linear_native.default(3, 2, x, native, scale))   # both host paths
 
 
+@pytest.mark.parametrize("M,N,K,tiled", [
+    (32, 14336, 2048, False), (33, 14336, 2048, True), (48, 14336, 2048, True), (49, 14336, 2048, False), (48, 8192, 2048, False),
+    (64, 4096, 14336, False), (65, 4096, 14336, True), (96, 4096, 14336, True), (97, 4096, 14336, False), (80, 4096, 8192, False),
+])
+def test_fp6_tiles_at_33_to_96_rows(M, N, K, tiled):
+    """Both sides of the rule on rows and weight size, operator against the fp32 product (the tolerance of _fp6_tiles: the
+    order of at most 14336 exact products' fp32 sums)."""
+    from ao_amd import ops
+
+    assert (_tiled_bytes("fp6", M, N, K) >= 0) == tiled
+    x, native, scale, y = _fp6_tiles(M, N, K, 3, 2)
+    rel = ((ops.fp6_linear_native(3, 2, x, native, scale).float() - y.float()).norm() / y.float().norm()).item()
+    assert rel <= 1e-4, rel
+
+
 # (M, N, K, group): every tile shape of the int4 table, groups below, at and beyond a K step, widths with part of a row block,
 # in_features that the packed layout pads (to a multiple of 128 or of the group)
 INT4_TILES = [
