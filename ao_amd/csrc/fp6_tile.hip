@@ -72,7 +72,7 @@ static const TileShape kFp6Shapes[] = {
 template <bool E3M2>
 static void launch_shape(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
     typedef Fp6Tile<E3M2> F;
-    tile_grid(a, kFp6Shapes[p.shape], p.parts);
+    tile_grid(a, kFp6Shapes[p.shape], 48, p.parts);
     switch (p.shape) {
         case 0: tile_launch<F, 2, 4, 2, 1>(a, p.parts, st); break;
         case 1: tile_launch<F, 4, 2, 2, 1>(a, p.parts, st); break;
@@ -155,7 +155,7 @@ extern "C" int ao_amd_fp6_linear_tiled(const void* x_f16, int64_t M, int64_t K, 
     TilePlan p = fp6_tile_plan(M, N, K, 8);
     if (p.parts > 1 && (!workspace || workspace_bytes < p.parts * M * N * (int64_t)sizeof(float))) p = fp6_tile_plan(M, N, K, 1);
     const TileGemmArgs a{(const uint16_t*)x_f16, M, K, K, (const uint8_t*)weights_native, round_up(K, 128) / 128 * 1536, scale_f16, nullptr, N,
-                         (uint16_t*)out_f16, N, 0, 0, 0, nullptr, 0, nullptr, 0, 0, (float*)workspace};
+                         (uint16_t*)out_f16, N, TileOrder(), nullptr, 0, nullptr, 0, 0, (float*)workspace};
     if (ebits == 3) launch_shape<true>(a, p, (hipStream_t)stream);
     else launch_shape<false>(a, p, (hipStream_t)stream);
     AO_LAUNCH_CHECK();

@@ -220,9 +220,9 @@ extern "C" int ao_amd_int4wo_linear_tiled(const void* x_bf16, int64_t M, int64_t
     TilePlan p = int4wo_tile_plan(M, N, K, 8);
     if (p.parts > 1 && (!workspace || workspace_bytes < p.parts * M * N * (int64_t)sizeof(float))) p = int4wo_tile_plan(M, N, K, 1);
     TileGemmArgs a{(const uint16_t*)x_bf16, M, K, ldx, (const uint8_t*)packed, round_up(K, g > 128 ? g : 128) * 8, qparams, (const uint16_t*)bias_bf16, N,
-                   (uint16_t*)y_bf16, ldy, 0, 0, 0, nullptr, 0, nullptr, 0, g == 32 ? 5 : g == 64 ? 6 : g == 128 ? 7 : 8, (float*)workspace};
+                   (uint16_t*)y_bf16, ldy, TileOrder(), nullptr, 0, nullptr, 0, g == 32 ? 5 : g == 64 ? 6 : g == 128 ? 7 : 8, (float*)workspace};
     hipStream_t st = (hipStream_t)stream;
-    tile_grid(a, kInt4Shapes[p.shape], p.parts);
+    tile_grid(a, kInt4Shapes[p.shape], 32, p.parts);
     switch (p.shape) {
         case 0: tile_launch<Int4Tile, 2, 4, 2, 1>(a, p.parts, st); break;
         case 1: tile_launch<Int4Tile, 4, 2, 2, 1>(a, p.parts, st); break;

@@ -99,7 +99,7 @@ void int8wo_gemm_describe(const TilePlan& p, char* out, size_t cap) {
 }
 
 void launch_int8wo_gemm(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
-    tile_grid(a, kInt8Shapes[p.shape], p.parts);
+    tile_grid(a, kInt8Shapes[p.shape], 64, p.parts);
     switch (p.shape) {
         case 0: tile_launch<Int8Tile, 4, 2, 2, 1>(a, p.parts, st); break;
         case 1: tile_launch<Int8Tile, 4, 1, 3, 1>(a, p.parts, st); break;

@@ -614,7 +614,7 @@ static int int8wo_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, c
     TilePlan p = int8wo_gemm_plan(M, N, K, 8);
     if (p.parts > 1 && (!workspace || workspace_bytes < p.parts * M * N * (int64_t)sizeof(float))) p = int8wo_gemm_plan(M, N, K, 1);
     launch_int8wo_gemm(TileGemmArgs{(const uint16_t*)x_bf16, M, K, ldx, (const uint8_t*)w_int8, ldw, scale_bf16,
-                                    (const uint16_t*)bias_bf16, N, (uint16_t*)y, ldy, 0, 0, 0, (const uint16_t*)residual, ldres,
+                                    (const uint16_t*)bias_bf16, N, (uint16_t*)y, ldy, TileOrder(), (const uint16_t*)residual, ldres,
                                     (const uint16_t*)gate, ldgate, 0, workspace},
                        p, (hipStream_t)stream);
     AO_LAUNCH_CHECK();

@@ -19,7 +19,7 @@
 // those behind a weight wait with it.  More buffers than four change nothing then (six measured), and neither do wider
 // tiles for a wave (64 columns, half the LDS reads).
 #pragma once
-#include "common.h"
+#include "tile_order.h"
 
 namespace ao {
 
@@ -32,7 +32,7 @@ struct TileGemmArgs {
     const uint16_t* bias;               // or null
     int64_t N;
     uint16_t* y; int64_t ldy;
-    int tiles_n, tiles, per_xcd;
+    TileOrder order;
     const uint16_t* residual; int64_t ldres;   // y += residual, or null
     const uint16_t* gate; int64_t ldgate;      // y = silu(gate) * y, or null
     int group_shift;                    // int4: log2 of the group size
@@ -76,10 +76,9 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int group = wave / G, gw = wave % G;
-    // consecutive tiles of one XCD share an activation slice
-    const int tile = (int)(blockIdx.x & 7) * a.per_xcd + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= a.per_xcd || tile >= a.tiles) return;
-    const int64_t m0 = (int64_t)(tile / a.tiles_n) * BM, n0 = (int64_t)(tile % a.tiles_n) * BN;
+    int tile_m, tile_n;
+    if (!tile_at(a.order, (int)blockIdx.x, tile_m, tile_n)) return;
+    const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
     // this workgroup's run of 64-wide K steps: all of them, or the blockIdx.y-th of gridDim.y equal parts
     const int all = (int)(a.K / 64), per = (all + (int)gridDim.y - 1) / (int)gridDim.y, first = per * (int)blockIdx.y;
     const int KS = min(per, all - first), nst = (KS + KW - 1) / KW;
@@ -316,17 +315,16 @@ inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64
 }
 
 // The launches of a plan: tile_grid once, tile_launch with the shape's constants, tile_finish.
-inline void tile_grid(TileGemmArgs& a, const TileShape& s, int parts) {
-    a.tiles_n = (int)((a.N + s.bn - 1) / s.bn);
-    a.tiles = a.tiles_n * (int)((a.M + s.bm - 1) / s.bm);
-    a.per_xcd = (a.tiles + 7) / 8;
+// row_bytes: a weight row's bytes in a 64-wide step.
+inline void tile_grid(TileGemmArgs& a, const TileShape& s, int row_bytes, int parts) {
+    a.order = tile_order((a.M + s.bm - 1) / s.bm, (a.N + s.bn - 1) / s.bn, s.bm * 128, s.bn * row_bytes);
     if (parts == 1) a.parts = nullptr;
 }
 template <class F, int WN, int KW, int MT, int NT>
 void tile_launch(const TileGemmArgs& a, int parts, hipStream_t st) {
     hipEvent_t ev0 = g_prof_start, ev1 = g_prof_stop;
     g_prof_start = g_prof_stop = nullptr;
-    hipExtLaunchKernelGGL((tile_gemm_kernel<F, WN, KW, MT, NT>), dim3((unsigned)(a.per_xcd * 8), (unsigned)parts), dim3(64 * WN * KW), 0, st,
+    hipExtLaunchKernelGGL((tile_gemm_kernel<F, WN, KW, MT, NT>), dim3((unsigned)(a.order.per_xcd * 8), (unsigned)parts), dim3(64 * WN * KW), 0, st,
                           ev0, ev1, 0, a);
 }
 template <class F>

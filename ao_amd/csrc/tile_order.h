@@ -1,0 +1,44 @@
+// The order in which 8 per_xcd workgroups take tiles_m x tiles_n output tiles of a product.
+//
+// Consecutive workgroups go to the eight XCDs in turn, each with an L2 of its own, so an XCD takes per_xcd neighbouring tiles:
+// panels of `panel` tile rows, column by column.  What its 32 CUs work on at a time then comes from `panel` activation slices and
+// 32 / panel weight tiles, each read once into that L2.  A weight's bytes count twice, since the activations, which every XCD
+// reads, come from the last-level cache and the weight from memory: time is least near panel^2 = 64 (weight tile) / (activation
+// slice), with the tile rows dealt out evenly over that many panels.  Row by row (panel 1, all of one activation slice
+// first) the weight came once per tile row; measured us, row by row / in panels: int8 14336 x 4096 at 190 / 450 / 1149 rows
+// 35.4 / 34.0, 64.4 / 62.2, 138 / 134, 4096 x 14336 at 300 rows 57.6 / 51.2; FP6 14336 x 4096 at 80 / 450 rows 23.6 / 22.9, 63.9 / 60.6;
+// int4 5120 x 13824 at 427 rows 102.3 / 96.2 (counting the weight once 102.0), 14336 x 4096 at 2048 rows 216 / 211.  All
+// rows in one panel is too much for many short rows (int4 1024 x 4096 at 2750 rows, 29 tile rows: 34.6 / 36.6).
+#pragma once
+#include "common.h"
+#include <math.h>
+
+namespace ao {
+
+struct TileOrder {
+    int tiles_m, tiles_n, panel, per_xcd;
+};
+
+// x_bytes, w_bytes: what a tile reads of the activations and of the weight for the same stretch of K
+inline TileOrder tile_order(int64_t tiles_m, int64_t tiles_n, int64_t x_bytes, int64_t w_bytes) {
+    const int64_t per_xcd = (tiles_m * tiles_n + 7) / 8, at_once = per_xcd < 32 ? per_xcd : 32;
+    const double high = sqrt(2.0 * (double)at_once * (double)w_bytes / (double)x_bytes);
+    int64_t panels = high >= 1.0 ? (int64_t)((double)tiles_m / high + 0.5) : tiles_m;
+    panels = panels < 1 ? 1 : panels;
+    return TileOrder{(int)tiles_m, (int)tiles_n, (int)((tiles_m + panels - 1) / panels), (int)per_xcd};
+}
+
+// The tile of workgroup `block`; false past the last one
+__device__ __forceinline__ bool tile_at(const TileOrder& o, int block, int& tile_m, int& tile_n) {
+    const int tile = (block & 7) * o.per_xcd + (block >> 3);
+    if (block >> 3 >= o.per_xcd || tile >= o.tiles_m * o.tiles_n) return false;
+    const int per_panel = o.panel * o.tiles_n;
+    int p = 0, in = tile;
+    if (tile >= per_panel) p = tile / per_panel, in = tile - p * per_panel;
+    const int high = min(o.panel, o.tiles_m - p * o.panel);
+    tile_n = in / high;
+    tile_m = p * o.panel + in - tile_n * high;
+    return true;
+}
+
+}  // namespace ao

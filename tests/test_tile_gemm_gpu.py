@@ -310,3 +310,32 @@ def test_int4_rows_that_are_read_as_they_end(M, N, K, group, name):
     x.zero_()
     x[torch.arange(M, device="cuda"), at] = 1.0
     assert torch.equal(ops.int4wo_linear(x, packed, qp, group, N), dq[:, at].t())
+
+
+@pytest.mark.parametrize("fmt,M,N,K,group,name", [
+    ("int4", 1700, 7000, 512, 64, "int4wo_gemm_lds_kernel<64,2>"), ("int4", 1000, 6400, 512, 128, "int4wo_gemm_lds_kernel<128,1>"),
+    ("int4", 300, 4100, 1024, 32, "int4wo_gemm_kwave_kernel"), ("int4", 2750, 1024, 4096, 64, ""), ("int4", 5000, 64, 256, 64, ""),
+    ("int8", 2100, 1100, 256, 0, ""), ("int8", 450, 14336, 256, 0, ""), ("fp6", 900, 2048, 256, 0, ""), ("fp6", 3000, 320, 512, 0, ""),
+])
+def test_every_tile_once(fmt, M, N, K, group, name):
+    """Tiles are taken in panels of tile rows, the last of them lower: single weights bit for bit in every tile, panels of one to
+    many rows, one or few columns."""
+    from ao_amd import _lib, ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w = torch.randn(N, K, device="cuda", generator=g) * 0.02
+    at = torch.randint(0, K, (M,), device="cuda", generator=g)
+    x = torch.zeros(M, K, device="cuda", dtype=torch.float16 if fmt == "fp6" else torch.bfloat16)
+    x[torch.arange(M, device="cuda"), at] = 1.0
+    if fmt == "int4":
+        assert _lib.int4wo_linear_plan(M, K, N, group).startswith(name)
+        packed, qp = ops.int4wo_quantize_pack(w.bfloat16(), group)
+        dq, y = ops.int4wo_dequantize(packed, qp, N, K, group), ops.int4wo_linear(x, packed, qp, group, N)
+    elif fmt == "int8":
+        q, scale = (w * 3000).round().clamp(-127, 127).to(torch.int8), torch.rand(N, device="cuda", generator=g).bfloat16()
+        dq, y = (q.float() * scale.float()[:, None]).bfloat16(), ops.int8wo_linear(x, q, scale)
+    else:
+        tc, scale = ops.fp6_quantize_pack(w.half(), 3, 2)
+        native = ops.fp6_repack(tc, 6)
+        dq, y = ops.fp6_dequantize(tc, scale, 3, 2).half(), ops.fp6_linear_native(3, 2, x, native, scale)
+    assert torch.equal(y, dq[:, at].t())
