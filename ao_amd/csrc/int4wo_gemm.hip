@@ -164,7 +164,7 @@ __device__ __forceinline__ const T* uniform_ptr(const T* p) {
 //              the activation slice of step s + 2, into this step's buffer;
 //   ks 0:      requests the second half of the activation slice of step s + 1.
 template <int G, int NT>
-__global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a, const TileOrder order) {
+__global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a, int tiles_m, int tiles_n, int panel) {
     // NT 32-column blocks per wave: workgroup tile 256 x 128 NT.  NT = 1 halves the tile for shapes whose 256 x 256
     // tiles would leave CUs idle; it pays with twice the LDS reads and dequantization issue slots per matrix instruction.
     constexpr int BM = 256, WN = 32 * NT, BN = 4 * WN, MT = 8, XCH = 8, SLOTS = MT * NT;
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int tile_m, tile_n;
-    if (!tile_at(order, (int)blockIdx.x, tile_m, tile_n)) return;
+    if (!tile_at(TileOrder{tiles_m, tiles_n, panel}, (int)blockIdx.x, tile_m, tile_n)) return;
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
     // the 64-wide K steps of this workgroup: all of them, or with a.ksplit > 1 the blockIdx.y-th run of an even number of them,
     // whose fp32 products go to part blockIdx.y of a.y [ksplit][M][ldy]
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a
 // for the step after next, into the slice that the step before has left) have a whole step to arrive.  13824 x 5120 at 77 rows
 // 31.0 us on 128-row tiles, 27.9 on 96-row tiles with two slices, 24.7 with three.
 template <int G, int MT>
-__device__ __forceinline__ void gemm_kwave(const LinearArgs& a, const TileOrder& order) {
+__device__ __forceinline__ void gemm_kwave(const LinearArgs& a, int tiles_m, int tiles_n, int panel) {
     constexpr int BM = 32 * MT, BN = 64, NT = 2, XCH = 4 * MT, SLOTS = MT * NT;
     constexpr int NB = MT == 3 ? 3 : 2, BUF = BM * 128;   // activation slices of a wave in LDS: as many as 160 KB hold
     __shared__ __align__(16) uint8_t lds[4][NB][BUF];
@@ -423,7 +423,7 @@ __device__ __forceinline__ void gemm_kwave(const LinearArgs& a, const TileOrder&
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int tile_m, tile_n;
-    if (!tile_at(order, (int)blockIdx.x, tile_m, tile_n)) return;
+    if (!tile_at(TileOrder{tiles_m, tiles_n, panel}, (int)blockIdx.x, tile_m, tile_n)) return;
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
     const int KS = (int)(a.Kp / 64);
     const int KB = (int)(a.Kp / 128);
@@ -639,12 +639,12 @@ __device__ __forceinline__ void gemm_kwave(const LinearArgs& a, const TileOrder&
 }
 
 template <int G>
-__global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs a, const TileOrder order) {
-    gemm_kwave<G, 4>(a, order);
+__global__ __launch_bounds__(256) void int4wo_gemm_kwave_kernel(const LinearArgs a, int tiles_m, int tiles_n, int panel) {
+    gemm_kwave<G, 4>(a, tiles_m, tiles_n, panel);
 }
 template <int G>
-__global__ __launch_bounds__(256) void int4wo_gemm_kwave96_kernel(const LinearArgs a, const TileOrder order) {
-    gemm_kwave<G, 3>(a, order);
+__global__ __launch_bounds__(256) void int4wo_gemm_kwave96_kernel(const LinearArgs a, int tiles_m, int tiles_n, int panel) {
+    gemm_kwave<G, 3>(a, tiles_m, tiles_n, panel);
 }
 
 struct GemmLdsPlan {
@@ -718,13 +718,13 @@ bool int4wo_gemm_lds_plan(const LinearArgs& a, int64_t g, Int4Plan* plan) {
 static void launch_gemm_kwave(const LinearArgs& a, int64_t g, const GemmLdsPlan& p, hipStream_t st) {
     const bool three = (a.M + 95) / 96 == p.tiles_m;   // 96-row tiles where they are no more
     const TileOrder order = tile_order(p.tiles_m, p.tiles_n, (three ? 96 : 128) * 128, 64 * 32);
-    const dim3 grid((unsigned)(order.per_xcd * 8)), block(256);
+    const dim3 grid((unsigned)(order.per_xcd() * 8)), block(256);
     auto go = [&](auto kernel) {
         if (g_prof_start && g_prof_stop) {
-            hipExtLaunchKernelGGL(kernel, grid, block, 0, st, g_prof_start, g_prof_stop, 0, a, order);
+            hipExtLaunchKernelGGL(kernel, grid, block, 0, st, g_prof_start, g_prof_stop, 0, a, order.tiles_m, order.tiles_n, order.panel);
             g_prof_start = g_prof_stop = nullptr;
         } else {
-            hipLaunchKernelGGL(kernel, grid, block, 0, st, a, order);
+            hipLaunchKernelGGL(kernel, grid, block, 0, st, a, order.tiles_m, order.tiles_n, order.panel);
         }
     };
     switch (g) {
@@ -738,13 +738,13 @@ static void launch_gemm_kwave(const LinearArgs& a, int64_t g, const GemmLdsPlan&
 template <int NT>
 static void launch_gemm_lds_nt(const LinearArgs& a, int64_t g, const GemmLdsPlan& p, hipStream_t st) {
     const TileOrder order = tile_order(p.tiles_m, p.tiles_n, 256 * 128, 128 * NT * 32);
-    const dim3 grid((unsigned)(order.per_xcd * 8), (unsigned)a.ksplit), block(256);
+    const dim3 grid((unsigned)(order.per_xcd() * 8), (unsigned)a.ksplit), block(256);
     auto go = [&](auto kernel) {
         if (g_prof_start && g_prof_stop) {
-            hipExtLaunchKernelGGL(kernel, grid, block, 0, st, g_prof_start, g_prof_stop, 0, a, order);
+            hipExtLaunchKernelGGL(kernel, grid, block, 0, st, g_prof_start, g_prof_stop, 0, a, order.tiles_m, order.tiles_n, order.panel);
             g_prof_start = g_prof_stop = nullptr;
         } else {
-            hipLaunchKernelGGL(kernel, grid, block, 0, st, a, order);
+            hipLaunchKernelGGL(kernel, grid, block, 0, st, a, order.tiles_m, order.tiles_n, order.panel);
         }
     };
     switch (g) {

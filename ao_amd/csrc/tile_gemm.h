@@ -324,7 +324,7 @@ template <class F, int WN, int KW, int MT, int NT>
 void tile_launch(const TileGemmArgs& a, int parts, hipStream_t st) {
     hipEvent_t ev0 = g_prof_start, ev1 = g_prof_stop;
     g_prof_start = g_prof_stop = nullptr;
-    hipExtLaunchKernelGGL((tile_gemm_kernel<F, WN, KW, MT, NT>), dim3((unsigned)(a.order.per_xcd * 8), (unsigned)parts), dim3(64 * WN * KW), 0, st,
+    hipExtLaunchKernelGGL((tile_gemm_kernel<F, WN, KW, MT, NT>), dim3((unsigned)(a.order.per_xcd() * 8), (unsigned)parts), dim3(64 * WN * KW), 0, st,
                           ev0, ev1, 0, a);
 }
 template <class F>

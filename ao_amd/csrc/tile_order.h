@@ -16,7 +16,8 @@
 namespace ao {
 
 struct TileOrder {
-    int tiles_m, tiles_n, panel, per_xcd;
+    int tiles_m, tiles_n, panel;
+    __host__ __device__ int per_xcd() const { return (tiles_m * tiles_n + 7) / 8; }
 };
 
 // x_bytes, w_bytes: what a tile reads of the activations and of the weight for the same stretch of K
@@ -25,13 +26,13 @@ inline TileOrder tile_order(int64_t tiles_m, int64_t tiles_n, int64_t x_bytes, i
     const double high = sqrt(2.0 * (double)at_once * (double)w_bytes / (double)x_bytes);
     int64_t panels = high >= 1.0 ? (int64_t)((double)tiles_m / high + 0.5) : tiles_m;
     panels = panels < 1 ? 1 : panels;
-    return TileOrder{(int)tiles_m, (int)tiles_n, (int)((tiles_m + panels - 1) / panels), (int)per_xcd};
+    return TileOrder{(int)tiles_m, (int)tiles_n, (int)((tiles_m + panels - 1) / panels)};
 }
 
 // The tile of workgroup `block`; false past the last one
 __device__ __forceinline__ bool tile_at(const TileOrder& o, int block, int& tile_m, int& tile_n) {
-    const int tile = (block & 7) * o.per_xcd + (block >> 3);
-    if (block >> 3 >= o.per_xcd || tile >= o.tiles_m * o.tiles_n) return false;
+    const int per_xcd = o.per_xcd(), tile = (block & 7) * per_xcd + (block >> 3);
+    if (block >> 3 >= per_xcd || tile >= o.tiles_m * o.tiles_n) return false;
     const int per_panel = o.panel * o.tiles_n;
     int p = 0, in = tile;
     if (tile >= per_panel) p = tile / per_panel, in = tile - p * per_panel;
