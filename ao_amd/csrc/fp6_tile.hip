@@ -14,6 +14,9 @@ typedef uint32_t ft_u32x6 __attribute__((ext_vector_type(6)));
 
 template <bool E3M2>
 struct Fp6Tile {
+    static constexpr bool PAIR = false;
+    typedef uint32_t Piece;
+    static __device__ __forceinline__ uint32_t pack(Piece p) { return p; }
     static constexpr int REQ = 2, BLOCK_BYTES = 2048;   // 1 KB of first dwords, 512 bytes of last dwords and their repetition
     struct Row { ft_f16x2 scale; };
     struct Raw { uint4 lo; uint2 hi; };     // 32 codes of 6 bits
@@ -35,7 +38,7 @@ struct Fp6Tile {
         const _Float16 s = __builtin_bit_cast(_Float16, ((const uint16_t*)a.scale)[n < a.N ? n : a.N - 1]);
         return Row{{s, s}};
     }
-    static __device__ __forceinline__ Raw read(const uint8_t* block, int lane) {
+    static __device__ __forceinline__ Raw read(const uint8_t* block, int lane, bool) {
         const int slot = ((lane & 16) << 1) + (lane >> 5) * 16 + (lane & 15);   // row lane % 32, half lane / 32
         return Raw{*(const uint4*)(block + slot * 16), *(const uint2*)(block + 1024 + slot * 8)};
     }

@@ -12,6 +12,9 @@
 namespace ao {
 
 struct Int4Tile {
+    static constexpr bool PAIR = false;
+    typedef uint32_t Piece;
+    static __device__ __forceinline__ uint32_t pack(Piece p) { return p; }
     static constexpr int REQ = 2, BLOCK_BYTES = 1024 + 256;
     struct Row {};
     struct Raw { uint4 codes; uint32_t qp; };   // 32 consecutive k of one row, the scale and zero of their group
@@ -38,7 +41,7 @@ struct Int4Tile {
             tg_dma4(lds + 1024, (const uint8_t*)a.scale + (n0 / 16) * (padded_k(a) >> a.group_shift) * 64 + (((int64_t)s * 64) >> a.group_shift) * 64, off);
     }
     static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) { return Row(); }
-    static __device__ __forceinline__ Raw read(const uint8_t* block, int lane) {
+    static __device__ __forceinline__ Raw read(const uint8_t* block, int lane, bool) {
         const int slot = ((lane & 16) << 1) + (lane >> 5) * 16 + (lane & 15);   // row lane % 32, half lane / 32
         return Raw{*(const uint4*)(block + slot * 16), *(const uint32_t*)(block + 1024 + slot * 4)};
     }

@@ -10,33 +10,40 @@ namespace ao {
 
 typedef __bf16 i8_bf16x8 __attribute__((ext_vector_type(8)));
 
+template <bool PAIR_>
 struct Int8Tile {
+    static constexpr bool PAIR = PAIR_;
     static constexpr int REQ = 2, BLOCK_BYTES = 2048;   // 32 rows x 64 bytes
     struct Row {};
     struct Raw { uint4 v[2]; };             // 32 consecutive k of one row
     typedef Raw Ready;
     struct Cols { float scale[4], bias[4]; bool has_bias; };
 
-    // request r: 16 rows x 64 bytes; slot (row, p) holds 16-byte chunk p ^ (row / 4 % 4): conflict-free reads
+    // request r: 8 rows x 128 bytes, two steps; slot (row, p) holds 16-byte chunk p ^ (row / 2 % 8): conflict-free reads.  Where K is no
+    // multiple of 128, 16 rows x 64 bytes with chunk p ^ (row / 4 % 4).
     static __device__ __forceinline__ uint32_t lane_offset(const TileGemmArgs& a, int64_t n0, int64_t n, int r, int lane) {
-        const int row = r * 16 + (lane >> 2);
+        const int row = PAIR ? r * 8 + (lane >> 3) : r * 16 + (lane >> 2);
         const int64_t rel = (n + row < a.N ? n + row : a.N - 1) - n0;   // rows past N repeat the last one
-        return (uint32_t)(rel * a.ldw) + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
+        return (uint32_t)(rel * a.ldw) + ((PAIR ? (lane & 7) ^ ((row >> 1) & 7) : (lane & 3) ^ ((row >> 2) & 3)) << 4);
     }
     static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, uint32_t off) {
         tg_dma(lds + r * 1024, a.w + n0 * a.ldw + (int64_t)s * 64, off);
     }
     static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) { return Row(); }
-    static __device__ __forceinline__ Raw read(const uint8_t* block, int lane) {
+    static __device__ __forceinline__ Raw read(const uint8_t* block, int lane, bool odd) {
         const int n = lane & 31, half = lane >> 5;
         Raw r;
-        r.v[0] = *(const uint4*)(block + n * 64 + (((2 * half) ^ ((n >> 2) & 3)) << 4));
-        r.v[1] = *(const uint4*)(block + n * 64 + (((2 * half + 1) ^ ((n >> 2) & 3)) << 4));
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+            r.v[c] = *(const uint4*)(block + (PAIR ? n * 128 + (((4 * odd + 2 * half + c) ^ ((n >> 1) & 7)) << 4)
+                                                   : n * 64 + (((2 * half + c) ^ ((n >> 2) & 3)) << 4)));
         return r;
     }
     static __device__ __forceinline__ Ready prepare(const Raw& r, const Row&) { return r; }
-    // dword d (k = 8 s + 2 d, + 1) of slice s
-    static __device__ __forceinline__ uint32_t piece(const Ready& r, int s, int d) {
+    // dword d (k = 8 s + 2 d, + 1) of slice s; a pack right behind its byte conversions would wait for them
+    struct Piece { float f0, f1; };
+    static __device__ __forceinline__ uint32_t pack(const Piece& p) { return hw_bf16_pack(p.f0, p.f1); }
+    static __device__ __forceinline__ Piece piece(const Ready& r, int s, int d) {
         const uint4 v = r.v[s >> 1];
         const uint32_t w = s & 1 ? (d < 2 ? v.z : v.w) : (d < 2 ? v.x : v.y);
         float f0, f1;
@@ -46,7 +53,7 @@ struct Int8Tile {
         else
             asm("v_cvt_f32_i32_sdwa %0, sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0\n\t"
                 "v_cvt_f32_i32_sdwa %1, sext(%2) dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1" : "=&v"(f0), "=&v"(f1) : "v"(w));
-        return hw_bf16_pack(f0, f1);
+        return Piece{f0, f1};
     }
     static __device__ __forceinline__ tg_f32x16 mul(uint4 w, uint4 x, tg_f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(i8_bf16x8, w), __builtin_bit_cast(i8_bf16x8, x), c, 0, 0, 0);
@@ -98,18 +105,28 @@ void int8wo_gemm_describe(const TilePlan& p, char* out, size_t cap) {
     snprintf(out, cap, "tile %dx%d parts=%d", kInt8Shapes[p.shape].bm, kInt8Shapes[p.shape].bn, p.parts);
 }
 
+template <bool PAIR>
+static bool launch_paired(const TileGemmArgs& a, const TilePlan& p, hipStream_t st) {
+    typedef Int8Tile<PAIR> F;
+    switch (p.shape) {
+        case 0: tile_launch<F, 4, 2, 2, 1>(a, p.parts, st); return true;
+        case 4: tile_launch<F, 8, 1, 4, 1>(a, p.parts, st); return true;
+        default: return false;
+    }
+}
+
 void launch_int8wo_gemm(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
     tile_grid(a, kInt8Shapes[p.shape], 64, p.parts);
-    switch (p.shape) {
-        case 0: tile_launch<Int8Tile, 4, 2, 2, 1>(a, p.parts, st); break;
-        case 1: tile_launch<Int8Tile, 4, 1, 3, 1>(a, p.parts, st); break;
-        case 2: tile_launch<Int8Tile, 4, 2, 4, 1>(a, p.parts, st); break;
-        case 3: tile_launch<Int8Tile, 4, 1, 6, 1>(a, p.parts, st); break;
-        case 4: tile_launch<Int8Tile, 8, 1, 4, 1>(a, p.parts, st); break;
-        case 5: tile_launch<Int8Tile, 2, 4, 2, 1>(a, p.parts, st); break;
-        default: tile_launch<Int8Tile, 8, 1, 6, 1>(a, p.parts, st); break;
+    if (!(a.K % 128 == 0 ? launch_paired<true>(a, p, st) : launch_paired<false>(a, p, st))) {
+        switch (p.shape) {
+            case 1: tile_launch<Int8Tile<false>, 4, 1, 3, 1>(a, p.parts, st); break;
+            case 2: tile_launch<Int8Tile<false>, 4, 2, 4, 1>(a, p.parts, st); break;
+            case 3: tile_launch<Int8Tile<false>, 4, 1, 6, 1>(a, p.parts, st); break;
+            case 5: tile_launch<Int8Tile<false>, 2, 4, 2, 1>(a, p.parts, st); break;
+            default: tile_launch<Int8Tile<false>, 8, 1, 6, 1>(a, p.parts, st); break;
+        }
     }
-    tile_finish<Int8Tile>(a, p.parts, st);
+    tile_finish<Int8Tile<false>>(a, p.parts, st);
 }
 
 }  // namespace ao

@@ -20,6 +20,7 @@
 // tiles for a wave (64 columns, half the LDS reads).
 #pragma once
 #include "tile_order.h"
+#include <type_traits>
 
 namespace ao {
 
@@ -56,21 +57,27 @@ __device__ __forceinline__ void tg_dma4(uint32_t lds, const void* base, uint32_t
 
 // A weight format F describes a block of 32 weight rows of one 64-wide K step:
 //   REQ, BLOCK_BYTES      requests that bring it into LDS, and its bytes there
+//   PAIR                  whether two steps' worth is brought in at once (a row's 64 k are half a 128-byte line)
 //   lane_offset(a, n0, n, r, lane)   this lane's offset of request r from the tile's base, rows n ..
 //   request(a, n0, s, r, lds, off)   issues request r of step s for a block at `lds`
-//   Raw read(block, lane)            a lane's share: row lane % 32, the 32 k of half lane / 32
+//   Raw read(block, lane, odd)       a lane's share: row lane % 32, the 32 k of half lane / 32 (PAIR: of the first or second step)
 //   Ready prepare(raw, row)          whatever is computed once per step
-//   uint32_t piece(ready, s, d)      two dequantized weights: dword d of the 8 k of slice s
+//   Piece piece(ready, s, d)         two dequantized weights: dword d of the 8 k of slice s, up to
+//   uint32_t pack(piece)             the work left for the end of the slice
 //   mul, columns, finish, combine    the matrix instruction and the epilogue
 template <class F, int WN, int KW, int MT, int NT>
 __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmArgs a) {
     constexpr int G = WN, BM = 32 * MT, BN = 32 * NT * WN;
-    constexpr int ABYTES = BM * 128, STAGE = ABYTES + WN * NT * F::BLOCK_BYTES;
+    constexpr bool PAIR = F::PAIR;
+    constexpr int ABYTES = BM * 128, BBYTES = WN * NT * F::BLOCK_BYTES, STAGE = ABYTES + BBYTES;
     constexpr int STAGES = KW * 4 * STAGE <= 160 * 1024 ? 4 : 3;
-    constexpr int AREQ = ABYTES / 1024 / G, BREQ = NT * F::REQ, REQ = AREQ + BREQ;
+    // with PAIR the weights have a ring of their own, of three pairs of steps
+    constexpr int RING = PAIR ? STAGES * ABYTES + 6 * BBYTES : STAGES * STAGE;
+    static_assert(!PAIR || KW * RING <= 160 * 1024, "LDS of a CU");
+    constexpr int AREQ = ABYTES / 1024 / G, BREQ = NT * F::REQ * (PAIR ? 2 : 1), REQ = AREQ + BREQ;
     static_assert(AREQ * G * 1024 == ABYTES, "every wave issues the same number of requests");
     constexpr int ACC = MT * NT * 4096;   // bytes of one wave's accumulators
-    constexpr int LDS = KW * STAGES * STAGE > (KW - 1) * G * ACC ? KW * STAGES * STAGE : (KW - 1) * G * ACC;
+    constexpr int LDS = KW * RING > (KW - 1) * G * ACC ? KW * RING : (KW - 1) * G * ACC;
     __shared__ __align__(1024) uint8_t lds[LDS];
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -80,8 +87,11 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
     if (!tile_at(a.order, (int)blockIdx.x, tile_m, tile_n)) return;
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
     // this workgroup's run of 64-wide K steps: all of them, or the blockIdx.y-th of gridDim.y equal parts
-    const int all = (int)(a.K / 64), per = (all + (int)gridDim.y - 1) / (int)gridDim.y, first = per * (int)blockIdx.y;
-    const int KS = min(per, all - first), nst = (KS + KW - 1) / KW;
+    // (PAIR: whole pairs, and the groups take pairs; a last part may be left without any and stores zeros)
+    constexpr int UNIT = PAIR ? 2 : 1;
+    const int all = (int)(a.K / 64), per = (all / UNIT + (int)gridDim.y - 1) / (int)gridDim.y * UNIT, first = per * (int)blockIdx.y;
+    const int KS = PAIR ? max(min(per, all - first), 0) : min(per, all - first);
+    const int nst = PAIR ? KS / (2 * KW) * 2 + min(KS % (2 * KW), 2) : (KS + KW - 1) / KW;
 
     // Activation request j of a wave: 8 rows x 128 bytes, slot (row, p) holds k chunk p ^ (row / 2 % 8), so that the fragment
     // reads below (16 rows, one chunk) cover all banks.  Rows past M repeat the last one; their outputs are not stored.
@@ -93,12 +103,25 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
         aoff[j] = (uint32_t)(rel * a.ldx * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
     }
 #pragma unroll
-    for (int j = 0; j < BREQ; ++j) boff[j] = F::lane_offset(a, n0, n0 + (gw * NT + j / F::REQ) * 32, j % F::REQ, lane);
+    for (int j = 0; j < BREQ; ++j) boff[j] = F::lane_offset(a, n0, n0 + (gw * NT + j / (UNIT * F::REQ)) * 32, j % (UNIT * F::REQ), lane);
     const uint16_t* const abase = a.x + m0 * a.ldx;
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + group * STAGES * STAGE;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + group * RING;
+    // request r of step t: the activations' into `buf`, then the weights'; with PAIR first the weights of steps t .. t + 1, into pair
+    // buffer `buf`, then the activations
     auto request = [&](int r, int t, int buf) __attribute__((always_inline)) {
+        // (a request past the end repeats the last step's and is not used)
+        if constexpr (PAIR) {
+            const bool weights = r < BREQ;
+            const int s = min(first + (t >> 1) * 2 * KW + 2 * group + (t & 1), max(min(first + KS, all) - (weights ? 2 : 1), 0));
+            if (weights)
+                F::request(a, n0, s, r % (2 * F::REQ),
+                           lds0 + STAGES * ABYTES + buf * 2 * BBYTES + (gw * NT + r / (2 * F::REQ)) * 2 * F::BLOCK_BYTES, boff[r]);
+            else
+                tg_dma(lds0 + buf * ABYTES + (gw * AREQ + r - BREQ) * 1024, abase + (int64_t)s * 64, aoff[r - BREQ]);
+            return;
+        }
         int s = t * KW + group;
-        s = first + (s < KS ? s : KS - 1);   // a request past the end repeats the last step's and is not used
+        s = first + (s < KS ? s : KS - 1);
         const uint32_t at = lds0 + buf * STAGE;
         if (r < AREQ)
             tg_dma(at + (gw * AREQ + r) * 1024, abase + (int64_t)s * 64, aoff[r]);
@@ -125,13 +148,25 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
     // step, which then had to see step t + 2 arrive, the three-buffer shapes had less than one: 64 x 64 tiles of int8 at 106
     // rows, 4888 x 3456, 18.4 -> 14.4 us.)  A slice is MT x NT slots of one matrix instruction each; its share of the
     // conversion, the LDS reads and the requests are dealt out over the slots.
+    //
+    // PAIR: an even step t requests the weights of steps t + 4 and t + 5 into the pair buffer that steps t - 2 and t - 1 have left.
+    // An int8 row's 64 k of one step are half a line of the L1, which has passed on by the time the other half is asked for:
+    // 13824 x 5120 at 113 rows 37.5 -> 34.0 us, 14336 x 4096 at 128 / 1149 / 2000 rows 29.5 / 133.8 / 242 -> 27.3 / 129.8 / 234.  (With
+    // two pairs in the ring, requested two steps ahead, 96 x 128 tiles lost 8 %; with three they do not gain, nor do 192 x 128.)
     constexpr int SLOTS = MT * NT, PIECES = NT * 4;
 #pragma unroll
     for (int t = 0; t < STAGES - 1; ++t)
 #pragma unroll
-        for (int r = 0; r < REQ; ++r) request(r, t, t);
-    auto a_at = [&](int buf) { return lds + (group * STAGES + buf) * STAGE; };
-    auto b_at = [&](int buf, int j) { return lds + (group * STAGES + buf) * STAGE + ABYTES + (gw * NT + j) * F::BLOCK_BYTES; };
+        for (int r = 0; r < REQ; ++r) {
+            if (!PAIR || r >= BREQ) request(r, t, t);
+            else if (t < 2) request(r, 2 * t, t);
+        }
+    auto a_at = [&](int buf) { return lds + group * RING + buf * (PAIR ? ABYTES : STAGE); };
+    // the weights of a step, or with PAIR of a pair, in buffer `buf`
+    auto b_at = [&](int buf, int j) {
+        if constexpr (PAIR) return lds + group * RING + STAGES * ABYTES + buf * 2 * BBYTES + (gw * NT + j) * 2 * F::BLOCK_BYTES;
+        else return lds + group * RING + buf * STAGE + ABYTES + (gw * NT + j) * F::BLOCK_BYTES;
+    };
     auto read_a = [&](const uint8_t* A, int i, int s) __attribute__((always_inline)) {
         return *(const uint4*)(A + (i * 32 + r32) * 128 + (((4 * half + s) ^ ((r32 >> 1) & 7)) << 4));
     };
@@ -139,27 +174,32 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
     Frag fa[2][MT], fb[2][NT];
     typename F::Raw raw[NT];
     typename F::Ready ready[NT];
-    tg_wait_barrier<(STAGES - 2) * REQ>();
+    tg_wait_barrier<PAIR ? (STAGES - 2) * AREQ + BREQ : (STAGES - 2) * REQ>();
 #pragma unroll
-    for (int j = 0; j < NT; ++j) ready[j] = F::prepare(F::read(b_at(0, j), lane), row_const[j]);
+    for (int j = 0; j < NT; ++j) ready[j] = F::prepare(F::read(b_at(0, j), lane, false), row_const[j]);
 #pragma unroll
     for (int i = 0; i < MT; ++i) fa[0][i].q = read_a(a_at(0), i, 0);
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int d = 0; d < 4; ++d) fb[0][j].u[d] = F::piece(ready[j], 0, d);
-    int buf = 0;
+        for (int d = 0; d < 4; ++d) fb[0][j].u[d] = F::pack(F::piece(ready[j], 0, d));
+    int buf = 0, pair = 0;   // this step's buffer, its pair's
     // (a group that has one step less runs one less; a test around every matrix instruction of that step cost 2 to 5 %)
-    const int own = (KS - group + KW - 1) / KW;
-    for (int t = 0; t < own; ++t) {
+    const int own = PAIR ? KS / (2 * KW) * 2 + min(max(KS % (2 * KW) - 2 * group, 0), 2) : (KS - group + KW - 1) / KW;
+    auto step = [&](int t, auto odd) __attribute__((always_inline)) {
+        constexpr bool ODD = decltype(odd)::value;   // of PAIR's two steps
+        constexpr int NREQ = PAIR && ODD ? AREQ : REQ;
         const int next = buf + 1 == STAGES ? 0 : buf + 1, ahead = buf == 0 ? STAGES - 1 : buf - 1;
+        const int pair_ahead = pair == 0 ? 2 : pair - 1;
+        if (PAIR && ODD) pair = pair == 2 ? 0 : pair + 1;   // (from here on the next step's)
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const int cur = s & 1, nxt = cur ^ 1;
+            typename F::Piece piece[PIECES];
             if (s == 3) {
-                tg_wait_barrier<(STAGES - 2) * REQ>();
+                tg_wait_barrier<PAIR ? (STAGES - 2) * AREQ + BREQ : (STAGES - 2) * REQ>();
 #pragma unroll
-                for (int j = 0; j < NT; ++j) raw[j] = F::read(b_at(next, j), lane);
+                for (int j = 0; j < NT; ++j) raw[j] = F::read(b_at(PAIR ? pair : next, j), lane, !ODD);
             }
 #pragma unroll
             for (int q = 0; q < SLOTS; ++q) {
@@ -173,16 +213,31 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
                 const int p0 = s < 3 ? q * PIECES / SLOTS : q == 0 ? 0 : (q - 1) * PIECES / (SLOTS - 1);
                 const int p1 = s < 3 ? (q + 1) * PIECES / SLOTS : q * PIECES / (SLOTS - 1);
 #pragma unroll
-                for (int p = p0; p < p1; ++p) fb[nxt][p / 4].u[p % 4] = F::piece(ready[p / 4], (s + 1) & 3, p % 4);
+                for (int p = p0; p < p1; ++p) piece[p] = F::piece(ready[p / 4], (s + 1) & 3, p % 4);
+                if (q == SLOTS - 1)
+#pragma unroll
+                    for (int p = 0; p < PIECES; ++p) fb[nxt][p / 4].u[p % 4] = F::pack(piece[p]);
                 if (s < 2)
 #pragma unroll
-                    for (int r = (s * SLOTS + q) * REQ / (2 * SLOTS); r < (s * SLOTS + q + 1) * REQ / (2 * SLOTS); ++r) request(r, t + STAGES - 1, ahead);
+                    for (int r = (s * SLOTS + q) * NREQ / (2 * SLOTS); r < (s * SLOTS + q + 1) * NREQ / (2 * SLOTS); ++r) {
+                        if (PAIR && !ODD && r < BREQ) request(r, t + 4, pair_ahead);
+                        else request(PAIR && ODD ? r + BREQ : r, t + STAGES - 1, ahead);
+                    }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
         buf = next;
+    };
+    if constexpr (PAIR) {
+        for (int t = 0; t < own; t += 2) {   // (a group's steps are whole pairs)
+            step(t, std::false_type());
+            step(t + 1, std::true_type());
+        }
+    } else {
+        for (int t = 0; t < own; ++t) step(t, std::false_type());
     }
-    if (KW > 1 && own < nst) tg_wait_barrier<0>();   // the barrier of the step that this group does not have
+    if (KW > 1)
+        for (int t = own; t < nst; ++t) tg_wait_barrier<0>();   // the barriers of the steps that this group does not have
     // requests past the end have landed before LDS is used again or the workgroup ends
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
     if (KW > 1) {

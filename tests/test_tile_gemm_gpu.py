@@ -58,6 +58,19 @@ def test_int8_tiles(case):
     _run(*case)
 
 
+# weights that come in two steps at a time: one pair, one more or fewer than the ring and the groups hold, K parts of
+# different lengths, a last row of the weight that ends the buffer, and the widths that end within a pair
+@pytest.mark.parametrize("case,plan", [
+    ((390, 14336, 128), "tile 128x256 parts=1"), ((390, 14336, 384), "tile 128x256 parts=1"), ((391, 14330, 640), "tile 128x256 parts=1"),
+    ((390, 14336, 576), "tile 128x256 parts=1"), ((131, 8192, 256), "tile 64x128 parts=1"), ((257, 4096, 384), "tile 64x128 parts=1"),
+    ((257, 4096, 640), "tile 64x128 parts=1"), ((516, 2048, 1152), "tile 64x128 parts=1"), ((257, 4096, 704), "tile 64x128 parts=1"),
+    ((40, 14336, 6400), "tile 64x128 parts=2"), ((257, 1024, 6400), "tile 64x128 parts=4"), ((131, 1024, 9088), "tile 64x128 parts=8"),
+])
+def test_int8_weights_in_pairs_of_steps(case, plan):
+    assert _plan(*case) == plan
+    _run(*case)   # (the bound of _run: at most 9088 exact products a sum)
+
+
 @pytest.mark.parametrize("case", [(65, 5121, 6528), (257, 21000, 1024), (129, 1100, 4096)])
 def test_int8_tiles_bias_and_row_stride(case):
     _run(*case, bias=True, pad=72)
