@@ -30,9 +30,9 @@ struct Fp6Tile {
         if (nb >= nblocks) nb = nblocks - 1;   // a row block past N repeats the last one; its columns are not stored
         return (uint32_t)((nb - n0 / 16) * a.ldw) + (r == 0 ? lane & 31 : lane & 15) * 16;
     }
-    static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, uint32_t off) {
-        const uint8_t* const tile = a.w + (n0 / 16) * a.ldw + (int64_t)(s >> 1) * 1536;
-        tg_dma(lds + r * 1024, tile + (r == 0 ? (s & 1) * 512 : 1024 + (s & 1) * 256), off);
+    static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, int at, uint32_t off) {
+        const uint8_t* const tile = a.w + (n0 / 16) * a.ldw + (uint32_t)((s >> 1) * 1536 + (s & 1) * (r == 0 ? 512 : 256));
+        tg_dma(lds, at + r * 1024, tile, off + (r == 0 ? 0 : 1024));
     }
     static __device__ __forceinline__ Row row(const TileGemmArgs& a, int64_t n) {
         const _Float16 s = __builtin_bit_cast(_Float16, ((const uint16_t*)a.scale)[n < a.N ? n : a.N - 1]);

@@ -2,7 +2,7 @@
 // y[M, N] = x[M, K] . dequant(W)[N, K]^T, torchao/dtypes/affine_quantized_tensor.py:600-640.  The packed codes of 32 weight
 // rows and one 64-wide K step are one request of 1 KB (two runs of 512 bytes), their (scale, zero) words a second one.
 //
-// What bounds it: the exact two-rounding dequantization, 34 VALU instructions per 8 weights, against MT matrix instructions
+// What bounds it: the exact two-rounding dequantization, 33 VALU instructions per 8 weights, against MT matrix instructions
 // (MT = rows of the tile / 32).  Two waves per SIMD (two groups along K) overlap one wave's dequantization with the other's
 // matrix instructions: 96 x 128 tiles of 14336 x 4096 at 160 rows take 36 us, where the 128 x 64 tiles of int4wo_gemm.hip, one
 // wave per SIMD and a second round, take 45.
@@ -16,9 +16,9 @@ struct Int4Tile {
     typedef uint32_t Piece;
     static __device__ __forceinline__ uint32_t pack(Piece p) { return p; }
     static constexpr int REQ = 2, BLOCK_BYTES = 1024 + 256;
-    struct Row {};
+    struct Row { uint32_t even, odd, one; };   // masks of the even and odd pairs, the fp16 pair (1024, 1024)
     struct Raw { uint4 codes; uint32_t qp; };   // 32 consecutive k of one row, the scale and zero of their group
-    struct Ready { uint32_t w[4]; float s, c, s16, c16, z; };   // c = -1032 s, s16 = s / 16, c16 = -72 s
+    struct Ready { uint32_t w[4]; float s, c, s16, c16, z; Row k; };   // c = -1032 s, s16 = s / 16, c16 = -72 s
     struct Cols { float bias[4]; };
 
     // in_features as packed, a multiple of max(128, group); the K steps end at in_features, a multiple of 64
@@ -34,35 +34,45 @@ struct Int4Tile {
         // one word per row and group: a 64-wide step has two groups of 32 or lies within one
         return (uint32_t)(rel * (padded_k(a) >> a.group_shift) * 64) + (a.group_shift == 5 ? half * 64 : 0) + row * 4;
     }
-    static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, uint32_t off) {
+    static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, int at, uint32_t off) {
         if (r == 0)
-            tg_dma(lds, a.w + (n0 / 16) * a.ldw + (int64_t)s * 512, off);
+            tg_dma(lds, at, a.w + (n0 / 16) * a.ldw + (uint32_t)s * 512u, off);
         else
-            tg_dma4(lds + 1024, (const uint8_t*)a.scale + (n0 / 16) * (padded_k(a) >> a.group_shift) * 64 + (((int64_t)s * 64) >> a.group_shift) * 64, off);
+            tg_dma4(lds, at + 1024, (const uint8_t*)a.scale + (n0 / 16) * (padded_k(a) >> a.group_shift) * 64 + (((uint32_t)s * 64u) >> a.group_shift) * 64u, off);
     }
-    static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) { return Row(); }
+    static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) {
+        Row k;   // in registers, so that one instruction masks and inserts
+        asm("s_mov_b32 %0, 0x000F000F" : "=s"(k.even));
+        asm("s_mov_b32 %0, 0x00F000F0" : "=s"(k.odd));
+        asm("v_mov_b32 %0, 0x64006400" : "=v"(k.one));
+        return k;
+    }
     static __device__ __forceinline__ Raw read(const uint8_t* block, int lane, bool) {
         const int slot = ((lane & 16) << 1) + (lane >> 5) * 16 + (lane & 15);   // row lane % 32, half lane / 32
         return Raw{*(const uint4*)(block + slot * 16), *(const uint32_t*)(block + 1024 + slot * 4)};
     }
-    static __device__ __forceinline__ Ready prepare(const Raw& r, const Row&) {
+    static __device__ __forceinline__ Ready prepare(const Raw& r, const Row& k) {
         const float s = __uint_as_float(r.qp << 16);
-        return Ready{{r.codes.x, r.codes.y, r.codes.z, r.codes.w}, s, -1032.0f * s, 0.0625f * s, -72.0f * s, __uint_as_float(r.qp & 0xffff0000u)};
+        return Ready{{r.codes.x, r.codes.y, r.codes.z, r.codes.w}, s, -1032.0f * s, 0.0625f * s, -72.0f * s, __uint_as_float(r.qp & 0xffff0000u), k};
     }
+    // (vector conversions: element by element, the compiler adds a permutation to each packed one)
+    static __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+        typedef float f32x2 __attribute__((ext_vector_type(2)));
+        typedef __bf16 b16x2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), b16x2));
+    }
+    // a zero low operand: the rounded value lands in the high half, where it is an fp32 again
+    static __device__ __forceinline__ float high_bf16(float f) { return __uint_as_float(pack_bf16(0.f, f)); }
     // Codes 2 d and 2 d + 1 of dword s as dequantize_affine rounds them: t = bf16((q - 8) * scale), w = bf16(t + zero).  The
     // pairs sit at bits (0, 16), (4, 20), (8, 24), (12, 28): masked and or'ed into the fp16 pair 1024 + q (1024 + 16 q for odd
     // pairs, whose factor goes into the scale), widened and scaled by one mixed fma each, exact in fp32.
     static __device__ __forceinline__ uint32_t piece(const Ready& r, int s, int d) {
         const uint32_t w = d < 2 ? r.w[s] : r.w[s] >> 8;
-        const uint32_t p = (w & (d & 1 ? 0x00F000F0u : 0x000F000Fu)) | 0x64006400u;
+        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+        const f16x2 p = __builtin_bit_cast(f16x2, (w & (d & 1 ? r.k.odd : r.k.even)) | r.k.one);
         const float sc = d & 1 ? r.s16 : r.s, c = d & 1 ? r.c16 : r.c;
-        float t0, t1;
-        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(t0) : "v"(p), "v"(sc), "v"(c));
-        asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(t1) : "v"(p), "v"(sc), "v"(c));
-        // a zero low operand: the rounded value lands in the high half, where it is an fp32 again
-        asm("v_cvt_pk_bf16_f32 %0, 0, %0" : "+v"(t0));
-        asm("v_cvt_pk_bf16_f32 %0, 0, %0" : "+v"(t1));
-        return hw_bf16_pack(t0 + r.z, t1 + r.z);
+        const float t0 = high_bf16(__builtin_fmaf((float)p.x, sc, c)), t1 = high_bf16(__builtin_fmaf((float)p.y, sc, c));
+        return pack_bf16(t0 + r.z, t1 + r.z);
     }
     static __device__ __forceinline__ tg_f32x16 mul(uint4 w, uint4 x, tg_f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), c, 0, 0, 0);

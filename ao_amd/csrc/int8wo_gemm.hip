@@ -26,8 +26,8 @@ struct Int8Tile {
         const int64_t rel = (n + row < a.N ? n + row : a.N - 1) - n0;   // rows past N repeat the last one
         return (uint32_t)(rel * a.ldw) + ((PAIR ? (lane & 7) ^ ((row >> 1) & 7) : (lane & 3) ^ ((row >> 2) & 3)) << 4);
     }
-    static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, uint32_t off) {
-        tg_dma(lds + r * 1024, a.w + n0 * a.ldw + (int64_t)s * 64, off);
+    static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, int at, uint32_t off) {
+        tg_dma(lds, at + r * 1024, a.w + n0 * a.ldw + (uint32_t)s * 64u, off);
     }
     static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) { return Row(); }
     static __device__ __forceinline__ Raw read(const uint8_t* block, int lane, bool odd) {

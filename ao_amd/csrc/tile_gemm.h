@@ -17,7 +17,11 @@
 // at 256 rows from 51 to 38 us; two groups along K (two waves per SIMD) took 64 x 128 tiles from 29 to 24 us.  A CU takes 125
 // bytes a nanosecond from its XCD's L2, but only 55 to 70 while the weights come from memory: requests return in order, so
 // those behind a weight wait with it.  More buffers than four change nothing then (six measured), and neither do wider
-// tiles for a wave (64 columns, half the LDS reads).
+// tiles for a wave (64 columns, half the LDS reads).  Every instruction of the loop counts, also the scalar ones and the
+// wait states: buffers named by their byte offset, 32-bit step offsets, the LDS address added into m0 by one instruction and
+// conversions that the compiler knows (in place of asm statements, behind which it places a wait state each) took the int4
+// loop of 96 x 128 tiles from 273 to 224 instructions and 5120 x 13824 at 427 rows from 96.3 to 89.6 us, 4096 x 14336 at 1254 rows
+// from 179 to 164; int8 and FP6 loops are 5 to 10 % shorter and 0 to 2 % faster.
 #pragma once
 #include "tile_order.h"
 #include <type_traits>
@@ -40,9 +44,10 @@ struct TileGemmArgs {
     float* parts;                       // K split over blockIdx.y: fp32 partial products [gridDim.y][M][N], or null
 };
 
-// 16 bytes per lane, global -> LDS: lane L of the wave lands at lds + 16 L.  Scalar base + 32-bit byte offset per lane.
-__device__ __forceinline__ void tg_dma(uint32_t lds, const void* base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+// 16 bytes per lane, global -> LDS: lane L of the wave lands at lds + at + 16 L, `at` a constant.  Scalar base + 32-bit byte
+// offset per lane.
+__device__ __forceinline__ void tg_dma(uint32_t lds, int at, const void* base, uint32_t off) {
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds), "i"(at) : "memory", "scc");
 }
 template <int N>
 __device__ __forceinline__ void tg_wait_barrier() {
@@ -51,15 +56,15 @@ __device__ __forceinline__ void tg_wait_barrier() {
 }
 
 // 4 bytes per lane
-__device__ __forceinline__ void tg_dma4(uint32_t lds, const void* base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+__device__ __forceinline__ void tg_dma4(uint32_t lds, int at, const void* base, uint32_t off) {
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds), "i"(at) : "memory", "scc");
 }
 
 // A weight format F describes a block of 32 weight rows of one 64-wide K step:
 //   REQ, BLOCK_BYTES      requests that bring it into LDS, and its bytes there
 //   PAIR                  whether two steps' worth is brought in at once (a row's 64 k are half a 128-byte line)
 //   lane_offset(a, n0, n, r, lane)   this lane's offset of request r from the tile's base, rows n ..
-//   request(a, n0, s, r, lds, off)   issues request r of step s for a block at `lds`
+//   request(a, n0, s, r, lds, at, off)   issues request r of step s for a block at `lds` + the constant `at`
 //   Raw read(block, lane, odd)       a lane's share: row lane % 32, the 32 k of half lane / 32 (PAIR: of the first or second step)
 //   Ready prepare(raw, row)          whatever is computed once per step
 //   Piece piece(ready, s, d)         two dequantized weights: dword d of the 8 k of slice s, up to
@@ -105,28 +110,27 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
 #pragma unroll
     for (int j = 0; j < BREQ; ++j) boff[j] = F::lane_offset(a, n0, n0 + (gw * NT + j / (UNIT * F::REQ)) * 32, j % (UNIT * F::REQ), lane);
     const uint16_t* const abase = a.x + m0 * a.ldx;
+    // Buffers are named by their byte offset within the ring: activations A_STEP apart, weights behind them
+    constexpr int A_STEP = PAIR ? ABYTES : STAGE, A_END = STAGES * A_STEP, B_STEP = 2 * BBYTES, B_END = 3 * B_STEP;   // (B_: PAIR)
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + group * RING;
+    const uint32_t lds_a = lds0 + gw * AREQ * 1024, lds_b = lds0 + (PAIR ? A_END : ABYTES) + gw * NT * UNIT * F::BLOCK_BYTES;
     // request r of step t: the activations' into `buf`, then the weights'; with PAIR first the weights of steps t .. t + 1, into pair
     // buffer `buf`, then the activations
     auto request = [&](int r, int t, int buf) __attribute__((always_inline)) {
+        const bool weights = PAIR ? r < BREQ : r >= AREQ;
+        const int i = PAIR == weights ? r : weights ? r - AREQ : r - BREQ;
         // (a request past the end repeats the last step's and is not used)
+        int s;
         if constexpr (PAIR) {
-            const bool weights = r < BREQ;
-            const int s = min(first + (t >> 1) * 2 * KW + 2 * group + (t & 1), max(min(first + KS, all) - (weights ? 2 : 1), 0));
-            if (weights)
-                F::request(a, n0, s, r % (2 * F::REQ),
-                           lds0 + STAGES * ABYTES + buf * 2 * BBYTES + (gw * NT + r / (2 * F::REQ)) * 2 * F::BLOCK_BYTES, boff[r]);
-            else
-                tg_dma(lds0 + buf * ABYTES + (gw * AREQ + r - BREQ) * 1024, abase + (int64_t)s * 64, aoff[r - BREQ]);
-            return;
+            s = min(first + (t >> 1) * 2 * KW + 2 * group + (t & 1), max(min(first + KS, all) - (weights ? 2 : 1), 0));
+        } else {
+            s = t * KW + group;
+            s = first + (s < KS ? s : KS - 1);
         }
-        int s = t * KW + group;
-        s = first + (s < KS ? s : KS - 1);
-        const uint32_t at = lds0 + buf * STAGE;
-        if (r < AREQ)
-            tg_dma(at + (gw * AREQ + r) * 1024, abase + (int64_t)s * 64, aoff[r]);
+        if (weights)
+            F::request(a, n0, s, i % (UNIT * F::REQ), lds_b + buf, i / (UNIT * F::REQ) * UNIT * F::BLOCK_BYTES, boff[i]);
         else
-            F::request(a, n0, s, (r - AREQ) % F::REQ, at + ABYTES + (gw * NT + (r - AREQ) / F::REQ) * F::BLOCK_BYTES, boff[r - AREQ]);
+            tg_dma(lds_a + buf, i * 1024, (const uint8_t*)abase + (uint32_t)s * 128u, aoff[i]);
     };
 
     tg_f32x16 acc[MT][NT];
@@ -158,18 +162,15 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
     for (int t = 0; t < STAGES - 1; ++t)
 #pragma unroll
         for (int r = 0; r < REQ; ++r) {
-            if (!PAIR || r >= BREQ) request(r, t, t);
-            else if (t < 2) request(r, 2 * t, t);
+            if (!PAIR || r >= BREQ) request(r, t, t * A_STEP);
+            else if (t < 2) request(r, 2 * t, t * B_STEP);
         }
-    auto a_at = [&](int buf) { return lds + group * RING + buf * (PAIR ? ABYTES : STAGE); };
-    // the weights of a step, or with PAIR of a pair, in buffer `buf`
-    auto b_at = [&](int buf, int j) {
-        if constexpr (PAIR) return lds + group * RING + STAGES * ABYTES + buf * 2 * BBYTES + (gw * NT + j) * 2 * F::BLOCK_BYTES;
-        else return lds + group * RING + buf * STAGE + ABYTES + (gw * NT + j) * F::BLOCK_BYTES;
-    };
-    auto read_a = [&](const uint8_t* A, int i, int s) __attribute__((always_inline)) {
-        return *(const uint4*)(A + (i * 32 + r32) * 128 + (((4 * half + s) ^ ((r32 >> 1) & 7)) << 4));
-    };
+    // this lane's weights of a step (with PAIR of a pair) in buffer `buf`, its activation fragment of slice s
+    auto b_at = [&](int buf, int j) { return lds + group * RING + (PAIR ? A_END : ABYTES) + buf + (gw * NT + j) * UNIT * F::BLOCK_BYTES; };
+    int a_lane[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) a_lane[s] = group * RING + r32 * 128 + (((4 * half + s) ^ ((r32 >> 1) & 7)) << 4);
+    auto read_a = [&](int buf, int i, int s) __attribute__((always_inline)) { return *(const uint4*)(lds + (a_lane[s] + buf) + i * 4096); };
     union Frag { uint32_t u[4]; uint4 q; };
     Frag fa[2][MT], fb[2][NT];
     typename F::Raw raw[NT];
@@ -178,20 +179,20 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
 #pragma unroll
     for (int j = 0; j < NT; ++j) ready[j] = F::prepare(F::read(b_at(0, j), lane, false), row_const[j]);
 #pragma unroll
-    for (int i = 0; i < MT; ++i) fa[0][i].q = read_a(a_at(0), i, 0);
+    for (int i = 0; i < MT; ++i) fa[0][i].q = read_a(0, i, 0);
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int d = 0; d < 4; ++d) fb[0][j].u[d] = F::pack(F::piece(ready[j], 0, d));
-    int buf = 0, pair = 0;   // this step's buffer, its pair's
+    int prev = A_END - A_STEP, buf = 0, pair = 0;   // the buffer of the step before, this step's, its pair's
     // (a group that has one step less runs one less; a test around every matrix instruction of that step cost 2 to 5 %)
     const int own = PAIR ? KS / (2 * KW) * 2 + min(max(KS % (2 * KW) - 2 * group, 0), 2) : (KS - group + KW - 1) / KW;
     auto step = [&](int t, auto odd) __attribute__((always_inline)) {
         constexpr bool ODD = decltype(odd)::value;   // of PAIR's two steps
         constexpr int NREQ = PAIR && ODD ? AREQ : REQ;
-        const int next = buf + 1 == STAGES ? 0 : buf + 1, ahead = buf == 0 ? STAGES - 1 : buf - 1;
-        const int pair_ahead = pair == 0 ? 2 : pair - 1;
-        if (PAIR && ODD) pair = pair == 2 ? 0 : pair + 1;   // (from here on the next step's)
+        const int next = buf + A_STEP == A_END ? 0 : buf + A_STEP;
+        const int pair_prev = pair == 0 ? B_END - B_STEP : pair - B_STEP;
+        if (PAIR && ODD) pair = pair + B_STEP == B_END ? 0 : pair + B_STEP;   // (from here on the next step's)
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const int cur = s & 1, nxt = cur ^ 1;
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
             for (int q = 0; q < SLOTS; ++q) {
                 const int i = q % MT, j = q / MT;
                 acc[i][j] = F::mul(fb[cur][j].q, fa[cur][i].q, acc[i][j]);
-                if (q < MT) fa[nxt][q].q = s < 3 ? read_a(a_at(buf), q, s + 1) : read_a(a_at(next), q, 0);
+                if (q < MT) fa[nxt][q].q = s < 3 ? read_a(buf, q, s + 1) : read_a(next, q, 0);
                 if (s == 3 && q == 1)
 #pragma unroll
                     for (int j2 = 0; j2 < NT; ++j2) ready[j2] = F::prepare(raw[j2], row_const[j2]);
@@ -220,12 +221,13 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
                 if (s < 2)
 #pragma unroll
                     for (int r = (s * SLOTS + q) * NREQ / (2 * SLOTS); r < (s * SLOTS + q + 1) * NREQ / (2 * SLOTS); ++r) {
-                        if (PAIR && !ODD && r < BREQ) request(r, t + 4, pair_ahead);
-                        else request(PAIR && ODD ? r + BREQ : r, t + STAGES - 1, ahead);
+                        if (PAIR && !ODD && r < BREQ) request(r, t + 4, pair_prev);
+                        else request(PAIR && ODD ? r + BREQ : r, t + STAGES - 1, prev);
                     }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        prev = buf;
         buf = next;
     };
     if constexpr (PAIR) {
