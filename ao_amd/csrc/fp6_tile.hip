@@ -32,7 +32,7 @@ struct Fp6Tile {
     }
     static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, int at, uint32_t off) {
         const uint8_t* const tile = a.w + (n0 / 16) * a.ldw + (uint32_t)((s >> 1) * 1536 + (s & 1) * (r == 0 ? 512 : 256));
-        tg_dma(lds, at + r * 1024, tile, off + (r == 0 ? 0 : 1024));
+        tg_dma(lds, at, tile, off + (r == 0 ? 0 : 1024));
     }
     static __device__ __forceinline__ Row row(const TileGemmArgs& a, int64_t n) {
         const _Float16 s = __builtin_bit_cast(_Float16, ((const uint16_t*)a.scale)[n < a.N ? n : a.N - 1]);
@@ -67,7 +67,7 @@ static const TileShape kFp6Shapes[] = {
     {64, 128, 24.6, 0.0},    // two groups
     {96, 128, 30.5, 0.0},    // two groups
     {128, 128, 35.9, 0.0},   // two groups
-    {192, 128, 49.8, 0.0},
+    {192, 128, 47.7, 0.0},   // eight waves of 96 x 32
     {128, 256, 62.0, 0.0},   // 128 x 64 a wave
     {192, 256, 87.0, 0.0},   // eight waves
 };
@@ -81,7 +81,7 @@ static void launch_shape(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
         case 1: tile_launch<F, 4, 2, 2, 1>(a, p.parts, st); break;
         case 2: tile_launch<F, 4, 2, 3, 1>(a, p.parts, st); break;
         case 3: tile_launch<F, 4, 2, 4, 1>(a, p.parts, st); break;
-        case 4: tile_launch<F, 4, 1, 6, 1>(a, p.parts, st); break;
+        case 4: tile_launch<F, 4, 1, 3, 1, 2>(a, p.parts, st); break;
         case 5: tile_launch<F, 4, 1, 4, 2>(a, p.parts, st); break;
         default: tile_launch<F, 8, 1, 6, 1>(a, p.parts, st); break;
     }

@@ -38,7 +38,7 @@ struct Int4Tile {
         if (r == 0)
             tg_dma(lds, at, a.w + (n0 / 16) * a.ldw + (uint32_t)s * 512u, off);
         else
-            tg_dma4(lds, at + 1024, (const uint8_t*)a.scale + (n0 / 16) * (padded_k(a) >> a.group_shift) * 64 + (((uint32_t)s * 64u) >> a.group_shift) * 64u, off);
+            tg_dma4(lds, at, (const uint8_t*)a.scale + (n0 / 16) * (padded_k(a) >> a.group_shift) * 64 + (((uint32_t)s * 64u) >> a.group_shift) * 64u, off);
     }
     static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) {
         Row k;   // in registers, so that one instruction masks and inserts

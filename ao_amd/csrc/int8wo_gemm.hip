@@ -27,7 +27,7 @@ struct Int8Tile {
         return (uint32_t)(rel * a.ldw) + ((PAIR ? (lane & 7) ^ ((row >> 1) & 7) : (lane & 3) ^ ((row >> 2) & 3)) << 4);
     }
     static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, int at, uint32_t off) {
-        tg_dma(lds, at + r * 1024, a.w + n0 * a.ldw + (uint32_t)s * 64u, off);
+        tg_dma(lds, at, a.w + n0 * a.ldw + (uint32_t)s * 64u, off);
     }
     static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) { return Row(); }
     static __device__ __forceinline__ Raw read(const uint8_t* block, int lane, bool odd) {
@@ -91,7 +91,7 @@ static const TileShape kInt8Shapes[] = {
     {64, 128, 26.4, 0.0},    // two groups of 4 waves along K
     {96, 128, 32.0, 52.7},
     {128, 128, 35.2, 0.0},   // two groups; 14336 of K 115 us, one group of four waves 122
-    {192, 128, 47.4, 0.0},
+    {192, 128, 44.4, 0.0},   // eight waves of 96 x 32
     {128, 256, 57.0, 0.0},   // eight waves; four of 128 x 64 each are 7 % slower
     {64, 64, 20.0, 0.0},     // four groups along K
     {192, 256, 77.8, 0.0},   // eight waves
@@ -121,7 +121,7 @@ void launch_int8wo_gemm(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
         switch (p.shape) {
             case 1: tile_launch<Int8Tile<false>, 4, 1, 3, 1>(a, p.parts, st); break;
             case 2: tile_launch<Int8Tile<false>, 4, 2, 4, 1>(a, p.parts, st); break;
-            case 3: tile_launch<Int8Tile<false>, 4, 1, 6, 1>(a, p.parts, st); break;
+            case 3: tile_launch<Int8Tile<false>, 4, 1, 3, 1, 2>(a, p.parts, st); break;
             case 5: tile_launch<Int8Tile<false>, 2, 4, 2, 1>(a, p.parts, st); break;
             default: tile_launch<Int8Tile<false>, 8, 1, 6, 1>(a, p.parts, st); break;
         }

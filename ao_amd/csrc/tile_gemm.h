@@ -1,7 +1,10 @@
 // Tiled product y[M,N] = x[M,K] @ dequant(W[N,K])^T for batches beyond the streaming kernels, generic over the weight format.
 //
-// A workgroup of WN x KW waves computes a tile of 32 MT activation rows x 32 NT WN weight rows; a wave owns MT x NT blocks of
-// 32x32x16 matrix instructions over all rows of the tile, so every weight is dequantized once per tile, and with KW > 1 the
+// A workgroup of WM x WN x KW waves computes a tile of 32 MT WM activation rows x 32 NT WN weight rows; a wave owns MT x NT blocks of
+// 32x32x16 matrix instructions.  With WM = 1 it has all rows of the tile, so every weight is dequantized once per tile.  192 x 128
+// tiles of int8 and FP6, whose dequantization is short, have WM = 2: twice the conversions, but two waves on a SIMD (int8
+// 192 rows, 14336 x 4096 46.0 -> 42.7 us, 333 rows 11008 x 4096 44.5 -> 42.1; FP6 40.6 -> 38.9, 41.7 -> 40.8; int4 45.9 -> 57.8, so not there.
+// 256 x 128, 192 x 256 and 256 x 256 tiles of that kind were no faster than what they would replace).  With KW > 1 the
 // groups of WN waves take the 64-wide K steps round-robin and add their accumulators through LDS at the end.  Both
 // operands of a step come into LDS by direct loads (no registers, no LDS store instructions) through a ring of STAGES
 // buffers with one barrier per step.  Weights are stored in LDS as they are in memory and dequantized by the wave that
@@ -64,30 +67,30 @@ __device__ __forceinline__ void tg_dma4(uint32_t lds, int at, const void* base, 
 //   REQ, BLOCK_BYTES      requests that bring it into LDS, and its bytes there
 //   PAIR                  whether two steps' worth is brought in at once (a row's 64 k are half a 128-byte line)
 //   lane_offset(a, n0, n, r, lane)   this lane's offset of request r from the tile's base, rows n ..
-//   request(a, n0, s, r, lds, at, off)   issues request r of step s for a block at `lds` + the constant `at`
+//   request(a, n0, s, r, lds, at, off)   issues request r of step s, which lands at `lds` + the constant `at`
 //   Raw read(block, lane, odd)       a lane's share: row lane % 32, the 32 k of half lane / 32 (PAIR: of the first or second step)
 //   Ready prepare(raw, row)          whatever is computed once per step
 //   Piece piece(ready, s, d)         two dequantized weights: dword d of the 8 k of slice s, up to
 //   uint32_t pack(piece)             the work left for the end of the slice
 //   mul, columns, finish, combine    the matrix instruction and the epilogue
-template <class F, int WN, int KW, int MT, int NT>
-__global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmArgs a) {
-    constexpr int G = WN, BM = 32 * MT, BN = 32 * NT * WN;
+template <class F, int WN, int KW, int MT, int NT, int WM>
+__global__ __launch_bounds__(64 * WM * WN * KW) void tile_gemm_kernel(const TileGemmArgs a) {
+    constexpr int G = WM * WN, BM = 32 * MT * WM, BN = 32 * NT * WN;
     constexpr bool PAIR = F::PAIR;
     constexpr int ABYTES = BM * 128, BBYTES = WN * NT * F::BLOCK_BYTES, STAGE = ABYTES + BBYTES;
     constexpr int STAGES = KW * 4 * STAGE <= 160 * 1024 ? 4 : 3;
     // with PAIR the weights have a ring of their own, of three pairs of steps
     constexpr int RING = PAIR ? STAGES * ABYTES + 6 * BBYTES : STAGES * STAGE;
     static_assert(!PAIR || KW * RING <= 160 * 1024, "LDS of a CU");
-    constexpr int AREQ = ABYTES / 1024 / G, BREQ = NT * F::REQ * (PAIR ? 2 : 1), REQ = AREQ + BREQ;
-    static_assert(AREQ * G * 1024 == ABYTES, "every wave issues the same number of requests");
+    constexpr int AREQ = ABYTES / 1024 / G, WREQ = F::REQ * (PAIR ? 2 : 1), BREQ = NT * WREQ / WM, REQ = AREQ + BREQ;
+    static_assert(AREQ * G * 1024 == ABYTES && BREQ * WM == NT * WREQ && (NT % WM == 0 || NT == 1), "every wave issues the same number of requests");
     constexpr int ACC = MT * NT * 4096;   // bytes of one wave's accumulators
     constexpr int LDS = KW * RING > (KW - 1) * G * ACC ? KW * RING : (KW - 1) * G * ACC;
     __shared__ __align__(1024) uint8_t lds[LDS];
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int group = wave / G, gw = wave % G;
+    const int group = wave / G, gw = wave % G, wn = gw % WN, wm = WM == 1 ? 0 : gw / WN;
     int tile_m, tile_n;
     if (!tile_at(a.order, (int)blockIdx.x, tile_m, tile_n)) return;
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
@@ -108,12 +111,16 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
         aoff[j] = (uint32_t)(rel * a.ldx * 2) + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
     }
 #pragma unroll
-    for (int j = 0; j < BREQ; ++j) boff[j] = F::lane_offset(a, n0, n0 + (gw * NT + j / (UNIT * F::REQ)) * 32, j % (UNIT * F::REQ), lane);
+    for (int j = 0; j < BREQ; ++j) {
+        const int r = wm * BREQ + j;   // of the NT x WREQ requests of its columns, which WM waves share
+        boff[j] = F::lane_offset(a, n0, n0 + (wn * NT + r / WREQ) * 32, r % WREQ, lane);
+    }
     const uint16_t* const abase = a.x + m0 * a.ldx;
     // Buffers are named by their byte offset within the ring: activations A_STEP apart, weights behind them
     constexpr int A_STEP = PAIR ? ABYTES : STAGE, A_END = STAGES * A_STEP, B_STEP = 2 * BBYTES, B_END = 3 * B_STEP;   // (B_: PAIR)
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds + group * RING;
-    const uint32_t lds_a = lds0 + gw * AREQ * 1024, lds_b = lds0 + (PAIR ? A_END : ABYTES) + gw * NT * UNIT * F::BLOCK_BYTES;
+    const uint32_t lds_a = lds0 + gw * AREQ * 1024, lds_b = lds0 + (PAIR ? A_END : ABYTES) + wn * NT * UNIT * F::BLOCK_BYTES +
+                   wm * (NT % WM == 0 ? NT / WM * UNIT * F::BLOCK_BYTES : BREQ * 1024);
     // request r of step t: the activations' into `buf`, then the weights'; with PAIR first the weights of steps t .. t + 1, into pair
     // buffer `buf`, then the activations
     auto request = [&](int r, int t, int buf) __attribute__((always_inline)) {
@@ -128,7 +135,7 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
             s = first + (s < KS ? s : KS - 1);
         }
         if (weights)
-            F::request(a, n0, s, i % (UNIT * F::REQ), lds_b + buf, i / (UNIT * F::REQ) * UNIT * F::BLOCK_BYTES, boff[i]);
+            F::request(a, n0, s, NT % WM == 0 ? i % WREQ : wm * BREQ + i, lds_b + buf, i / WREQ * UNIT * F::BLOCK_BYTES + i % WREQ * 1024, boff[i]);
         else
             tg_dma(lds_a + buf, i * 1024, (const uint8_t*)abase + (uint32_t)s * 128u, aoff[i]);
     };
@@ -143,7 +150,7 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
     const int r32 = lane & 31, half = lane >> 5;
     typename F::Row row_const[NT];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) row_const[j] = F::row(a, n0 + (gw * NT + j) * 32 + r32);
+    for (int j = 0; j < NT; ++j) row_const[j] = F::row(a, n0 + (wn * NT + j) * 32 + r32);
 
     // Steps 0 .. STAGES - 2 are requested; from then on step t multiplies buffer t and requests step t + STAGES - 1 into the buffer
     // that step t - 1 has left.  The step's barrier stands in front of its last slice, where every wave has read what it needs of
@@ -166,10 +173,10 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
             else if (t < 2) request(r, 2 * t, t * B_STEP);
         }
     // this lane's weights of a step (with PAIR of a pair) in buffer `buf`, its activation fragment of slice s
-    auto b_at = [&](int buf, int j) { return lds + group * RING + (PAIR ? A_END : ABYTES) + buf + (gw * NT + j) * UNIT * F::BLOCK_BYTES; };
+    auto b_at = [&](int buf, int j) { return lds + group * RING + (PAIR ? A_END : ABYTES) + buf + (wn * NT + j) * UNIT * F::BLOCK_BYTES; };
     int a_lane[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) a_lane[s] = group * RING + r32 * 128 + (((4 * half + s) ^ ((r32 >> 1) & 7)) << 4);
+    for (int s = 0; s < 4; ++s) a_lane[s] = group * RING + wm * MT * 4096 + r32 * 128 + (((4 * half + s) ^ ((r32 >> 1) & 7)) << 4);
     auto read_a = [&](int buf, int i, int s) __attribute__((always_inline)) { return *(const uint4*)(lds + (a_lane[s] + buf) + i * 4096); };
     union Frag { uint32_t u[4]; uint4 q; };
     Frag fa[2][MT], fb[2][NT];
@@ -274,11 +281,11 @@ __global__ __launch_bounds__(64 * WN * KW) void tile_gemm_kernel(const TileGemmA
     for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int e = 0; e < 16; e += 4) {
-            const int64_t n = n0 + (gw * NT + j) * 32 + 8 * (e >> 2) + 4 * half;
+            const int64_t n = n0 + (wn * NT + j) * 32 + 8 * (e >> 2) + 4 * half;
             const typename F::Cols cols = F::columns(a, n);
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                const int64_t m = m0 + i * 32 + r32;
+                const int64_t m = m0 + (wm * MT + i) * 32 + r32;
                 if (m >= a.M) continue;
                 if (a.parts) {
                     float* dst = a.parts + ((int64_t)blockIdx.y * a.M + m) * a.N + n;
@@ -377,11 +384,11 @@ inline void tile_grid(TileGemmArgs& a, const TileShape& s, int row_bytes, int pa
     a.order = tile_order((a.M + s.bm - 1) / s.bm, (a.N + s.bn - 1) / s.bn, s.bm * 128, s.bn * row_bytes);
     if (parts == 1) a.parts = nullptr;
 }
-template <class F, int WN, int KW, int MT, int NT>
+template <class F, int WN, int KW, int MT, int NT, int WM = 1>
 void tile_launch(const TileGemmArgs& a, int parts, hipStream_t st) {
     hipEvent_t ev0 = g_prof_start, ev1 = g_prof_stop;
     g_prof_start = g_prof_stop = nullptr;
-    hipExtLaunchKernelGGL((tile_gemm_kernel<F, WN, KW, MT, NT>), dim3((unsigned)(a.order.per_xcd() * 8), (unsigned)parts), dim3(64 * WN * KW), 0, st,
+    hipExtLaunchKernelGGL((tile_gemm_kernel<F, WN, KW, MT, NT, WM>), dim3((unsigned)(a.order.per_xcd() * 8), (unsigned)parts), dim3(64 * WM * WN * KW), 0, st,
                           ev0, ev1, 0, a);
 }
 template <class F>
