@@ -99,8 +99,9 @@ static TilePlan fp6_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
 // 57 / 35, 97 / 74, 169 / 120; 4096 x 4096 at 128 / 384 / 1000 rows 12.3 / 15.0, 27 / 21, 50 / 39; 5120 x 5120 at 96 / 384 rows 14.4 /
 // 18.0, 34 / 32; 1024 x 4096 at 512 / 640 rows 12.6 / 15.4, 17.8 / 16.8.  Up to 64 rows the streaming kernels and small tiles
 // hold on for weights of up to 25 M (6144 x 4096 at 48 rows 12.1 / 12.7; 5120 x 5120 14.1 / 13.2; 14336 x 4096 at 33 / 48 rows 18.8 / 15.5,
-// 19.2 / 16.1; 13824 x 5120 at 48 rows 22.3 / 20.0), from 49 rows on for all but the largest (28672 x 8192; the others' routes and
-// workspaces there stand as they were: 14336 x 4096 at 64 rows 19.4 / 17.0).  Where they split K over workgroups (fp6.hip:
+// 19.2 / 16.1; 13824 x 5120 at 48 rows 22.3 / 20.0; at 52 rows 14336 x 4096 19.7 / 14.7, 13824 x 5120 23.6 / 17.0, 5120 x 5120 15.4 / 13.9), at
+// 64 rows for all but the largest (13824 x 5120 24.0 / 18.8; the routes of others are what callers there know: 14336 x 4096 20.0 / 14.8).
+// Where they split K over workgroups (fp6.hip:
 // fp6_ws_parts) they are kept but for 65 to 96 rows of weights from 50 M on (4096 x 14336 at 64 / 66 / 96 rows 20.9 / 20.9, 31.0 / 22.2, 32.3 / 24.1;
 // 4096 x 4096 at 66 rows 11.9 / 13.4).
 static bool fp6_tiled(int64_t M, int64_t N, int64_t K) {
@@ -110,7 +111,7 @@ static bool fp6_tiled(int64_t M, int64_t N, int64_t K) {
     // streamed once per 16 rows there (14336 x 4032 at 33 / 128 / 1000 rows 22 / 50 / 305 us, tiled 20 / 24 / 119; 4096 x 4160 at 65 / 128 /
     // 1000 rows 14 / 17 / 96, tiled 16 / 16 / 41)
     if (K % 128 != 0) return tile_us < 5.0 + 8.5e-8 * (double)(N * K) * (double)((M + 15) / 16);
-    if (M <= 64) return N * K >= (M <= 48 ? (int64_t)26000000 : (int64_t)1 << 27);
+    if (M <= 64) return N * K >= (M < 64 ? (int64_t)26000000 : (int64_t)60000000);
     // (the 128 x 128 tiles of fp6.hip were never ahead there: 14336 x 4096 at 1200 / 1500 rows 169 / 178 tiled)
     if (M >= 1024 && N >= 2048) return true;
     const int64_t big = (N + 127) / 128 * ((M + 127) / 128), mid = (N + 63) / 64 * ((M + 63) / 64), small = (N + 63) / 64 * ((M + 31) / 32);

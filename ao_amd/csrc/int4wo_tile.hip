@@ -87,22 +87,27 @@ struct Int4Tile {
     static __device__ __forceinline__ void combine(const TileGemmArgs&, int64_t, int64_t, uint16_t (&)[4]) {}
 };
 
-// us at K = 4096, 192 to 256 workgroups (14336, 6144 and 4096 columns)
+// us at K = 4096, fitted to 128 calls (36 to 2000 rows of eight weights from 1024 x 4096 to 28672 x 8192), every shape and number of parts
+// timed: the choice is within 0.7 % of the fastest on average (1.2 % with the costs from before the loops were shortened: 100 rows of
+// 14336 x 4096 28.1 -> 25.9 us, 128 of 13824 x 5120 34.0 -> 30.8, 333 of 5120 x 5120 39.7 -> 31.3, 1400 of 6144 x 4096 99 -> 90).  Sums of parts
+// cost more than a call alone shows: 1000 rows of 4096 x 14336 take 127 us on 256 x 256 tiles in four parts, 126 on 128 x 128 tiles and 141 on
+// 256 x 128 in two, but within a prompt the four parts are 2 to 3 % of the pass slower than either.
 static const TileShape kInt4Shapes[] = {
-    {64, 64, 19.4, 0.0},     // four groups along K
-    {64, 128, 31.0, 0.0},    // two groups
-    {96, 128, 36.4, 0.0},    // two groups
-    {128, 128, 41.8, 0.0},   // two groups
-    {192, 128, 57.0, 0.0},
-    {256, 128, 66.0, 0.0},
+    {64, 64, 17.9, 0.0},     // four groups along K
+    {64, 128, 31.2, 0.0},    // two groups
+    {96, 128, 34.5, 0.0},    // two groups
+    {128, 128, 36.9, 0.0},   // two groups
+    {192, 128, 55.2, 0.0},
+    {256, 128, 68.0, 0.0},
     // the kernels of int4wo_gemm.hip, which have no K parts of their own: in_features of the packed width only
-    {256, 128, 64.0, 0.0, 4},
-    {256, 256, 104.0, 0.0, 4},
+    {256, 128, 59.0, 120.0, 4},
+    {256, 256, 96.2, 0.0, 4},
 };
+static constexpr TilePartCost kInt4Parts{0.5, 0.5, 7.2};
 static constexpr int kInt4Own = 6, kInt4All = 8;
 
 static TilePlan int4wo_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
-    return tile_plan(kInt4Shapes, K % 256 == 0 && M >= 128 ? kInt4All : kInt4Own, M, N, K, max_parts);
+    return tile_plan(kInt4Shapes, K % 256 == 0 && M >= 128 ? kInt4All : kInt4Own, M, N, K, max_parts, kInt4Parts);
 }
 
 // us of the kernel that ao_amd_int4wo_linear(_ws) runs, by measurement at 33 to 1000 rows on 16 weights from 768 x 1024 to 28672 x
@@ -116,13 +121,15 @@ static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
     if (kernel == Int4Kernel::lds_256x256 || kernel == Int4Kernel::lds_256x128) {
         const double rw = rounds(256, 256);
         if (kernel == Int4Kernel::lds_256x256) return 6.0 + 100.0 * k * (rw < 1.0 ? 0.4 + 0.6 * rw : up(rw));   // CUs that run at once slow each other down
-        const double r = rounds(256, 128), full = (double)(int64_t)r, rest = r - full;
-        return 14.0 + k * (52.5 * full + (rest == 0.0 ? 0.0 : full > 0.0 && rest <= 0.5 ? 28.0 : 52.5));
+        // (1400 / 2000 rows of 4096 x 14336 230 / 247 us, tiled 186 / 217)
+        const double r = rounds(256, 128), full = (double)(int64_t)r, rest = r - full, round = K > 8192 ? 62.0 : 52.5;
+        return 14.0 + k * (round * full + (rest == 0.0 ? 0.0 : full > 0.0 && rest <= 0.5 ? 28.0 : round));
     }
     if (kernel == Int4Kernel::kwave) {
         const double r = up(rounds(128, 64));
         const bool three = (M + 95) / 96 == (M + 127) / 128;   // its 96-row tiles
-        return 6.0 + (three ? (r > 1.0 ? 17.5 : 16.5) : r > 1.0 ? 20.0 : 18.5) * k * r;
+        // (one round over 14336 of K: 427 / 512 rows of 4096 x 14336 80 / 78 us, tiled 70 / 73)
+        return 6.0 + (three ? (r > 1.0 ? 17.5 : 16.5) : r > 1.0 || K >= 8192 ? 20.5 : 18.5) * k * r;
     }
     if (ao_amd_int4wo_linear_ws_parts(M, K, N, g) > 1) return M <= 64 ? 0.0 : 4.0 + 8.0 * k;
     if (kernel == Int4Kernel::tiles_128x128) return 90.0 * k * rounds(128, 128) / 2.0;
@@ -139,7 +146,13 @@ static bool int4wo_tiled(int64_t M, int64_t N, int64_t K, int64_t g) {
     // in_features that were padded to whole tiles of the packed layout: the others take activations copied to that width first
     const int64_t Kp = round_up(K, g > 128 ? g : 128);
     const double other = int4wo_other_us(M, N, Kp, g);
-    return other > 0.0 && int4wo_tile_plan(M, N, K, 8).us < (Kp == K ? 0.95 * other : other + 4.0);
+    const TilePlan plan = int4wo_tile_plan(M, N, K, 8);
+    Int4Kernel kernel;
+    // (the plan may be the very launch that the dispatch makes)
+    if (plan.shape >= kInt4Own && plan.parts == 1 && int4wo_plain_kernel(M, Kp, N, g, &kernel) &&
+        kernel == (plan.shape == kInt4Own ? Int4Kernel::lds_256x128 : Int4Kernel::lds_256x256))
+        return false;
+    return other > 0.0 && plan.us < (Kp == K ? 0.95 * other : other + 4.0);
 }
 
 // x [M, K] with row stride ldx -> y [M, Kp], zeros beyond K, 8 elements a thread: activations whose rows are not 16-byte aligned

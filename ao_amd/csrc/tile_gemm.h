@@ -348,7 +348,7 @@ __global__ __launch_bounds__(256) void tile_finish_kernel(const TileGemmArgs a, 
 
 // Tile shape and K parts for M x N x K: the cheapest by a measured model.  A shape costs `one` us for a wave of workgroups
 // over 4096 of K with one workgroup on a CU and `two` with two (0: only one fits), 6 us of it whatever K is; K parts add a
-// second launch, 1 us with each doubling and 8 bytes of fp32 per output and part.
+// second launch, something with each doubling and the traffic of their fp32 sums (TilePartCost: us, us, us for four million sums).
 struct TileShape {
     int bm, bn;
     double one, two;
@@ -358,21 +358,30 @@ struct TilePlan {
     int shape, parts;
     double us;
 };
-inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64_t N, int64_t K, int max_parts) {
+struct TilePartCost {
+    double launch = 1.5, doubling = 1.0, sums = 8.0;
+};
+// us of one shape with K in `z` parts
+inline double tile_us(const TileShape& s, int64_t M, int64_t N, int64_t K, int z, const TilePartCost& c = TilePartCost()) {
+    const int64_t per = (K / 64 + z - 1) / z, wgs = (M + s.bm - 1) / s.bm * ((N + s.bn - 1) / s.bn) * z;
+    const int64_t fit = s.two > 0 ? 512 : 256, full = wgs / fit, rest = wgs % fit;
+    auto us = [&](double t) { return 6.0 + (t - 6.0) * (double)per / 64.0; };
+    const double one = us(s.one), wave = s.two > 0 ? us(s.two) : one;
+    // (CUs that read a large weight at once share the memory: 120 workgroups take 0.7 to 0.97 of the time of 224)
+    const double alone = full == 0 && rest < 256 && N * K >= ((int64_t)1 << 25) ? 0.85 + 0.15 * (double)rest / 256.0 : 1.0;
+    // (the first CU with two workgroups sets the time, and the more there are the more they slow each other down)
+    const double t = full * wave + (rest == 0 ? 0.0 : rest <= 256 ? one * alone : one + (wave - one) * (0.4 + 0.6 * (double)(rest - 256) / 256.0));
+    return z == 1 ? t : t + c.launch + (z == 2 ? 1.0 : z == 4 ? 2.0 : 3.0) * c.doubling + c.sums * 1e-6 * (double)(M * N * z) / 4.0;
+}
+inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64_t N, int64_t K, int max_parts,
+                          const TilePartCost& c = TilePartCost()) {
     TilePlan best{-1, 1, 1e30};
     const int64_t steps = K / 64;
     for (int i = 0; i < nshapes; ++i)
         for (int z = 1; z <= (max_parts < shapes[i].max_parts ? max_parts : shapes[i].max_parts); z *= 2) {
             const int64_t per = (steps + z - 1) / z;
             if (z > 1 && (per < 8 || (z - 1) * per >= steps)) break;
-            const int64_t wgs = (M + shapes[i].bm - 1) / shapes[i].bm * ((N + shapes[i].bn - 1) / shapes[i].bn) * z;
-            const int64_t fit = shapes[i].two > 0 ? 512 : 256, full = wgs / fit, rest = wgs % fit;
-            auto us = [&](double t) { return 6.0 + (t - 6.0) * (double)per / 64.0; };
-            const double wave = us(shapes[i].two > 0 ? shapes[i].two : shapes[i].one);
-            // (CUs that read a large weight at once share the memory: 120 workgroups take 0.7 to 0.97 of the time of 224)
-            const double alone = full == 0 && rest < 256 && N * K >= ((int64_t)1 << 25) ? 0.85 + 0.15 * (double)rest / 256.0 : 1.0;
-            double t = full * wave + (rest == 0 ? 0.0 : rest <= 256 ? us(shapes[i].one) * alone : wave);
-            if (z > 1) t += 1.5 + (z == 2 ? 1.0 : z == 4 ? 2.0 : 3.0) + 8e-6 * (double)(M * N * z) / 4.0;
+            const double t = tile_us(shapes[i], M, N, K, z, c);
             if (t < best.us) best = TilePlan{i, z, t};
         }
     return best;

@@ -158,7 +158,8 @@ def test_fp6_tiles_cover_every_shape_and_the_operator_takes_them():
 
 
 @pytest.mark.parametrize("M,N,K,tiled", [
-    (32, 14336, 2048, False), (33, 14336, 2048, True), (48, 14336, 2048, True), (49, 14336, 2048, False), (48, 8192, 2048, False),
+    (32, 14336, 2048, False), (33, 14336, 2048, True), (48, 14336, 2048, True), (63, 14336, 2048, True), (64, 14336, 2048, False),
+    (64, 14336, 4224, True), (48, 8192, 2048, False),
     (64, 4096, 14336, False), (65, 4096, 14336, True), (96, 4096, 14336, True), (97, 4096, 14336, False), (80, 4096, 8192, False),
 ])
 def test_fp6_tiles_at_33_to_96_rows(M, N, K, tiled):
