@@ -236,7 +236,8 @@ int ao_amd_hqq_mixed_mm(const void* a, int64_t M, int64_t K, int64_t lda, const 
  * exactly as ao_amd_hqq_dequantize rounds it; fp32 accumulation; y in `dtype`, contiguous.  a: `dtype`, row stride lda
  * a multiple of 8 elements, 16-byte aligned like the packed codes, scales and zeros.  The reduction is cut into slices
  * whose fp32 partial sums go through `workspace` (ao_amd_hqq_mixed_mm_mfma_workspace gives its size; caller-owned,
- * device memory, 16-byte aligned).  More than 64 rows take ao_amd_hqq_dequantize and a library GEMM. */
+ * device memory, 16-byte aligned).  More than 64 rows take ao_amd_hqq_mixed_mm_tiled, or
+ * ao_amd_hqq_dequantize and a library GEMM. */
 int ao_amd_hqq_mixed_mm_mfma_workspace(int64_t M, int64_t K, int64_t N, int transposed, int64_t* bytes);
 int ao_amd_hqq_mixed_mm_mfma(const void* a, int64_t M, int64_t lda, const void* packed_2xint4, int is_signed, int64_t K,
                              int64_t N, const void* scales, const void* zeros, int64_t group_size, int dtype,
