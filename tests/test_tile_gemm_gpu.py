@@ -71,6 +71,17 @@ def test_int8_weights_in_pairs_of_steps(case, plan):
     _run(*case)   # (the bound of _run: at most 9088 exact products a sum)
 
 
+# two waves share a column block, each with 96 rows: the second one with one, two or all of its rows, K shorter than the ring of
+# buffers and just past it, columns that end within a block
+@pytest.mark.parametrize("M,N,K", [(290, 14336, 64), (289, 14290, 128), (380, 11008, 320), (384, 14290, 192), (300, 14336, 1088)])
+def test_tiles_of_two_waves_a_column_block(M, N, K):
+    assert _plan(M, N, K) == "tile 192x128 parts=1"
+    _run(M, N, K)
+    N = N // 64 * 64
+    assert _tiled_plan("fp6", M, N, K) == "tile 192x128 parts=1"
+    _fp6_tiles(M, N, K, 3, 2)
+
+
 @pytest.mark.parametrize("case", [(65, 5121, 6528), (257, 21000, 1024), (129, 1100, 4096)])
 def test_int8_tiles_bias_and_row_stride(case):
     _run(*case, bias=True, pad=72)
