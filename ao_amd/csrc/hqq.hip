@@ -172,30 +172,41 @@ __global__ __launch_bounds__(256) void hqq_mm_small_kernel(const uint8_t* __rest
     }
 }
 
-// four sums a thread; N is a multiple of 4
-template <bool BF16>
-__global__ __launch_bounds__(256) void hqq_mm_finish_kernel(const float* __restrict__ part, int slices, int64_t MN,
+// V sums a thread: four where all of them are whole aligned runs, one elsewhere (an odd number of rows over K = 2 mod 4 outputs of the
+// transposed product, a workspace that is only 4-byte aligned)
+template <bool BF16, int V>
+__global__ __launch_bounds__(256) void hqq_mm_finish_kernel(const float* __restrict__ part, int slices, int64_t count,
                                                             uint16_t* __restrict__ y) {
-    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (i >= MN) return;
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int z = 0; z < slices; ++z) {
-        const float4 v = *reinterpret_cast<const float4*>(part + (int64_t)z * MN + i);
-        s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
-    }
-    uint16_t o[4];
+    const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+    if (i >= count) return;   // (V divides count)
+    float s[V];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = BF16 ? hw_bf16_bits(s[e]) : f32_to_f16_bits(s[e]);
-    if (((uintptr_t)y & 7) == 0)
-        *reinterpret_cast<uint2*>(y + i) = make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
+    for (int e = 0; e < V; ++e) s[e] = 0.f;
+    for (int z = 0; z < slices; ++z) {
+        const float* const src = part + (int64_t)z * count + i;
+        if constexpr (V == 4) {
+            const float4 v = *reinterpret_cast<const float4*>(src);
+            s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
+        } else {
+            s[0] += src[0];
+        }
+    }
+    uint16_t o[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) o[e] = BF16 ? hw_bf16_bits(s[e]) : f32_to_f16_bits(s[e]);
+    if (V == 4 && ((uintptr_t)y & 7) == 0)
+        *reinterpret_cast<uint2*>(y + i) = make_uint2(o[0] | ((uint32_t)o[1 % V] << 16), o[2 % V] | ((uint32_t)o[3 % V] << 16));
     else
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[i + e] = o[e];
+        for (int e = 0; e < V; ++e) y[i + e] = o[e];
 }
 void launch_hqq_finish(const float* part, int slices, int64_t count, bool bf16, uint16_t* y, hipStream_t st) {
-    const dim3 grid((unsigned)((count / 4 + 255) / 256));
-    if (bf16) hipLaunchKernelGGL(hqq_mm_finish_kernel<true>, grid, dim3(256), 0, st, part, slices, count, y);
-    else hipLaunchKernelGGL(hqq_mm_finish_kernel<false>, grid, dim3(256), 0, st, part, slices, count, y);
+    auto go = [&](auto kernel, int v) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((count / v + 255) / 256)), dim3(256), 0, st, part, slices, count, y);
+    };
+    // (part is 16-byte aligned and so is every slice behind it)
+    if (count % 4 == 0 && ((uintptr_t)part & 15) == 0) bf16 ? go(hqq_mm_finish_kernel<true, 4>, 4) : go(hqq_mm_finish_kernel<false, 4>, 4);
+    else bf16 ? go(hqq_mm_finish_kernel<true, 1>, 1) : go(hqq_mm_finish_kernel<false, 1>, 1);
 }
 
 // K slices of the small-M product: enough waves to occupy the chip, at least 8 byte rows per wave

@@ -83,7 +83,7 @@ __device__ __forceinline__ void hqq_row(uint32_t d, const float* z, const float*
     p1 = hw_bf16_pack(w2, w3);
 }
 
-// fp32 partial sums [slices][rows x columns], a multiple of 4 of them, added and rounded to bf16 or fp16
+// fp32 partial sums [slices][count] added and rounded to bf16 or fp16
 void launch_hqq_finish(const float* part, int slices, int64_t count, bool bf16, uint16_t* y, hipStream_t st);
 
 // hqq_tile.hip: the product on 32- to 96-row tiles.  The plan's `rows` is 0 where it does not take the problem.

@@ -1,6 +1,8 @@
 """GPU tests of the HQQ prototype path: the dequantize kernel bit-exact against the oracle, the mixed matmul (forward and
 transposed) at the reference test's shapes against `x @ W_dq` / `x @ W_dq.T` (test/hqq/test_triton_mm.py:18-29, 118-139),
 and the HQQ -> int4 weight-only converter module."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -383,3 +385,50 @@ def test_mixed_mm_of_many_rows_keeps_its_other_routes(transposed):
     b, s, z, g = case(32)
     w = ops.hqq_dequantize(b, s, z, g)
     assert torch.equal(mixed_mm(x, b, s, z, g, transposed=transposed), torch.matmul(x, w.t() if transposed else w))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K,g", [(1, 16, 6, 2), (1, 16, 66, 2), (1, 2048, 1026, 18), (3, 48, 342, 18), (3, 4096, 1026, 18), (5, 16, 2050, 2), (2, 16, 66, 2)])
+def test_transposed_product_of_outputs_that_are_no_multiple_of_four(M, N, K, g, dtype):
+    """M K = 2 mod 4 outputs, among them 2 mod 1024 (K = 1026, 2050), from one and several slices of the reduction: every one is written, and
+    nothing behind them.  Tolerance as for the others above."""
+    from ao_amd import ops
+    from ao_amd._lib import BF16, F16, check, current_stream, lib
+    from ao_amd.prototype.hqq.mixed_mm import mixed_mm, pack_2xint4
+
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    packed = pack_2xint4(torch.randint(0, 16, (K, N), dtype=torch.uint8, device="cuda", generator=gen))
+    s = (torch.rand(K // g, N, device="cuda", generator=gen) * 0.02 + 1e-3).to(dtype)
+    z = (torch.rand(K // g, N, device="cuda", generator=gen) * 6 + 5).to(dtype)
+    x = torch.randn(M, N, device="cuda", generator=gen).to(dtype)
+    want = (x.double() @ ops.hqq_dequantize(packed, s, z, g).double().t()).to(dtype)
+    need = ctypes.c_int64(0)
+    check(lib().ao_amd_hqq_mixed_mm_mfma_workspace(M, K, N, 1, ctypes.byref(need)))
+    ws = torch.full((need.value // 4 + 4,), float("nan"), device="cuda")   # what lies behind the last slice is not added
+    y = torch.full((M * K + 8,), 123.0, dtype=dtype, device="cuda")
+    check(lib().ao_amd_hqq_mixed_mm_mfma(x.data_ptr(), M, N, packed.data_ptr(), 0, K, N, s.data_ptr(), z.data_ptr(), g,
+                                         BF16 if dtype is torch.bfloat16 else F16, 1, ws.data_ptr(), need.value, y.data_ptr(), current_stream(x.device)))
+    assert bool((y[M * K:] == 123.0).all())
+    for got in (y[:M * K].view(M, K), mixed_mm(x, packed, s, z, g, transposed=True)):
+        assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 1.5e-3
+
+
+def test_small_product_with_a_workspace_of_four_byte_alignment():
+    """The scalar kernel's workspace need be aligned to its floats only."""
+    from ao_amd import ops
+    from ao_amd._lib import BF16, check, current_stream, lib
+    from ao_amd.prototype.hqq.mixed_mm import pack_2xint4
+
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    M, N, K, g = 3, 1000, 512, 64
+    packed = pack_2xint4(torch.randint(0, 16, (K, N), dtype=torch.uint8, device="cuda", generator=gen))
+    s = (torch.rand(K // g, N, device="cuda", generator=gen) * 0.02 + 1e-3).bfloat16()
+    z = (torch.rand(K // g, N, device="cuda", generator=gen) * 6 + 5).bfloat16()
+    x = torch.randn(M, K, device="cuda", generator=gen).bfloat16()
+    need = ctypes.c_int64(0)
+    check(lib().ao_amd_hqq_mixed_mm_workspace(M, K, N, ctypes.byref(need)))
+    ws = torch.empty(need.value // 4 + 1, device="cuda")
+    y = torch.full((M, N), float("nan"), device="cuda").bfloat16()
+    check(lib().ao_amd_hqq_mixed_mm(x.data_ptr(), M, K, K, packed.data_ptr(), 0, N, s.data_ptr(), z.data_ptr(), g, BF16, ws[1:].data_ptr(),
+                                    need.value, y.data_ptr(), current_stream(x.device)))
+    assert torch.equal(y, ops.hqq_mixed_mm_small(x, packed, s, z, g))
