@@ -1150,6 +1150,12 @@ def hqq_mixed_mm_mfma(a: Tensor, packed_2xint4: Tensor, scales: Tensor, zeros: T
     return torch.ops.torchao.hqq_mixed_mm_mfma.default(a, packed_2xint4, scales, zeros, group_size, transposed)
 
 
+def hqq_mixed_mm_tiled(a: Tensor, packed_2xint4: Tensor, scales: Tensor, zeros: Tensor, group_size: int, transposed: bool = False):
+    """The product of more than 64 rows on tiles, or NotImplemented: a call that the native host path declines, one that is traced, or one
+    that the dequantized weight and a library product serve better."""
+    return NotImplemented if _tracing() else host.hqq_mixed_mm_many(a, packed_2xint4, scales, zeros, group_size, transposed)
+
+
 def hqq_dequantize(packed_2xint4: Tensor, scales: Tensor, zeros: Tensor, group_size: int) -> Tensor:
     """HQQ two-per-byte codes [K/2, N] -> (q - zero) * scale as a [K, N] matrix in the dtype of the scales."""
     return torch.ops.torchao.hqq_dequantize.default(packed_2xint4, scales, zeros, group_size)

@@ -55,7 +55,7 @@ def mixed_mm(a, b, scales, zeros, group_size, transposed=False, acc_dtype=None, 
     if not transposed and 1 <= M <= FUSED_MAX_ROWS and N % 4 == 0:
         return ops.hqq_mixed_mm_small(a, b, scales, zeros, group_size)
     if M > MFMA_MAX_ROWS and scales.shape[0] * group_size == 2 * K2:
-        y = ops.host.hqq_mixed_mm_many(a, b, scales, zeros, group_size, transposed)
+        y = ops.hqq_mixed_mm_tiled(a, b, scales, zeros, group_size, transposed)
         if y is not NotImplemented:
             return y
     w = ops.hqq_dequantize(b, scales, zeros, group_size)  # [K, N]

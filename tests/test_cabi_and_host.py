@@ -343,3 +343,25 @@ def test_int4_tiled_product_is_priced_against_every_tile_kernel(cabi):
         assert not offered(*shape), shape
     with open(os.path.join(os.path.dirname(cabi.__file__), "csrc", "int4wo_tile.hip")) as f:
         assert not re.search(r"\bstr(n?cmp|str)\b", f.read())
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("rows", [1, 64, 65, 100])
+def test_mixed_mm_traces_in_one_graph(rows, transposed):
+    """torch.compile sees registered operators and torch's own at every number of rows: one graph, no call of the native host path in it."""
+    from ao_amd.prototype.hqq.mixed_mm import mixed_mm
+
+    K, N, g, seen = 256, 512, 64, []
+
+    def backend(graph, example_inputs):
+        seen.append([str(n.target) for n in graph.graph.nodes if n.op.startswith("call")])
+        return graph.forward
+
+    def meta(*shape, dtype=torch.bfloat16):
+        return torch.empty(shape, dtype=dtype, device="meta")
+
+    torch._dynamo.reset()
+    y = torch.compile(mixed_mm, fullgraph=True, backend=backend)(
+        meta(rows, N if transposed else K), meta(K // 2, N, dtype=torch.uint8), meta(K // g, N), meta(K // g, N), g, transposed=transposed)
+    assert y.shape == (rows, K if transposed else N) and len(seen) == 1
+    assert ("torchao.hqq_mixed_mm_mfma.default" if rows <= 64 else "torchao.hqq_dequantize.default") in seen[0], seen
