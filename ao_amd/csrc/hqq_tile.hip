@@ -30,7 +30,7 @@ struct HqqTileArgs {
     const uint16_t *scales, *zeros, *a;
     int64_t lda, M, K, N, group;
     int tiles_m, tiles, per_xcd;
-    uint32_t per_group;   // forward: 2^32 / (group / 64) rounded up, or 0 where a step is a group
+    uint32_t per_group;   // forward: 2^32 / (group / 64) rounded up, exact for the steps that hqq_tile_plan admits, or 0 where a step is a group
     float* part;      // [gridDim.y][M][columns], or null: y is written
     uint16_t* y;
 };
@@ -402,6 +402,8 @@ HqqTilePlan hqq_tile_plan(int64_t M, int64_t K, int64_t N, int64_t group, bool t
     const int64_t R = transposed ? N : K, C = transposed ? K : N;
     if (group <= 0 || group % 64 || K % group || N % 16 || M < 1 || M >= (1 << 24) || R >= (1 << 24) || C >= (1 << 24)) return best;
     const int64_t steps = (R + 63) / 64, tiles_n = (C + 127) / 128;
+    // the kernel divides a step by d = group / 64 as the high word of step * ceil(2^32 / d), exact while step * (d - 1) < 2^32
+    if (!transposed && (steps - 1) * (group / 64 - 1) >= ((int64_t)1 << 32)) return best;
     for (int mt = 1; mt <= 3; ++mt) {
         const int64_t tiles_m = (M + 32 * mt - 1) / (32 * mt);
         if (tiles_m * tiles_n >= (1 << 24)) continue;
@@ -479,7 +481,7 @@ extern "C" int ao_amd_hqq_mixed_mm_tiled(const void* a, int64_t M, int64_t lda, 
     AO_REQUIRE(dtype == AO_BF16 || dtype == AO_F16, "activations, scales, zeros and output must be bf16 or f16, got code %d", dtype);
     AO_REQUIRE(M >= 1 && K > 0 && N > 0, "need positive M, K and N");
     HqqTilePlan p = hqq_tile_plan(M, K, N, group_size, transposed != 0, dtype == AO_BF16);
-    AO_REQUIRE(p.rows, "the tiled product needs the group size a multiple of 64 that divides K, and N a multiple of 16, got K=%lld N=%lld group=%lld",
+    AO_REQUIRE(p.rows, "the tiled product needs the group size a multiple of 64 that divides K, N a multiple of 16 and sizes below 2^24, got K=%lld N=%lld group=%lld",
                (long long)K, (long long)N, (long long)group_size);
     AO_REQUIRE(lda >= (transposed ? N : K) && lda % 8 == 0 && lda < (1ll << 24), "activation rows must be 16-byte aligned and as long as the reduction");
     AO_REQUIRE(((((uintptr_t)a) | ((uintptr_t)packed_2xint4) | ((uintptr_t)scales) | ((uintptr_t)zeros) | ((uintptr_t)y) | ((uintptr_t)workspace)) & 15) == 0,

@@ -365,3 +365,22 @@ def test_mixed_mm_traces_in_one_graph(rows, transposed):
         meta(rows, N if transposed else K), meta(K // 2, N, dtype=torch.uint8), meta(K // g, N), meta(K // g, N), g, transposed=transposed)
     assert y.shape == (rows, K if transposed else N) and len(seen) == 1
     assert ("torchao.hqq_mixed_mm_mfma.default" if rows <= 64 else "torchao.hqq_dequantize.default") in seen[0], seen
+
+
+def test_hqq_tiles_take_groups_that_their_reciprocal_divides(cabi):
+    """The forward kernel's group of a 64-wide step is the high word of step * ceil(2^32 / (group / 64)).  Offered shapes: exact at both
+    ends of every group.  The first three are not: their last steps came out a group too high."""
+
+    def offered(K, g, transposed=0, N=1024):
+        need = ctypes.c_int64(-2)
+        cabi.check(cabi.lib().ao_amd_hqq_mixed_mm_tiled_bytes(100, K, N, g, cabi.BF16, transposed, ctypes.byref(need)))
+        return need.value >= 0
+
+    for K, g, taken in ((4194368, 4194368, False), (16000000, 3200000, False), (15728640, 15728640, False), (4194304, 4194304, True),
+                        (8388608, 131072, True), (14336, 192, False), (14400, 192, True), (12288, 4096, True)):
+        assert offered(K, g) == taken, (K, g)
+        if taken:
+            d, steps = g // 64, K // 64
+            m = ((1 << 32) + d - 1) // d
+            assert all((s * m) >> 32 == s // d for i in range(0, steps, d) for s in (i, min(i + d, steps) - 1)), (K, g)
+    assert offered(4194368, 4194368, transposed=1)   # (which divides in 64 bits)
