@@ -82,6 +82,8 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void tile_gemm_kernel(const Tile
     // with PAIR the weights have a ring of their own, of three pairs of steps
     constexpr int RING = PAIR ? STAGES * ABYTES + 6 * BBYTES : STAGES * STAGE;
     static_assert(!PAIR || KW * RING <= 160 * 1024, "LDS of a CU");
+    // With three buffers an odd step would wait for its own requests and those of the pair, and not for the step that it reads next
+    static_assert(!PAIR || STAGES == 4, "PAIR's waits count four activation buffers");
     constexpr int AREQ = ABYTES / 1024 / G, WREQ = F::REQ * (PAIR ? 2 : 1), BREQ = NT * WREQ / WM, REQ = AREQ + BREQ;
     static_assert(AREQ * G * 1024 == ABYTES && BREQ * WM == NT * WREQ && (NT % WM == 0 || NT == 1), "every wave issues the same number of requests");
     constexpr int ACC = MT * NT * 4096;   // bytes of one wave's accumulators
