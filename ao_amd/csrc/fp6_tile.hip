@@ -97,13 +97,14 @@ static TilePlan fp6_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
 // 128 x 128 tiles 50 for one round and 37 for each of several.  us, those /
 // tiled: 14336 x 4096 at 65 / 160 / 256 / 384 / 768 rows 30 / 24, 44 / 30, 56 / 40, 68 / 49, 114 / 88; 4096 x 14336 at 160 / 512 / 1000 rows
 // 57 / 35, 97 / 74, 169 / 120; 4096 x 4096 at 128 / 384 / 1000 rows 12.3 / 15.0, 27 / 21, 50 / 39; 5120 x 5120 at 96 / 384 rows 14.4 /
-// 18.0, 34 / 32; 1024 x 4096 at 512 / 640 rows 12.6 / 15.4, 17.8 / 16.8.  Up to 64 rows the streaming kernels and small tiles
-// hold on for weights of up to 25 M (6144 x 4096 at 48 rows 12.1 / 12.7; 5120 x 5120 14.1 / 13.2; 14336 x 4096 at 33 / 48 rows 18.8 / 15.5,
-// 19.2 / 16.1; 13824 x 5120 at 48 rows 22.3 / 20.0; at 52 rows 14336 x 4096 19.7 / 14.7, 13824 x 5120 23.6 / 17.0, 5120 x 5120 15.4 / 13.9), at
-// 64 rows for all but the largest (13824 x 5120 24.0 / 18.8; the routes of others are what callers there know: 14336 x 4096 20.0 / 14.8).
-// Where they split K over workgroups (fp6.hip:
-// fp6_ws_parts) they are kept but for 65 to 96 rows of weights from 50 M on (4096 x 14336 at 64 / 66 / 96 rows 20.9 / 20.9, 31.0 / 22.2, 32.3 / 24.1;
-// 4096 x 4096 at 66 rows 11.9 / 13.4).
+// 18.0, 34 / 32; 1024 x 4096 at 512 / 640 rows 12.6 / 15.4, 17.8 / 16.8.  At 33 to 64 rows the others are 32 x 64 tiles, whose one round over
+// the CUs ends at 8192 columns: beyond, the tiles are ahead by 0 to 32 % (those / tiled at 33 and 64 rows: 8448 x 4096 16.9 / 11.8, 17.7 /
+// 12.1; 14336 x 4096 18.0 / 16.3, 19.0 / 17.6; 14336 x 2048 10.5 / 8.7, 11.0 / 9.4; 16384 x 2048 10.6 / 9.9, 11.4 / 11.2; 28672 x 8192 54 / 43, 60 /
+// 46); below it only where that round is long and its workgroups leave room for two K parts (5120 x 5120 14.0 / 12.4, 14.1 / 13.7; 6400 x
+// 7168 19.2 / 16.7, 19.6 / 18.9; but 8192 x 4096 12.2 / 13.1 at 33 and 12.5 / 13.6 at 56 rows, 7168 x 6144 16.8 / 15.7, 16.9 / 17.7, 8192 x 7168 20.0 / 20.4,
+// 20.6 / 22.3).  Weights below 26 M were not measured there.
+// Where the others split K over workgroups (fp6.hip: fp6_ws_parts) they are kept but for 65 to 96 rows of weights from 50 M on (4096 x
+// 14336 at 64 / 66 / 96 rows 20.9 / 20.9, 31.0 / 22.2, 32.3 / 24.1; 4096 x 4096 at 66 rows 11.9 / 13.4).
 static bool fp6_tiled(int64_t M, int64_t N, int64_t K) {
     if (K % 64 != 0 || N % 16 != 0 || M <= 32 || M * N >= ((int64_t)1 << 40) || 192 * K * 2 >= ((int64_t)1 << 32)) return false;
     if (ao_amd_fp6_linear_ws_parts(M, K, N) != 1 && (M <= 64 || M > 96 || N * K < 50000000)) return false;
@@ -111,7 +112,7 @@ static bool fp6_tiled(int64_t M, int64_t N, int64_t K) {
     // streamed once per 16 rows there (14336 x 4032 at 33 / 128 / 1000 rows 22 / 50 / 305 us, tiled 20 / 24 / 119; 4096 x 4160 at 65 / 128 /
     // 1000 rows 14 / 17 / 96, tiled 16 / 16 / 41)
     if (K % 128 != 0) return tile_us < 5.0 + 8.5e-8 * (double)(N * K) * (double)((M + 15) / 16);
-    if (M <= 64) return N * K >= (M < 64 ? (int64_t)26000000 : (int64_t)60000000);
+    if (M <= 64) return N * K >= 26000000 && (N > 8192 || (N <= 6400 && K >= 5120));
     // (the 128 x 128 tiles of fp6.hip were never ahead there: 14336 x 4096 at 1200 / 1500 rows 169 / 178 tiled)
     if (M >= 1024 && N >= 2048) return true;
     const int64_t big = (N + 127) / 128 * ((M + 127) / 128), mid = (N + 63) / 64 * ((M + 63) / 64), small = (N + 63) / 64 * ((M + 31) / 32);
