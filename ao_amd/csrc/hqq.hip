@@ -596,8 +596,8 @@ extern "C" int ao_amd_hqq_mixed_mm_mfma_workspace(int64_t M, int64_t K, int64_t 
     const int a = hqq_mfma_plan(M, K, N, transposed != 0, 64).slices, b = hqq_mfma_plan(M, K, N, transposed != 0, 2).slices;
     int most = a > b ? a : b;
     for (int bf16 = 0; bf16 < 2; ++bf16) {
-        const HqqTilePlan t = hqq_tile_plan(M, K, N, 64, transposed != 0, bf16 != 0);
-        if (hqq_tiled(t, M, K, N, transposed != 0, bf16 != 0) && t.parts > most) most = t.parts;
+        const HqqTilePlan t = hqq_tile_route(M, K, N, 64, transposed != 0, bf16 != 0);
+        if (t.rows && t.parts > most) most = t.parts;
     }
     *bytes = (int64_t)most * M * (transposed ? K : N) * (int64_t)sizeof(float);
     return 0;
@@ -630,8 +630,8 @@ extern "C" int ao_amd_hqq_mixed_mm_mfma(const void* a, int64_t M, int64_t lda, c
     if (int rc = ao_amd_hqq_mixed_mm_mfma_workspace(M, K, N, transposed, &need)) return rc;
     AO_REQUIRE(workspace_bytes >= need && (((uintptr_t)workspace) & 15) == 0, "16-byte aligned workspace of %lld bytes needed, got %lld",
                (long long)need, (long long)workspace_bytes);
-    const HqqTilePlan t = hqq_tile_plan(M, K, N, group_size, transposed != 0, dtype == AO_BF16);
-    if (hqq_tiled(t, M, K, N, transposed != 0, dtype == AO_BF16) && (((uintptr_t)y) & 15) == 0 && lda < (1 << 24)) {
+    const HqqTilePlan t = hqq_tile_route(M, K, N, group_size, transposed != 0, dtype == AO_BF16);
+    if (t.rows && (((uintptr_t)y) & 15) == 0 && lda < (1 << 24)) {
         launch_hqq_tile(t, (const uint8_t*)packed_2xint4, (const uint16_t*)scales, (const uint16_t*)zeros, (const uint16_t*)a, lda, M, K, N, group_size,
                         is_signed != 0, dtype == AO_BF16, transposed != 0, (float*)workspace, (uint16_t*)y, (hipStream_t)stream);
         AO_LAUNCH_CHECK();

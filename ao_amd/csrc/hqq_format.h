@@ -89,7 +89,7 @@ void launch_hqq_finish(const float* part, int slices, int64_t count, bool bf16, 
 // hqq_tile.hip: the product on 32- to 96-row tiles.  The plan's `rows` is 0 where it does not take the problem.
 struct HqqTilePlan { int rows, tiles_m, tiles_n, parts; double us; };
 HqqTilePlan hqq_tile_plan(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed, bool bf16, int max_parts = 16);
-bool hqq_tiled(const HqqTilePlan& p, int64_t M, int64_t K, int64_t N, bool transposed, bool bf16);
+HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed, bool bf16);   // .. or is not the fastest
 void launch_hqq_tile(const HqqTilePlan& p, const uint8_t* packed, const uint16_t* scales, const uint16_t* zeros, const uint16_t* a, int64_t lda,
                      int64_t M, int64_t K, int64_t N, int64_t group, bool is_signed, bool bf16, bool transposed, float* part, uint16_t* y,
                      hipStream_t st);

@@ -420,20 +420,28 @@ HqqTilePlan hqq_tile_plan(int64_t M, int64_t K, int64_t N, int64_t group, bool t
     return best;
 }
 
-// Whether the tiles are the faster route.  Beyond 64 rows the other one writes the weight in 16 bits and calls the library product: 11008 x
+// The tiles' plan where they are the faster route.  Beyond 64 rows the other one writes the weight in 16 bits and calls the library product: 11008 x
 // 4096 at 96 / 235 rows 68 / 76 us against 28 / 56; 128256 x 4096 at 79 / 253 rows 749 / 899 against 170 / 427; 1024 x 4096 at 228 rows
 // 16.4 against 14.5; 14336 x 4096 at 433 rows 94 against 99.  Its time is estimated with a lead for products of 45 GFLOP on, where the
 // library catches up (and twice the rate beyond the rows that were measured).  Up to 64 rows the other one is the streaming kernel of
 // hqq.hip, whose time follows the activations it reads again for every 64 columns: 4096 x 14336 at 47 rows 30 us against 22, 28672 x 8192
 // at 7 rows 61 against 51, 14336 x 4096 transposed at 64 rows 29 against 22; with 32 rows of bf16 transposed it is ahead (11008 x 4096 18.8
 // against 21.2) and with small weights (4096 x 4096 at 64 rows transposed 17.0 against 18.1).
-bool hqq_tiled(const HqqTilePlan& p, int64_t M, int64_t K, int64_t N, bool transposed, bool bf16) {
-    if (!p.rows) return false;
-    const double weights = (double)K * (double)N, flops = 2.0 * (double)M * weights;
-    if (M > 512) return p.us < 10.0 + weights * 0.55e-6 + flops / 1.2e9;
-    if (M > 64) return p.us < (flops < 4.5e10 ? 1.0 : 0.82) * (14.0 + weights * 0.8e-6 + flops / 0.9e9);
-    if (M > 32) return weights >= 2e7;
-    return transposed ? M > 16 && !bf16 && weights >= 6.4e7 : weights >= (M > 16 ? 3e7 : 6.4e7);
+HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed, bool bf16) {
+    const HqqTilePlan none{0, 0, 0, 1, 1e30};
+    const double weights = (double)K * (double)N, rows = (double)M, flops = 2.0 * rows * weights;
+    // the size of the weight first: a plan takes a tenth of a microsecond of host time, which bounds calls on small weights
+    if (weights < (M > 64 ? 0.0 : M > 32 ? 2e7 : !transposed ? (M > 16 ? 3e7 : 6.4e7) : M > 16 && !bf16 ? 6.4e7 : 1e30)) return none;
+    const HqqTilePlan p = hqq_tile_plan(M, K, N, group, transposed, bf16);
+    if (!p.rows) return none;
+    double other = 1e30;
+    if (M > 512) {
+        other = 10.0 + weights * 0.55e-6 + flops / 1.2e9;
+    } else if (M > 64) {
+        other = 14.0 + weights * 0.8e-6 + flops / 0.9e9;
+        if (flops >= 4.5e10) other *= 0.82;
+    }
+    return p.us < other ? p : none;
 }
 
 template <bool BF16, bool SIGNED, bool TR>
@@ -469,8 +477,8 @@ using namespace ao;
 extern "C" int ao_amd_hqq_mixed_mm_tiled_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size, int dtype, int transposed, int64_t* bytes) {
     AO_REQUIRE(bytes, "null pointer argument");
     AO_REQUIRE(M >= 1 && K > 0 && N > 0 && group_size > 0, "need positive M, K, N and group size");
-    const HqqTilePlan p = hqq_tile_plan(M, K, N, group_size, transposed != 0, dtype == AO_BF16);
-    *bytes = !hqq_tiled(p, M, K, N, transposed != 0, dtype == AO_BF16) ? -1 : p.parts > 1 ? (int64_t)p.parts * M * (transposed ? K : N) * (int64_t)sizeof(float) : 0;
+    const HqqTilePlan p = hqq_tile_route(M, K, N, group_size, transposed != 0, dtype == AO_BF16);
+    *bytes = !p.rows ? -1 : p.parts > 1 ? (int64_t)p.parts * M * (transposed ? K : N) * (int64_t)sizeof(float) : 0;
     return 0;
 }
 
