@@ -423,25 +423,37 @@ HqqTilePlan hqq_tile_plan(int64_t M, int64_t K, int64_t N, int64_t group, bool t
 // The tiles' plan where they are the faster route.  Beyond 64 rows the other one writes the weight in 16 bits and calls the library product: 11008 x
 // 4096 at 96 / 235 rows 68 / 76 us against 28 / 56; 128256 x 4096 at 79 / 253 rows 749 / 899 against 170 / 427; 1024 x 4096 at 228 rows
 // 16.4 against 14.5; 14336 x 4096 at 433 rows 94 against 99.  Its time is estimated with a lead for products of 45 GFLOP on, where the
-// library catches up (and twice the rate beyond the rows that were measured).  Up to 64 rows the other one is the streaming kernel of
-// hqq.hip, whose time follows the activations it reads again for every 64 columns: 4096 x 14336 at 47 rows 30 us against 22, 28672 x 8192
-// at 7 rows 61 against 51, 14336 x 4096 transposed at 64 rows 29 against 22; with 32 rows of bf16 transposed it is ahead (11008 x 4096 18.8
-// against 21.2) and with small weights (4096 x 4096 at 64 rows transposed 17.0 against 18.1).
+// library catches up (and twice the rate beyond the rows that were measured).
+// Up to 64 rows the other one is the streaming kernel of hqq.hip, timed against the tiles on 14 weights (K x N below, us streamed / tiled).
+// Forward from 17 rows on the size of the weight decides (17 rows of bf16: 4096 x 4096 11.0 / 12.1, 5120 x 5120 13.2 / 14.0, 4096 x 8192 14.5 / 12.9,
+// 5120 x 13824 31.5 / 21.2; 33 rows 5120 x 5120 16.2 / 16.4, 4096 x 6144 17.2 / 15.1).  With fewer rows, and transposed, the tiles' own time
+// does too: 5120 output columns are 40 tiles, which fill the CUs badly whatever the K parts.  One row of bf16 8192 x 28672 53.8 / 49.3,
+// 4096 x 32000 41.0 / 27.1, 8192 x 8192 20.4 / 19.2, but 13824 x 5120 23.1 / 26.6; transposed at 33 / 64 rows of bf16 8192 x 28672 72 / 67, 90 / 67,
+// 4096 x 14336 24.0 / 24.9, 28.6 / 25.3, but 5120 x 13824 28.3 / 42.4, 35.5 / 37.8, 4096 x 8192 17.3 / 19.3, 20.5 / 20.2; of fp16 at 17 / 32 rows 8192 x
+// 28672 48 / 43, 59 / 44, but 5120 x 13824 20.0 / 24.9, 22.9 / 25.3.  The streaming kernel's time is therefore estimated, from those weights:
+// a part for every weight, one for every weight and row (the activations are read again for every 64 columns), the fp32 sums; the tiles' estimate
+// is 5 to 8 % long.
 HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed, bool bf16) {
     const HqqTilePlan none{0, 0, 0, 1, 1e30};
     const double weights = (double)K * (double)N, rows = (double)M, flops = 2.0 * rows * weights;
     // the size of the weight first: a plan takes a tenth of a microsecond of host time, which bounds calls on small weights
-    if (weights < (M > 64 ? 0.0 : M > 32 ? 2e7 : !transposed ? (M > 16 ? 3e7 : 6.4e7) : M > 16 && !bf16 ? 6.4e7 : 1e30)) return none;
+    if (weights < (M > 64 ? 0.0 : !transposed ? (M > 32 ? 2e7 : M > 16 ? 3e7 : 6.4e7) : M > 32 ? (bf16 ? 4e7 : 2e7) : M > 16 && !bf16 ? 6.4e7 : 1e30)) return none;
     const HqqTilePlan p = hqq_tile_plan(M, K, N, group, transposed, bf16);
     if (!p.rows) return none;
-    double other = 1e30;
+    double other = 1e30, lead = 1.0;
     if (M > 512) {
         other = 10.0 + weights * 0.55e-6 + flops / 1.2e9;
     } else if (M > 64) {
         other = 14.0 + weights * 0.8e-6 + flops / 0.9e9;
         if (flops >= 4.5e10) other *= 0.82;
+    } else if (transposed) {
+        other = 5.6 + ((bf16 ? 0.18 : 0.14) + (bf16 ? 0.0022 : 0.0028) * rows) * weights * 1e-6 + (bf16 ? 0.065 : 0.055) * rows + 4.5e-6 * rows * (double)K;
+        lead = bf16 ? 0.92 : 0.95;
+    } else if (M <= 16) {
+        other = 6.2 + ((bf16 ? 0.22 : 0.2) + (bf16 ? 0.0011 : 0.0015) * rows) * weights * 1e-6;
+        lead = 0.92;
     }
-    return p.us < other ? p : none;
+    return lead * p.us < other ? p : none;
 }
 
 template <bool BF16, bool SIGNED, bool TR>

@@ -384,3 +384,30 @@ def test_hqq_tiles_take_groups_that_their_reciprocal_divides(cabi):
             m = ((1 << 32) + d - 1) // d
             assert all((s * m) >> 32 == s // d for i in range(0, steps, d) for s in (i, min(i + d, steps) - 1)), (K, g)
     assert offered(4194368, 4194368, transposed=1)   # (which divides in 64 bits)
+
+
+@pytest.mark.parametrize("transposed,dtype,M,K,N,tiled", [
+    # streamed / tiled, us: forward
+    (0, "BF16", 1, 13824, 5120, False),   # 23.1 / 26.6
+    (0, "BF16", 1, 5120, 13824, True),    # 23.9 / 20.9
+    (0, "F16", 16, 8192, 8192, True),     # 19.9 / 17.5
+    (0, "BF16", 17, 13824, 5120, True),   # 29.7 / 26.8
+    (0, "BF16", 64, 4096, 4096, False),   # 14.7 / 16.5
+    # transposed
+    (1, "F16", 17, 5120, 13824, False),   # 20.0 / 24.9
+    (1, "F16", 32, 5120, 13824, False),   # 22.9 / 25.3
+    (1, "F16", 17, 8192, 28672, True),    # 48.2 / 43.5
+    (1, "BF16", 32, 8192, 28672, False),  # 59.9 / 58.2
+    (1, "BF16", 33, 5120, 13824, False),  # 28.3 / 42.4
+    (1, "BF16", 64, 5120, 13824, False),  # 35.5 / 37.8
+    (1, "BF16", 64, 13824, 5120, True),   # 39.3 / 30.2
+    (1, "BF16", 33, 4096, 8192, False),   # 17.3 / 19.3
+    (1, "BF16", 33, 5120, 5120, False),   # 16.5 / 19.5
+    (1, "F16", 64, 5120, 5120, True),     # 19.4 / 17.5
+    (1, "BF16", 64, 4096, 14336, True),   # 28.6 / 25.3
+])
+def test_hqq_tiles_only_where_they_are_ahead(cabi, transposed, dtype, M, K, N, tiled):
+    """Both sides of the rule up to 64 rows, by the measured times of the two kernels."""
+    need = ctypes.c_int64(-2)
+    cabi.check(cabi.lib().ao_amd_hqq_mixed_mm_tiled_bytes(M, K, N, 64, getattr(cabi, dtype), transposed, ctypes.byref(need)))
+    assert (need.value >= 0) == tiled
