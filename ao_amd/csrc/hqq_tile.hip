@@ -15,6 +15,7 @@
 // 4 MT + 6 of 1 KB a step, each of which holds its wave's issue for some 120 cycles: 1.3 - 2.8 us a step.  96-row tiles convert
 // each weight the least often.  11008 x 4096 at 96 rows 68 -> 28 us, 4096 x 4096 at 128 rows 44 -> 20, 12416 x 1600 at 425 rows 71 -> 41
 // (dequantization and library product before).
+#include <algorithm>
 #include <type_traits>
 
 #include "hqq_format.h"
@@ -423,7 +424,11 @@ HqqTilePlan hqq_tile_plan(int64_t M, int64_t K, int64_t N, int64_t group, bool t
 // The tiles' plan where they are the faster route.  Beyond 64 rows the other one writes the weight in 16 bits and calls the library product: 11008 x
 // 4096 at 96 / 235 rows 68 / 76 us against 28 / 56; 128256 x 4096 at 79 / 253 rows 749 / 899 against 170 / 427; 1024 x 4096 at 228 rows
 // 16.4 against 14.5; 14336 x 4096 at 433 rows 94 against 99.  Its time is estimated with a lead for products of 45 GFLOP on, where the
-// library catches up (and twice the rate beyond the rows that were measured).
+// library catches up (and twice the rate beyond the rows that were measured).  Transposed products whose reduction is at most one and
+// a half times as long as their output is wide have an estimate of their own, from weights of up to 71 M at 65 to 512 rows: the library holds up there (K x
+// N, bf16, 16-bit weight and library / tiles at 192 and 384 rows: 11008 x 4096 60 / 45, 70 / 86; 14336 x 4096 70 / 45, 86 / 86; 4096 x 6144 52 / 27, 44 / 40, 51 / 58 at 512;
+// 5120 x 5120 49 / 30, 44 / 47; 8192 x 8192 92 / 50, 96 / 84, 106 / 135 at 448), and a little on wide weights forward (4096 x 14336 at 448 rows 95 / 98,
+// 4096 x 32000 of fp16 at 512 193 / 198).
 // Up to 64 rows the other one is the streaming kernel of hqq.hip, timed against the tiles on 14 weights (K x N below, us streamed / tiled).
 // Forward from 17 rows on the size of the weight decides (17 rows of bf16: 4096 x 4096 11.0 / 12.1, 5120 x 5120 13.2 / 14.0, 4096 x 8192 14.5 / 12.9,
 // 5120 x 13824 31.5 / 21.2; 33 rows 5120 x 5120 16.2 / 16.4, 4096 x 6144 17.2 / 15.1).  With fewer rows, and transposed, the tiles' own time
@@ -445,7 +450,8 @@ HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool 
         other = 10.0 + weights * 0.55e-6 + flops / 1.2e9;
     } else if (M > 64) {
         other = 14.0 + weights * 0.8e-6 + flops / 0.9e9;
-        if (flops >= 4.5e10) other *= 0.82;
+        if (flops >= 4.5e10) other *= transposed || N <= 2 * K ? 0.82 : 0.8;
+        if (transposed && 2 * N <= 3 * K && weights < 1e8) other = std::min(other, 20.0 + 0.61e-6 * weights + rows * (0.0016e-6 * weights - 0.009));
     } else if (transposed) {
         other = 5.6 + ((bf16 ? 0.18 : 0.14) + (bf16 ? 0.0022 : 0.0028) * rows) * weights * 1e-6 + (bf16 ? 0.065 : 0.055) * rows + 4.5e-6 * rows * (double)K;
         lead = bf16 ? 0.92 : 0.95;

@@ -405,9 +405,20 @@ def test_hqq_tiles_take_groups_that_their_reciprocal_divides(cabi):
     (1, "BF16", 33, 5120, 5120, False),   # 16.5 / 19.5
     (1, "F16", 64, 5120, 5120, True),     # 19.4 / 17.5
     (1, "BF16", 64, 4096, 14336, True),   # 28.6 / 25.3
+    # beyond 64 rows, 16-bit weight and library / tiles
+    (1, "BF16", 192, 11008, 4096, True),  # 59.7 / 44.5
+    (1, "BF16", 384, 11008, 4096, False), # 69.6 / 85.5
+    (1, "BF16", 320, 14336, 4096, False), # 78.4 / 88.0
+    (1, "BF16", 512, 4096, 6144, False),  # 50.8 / 57.8
+    (1, "BF16", 384, 4096, 6144, True),   # 44.2 / 40.2
+    (1, "F16", 448, 14336, 2448, False),  # 66.5 / 72.0
+    (1, "F16", 384, 14336, 2448, True),   # 60.1 / 50.1
+    (1, "BF16", 320, 4096, 11008, True),  # 76.5 / 62.9
+    (0, "BF16", 512, 4096, 14336, False), # 95.3 / 99.0
+    (0, "BF16", 448, 8192, 8192, True),   # 113.9 / 103.7
 ])
 def test_hqq_tiles_only_where_they_are_ahead(cabi, transposed, dtype, M, K, N, tiled):
-    """Both sides of the rule up to 64 rows, by the measured times of the two kernels."""
+    """Both sides of the rule, by the measured times of the routes."""
     need = ctypes.c_int64(-2)
     cabi.check(cabi.lib().ao_amd_hqq_mixed_mm_tiled_bytes(M, K, N, 64, getattr(cabi, dtype), transposed, ctypes.byref(need)))
     assert (need.value >= 0) == tiled
