@@ -111,10 +111,17 @@ static TilePlan int4wo_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts)
 }
 
 // us of the kernel that ao_amd_int4wo_linear(_ws) runs, by measurement at 33 to 1000 rows on 16 weights from 768 x 1024 to 28672 x
-// 8192; 0 where it is not one of the tile kernels (few rows: the weight is streamed).
-static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
+// 8192; 0 where it is not one of the tile kernels (few rows: the weight is streamed).  K as packed; `ends`: the rows end before it.
+static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g, bool ends) {
     Int4Kernel kernel;
-    if (!int4wo_plain_kernel(M, K, N, g, &kernel) || kernel == Int4Kernel::streaming) return 0.0;
+    if (!int4wo_plain_kernel(M, K, N, g, &kernel)) return 0.0;
+    if (kernel == Int4Kernel::streaming) {
+        // Four blocks of streamed rows in the variant for rows that end early and row blocks that are no multiple of four are behind the tiles:
+        // us at 33 / 48 rows, streamed / tiled, 12304 x 4096 19.0 / 16.9, 19.6 / 17.0, 18837 x 1088 14.9 / 12.0, 16.1 / 12.8, 14336 x 4160 19.9 / 17.3,
+        // 21.0 / 17.7, 28000 x 5312 39.9 / 38.4, 42.8 / 38.7; but 65552 x 1024 28.1 / 29.9, 30.3 / 30.4 (and 35.0 / 31.3 at 64 rows).
+        const int64_t blocks = (N + 15) / 16;
+        return (ends || blocks % 4 != 0) && blocks >= 768 && (blocks < 4096 || M > 48) ? 1e9 : 0.0;
+    }
     const double k = (double)K / 4096.0;
     auto rounds = [&](int bm, int bn) { return (double)((M + bm - 1) / bm * ((N + bn - 1) / bn)) / 256.0; };
     auto up = [](double r) { return (double)(int64_t)(r + 255.0 / 256.0); };
@@ -145,7 +152,7 @@ static bool int4wo_tiled(int64_t M, int64_t N, int64_t K, int64_t g) {
     if (!valid_group(g) || K % 64 != 0 || M <= 32 || M * N >= ((int64_t)1 << 40)) return false;
     // in_features that were padded to whole tiles of the packed layout: the others take activations copied to that width first
     const int64_t Kp = round_up(K, g > 128 ? g : 128);
-    const double other = int4wo_other_us(M, N, Kp, g);
+    const double other = int4wo_other_us(M, N, Kp, g, K != Kp);
     const TilePlan plan = int4wo_tile_plan(M, N, K, 8);
     Int4Kernel kernel;
     // (the plan may be the very launch that the dispatch makes)

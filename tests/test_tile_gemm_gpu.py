@@ -341,6 +341,28 @@ def test_int4_rows_that_are_read_as_they_end(M, N, K, group, name):
     assert torch.equal(ops.int4wo_linear(x, packed, qp, group, N), dq[:, at].t())
 
 
+@pytest.mark.parametrize("M,N,K,group,tiled", [
+    (32, 12304, 1088, 128, False), (33, 12304, 1088, 128, True), (48, 12304, 1024, 64, True), (33, 12288, 1088, 32, True), (33, 12288, 1024, 64, False),
+    (33, 12290, 1032, 64, False),                                   # a width that the tiles do not take
+    (48, 65552, 192, 64, False), (49, 65552, 192, 64, True), (64, 65540, 256, 32, True),
+])
+def test_int4_ragged_weights_at_33_to_64_rows(M, N, K, group, tiled):
+    """Rows that end before the packed width, and row blocks that are no multiple of four: from 33 rows on the tiles are ahead of the
+    streaming kernel that could read them (18837 x 1088 at 33 rows 12.0 / 14.9 us, 12304 x 4096 at 48 17.0 / 19.6).  The operator against the fp32
+    product (as for the tiles); what lies behind a row's end is NaN."""
+    from ao_amd import ops
+
+    assert (_tiled_bytes("int4wo", M, N, K, group) >= 0) == tiled
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    packed, qp = ops.int4wo_quantize_pack((torch.randn(N, K, device="cuda", generator=g) * 0.02).bfloat16(), group)
+    rows = torch.full((M, K + 8), float("nan"), device="cuda").bfloat16()
+    x = rows[:, :K]
+    x.copy_(torch.randn(M, K, device="cuda", generator=g))
+    y, want = ops.int4wo_linear(x, packed, qp, group, N), (x.float() @ ops.int4wo_dequantize(packed, qp, N, K, group).float().t()).bfloat16()
+    rel = ((y.float() - want.float()).norm() / want.float().norm()).item()
+    assert rel <= 1e-3 and (y != want).float().mean() <= 0.01, rel
+
+
 @pytest.mark.parametrize("fmt,M,N,K,group,name", [
     ("int4", 1700, 7000, 512, 64, "int4wo_gemm_lds_kernel<64,2>"), ("int4", 1000, 6400, 512, 128, "int4wo_gemm_lds_kernel<128,1>"),
     ("int4", 300, 4100, 1024, 32, "int4wo_gemm_kwave_kernel"), ("int4", 2750, 1024, 4096, 64, ""), ("int4", 5000, 64, 256, 64, ""),
