@@ -1326,9 +1326,10 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
             AO_LAUNCH_CHECK();
             return 0;
         }
-        if (int4wo_gemv1_plan(a, g, RB, name, sizeof(name))) {
+        if (plan && int4wo_gemv1_plan(a, g, RB, name, sizeof(name))) {
             AO_PLAN(Int4Kernel::streaming, "%s", name);
-            launch_int4wo_gemv1(a, g, RB, st);
+        }
+        if (!plan && launch_int4wo_gemv1(a, g, RB, st)) {
             AO_LAUNCH_CHECK();
             return 0;
         }

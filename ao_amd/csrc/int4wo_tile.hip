@@ -153,13 +153,14 @@ static bool int4wo_tiled(int64_t M, int64_t N, int64_t K, int64_t g) {
     // in_features that were padded to whole tiles of the packed layout: the others take activations copied to that width first
     const int64_t Kp = round_up(K, g > 128 ? g : 128);
     const double other = int4wo_other_us(M, N, Kp, g, K != Kp);
+    if (other <= 0.0) return false;
     const TilePlan plan = int4wo_tile_plan(M, N, K, 8);
     Int4Kernel kernel;
     // (the plan may be the very launch that the dispatch makes)
     if (plan.shape >= kInt4Own && plan.parts == 1 && int4wo_plain_kernel(M, Kp, N, g, &kernel) &&
         kernel == (plan.shape == kInt4Own ? Int4Kernel::lds_256x128 : Int4Kernel::lds_256x256))
         return false;
-    return other > 0.0 && plan.us < (Kp == K ? 0.95 * other : other + 4.0);
+    return plan.us < (Kp == K ? 0.95 * other : other + 4.0);
 }
 
 // x [M, K] with row stride ldx -> y [M, Kp], zeros beyond K, 8 elements a thread: activations whose rows are not 16-byte aligned
