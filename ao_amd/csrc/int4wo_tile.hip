@@ -138,7 +138,9 @@ static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g, bool e
         // (one round over 14336 of K: 427 / 512 rows of 4096 x 14336 80 / 78 us, tiled 70 / 73)
         return 6.0 + (three ? (r > 1.0 ? 17.5 : 16.5) : r > 1.0 || K >= 8192 ? 20.5 : 18.5) * k * r;
     }
-    if (ao_amd_int4wo_linear_ws_parts(M, K, N, g) > 1) return M <= 64 ? 0.0 : 4.0 + 8.0 * k;
+    // (short K: the sums of eight parts cost the tiles more than they save.  us in K parts there / tiled at 100 rows: 512 x 4096 10.7 / 11.4, 1024 x 4096
+    // 11.1 / 12.6, 1536 x 4096 11.5 / 12.0, 1024 x 2048 10.3 / 10.4, 1024 x 6144 12.5 / 12.9; 512 x 8192 14.1 / 13.3, 1024 x 14336 20.0 / 16.5)
+    if (ao_amd_int4wo_linear_ws_parts(M, K, N, g) > 1) return M <= 64 || K < 7168 ? 0.0 : 4.0 + 8.0 * k;
     if (kernel == Int4Kernel::tiles_128x128) return 90.0 * k * rounds(128, 128) / 2.0;
     if (rounds(64, 64) >= 0.75) return 5.0 + (K >= 8192 ? 14.0 : 18.0) * k * up(rounds(64, 64));
     return 4.0 + 10.4 * k * up(rounds(32, 64));

@@ -363,6 +363,14 @@ def test_int4_ragged_weights_at_33_to_64_rows(M, N, K, group, tiled):
     assert rel <= 1e-3 and (y != want).float().mean() <= 0.01, rel
 
 
+def test_int4_tiles_where_their_k_parts_pay():
+    """Narrow weights at 65 and more rows: K parts of the 32-row tiles (us at 100 rows 10.7 on 512 x 4096, 12.5 on 1024 x 6144) against the tiles' eight
+    (11.4, 12.9), which are ahead from about 7000 of K on (512 x 8192 14.1 / 13.3)."""
+    for M, N, K, tiled in ((100, 512, 4096, False), (256, 512, 4096, False), (80, 1536, 4096, False), (100, 1024, 6144, False), (100, 512, 8192, True),
+                           (128, 1024, 14336, True)):
+        assert (_tiled_bytes("int4wo", M, N, K, 128) >= 0) == tiled, (M, N, K)
+
+
 @pytest.mark.parametrize("fmt,M,N,K,group,name", [
     ("int4", 1700, 7000, 512, 64, "int4wo_gemm_lds_kernel<64,2>"), ("int4", 1000, 6400, 512, 128, "int4wo_gemm_lds_kernel<128,1>"),
     ("int4", 300, 4100, 1024, 32, "int4wo_gemm_kwave_kernel"), ("int4", 2750, 1024, 4096, 64, ""), ("int4", 5000, 64, 256, 64, ""),
