@@ -735,9 +735,13 @@ static void launch_gemm_kwave(const LinearArgs& a, int64_t g, const GemmLdsPlan&
     }
 }
 
+// Activations that were copied by the launch in front are taken row by row: each XCD then reads an eighth of them, in panels a third to all,
+// and the copy, which reads behind the product of the call before, is slower too.  us a call, copy and product, in panels / row by row: 5088 x 2496 at
+// 1703 / 2300 rows 68.5 / 64.9, 75.1 / 72.7; 5920 x 2240 at 2048 / 3000 rows 67.5 / 65.5, 112.0 / 110.0; 4096 x 4032 at 2300 / 3000 rows 98.1 / 95.1,
+// 105.1 / 103.0; level up to 1500 rows.
 template <int NT>
-static void launch_gemm_lds_nt(const LinearArgs& a, int64_t g, const GemmLdsPlan& p, hipStream_t st) {
-    const TileOrder order = tile_order(p.tiles_m, p.tiles_n, 256 * 128, 128 * NT * 32);
+static void launch_gemm_lds_nt(const LinearArgs& a, int64_t g, const GemmLdsPlan& p, hipStream_t st, bool copied = false) {
+    const TileOrder order = copied ? TileOrder{p.tiles_m, p.tiles_n, 1} : tile_order(p.tiles_m, p.tiles_n, 256 * 128, 128 * NT * 32);
     const dim3 grid((unsigned)(order.per_xcd() * 8), (unsigned)a.ksplit), block(256);
     auto go = [&](auto kernel) {
         if (g_prof_start && g_prof_stop) {
@@ -761,11 +765,11 @@ void launch_int4wo_gemm_lds_parts(const LinearArgs& a, int64_t g, int nt, hipStr
     else launch_gemm_lds_nt<2>(a, g, p, st);
 }
 
-bool launch_int4wo_gemm_lds(const LinearArgs& a, int64_t g, hipStream_t st) {
+bool launch_int4wo_gemm_lds(const LinearArgs& a, int64_t g, hipStream_t st, bool copied) {
     GemmLdsPlan p;
     if (gemm_lds_plan(a, g, &p)) {
-        if (p.nt == 1) launch_gemm_lds_nt<1>(a, g, p, st);
-        else launch_gemm_lds_nt<2>(a, g, p, st);
+        if (p.nt == 1) launch_gemm_lds_nt<1>(a, g, p, st, copied);
+        else launch_gemm_lds_nt<2>(a, g, p, st, copied);
         return true;
     }
     if (gemm_kwave_plan(a, g, &p)) {

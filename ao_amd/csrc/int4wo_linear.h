@@ -151,6 +151,9 @@ struct Int4Plan {
 bool int4wo_plain_kernel(int64_t M, int64_t K, int64_t N, int64_t g, Int4Kernel* kernel);
 // Whether the dispatch reads activation rows of a multiple of 8 elements that end before the packed width as they are
 bool int4wo_takes_short_rows(int64_t M, int64_t N, int64_t g);
+// The plain product on contiguous rows of the packed width that a kernel on the same stream has just written: another order of the tiles
+int int4wo_linear_copied_rows(const void* x_bf16, int64_t M, int64_t K, const void* packed, const void* qparams, int64_t N, int64_t g,
+                              const void* bias_bf16, void* y, int y_dtype, int64_t ldy, void* stream);
 
 // Single-row GEMV on the 4x4x4 matrix instructions (int4wo_gemv1.hip).  Returns true when it took the launch;
 // false when the shape is outside what it handles (the caller then uses the general kernels).
@@ -165,7 +168,8 @@ bool launch_int4wo_gemv2(const LinearArgs& a, int64_t g, int64_t RB, hipStream_t
 bool int4wo_gemv2_plan(const LinearArgs& a, int64_t g, int64_t RB, char* out, size_t cap);
 
 // Prefill GEMM with the weight tile dequantized once per workgroup into LDS (int4wo_gemm.hip); same contract as above.
-bool launch_int4wo_gemm_lds(const LinearArgs& a, int64_t g, hipStream_t st);
+// `copied`: the activations were written by the launch in front.
+bool launch_int4wo_gemm_lds(const LinearArgs& a, int64_t g, hipStream_t st, bool copied);
 bool int4wo_gemm_lds_plan(const LinearArgs& a, int64_t g, Int4Plan* plan);
 // Its 256 x 128 nt tiles with K split over a.ksplit workgroups: a.y takes fp32 parts [ksplit][M][ldy], no bias.  K is the packed
 // width, every part has at least 8 of the 64-wide steps and a.ksplit is at most 4 (no part is empty then).

@@ -1170,7 +1170,7 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
                            const void* packed2, const void* qparams2, int64_t N, int64_t g, const void* bias_bf16,
                            const void* residual_bf16, int64_t ldres, void* y, int y_dtype, int64_t ldy, void* stream,
                            const void* norm_weight_bf16 = nullptr, float norm_eps = 0.f, bool pair8 = false,
-                           int ksplit = 1, Int4Plan* plan = nullptr) {
+                           int ksplit = 1, Int4Plan* plan = nullptr, bool copied = false) {
     // plan: do not launch; say which kernel the arguments select
 #define AO_PLAN(which, ...)                                             \
     if (plan) {                                                         \
@@ -1279,7 +1279,7 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
         (ws_tiles || (!gemm_starved && !rb4_two_blocks))) {
         if (!ws_tiles) {
             if (plan && int4wo_gemm_lds_plan(a, g, plan)) return 0;
-            if (!plan && launch_int4wo_gemm_lds(a, g, st)) {
+            if (!plan && launch_int4wo_gemm_lds(a, g, st, copied)) {
                 AO_LAUNCH_CHECK();
                 return 0;
             }
@@ -1443,6 +1443,12 @@ extern "C" int ao_amd_int4wo_linear(const void* x_bf16, int64_t M, int64_t K, in
                                     int y_dtype, int64_t ldy, void* stream) {
     return linear_dispatch(x_bf16, M, K, ldx, packed, qparams, nullptr, nullptr, N, g, bias_bf16, nullptr, 0, y, y_dtype,
                            ldy, stream);
+}
+
+int ao::int4wo_linear_copied_rows(const void* x_bf16, int64_t M, int64_t K, const void* packed, const void* qparams, int64_t N, int64_t g,
+                                  const void* bias_bf16, void* y, int y_dtype, int64_t ldy, void* stream) {
+    return linear_dispatch(x_bf16, M, K, K, packed, qparams, nullptr, nullptr, N, g, bias_bf16, nullptr, 0, y, y_dtype, ldy, stream, nullptr, 0.f,
+                           false, 1, nullptr, true);
 }
 
 // K split over workgroups through a caller's workspace: where it is used and how many parts.  The fp32 partial outputs

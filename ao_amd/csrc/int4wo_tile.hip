@@ -325,6 +325,7 @@ extern "C" int ao_amd_int4wo_linear_auto(const void* x_bf16, int64_t M, int64_t 
         if (int rc = ao_amd_pad_rows(x_bf16, M, K, ldx, r.Kp, workspace, stream)) return rc;
         x_bf16 = workspace;
         K = ldx = r.Kp;
+        if (!r.parts) return int4wo_linear_copied_rows(x_bf16, M, K, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, stream);
     }
     if (!r.parts) return ao_amd_int4wo_linear(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, stream);
     return ao_amd_int4wo_linear_ws(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, (uint8_t*)workspace + r.copy,

@@ -265,7 +265,7 @@ def test_int4_tiles_cover_every_shape_and_the_operator_takes_them():
 
 @pytest.mark.parametrize("M,N,K,group,shift", [
     (1, 14336, 4032, 64, 0), (1, 8192, 4100, 128, 0), (3, 4099, 4160, 32, 0), (16, 4096, 4041, 256, 0), (17, 4096, 4032, 256, 0), (33, 4100, 4160, 64, 0),
-    (300, 4096, 4100, 64, 0), (600, 14336, 1090, 128, 0),                    # rows that end before the packed width
+    (300, 4096, 4100, 64, 0), (600, 14336, 1090, 128, 0), (1703, 5088, 700, 64, 0),   # rows that end before the packed width
     (1, 14336, 4096, 64, 1), (9, 4096, 4096, 128, 3), (200, 4096, 4096, 64, 1),  # rows that are not 16-byte aligned
     (2, 64, 192, 64, 0), (1, 1024, 704, 64, 1),                              # too small for the copy to pay
 ])
