@@ -243,12 +243,13 @@ int ao_amd_hqq_mixed_mm_mfma(const void* a, int64_t M, int64_t lda, const void* 
                              int64_t N, const void* scales, const void* zeros, int64_t group_size, int dtype,
                              int transposed, void* workspace, int64_t workspace_bytes, void* y, void* stream);
 /* Both products for any number of rows on 32- to 96-row tiles: K and the group size multiples of 64, N of 16, every buffer
- * 16-byte aligned.  ao_amd_hqq_mixed_mm_tiled_bytes gives the workspace (0: none), or -1 for a shape that it does not take. */
+ * 16-byte aligned.  ao_amd_hqq_mixed_mm_tiled_bytes gives the workspace (0: none), or -1 for a shape that it does not take or that
+ * another route is expected to serve faster.  The product itself runs the latter too: with 16 x M x output columns floats of workspace in
+ * as many parts of the reduction as it likes, with less (or none) in one. */
 int ao_amd_hqq_mixed_mm_tiled_bytes(int64_t M, int64_t K, int64_t N, int64_t group_size, int dtype, int transposed, int64_t* bytes);
 int ao_amd_hqq_mixed_mm_tiled(const void* a, int64_t M, int64_t lda, const void* packed_2xint4, int is_signed, int64_t K, int64_t N,
                               const void* scales, const void* zeros, int64_t group_size, int dtype, int transposed, void* workspace,
                               int64_t workspace_bytes, void* y, void* stream);
-
 
 /* ---------------------------------------------------------------- int8 weight-only linear
  * y[M,N] = bf16( bf16(x[M,K] @ bf16(w)^T) * scale[N] ) (+ bias, rounded to bf16 again): the per-channel int8
