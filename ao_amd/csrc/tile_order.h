@@ -24,9 +24,7 @@ struct TileOrder {
 inline TileOrder tile_order(int64_t tiles_m, int64_t tiles_n, int64_t x_bytes, int64_t w_bytes) {
     const int64_t per_xcd = (tiles_m * tiles_n + 7) / 8, at_once = per_xcd < 32 ? per_xcd : 32;
     const double high = sqrt(2.0 * (double)at_once * (double)w_bytes / (double)x_bytes);
-    // (rounded up from .45 on: 7 tile rows of 256 in panels of 3 + 3 + 1, not 4 + 3: int4 5088 x 2560 at 1703 rows 58.9 / 61.2, 5920 x 2304 55.5 /
-    // 58.6, 11008 x 4096 162.6 / 164.4)
-    int64_t panels = high >= 1.0 ? (int64_t)((double)tiles_m / high + 0.55) : tiles_m;
+    int64_t panels = high >= 1.0 ? (int64_t)((double)tiles_m / high + 0.5) : tiles_m;
     panels = panels < 1 ? 1 : panels;
     return TileOrder{(int)tiles_m, (int)tiles_n, (int)((tiles_m + panels - 1) / panels)};
 }
