@@ -735,13 +735,17 @@ static void launch_gemm_kwave(const LinearArgs& a, int64_t g, const GemmLdsPlan&
     }
 }
 
+// Up to four tile rows in one panel (8192 x 8192 at 1000 rows 128.6 us, 142 in panels of two), more in panels of two, whose columns the 32 CUs of an XCD
+// take evenly.  Panels of three, tile_order's choice for 5, 6 and 8 and more rows, do not (us in panels of three or so / of two / row by row: 11008 x 4096 at
+// 1800 rows 181 / 175 / 177, 12288 x 4096 189 / 182 / 183, 8192 x 4096 at 2816 rows 182 / 177 / 178, 5920 x 2304 at 1500 rows 56.4 / 52.4 / 56.9), and 4 + 3 rows
+// are behind as well (5088 x 2560 at 1703 rows 61.2 / 59.1 / 59.0).
 // Activations that were copied by the launch in front are taken row by row: each XCD then reads an eighth of them, in panels a third to all,
 // and the copy, which reads behind the product of the call before, is slower too.  us a call, copy and product, in panels / row by row: 5088 x 2496 at
 // 1703 / 2300 rows 68.5 / 64.9, 75.1 / 72.7; 5920 x 2240 at 2048 / 3000 rows 67.5 / 65.5, 112.0 / 110.0; 4096 x 4032 at 2300 / 3000 rows 98.1 / 95.1,
 // 105.1 / 103.0; level up to 1500 rows.
 template <int NT>
 static void launch_gemm_lds_nt(const LinearArgs& a, int64_t g, const GemmLdsPlan& p, hipStream_t st, bool copied = false) {
-    const TileOrder order = copied ? TileOrder{p.tiles_m, p.tiles_n, 1} : tile_order(p.tiles_m, p.tiles_n, 256 * 128, 128 * NT * 32);
+    const TileOrder order{p.tiles_m, p.tiles_n, copied ? 1 : p.tiles_m <= 4 ? p.tiles_m : 2};
     const dim3 grid((unsigned)(order.per_xcd() * 8), (unsigned)a.ksplit), block(256);
     auto go = [&](auto kernel) {
         if (g_prof_start && g_prof_stop) {
