@@ -98,7 +98,15 @@ static const TileShape kInt8Shapes[] = {
 };
 
 TilePlan int8wo_gemm_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
-    return tile_plan(kInt8Shapes, (int)(sizeof(kInt8Shapes) / sizeof(kInt8Shapes[0])), M, N, K, max_parts);
+    TileShape shapes[7];
+    for (int i = 0; i < 7; ++i) shapes[i] = kInt8Shapes[i];
+    // (128 x 128 tiles take 8 % more for every K step of long rows: 5120 x 13824 at 640 rows 114 us, 128 x 256 in two K parts 106; 4096 x 14336 at 780 rows
+    // 120 / 113, at 400 rows in two parts 71.5, 128 x 256 in four 70.4; 8192 x 8192 at 512 rows 71)
+    if (K >= 8192) shapes[2].one = 37.5;
+    // (the figures above are those of a weight from memory; 96 x 128 tiles of a smaller one with long rows take less: 1024 x 8192 at 1280 / 1400 rows in two K parts 36.3 /
+    // 37.5 us, 192 x 128 in four 38.9 / 42.0; 2048 x 8192 at 700 rows 40.3 / 41.6, 2048 x 14336 at 290 rows 35.4 / 36.6)
+    if (K >= 8192 && N * K < ((int64_t)1 << 25)) shapes[1].one = 30.0;
+    return tile_plan(shapes, 7, M, N, K, max_parts);
 }
 
 void int8wo_gemm_describe(const TilePlan& p, char* out, size_t cap) {
