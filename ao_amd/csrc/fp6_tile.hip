@@ -89,7 +89,12 @@ static void launch_shape(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
 }
 
 static TilePlan fp6_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
-    return tile_plan(kFp6Shapes, (int)(sizeof(kFp6Shapes) / sizeof(kFp6Shapes[0])), M, N, K, max_parts);
+    // (a short lead of K parts over the whole K is none; us in the parts that the estimates prefer / whole: 8192 x 8192 at 65 / 96 rows, four of 96 x 128, 29.8 /
+    // 25.1, 32.4 / 26.5, 8192 x 7168 at 80 rows 27.4 / 22.7; two of 96 x 128: 6144 x 4096 at 140 rows 20.2 / 16.2, 5120 x 5120 at 256 rows 25.2 / 20.8; but
+    // 4096 x 14336 at 256 rows, four of 128 x 128, 43.0 / 44.2, 5120 x 13824 at 129 rows, two of 64 x 128, 36.9 / 39.2)
+    TilePartCost parts;
+    parts.lead = 0.89;
+    return tile_plan(kFp6Shapes, (int)(sizeof(kFp6Shapes) / sizeof(kFp6Shapes[0])), M, N, K, max_parts, parts);
 }
 
 // Whether the tiled product is the faster one.  The kernels of fp6.hip cost, by measurement at 33 to 1000 rows on 16 weights from

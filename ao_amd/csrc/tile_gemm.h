@@ -362,6 +362,7 @@ struct TilePlan {
 };
 struct TilePartCost {
     double launch = 1.5, doubling = 1.0, sums = 8.0;
+    double lead = 1.0;   // K parts have to take less than this share of the whole K's estimate
 };
 // us of one shape with K in `z` parts
 inline double tile_us(const TileShape& s, int64_t M, int64_t N, int64_t K, int z, const TilePartCost& c = TilePartCost()) {
@@ -377,7 +378,7 @@ inline double tile_us(const TileShape& s, int64_t M, int64_t N, int64_t K, int z
 }
 inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64_t N, int64_t K, int max_parts,
                           const TilePartCost& c = TilePartCost()) {
-    TilePlan best{-1, 1, 1e30};
+    TilePlan best{-1, 1, 1e30}, whole = best;
     const int64_t steps = K / 64;
     for (int i = 0; i < nshapes; ++i)
         for (int z = 1; z <= (max_parts < shapes[i].max_parts ? max_parts : shapes[i].max_parts); z *= 2) {
@@ -385,8 +386,9 @@ inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64
             if (z > 1 && (per < 8 || (z - 1) * per >= steps)) break;
             const double t = tile_us(shapes[i], M, N, K, z, c);
             if (t < best.us) best = TilePlan{i, z, t};
+            if (z == 1 && t < whole.us) whole = TilePlan{i, z, t};
         }
-    return best;
+    return best.us < c.lead * whole.us ? best : whole;
 }
 
 // The launches of a plan: tile_grid once, tile_launch with the shape's constants, tile_finish.
