@@ -3,7 +3,8 @@
 // A workgroup of WM x WN x KW waves computes a tile of 32 MT WM activation rows x 32 NT WN weight rows; a wave owns MT x NT blocks of
 // 32x32x16 matrix instructions.  With WM = 1 it has all rows of the tile, so every weight is dequantized once per tile.  192 x 128
 // tiles of int8 and FP6, whose dequantization is short, have WM = 2: twice the conversions, but two waves on a SIMD (int8
-// 192 rows, 14336 x 4096 46.0 -> 42.7 us, 333 rows 11008 x 4096 44.5 -> 42.1; FP6 40.6 -> 38.9, 41.7 -> 40.8; int4 45.9 -> 57.8, so not there.
+// 192 rows, 14336 x 4096 46.0 -> 42.7 us, 333 rows 11008 x 4096 44.5 -> 42.1, by this alone; with the rest below 45.9 -> 40.3; FP6 40.6 -> 38.9, 41.7 -> 40.8; int4
+// 45.9 -> 57.8, so not there.
 // 256 x 128, 192 x 256 and 256 x 256 tiles of that kind were no faster than what they would replace).  With KW > 1 the
 // groups of WN waves take the 64-wide K steps round-robin and add their accumulators through LDS at the end.  Both
 // operands of a step come into LDS by direct loads (no registers, no LDS store instructions) through a ring of STAGES

@@ -7,8 +7,8 @@
 // slice), with the tile rows dealt out evenly over that many panels.  Row by row (panel 1, all of one activation slice
 // first) the weight came once per tile row; measured us, row by row / in panels: int8 14336 x 4096 at 190 / 450 / 1149 rows
 // 35.4 / 34.0, 64.4 / 62.2, 138 / 134, 4096 x 14336 at 300 rows 57.6 / 51.2; FP6 14336 x 4096 at 80 / 450 rows 23.6 / 22.9, 63.9 / 60.6;
-// int4 5120 x 13824 at 427 rows 102.3 / 96.2 (counting the weight once 102.0), 14336 x 4096 at 2048 rows 216 / 211.  All
-// rows in one panel is too much for many short rows (int4 1024 x 4096 at 2750 rows, 29 tile rows: 34.6 / 36.6).
+// int4 5120 x 13824 at 427 rows 102.3 / 96.2 (counting the weight once 102.0).  All rows in one panel is too much for many short rows (int4 1024 x
+// 4096 at 2750 rows, 29 tile rows: 34.6 / 36.6).  The 256-row int4 tiles choose their own panels (int4wo_gemm.hip).
 #pragma once
 #include "common.h"
 #include <math.h>
