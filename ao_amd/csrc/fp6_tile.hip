@@ -32,7 +32,7 @@ struct Fp6Tile {
     }
     static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, int at, uint32_t off) {
         const uint8_t* const tile = a.w + (n0 / 16) * a.ldw + (uint32_t)((s >> 1) * 1536 + (s & 1) * (r == 0 ? 512 : 256));
-        tg_dma(lds, at, tile, off + (r == 0 ? 0 : 1024));
+        lds_dma16(lds, at, tile, off + (r == 0 ? 0 : 1024));
     }
     static __device__ __forceinline__ Row row(const TileGemmArgs& a, int64_t n) {
         const _Float16 s = __builtin_bit_cast(_Float16, ((const uint16_t*)a.scale)[n < a.N ? n : a.N - 1]);

@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "hqq_format.h"
+#include "lds_dma.h"
 
 namespace ao {
 
@@ -45,20 +46,6 @@ __device__ __forceinline__ void ht_for(F&& f) {
         f(std::integral_constant<int, B>{});
         ht_for<B + 1, E>(f);
     }
-}
-
-// global -> LDS, 16 (4) bytes a lane, from a scalar base and a 32-bit lane offset or from a lane's own address
-__device__ __forceinline__ void ht_dma(uint32_t lds, const void* base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
-}
-__device__ __forceinline__ void ht_dma4(uint32_t lds, const void* base, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
-}
-__device__ __forceinline__ void ht_dma(uint32_t lds, const void* p) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"((uint64_t)(uintptr_t)p), "s"(lds) : "memory");
-}
-__device__ __forceinline__ void ht_dma4(uint32_t lds, const void* p) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"((uint64_t)(uintptr_t)p), "s"(lds) : "memory");
 }
 
 template <bool BF16, bool SIGNED, bool TR, int MT>
@@ -126,35 +113,37 @@ __global__ __launch_bounds__(256) void hqq_tile_kernel(const HqqTileArgs g) {
     auto step_of = [&](int t) __attribute__((always_inline)) { return first + wave + W * (t < nst ? t : nst - 1); };
     auto request_a = [&](int j, int t, int slot) __attribute__((always_inline)) {
         const int s = step_of(t);
-        const uint32_t at = lds0 + slot * ASTEP + j * 1024;
+        const uint32_t to = lds0 + slot * ASTEP;
+        const int at = j * 1024;
         if (TR && s == tail) {
             const int chunk = (lane & 7) ^ (((8 * j + (lane >> 3)) >> 1) & 7);
             const uint8_t* const p = (const uint8_t*)(abase + (int64_t)s * 64) + aoff[j];
-            ht_dma(at, (int64_t)s * 64 + 8 * chunk < g.N ? p : (const uint8_t*)&hqq_zeros);
+            lds_dma16(to, at, (int64_t)s * 64 + 8 * chunk < g.N ? p : (const uint8_t*)&hqq_zeros);
         } else {
-            ht_dma(at, abase + (int64_t)s * 64, aoff[j]);
+            lds_dma16(to, at, abase + (int64_t)s * 64, aoff[j]);
         }
     };
     auto request_c = [&](int j, int t, int slot) __attribute__((always_inline)) {
         const int s = step_of(t);
-        const uint32_t at = lds0 + NA * ASTEP + slot * CSTEP + (j < 4 ? j * 1024 : 4096 + (j - 4) * 256);
+        const uint32_t to = lds0 + NA * ASTEP + slot * CSTEP;
+        const int at = j < 4 ? j * 1024 : 4096 + (j - 4) * 256;
         if (TR) {
             if (j < 4) {
                 const uint8_t* const base = cbase + (int64_t)s * 64;
                 const int chunk = (lane & 3) ^ (((16 * j + (lane >> 2)) >> 2) & 3);
                 // (codes past the end: the row's first ones of the step, with zero scales)
-                ht_dma(at, base, s == tail && (int64_t)s * 64 + 16 * chunk >= g.N ? coff[j] - 16 * chunk : coff[j]);
+                lds_dma16(to, at, base, s == tail && (int64_t)s * 64 + 16 * chunk >= g.N ? coff[j] - 16 * chunk : coff[j]);
             } else {
                 const uint16_t* const base = (j == 4 ? sbase : zbase) + (int64_t)s * 64;
                 if (s == tail)
-                    ht_dma4(at, (int64_t)s * 64 + 2 * r32 < g.N ? (const uint8_t*)base + soff : (const uint8_t*)&hqq_zeros);
+                    lds_dma4(to, at, (int64_t)s * 64 + 2 * r32 < g.N ? (const uint8_t*)base + soff : (const uint8_t*)&hqq_zeros);
                 else
-                    ht_dma4(at, base, soff);
+                    lds_dma4(to, at, base, soff);
             }
         } else if (j < 4) {
-            ht_dma(at, cbase + (int64_t)s * 32 * g.N, coff[j]);
+            lds_dma16(to, at, cbase + (int64_t)s * 32 * g.N, coff[j]);
         } else {
-            ht_dma4(at, (j == 4 ? sbase : zbase) + (int64_t)(g.per_group ? __umulhi((uint32_t)s, g.per_group) : (uint32_t)s) * g.N, soff);
+            lds_dma4(to, at, (j == 4 ? sbase : zbase) + (int64_t)(g.per_group ? __umulhi((uint32_t)s, g.per_group) : (uint32_t)s) * g.N, soff);
         }
     };
     auto a_at = [&](int slot) __attribute__((always_inline)) { return mine + slot * ASTEP; };

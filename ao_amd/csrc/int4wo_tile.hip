@@ -36,9 +36,9 @@ struct Int4Tile {
     }
     static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, int at, uint32_t off) {
         if (r == 0)
-            tg_dma(lds, at, a.w + (n0 / 16) * a.ldw + (uint32_t)s * 512u, off);
+            lds_dma16(lds, at, a.w + (n0 / 16) * a.ldw + (uint32_t)s * 512u, off);
         else
-            tg_dma4(lds, at, (const uint8_t*)a.scale + (n0 / 16) * (padded_k(a) >> a.group_shift) * 64 + (((uint32_t)s * 64u) >> a.group_shift) * 64u, off);
+            lds_dma4(lds, at, (const uint8_t*)a.scale + (n0 / 16) * (padded_k(a) >> a.group_shift) * 64 + (((uint32_t)s * 64u) >> a.group_shift) * 64u, off);
     }
     static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) {
         Row k;   // in registers, so that one instruction masks and inserts

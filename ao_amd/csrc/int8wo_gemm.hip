@@ -27,7 +27,7 @@ struct Int8Tile {
         return (uint32_t)(rel * a.ldw) + ((PAIR ? (lane & 7) ^ ((row >> 1) & 7) : (lane & 3) ^ ((row >> 2) & 3)) << 4);
     }
     static __device__ __forceinline__ void request(const TileGemmArgs& a, int64_t n0, int s, int r, uint32_t lds, int at, uint32_t off) {
-        tg_dma(lds, at, a.w + n0 * a.ldw + (uint32_t)s * 64u, off);
+        lds_dma16(lds, at, a.w + n0 * a.ldw + (uint32_t)s * 64u, off);
     }
     static __device__ __forceinline__ Row row(const TileGemmArgs&, int64_t) { return Row(); }
     static __device__ __forceinline__ Raw read(const uint8_t* block, int lane, bool odd) {

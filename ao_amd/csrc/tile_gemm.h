@@ -27,6 +27,7 @@
 // loop of 96 x 128 tiles from 273 to 224 instructions and 5120 x 13824 at 427 rows from 96.3 to 89.6 us, 4096 x 14336 at 1254 rows
 // from 179 to 164; int8 and FP6 loops are 5 to 10 % shorter and 0 to 2 % faster.
 #pragma once
+#include "lds_dma.h"
 #include "tile_order.h"
 #include <type_traits>
 
@@ -48,20 +49,10 @@ struct TileGemmArgs {
     float* parts;                       // K split over blockIdx.y: fp32 partial products [gridDim.y][M][N], or null
 };
 
-// 16 bytes per lane, global -> LDS: lane L of the wave lands at lds + at + 16 L, `at` a constant.  Scalar base + 32-bit byte
-// offset per lane.
-__device__ __forceinline__ void tg_dma(uint32_t lds, int at, const void* base, uint32_t off) {
-    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds), "i"(at) : "memory", "scc");
-}
 template <int N>
 __device__ __forceinline__ void tg_wait_barrier() {
     // lgkmcnt: this wave's reads of the buffer that the next requests overwrite have returned
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-// 4 bytes per lane
-__device__ __forceinline__ void tg_dma4(uint32_t lds, int at, const void* base, uint32_t off) {
-    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds), "i"(at) : "memory", "scc");
 }
 
 // A weight format F describes a block of 32 weight rows of one 64-wide K step:
@@ -140,7 +131,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void tile_gemm_kernel(const Tile
         if (weights)
             F::request(a, n0, s, NT % WM == 0 ? i % WREQ : wm * BREQ + i, lds_b + buf, i / WREQ * UNIT * F::BLOCK_BYTES + i % WREQ * 1024, boff[i]);
         else
-            tg_dma(lds_a + buf, i * 1024, (const uint8_t*)abase + (uint32_t)s * 128u, aoff[i]);
+            lds_dma16(lds_a + buf, i * 1024, (const uint8_t*)abase + (uint32_t)s * 128u, aoff[i]);
     };
 
     tg_f32x16 acc[MT][NT];
