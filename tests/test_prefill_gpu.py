@@ -24,7 +24,7 @@ def _qkv(T, n_head, n_kv, dtype, seed=0):
     return torch.randn(T, (n_head + 2 * n_kv) * 128, device="cuda", generator=g).to(dtype)
 
 
-# tile edges: 32 query rows a wave (128 a workgroup when the waves share a head), 64 positions a tile
+# tile edges: 32 query rows a wave (64 a workgroup when the waves share a head), 32 positions a tile, every fourth one a group's
 @pytest.mark.parametrize("T", [2, 31, 32, 33, 64, 65, 127, 129, 200])
 @pytest.mark.parametrize("heads", [(8, 2), (8, 1), (3, 3), (4, 2)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -100,6 +100,49 @@ def test_add_rmsnorm_and_silu_mul(rows, dim, dtype):
         want = F.silu(x) * y
         _call("ao_amd_silu_mul", x, y, int(dtype is torch.float16), rows * dim, x)  # in place over the gate
         assert ((x.float() - want.float()).abs() <= 2 * step * want.float().abs() + 2 ** -24).all() and (x != want).float().mean() <= 0.02
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_silu_mul_over_all_values(dtype):
+    """Every finite 16-bit gate and the special ones, times one.  fp32 within a few steps of 2^-24, rounded once: one step of the type at most,
+    few values off; below 2^-100 an absolute bound (F.silu's own e^-x overflows there)."""
+    x = torch.arange(65536, device="cuda", dtype=torch.int32).to(torch.int16).view(dtype)
+    want = (x.double() / (1 + torch.exp(-x.double()))).to(dtype)
+    out = torch.empty_like(x)
+    _call("ao_amd_silu_mul", x, torch.ones_like(x), int(dtype is torch.float16), x.numel(), out)
+    assert torch.equal(out.isnan(), want.isnan())
+    ok = ~want.isnan()
+    a, b = out[ok].double(), want[ok].double()
+    infinite = b.isinf()
+    assert torch.equal(a[infinite], b[infinite])
+    a, b = a[~infinite], b[~infinite]
+    step = 2.0 ** (-7 if dtype is torch.bfloat16 else -10)
+    assert ((a - b).abs() <= step * b.abs() + (2.0 ** -100 if dtype is torch.bfloat16 else 2.0 ** -24)).all() and (a != b).double().mean() <= 0.02
+
+
+@pytest.mark.parametrize("rise", [0.4, 6.0, 60.0])
+@pytest.mark.parametrize("heads,dtype", [((4, 2), torch.bfloat16), ((3, 3), torch.float16)])
+def test_attention_with_rising_scores(rise, heads, dtype):
+    """Scores that grow by `rise` every 32 positions, so that a row's maximum passes the kept one by less than 2^8 or by far more in
+    every tile; and the same ones falling.  Bound as in test_attention_matches_fp32, doubled for the sums of few large terms."""
+    n_head, n_kv = heads
+    T = S = 321
+    qkv = _qkv(T, n_head, n_kv, dtype) * 0.25
+    qkv.view(T, -1, 128)[:, :n_head, 0] = 8.0   # the queries' share of the ramp
+    freqs = torch.zeros(S, 64, 2, device="cuda", dtype=dtype)
+    freqs[..., 0] = 1.0                         # no rotation
+    pos = torch.arange(T, device="cuda")
+    for sign in (1, -1):
+        qkv.view(T, -1, 128)[:, n_head:n_head + n_kv, 0] = (sign * rise * math.sqrt(128) / 8.0 / 32 * pos)[:, None].to(dtype)
+        kc, vc = (torch.zeros(n_kv, S, 128, device="cuda", dtype=dtype) for _ in range(2))
+        out = torch.empty(T, n_head * 128, device="cuda", dtype=dtype)
+        _call("ao_amd_llama_prefill_attention", qkv, int(dtype is torch.float16), freqs, pos, 1, T, kc, vc, n_head, n_kv, 128, S, out)
+        later = torch.ones(T, T, device="cuda", dtype=torch.bool).triu(1)
+        for h in range(n_head):
+            kv = h * n_kv // n_head
+            s = (qkv.view(T, -1, 128)[:, h].float() @ kc[kv].float().t().contiguous() / math.sqrt(128)).masked_fill_(later, float("-inf"))
+            want = s.softmax(-1) @ vc[kv].float()
+            assert _rel(out.view(T, n_head, 128)[:, h], want) <= 2 * (2 ** -8 if dtype is torch.bfloat16 else 2 ** -11)
 
 
 @pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
@@ -184,7 +227,7 @@ def test_attention_with_negative_positions(T, heads, dtype, long):
 @pytest.mark.parametrize("T,heads", [(1025, (8, 2)), (4096, (4, 1)), (2049, (3, 3))])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_long_attention_matches_fp32(T, heads, dtype):
-    """As test_attention_matches_fp32, over 17 to 65 tiles of positions; one query head at a time in fp32."""
+    """As test_attention_matches_fp32, over 33 to 128 tiles of positions; one query head at a time in fp32."""
     from ao_amd._models.llama.model import apply_rotary_emb, precompute_freqs_cis
 
     n_head, n_kv = heads
