@@ -256,31 +256,46 @@ __device__ __forceinline__ hqq_f32x4_t hqq_mfma(const u32x4_t a, const uint32_t 
     }
 }
 
-// One wave's run of steps, loaded one ahead into two fragment sets that are used in turn (a copy from the one to the other was
-// a seventh of the loop).  COPY: where the two halves together need more registers than they save time.
-template <class Frag, bool COPY, class Load, class Compute>
+// One wave's run of steps, loaded AHEAD steps ahead into AHEAD + 1 fragment sets that are used in turn (a copy from the one to the other
+// was a seventh of the loop).  `load` makes the same requests whatever the step (past the end the last one's again): behind requests under a
+// condition the compiler waits for every request of the wave, and with them each step took the latency of its successor's: one row of 14336 x
+// 4096 19.3 -> 16.3 us, 16 rows 20.6 -> 18.4, 32 rows of 5120 x 5120 15.2 -> 13.0.
+// AHEAD 0: one ahead, with the copy and nothing requested past the end, for the short runs of 64 rows (14 requests a step: 1024 x
+// 4096 transposed 11.1 -> 10.2 us).
+template <class Frag, int AHEAD, class Load, class Compute>
 __device__ __forceinline__ void hqq_run(int s0, int s1, const Load& load, const Compute& compute) {
-    Frag fa, fb;
-    load(s0, fa);
-    if (COPY) {
-        for (int s = s0; s < s1; ++s) {
-            load(s + 1, fb);
-            compute(s, fa);
-            fa = fb;
+    constexpr int SETS = AHEAD + 1;
+    if (s0 >= s1) return;
+    if constexpr (AHEAD == 0) {
+        Frag now, next;
+        load(s0, now);
+        for (int s = s0; s + 1 < s1; ++s) {
+            load(s + 1, next);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(s, now);
+            now = next;
         }
-        return;
+        return compute(s1 - 1, now);
     }
-    for (int s = s0; s < s1; s += 2) {
-        load(s + 1, fb);
-        compute(s, fa);
-        if (s + 1 >= s1) break;
-        load(s + 2, fa);
-        compute(s + 1, fb);
+    Frag f[SETS];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+        load(s0 + i < s1 ? s0 + i : s1 - 1, f[i]);
+        __builtin_amdgcn_sched_barrier(0);
     }
+    for (int s = s0; s < s1; s += SETS)
+#pragma unroll
+        for (int i = 0; i < SETS; ++i) {
+            if (s + i >= s1) return;
+            load(s + i + AHEAD < s1 ? s + i + AHEAD : s1 - 1, f[(i + AHEAD) % SETS]);
+            __builtin_amdgcn_sched_barrier(0);
+            compute(s + i, f[i]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 }
 
 // Waves of a workgroup: each takes a run of the reduction, and they add up in LDS.  A step's loads take a microsecond and a
-// wave keeps one step ahead in flight, so the runs are kept short (2 - 4 steps) and the waves many; eight of them to a
+// wave keeps one or two steps ahead in flight, so the runs are kept short and the waves many; eight of them to a
 // workgroup keep the number of fp32 partial sums in memory where four waves with runs of eight steps had it.
 
 // RB (transposed product): blocks of 16 byte rows per wave.  With two of them in one quantization group the activation
@@ -314,36 +329,44 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
     const u32x4_t zero4 = {0u, 0u, 0u, 0u};
 
     if (!TRANSPOSED) {
-        const int64_t n0 = (int64_t)blockIdx.x * 64 + 4 * j;
-        const bool live = n0 < N;   // N is a multiple of 4
-        struct Frag { uint32_t d[4]; u32x4_t x[MB]; };
-        int64_t g_cur = -1;
-        uint32_t sv[4] = {0u, 0u, 0u, 0u}, zv[4] = {0u, 0u, 0u, 0u};   // a column's value twice
-        float sf[4] = {0.f, 0.f, 0.f, 0.f}, zf[4] = {0.f, 0.f, 0.f, 0.f};
-        auto load = [&](int s, Frag& f) {
-            const int64_t k2 = (int64_t)s * 16 + 4 * q4;
-            const bool ok = s < s1 && k2 < K2;   // K is a multiple of 8: the lane's 4 byte rows exist together
+        // columns past N (a multiple of 4) repeat the last ones and are not stored
+        const int64_t n_at = (int64_t)blockIdx.x * 64 + 4 * j, n0 = n_at < N ? n_at : N - 4;
+        struct Frag { uint32_t d[4]; uint2 s, z; u32x4_t x[MB]; };
+        const uint32_t eighths = (uint32_t)(group / 8);
+        const int shift = (eighths & (eighths - 1)) == 0 ? __builtin_ctz(eighths) : -1;
+        const int tail = K2 % 16 ? steps - 1 : -1;   // the step that ends before its 16 byte rows
+        auto load = [&](int s, Frag& f) __attribute__((always_inline)) {
+            const int64_t at = (int64_t)s * 16 + 4 * q4, k2 = at < K2 ? at : K2 - 4;   // K is a multiple of 8: the lane's 4 byte rows exist together
+            // group is a multiple of 8: one group for the lane's 8 k
+            const uint32_t eighth = (uint32_t)k2 >> 2;
+            const int64_t g = shift >= 0 ? eighth >> shift : eighth / eighths;
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                f.d[r] = ok && live ? *reinterpret_cast<const uint32_t*>(packed + (k2 + r) * N + n0) : 0u;
+            for (int r = 0; r < 4; ++r) f.d[r] = *reinterpret_cast<const uint32_t*>(packed + (k2 + r) * N + n0);
+            f.s = *reinterpret_cast<const uint2*>(scales + g * N + n0);
+            f.z = *reinterpret_cast<const uint2*>(zeros + g * N + n0);
 #pragma unroll
-            for (int mb = 0; mb < MB; ++mb) f.x[mb] = ok ? *reinterpret_cast<const u32x4_t*>(arow[mb] + 2 * k2) : zero4;
+            for (int mb = 0; mb < MB; ++mb) f.x[mb] = *reinterpret_cast<const u32x4_t*>(arow[mb] + 2 * k2);
         };
-        auto compute = [&](int s, const Frag& f) {
-            const int64_t k2 = (int64_t)s * 16 + 4 * q4;
-            const int64_t g = (2 * k2) / group;   // group is a multiple of 8: one group for the lane's 8 k
-            if (g != g_cur && live && s < s1 && k2 < K2) {
-                g_cur = g;
-                const uint2 s2 = *reinterpret_cast<const uint2*>(scales + g * N + n0);
-                const uint2 z2 = *reinterpret_cast<const uint2*>(zeros + g * N + n0);
-                const uint32_t ss[2] = {s2.x, s2.y}, zz[2] = {z2.x, z2.y};
+        auto compute = [&](int s, Frag& f) __attribute__((always_inline)) {
+            if (s == tail && (int64_t)s * 16 + 4 * q4 >= K2) {   // 0 x (0 - 0) * 0
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
+                for (int r = 0; r < 4; ++r) f.d[r] = 0u;
+                f.s = f.z = uint2{0u, 0u};
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) f.x[mb] = zero4;
+            }
+            uint32_t sv[4], zv[4];   // a column's value twice
+            float sf[4], zf[4];
+            const uint32_t ss[2] = {f.s.x, f.s.y}, zz[2] = {f.z.x, f.z.y};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if constexpr (BF16) {
+                    sf[c] = __uint_as_float(c & 1 ? ss[c >> 1] & 0xffff0000u : ss[c >> 1] << 16);
+                    zf[c] = __uint_as_float(c & 1 ? zz[c >> 1] & 0xffff0000u : zz[c >> 1] << 16);
+                } else {
                     const uint32_t sh = (c & 1) ? ss[c >> 1] >> 16 : ss[c >> 1] & 0xffffu, zh = (c & 1) ? zz[c >> 1] >> 16 : zz[c >> 1] & 0xffffu;
                     sv[c] = sh | (sh << 16);
                     zv[c] = zh | (zh << 16);
-                    sf[c] = __uint_as_float(sh << 16);
-                    zf[c] = __uint_as_float(zh << 16);
                 }
             }
             uint32_t lo[4], hi[4], w[4][4];   // w: [column][byte row]
@@ -366,7 +389,7 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
             column(std::integral_constant<int, 2>());
             column(std::integral_constant<int, 3>());
         };
-        hqq_run<Frag, (MB >= 2)>(s0, s1, load, compute);
+        hqq_run<Frag, MB == 4 ? 0 : MB == 2 ? 1 : 2>(s0, s1, load, compute);
     } else {
         int64_t k2[RB];
         bool live[RB];
@@ -378,28 +401,58 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
             prow[rb] = packed + (live[rb] ? k2[rb] : 0) * N;
         }
         const int64_t g = live[0] ? (2 * k2[0]) / group : 0;   // RB == 2: the host has checked that both blocks share it
+        const int64_t g_block = (int64_t)blockIdx.x * 32 * RB / group;   // of the block's first row, which exists
         const uint16_t* srow = scales + g * N;
         const uint16_t* zrow = zeros + g * N;
-        struct Frag { u32x4_t d[RB], s[2], z[2], x[MB][2]; };
-        auto load = [&](int s, Frag& f) {
-            const int64_t n = (int64_t)s * 64 + 16 * q4;
-            const bool ok = s < s1 && n < N;   // N is a multiple of 16
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) f.d[rb] = ok && live[rb] ? *reinterpret_cast<const u32x4_t*>(prow[rb] + n) : zero4;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                f.s[h] = ok ? *reinterpret_cast<const u32x4_t*>(srow + n + 8 * h) : zero4;
-                f.z[h] = ok ? *reinterpret_cast<const u32x4_t*>(zrow + n + 8 * h) : zero4;
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb)
-                    f.x[mb][h] = ok ? *reinterpret_cast<const u32x4_t*>(arow[mb] + n + 8 * h) : zero4;
-            }
+        struct Frag { u32x4_t d[RB], x[MB][2]; };
+        const int tail = N % 64 ? steps - 1 : -1;   // the step that ends before its 64 columns
+        auto column = [&](int s) {
+            const int64_t at = (int64_t)s * 64 + 16 * q4;
+            return at < N ? at : N - 16;   // N is a multiple of 16
         };
-        auto compute = [&](int, const Frag& f) {
+        auto load = [&](int s, Frag& f) __attribute__((always_inline)) {
+            const int64_t n = column(s);
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) f.d[rb] = *reinterpret_cast<const u32x4_t*>(prow[rb] + n);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) f.x[mb][h] = *reinterpret_cast<const u32x4_t*>(arow[mb] + n + 8 * h);
+        };
+        const HqqRowMatrices rows(lane);
+        auto compute = [&](int s, Frag& f, u32x4_t (&sc)[2], u32x4_t (&ze)[2], auto element_wise) __attribute__((always_inline)) {
+            if (s == tail && (int64_t)s * 64 + 16 * q4 >= N) {   // 0 x (0 - 0) * 0
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) f.d[rb] = zero4;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    sc[h] = ze[h] = zero4;
+#pragma unroll
+                    for (int mb = 0; mb < MB; ++mb) f.x[mb][h] = zero4;
+                }
+            }
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const uint32_t ss[4] = {f.s[h].x, f.s[h].y, f.s[h].z, f.s[h].w};
-                const uint32_t zz[4] = {f.z[h].x, f.z[h].y, f.z[h].z, f.z[h].w};
+                if constexpr (BF16 && !decltype(element_wise)::value) {
+                    HqqRowScales sz[2];   // of indices 8 h .. + 3, + 4 .. + 7
+                    sz[0] = rows.scales(sc[h].x, sc[h].y, ze[h].x, ze[h].y);
+                    sz[1] = rows.scales(sc[h].z, sc[h].w, ze[h].z, ze[h].w);
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb) {
+                        const uint32_t dd[4] = {f.d[rb].x, f.d[rb].y, f.d[rb].z, f.d[rb].w};
+                        uint32_t lo[4], hi[4];
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) rows.template weights<SIGNED>(dd[2 * h + i], sz[i], lo[2 * i], lo[2 * i + 1], hi[2 * i], hi[2 * i + 1]);
+#pragma unroll
+                        for (int mb = 0; mb < MB; ++mb) {
+                            acc[mb][2 * rb] = hqq_mfma<BF16>(f.x[mb][h], lo, acc[mb][2 * rb]);
+                            acc[mb][2 * rb + 1] = hqq_mfma<BF16>(f.x[mb][h], hi, acc[mb][2 * rb + 1]);
+                        }
+                    }
+                    continue;
+                }
+                const uint32_t ss[4] = {sc[h].x, sc[h].y, sc[h].z, sc[h].w};
+                const uint32_t zz[4] = {ze[h].x, ze[h].y, ze[h].z, ze[h].w};
                 float sf[8], zf[8];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
@@ -436,7 +489,75 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
                 }
             }
         };
-        hqq_run<Frag, MB == 4>(s0, s1, load, compute);
+        // Where all 16 byte rows of a block share their group, a wave brings the scales and zeros of its columns into LDS, CHUNK steps at a
+        // time: read by each lane they were 4 of the 8 (16 rows) to 14 (64 rows) requests of a step, for a sixteenth of their bytes, and a CU takes
+        // some 45 bytes a cycle of them (32 rows x 4096 x 11008 of bf16 / fp16 with the unconditional requests alone 18.5 / 18.9 us, with this 16.2 / 16.9).
+        constexpr int CHUNK = NACC * 4;   // 256 bytes a step, in the wave's own part of what the waves add up in later
+        uint16_t* const s_lds = reinterpret_cast<uint16_t*>(&red[wave][0][0]);
+        uint16_t* const z_lds = s_lds + CHUNK * 64;
+        bool direct = group % 32 != 0;
+        if (!direct) {
+            for (int c0 = s0; c0 < s1; c0 += CHUNK) {
+                const int c1 = c0 + CHUNK < s1 ? c0 + CHUNK : s1;
+                const int64_t n_end = (int64_t)c1 * 64 < N ? (int64_t)c1 * 64 : N;
+                u32x4_t in[2][CHUNK / 8];
+#pragma unroll
+                for (int i = 0; i < CHUNK / 8; ++i) {
+                    const int64_t at = (int64_t)c0 * 64 + i * 512 + lane * 8, n = at < n_end ? at : n_end - 8;
+                    in[0][i] = *reinterpret_cast<const u32x4_t*>(scales + g_block * N + n);
+                    in[1][i] = *reinterpret_cast<const u32x4_t*>(zeros + g_block * N + n);
+                }
+#pragma unroll
+                for (int i = 0; i < CHUNK / 8; ++i) {
+                    *reinterpret_cast<u32x4_t*>(s_lds + i * 512 + lane * 8) = in[0][i];
+                    *reinterpret_cast<u32x4_t*>(z_lds + i * 512 + lane * 8) = in[1][i];
+                }
+                asm volatile("" ::: "memory");   // (one wave: its LDS operations are done in order)
+                hqq_run<Frag, MB == 4 ? 0 : MB == 2 ? 1 : 2>(c0, c1, load, [&](int s, Frag& f) __attribute__((always_inline)) {
+                    const uint16_t* const at = s_lds + (s - c0) * 64 + 16 * q4;
+                    u32x4_t sc[2], ze[2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        sc[h] = *reinterpret_cast<const u32x4_t*>(at + 8 * h);
+                        ze[h] = *reinterpret_cast<const u32x4_t*>(at + CHUNK * 64 + 8 * h);
+                    }
+                    compute(s, f, sc, ze, std::integral_constant<bool, !BF16>());
+                });
+                asm volatile("" ::: "memory");
+            }
+        }
+        if (BF16 && !direct) {
+            bool nan = false;
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int c = 0; c < NACC; ++c)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        acc[mb][c][r] *= HqqRowMatrices::DOWN;
+                        nan |= acc[mb][c][r] != acc[mb][c][r];
+                    }
+            if (__any(nan)) {   // an infinite zero may have reached its neighbours
+                direct = true;
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                    for (int c = 0; c < NACC; ++c) acc[mb][c] = hqq_f32x4_t{0.f, 0.f, 0.f, 0.f};
+            }
+        }
+        if (direct)
+            for (int s = s0; s < s1; ++s) {
+                Frag f;
+                u32x4_t sc[2], ze[2];
+                load(s, f);
+                const int64_t n = column(s);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    sc[h] = *reinterpret_cast<const u32x4_t*>(srow + n + 8 * h);
+                    ze[h] = *reinterpret_cast<const u32x4_t*>(zrow + n + 8 * h);
+                }
+                compute(s, f, sc, ze, std::true_type());
+            }
     }
 
     // the waves of the workgroup add up, one block of 16 rows at a time: thread (wave w < 4, lane) sums element r = w of

@@ -419,19 +419,19 @@ HqqTilePlan hqq_tile_plan(int64_t M, int64_t K, int64_t N, int64_t group, bool t
 // 5120 x 5120 49 / 30, 44 / 47; 8192 x 8192 92 / 50, 96 / 84, 106 / 135 at 448), and a little on wide weights forward (4096 x 14336 at 448 rows 95 / 98,
 // 4096 x 32000 of fp16 at 512 193 / 198).
 // Up to 64 rows the other one is the streaming kernel of hqq.hip, timed against the tiles on 14 weights (K x N below, us streamed / tiled).
-// Forward from 17 rows on the size of the weight decides (17 rows of bf16: 4096 x 4096 11.0 / 12.1, 5120 x 5120 13.2 / 14.0, 4096 x 8192 14.5 / 12.9,
-// 5120 x 13824 31.5 / 21.2; 33 rows 5120 x 5120 16.2 / 16.4, 4096 x 6144 17.2 / 15.1).  With fewer rows, and transposed, the tiles' own time
-// does too: 5120 output columns are 40 tiles, which fill the CUs badly whatever the K parts.  One row of bf16 8192 x 28672 53.8 / 49.3,
-// 4096 x 32000 41.0 / 27.1, 8192 x 8192 20.4 / 19.2, but 13824 x 5120 23.1 / 26.6; transposed at 33 / 64 rows of bf16 8192 x 28672 72 / 67, 90 / 67,
-// 4096 x 14336 24.0 / 24.9, 28.6 / 25.3, but 5120 x 13824 28.3 / 42.4, 35.5 / 37.8, 4096 x 8192 17.3 / 19.3, 20.5 / 20.2; of fp16 at 17 / 32 rows 8192 x
-// 28672 48 / 43, 59 / 44, but 5120 x 13824 20.0 / 24.9, 22.9 / 25.3.  The streaming kernel's time is therefore estimated, from those weights:
+// Forward from 17 rows on the size of the weight decides, between 25 and 32 rows its shape as well (17 rows of bf16: 4096 x 4096 9.5 / 12.1, 11008 x
+// 4096 16.2 / 19.0, 4096 x 14336 20.2 / 19.1, 5120 x 13824 23.4 / 21.5; 32 rows 11008 x 4096 18.1 / 19.3, 4096 x 11008 19.5 / 18.8; 33 rows 5120 x 5120 14.1 / 16.6;
+// 64 rows 4096 x 6144 of fp16 17.4 / 16.8).  With fewer rows, and transposed, the tiles' own time does too: 5120 output columns are 40 tiles, which
+// fill the CUs badly whatever the K parts.  One row of bf16 4096 x 32000 30.1 / 27.2, 8192 x 8192 18.5 / 20.4, 8 rows 8192 x 28672 54.1 / 48.4; transposed at
+// 33 / 64 rows of bf16 8192 x 28672 60.7 / 65.6, 77.2 / 66.7, 14336 x 4096 23.2 / 25.0, 28.3 / 26.4; of fp16 at 32 rows 8192 x 28672 56.0 / 46.4, 13824 x 5120
+// 25.2 / 22.4.  The streaming kernel's time is therefore estimated, from those weights:
 // a part for every weight, one for every weight and row (the activations are read again for every 64 columns), the fp32 sums; the tiles' estimate
 // is 5 to 8 % long.
 HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed, bool bf16) {
     const HqqTilePlan none{0, 0, 0, 1, 1e30};
     const double weights = (double)K * (double)N, rows = (double)M, flops = 2.0 * rows * weights;
     // the size of the weight first: a plan takes a tenth of a microsecond of host time, which bounds calls on small weights
-    if (weights < (M > 64 ? 0.0 : !transposed ? (M > 32 ? 2e7 : M > 16 ? 3e7 : 6.4e7) : M > 32 ? (bf16 ? 4e7 : 2e7) : M > 16 && !bf16 ? 6.4e7 : 1e30)) return none;
+    if (weights < (M > 64 ? 0.0 : !transposed ? (M > 48 ? 2e7 : M > 32 ? 3e7 : M <= 16 ? 6.4e7 : M > 24 && N > K ? 3.5e7 : 5e7) : M > 32 ? (bf16 ? 4e7 : 2e7) : M > 16 && !bf16 ? 6.4e7 : 1e30)) return none;
     const HqqTilePlan p = hqq_tile_plan(M, K, N, group, transposed, bf16);
     if (!p.rows) return none;
     double other = 1e30, lead = 1.0;
@@ -443,9 +443,10 @@ HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool 
         if (transposed && 2 * N <= 3 * K && weights < 1e8) other = std::min(other, 20.0 + 0.61e-6 * weights + rows * (0.0016e-6 * weights - 0.009));
     } else if (transposed) {
         other = 5.6 + ((bf16 ? 0.18 : 0.14) + (bf16 ? 0.0022 : 0.0028) * rows) * weights * 1e-6 + (bf16 ? 0.065 : 0.055) * rows + 4.5e-6 * rows * (double)K;
+        if (bf16) other *= 0.88;
         lead = bf16 ? 0.92 : 0.95;
     } else if (M <= 16) {
-        other = 6.2 + ((bf16 ? 0.22 : 0.2) + (bf16 ? 0.0011 : 0.0015) * rows) * weights * 1e-6;
+        other = 0.92 * (6.2 + ((bf16 ? 0.22 : 0.2) + (bf16 ? 0.0011 : 0.0015) * rows) * weights * 1e-6);
         lead = 0.92;
     }
     return lead * p.us < other ? p : none;

@@ -432,3 +432,25 @@ def test_small_product_with_a_workspace_of_four_byte_alignment():
     check(lib().ao_amd_hqq_mixed_mm(x.data_ptr(), M, K, K, packed.data_ptr(), 0, N, s.data_ptr(), z.data_ptr(), g, BF16, ws[1:].data_ptr(),
                                     need.value, y.data_ptr(), current_stream(x.device)))
     assert torch.equal(y, ops.hqq_mixed_mm_small(x, packed, s, z, g))
+
+
+@pytest.mark.parametrize("special", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("M,N,K,g", [(1, 80, 64, 8), (17, 1008, 192, 64), (40, 528, 320, 32)])
+def test_transposed_product_with_a_special_zero(M, N, K, g, special):
+    """A zero that is no finite number makes its own weights special, and so the outputs of its group, as the formula has it: infinite
+    of the other sign times the activation.  The other groups' outputs are those of the finite weight, bit for bit."""
+    from ao_amd import ops
+    from ao_amd.prototype.hqq import pack_2xint4
+
+    dev = _dev()
+    W_q, scale, zero = _hqq_like(N, K, g, torch.bfloat16, seed=N, signed=False)
+    packed, s, z = pack_2xint4(W_q.T.contiguous()).to(dev), scale.T.contiguous().abs().to(dev), zero.T.contiguous().to(dev)
+    x = torch.randn(M, N, generator=torch.Generator().manual_seed(5)).bfloat16().to(dev)
+    x = torch.where(x == 0, 1.0, x)
+    finite = ops.hqq_mixed_mm_mfma(x, packed, s, z, g, True)
+    at = K // g - 1
+    z[at, 6] = special
+    y = ops.hqq_mixed_mm_mfma(x, packed, s, z, g, True)
+    assert torch.equal(y[:, : at * g], finite[:, : at * g]) and not finite.isnan().any()
+    want = (-special * x[:, 6:7].float()).expand(M, g)
+    assert torch.equal(y[:, at * g :].float().nan_to_num(7.0), want.nan_to_num(7.0))
