@@ -358,7 +358,9 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_kernel(const LinearA
 // tile once and runs them against the tiles of four row blocks: a quarter of the activation traffic, four accumulators.
 // EDGE: activation rows that end before the packed width, and row blocks that are no multiple of four (the tests of both cost the
 // others 2 to 5 %).
-template <int G, int WAVES, int MB, bool EDGE>
+// AHEAD: the next tile is requested before the present one is multiplied, for launches that leave one workgroup to a CU: 14336 x 4096 at 6 / 16 rows
+// 12.6 -> 11.4, 13.8 -> 13.2 us, 13824 x 8192 at 6 rows 22.5 -> 20.4, 12288 x 4096 12.8 -> 11.6.  From 17 rows on (two blocks) it gave nothing.
+template <int G, int WAVES, int MB, bool EDGE, bool AHEAD = false>
 __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const LinearArgs a) {
     // MB 16-row blocks of activations per workgroup (17 to 32 rows with MB = 2): every dequantized dword then feeds MB
     // matrix instructions, and the dequantization, which bounds the kernel, is done once for all of them
@@ -411,7 +413,9 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
         }
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
-            if (xact[mb]) load_x_tile<EDGE>(b.x[mb], xp[mb], kb, qd, a.K);
+            // (AHEAD: behind requests under a condition the compiler waits for all of them, the next tile's too; what the lanes of
+            // rows past M, which read row 0, add up is not stored)
+            if (AHEAD || xact[mb]) load_x_tile<EDGE>(b.x[mb], xp[mb], kb, qd, a.K);
     };
     u32x4_t tcur = {0, 0, 0, 0};
     // one tile = 16 dwords per lane (4 row blocks x 4); the three dequantization stages run as in int4wo_linear_kernel
@@ -442,7 +446,7 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
         }
     };
 
-    // One tile buffer and no look-ahead: with a second buffer the kernel needs 160 to 200 registers, which leaves one
+    // Otherwise one tile buffer and no look-ahead: with a second buffer the kernel needs 160 to 200 registers, which leaves one
     // 8-wave workgroup per CU; with one it needs 105 to 140, and the second workgroup on the CU hides the load latency
     // better than the look-ahead did (14336 x 4096 at 4-16 rows 14.2 -> 13.9 us; 28672 x 4096, 448 workgroups, 24 -> 21;
     // the vocabulary head 81 -> 71).
@@ -457,9 +461,23 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
 #pragma unroll
         for (int sl = 0; sl < 4; ++sl) buf.x[mb][sl] = make_uint4(0, 0, 0, 0);   // rows >= M keep these zeros
     const int nt = wave < KB ? (KB - wave + WAVES - 1) / WAVES : 0;
-    for (int i = 0; i < nt; ++i) {
-        load_tile(buf, wave + i * WAVES);
-        compute_tile(buf);
+    if constexpr (AHEAD) {
+        if (nt > 0) {
+            load_tile(buf, wave);
+            for (int i = 1; i < nt; ++i) {
+                Buf next;
+                load_tile(next, wave + i * WAVES);
+                __builtin_amdgcn_sched_barrier(0);
+                compute_tile(buf);
+                buf = next;
+            }
+            compute_tile(buf);
+        }
+    } else {
+        for (int i = 0; i < nt; ++i) {
+            load_tile(buf, wave + i * WAVES);
+            compute_tile(buf);
+        }
     }
 
     // acc[j][mb][i] = C[m = m0 + 16 mb + 4*qd + i][n = 16 (rb0 + j) + r]; one pass of the reduction buffer per
@@ -1363,8 +1381,12 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
                 }
             };
             const bool edge = short_rows || RB % 4 != 0;
+            // (one workgroup a CU and at least four tiles a wave: with two the second copy of the tile's code costs more than the wait it saves,
+            // 16384 x 2048 at 6 rows 8.4 -> 9.7 us)
+            const bool ahead = !edge && w4 == 8 && mb == 1 && wgs <= 256 && a.Kp >= 4096;
 #define AO_RB4_MB(GG, MBV)                                                 \
-    if (w4 == 4 && !edge) go(int4wo_linear_rb4_kernel<GG, 4, MBV, false>, 4); \
+    if (ahead) go(int4wo_linear_rb4_kernel<GG, 8, 1, false, true>, 8);     \
+    else if (w4 == 4 && !edge) go(int4wo_linear_rb4_kernel<GG, 4, MBV, false>, 4); \
     else if (w4 == 4) go(int4wo_linear_rb4_kernel<GG, 4, MBV, true>, 4);   \
     else if (!edge) go(int4wo_linear_rb4_kernel<GG, 8, MBV, false>, 8);    \
     else go(int4wo_linear_rb4_kernel<GG, 8, MBV, true>, 8)
