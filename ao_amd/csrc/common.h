@@ -114,6 +114,22 @@ __device__ __forceinline__ uint32_t hw_bf16_pack(float lo, float hi) {
     return u;
 }
 
+// Tiles kb, kb + stride, .. below KB of one wave, each requested while the one before it is multiplied.  No request stands under a
+// condition: behind one the compiler waits for every request of the wave, the next tile's too, and a tile takes the latency of its successor.
+template <class Buf, class Load, class Compute>
+__device__ __forceinline__ void tiles_ahead(int kb, int KB, int stride, const Load& load, const Compute& compute) {
+    if (kb >= KB) return;
+    Buf now, next;
+    load(now, kb);
+    for (int n = kb + stride; n < KB; n += stride) {
+        load(next, n);
+        __builtin_amdgcn_sched_barrier(0);
+        compute(now);
+        now = next;
+    }
+    compute(now);
+}
+
 // Cross-lane reductions on the VALU's data-parallel-primitive path instead of ds_bpermute (an LDS round trip per
 // step): DPP control words for gfx9: quad_perm [1,0,3,2] = 0xB1, [2,3,0,1] = 0x4E, row_half_mirror = 0x141 (lane i <-> 7-i
 // of each 8), row_mirror = 0x140 (lane i <-> 15-i of each 16).  After the four steps every lane of a 16-lane row holds

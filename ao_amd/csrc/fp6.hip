@@ -672,7 +672,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_kernel(const uint16_t* 
         const u32x2v_t hi = reinterpret_cast<const u32x2v_t*>(t + 256)[lane];
         return __builtin_shufflevector(lo, __builtin_shufflevector(hi, hi, 0, 1, -1, -1), 0, 1, 2, 3, 4, 5);
     };
-    auto load_tile = [&](Buf& b, int kb) __attribute__((always_inline)) {
+    auto load_tile = [&](Buf& b, int kb, auto whole_rows) __attribute__((always_inline)) {
         const uint32_t* t = tiles + (int64_t)kb * 384;
         const int64_t next = (int64_t)KB * 384;  // same k tile of the next row block
         b.w0 = load_w(t);
@@ -681,7 +681,11 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_kernel(const uint16_t* 
             b.w2 = load_w(t + 2 * next);
             b.w3 = load_w(t + 3 * next);
         }
-        if (xact) {
+        if constexpr (decltype(whole_rows)::value) {
+            const u32x4v_t* xv = reinterpret_cast<const u32x4v_t*>(xp + (int64_t)kb * 128);
+#pragma unroll
+            for (int sl = 0; sl < 4; ++sl) b.x[sl] = xv[sl];
+        } else if (xact) {
             const int64_t k0 = (int64_t)kb * 128 + qd * 32;
             if (k0 + 32 <= K) {
                 const u32x4v_t* xv = reinterpret_cast<const u32x4v_t*>(xp + (int64_t)kb * 128);
@@ -727,23 +731,38 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_kernel(const uint16_t* 
         }
     };
 
-    Buf b0, b1;
+    if constexpr (RBW == 4) {
+        // Every tile but the one in which the activation rows end, all rows (those past M read row 0; what they add up is not stored).  With
+        // one or two row blocks the activations are most of what a wave requests, and the tests of the rows are cheaper than the requests
+        // of all 16: 4 rows of 14336 -> 4096 14.0 / 14.8 us.  5120 -> 13824 at 7 rows 15.4 -> 14.9, 8192 -> 28672 at 3 rows 45.2 -> 43.5.
+        const int whole = (int)(K / 128);
+        tiles_ahead<Buf>(wave, whole, WAVES, [&](Buf& b, int kb) __attribute__((always_inline)) { load_tile(b, kb, std::true_type()); }, compute_tile);
+        if (whole < KB && whole % WAVES == wave) {
+            Buf b;
 #pragma unroll
-    for (int sl = 0; sl < 4; ++sl) {
-        b0.x[sl] = u32x4v_t{0, 0, 0, 0};
-        b1.x[sl] = u32x4v_t{0, 0, 0, 0};
-    }
-    int kb = wave;
-    if (kb < KB) load_tile(b0, kb);
-    while (kb < KB) {
-        const int kb1 = kb + WAVES, kb2 = kb + 2 * WAVES;
-        if (kb1 < KB) load_tile(b1, kb1);
-        compute_tile(b0);
-        if (kb1 < KB) {
-            if (kb2 < KB) load_tile(b0, kb2);
-            compute_tile(b1);
+            for (int sl = 0; sl < 4; ++sl) b.x[sl] = u32x4v_t{0, 0, 0, 0};
+            load_tile(b, whole, std::false_type());
+            compute_tile(b);
         }
-        kb = kb2;
+    } else {
+        Buf b0, b1;
+#pragma unroll
+        for (int sl = 0; sl < 4; ++sl) {
+            b0.x[sl] = u32x4v_t{0, 0, 0, 0};
+            b1.x[sl] = u32x4v_t{0, 0, 0, 0};
+        }
+        int kb = wave;
+        if (kb < KB) load_tile(b0, kb, std::false_type());
+        while (kb < KB) {
+            const int kb1 = kb + WAVES, kb2 = kb + 2 * WAVES;
+            if (kb1 < KB) load_tile(b1, kb1, std::false_type());
+            compute_tile(b0);
+            if (kb1 < KB) {
+                if (kb2 < KB) load_tile(b0, kb2, std::false_type());
+                compute_tile(b1);
+            }
+            kb = kb2;
+        }
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -800,12 +819,11 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
     const int64_t rb0 = (int64_t)blockIdx.x * RBW, m0 = (int64_t)blockIdx.y * (16 * MB);
     const int KB = (int)(K / 128);
     const uint32_t* tiles = native + rb0 * KB * 384;
-    bool xact[MB];
     const uint16_t* xp[MB];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
-        xact[mb] = (m0 + 16 * mb + r) < M;
-        xp[mb] = x + (xact[mb] ? (m0 + 16 * mb + r) : 0) * K + qd * 32;
+        const int64_t m = m0 + 16 * mb + r;
+        xp[mb] = x + (m < M ? m : 0) * K + qd * 32;
     }
     f16x2_t sc2[RBW];
 #pragma unroll
@@ -821,7 +839,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
         for (int mb = 0; mb < MB; ++mb) acc[j][mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
     struct Buf { u32x6_t w[RBW]; u32x4v_t x[MB][4]; };
-    auto load_tile = [&](Buf& b, int kb) __attribute__((always_inline)) {
+    auto load_tile = [&](Buf& b, int kb, int blocks = MB) __attribute__((always_inline)) {
         const uint32_t* t = tiles + (int64_t)kb * 384;
 #pragma unroll
         for (int j = 0; j < RBW; ++j) {
@@ -831,12 +849,12 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
             b.w[j] = __builtin_shufflevector(lo, __builtin_shufflevector(hi, hi, 0, 1, -1, -1), 0, 1, 2, 3, 4, 5);
         }
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-            if (xact[mb]) {
-                const u32x4v_t* xv = reinterpret_cast<const u32x4v_t*>(xp[mb] + (int64_t)kb * 128);
+        for (int mb = 0; mb < MB; ++mb) {   // (lanes of rows past M read row 0; what they add up is not stored)
+            if (mb >= blocks) continue;
+            const u32x4v_t* xv = reinterpret_cast<const u32x4v_t*>(xp[mb] + (int64_t)kb * 128);
 #pragma unroll
-                for (int sl = 0; sl < 4; ++sl) b.x[mb][sl] = xv[sl];
-            }
+            for (int sl = 0; sl < 4; ++sl) b.x[mb][sl] = xv[sl];
+        }
     };
     auto compute_tile = [&](const Buf& b) __attribute__((always_inline)) {
 #pragma unroll
@@ -862,25 +880,16 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
         }
     };
 
-    Buf b0, b1;
+    if (m0 + 16 * (MB - 1) < M) {
+        tiles_ahead<Buf>(wave, KB, WAVES, load_tile, compute_tile);   // 4096 x 14336 at 24 rows 16.1 -> 15.1 us, 28672 x 8192 49.0 -> 47.4
+    } else {   // a last chunk of so few rows that a whole block has none: one tile at a time, without that block's requests
+        Buf b;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int sl = 0; sl < 4; ++sl) {
-            b0.x[mb][sl] = u32x4v_t{0, 0, 0, 0};   // rows >= M keep these zeros
-            b1.x[mb][sl] = u32x4v_t{0, 0, 0, 0};
+        for (int sl = 0; sl < 4; ++sl) b.x[MB - 1][sl] = u32x4v_t{0, 0, 0, 0};
+        for (int kb = wave; kb < KB; kb += WAVES) {
+            load_tile(b, kb, MB - 1);
+            compute_tile(b);
         }
-    int kb = wave;
-    if (kb < KB) load_tile(b0, kb);
-    while (kb < KB) {
-        const int kb1 = kb + WAVES, kb2 = kb + 2 * WAVES;
-        if (kb1 < KB) load_tile(b1, kb1);
-        compute_tile(b0);
-        if (kb1 < KB) {
-            if (kb2 < KB) load_tile(b0, kb2);
-            compute_tile(b1);
-        }
-        kb = kb2;
     }
     // one pass of the reduction buffer per activation block; wave j sums and stores row block j
 #pragma unroll

@@ -322,6 +322,7 @@ __global__ __launch_bounds__(WAVES * 64) void int8wo_linear_kernel(const Int8Arg
 // (9 and more rows at K = 4096): every row block re-reads all activation rows from L2 there, twice the bytes of its int8
 // weights at 16 rows, and a CU's L1 fill rate (about 20 bytes per cycle), not memory, sets the time.  A wave loads the
 // activation fragments of a K tile once and runs them against the tiles of four row blocks; wave j finishes block j.
+// The next tile is requested ahead, under no condition: 14336 x 4096 at 7 / 16 rows 17.4 / 19.2 -> 16.7 / 18.5 us, 28672 x 8192 at 4 rows 56.6 -> 54.1.
 template <int WAVES, int MB>
 __global__ __launch_bounds__(WAVES * 64) void int8wo_linear_rb4_kernel(const Int8Args a) {
     // MB 16-row blocks of activations per workgroup (MB = 2 from 17 rows on): a converted weight fragment feeds MB
@@ -385,21 +386,7 @@ __global__ __launch_bounds__(WAVES * 64) void int8wo_linear_rb4_kernel(const Int
             }
         }
     };
-    {
-        Buf b0, b1;
-        int kb = wave;
-        if (kb < KB) load_tile(b0, kb);
-        while (kb < KB) {
-            const int kb1 = kb + WAVES, kb2 = kb + 2 * WAVES;
-            if (kb1 < KB) load_tile(b1, kb1);
-            compute_tile(b0);
-            if (kb1 < KB) {
-                if (kb2 < KB) load_tile(b0, kb2);
-                compute_tile(b1);
-            }
-            kb = kb2;
-        }
-    }
+    tiles_ahead<Buf>(wave, KB, WAVES, load_tile, compute_tile);
     // acc[j][mb][i] = C[m = m0 + 16 mb + 4*qd + i][n = 16 (rb0 + j) + r]; one pass of the reduction buffer per
     // activation block
 #pragma unroll
