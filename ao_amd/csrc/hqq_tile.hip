@@ -446,7 +446,7 @@ HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool 
         if (bf16) other *= 0.88;
         lead = bf16 ? 0.92 : 0.95;
     } else if (M <= 16) {
-        other = 0.92 * (6.2 + ((bf16 ? 0.22 : 0.2) + (bf16 ? 0.0011 : 0.0015) * rows) * weights * 1e-6);
+        other = 0.97 * (6.2 + ((bf16 ? 0.22 : 0.2) + (bf16 ? 0.0011 : 0.0015) * rows) * weights * 1e-6);
         lead = 0.92;
     }
     return lead * p.us < other ? p : none;
