@@ -123,8 +123,8 @@ def test_silu_mul_over_all_values(dtype):
 @pytest.mark.parametrize("rise", [0.4, 6.0, 60.0])
 @pytest.mark.parametrize("heads,dtype", [((4, 2), torch.bfloat16), ((3, 3), torch.float16)])
 def test_attention_with_rising_scores(rise, heads, dtype):
-    """Scores that grow by `rise` every 32 positions, so that a row's maximum passes the kept one by less than 2^8 or by far more in
-    every tile; and the same ones falling.  Bound as in test_attention_matches_fp32, doubled for the sums of few large terms."""
+    """Scores that grow by `rise` every 32 positions, so that every tile raises a row's maximum, by little or by far; and the same ones
+    falling, where no tile after a group's first does.  Bound as in test_attention_matches_fp32, doubled for the sums of few large terms."""
     n_head, n_kv = heads
     T = S = 321
     qkv = _qkv(T, n_head, n_kv, dtype) * 0.25
