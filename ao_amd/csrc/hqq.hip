@@ -597,9 +597,10 @@ struct HqqMfmaPlan { int waves, rb, tiles, steps, slices, steps_per_wave; };
 static HqqMfmaPlan hqq_mfma_plan(int64_t M, int64_t K, int64_t N, bool transposed, int64_t group) {
     HqqMfmaPlan p{};
     p.steps = (int)(transposed ? (N + 63) / 64 : (K + 31) / 32);
-    // Cheapest by a measured model (in us, 1 to 64 rows, 4096 and 11008 wide): a CU takes 0.15 us for a kilobyte of codes with
-    // all its waves together, eight at least (a step of one wave alone lasts 1.2), plus the start of each run, and its
-    // workgroups come in whole rounds; a slice costs its fp32 partial sums, written and read.
+    // Cheapest by a measured model (in us, 1 to 64 rows, 4096 and 11008 wide): a CU takes 0.12 us for a kilobyte of codes with
+    // all its waves together, eight at least, plus the start of each run, and its workgroups come in whole rounds; a slice costs its fp32 partial
+    // sums, written and read.  (With 0.15 us and half the start, from when every step waited for the next one's requests, 32 rows
+    // transposed of 11008 x 4096 took 22.6 us, now 19.8, and one row 16.0, now 13.8; eight weights at 1 to 48 rows are level on average.)
     // Two blocks of 16 byte rows (64 values of k) per wave in the transposed product where they share their group.
     const int most_slices = M <= 16 ? 16 : 8;
     double best = 1e30;
@@ -612,7 +613,7 @@ static HqqMfmaPlan hqq_mfma_plan(int64_t M, int64_t K, int64_t N, bool transpose
                 if (z != slices) continue;
                 // (a block pair reads scales, zeros and activations once for both)
                 const int64_t on_cu = ((int64_t)tiles * z + 255) / 256 * waves;
-                const double us = 0.15 * (rb == 2 ? 1.6 : 1.0) * (double)(on_cu > 8 ? on_cu : 8) * (per + 0.7) +
+                const double us = 0.12 * (rb == 2 ? 1.4 : 1.0) * (double)(on_cu > 8 ? on_cu : 8) * (per + 1.5) +
                                   2e-6 * (double)(M * (transposed ? K : N)) * z;
                 if (us < best) {
                     best = us;
