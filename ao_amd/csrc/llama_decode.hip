@@ -206,9 +206,10 @@ __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const uin
     // A slot (16 lanes) keeps its own softmax: the scores of its positions stay in registers, its maximum is raised chunk by chunk, and the 64
     // slots meet once at the end.  (Scores and probabilities went through LDS, with a maximum over all of them in between: two barriers more, a
     // second walk over the positions and, beyond 512 of them, a second wait for the cache.  Per layer of a step, 0.5 us at 300 positions, 3.1
-    // at 936.)
-    const float scale = 0.08838834764831845f;  // 1 / sqrt(128)
-    constexpr float LOG2E = 1.4426950408889634f;
+    // at 936.)  Maxima are kept in base 2, and an exponent is one fma of the dot product with 1 / sqrt(128) log2(e): rounded once, at the size of the
+    // difference (scaling, subtracting and turning to base 2 in steps was 2.00e-7 from 64 bits at 300 positions, e^x of the scaled score 1.94e-7,
+    // this 1.69e-7; 5.0, 5.0 and 4.4e-7 at 936 positions with scores three times as large).
+    constexpr float SCALE2 = (float)(0.08838834764831845 * 1.4426950408889634);
     float m = -INFINITY, sum = 0.f, oacc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) oacc[e] = 0.f;
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const uin
                 }
             }
         }
-        float s[U], top = m;
+        float s[U], top = -INFINITY;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             s[u] = -INFINITY;
@@ -242,14 +243,14 @@ __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const uin
                     }
                 }
                 d = row16_sum(d);
-                d *= scale;
                 if (t < T) s[u] = d;
                 top = fmaxf(top, s[u]);
             }
         }
+        top = fmaxf(m, top * SCALE2);
         const float base = top == -INFINITY ? 0.f : top;   // a slot without positions
         if (c > 0) {
-            const float alpha = __builtin_amdgcn_exp2f((m - base) * LOG2E);
+            const float alpha = __builtin_amdgcn_exp2f(m - base);
             sum *= alpha;
 #pragma unroll
             for (int e = 0; e < 8; ++e) oacc[e] *= alpha;
@@ -261,7 +262,7 @@ __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const uin
             if (c * U + u >= npass) break;
             const int t = tpos(c * U + u);
             if (t < T) {
-                const float p = __builtin_amdgcn_exp2f((s[u] - base) * LOG2E);
+                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u], SCALE2, -base));
                 sum += p;
                 if (t == pos) {
 #pragma unroll
@@ -288,7 +289,7 @@ __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const uin
     const float2 slot = stats[lane];
     const float gmax = wave_max(slot.x);
     // (a workgroup without positions, in split mode: every factor is 0)
-    const float factor = slot.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((slot.x - gmax) * LOG2E);
+    const float factor = slot.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(slot.x - gmax);
     const float tot = wave_sum(slot.y * factor);
     const float inv = 1.0f / tot;
     // the 64 rows are added in two steps of 8 (a chain of 16 additions instead of 64): every thread adds the 8 rows of
@@ -315,7 +316,7 @@ __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const uin
     }
 }
 
-// Combines the `nsplit` partial results of one head: out = sum_z e^(m_z - M) o_z / sum_z e^(m_z - M) l_z, M = max_z m_z.
+// Combines the `nsplit` partial results of one head: out = sum_z 2^(m_z - M) o_z / sum_z 2^(m_z - M) l_z, M = max_z m_z.
 template <class E>
 __global__ __launch_bounds__(128) void attention_merge_kernel(const float* __restrict__ part, int nsplit,
                                                               uint16_t* __restrict__ out) {
@@ -327,7 +328,7 @@ __global__ __launch_bounds__(128) void attention_merge_kernel(const float* __res
     float L = 0.f, o = 0.f;
     for (int z = 0; z < nsplit; ++z) {
         const float m = p[z * (HD + 2)];
-        const float w = m == -INFINITY ? 0.f : expf(m - M);
+        const float w = m == -INFINITY ? 0.f : exp2f(m - M);
         L += w * p[z * (HD + 2) + 1];
         o += w * p[z * (HD + 2) + 2 + d];
     }

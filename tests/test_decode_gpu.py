@@ -344,6 +344,43 @@ def test_linear_partials_sum_to_the_linear(M, N, K, g, ksplit):
     assert rel_l2(parts_n.sum(0).cpu().numpy(), full_n.cpu().numpy()) <= 1e-3
 
 
+def _attention_on_exact_dots(pos, S, ramp, offset, dtype=torch.bfloat16):
+    """One token of two query heads over one KV head without rotation.  Dimension 0 carries `offset` and `ramp` (a score's share that
+    moves with the position), the other products are small integers: every dot product is exact in fp32 where the ramp is 0."""
+    gen = torch.Generator().manual_seed(pos)
+    qkv = torch.randint(-2, 3, (1, 4 * 128), generator=gen).to(dtype)
+    k_cache = torch.randint(-3, 4, (1, 1, S, 128), generator=gen).to(dtype)
+    v_cache = torch.randn(1, 1, S, 128, generator=gen).to(dtype)
+    qkv[0, [0, 128]], qkv[0, 256] = 128.0, offset + ramp * pos
+    k_cache[0, 0, :, 0] = offset + ramp * torch.arange(S)
+    freqs = torch.zeros(S, 64, 2)
+    freqs[..., 0] = 1.0
+    k, v = k_cache.double()[0, 0, : pos + 1], v_cache.double()[0, 0, : pos + 1]
+    k[pos], v[pos] = qkv[0, 256:384].double(), qkv[0, 384:].double()
+    scores = qkv[0, :256].double().view(2, 128) @ k.t() / 128**0.5
+    tensors = [t.to(_dev()) for t in (qkv, freqs.to(dtype), torch.tensor([pos], dtype=torch.int32), k_cache, v_cache)]
+    return tensors, scores, v
+
+
+def test_decode_attention_rounds_an_exponent_once():
+    """Scores of 1448 and a few units around it, from exact dot products: the probabilities depend on their differences only, which are small.
+    Per workgroup of a split context (whose sums are fp32): 2^-24 of a difference below 32 and of a dozen additions, 1e-6 in all.
+    A score that is itself rounded is 2^-24 * 1448 off, 6e-5."""
+    from ao_amd._lib import check, current_stream, lib
+
+    pos, S, nsplit = 1400, 2048, 2
+    (qkv, freqs, p, kc, vc), scores, v = _attention_on_exact_dots(pos, S, 0.0, 128.0)
+    part, out = torch.full((2, nsplit, 130), 7.0, device=qkv.device), torch.empty(2 * 128, dtype=torch.bfloat16, device=qkv.device)
+    check(lib().ao_amd_llama_decode_attention_split(qkv.data_ptr(), None, 0, freqs.data_ptr(), p.data_ptr(), kc.data_ptr(), vc.data_ptr(), 2, 1, 128, S,
+                                                    nsplit, part.data_ptr(), out.data_ptr(), current_stream(qkv.device)))
+    got = part.cpu().double()
+    for z in range(nsplit):
+        mine = (torch.arange(pos + 1) // 64) % nsplit == z
+        want = scores[:, mine].softmax(-1) @ v[mine]
+        assert rel_l2((got[:, z, 2:] / got[:, z, 1:2]).numpy(), want.numpy()) <= 1e-6
+    assert rel_l2(out.float().cpu().view(2, 128).numpy(), (scores.softmax(-1) @ v).numpy()) <= 2**-8
+
+
 @pytest.mark.parametrize("S", [64, 4096])
 def test_decode_attention_from_partial_rows(S):
     """fp32 partial qkv rows are added and rounded to bf16 inside the attention kernel: same result as handing it the
