@@ -381,6 +381,26 @@ def test_decode_attention_rounds_an_exponent_once():
     assert rel_l2(out.float().cpu().view(2, 128).numpy(), (scores.softmax(-1) @ v).numpy()) <= 2**-8
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rise", [0.4, 6.0, 60.0, -0.4, -6.0, -60.0])
+@pytest.mark.parametrize("pos,nsplit", [(511, 1), (1023, 1), (1800, 1), (1800, 2)])
+def test_decode_attention_with_rising_scores(pos, nsplit, rise, dtype):
+    """Scores that move by `rise` every 512 positions, so that every chunk raises the maxima, or none after the first does.  16-bit outputs
+    of fp32 sums: two roundings' worth."""
+    from ao_amd._lib import check, current_stream, lib
+
+    S = 2048
+    (qkv, freqs, p, kc, vc), scores, v = _attention_on_exact_dots(pos, S, rise * 128**0.5 / 128 / 512, 0.0, dtype)
+    work, out = torch.empty(2 * 16 * 130, device=qkv.device), torch.empty(2 * 128, dtype=dtype, device=qkv.device)
+    if dtype is torch.bfloat16:
+        check(lib().ao_amd_llama_decode_attention_split(qkv.data_ptr(), None, 0, freqs.data_ptr(), p.data_ptr(), kc.data_ptr(), vc.data_ptr(), 2, 1, 128, S,
+                                                        nsplit, work.data_ptr(), out.data_ptr(), current_stream(qkv.device)))
+    else:
+        check(lib().ao_amd_llama_decode_attention_f16(qkv.data_ptr(), freqs.data_ptr(), p.data_ptr(), kc.data_ptr(), vc.data_ptr(), 2, 1, 128, S,
+                                                      nsplit, work.data_ptr(), out.data_ptr(), current_stream(qkv.device)))
+    assert rel_l2(out.float().cpu().view(2, 128).numpy(), (scores.softmax(-1) @ v).numpy()) <= (2**-8 if dtype is torch.bfloat16 else 2**-11)
+
+
 @pytest.mark.parametrize("S", [64, 4096])
 def test_decode_attention_from_partial_rows(S):
     """fp32 partial qkv rows are added and rounded to bf16 inside the attention kernel: same result as handing it the
