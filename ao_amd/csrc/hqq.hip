@@ -507,6 +507,27 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
                     in[0][i] = *reinterpret_cast<const u32x4_t*>(scales + g_block * N + n);
                     in[1][i] = *reinterpret_cast<const u32x4_t*>(zeros + g_block * N + n);
                 }
+                if (BF16) {   // (a lane's columns past the end of the run are the last ones again)
+                    HqqOrdinary ordinary;
+#pragma unroll
+                    for (int i = 0; i < CHUNK / 8; ++i)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (i == 0 || i * 8 < c1 - c0) {
+                                ordinary.see(in[0][i][e]);
+                                ordinary.see(in[1][i][e]);
+                            }
+                    bool all = ordinary.all();
+                    if (!all) {
+                        all = true;
+#pragma unroll
+                        for (int i = 0; i < 2 * (CHUNK / 8); ++i)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) all &= HqqOrdinary::with_zeros(in[i & 1][i >> 1][e]);
+                    }
+                    direct = __any(!all);
+                    if (direct) break;
+                }
 #pragma unroll
                 for (int i = 0; i < CHUNK / 8; ++i) {
                     *reinterpret_cast<u32x4_t*>(s_lds + i * 512 + lane * 8) = in[0][i];
@@ -526,24 +547,13 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
                 asm volatile("" ::: "memory");
             }
         }
-        if (BF16 && !direct) {
-            bool nan = false;
+        if (BF16) {   // 2^-9 of the sums; of no use where a scale or zero of a later chunk is beyond the range
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
                 for (int c = 0; c < NACC; ++c)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        acc[mb][c][r] *= HqqRowMatrices::DOWN;
-                        nan |= acc[mb][c][r] != acc[mb][c][r];
-                    }
-            if (__any(nan)) {   // an infinite zero may have reached its neighbours
-                direct = true;
-#pragma unroll
-                for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-                    for (int c = 0; c < NACC; ++c) acc[mb][c] = hqq_f32x4_t{0.f, 0.f, 0.f, 0.f};
-            }
+                    for (int r = 0; r < 4; ++r) acc[mb][c][r] = direct ? 0.f : acc[mb][c][r] * HqqRowMatrices::DOWN;
         }
         if (direct)
             for (int s = s0; s < s1; ++s) {

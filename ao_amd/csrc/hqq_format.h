@@ -89,9 +89,10 @@ __device__ __forceinline__ void hqq_row(uint32_t d, const float* z, const float*
 //   t = q - z     B: the masked nibbles, fp16 subnormals q 2^-24 or q 2^-20, in the order of bytes 0, 2, 1, 3;  A: 2^15 or 2^11 where it puts
 //                 them in order;  C = -z 2^-9, itself such a product.  One value is rounded to fp32 once, then to bf16: bf16(t) 2^-9.
 //   w = t * s     A: the scales on the diagonal; the product of two bf16 is exact.  Rounded: w 2^-9.
-// The caller multiplies its sums by DOWN (weights below 2^-117 are subnormals on the way).  13 VALU and 4 two-pass matrix instructions for 8 weights, where mixed fmas and
-// multiplications take 37 VALU (32 rows x 4096 x 11008 18.2 -> 17.6 us by this alone).  Zeros off the diagonal meet the other values: an infinite z, or a
-// NaN, makes NaNs of its three neighbours.  They go into the same sums, so a caller that finds a NaN there adds up again element-wise.
+// The caller multiplies its sums by DOWN.  13 VALU and 4 two-pass matrix instructions for 8 weights, where mixed fmas and
+// multiplications take 37 VALU (32 rows x 4096 x 11008 18.2 -> 17.6 us by this alone).  For scales and zeros in HqqOrdinary's range only, whose weights (0
+// or 2^-80 .. 2^81) the factor leaves exact: beyond it bf16(t * s) may overflow, which 2^-9 of it does not, or be a subnormal on the way, and the zeros off
+// the diagonal meet an infinite z as 0 * inf, a NaN for its three neighbours.
 typedef float hqq_f4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 hqq_f16x4_t __attribute__((ext_vector_type(4)));
 typedef short hqq_s16x4_t __attribute__((ext_vector_type(4)));
@@ -139,6 +140,23 @@ struct HqqRowMatrices {
         }
         half(l0, l1, low, lo0, lo1);
         half(h0, h1, high, hi0, hi1);
+    }
+};
+
+// Whether every scale and zero seen is 2^-40 .. 2^40 in magnitude, or 0, both 16 bits of a dword at once: two instructions a dword, which know no
+// 0; a lane that met something else looks again.
+typedef uint16_t hqq_u16x2_t __attribute__((ext_vector_type(2)));
+struct HqqOrdinary {
+    static constexpr uint16_t LO = (127 - 40) << 7, HI = (127 + 40) << 7;
+    hqq_u16x2_t most = {0, 0};   // of twice the magnitude's bits less 2 LO, where a magnitude below LO wraps beyond all others
+    __device__ __forceinline__ void see(uint32_t d) {
+        const hqq_u16x2_t b = __builtin_bit_cast(hqq_u16x2_t, d) * (uint16_t)2 - hqq_u16x2_t{2 * LO, 2 * LO};
+        most = __builtin_elementwise_max(most, b);
+    }
+    __device__ __forceinline__ bool all() const { return most.x <= 2 * (HI - LO) && most.y <= 2 * (HI - LO); }
+    static __device__ __forceinline__ bool with_zeros(uint32_t d) {
+        const uint32_t lo = d & 0x7fffu, hi = (d >> 16) & 0x7fffu;
+        return (lo == 0 || (lo >= LO && lo <= HI)) && (hi == 0 || (hi >= LO && hi <= HI));
     }
 };
 
