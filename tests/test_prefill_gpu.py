@@ -120,6 +120,28 @@ def test_silu_mul_over_all_values(dtype):
     assert ((a - b).abs() <= step * b.abs() + (2.0 ** -100 if dtype is torch.bfloat16 else 2.0 ** -24)).all() and (a != b).double().mean() <= 0.02
 
 
+@pytest.mark.parametrize("special", [0.0, 69.0, -100.0, float("inf"), float("nan")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_silu_mul_beside_special_values(dtype, special):
+    """Waves of ordinary values (0 < |gate| < 69) leave out what zeros, infinities and large values need; one such value among them changes
+    no other's bits.  Every ordinary value, the nearest 16 bits of the fp32 function but for ties that fp32 rounds onto."""
+    x = torch.arange(65536, device="cuda", dtype=torch.int32).to(torch.int16).view(dtype)
+    x = x[(x != 0) & (x.abs() < 69)]
+    x = x[: len(x) // 512 * 512]
+    y = x.clone()
+    y[5::512] = special
+    out = []
+    for gate in (x, y):
+        out.append(torch.empty_like(gate))
+        _call("ao_amd_silu_mul", gate, torch.ones_like(gate), int(dtype is torch.float16), gate.numel(), out[-1])
+    same = torch.ones_like(x, dtype=torch.bool)
+    same[5::512] = False
+    assert torch.equal(out[0][same], out[1][same])
+    want = (x.double() / (1 + torch.exp(-x.double()))).to(dtype)
+    normal = want.abs() >= torch.finfo(dtype).tiny
+    assert (out[0] != want)[normal].sum() <= 2
+
+
 @pytest.mark.parametrize("rise", [0.4, 6.0, 60.0])
 @pytest.mark.parametrize("heads,dtype", [((4, 2), torch.bfloat16), ((3, 3), torch.float16)])
 def test_attention_with_rising_scores(rise, heads, dtype):
