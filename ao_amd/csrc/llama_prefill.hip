@@ -86,10 +86,9 @@ __global__ __launch_bounds__(256) void prefill_cache_kernel(const uint16_t* __re
 
 // Causal attention of T query rows over the cache, flash style.
 //
-// Four groups of 2 waves walk the cache in tiles of 32 positions, every fourth one each; a wave owns 32 query rows of one head, the same
-// ones in all groups, whose maxima, sums and accumulators meet at the end: each group finishes a quarter of the columns.  HEADS: the two
-// waves are two query heads of one KV head (grouped-query models: one K / V tile serves both); otherwise they are two consecutive
-// 32-row blocks of one head.
+// GROUPS = 8 / WAVES groups of WAVES waves walk the cache in tiles of 32 positions, every GROUPS-th one each; a wave owns 32 query rows of one
+// head, the same ones in all groups, whose maxima, sums and accumulators meet at the end: each group finishes its share of the columns.  HEADS of a
+// group's waves are query heads of one KV head (grouped-query models: one K / V tile serves them all), the others are consecutive 32-row blocks.
 //
 // Both products are 32x32x16 matrix instructions with the query on the column side: S^T = K Q^T leaves a lane with 16 scores
 // of ONE query row per 32 positions, so the softmax statistics are lane-local up to one exchange between the wave's
@@ -104,66 +103,63 @@ __global__ __launch_bounds__(256) void prefill_cache_kernel(const uint16_t* __re
 // multiplications, but then the largest probability of a row is no longer 1, which 16 bits hold exactly: 400 rows over 40 heads were 0.00188
 // from the result in 64 bits instead of 0.00174, for 1 us of 28 at 1000 positions.)
 //
-// Bound by the chain of a tile (scores, maximum, exponentials, second product) and, for long prompts, by the rows that see most positions:
-// with two groups of four waves and 64 positions a tile, 256 workgroups of 1000 rows were resident at once and the longest set the time; now
-// 512 follow each other, longest first.  A short prompt pays the start: a group rotates two of the eight query fragments and reads
-// the others from LDS (each rotated all eight, some 450 instructions).  Llama-3-8B widths, 61 / 130 / 1000 positions: 11.4 / 13.4 / 34.8 ->
-// 8.1 / 7.9 / 27.8 us; 13B, 79 positions 11.8 -> 7.7.
-template <class E, bool HEADS>
+// Bound by the chain of a tile (scores, maximum, exponentials, second product) and by what brings tiles into LDS (requests, V's turn, writes).  Groups
+// of two: a short prompt pays the start, where a group rotates its share of the eight query fragments and reads the others from LDS (some 450
+// instructions for all), and one whose workgroups are resident at once its longest rows, which four groups share.  Llama-3-8B widths, 61 / 130 / 1000
+// positions 8.1 / 7.9 / 27.8 us; with two groups of four waves, 64 positions a tile and all fragments rotated by each wave 11.4 / 13.4 / 34.8.  Groups of
+// four: a tile serves 128 rows instead of 64, for half the staging a wave.  Both at 2048 / 4096 / 8192 positions: 32 heads over 8 77 / 241 / 842 -> 63 / 197 /
+// 690 us, 64 over 8 143 / 466 / 1714 -> 114 / 372 / 1355, 40 over 40 105 / 324 / 1131 -> 93 / 274 / 918; each group's largest probability of a row is
+// exact in 16 bits, so fewer groups are a little further from 64 bits (bf16, 1300 positions 0.00196 -> 0.00198, as far as two groups always were).
+template <class E, int WAVES, int HEADS>
 __global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ freqs,
                                                                 int64_t wrap, const void* __restrict__ pos, int pos_is_i64,
                                                                 int T, int n_head, int n_kv, int64_t S, const uint16_t* __restrict__ k_cache,
                                                                 const uint16_t* __restrict__ v_cache, uint16_t* __restrict__ out) {
     typedef Mfma32<E> MM;
-    constexpr int GROUPS = 4, KEYS = 32;
+    constexpr int GROUPS = 8 / WAVES, KEYS = 32;
     __shared__ uint4 lds[GROUPS][2][2][KEYS * 16];   // [group][K / V][buffer]
-    __shared__ uint4 q_lds[2][8][64];                // [wave][fragment][lane]
-    __shared__ int wave_last[2];
-    const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7);
+    __shared__ uint4 q_lds[WAVES][8][64];            // [wave][fragment][lane]
+    __shared__ int wave_last[WAVES];
+    const int group = __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * WAVES));
     uint4 (*const ks)[KEYS * 16] = lds[group][0];   // [key][chunk of 8 d], chunk ^ (key & 15)
     uint4 (*const vs)[KEYS * 16] = lds[group][1];   // [d / 2][(d & 1) * 4 + (chunk of 8 keys ^ (d / 4 & 3))]
-    const int tid = threadIdx.x & 127, lane = tid & 63, col = lane & 31, half = lane >> 5;
+    const int tid = threadIdx.x % (64 * WAVES), lane = tid & 63, col = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tile = gridDim.y - 1 - blockIdx.y;   // the rows that see most positions start first
-    int head, row0;
-    if (HEADS) {
-        head = blockIdx.x * 2 + wave;
-        row0 = tile * 32;
-    } else {
-        head = blockIdx.x;
-        row0 = tile * 64 + wave * 32;
-    }
+    const int head = blockIdx.x * HEADS + wave % HEADS, row0 = (tile * (WAVES / HEADS) + wave / HEADS) * 32;
     const int kv = head / (n_head / n_kv);
     const uint16_t* kc = k_cache + (int64_t)kv * S * 128;
     const uint16_t* vc = v_cache + (int64_t)kv * S * 128;
 
-    u32x4p_t kr[4];
-    uint32_t vr[16];
+    constexpr int KROWS = 4 * WAVES, KLOADS = KEYS / KROWS, RUNS = KEYS / 8 / WAVES;   // rows of K a pass of the threads, passes; runs of 8 positions of V
+    u32x4p_t kr[KLOADS];
+    uint32_t vr[8 * RUNS];
     const int smax = (int)S - 1;
-    // this lane's shares of a tile: 16 bytes of rows tid / 16 + 8 i, two columns of the 8 positions of (step `wave`, half g)
-    const uint32_t koff = (tid >> 4) * 256 + (tid & 15) * 16, voff = wave * 4096 + lane * 4;
+    // this lane's shares of a tile: 16 bytes of rows tid / 16 + KROWS i, two columns of the 8 positions of run (step, half) = wave * RUNS + g
+    auto vrow = [&](int g, int j) { return 16 * ((wave * RUNS + g) >> 1) + 4 * ((wave * RUNS + g) & 1) + (j & 3) + 8 * (j >> 2); };
+    const uint32_t koff = (tid >> 4) * 256 + (tid & 15) * 16, voff = vrow(0, 0) * 256 + lane * 4;
     auto fetch = [&](int t) {
         const int base = t * KEYS;
         if (base + KEYS - 1 <= smax) {
             const char* const kb = (const char*)(kc + (int64_t)base * 128);
             const char* const vb = (const char*)(vc + (int64_t)base * 128);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) kr[i] = *(const u32x4p_t*)(kb + koff + i * 2048);
+            for (int i = 0; i < KLOADS; ++i) kr[i] = *(const u32x4p_t*)(kb + koff + i * (KROWS * 256));
 #pragma unroll
-            for (int g = 0; g < 2; ++g)
+            for (int g = 0; g < RUNS; ++g)
 #pragma unroll
                 for (int j = 0; j < 8; ++j) vr[g * 8 + j] = *(const uint32_t*)(vb + voff + (4 * g + (j & 3) + 8 * (j >> 2)) * 256);
         } else {   // the cache ends within the tile: its last row instead
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int key = min(base + i * 8 + (tid >> 4), smax);
+            for (int i = 0; i < KLOADS; ++i) {
+                const int key = min(base + i * KROWS + (tid >> 4), smax);
                 kr[i] = *(const u32x4p_t*)(kc + (int64_t)key * 128 + (tid & 15) * 8);
             }
 #pragma unroll
-            for (int g = 0; g < 2; ++g)
+            for (int g = 0; g < RUNS; ++g)
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const int key = min(base + 16 * wave + 4 * g + (j & 3) + 8 * (j >> 2), smax);
+                    const int key = min(base + vrow(g, j), smax);
                     vr[g * 8 + j] = *(const uint32_t*)(vc + (int64_t)key * 128 + 2 * lane);
                 }
             asm volatile("");   // (keeps the compiler from making one set of loads, with computed addresses, of both)
@@ -171,13 +167,13 @@ __global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* 
     };
     auto stash = [&](int b) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int key = i * 8 + (tid >> 4);
+        for (int i = 0; i < KLOADS; ++i) {
+            const int key = i * KROWS + (tid >> 4);
             *(u32x4p_t*)&ks[b][key * 16 + ((tid & 15) ^ (key & 15))] = kr[i];
         }
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-            const int c = (wave * 2 + g) ^ ((lane >> 1) & 3);
+        for (int g = 0; g < RUNS; ++g) {
+            const int c = (wave * RUNS + g) ^ ((lane >> 1) & 3);
             uint32_t even[4], odd[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -196,9 +192,9 @@ __global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* 
     const Position p = locate(pos, pos_is_i64, srow, S, wrap);
     const int last = row < T ? (int)p.row : -1;     // last position the row sees; -1: none
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {   // each group rotates two of the eight
-        const int d = 16 * (2 * group + s) + 8 * half;
-        q_lds[wave][2 * group + s][lane] = rotate8<E>(*(const uint4*)(qkv + ((int64_t)srow * (n_head + 2 * n_kv) + head) * 128 + d),
+    for (int s = 0; s < WAVES; ++s) {   // each group rotates its share of the eight
+        const int d = 16 * (WAVES * group + s) + 8 * half;
+        q_lds[wave][WAVES * group + s][lane] = rotate8<E>(*(const uint4*)(qkv + ((int64_t)srow * (n_head + 2 * n_kv) + head) * 128 + d),
                                                       *(const uint4*)(freqs + p.freq * 128 + d));
     }
     int hi = last, lo = last;
@@ -215,7 +211,10 @@ __global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* 
     uint4 q[8];
 #pragma unroll
     for (int s = 0; s < 8; ++s) q[s] = q_lds[wave][s][lane];
-    const int ntile = __builtin_amdgcn_readfirstlane((max(wave_last[0], wave_last[1]) + KEYS) / KEYS);
+    int seen = wave_last[0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) seen = max(seen, wave_last[w]);
+    const int ntile = __builtin_amdgcn_readfirstlane((seen + KEYS) / KEYS);
 
     f32x16_t o[4];
 #pragma unroll
@@ -283,24 +282,27 @@ __global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* 
         }
         if (t + GROUPS < ntile) stash(b ^ 1);
     }
-    // The groups' maxima, sums and accumulators meet: group g finishes block g of 32 columns
+    // The groups' maxima, sums and accumulators meet: a group finishes its share of the four blocks of 32 columns
     __syncthreads();
-    float4* const parts = (float4*)lds;                                   // [to][from][wave][4][lane]
-    float2* const stats = (float2*)(parts + GROUPS * 3 * 2 * 4 * 64);     // [group][wave][lane]
-    static_assert(GROUPS * 3 * 2 * 4 * 64 * 16 + GROUPS * 2 * 64 * 8 <= sizeof(lds), "partial sums");
-    auto part_at = [&](int to, int from) { return parts + ((to * 3 + (from < to ? from : from - 1)) * 2 + wave) * 256 + lane; };
+    constexpr int BLOCKS = 4 / GROUPS;
+    float4* const parts = (float4*)lds;        // [block][from][wave][4][lane]
+    float2* const stats = (float2*)q_lds;      // [group][wave][lane]
+    static_assert(4 * (GROUPS - 1) * WAVES * 4 * 64 * 16 <= sizeof(lds) && 8 * 64 * 8 <= sizeof(q_lds), "partial sums");
+    auto part_at = [&](int block, int from) {
+        return parts + ((block * (GROUPS - 1) + (from < block / BLOCKS ? from : from - 1)) * WAVES + wave) * 256 + lane;
+    };
 #pragma unroll
-    for (int g = 0; g < GROUPS; ++g)
-        if (g != group)
+    for (int b = 0; b < 4; ++b)
+        if (b / BLOCKS != group)
 #pragma unroll
-            for (int r = 0; r < 16; r += 4) part_at(g, group)[r * 16] = make_float4(o[g][r], o[g][r + 1], o[g][r + 2], o[g][r + 3]);
-    stats[(group * 2 + wave) * 64 + lane] = make_float2(m, sum);
+            for (int r = 0; r < 16; r += 4) part_at(b, group)[r * 16] = make_float4(o[b][r], o[b][r + 1], o[b][r + 2], o[b][r + 3]);
+    stats[(group * WAVES + wave) * 64 + lane] = make_float2(m, sum);
     __syncthreads();
     float2 ms[GROUPS];
     float top = -INFINITY;
 #pragma unroll
     for (int g = 0; g < GROUPS; ++g) {
-        ms[g] = stats[(g * 2 + wave) * 64 + lane];
+        ms[g] = stats[(g * WAVES + wave) * 64 + lane];
         top = fmaxf(top, ms[g].x);
     }
     const float base = top == -INFINITY ? 0.f : top;
@@ -313,27 +315,27 @@ __global__ __launch_bounds__(512) void prefill_attention_kernel(const uint16_t* 
     sum += __shfl_xor(sum, 32, 64);
     const float inv = 1.0f / sum;                   // a row that sees nothing (a position outside the cache) becomes NaN
 #pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
-        if (g != group) continue;
+    for (int b = 0; b < 4; ++b) {
+        if (b / BLOCKS != group) continue;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[g][r] *= ms[g].x;
+        for (int r = 0; r < 16; ++r) o[b][r] *= ms[b / BLOCKS].x;
 #pragma unroll
         for (int from = 0; from < GROUPS; ++from) {
-            if (from == g) continue;
+            if (from == b / BLOCKS) continue;
 #pragma unroll
             for (int r = 0; r < 16; r += 4) {
-                const float4 v = part_at(g, from)[r * 16];
-                o[g][r] += v.x * ms[from].x;
-                o[g][r + 1] += v.y * ms[from].x;
-                o[g][r + 2] += v.z * ms[from].x;
-                o[g][r + 3] += v.w * ms[from].x;
+                const float4 v = part_at(b, from)[r * 16];
+                o[b][r] += v.x * ms[from].x;
+                o[b][r + 1] += v.y * ms[from].x;
+                o[b][r + 2] += v.z * ms[from].x;
+                o[b][r + 3] += v.w * ms[from].x;
             }
         }
         if (row < T) {
-            uint16_t* const dst = out + ((int64_t)row * n_head + head) * 128 + g * 32 + 4 * half;
+            uint16_t* const dst = out + ((int64_t)row * n_head + head) * 128 + b * 32 + 4 * half;
 #pragma unroll
             for (int r = 0; r < 16; r += 4)
-                *(uint2*)(dst + 8 * (r >> 2)) = make_uint2(MM::pack(o[g][r] * inv, o[g][r + 1] * inv), MM::pack(o[g][r + 2] * inv, o[g][r + 3] * inv));
+                *(uint2*)(dst + 8 * (r >> 2)) = make_uint2(MM::pack(o[b][r] * inv, o[b][r + 1] * inv), MM::pack(o[b][r + 2] * inv, o[b][r + 3] * inv));
         }
     }
 }
@@ -463,12 +465,24 @@ static void prefill_attention(const PrefillAttention& a, hipStream_t st) {
     const int64_t chunks = a.T * 2 * a.n_kv * 16;
     hipLaunchKernelGGL(prefill_cache_kernel<E>, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st, a.qkv, a.freqs, a.wrap,
                        a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache);
-    if (a.n_head / a.n_kv % 2 == 0)
-        hipLaunchKernelGGL((prefill_attention_kernel<E, true>), dim3(a.n_head / 2, (T + 31) / 32), dim3(512), 0, st, a.qkv, a.freqs,
-                           a.wrap, a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache, a.out);
-    else
-        hipLaunchKernelGGL((prefill_attention_kernel<E, false>), dim3(a.n_head, (T + 63) / 64), dim3(512), 0, st, a.qkv, a.freqs,
-                           a.wrap, a.pos, a.pos_is_i64, T, a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache, a.out);
+    const int rep = a.n_head / a.n_kv;
+    auto go = [&](auto kernel, int waves, int heads) {
+        const int rows = 32 * waves / heads;
+        hipLaunchKernelGGL(kernel, dim3(a.n_head / heads, (T + rows - 1) / rows), dim3(512), 0, st, a.qkv, a.freqs, a.wrap, a.pos, a.pos_is_i64, T,
+                           a.n_head, a.n_kv, a.S, a.k_cache, a.v_cache, a.out);
+    };
+    // Groups of two until their workgroups take a third round (us of groups of two / four: 32 heads over 8 at 1000 / 1200 positions 29.2 / 31.0, 40.7 /
+    // 36.6; 40 over 40 at 700 / 800 28.3 / 29.0, 35.6 / 31.4; 8 over 4 at 4096 / 8192 72 / 92, 232 / 205), or, where a short prompt's tiles serve four heads
+    // and starting is most of the time, a second (64 over 8 at 200 / 300 / 500 11.3 / 13.4, 17.0 / 15.8, 22.6 / 21.3; 32 over 8 at 600 / 900 18.8 / 23.1, 27.0 / 28.3).
+    const int64_t workgroups = rep % 2 == 0 ? (int64_t)a.n_head / 2 * ((T + 31) / 32) : (int64_t)a.n_head * ((T + 63) / 64);
+    if (workgroups > (rep % 4 == 0 && T <= 512 ? 256 : 512)) {
+        if (rep % 4 == 0) go(prefill_attention_kernel<E, 4, 4>, 4, 4);
+        else go(prefill_attention_kernel<E, 4, 1>, 4, 1);
+    } else if (rep % 2 == 0) {
+        go(prefill_attention_kernel<E, 2, 2>, 2, 2);
+    } else {
+        go(prefill_attention_kernel<E, 2, 1>, 2, 1);
+    }
 }
 
 static int prefill_attention_entry(const PrefillAttention& a, int is_f16, int head_dim, void* stream) {

@@ -266,3 +266,35 @@ def test_long_attention_matches_fp32(T, heads, dtype):
         s = (q[:, h] @ kc[kv].float().t().contiguous() / math.sqrt(128)).masked_fill_(later, float("-inf"))
         want = s.softmax(-1) @ vc[kv].float()
         assert _rel(out.view(T, n_head, 128)[:, h], want) <= (2 ** -8 if dtype is torch.bfloat16 else 2 ** -11)
+
+
+@pytest.mark.parametrize("T,heads", [(257, (64, 16)), (288, (64, 8)), (1030, (32, 8)), (257, (128, 128)), (352, (132, 22)), (386, (90, 90))])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_attention_of_many_workgroups(T, heads, dtype):
+    """The kernel whose tiles serve 128 rows (four heads of 32, or 128 of one): rows and a cache that end within its blocks and tiles, positions in
+    any order, two of them outside.  Bound as in test_attention_matches_fp32."""
+    from ao_amd._models.llama.model import apply_rotary_emb, precompute_freqs_cis
+
+    n_head, n_kv = heads
+    S = T + 9
+    qkv = _qkv(T, n_head, n_kv, dtype)
+    freqs = precompute_freqs_cis(S, 128, dtype=dtype, device="cuda")
+    g = torch.Generator(device="cuda").manual_seed(T)
+    pos = torch.randperm(S, device="cuda", generator=g)[:T]
+    rows = torch.arange(T, device="cuda") % 100 != 40
+    pos[~rows] = S
+    kc, vc = (torch.randn(n_kv, S, 128, device="cuda", generator=g).to(dtype) for _ in range(2))
+    k_want, v_want = kc.clone(), vc.clone()
+    q, k, v = qkv.view(T, n_head + 2 * n_kv, 128)[rows].split([n_head, n_kv, n_kv], 1)
+    q = apply_rotary_emb(q[None], freqs[pos[rows]])[0].float()
+    k_want[:, pos[rows]] = apply_rotary_emb(k[None], freqs[pos[rows]])[0].transpose(0, 1)
+    v_want[:, pos[rows]] = v.transpose(0, 1)
+    out = torch.full((T, n_head * 128), 7.0, device="cuda", dtype=dtype)
+    _call("ao_amd_llama_prefill_attention", qkv, int(dtype is torch.float16), freqs, pos, 1, T, kc, vc, n_head, n_kv, 128, S, out)
+    assert torch.equal(kc, k_want) and torch.equal(vc, v_want) and out[~rows].isnan().all()
+    later = torch.arange(S, device="cuda")[None, :] > pos[rows, None]
+    for h in range(n_head):
+        kv = h * n_kv // n_head
+        s = (q[:, h] @ kc[kv].float().t().contiguous() / math.sqrt(128)).masked_fill_(later, float("-inf"))
+        want = s.softmax(-1) @ vc[kv].float()
+        assert _rel(out.view(T, n_head, 128)[rows, h], want) <= (2 ** -8 if dtype is torch.bfloat16 else 2 ** -11)
