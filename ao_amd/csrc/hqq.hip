@@ -496,6 +496,10 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
         uint16_t* const s_lds = reinterpret_cast<uint16_t*>(&red[wave][0][0]);
         uint16_t* const z_lds = s_lds + CHUNK * 64;
         bool direct = group % 32 != 0;
+        // bf16: whether scales and zeros allow the matrix instructions is looked at as they pass, and once more where one may be 0.  Two block rows: in front
+        // of a chunk's products; one: at the end, as the chunks are short (16 rows of 13824 x 5120 in groups of 32 22.6 -> 24.1 us in front, 23.0 at the end; 32
+        // rows x 4096 x 11008 in groups of 64 16.0 -> 16.2 in front, 16.5 at the end).
+        HqqOrdinary ordinary;
         if (!direct) {
             for (int c0 = s0; c0 < s1; c0 += CHUNK) {
                 const int c1 = c0 + CHUNK < s1 ? c0 + CHUNK : s1;
@@ -508,25 +512,25 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
                     in[1][i] = *reinterpret_cast<const u32x4_t*>(zeros + g_block * N + n);
                 }
                 if (BF16) {   // (a lane's columns past the end of the run are the last ones again)
-                    HqqOrdinary ordinary;
+                    HqqOrdinary here;
 #pragma unroll
-                    for (int i = 0; i < CHUNK / 8; ++i)
+                    for (int i = 0; i < 2 * (CHUNK / 8); ++i)
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            if (i == 0 || i * 8 < c1 - c0) {
-                                ordinary.see(in[0][i][e]);
-                                ordinary.see(in[1][i][e]);
-                            }
-                    bool all = ordinary.all();
-                    if (!all) {
-                        all = true;
+                        for (int e = 0; e < 4; ++e) here.see(in[i & 1][i >> 1][e]);
+                    if (RB == 1) {
+                        ordinary.most = __builtin_elementwise_max(ordinary.most, here.most);
+                    } else {
+                        bool all = here.all();
+                        if (!all) {
+                            all = true;
 #pragma unroll
-                        for (int i = 0; i < 2 * (CHUNK / 8); ++i)
+                            for (int i = 0; i < 2 * (CHUNK / 8); ++i)
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) all &= HqqOrdinary::with_zeros(in[i & 1][i >> 1][e]);
+                                for (int e = 0; e < 4; ++e) all &= HqqOrdinary::with_zeros(in[i & 1][i >> 1][e]);
+                        }
+                        direct = __any(!all);
+                        if (direct) break;
                     }
-                    direct = __any(!all);
-                    if (direct) break;
                 }
 #pragma unroll
                 for (int i = 0; i < CHUNK / 8; ++i) {
@@ -547,7 +551,17 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
                 asm volatile("" ::: "memory");
             }
         }
-        if (BF16) {   // 2^-9 of the sums; of no use where a scale or zero of a later chunk is beyond the range
+        if (BF16 && group % 32 == 0) {   // 2^-9 of the sums; of no use where a scale or zero was beyond the range
+            if (RB == 1 && __any(!ordinary.all())) {
+                const int64_t n_end = (int64_t)s1 * 64 < N ? (int64_t)s1 * 64 : N;
+                bool all = true;
+                for (int64_t n = (int64_t)s0 * 64 + lane * 8; n < n_end; n += 512) {
+                    const u32x4_t sc = *reinterpret_cast<const u32x4_t*>(scales + g_block * N + n), ze = *reinterpret_cast<const u32x4_t*>(zeros + g_block * N + n);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) all &= HqqOrdinary::with_zeros(sc[e]) & HqqOrdinary::with_zeros(ze[e]);
+                }
+                direct = __any(!all);
+            }
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll

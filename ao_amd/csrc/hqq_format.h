@@ -144,7 +144,7 @@ struct HqqRowMatrices {
 };
 
 // Whether every scale and zero seen is 2^-40 .. 2^40 in magnitude, or 0, both 16 bits of a dword at once: two instructions a dword, which know no
-// 0; a lane that met something else looks again.
+// 0; a wave that met something else looks again.
 typedef uint16_t hqq_u16x2_t __attribute__((ext_vector_type(2)));
 struct HqqOrdinary {
     static constexpr uint16_t LO = (127 - 40) << 7, HI = (127 + 40) << 7;
