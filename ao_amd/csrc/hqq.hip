@@ -569,7 +569,7 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
 #pragma unroll
                     for (int r = 0; r < 4; ++r) acc[mb][c][r] = direct ? 0.f : acc[mb][c][r] * HqqRowMatrices::DOWN;
         }
-        if (direct)
+        if (direct)   // other group sizes, and scales or zeros beyond the range
             for (int s = s0; s < s1; ++s) {
                 Frag f;
                 u32x4_t sc[2], ze[2];
@@ -626,6 +626,11 @@ static HqqMfmaPlan hqq_mfma_plan(int64_t M, int64_t K, int64_t N, bool transpose
     // sums, written and read.  (With 0.15 us and half the start, from when every step waited for the next one's requests, 32 rows
     // transposed of 11008 x 4096 took 22.6 us, now 19.8, and one row 16.0, now 13.8; eight weights at 1 to 48 rows are level on average.)
     // Two blocks of 16 byte rows (64 values of k) per wave in the transposed product where they share their group.
+    // Transposed products whose groups leave one block row to a wave keep those costs: short chunks of scales, or (groups that are no multiple of 32)
+    // scales that each lane requests itself, with no step ahead: 13824 x 5120 at one row in groups of 8 21.3 us at the lower costs, 19.3 at
+    // these, 64 rows of fp16 4608 x 11008 39.4, 36.6.  (A step ahead for groups of 8 gives one row 1 us and takes 0.7 to 1.7 us from 16 to 32 rows: eight waves
+    // a CU hide the requests, and the second set of scales costs registers.)
+    const bool single = transposed && group % 64 != 0;
     const int most_slices = M <= 16 ? 16 : 8;
     double best = 1e30;
     for (int rb = 1; rb <= (transposed && group % 64 == 0 ? 2 : 1); ++rb) {
@@ -637,7 +642,7 @@ static HqqMfmaPlan hqq_mfma_plan(int64_t M, int64_t K, int64_t N, bool transpose
                 if (z != slices) continue;
                 // (a block pair reads scales, zeros and activations once for both)
                 const int64_t on_cu = ((int64_t)tiles * z + 255) / 256 * waves;
-                const double us = 0.12 * (rb == 2 ? 1.4 : 1.0) * (double)(on_cu > 8 ? on_cu : 8) * (per + 1.5) +
+                const double us = (single ? 0.15 : 0.12) * (rb == 2 ? 1.4 : 1.0) * (double)(on_cu > 8 ? on_cu : 8) * (per + (single ? 0.7 : 1.5)) +
                                   2e-6 * (double)(M * (transposed ? K : N)) * z;
                 if (us < best) {
                     best = us;
