@@ -839,7 +839,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
         for (int mb = 0; mb < MB; ++mb) acc[j][mb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
     struct Buf { u32x6_t w[RBW]; u32x4v_t x[MB][4]; };
-    auto load_tile = [&](Buf& b, int kb, int blocks = MB) __attribute__((always_inline)) {
+    auto load_tile = [&](Buf& b, int kb) __attribute__((always_inline)) {
         const uint32_t* t = tiles + (int64_t)kb * 384;
 #pragma unroll
         for (int j = 0; j < RBW; ++j) {
@@ -850,7 +850,6 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
         }
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb) {   // (lanes of rows past M read row 0; what they add up is not stored)
-            if (mb >= blocks) continue;
             const u32x4v_t* xv = reinterpret_cast<const u32x4v_t*>(xp[mb] + (int64_t)kb * 128);
 #pragma unroll
             for (int sl = 0; sl < 4; ++sl) b.x[mb][sl] = xv[sl];
@@ -880,17 +879,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
         }
     };
 
-    if (m0 + 16 * (MB - 1) < M) {
-        tiles_ahead<Buf>(wave, KB, WAVES, load_tile, compute_tile);   // 4096 x 14336 at 24 rows 16.1 -> 15.1 us, 28672 x 8192 49.0 -> 47.4
-    } else {   // a last chunk of so few rows that a whole block has none: one tile at a time, without that block's requests
-        Buf b;
-#pragma unroll
-        for (int sl = 0; sl < 4; ++sl) b.x[MB - 1][sl] = u32x4v_t{0, 0, 0, 0};
-        for (int kb = wave; kb < KB; kb += WAVES) {
-            load_tile(b, kb, MB - 1);
-            compute_tile(b);
-        }
-    }
+    tiles_ahead<Buf>(wave, KB, WAVES, load_tile, compute_tile);   // 4096 x 14336 at 24 rows 16.1 -> 15.1 us, 28672 x 8192 49.0 -> 47.4
     // one pass of the reduction buffer per activation block; wave j sums and stores row block j
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
