@@ -461,7 +461,7 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
 #pragma unroll
         for (int sl = 0; sl < 4; ++sl) buf.x[mb][sl] = make_uint4(0, 0, 0, 0);   // rows >= M keep these zeros
     const int nt = wave < KB ? (KB - wave + WAVES - 1) / WAVES : 0;
-    if constexpr (AHEAD) {
+    if constexpr (AHEAD) {   // (tiles_ahead, whose loop counts in tiles of K, is compiled to 4 % more at 16 rows: 14336 x 4096 11.9 -> 12.4 us)
         if (nt > 0) {
             load_tile(buf, wave);
             for (int i = 1; i < nt; ++i) {
@@ -1369,7 +1369,11 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
             // two activation blocks (140 registers): beyond one workgroup per CU, three 4-wave workgroups share a CU
             // where 8-wave ones would queue (28672 x 4096 at 24-32 rows: 32 -> 25.5 us)
             if (mb >= 2 && wgs > 256) w4 = 4;
-            if (mb == 1) AO_PLAN(Int4Kernel::streaming, "int4wo_linear_rb4_kernel<%lld,%d>", (long long)g, w4);
+            const bool edge = short_rows || RB % 4 != 0;
+            // (one workgroup a CU and at least four tiles a wave: with two the second copy of the tile's code costs more than the wait it saves,
+            // 16384 x 2048 at 6 rows 8.4 -> 9.7 us)
+            const bool ahead = !edge && w4 == 8 && mb == 1 && wgs <= 256 && a.Kp >= 4096;
+            if (mb == 1) AO_PLAN(Int4Kernel::streaming, "int4wo_linear_rb4_kernel<%lld,%d>%s", (long long)g, w4, w4 == 8 && !ahead ? " tile by tile" : "");
             AO_PLAN(Int4Kernel::streaming, "int4wo_linear_rb4_kernel<%lld,%d,%d>", (long long)g, w4, mb);
             const dim3 grid4((unsigned)((RB + 3) / 4), (unsigned)mch);
             auto go = [&](auto kernel, int nw) {
@@ -1380,10 +1384,6 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
                     hipLaunchKernelGGL(kernel, grid4, dim3(nw * 64), 0, st, a);
                 }
             };
-            const bool edge = short_rows || RB % 4 != 0;
-            // (one workgroup a CU and at least four tiles a wave: with two the second copy of the tile's code costs more than the wait it saves,
-            // 16384 x 2048 at 6 rows 8.4 -> 9.7 us)
-            const bool ahead = !edge && w4 == 8 && mb == 1 && wgs <= 256 && a.Kp >= 4096;
 #define AO_RB4_MB(GG, MBV)                                                 \
     if (ahead) go(int4wo_linear_rb4_kernel<GG, 8, 1, false, true>, 8);     \
     else if (w4 == 4 && !edge) go(int4wo_linear_rb4_kernel<GG, 4, MBV, false>, 4); \

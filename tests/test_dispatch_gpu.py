@@ -55,7 +55,7 @@ def test_dispatch_walk_finds_every_kernel_family():
                      "int4wo_gemm_ksplit_kernel<%d,4,4>", "int4wo_gemm_ksplit_kernel<%d,2,4>",
                      "int4wo_gemm_lds_kernel<%d,1>", "int4wo_gemm_lds_kernel<%d,2>", "int4wo_gemm_kwave_kernel<%d>",
                      "int4wo_linear_rb4_kernel<%d,4>", "int4wo_linear_rb4_kernel<%d,8>", "int4wo_linear_rb4_kernel<%d,4,2>",
-                     "int4wo_linear_rb4_kernel<%d,8,2>", "int4wo_linear_rb4_kernel<%d,4,4>", "int4wo_linear_rb4_kernel<%d,8,4>"):
+                     "int4wo_linear_rb4_kernel<%d,8> tile by tile", "int4wo_linear_rb4_kernel<%d,8,2>", "int4wo_linear_rb4_kernel<%d,4,4>", "int4wo_linear_rb4_kernel<%d,8,4>"):
             assert tile % g in plans, tile % g
     # the single-row kernel: exactly the instantiations that int4wo_gemv1.hip compiles (waves, chunks per lane, norm)
     gemv1 = {n.split(" ")[0] for n in plans if n.startswith("int4wo_gemv1_kernel<")}
@@ -93,6 +93,10 @@ def test_dispatch_walk_finds_every_kernel_family():
     # 4 to 16 rows on weights with 768 or more 16-row blocks: four row blocks per workgroup share the activation loads
     assert _lib.int4wo_linear_plan(16, 4096, 14336, 64) == "int4wo_linear_rb4_kernel<64,8>"
     assert _lib.int4wo_linear_plan(4, 4096, 128256, 64) == "int4wo_linear_rb4_kernel<64,4>"
+    # (the next tile requested ahead where a CU has one workgroup and a wave four tiles)
+    assert _lib.int4wo_linear_plan(4, 4096, 28672, 64) == "int4wo_linear_rb4_kernel<64,8> tile by tile"
+    assert _lib.int4wo_linear_plan(4, 2048, 14336, 64) == "int4wo_linear_rb4_kernel<64,8> tile by tile"
+    assert _lib.int4wo_linear_plan(16, 4096, 16384, 64) == "int4wo_linear_rb4_kernel<64,8>"
     assert not _lib.int4wo_linear_plan(16, 14336, 4096, 64).startswith("int4wo_linear_rb4_kernel")   # 64 workgroups
     assert not _lib.int4wo_linear_plan(3, 4096, 14336, 64).startswith("int4wo_linear_rb4_kernel")
     # ... and 17 to 32 rows there take it with two activation blocks per workgroup instead of the 64-row tiles
