@@ -111,19 +111,19 @@ static TilePlan int4wo_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts)
 }
 
 // us of the kernel that ao_amd_int4wo_linear(_ws) runs, by measurement at 33 to 1000 rows on 16 weights from 768 x 1024 to 28672 x
-// 8192; 0 where it is not one of the tile kernels (few rows: the weight is streamed).  K as packed; `K_ends`: the rows end before it.
-static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g, bool K_ends) {
+// 8192; 0 where it is not one of the tile kernels (few rows: the weight is streamed).  K as packed.
+static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
     Int4Kernel kernel;
     if (!int4wo_plain_kernel(M, K, N, g, &kernel)) return 0.0;
     if (kernel == Int4Kernel::streaming) {
-        // Four blocks of streamed rows (weights of 768 row blocks and up) are behind the tiles from 1024 row blocks on, except where the weight has
-        // very many rows and the batch few (below that the lead is small, and 14336 x 4096 keeps the kernel it has had up to 48 rows).  us at 33 / 48 / 64 rows, streamed / tiled (64 rows below 4096 row blocks: the 64-row kernels): 14336 x 4096 20.3 / 19.1,
-        // 20.6 / 18.8, 24.2 / 18.5; 28672 x 8192 54.5 / 52.3, 57.5 / 52.5, 69.7 / 52.5; 16384 x 2048 12.4 / 11.8, 13.4 / 12.0, 14.1 / 12.4; 65536 x 1024 24.4 / 22.3,
-        // 25.9 / 22.4, 30.2 / 22.9; 65536 x 4096 59.3 / 59.0, 62.9 / 59.5, 78.0 / 60.8; 128256 x 4096 107 / 111, 118 / 113, 145 / 115; rows that end early, 18837 x
-        // 1088 14.9 / 12.0, 16.1 / 12.8.  Up to 32 rows (two blocks) the streaming kernel is ahead: 14336 x 1024 at 32 rows 7.7 / 8.3, 65536 x 4096 49.0 / 58.1.
+        // Four blocks of streamed rows (weights of 768 row blocks and up) are behind the tiles, except where the weight has very many rows and the batch
+        // few.  us at 33 / 48 rows, streamed / tiled: 12288 x 1024 8.6 / 8.4, 9.1 / 8.3; 14336 x 4096 18.9 / 17.2, 19.3 / 17.3; 13824 x 5120 22.1 / 19.9, 23.8 / 20.2; 16384
+        // x 8192 31.8 / 29.8, 32.9 / 30.8; 28672 x 8192 53.4 / 50.6, 57.0 / 51.4; 65536 x 1024 23.6 / 21.3, 25.5 / 22.0; 65600 x 4096 (whose last tiles begin a third
+        // round) 69.8 / 80.7, 77.4 / 83.8, 88.9 / 84.0 at 56; 128256 x 4096 111 / 121, 124 / 126, 142 / 128 at 56; but 128256 x 1024 42.3 / 40.3, 46.0 / 41.4.  Rows that
+        // end early, 18837 x 1088 14.9 / 12.0, 16.1 / 12.8.  Up to 32 rows (two blocks) the streaming kernel is ahead: 14336 x 1024 at 32 rows 7.7 / 8.3,
+        // 65536 x 4096 49.0 / 58.1.
         const int64_t blocks = (N + 15) / 16;
-        const bool edge = K_ends || blocks % 4 != 0;   // (whose kernel variant is slower: the tiles from 768 blocks on)
-        return blocks >= (edge ? 768 : 1024) && (blocks <= 4096 || M > 48) ? 1e9 : 0.0;
+        return blocks >= 768 && (blocks <= 4096 || M > 48) ? 1e9 : 0.0;
     }
     const double k = (double)K / 4096.0;
     auto rounds = [&](int bm, int bn) { return (double)((M + bm - 1) / bm * ((N + bn - 1) / bn)) / 256.0; };
@@ -157,7 +157,7 @@ static bool int4wo_tiled(int64_t M, int64_t N, int64_t K, int64_t g) {
     if (!valid_group(g) || K % 64 != 0 || M <= 32 || M * N >= ((int64_t)1 << 40)) return false;
     // in_features that were padded to whole tiles of the packed layout: the others take activations copied to that width first
     const int64_t Kp = round_up(K, g > 128 ? g : 128);
-    const double other = int4wo_other_us(M, N, Kp, g, K != Kp);
+    const double other = int4wo_other_us(M, N, Kp, g);
     if (other <= 0.0) return false;
     const TilePlan plan = int4wo_tile_plan(M, N, K, 8);
     Int4Kernel kernel;

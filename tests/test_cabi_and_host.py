@@ -339,6 +339,12 @@ def test_int4_tiled_product_is_priced_against_every_tile_kernel(cabi):
                          ((96, 28672, 8192), "int4wo_gemm_ksplit_kernel<64,4,4>")):
         M, K, N = shape
         assert cabi.int4wo_linear_plan(M, K, N, 64) == rival and offered(*shape), shape
+    # streamed weights, us streamed / tiled: 14336 x 4096 at 33 / 48 rows 18.9 / 17.2, 19.3 / 17.3; 28672 x 8192 53.4 / 50.6; 128256 x 4096 at 33 / 48 / 56 rows
+    # 111 / 121, 124 / 126, 142 / 128
+    for shape in ((33, 4096, 14336), (48, 4096, 14336), (33, 8192, 28672), (56, 4096, 128256)):
+        M, K, N = shape
+        assert cabi.int4wo_linear_plan(M, K, N, 64).startswith("int4wo_linear_rb4_kernel") and offered(*shape), shape
+    assert not offered(33, 4096, 128256) and not offered(48, 4096, 128256)
     for shape in ((32, 4096, 14336), (128, 4096, 14336), (1000, 4096, 14336), (900, 8192, 8192)):
         assert not offered(*shape), shape
     with open(os.path.join(os.path.dirname(cabi.__file__), "csrc", "int4wo_tile.hip")) as f:

@@ -254,7 +254,8 @@ def test_int4_tiles_cover_every_shape_and_the_operator_takes_them():
     assert {p.split()[1] for p in plans.values()} == {"64x64", "64x128", "96x128", "128x128", "192x128", "256x128", "256x256"}, plans
     assert {f"tile 256x{n} parts={z}" for n, z in ((128, 2), (128, 4), (256, 2), (256, 4))} <= set(plans.values()), plans
     assert any(p.endswith("parts=1") for p in plans.values()) and any(not p.endswith("parts=1") for p in plans.values())
-    for rows, taken in ((32, False), (48, False), (128, False), (160, True), (256, True), (384, True), (768, False)):
+    # (us streamed / tiled at 33 / 48 rows 18.9 / 17.2, 19.3 / 17.3)
+    for rows, taken in ((32, False), (33, True), (48, True), (128, False), (160, True), (256, True), (384, True), (768, False)):
         assert (_tiled_bytes("int4wo", rows, 14336, 4096, 64) >= 0) == taken, rows
     for case in ((160, 14336, 1024, 64), (96, 4096, 14336, 128), (130, 4099, 1088, 64)):
         for bias in (False, True):
@@ -342,7 +343,8 @@ def test_int4_rows_that_are_read_as_they_end(M, N, K, group, name):
 
 
 @pytest.mark.parametrize("M,N,K,group,tiled", [
-    (32, 12304, 1088, 128, False), (33, 12304, 1088, 128, True), (48, 12304, 1024, 64, True), (33, 12288, 1088, 32, True), (33, 12288, 1024, 64, False),
+    (32, 12304, 1088, 128, False), (33, 12304, 1088, 128, True), (48, 12304, 1024, 64, True), (33, 12288, 1088, 32, True),
+    (33, 12288, 1024, 64, True), (48, 12288, 1024, 64, True),       # us streamed / tiled 8.6 / 8.4, 9.1 / 8.3
     (33, 12290, 1032, 64, False),                                   # a width that the tiles do not take
     (48, 65552, 192, 64, False), (49, 65552, 192, 64, True), (64, 65540, 256, 32, True),
 ])
