@@ -617,7 +617,7 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
 }
 
 // reduction steps (32 k forward, 64 n transposed), output tiles and the slices of the reduction over workgroups
-struct HqqMfmaPlan { int waves, rb, tiles, steps, slices, steps_per_wave; };
+struct HqqMfmaPlan { int waves, rb, tiles, steps, slices, steps_per_wave; double us; };
 static HqqMfmaPlan hqq_mfma_plan(int64_t M, int64_t K, int64_t N, bool transposed, int64_t group) {
     HqqMfmaPlan p{};
     p.steps = (int)(transposed ? (N + 63) / 64 : (K + 31) / 32);
@@ -646,12 +646,14 @@ static HqqMfmaPlan hqq_mfma_plan(int64_t M, int64_t K, int64_t N, bool transpose
                                   2e-6 * (double)(M * (transposed ? K : N)) * z;
                 if (us < best) {
                     best = us;
-                    p = HqqMfmaPlan{waves, rb, tiles, p.steps, z, per};
+                    p = HqqMfmaPlan{waves, rb, tiles, p.steps, z, per, us};
                 }
             }
     }
     return p;
 }
+
+double hqq_stream_us(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed) { return hqq_mfma_plan(M, K, N, transposed, group).us; }
 
 }  // namespace ao
 

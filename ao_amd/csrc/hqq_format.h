@@ -167,6 +167,7 @@ void launch_hqq_finish(const float* part, int slices, int64_t count, bool bf16, 
 struct HqqTilePlan { int rows, tiles_m, tiles_n, parts; double us; };
 HqqTilePlan hqq_tile_plan(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed, bool bf16, int max_parts = 16);
 HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed, bool bf16);   // .. or is not the fastest
+double hqq_stream_us(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed);   // the streaming kernel's estimate, of its plan's costs
 void launch_hqq_tile(const HqqTilePlan& p, const uint8_t* packed, const uint16_t* scales, const uint16_t* zeros, const uint16_t* a, int64_t lda,
                      int64_t M, int64_t K, int64_t N, int64_t group, bool is_signed, bool bf16, bool transposed, float* part, uint16_t* y,
                      hipStream_t st);

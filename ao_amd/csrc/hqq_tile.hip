@@ -418,20 +418,20 @@ HqqTilePlan hqq_tile_plan(int64_t M, int64_t K, int64_t N, int64_t group, bool t
 // N, bf16, 16-bit weight and library / tiles at 192 and 384 rows: 11008 x 4096 60 / 45, 70 / 86; 14336 x 4096 70 / 45, 86 / 86; 4096 x 6144 52 / 27, 44 / 40, 51 / 58 at 512;
 // 5120 x 5120 49 / 30, 44 / 47; 8192 x 8192 92 / 50, 96 / 84, 106 / 135 at 448), and a little on wide weights forward (4096 x 14336 at 448 rows 95 / 98,
 // 4096 x 32000 of fp16 at 512 193 / 198).
-// Up to 64 rows the other one is the streaming kernel of hqq.hip, timed against the tiles on 14 weights (K x N below, us streamed / tiled).
-// Forward from 17 rows on the size of the weight decides, between 25 and 32 rows its shape as well (17 rows of bf16: 4096 x 4096 9.5 / 12.1, 11008 x
-// 4096 16.2 / 19.0, 4096 x 14336 20.2 / 19.1, 5120 x 13824 23.4 / 21.5; 32 rows 11008 x 4096 18.1 / 19.3, 4096 x 11008 19.5 / 18.8; 33 rows 5120 x 5120 14.1 / 16.6;
-// 64 rows 4096 x 6144 of fp16 17.4 / 16.8).  With fewer rows, and transposed, the tiles' own time does too: 5120 output columns are 40 tiles, which
-// fill the CUs badly whatever the K parts.  One row of bf16 4096 x 32000 30.1 / 27.2, 8192 x 8192 18.5 / 20.4, 8 rows 8192 x 28672 54.1 / 48.4; transposed at
-// 33 / 64 rows of bf16 8192 x 28672 60.7 / 65.6, 77.2 / 66.7, 14336 x 4096 23.2 / 25.0, 28.3 / 26.4; of fp16 at 32 rows 8192 x 28672 56.0 / 46.4, 13824 x 5120
-// 25.2 / 22.4.  The streaming kernel's time is therefore estimated, from those weights:
-// a part for every weight, one for every weight and row (the activations are read again for every 64 columns), the fp32 sums; the tiles' estimate
-// is 5 to 8 % long.
+// Up to 64 rows the other one is the streaming kernel of hqq.hip, timed against the tiles on 31 weights from 4096 x 4096 to 14336 x 14336 and 4096 x
+// 128256, groups of 64.  Its time is estimated from its plan's costs, the weight and the rows times the weight (the activations are read again for every 64
+// columns), with the factors that lose least by choosing wrong: 0.2 % of the best of both over all of them (3.2 % of bf16 and 1.4 % of fp16 forward by the
+// weight's size and a lead), and no tiles where they were never ahead.  us streamed / tiled, forward, bf16 (K x N): one row 8192 x 8192 16.4 / 19.0, 5120 x 13824 18.6 / 20.3,
+// 4096 x 32000 27.8 / 26.8; 17 rows 14336 x 4096 16.0 / 18.8, 13824 x 5120 19.3 / 25.6, 8192 x 28672 50.7 / 48.0; 33 rows 4096 x 4096 10.7 / 13.8, 13824 x 5120 22.8 / 28.9,
+// 5120 x 13824 23.9 / 23.3; 64 rows 13824 x 5120 28.6 / 29.9, 4096 x 11008 24.7 / 22.0.  fp16: 32 rows 13824 x 5120 20.7 / 22.8, 5120 x 13824 20.3 / 19.0.  Transposed,
+// fp16: 17 rows 8192 x 28672 38.6 / 42.1, 32 rows 48.1 / 42.6, 40 rows 4096 x 11008 18.8 / 19.0, 11008 x 4096 21.9 / 20.2; bf16, whose rule is the older one (0.3 % lost): 33 / 64 rows
+// 8192 x 28672 55.0 / 64.6, 71.9 / 64.9, 14336 x 4096 22.0 / 24.8, 26.7 / 26.0.  What is chosen wrong by most: 4096 x 65536 of bf16 at 8 rows 56.4 / 51.3, transposed fp16 8192 x
+// 4096 at 56 rows 16.6 / 14.6.
 HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed, bool bf16) {
     const HqqTilePlan none{0, 0, 0, 1, 1e30};
     const double weights = (double)K * (double)N, rows = (double)M, flops = 2.0 * rows * weights;
     // the size of the weight first: a plan takes a tenth of a microsecond of host time, which bounds calls on small weights
-    if (weights < (M > 64 ? 0.0 : !transposed ? (M > 48 ? 2e7 : M > 32 ? 3e7 : M <= 16 ? 6.4e7 : M > 24 && N > K ? 3.5e7 : 5e7) : M > 32 ? (bf16 ? 4e7 : 2e7) : M > 16 && !bf16 ? 6.4e7 : 1e30)) return none;
+    if (weights < (M > 64 ? 0.0 : !transposed ? (M > 32 ? 2e7 : 3e7) : M > 32 ? (bf16 ? 4e7 : 2e7) : M > 16 && !bf16 ? 2e7 : 1e30)) return none;
     const HqqTilePlan p = hqq_tile_plan(M, K, N, group, transposed, bf16);
     if (!p.rows) return none;
     double other = 1e30, lead = 1.0;
@@ -441,13 +441,16 @@ HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool 
         other = 14.0 + weights * 0.8e-6 + flops / 0.9e9;
         if (flops >= 4.5e10) other *= transposed || N <= 2 * K ? 0.82 : 0.8;
         if (transposed && 2 * N <= 3 * K && weights < 1e8) other = std::min(other, 20.0 + 0.61e-6 * weights + rows * (0.0016e-6 * weights - 0.009));
-    } else if (transposed) {
-        other = 5.6 + ((bf16 ? 0.18 : 0.14) + (bf16 ? 0.0022 : 0.0028) * rows) * weights * 1e-6 + (bf16 ? 0.065 : 0.055) * rows + 4.5e-6 * rows * (double)K;
-        if (bf16) other *= 0.88;
-        lead = bf16 ? 0.92 : 0.95;
-    } else if (M <= 16) {
-        other = 0.97 * (6.2 + ((bf16 ? 0.22 : 0.2) + (bf16 ? 0.0011 : 0.0015) * rows) * weights * 1e-6);
+    } else if (transposed && bf16) {
+        other = 0.88 * (5.6 + (0.18 + 0.0022 * rows) * weights * 1e-6 + 0.065 * rows + 4.5e-6 * rows * (double)K);
         lead = 0.92;
+    } else {
+        // constant, factor of the plan's costs, us a million weights, a row more; up to 32 rows and beyond
+        static const double by[3][2][4] = {{{3.4, 0.23, 0.13, 0.0022}, {3.1, 0.70, -0.002, 0.0030}},       // forward, fp16
+                                           {{4.4, 0.73, 0.013, 0.0007}, {1.8, 1.12, -0.064, 0.0018}},      // forward, bf16
+                                           {{6.3, 0.70, 0.020, 0.0014}, {4.4, 1.11, -0.021, 0.0017}}};     // transposed, fp16
+        const double* c = by[transposed ? 2 : bf16][M > 32];
+        other = c[0] + c[1] * hqq_stream_us(M, K, N, group, transposed) + (c[2] + c[3] * rows) * weights * 1e-6;
     }
     return lead * p.us < other ? p : none;
 }
