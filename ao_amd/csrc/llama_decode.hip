@@ -95,6 +95,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const uint16_t* __restrict
 constexpr int ATT_THREADS = 1024;
 constexpr int ATT_U = 8;                 // passes per chunk
 constexpr int ATT_CHUNK = 64 * ATT_U;    // positions per chunk
+constexpr int ATT_MOST = 31832;          // positions of a workgroup's share that the entry points take (a split serves longer caches, at 10 us per 1000 positions)
 
 template <class E>
 __global__ __launch_bounds__(ATT_THREADS) void decode_attention_kernel(const uint16_t* __restrict__ qkv,
@@ -463,11 +464,9 @@ static int attention_dispatch(const void* qkv_bf16, const void* qkv_f32_parts, i
     AO_REQUIRE(max_seq > 0 && max_seq <= 32768, "max_seq=%lld outside (0, 32768]", (long long)max_seq);
     AO_REQUIRE(nsplit >= 1 && nsplit <= 16, "context split %d outside [1, 16]", nsplit);
     AO_REQUIRE(nsplit == 1 || workspace_f32, "a split context needs a workspace of n_head * nsplit * 130 floats");
-    // (the bound of a kernel that kept its scores in LDS, which callers know)
+    AO_REQUIRE((max_seq + nsplit - 1) / nsplit <= ATT_MOST, "a cache of %lld positions is more than the %d that %d workgroup(s) per head take: use a larger split",
+               (long long)max_seq, ATT_MOST * nsplit, nsplit);
     const size_t smem = (size_t)(3 * 128 + 128 + 64 * 128) * sizeof(float);
-    const int64_t local = (max_seq + nsplit - 1) / nsplit + ATT_CHUNK;
-    AO_REQUIRE((size_t)(3 * 128 + 32 + 64 * 128 + local + 8) * sizeof(float) <= 160 * 1024, "a cache of %lld positions over %d workgroups per head does not fit the kernel's LDS "
-               "score buffer: use a larger split", (long long)max_seq, nsplit);
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid((unsigned)n_head, (unsigned)nsplit);
     if (f16)

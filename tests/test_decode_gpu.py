@@ -401,6 +401,27 @@ def test_decode_attention_with_rising_scores(pos, nsplit, rise, dtype):
     assert rel_l2(out.float().cpu().view(2, 128).numpy(), (scores.softmax(-1) @ v).numpy()) <= (2**-8 if dtype is torch.bfloat16 else 2**-11)
 
 
+@pytest.mark.parametrize("S,nsplit,taken", [(31832, 1, True), (31833, 1, False), (32768, 1, False), (32768, 2, True), (32769, 2, False)])
+def test_decode_attention_cache_lengths(S, nsplit, taken):
+    """The longest caches that the entry points take, at their last position; longer ones are refused on the host."""
+    from ao_amd._lib import AoAmdError, check, current_stream, lib
+
+    gen = torch.Generator(device="cuda").manual_seed(S)
+    qkv, kc, vc = (torch.randn(*shape, device="cuda", generator=gen).bfloat16() for shape in ((4 * 128,), (S, 128), (S, 128)))
+    freqs = torch.zeros(S, 64, 2, device="cuda").bfloat16()
+    freqs[..., 0] = 1.0
+    pos, work, out = torch.tensor([S - 1], dtype=torch.int32, device="cuda"), torch.empty(2 * 2 * 130, device="cuda"), torch.empty(2, 128, device="cuda").bfloat16()
+    args = (qkv.data_ptr(), None, 0, freqs.data_ptr(), pos.data_ptr(), kc.data_ptr(), vc.data_ptr(), 2, 1, 128, S, nsplit, work.data_ptr(), out.data_ptr(),
+            current_stream(qkv.device))
+    if not taken:
+        with pytest.raises(AoAmdError, match="max_seq|larger split"):
+            check(lib().ao_amd_llama_decode_attention_split(*args))
+        return
+    check(lib().ao_amd_llama_decode_attention_split(*args))
+    want = (qkv[:256].double().view(2, 128) @ kc.double().t().contiguous() / 128**0.5).softmax(-1) @ vc.double()
+    assert rel_l2(out.float().cpu().numpy(), want.float().cpu().numpy()) <= 2**-8
+
+
 @pytest.mark.parametrize("S", [64, 4096])
 def test_decode_attention_from_partial_rows(S):
     """fp32 partial qkv rows are added and rounded to bf16 inside the attention kernel: same result as handing it the
