@@ -124,10 +124,11 @@ __device__ __forceinline__ void tiles_ahead(int kb, int KB, int stride, const Lo
     for (int n = kb + stride; n < KB; n += stride) {
         load(next, n);
         __builtin_amdgcn_sched_barrier(0);
-        compute(now);
+        compute(now, kb);
         now = next;
+        kb = n;
     }
-    compute(now);
+    compute(now, kb);
 }
 
 // Cross-lane reductions on the VALU's data-parallel-primitive path instead of ds_bpermute (an LDS round trip per

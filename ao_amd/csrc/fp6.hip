@@ -722,7 +722,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_kernel(const uint16_t* 
             acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa.v, w.v, acc, 0, 0, 0);
         }
     };
-    auto compute_tile = [&](const Buf& b) __attribute__((always_inline)) {
+    auto compute_tile = [&](const Buf& b, int = 0) __attribute__((always_inline)) {
         block_mfma(b.w0, sc2_0, b, acc0);
         if (RBW > 1) block_mfma(b.w1, sc2_1, b, acc1);
         if (RBW > 2) {
@@ -855,7 +855,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
             for (int sl = 0; sl < 4; ++sl) b.x[mb][sl] = xv[sl];
         }
     };
-    auto compute_tile = [&](const Buf& b) __attribute__((always_inline)) {
+    auto compute_tile = [&](const Buf& b, int = 0) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < RBW; ++j) {
             f16x32_t v;

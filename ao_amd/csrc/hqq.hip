@@ -256,47 +256,11 @@ __device__ __forceinline__ hqq_f32x4_t hqq_mfma(const u32x4_t a, const uint32_t 
     }
 }
 
-// One wave's run of steps, loaded AHEAD steps ahead into AHEAD + 1 fragment sets that are used in turn (a copy from the one to the other
-// was a seventh of the loop).  `load` makes the same requests whatever the step (past the end the last one's again): behind requests under a
-// condition the compiler waits for every request of the wave, and with them each step took the latency of its successor's: one row of 14336 x
-// 4096 19.3 -> 16.3 us, 16 rows 20.6 -> 18.4, 32 rows of 5120 x 5120 15.2 -> 13.0.
-// AHEAD 0: one ahead, with the copy and nothing requested past the end, for the short runs of 64 rows (14 requests a step: 1024 x
-// 4096 transposed 11.1 -> 10.2 us).
-template <class Frag, int AHEAD, class Load, class Compute>
-__device__ __forceinline__ void hqq_run(int s0, int s1, const Load& load, const Compute& compute) {
-    constexpr int SETS = AHEAD + 1;
-    if (s0 >= s1) return;
-    if constexpr (AHEAD == 0) {
-        Frag now, next;
-        load(s0, now);
-        for (int s = s0; s + 1 < s1; ++s) {
-            load(s + 1, next);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(s, now);
-            now = next;
-        }
-        return compute(s1 - 1, now);
-    }
-    Frag f[SETS];
-#pragma unroll
-    for (int i = 0; i < AHEAD; ++i) {
-        load(s0 + i < s1 ? s0 + i : s1 - 1, f[i]);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    for (int s = s0; s < s1; s += SETS)
-#pragma unroll
-        for (int i = 0; i < SETS; ++i) {
-            if (s + i >= s1) return;
-            load(s + i + AHEAD < s1 ? s + i + AHEAD : s1 - 1, f[(i + AHEAD) % SETS]);
-            __builtin_amdgcn_sched_barrier(0);
-            compute(s + i, f[i]);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-}
-
 // Waves of a workgroup: each takes a run of the reduction, and they add up in LDS.  A step's loads take a microsecond and a
-// wave keeps one or two steps ahead in flight, so the runs are kept short and the waves many; eight of them to a
-// workgroup keep the number of fp32 partial sums in memory where four waves with runs of eight steps had it.
+// wave keeps one step ahead in flight (tiles_ahead), so the runs are kept short and the waves many; eight of them to a
+// workgroup keep the number of fp32 partial sums in memory where four waves with runs of eight steps had it.  Two steps ahead up to 16 rows, in three
+// sets of fragments used in turn, took 14.8 / 15.8 us for one and 16 rows of fp16 14336 x 4096 where one takes 13.6 / 14.3, one ahead in two such sets 32 rows
+// transposed of 4096 x 11008 16.2 where the copy from set to set takes 15.4: the step's code stands once then.
 
 // RB (transposed product): blocks of 16 byte rows per wave.  With two of them in one quantization group the activation
 // fragments and the scales and zeros, 128 bytes a lane and step, serve 32 bytes of codes instead of 16.
@@ -335,7 +299,7 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
         const uint32_t eighths = (uint32_t)(group / 8);
         const int shift = (eighths & (eighths - 1)) == 0 ? __builtin_ctz(eighths) : -1;
         const int tail = K2 % 16 ? steps - 1 : -1;   // the step that ends before its 16 byte rows
-        auto load = [&](int s, Frag& f) __attribute__((always_inline)) {
+        auto load = [&](Frag& f, int s) __attribute__((always_inline)) {
             const int64_t at = (int64_t)s * 16 + 4 * q4, k2 = at < K2 ? at : K2 - 4;   // K is a multiple of 8: the lane's 4 byte rows exist together
             // group is a multiple of 8: one group for the lane's 8 k
             const uint32_t eighth = (uint32_t)k2 >> 2;
@@ -347,7 +311,7 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb) f.x[mb] = *reinterpret_cast<const u32x4_t*>(arow[mb] + 2 * k2);
         };
-        auto compute = [&](int s, Frag& f) __attribute__((always_inline)) {
+        auto compute = [&](Frag& f, int s) __attribute__((always_inline)) {
             if (s == tail && (int64_t)s * 16 + 4 * q4 >= K2) {   // 0 x (0 - 0) * 0
 #pragma unroll
                 for (int r = 0; r < 4; ++r) f.d[r] = 0u;
@@ -389,7 +353,7 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
             column(std::integral_constant<int, 2>());
             column(std::integral_constant<int, 3>());
         };
-        hqq_run<Frag, MB == 4 ? 0 : MB == 2 ? 1 : 2>(s0, s1, load, compute);
+        tiles_ahead<Frag>(s0, s1, 1, load, compute);
     } else {
         int64_t k2[RB];
         bool live[RB];
@@ -410,7 +374,7 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
             const int64_t at = (int64_t)s * 64 + 16 * q4;
             return at < N ? at : N - 16;   // N is a multiple of 16
         };
-        auto load = [&](int s, Frag& f) __attribute__((always_inline)) {
+        auto load = [&](Frag& f, int s) __attribute__((always_inline)) {
             const int64_t n = column(s);
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) f.d[rb] = *reinterpret_cast<const u32x4_t*>(prow[rb] + n);
@@ -420,7 +384,7 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
                 for (int h = 0; h < 2; ++h) f.x[mb][h] = *reinterpret_cast<const u32x4_t*>(arow[mb] + n + 8 * h);
         };
         const HqqRowMatrices rows(lane);
-        auto compute = [&](int s, Frag& f, u32x4_t (&sc)[2], u32x4_t (&ze)[2], auto element_wise) __attribute__((always_inline)) {
+        auto compute = [&](Frag& f, int s, u32x4_t (&sc)[2], u32x4_t (&ze)[2], auto element_wise) __attribute__((always_inline)) {
             if (s == tail && (int64_t)s * 64 + 16 * q4 >= N) {   // 0 x (0 - 0) * 0
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb) f.d[rb] = zero4;
@@ -538,7 +502,7 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
                     *reinterpret_cast<u32x4_t*>(z_lds + i * 512 + lane * 8) = in[1][i];
                 }
                 asm volatile("" ::: "memory");   // (one wave: its LDS operations are done in order)
-                hqq_run<Frag, MB == 4 ? 0 : MB == 2 ? 1 : 2>(c0, c1, load, [&](int s, Frag& f) __attribute__((always_inline)) {
+                tiles_ahead<Frag>(c0, c1, 1, load, [&](Frag& f, int s) __attribute__((always_inline)) {
                     const uint16_t* const at = s_lds + (s - c0) * 64 + 16 * q4;
                     u32x4_t sc[2], ze[2];
 #pragma unroll
@@ -546,7 +510,7 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
                         sc[h] = *reinterpret_cast<const u32x4_t*>(at + 8 * h);
                         ze[h] = *reinterpret_cast<const u32x4_t*>(at + CHUNK * 64 + 8 * h);
                     }
-                    compute(s, f, sc, ze, std::integral_constant<bool, !BF16>());
+                    compute(f, s, sc, ze, std::integral_constant<bool, !BF16>());
                 });
                 asm volatile("" ::: "memory");
             }
@@ -573,14 +537,14 @@ __global__ __launch_bounds__(64 * WAVES) void hqq_mm_mfma_kernel(const uint8_t* 
             for (int s = s0; s < s1; ++s) {
                 Frag f;
                 u32x4_t sc[2], ze[2];
-                load(s, f);
+                load(f, s);
                 const int64_t n = column(s);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     sc[h] = *reinterpret_cast<const u32x4_t*>(srow + n + 8 * h);
                     ze[h] = *reinterpret_cast<const u32x4_t*>(zrow + n + 8 * h);
                 }
-                compute(s, f, sc, ze, std::true_type());
+                compute(f, s, sc, ze, std::true_type());
             }
     }
 

@@ -368,7 +368,7 @@ __global__ __launch_bounds__(WAVES * 64) void int8wo_linear_rb4_kernel(const Int
             for (int sl = 0; sl < 4; ++sl) b.x[mb][sl] = xv[sl];
         }
     };
-    auto compute_tile = [&](const Buf& b) {
+    auto compute_tile = [&](const Buf& b, int) {
 #pragma unroll
         for (int sl = 0; sl < 4; ++sl) {
 #pragma unroll
