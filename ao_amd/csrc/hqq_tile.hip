@@ -420,13 +420,13 @@ HqqTilePlan hqq_tile_plan(int64_t M, int64_t K, int64_t N, int64_t group, bool t
 // 4096 x 32000 of fp16 at 512 193 / 198).
 // Up to 64 rows the other one is the streaming kernel of hqq.hip, timed against the tiles on 31 weights from 4096 x 4096 to 14336 x 14336 and 4096 x
 // 128256, groups of 64.  Its time is estimated from its plan's costs, the weight and the rows times the weight (the activations are read again for every 64
-// columns), with the factors that lose least by choosing wrong: 0.2 % of the best of both over all of them (3.2 % of bf16 and 1.4 % of fp16 forward by the
-// weight's size and a lead), and no tiles where they were never ahead.  us streamed / tiled, forward, bf16 (K x N): one row 8192 x 8192 16.4 / 19.0, 5120 x 13824 18.6 / 20.3,
-// 4096 x 32000 27.8 / 26.8; 17 rows 14336 x 4096 16.0 / 18.8, 13824 x 5120 19.3 / 25.6, 8192 x 28672 50.7 / 48.0; 33 rows 4096 x 4096 10.7 / 13.8, 13824 x 5120 22.8 / 28.9,
-// 5120 x 13824 23.9 / 23.3; 64 rows 13824 x 5120 28.6 / 29.9, 4096 x 11008 24.7 / 22.0.  fp16: 32 rows 13824 x 5120 20.7 / 22.8, 5120 x 13824 20.3 / 19.0.  Transposed,
-// fp16: 17 rows 8192 x 28672 38.6 / 42.1, 32 rows 48.1 / 42.6, 40 rows 4096 x 11008 18.8 / 19.0, 11008 x 4096 21.9 / 20.2; bf16, whose rule is the older one (0.3 % lost): 33 / 64 rows
-// 8192 x 28672 55.0 / 64.6, 71.9 / 64.9, 14336 x 4096 22.0 / 24.8, 26.7 / 26.0.  What is chosen wrong by most: 4096 x 65536 of bf16 at 8 rows 56.4 / 51.3, transposed fp16 8192 x
-// 4096 at 56 rows 16.6 / 14.6.
+// columns), with the factors that lose least by choosing wrong: 0.3 % of the best of both over all of them (3.2 % of bf16 and 1.4 % of fp16 forward by the
+// weight's size and a lead), and no tiles where they were never ahead.  us streamed / tiled, forward, bf16 (K x N): one row 8192 x 8192 15.7 / 18.8, 5120 x 13824 18.0 / 20.3,
+// 4096 x 32000 27.4 / 26.9; 17 rows 14336 x 4096 16.3 / 18.8, 13824 x 5120 19.4 / 25.7, 24 rows 8192 x 28672 52.3 / 47.5; 33 rows 4096 x 4096 10.6 / 13.7, 13824 x 5120 23.3 / 29.1,
+// 5120 x 13824 23.7 / 23.2; 64 rows 13824 x 5120 28.5 / 29.6, 4096 x 11008 24.7 / 21.8.  fp16: 32 rows 13824 x 5120 20.2 / 22.6, 5120 x 13824 20.0 / 18.8.  Transposed,
+// fp16: 17 rows 8192 x 28672 36.6 / 42.3, 32 rows 44.9 / 42.2, 40 rows 4096 x 11008 18.6 / 19.0, 11008 x 4096 21.8 / 20.0; bf16, whose rule is an older one (0.3 % lost): 33 / 64 rows
+// 8192 x 28672 54.6 / 64.3, 71.2 / 64.1, 14336 x 4096 21.7 / 24.5, 26.4 / 25.5.  Chosen wrong by most: transposed bf16 18944 x 3584 at 48 rows 38.5 / 33.0, fp16 8192 x 4096 at
+// 56 rows 16.6 / 14.5; forward bf16 8192 x 28672 at 16 rows 43.7 / 47.6.
 HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool transposed, bool bf16) {
     const HqqTilePlan none{0, 0, 0, 1, 1e30};
     const double weights = (double)K * (double)N, rows = (double)M, flops = 2.0 * rows * weights;
@@ -447,8 +447,8 @@ HqqTilePlan hqq_tile_route(int64_t M, int64_t K, int64_t N, int64_t group, bool 
     } else {
         // constant, factor of the plan's costs, us a million weights, a row more; up to 32 rows and beyond
         static const double by[3][2][4] = {{{3.4, 0.23, 0.13, 0.0022}, {3.1, 0.70, -0.002, 0.0030}},       // forward, fp16
-                                           {{4.4, 0.73, 0.013, 0.0007}, {1.8, 1.12, -0.064, 0.0018}},      // forward, bf16
-                                           {{6.3, 0.70, 0.020, 0.0014}, {4.4, 1.11, -0.021, 0.0017}}};     // transposed, fp16
+                                           {{4.9, 0.56, 0.053, 0.0009}, {1.8, 1.12, -0.064, 0.0018}},      // forward, bf16
+                                           {{4.6, 0.65, -0.002, 0.0026}, {4.4, 1.11, -0.021, 0.0017}}};    // transposed, fp16
         const double* c = by[transposed ? 2 : bf16][M > 32];
         other = c[0] + c[1] * hqq_stream_us(M, K, N, group, transposed) + (c[2] + c[3] * rows) * weights * 1e-6;
     }
