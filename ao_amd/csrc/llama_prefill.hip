@@ -408,7 +408,8 @@ __device__ __forceinline__ float silu(float x) {
 }
 
 // out = silu(gate) * up, 8 elements per thread; silu is rounded to the element type before the product, as F.silu leaves it.
-// 1000 x 14336 in 16.5 us, 5.2 TB/s, the rate of a copy; with expf and a division 18.9.
+// 1000 x 14336, six sets of buffers in turn, 17.6 us, 4.9 TB/s, close to the rate of a copy; with expf and a division 18.5, with one Newton step on the
+// reciprocal 17.4 (one set of buffers 16.5 / 18.9 / 17.3).
 template <class E>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* gate, const uint16_t* __restrict__ up, int64_t n8,
                                                        uint16_t* out) {
