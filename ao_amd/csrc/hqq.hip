@@ -588,7 +588,7 @@ static HqqMfmaPlan hqq_mfma_plan(int64_t M, int64_t K, int64_t N, bool transpose
     // Cheapest by a measured model (in us, 1 to 64 rows, 4096 and 11008 wide): a CU takes 0.12 us for a kilobyte of codes with
     // all its waves together, eight at least, plus the start of each run, and its workgroups come in whole rounds; a slice costs its fp32 partial
     // sums, written and read.  (With 0.15 us and half the start, from when every step waited for the next one's requests, 32 rows
-    // transposed of 11008 x 4096 took 22.6 us, now 19.8, and one row 16.0, now 13.8; eight weights at 1 to 48 rows are level on average.)
+    // transposed of 11008 x 4096 took 22.6 us, with these 19.8, and one row 16.0, 13.8; by the present loop 17.6 and 12.6.)
     // Two blocks of 16 byte rows (64 values of k) per wave in the transposed product where they share their group.
     // Transposed products whose groups leave one block row to a wave keep those costs: short chunks of scales, or (groups that are no multiple of 32)
     // scales that each lane requests itself, with no step ahead: 13824 x 5120 at one row in groups of 8 21.3 us at the lower costs, 19.3 at

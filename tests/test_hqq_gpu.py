@@ -458,27 +458,28 @@ def test_transposed_product_with_a_special_zero(M, N, K, g, special):
 
 @pytest.mark.parametrize("special", [2.0**126, 2.0**100, 2.0**-125, 2.0**-60, 0.0, float("inf"), float("nan")])
 @pytest.mark.parametrize("of", ["scale", "zero"])
-@pytest.mark.parametrize("M,N,K", [(1, 80, 64), (20, 1104, 96), (40, 528, 320)])
-def test_transposed_product_with_scales_of_any_size(M, N, K, of, special):
+@pytest.mark.parametrize("M,N,K,g", [(1, 80, 64, 32), (20, 1104, 96, 32), (40, 528, 320, 32), (1, 80, 8320, 64), (20, 1104, 8320, 64), (40, 528, 8320, 64)])
+def test_transposed_product_with_scales_of_any_size(M, N, K, g, of, special):
     """A weight beyond the largest bf16 is infinite and one below the smallest normal keeps its bits, whichever way the kernel applies scales
-    and zeros: groups of 16 do it element by element, groups of 32 with matrix instructions.  Both add in the same order: equal bits."""
+    and zeros: groups of 16 do it element by element, groups of 32 (one block row) and 64 (two, where there are many) with matrix instructions.  Two
+    columns count, so that the order of the sums does not: equal bits."""
     from ao_amd import ops
     from ao_amd.prototype.hqq import pack_2xint4
 
     dev, gen = _dev(), torch.Generator().manual_seed(M + N)
     codes = torch.randint(0, 16, (K, N), dtype=torch.uint8, generator=gen)
-    s, z = (torch.rand(K // 32, N, generator=gen) * 8 + 4).bfloat16(), (torch.rand(K // 32, N, generator=gen) * 6 + 5).bfloat16()
+    s, z = (torch.rand(K // g, N, generator=gen) * 8 + 4).bfloat16(), (torch.rand(K // g, N, generator=gen) * 6 + 5).bfloat16()
     x = torch.zeros(M, N).bfloat16()
     for n in (6, N - 3):   # the first and the last of a wave's steps
         codes[::2, n] = 0
         (s if of == "scale" else z)[-1, n] = special
         x[:, n] = torch.randn(M, generator=gen).bfloat16() * 2.0**-8
     packed, s, z, x = pack_2xint4(codes).to(dev), s.to(dev), z.to(dev), x.to(dev)
-    got = ops.hqq_mixed_mm_mfma(x, packed, s, z, 32, True)
-    want = ops.hqq_mixed_mm_mfma(x, packed, s.repeat_interleave(2, 0), z.repeat_interleave(2, 0), 16, True)
+    got = ops.hqq_mixed_mm_mfma(x, packed, s, z, g, True)
+    want = ops.hqq_mixed_mm_mfma(x, packed, s.repeat_interleave(g // 16, 0), z.repeat_interleave(g // 16, 0), 16, True)
     assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0, 3e38, -3e38), want.nan_to_num(7.0, 3e38, -3e38))
     # and the reference's roundings, where the sums stay in range
-    w = ops.hqq_dequantize(packed, s, z, 32).float()
+    w = ops.hqq_dequantize(packed, s, z, g).float()
     ref = (x.float() @ w.t().contiguous()).to(torch.bfloat16)
     ok = ref.isfinite() & (ref.abs() > 2.0**-110)
     assert ((got.float() - ref.float()).abs()[ok] <= 2.0**-7 * ref.float().abs()[ok]).all()
