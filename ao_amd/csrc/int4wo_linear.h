@@ -151,6 +151,11 @@ struct Int4Plan {
 bool int4wo_plain_kernel(int64_t M, int64_t K, int64_t N, int64_t g, Int4Kernel* kernel);
 // Whether the dispatch reads activation rows of a multiple of 8 elements that end before the packed width as they are
 bool int4wo_takes_short_rows(int64_t M, int64_t N, int64_t g);
+// The product of 4 to 32 plain rows with K split over workgroups that take four row blocks each: how many parts serve a call best (1: no split),
+// and the launches, whose workspace holds parts x M x N fp32 sums
+int int4wo_stream_parts(int64_t M, int64_t K, int64_t N, int64_t g);
+int int4wo_linear_stream_parts(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams, int64_t N, int64_t g,
+                               const void* bias_bf16, void* y, int y_dtype, int64_t ldy, int parts, void* workspace, void* stream);
 // The plain product on contiguous rows of the packed width that a kernel on the same stream has just written: another order of the tiles
 int int4wo_linear_copied_rows(const void* x_bf16, int64_t M, int64_t K, const void* packed, const void* qparams, int64_t N, int64_t g,
                               const void* bias_bf16, void* y, int y_dtype, int64_t ldy, void* stream);

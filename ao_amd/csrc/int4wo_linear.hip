@@ -372,7 +372,9 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
     const int r = lane & 15, qd = lane >> 4;
     const int64_t rb0 = (int64_t)blockIdx.x * RBW;
     const int64_t m0 = (int64_t)blockIdx.y * (16 * MB);
-    const int KP = (int)(a.Kp / 128), KB = EDGE ? (int)((a.K + 127) / 128) : KP;   // (g = 256: the packed row may go on)
+    // this workgroup's K tiles, kb0 .. kb0 + KB - 1: all of them or, with K parts, the blockIdx.z-th run
+    const int KP = (int)(a.Kp / 128), KA = EDGE ? (int)((a.K + 127) / 128) : KP;   // (g = 256: the packed row may go on)
+    const int kb0 = (int)blockIdx.z * a.kb_per_split, KB = KA - kb0 < a.kb_per_split ? KA - kb0 : a.kb_per_split;
     // a row block past the end repeats the last one and is not stored
     auto row_block = [&](int j) __attribute__((always_inline)) {
         const int64_t last = (a.N + 15) / 16 - 1;
@@ -463,10 +465,10 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
     const int nt = wave < KB ? (KB - wave + WAVES - 1) / WAVES : 0;
     if constexpr (AHEAD) {   // (tiles_ahead, whose loop counts in tiles of K, is compiled to 4 % more at 16 rows: 14336 x 4096 11.9 -> 12.4 us)
         if (nt > 0) {
-            load_tile(buf, wave);
+            load_tile(buf, kb0 + wave);
             for (int i = 1; i < nt; ++i) {
                 Buf next;
-                load_tile(next, wave + i * WAVES);
+                load_tile(next, kb0 + wave + i * WAVES);
                 __builtin_amdgcn_sched_barrier(0);
                 compute_tile(buf);
                 buf = next;
@@ -475,7 +477,7 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
         }
     } else {
         for (int i = 0; i < nt; ++i) {
-            load_tile(buf, wave + i * WAVES);
+            load_tile(buf, kb0 + wave + i * WAVES);
             compute_tile(buf);
         }
     }
@@ -504,7 +506,7 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
                 if (m < a.M && n < a.N) {
                     sum += bv;
                     if (a.residual) sum = rne_bf16(sum) + bf16_bits_to_f32(a.residual[m * a.ldres + n]);
-                    if (a.y_is_f32) ((float*)a.y)[m * a.ldy + n] = sum;
+                    if (a.y_is_f32) ((float*)a.y)[((int64_t)blockIdx.z * a.M + m) * a.ldy + n] = sum;
                     else ((uint16_t*)a.y)[m * a.ldy + n] = f32_to_bf16_bits(sum);
                 }
             }
@@ -1172,6 +1174,31 @@ static void launch_group(int64_t g, int waves, dim3 grid, size_t smem, hipStream
     }
 }
 
+template <int G, int MB>
+static void launch_rb4_one(int waves, bool edge, bool ahead, dim3 grid, hipStream_t st, const LinearArgs& a) {
+    auto go = [&](auto kernel) { launch_timed(kernel, grid, dim3(waves * 64), 0, st, a); };
+    if (ahead) go(int4wo_linear_rb4_kernel<G, 8, 1, false, true>);
+    else if (waves == 4 && !edge) go(int4wo_linear_rb4_kernel<G, 4, MB, false>);
+    else if (waves == 4) go(int4wo_linear_rb4_kernel<G, 4, MB, true>);
+    else if (!edge) go(int4wo_linear_rb4_kernel<G, 8, MB, false>);
+    else go(int4wo_linear_rb4_kernel<G, 8, MB, true>);
+}
+template <int G>
+static void launch_rb4_rows(int waves, int mb, bool edge, bool ahead, dim3 grid, hipStream_t st, const LinearArgs& a) {
+    if (mb == 1) launch_rb4_one<G, 1>(waves, edge, ahead, grid, st, a);
+    else if (mb == 2) launch_rb4_one<G, 2>(waves, edge, ahead, grid, st, a);
+    else launch_rb4_one<G, 4>(waves, edge, ahead, grid, st, a);
+}
+// grid: groups of four row blocks, chunks of 16 mb rows, K parts
+static void launch_rb4(int64_t g, int waves, int mb, bool edge, bool ahead, dim3 grid, hipStream_t st, const LinearArgs& a) {
+    switch (g) {
+        case 32: launch_rb4_rows<32>(waves, mb, edge, ahead, grid, st, a); break;
+        case 64: launch_rb4_rows<64>(waves, mb, edge, ahead, grid, st, a); break;
+        case 128: launch_rb4_rows<128>(waves, mb, edge, ahead, grid, st, a); break;
+        default: launch_rb4_rows<256>(waves, mb, edge, ahead, grid, st, a); break;
+    }
+}
+
 // 17 and more rows on int4wo_linear_rb4_kernel: from 768 row blocks on, up to this many
 static int64_t int4wo_rb4_max_rows(int64_t RB) { return RB >= 4096 ? 64 : 48; }
 // Rows that end before the packed width: the single-row kernel and the two whose lanes load their own activation fragments fill up
@@ -1375,33 +1402,7 @@ static int linear_dispatch(const void* x_bf16, int64_t M, int64_t K, int64_t ldx
             const bool ahead = !edge && w4 == 8 && mb == 1 && wgs <= 256 && a.Kp >= 4096;
             if (mb == 1) AO_PLAN(Int4Kernel::streaming, "int4wo_linear_rb4_kernel<%lld,%d>%s", (long long)g, w4, w4 == 8 && !ahead ? " tile by tile" : "");
             AO_PLAN(Int4Kernel::streaming, "int4wo_linear_rb4_kernel<%lld,%d,%d>", (long long)g, w4, mb);
-            const dim3 grid4((unsigned)((RB + 3) / 4), (unsigned)mch);
-            auto go = [&](auto kernel, int nw) {
-                if (g_prof_start && g_prof_stop) {
-                    hipExtLaunchKernelGGL(kernel, grid4, dim3(nw * 64), 0, st, g_prof_start, g_prof_stop, 0, a);
-                    g_prof_start = g_prof_stop = nullptr;
-                } else {
-                    hipLaunchKernelGGL(kernel, grid4, dim3(nw * 64), 0, st, a);
-                }
-            };
-#define AO_RB4_MB(GG, MBV)                                                 \
-    if (ahead) go(int4wo_linear_rb4_kernel<GG, 8, 1, false, true>, 8);     \
-    else if (w4 == 4 && !edge) go(int4wo_linear_rb4_kernel<GG, 4, MBV, false>, 4); \
-    else if (w4 == 4) go(int4wo_linear_rb4_kernel<GG, 4, MBV, true>, 4);   \
-    else if (!edge) go(int4wo_linear_rb4_kernel<GG, 8, MBV, false>, 8);    \
-    else go(int4wo_linear_rb4_kernel<GG, 8, MBV, true>, 8)
-#define AO_RB4(GG)                                                         \
-    if (mb == 1) { AO_RB4_MB(GG, 1); }                                     \
-    else if (mb == 2) { AO_RB4_MB(GG, 2); }                                \
-    else { AO_RB4_MB(GG, 4); }
-            switch (g) {
-                case 32: AO_RB4(32); break;
-                case 64: AO_RB4(64); break;
-                case 128: AO_RB4(128); break;
-                default: AO_RB4(256); break;
-            }
-#undef AO_RB4
-#undef AO_RB4_MB
+            launch_rb4(g, w4, mb, edge, ahead, dim3((unsigned)((RB + 3) / 4), (unsigned)mch), st, a);
             AO_LAUNCH_CHECK();
             return 0;
         }
@@ -1473,6 +1474,14 @@ int ao::int4wo_linear_copied_rows(const void* x_bf16, int64_t M, int64_t K, cons
                            false, 1, nullptr, true);
 }
 
+static void launch_ws_finish(const float* parts, int z, int64_t M, int64_t N, const void* bias_bf16, void* y, int y_dtype, int64_t ldy, hipStream_t st) {
+    const dim3 grid((unsigned)((M * N / 4 + 255) / 256));
+    if (y_dtype == AO_F32)
+        hipLaunchKernelGGL(int4wo_ws_finish_kernel<true>, grid, dim3(256), 0, st, parts, z, M, N, (const uint16_t*)bias_bf16, y, ldy);
+    else
+        hipLaunchKernelGGL(int4wo_ws_finish_kernel<false>, grid, dim3(256), 0, st, parts, z, M, N, (const uint16_t*)bias_bf16, y, ldy);
+}
+
 // K split over workgroups through a caller's workspace: where it is used and how many parts.  The fp32 partial outputs
 // cost 8 bytes per output and part (written, then read by the finish kernel) and a second, small launch (about 3 us
 // with its gap), so the split is kept for grids of the 32- and 64-row tiles that leave most CUs idle.  Measured, group
@@ -1501,6 +1510,73 @@ static int ws_parts(int64_t M, int64_t K, int64_t N, int64_t g) {
     while (z > 1 && (int64_t)(z - 1) * ((KB + z - 1) / z) >= KB) --z;
     if (z > KB) z = (int)KB;
     return z < 1 ? 1 : z;
+}
+
+// Four row blocks a workgroup and K split over workgroups, for 4 to 32 rows of weights that have too few row blocks for the kernel to
+// fill the chip with all of K (768, linear_dispatch).  One block a workgroup reads all activation rows once per 16 weight rows, at 16
+// rows 3.5 times the bytes of its codes, and from 17 rows on the weight, or one of few tiles, twice: 28 us of 5120 x 13824 at 13 rows for
+// a weight that memory delivers in 8.  With parts the row is read once per 64 weight rows and a CU has one workgroup with a part of K;
+// the second launch, which adds the fp32 sums, costs about 3 us.  us before / in parts, g = 64: 5120 x 13824 at 8 / 13 / 16 / 20 rows 21.4 /
+// 16.4, 28.1 / 16.5, 24.9 / 17.3, 24.4 / 19.3; 2048 x 16384 at 8 / 16 / 20 rows 14.6 / 12.4, 20.3 / 12.7, 20.7 / 14.2; 10240 x 8192 at 8 / 16 rows 21.8 / 19.0,
+// 28.8 / 19.5; 8192 x 8192 at 16 rows 19.0 / 15.8; 7168 x 5120 at 11 / 20 rows 12.2 / 11.1, 20.5 / 13.5; 4096 x 14336 at 10 / 16 rows 15.4 / 14.7,
+// 17.2 / 14.8; 3072 x 8192 at 20 rows 16.6 / 12.4.  Not where it lost: 4096 x 4096 at 10 / 16 rows 7.1 / 8.4, 8.1 / 8.9, 4096 x 8192 at 8 rows 9.7 / 10.9.
+// The estimates below (us; a part's K tiles, rows, row blocks) are within 6 % of those calls, and the parts have to lead.
+int ao::int4wo_stream_parts(int64_t M, int64_t K, int64_t N, int64_t g) {
+    if (M < 4 || M > 32 || N % 4 != 0) return 1;
+    int64_t Np, Kp;
+    if (ao_amd_int4wo_packed_shape(N, K, g, &Np, &Kp, nullptr, nullptr) || Kp != K) return 1;
+    const int64_t KB = Kp / 128, RB = Np / 16, groups = (RB + 3) / 4;
+    if (groups >= 192 || KB < 8 || KB >= (1 << 21)) return 1;
+    const double m = (double)M;
+    auto whole = [&]() {   // one row block a workgroup, 16 rows at a time
+        const int64_t chunks = RB * ((M + 15) / 16);
+        return 4.0 + (double)((chunks + 255) / 256) * (double)KB * (0.029 + 0.0061 * (M < 16 ? m : 16.0));
+    };
+    double other = whole();
+    if (M > 16) {
+        const int z = ws_parts(M, K, N, g);
+        if (z > 1) other = 7.4 + 0.33 * (double)((KB + z - 1) / z);
+        else if (groups >= 128) other = 4.0 + 0.33 * (double)KB;   // 32 x 64 tiles
+    }
+    int best = 1;
+    double us = (M > 16 ? 0.88 : 0.97) * other;
+    for (int z = 2; z <= 8; ++z) {
+        const int64_t per = (KB + z - 1) / z, wgs = groups * z;
+        if (per < 4 || (z - 1) * per >= KB || wgs > (M > 16 ? 256 : 512)) continue;   // (105 registers a lane up to 16 rows: two workgroups share a CU)
+        const double t = M > 16 ? 6.2 + 0.05 * m + 0.35 * (double)per + 0.12 * z
+                                : 5.0 + 0.03 * m + 0.32 * (double)per * (wgs > 256 ? 1.95 : 1.0) + 0.2 * z;
+        if (t < us) {
+            us = t;
+            best = z;
+        }
+    }
+    return best;
+}
+
+int ao::int4wo_linear_stream_parts(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams, int64_t N, int64_t g,
+                                   const void* bias_bf16, void* y, int y_dtype, int64_t ldy, int parts, void* workspace, void* stream) {
+    AO_REQUIRE(x_bf16 && packed && qparams && y && workspace, "null pointer argument");
+    AO_REQUIRE(y_dtype == AO_BF16 || y_dtype == AO_F32, "output dtype must be bf16 or f32, got code %d", y_dtype);
+    AO_REQUIRE(ldx >= K && ldy >= N, "row strides (ldx=%lld, ldy=%lld) smaller than the rows (K=%lld, N=%lld)", (long long)ldx, (long long)ldy,
+               (long long)K, (long long)N);
+    AO_REQUIRE((((uintptr_t)packed) & 15) == 0 && (((uintptr_t)x_bf16) & 15) == 0 && (ldx & 7) == 0,
+               "packed codes and activation rows must be 16-byte aligned");
+    int64_t Np, Kp;
+    if (int rc = ao_amd_int4wo_packed_shape(N, K, g, &Np, &Kp, nullptr, nullptr)) return rc;
+    // (g = 256: the packed row may have a tile more than K reaches)
+    const int64_t KB = (K + 127) / 128, RB = Np / 16, per = (KB + parts - 1) / parts;
+    AO_REQUIRE(M > 0 && M <= 32 && K % 8 == 0 && N % 4 == 0 && parts >= 1 && parts <= 8 && (parts - 1) * per < KB,
+               "no such split (M=%lld N=%lld K=%lld parts=%d)", (long long)M, (long long)N, (long long)K, parts);
+    LinearArgs a{};
+    a.x = (const uint16_t*)x_bf16; a.M = M; a.K = K; a.Kp = Kp; a.ldx = ldx;
+    a.packed = (const uint4*)packed; a.qparams = (const uint32_t*)qparams; a.N = N;
+    a.y = workspace; a.y_is_f32 = 1; a.ldy = N;
+    a.ksplit = parts; a.kb_total = (int)KB; a.kb_per_split = (int)per;
+    hipStream_t st = (hipStream_t)stream;
+    launch_rb4(g, 8, M > 16 ? 2 : 1, RB % 4 != 0 || K != Kp, false, dim3((unsigned)((RB + 3) / 4), 1, (unsigned)parts), st, a);
+    launch_ws_finish((const float*)workspace, parts, M, N, bias_bf16, y, y_dtype, ldy, st);
+    AO_LAUNCH_CHECK();
+    return 0;
 }
 
 extern "C" int ao_amd_int4wo_linear_ws_bytes(int64_t M, int64_t K, int64_t N, int64_t g, int64_t* bytes) {
@@ -1532,15 +1608,7 @@ extern "C" int ao_amd_int4wo_linear_ws(const void* x_bf16, int64_t M, int64_t K,
     if (int rc = linear_dispatch(x_bf16, M, K, ldx, packed, qparams, nullptr, nullptr, N, g, nullptr, nullptr, 0, workspace,
                                  AO_F32, N, stream, nullptr, 0.f, false, z))
         return rc;
-    const int64_t quads = M * N / 4;
-    const dim3 grid((unsigned)((quads + 255) / 256));
-    hipStream_t st = (hipStream_t)stream;
-    if (y_dtype == AO_F32)
-        hipLaunchKernelGGL(int4wo_ws_finish_kernel<true>, grid, dim3(256), 0, st, (const float*)workspace, z, M, N,
-                           (const uint16_t*)bias_bf16, y, ldy);
-    else
-        hipLaunchKernelGGL(int4wo_ws_finish_kernel<false>, grid, dim3(256), 0, st, (const float*)workspace, z, M, N,
-                           (const uint16_t*)bias_bf16, y, ldy);
+    launch_ws_finish((const float*)workspace, z, M, N, bias_bf16, y, y_dtype, ldy, (hipStream_t)stream);
     AO_LAUNCH_CHECK();
     return 0;
 }

@@ -194,10 +194,11 @@ struct Int4Auto {
     bool tiled;
     bool as_is;           // the plain kernel reads the rows itself: nothing is copied (the workspace keeps the size that callers know)
     int64_t Kp;           // the width of the copied rows, 0: read as they are
+    int stream_parts;     // K parts of the streaming kernel with four row blocks, 1: not split
     int64_t copy, parts;  // bytes
 };
 static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t N, int64_t g, int y_dtype, Int4Auto* r) {
-    *r = Int4Auto{false, false, 0, 0, 0};
+    *r = Int4Auto{false, false, 0, 1, 0, 0};
     const bool aligned = (ldx & 7) == 0 && (((uintptr_t)x) & 15) == 0;
     if (M > 32 && y_dtype == AO_BF16 && aligned && 256 * ldx * 2 < ((int64_t)1 << 32)) {
         int64_t need = -1;
@@ -219,6 +220,11 @@ static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t
         r->Kp = Kp;
         r->copy = M * Kp * 2;
         r->as_is = aligned && K % 8 == 0 && int4wo_takes_short_rows(M, N, g);
+    }
+    r->stream_parts = (K == Kp && aligned) || r->Kp ? int4wo_stream_parts(M, Kp, N, g) : 1;
+    if (r->stream_parts > 1) {
+        r->parts = r->stream_parts * M * N * (int64_t)sizeof(float);
+        return 0;
     }
     return ao_amd_int4wo_linear_ws_bytes(M, r->Kp ? Kp : K, N, g, &r->parts);
 }
@@ -323,13 +329,16 @@ extern "C" int ao_amd_int4wo_linear_auto(const void* x_bf16, int64_t M, int64_t 
                (long long)workspace_bytes);
     if (r.tiled)
         return ao_amd_int4wo_linear_tiled(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, ldy, workspace, r.parts, stream);
-    if (r.as_is) return ao_amd_int4wo_linear(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, stream);
-    if (r.Kp) {
+    if (r.as_is && r.stream_parts == 1) return ao_amd_int4wo_linear(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, stream);
+    if (r.Kp && !r.as_is) {
         if (int rc = ao_amd_pad_rows(x_bf16, M, K, ldx, r.Kp, workspace, stream)) return rc;
         x_bf16 = workspace;
         K = ldx = r.Kp;
         if (!r.parts) return int4wo_linear_copied_rows(x_bf16, M, K, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, stream);
     }
+    if (r.stream_parts > 1)
+        return int4wo_linear_stream_parts(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, r.stream_parts,
+                                          (uint8_t*)workspace + r.copy, stream);
     if (!r.parts) return ao_amd_int4wo_linear(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, stream);
     return ao_amd_int4wo_linear_ws(x_bf16, M, K, ldx, packed, qparams, N, g, bias_bf16, y, y_dtype, ldy, (uint8_t*)workspace + r.copy,
                                    r.parts, stream);

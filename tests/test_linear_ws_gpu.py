@@ -109,6 +109,45 @@ def test_workspace_linear_refusals_and_fallbacks():
     assert rc == 0 and bool(torch.equal(ops.int4wo_linear(x, packed, qp, g, N), y_ws))
 
 
+# (N, K, group, M, K parts): an even split and a last part that is shorter; row blocks that are no multiple of four, the last one with 4 rows;
+# more workgroups than CUs; rows that end before the packed width, read as they are (up to 15) and copied; g = 256 with a packed tile that no row
+# reaches; 4, 16, 17 and 32 rows; and neighbours of those calls that are not split
+@pytest.mark.parametrize("N,K,g,M,parts", [
+    (8192, 8192, 64, 16, 2), (5120, 13824, 64, 4, 1), (5120, 13824, 64, 6, 3), (5120, 13824, 32, 13, 3), (5120, 13824, 128, 17, 3),
+    (5120, 13824, 64, 32, 3), (5120, 13824, 64, 33, 0), (10240, 8192, 64, 16, 3), (1000, 14336, 128, 16, 8), (2052, 16384, 256, 16, 7),
+    (5000, 8000, 256, 13, 3), (5000, 8000, 256, 20, 3), (5120, 13768, 128, 15, 3), (5120, 13768, 128, 18, 3), (4096, 4096, 64, 16, 1)])
+def test_few_rows_of_narrow_weights_in_parts(N, K, g, M, parts):
+    from ao_amd import _lib, ops
+
+    print(f"case int4 rows in parts N={N} K={K} g={g} M={M} parts={parts}", flush=True)
+    L, need = _lib.lib(), ctypes.c_int64(-1)
+    packed, qp, dq = _setup(N, K, g, seed=N + K + g)
+    gen = torch.Generator().manual_seed(M)
+    x, bias = torch.randn(M, K, generator=gen).bfloat16().cuda(), torch.randn(N, generator=gen).bfloat16().cuda()
+    q = max(128, g)
+    copy = 2 * M * (-(-K // q) * q) if K % q else 0
+    if parts:   # (0: another route's)
+        _lib.check(L.ao_amd_int4wo_linear_auto_bytes(x.data_ptr(), M, K, K, N, g, _lib.BF16, ctypes.byref(need)))
+        assert need.value == copy + (4 * parts * M * N if parts > 1 else 0)
+    for b in (None, bias):
+        ref = x.float() @ dq.float().t() + (0 if b is None else b.float())
+        y, y32 = ops.int4wo_linear(x, packed, qp, g, N, b), ops.int4wo_linear(x, packed, qp, g, N, b, True)
+        # one rounding to bf16 (2^-9 / sqrt 3 relative, 1.1e-3 against the unrounded, almost nothing against the rounded sum); fp32 sums of K terms
+        assert float((y.float() - ref.bfloat16().float()).norm() / ref.norm()) <= 1e-3
+        assert float((y32 - ref).norm() / ref.norm()) <= 2e-5
+    # one-hot rows read single columns of the dequantized weight back, bit for bit, at both ends of K and of every part
+    ks = torch.randint(0, K, (M,), generator=gen)
+    ks[0], ks[-1] = 0, K - 1
+    if parts > 1:
+        per = -(-(-(-K // 128)) // parts) * 128
+        for z in range(1, parts):
+            if 2 * z < M - 1:
+                ks[2 * z - 1], ks[2 * z] = z * per - 1, z * per
+    xh = torch.zeros(M, K, dtype=torch.bfloat16)
+    xh[torch.arange(M), ks] = 1.0
+    assert torch.equal(ops.int4wo_linear(xh.cuda(), packed, qp, g, N), dq[:, ks.cuda()].t().contiguous())
+
+
 # (N, K, M, parts the rule gives) for ao_amd_fp6_linear_ws
 FP6_CASES = [
     (4096, 14336, 16, 4), (4096, 14336, 32, 4), (4096, 14336, 64, 4), (4096, 14336, 100, 2), (4096, 14336, 256, 1),
