@@ -360,7 +360,8 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_kernel(const LinearA
 // others 2 to 5 %).
 // AHEAD: the next tile is requested before the present one is multiplied, for launches that leave one workgroup to a CU: 14336 x 4096 at 6 / 16 rows
 // 12.6 -> 11.4, 13.8 -> 13.2 us, 13824 x 8192 at 6 rows 22.5 -> 20.4, 12288 x 4096 12.8 -> 11.6.  From 17 rows on (two blocks) it gave nothing.
-template <int G, int WAVES, int MB, bool EDGE, bool AHEAD = false>
+// SPLIT: the workgroup takes the blockIdx.z-th run of a.kb_per_split K tiles and leaves fp32 sums (int4wo_stream_parts).
+template <int G, int WAVES, int MB, bool EDGE, bool AHEAD = false, bool SPLIT = false>
 __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const LinearArgs a) {
     // MB 16-row blocks of activations per workgroup (17 to 32 rows with MB = 2): every dequantized dword then feeds MB
     // matrix instructions, and the dequantization, which bounds the kernel, is done once for all of them
@@ -372,9 +373,9 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
     const int r = lane & 15, qd = lane >> 4;
     const int64_t rb0 = (int64_t)blockIdx.x * RBW;
     const int64_t m0 = (int64_t)blockIdx.y * (16 * MB);
-    // this workgroup's K tiles, kb0 .. kb0 + KB - 1: all of them or, with K parts, the blockIdx.z-th run
+    // this workgroup's K tiles: kb0 .. kb0 + KB - 1
     const int KP = (int)(a.Kp / 128), KA = EDGE ? (int)((a.K + 127) / 128) : KP;   // (g = 256: the packed row may go on)
-    const int kb0 = (int)blockIdx.z * a.kb_per_split, KB = KA - kb0 < a.kb_per_split ? KA - kb0 : a.kb_per_split;
+    const int kb0 = SPLIT ? (int)blockIdx.z * a.kb_per_split : 0, KB = SPLIT && KA - kb0 > a.kb_per_split ? a.kb_per_split : KA - kb0;
     // a row block past the end repeats the last one and is not stored
     auto row_block = [&](int j) __attribute__((always_inline)) {
         const int64_t last = (a.N + 15) / 16 - 1;
@@ -506,7 +507,7 @@ __global__ __launch_bounds__(WAVES * 64) void int4wo_linear_rb4_kernel(const Lin
                 if (m < a.M && n < a.N) {
                     sum += bv;
                     if (a.residual) sum = rne_bf16(sum) + bf16_bits_to_f32(a.residual[m * a.ldres + n]);
-                    if (a.y_is_f32) ((float*)a.y)[((int64_t)blockIdx.z * a.M + m) * a.ldy + n] = sum;
+                    if (SPLIT || a.y_is_f32) ((float*)a.y)[((SPLIT ? (int64_t)blockIdx.z : 0) * a.M + m) * a.ldy + n] = sum;
                     else ((uint16_t*)a.y)[m * a.ldy + n] = f32_to_bf16_bits(sum);
                 }
             }
@@ -1189,7 +1190,12 @@ static void launch_rb4_rows(int waves, int mb, bool edge, bool ahead, dim3 grid,
     else if (mb == 2) launch_rb4_one<G, 2>(waves, edge, ahead, grid, st, a);
     else launch_rb4_one<G, 4>(waves, edge, ahead, grid, st, a);
 }
-// grid: groups of four row blocks, chunks of 16 mb rows, K parts
+template <int G>
+static void launch_rb4_split(int mb, bool edge, dim3 grid, hipStream_t st, const LinearArgs& a) {
+    auto go = [&](auto kernel) { launch_timed(kernel, grid, dim3(512), 0, st, a); };
+    if (mb == 1) edge ? go(int4wo_linear_rb4_kernel<G, 8, 1, true, false, true>) : go(int4wo_linear_rb4_kernel<G, 8, 1, false, false, true>);
+    else edge ? go(int4wo_linear_rb4_kernel<G, 8, 2, true, false, true>) : go(int4wo_linear_rb4_kernel<G, 8, 2, false, false, true>);
+}
 static void launch_rb4(int64_t g, int waves, int mb, bool edge, bool ahead, dim3 grid, hipStream_t st, const LinearArgs& a) {
     switch (g) {
         case 32: launch_rb4_rows<32>(waves, mb, edge, ahead, grid, st, a); break;
@@ -1573,7 +1579,15 @@ int ao::int4wo_linear_stream_parts(const void* x_bf16, int64_t M, int64_t K, int
     a.y = workspace; a.y_is_f32 = 1; a.ldy = N;
     a.ksplit = parts; a.kb_total = (int)KB; a.kb_per_split = (int)per;
     hipStream_t st = (hipStream_t)stream;
-    launch_rb4(g, 8, M > 16 ? 2 : 1, RB % 4 != 0 || K != Kp, false, dim3((unsigned)((RB + 3) / 4), 1, (unsigned)parts), st, a);
+    const dim3 grid((unsigned)((RB + 3) / 4), 1, (unsigned)parts);
+    const int mb = M > 16 ? 2 : 1;
+    const bool edge = RB % 4 != 0 || K != Kp;
+    switch (g) {
+        case 32: launch_rb4_split<32>(mb, edge, grid, st, a); break;
+        case 64: launch_rb4_split<64>(mb, edge, grid, st, a); break;
+        case 128: launch_rb4_split<128>(mb, edge, grid, st, a); break;
+        default: launch_rb4_split<256>(mb, edge, grid, st, a); break;
+    }
     launch_ws_finish((const float*)workspace, parts, M, N, bias_bf16, y, y_dtype, ldy, st);
     AO_LAUNCH_CHECK();
     return 0;
