@@ -805,11 +805,14 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_kernel(const uint16_t* 
 // per workgroup, so that a converted and scaled weight fragment feeds MB matrix instructions and the activation rows are
 // fetched once per four row blocks (the tiled kernel takes 18 us on 14336 x 4096 at any of these row counts, this
 // kernel's 16-row form 9.5 us at 16 rows).
-template <int WAVES, bool E3M2, int MB>
+template <int WAVES, bool E3M2, int MB, bool SPLIT>
 __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_t* __restrict__ x, int64_t M, int64_t K,
                                                                     const uint32_t* __restrict__ native,
                                                                     const uint16_t* __restrict__ scale, int64_t N,
-                                                                    uint16_t* __restrict__ out) {
+                                                                    uint16_t* __restrict__ out, int kb_per_part,
+                                                                    float* __restrict__ parts) {
+    // SPLIT: blockIdx.z takes the z-th run of kb_per_part K tiles and stores its fp32 sums at parts + (z * M + m) * N + n; row blocks past the
+    // end repeat the last one and are not stored.  (Both at run time cost the others 5 %: 14336 x 4096 at 24 rows 13.6 -> 14.3 us)
     constexpr int RBW = 4;
     static_assert(WAVES >= RBW && WAVES <= 8, "wave j finishes row block j; 4 KB of reduction buffer per block and wave");
     __shared__ float red[RBW][WAVES][4][64];
@@ -817,7 +820,11 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, qd = lane >> 4;
     const int64_t rb0 = (int64_t)blockIdx.x * RBW, m0 = (int64_t)blockIdx.y * (16 * MB);
-    const int KB = (int)(K / 128);
+    const int KB = (int)(K / 128), kb0 = SPLIT ? (int)blockIdx.z * kb_per_part : 0, kb1 = SPLIT && kb0 + kb_per_part < KB ? kb0 + kb_per_part : KB;
+    auto block = [&](int j) __attribute__((always_inline)) {
+        const int64_t last = N / 16 - 1 - rb0;
+        return SPLIT && j > last ? last : (int64_t)j;
+    };
     const uint32_t* tiles = native + rb0 * KB * 384;
     const uint16_t* xp[MB];
 #pragma unroll
@@ -829,7 +836,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
 #pragma unroll
     for (int j = 0; j < RBW; ++j) {
         union { uint16_t h; _Float16 f; } sc;
-        sc.h = scale[(rb0 + j) * 16 + r];
+        sc.h = scale[(rb0 + block(j)) * 16 + r];
         sc2[j] = f16x2_t{sc.f, sc.f};
     }
     f32x4_t acc[RBW][MB];
@@ -843,7 +850,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
         const uint32_t* t = tiles + (int64_t)kb * 384;
 #pragma unroll
         for (int j = 0; j < RBW; ++j) {
-            const uint32_t* tj = t + (int64_t)j * KB * 384;
+            const uint32_t* tj = t + block(j) * KB * 384;
             const u32x4v_t lo = reinterpret_cast<const u32x4v_t*>(tj)[lane];
             const u32x2v_t hi = reinterpret_cast<const u32x2v_t*>(tj + 256)[lane];
             b.w[j] = __builtin_shufflevector(lo, __builtin_shufflevector(hi, hi, 0, 1, -1, -1), 0, 1, 2, 3, 4, 5);
@@ -879,7 +886,7 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
         }
     };
 
-    tiles_ahead<Buf>(wave, KB, WAVES, load_tile, compute_tile);   // 4096 x 14336 at 24 rows 16.1 -> 15.1 us, 28672 x 8192 49.0 -> 47.4
+    tiles_ahead<Buf>(kb0 + wave, kb1, WAVES, load_tile, compute_tile);   // 4096 x 14336 at 24 rows 16.1 -> 15.1 us, 28672 x 8192 49.0 -> 47.4
     // one pass of the reduction buffer per activation block; wave j sums and stores row block j
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
@@ -897,7 +904,10 @@ __global__ __launch_bounds__(WAVES * 64) void fp6_linear_mb_kernel(const uint16_
 #pragma unroll
                 for (int w = 0; w < WAVES; ++w) s += red[wave][w][i][lane];
                 const int64_t m = m0 + 16 * mb + 4 * qd + i;
-                if (m < M && n < N) out[m * N + n] = f32_to_f16_bits(s);
+                if (m < M && n < N) {
+                    if (SPLIT) parts[((int64_t)blockIdx.z * M + m) * N + n] = s;
+                    else out[m * N + n] = f32_to_f16_bits(s);
+                }
             }
         }
     }
@@ -1355,6 +1365,8 @@ static int check_fp6_format(int ebits, int mbits) {
     return 0;
 }
 
+int fp6_ws_parts(int64_t M, int64_t K, int64_t N);
+
 }  // namespace ao
 
 using namespace ao;
@@ -1611,7 +1623,7 @@ static int fp6_linear_dispatch(const void* x_f16, int64_t M, int64_t K, const vo
             while (w4 < 8 && wgs * w4 * 2 <= 4096 + wgs && w4 * 2 <= KB) w4 *= 2;
             const dim3 mgrid((unsigned)(RB / 4), 1u);
             AO_PLAN("fp6_linear_mb_kernel<%d,%d,2>", w4, ebits == 3 ? 1 : 0);
-#define AO_FP6_MB(W, E3) hipExtLaunchKernelGGL((fp6_linear_mb_kernel<W, E3, 2>), mgrid, dim3(W * 64), 0, st, ev0, ev1, 0, xx, M, K, nat, sc, N, o)
+#define AO_FP6_MB(W, E3) hipExtLaunchKernelGGL((fp6_linear_mb_kernel<W, E3, 2, false>), mgrid, dim3(W * 64), 0, st, ev0, ev1, 0, xx, M, K, nat, sc, N, o, (int)KB, (float*)nullptr)
             if (ebits == 3) { if (w4 == 4) AO_FP6_MB(4, true); else AO_FP6_MB(8, true); }
             else { if (w4 == 4) AO_FP6_MB(4, false); else AO_FP6_MB(8, false); }
 #undef AO_FP6_MB
@@ -1707,7 +1719,7 @@ extern "C" int ao_amd_fp6_linear(const void* x_f16, int64_t M, int64_t K, const 
 // 4096 x 4096 at 32 / 64 rows 11.9 / 9.0 (4), 12.5 / 11.7 (4), at 128 rows 13.5 / 15.3 (not split); 6144 x 4096 at 32 rows
 // 12.4 / 10.6 (2), at 64 rows 13.0 / 14.3 (not split); 1024 x 4096 at 32 / 64 / 128 / 256 rows 11.5 / 7.8, 11.6 / 9.7, 12.1 / 10.3,
 // 12.5 / 11.8 (4); 14336 x 4096: slower at every row count; at 16 rows only the long K gains (4096 x 4096: 6.6 / 8.1).
-static int fp6_ws_parts(int64_t M, int64_t K, int64_t N) {
+int ao::fp6_ws_parts(int64_t M, int64_t K, int64_t N) {
     if (K % 128 != 0 || N % 16 != 0 || M < 1) return 1;
     static const int forced = [] { const char* e = knob("AO_AMD_WS_PARTS"); return e ? atoi(e) : 0; }();
     const int64_t KB = K / 128, RB = N / 16;
@@ -1725,28 +1737,118 @@ static int fp6_ws_parts(int64_t M, int64_t K, int64_t N) {
     return z < 1 ? 1 : z;
 }
 
+// 4 to 64 rows with K split in other ways than fp6_ws_parts' power of two of the 32- and 64-row tiles, where they lead.  us before / now, e3m2:
+//  * rows: four row blocks a workgroup (fp6_linear_mb_kernel), 4 to 32 activation rows.  One block a workgroup reads all of x per 16 weight rows:
+//    5120 x 13824 at 8 / 12 / 16 / 24 rows 22.3 / 14.5, 26.5 / 14.7, 21.2 / 15.3, 21.5 / 17.9; 2048 x 16384 at 8 / 24 rows 13.9 / 10.2, 15.3 / 12.2; 10240 x 8192 at 12 rows
+//    20.1 / 17.0; 5120 x 5120 at 16 rows 12.6 / 8.6; but 4096 x 4096 at 16 rows 6.8 / 7.7;
+//  * tiles: fp6_gemm_kernel's 64 columns in parts that are no power of two (5120 x 13824 at 32 rows 21.5 / 18.4) or of narrow weights (1024 x 14336 at 40 rows
+//    18.9 / 13.2), 48 rows a tile up to 48 (4096 x 4096 at 48 rows 11.0 / 10.4, the fourth block was padding);
+//  * wide: 128 columns a tile and twice the parts, from 33 rows on: x, at 48 rows twice the bytes of the codes, is read half as often.  5120 x 13824 at 48 / 64 rows
+//    30.4 / 20.9, 31.6 / 23.2; 8192 x 8192 23.1 / 19.7, 23.6 / 22.0; 4096 x 14336 20.1 / 19.2, 21.1 / 21.0; 7168 x 5120 at 48 rows 15.0 / 14.0.
+// The estimates (us; a part's K tiles, rows, weight bytes) are within some 8 % of those calls.
+struct Fp6Rows {
+    enum Kind { none, rows, tiles, wide };
+    int kind, parts;
+};
+static Fp6Rows fp6_rows_plan(int64_t M, int64_t K, int64_t N) {
+    Fp6Rows best{Fp6Rows::none, 1};
+    if (K % 128 != 0 || N % 16 != 0 || M < 4 || M > 64) return best;
+    const int64_t KB = K / 128, RB = N / 16, groups = (RB + 3) / 4, wide = (RB + 7) / 8;
+    if (KB < 8 || groups >= 192) return best;
+    const double m = (double)M, kb = (double)KB, mb = (double)(N * K) * 0.75e-6;
+    const int z0 = fp6_ws_parts(M, K, N);
+    static const bool forced = knob("AO_AMD_WS_PARTS") != nullptr;
+    if (forced) return best;
+    double other;
+    if (z0 > 1) {
+        const double per = (double)((KB + z0 - 1) / z0);
+        other = M <= 32 ? (groups < 64 ? 6.1 : 6.9) + 0.315 * per : M <= 48 ? 7.6 + 0.45 * per : 8.0 + 0.47 * per;
+    } else if (M > 32) {
+        other = 4.0 + 0.25 * kb * (double)((groups * 2 + 255) / 256);
+    } else if (M > 16) {
+        other = 4.5 + 0.31 * kb;
+    } else {
+        const int rbw = fp6_row_blocks_per_wave(M, RB, 1);
+        const double per_tile = rbw == 1 ? (double)((RB + 255) / 256) * (0.043 + 0.0048 * m)
+                                         : (0.08 + 0.0063 * m) * (RB > 512 ? 1.7 : (double)RB / 512.0);
+        other = 3.5 + kb * per_tile;
+    }
+    double us = 0.96 * other;
+    auto offer = [&](int kind, int z, double t) {
+        if (t >= us) return;
+        us = t;
+        best = Fp6Rows{kind, z};
+    };
+    for (int z = 2; z <= 8; ++z) {
+        const int64_t per = (KB + z - 1) / z;
+        if (per < 4 || (z - 1) * per >= KB) continue;
+        const double p = (double)per, launch = (M <= 16 ? 0.1 : M <= 32 ? 0.14 : M <= 48 ? 0.1 : 0.2) * z;
+        if (M <= 16 && groups * z <= 512) offer(Fp6Rows::rows, z, 5.0 + 0.04 * m + (0.24 + 0.002 * m) * p * (groups * z > 256 ? 2.1 : 1.0) + launch);
+        if (M > 16 && M <= 32 && groups * z <= 256) {
+            offer(Fp6Rows::rows, z, 5.1 + 0.05 * m + (0.22 + 0.0044 * m) * p + launch);
+            if (z != z0 && (z0 == 1 || KB >= 64)) offer(Fp6Rows::tiles, z, 6.9 + 0.315 * p + launch);
+        }
+        // (short K that is split in four already gains by the 48-row tiles only)
+        if (M > 32 && groups * z <= 256 && (z == z0 ? M <= 48 : z0 == 1 || KB >= 64))
+            offer(Fp6Rows::tiles, z, (M <= 48 ? 6.9 + 0.43 * p : 7.6 + 0.47 * p) + launch);
+        // (few workgroups do not bring the weight in at that rate)
+        if (M > 32 && wide * z >= 190 && wide * z <= 256) offer(Fp6Rows::wide, z, (M <= 48 ? 7.0 + 0.235 * mb : 8.0 + 0.27 * mb) + 0.25 * z);
+    }
+    return best;
+}
+
+template <bool E3M2>
+static void launch_fp6_rows(const Fp6Rows& p, const uint16_t* x, int64_t M, int64_t K, const uint32_t* native, const uint16_t* scale, int64_t N, uint16_t* out,
+                            float* ws, hipStream_t st) {
+    const int64_t KB = K / 128, RB = N / 16;
+    const int per = (int)((KB + p.parts - 1) / p.parts);
+    const int64_t cols = p.kind == Fp6Rows::wide ? 8 : 4;
+    const dim3 grid((unsigned)((RB + cols - 1) / cols), 1, (unsigned)p.parts);
+    hipEvent_t ev0 = g_prof_start, ev1 = g_prof_stop;
+    g_prof_start = g_prof_stop = nullptr;
+    auto go = [&](auto kernel) { hipExtLaunchKernelGGL(kernel, grid, dim3(256), 0, st, ev0, ev1, 0, x, M, K, native, scale, N, out, per, ws); };
+    if (p.kind == Fp6Rows::rows) M <= 16 ? go(fp6_linear_mb_kernel<4, E3M2, 1, true>) : go(fp6_linear_mb_kernel<4, E3M2, 2, true>);
+    else if (p.kind == Fp6Rows::wide) M <= 48 ? go(fp6_gemm_kernel<E3M2, 2, 3, 4, 4>) : go(fp6_gemm_kernel<E3M2, 2, 4, 4, 2>);
+    else if (M <= 32) go(fp6_gemm_kernel<E3M2, 1, 2, 8, 8>);
+    else M <= 48 ? go(fp6_gemm_kernel<E3M2, 1, 3, 4, 4>) : go(fp6_gemm_kernel<E3M2, 1, 4, 4, 4>);
+    hipLaunchKernelGGL(fp6_ws_finish_kernel, dim3((unsigned)((M * N / 4 + 255) / 256)), dim3(256), 0, st, ws, p.parts, M * N, out);
+}
+
 extern "C" int ao_amd_fp6_linear_ws_bytes(int64_t M, int64_t K, int64_t N, int64_t* bytes) {
     AO_REQUIRE(bytes, "null pointer argument");
     AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
-    const int z = fp6_ws_parts(M, K, N);
+    const int z = ao_amd_fp6_linear_ws_parts(M, K, N);
     *bytes = z > 1 ? (int64_t)z * M * N * (int64_t)sizeof(float) : 0;
     return 0;
 }
 
-extern "C" int ao_amd_fp6_linear_ws_parts(int64_t M, int64_t K, int64_t N) { return fp6_ws_parts(M, K, N); }
+extern "C" int ao_amd_fp6_linear_ws_parts(int64_t M, int64_t K, int64_t N) {
+    const Fp6Rows rows = fp6_rows_plan(M, K, N);
+    return rows.kind != Fp6Rows::none ? rows.parts : fp6_ws_parts(M, K, N);
+}
 
 extern "C" int ao_amd_fp6_linear_ws(const void* x_f16, int64_t M, int64_t K, const void* weights_native, const void* scale_f16,
                                     int64_t N, int ebits, int mbits, void* out_f16, void* workspace, int64_t workspace_bytes,
                                     void* stream) {
-    const int z = fp6_ws_parts(M, K, N);
+    const Fp6Rows rows = fp6_rows_plan(M, K, N);
+    const int z = rows.kind != Fp6Rows::none ? rows.parts : fp6_ws_parts(M, K, N);
     if (z <= 1)
         return fp6_linear_dispatch(x_f16, M, K, weights_native, scale_f16, N, ebits, mbits, nullptr, nullptr, out_f16, stream);
     const int64_t need = (int64_t)z * M * N * (int64_t)sizeof(float);
     AO_REQUIRE(workspace && workspace_bytes >= need && (((uintptr_t)workspace) & 15) == 0,
                "16-byte aligned workspace of %lld bytes needed (ao_amd_fp6_linear_ws_bytes), got %lld", (long long)need,
                (long long)workspace_bytes);
-    return fp6_linear_dispatch(x_f16, M, K, weights_native, scale_f16, N, ebits, mbits, nullptr, nullptr, out_f16, stream, nullptr,
-                               0.f, nullptr, nullptr, nullptr, 0, z, (float*)workspace);
+    if (rows.kind == Fp6Rows::none)
+        return fp6_linear_dispatch(x_f16, M, K, weights_native, scale_f16, N, ebits, mbits, nullptr, nullptr, out_f16, stream, nullptr,
+                                   0.f, nullptr, nullptr, nullptr, 0, z, (float*)workspace);
+    AO_REQUIRE(x_f16 && weights_native && scale_f16 && out_f16, "null pointer argument");
+    if (int rc = check_fp6_format(ebits, mbits)) return rc;
+    AO_REQUIRE((((uintptr_t)x_f16) & 15) == 0 && (((uintptr_t)weights_native) & 15) == 0, "buffers must be 16-byte aligned");
+    const uint16_t *xx = (const uint16_t*)x_f16, *sc = (const uint16_t*)scale_f16;
+    if (ebits == 3) launch_fp6_rows<true>(rows, xx, M, K, (const uint32_t*)weights_native, sc, N, (uint16_t*)out_f16, (float*)workspace, (hipStream_t)stream);
+    else launch_fp6_rows<false>(rows, xx, M, K, (const uint32_t*)weights_native, sc, N, (uint16_t*)out_f16, (float*)workspace, (hipStream_t)stream);
+    AO_LAUNCH_CHECK();
+    return 0;
 }
 
 extern "C" int ao_amd_fp6_linear_fused(const void* x_f16, int64_t M, int64_t K, const void* weights_native,
@@ -1792,3 +1894,4 @@ extern "C" int ao_amd_fp6_native_to_f16(const void* weights_native, const void* 
     AO_LAUNCH_CHECK();
     return 0;
 }
+

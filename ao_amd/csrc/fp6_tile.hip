@@ -7,6 +7,8 @@
 
 namespace ao {
 
+int fp6_ws_parts(int64_t M, int64_t K, int64_t N);   // fp6.hip: the power of two that the 32- and 64-row tiles are split in
+
 typedef _Float16 ft_f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 ft_f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 ft_f16x32 __attribute__((ext_vector_type(32)));
@@ -112,7 +114,7 @@ static TilePlan fp6_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
 // 14336 at 64 / 66 / 96 rows 20.9 / 20.9, 31.0 / 22.2, 32.3 / 24.1; 4096 x 4096 at 66 rows 11.9 / 13.4).
 static bool fp6_tiled(int64_t M, int64_t N, int64_t K) {
     if (K % 64 != 0 || N % 16 != 0 || M <= 32 || M * N >= ((int64_t)1 << 40) || 192 * K * 2 >= ((int64_t)1 << 32)) return false;
-    if (ao_amd_fp6_linear_ws_parts(M, K, N) != 1 && (M <= 64 || M > 96 || N * K < 50000000)) return false;
+    if (fp6_ws_parts(M, K, N) != 1 && (M <= 64 || M > 96 || N * K < 50000000)) return false;
     const double tile_us = fp6_tile_plan(M, N, K, 8).us;
     // streamed once per 16 rows there (14336 x 4032 at 33 / 128 / 1000 rows 22 / 50 / 305 us, tiled 20 / 24 / 119; 4096 x 4160 at 65 / 128 /
     // 1000 rows 14 / 17 / 96, tiled 16 / 16 / 41)

@@ -211,6 +211,39 @@ def test_fp6_workspace_linear(N, K, M, parts, ebits, mbits):
     assert exact
 
 
+# (N, K, M, K parts): every kind of split (four row blocks a workgroup up to 32 rows, tiles of 64 and of 128 columns from 17 and 33 rows on) at the first and
+# last row counts of its kernels, a shorter last part, more workgroups than CUs, row blocks that fill neither four nor eight
+@pytest.mark.parametrize("ebits,mbits", [(3, 2), (2, 3)])
+@pytest.mark.parametrize("N,K,M,parts", [
+    (5120, 13824, 4, 3), (5120, 13824, 16, 3), (5120, 13824, 17, 3), (5120, 13824, 32, 3), (5120, 13824, 33, 5), (5120, 13824, 48, 5), (5120, 13824, 49, 5),
+    (5120, 13824, 64, 5), (10240, 8192, 16, 3), (4096, 14336, 48, 6), (4096, 4096, 40, 4), (1024, 14336, 30, 8), (1024, 14336, 48, 8), (1024, 14336, 64, 8),
+    (2064, 16384, 16, 7), (2064, 16384, 30, 7), (2064, 16384, 64, 7), (5008, 13824, 24, 3), (5008, 13824, 60, 5)])
+def test_fp6_rows_in_parts(N, K, M, parts, ebits, mbits):
+    from ao_amd import _lib, ops
+
+    print(f"case fp6 rows in parts N={N} K={K} M={M} parts={parts} e{ebits}m{mbits}", flush=True)
+    L, need = _lib.lib(), ctypes.c_int64(-1)
+    _lib.check(L.ao_amd_fp6_linear_auto_bytes(M, K, N, ctypes.byref(need)))
+    assert need.value == 4 * parts * M * N
+    n = -(-N // 64) * 64   # the interchange format's rows; the kernels take a multiple of 16 of them
+    data, scale = ops.fp6_quantize_pack((torch.randn(n, K, generator=torch.Generator().manual_seed(N)) * 0.02).half().cuda(), ebits, mbits)
+    native, w = ops.fp6_repack(data, 6).flatten()[: N // 16 * (K // 128) * 384], ops.fp6_dequantize(data, scale, ebits, mbits)[:N].half()
+    scale = scale[:N].contiguous()
+    gen = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=gen).half().cuda()
+    y = ops.fp6_linear_native(ebits, mbits, x, native, scale)
+    ref = (x.float() @ w.float().t()).half().float()
+    # one rounding to fp16 (2^-12 / sqrt 3 relative) and fp32 sums in another order: 1e-3 is what the other routes are held to
+    assert float((y.float() - ref).norm() / ref.norm()) <= 1e-3
+    # one-hot rows read single columns of the weight back, at both ends of K and of every part
+    per = -(-(K // 128) // parts) * 128
+    ends = [0, K - 1] + [k for z in range(1, parts) for k in (z * per - 1, z * per)]
+    ks = torch.tensor([ends[i % len(ends)] for i in range(M)])
+    xh = torch.zeros(M, K, dtype=torch.float16)
+    xh[torch.arange(M), ks] = 1.0
+    assert torch.equal(ops.fp6_linear_native(ebits, mbits, xh.cuda(), native, scale), w[:, ks.cuda()].t().contiguous())
+
+
 def _empty_ws(nbytes):
     return torch.empty(max(nbytes, 16), dtype=torch.uint8, device="cuda")
 
