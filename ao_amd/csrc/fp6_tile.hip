@@ -96,6 +96,9 @@ static TilePlan fp6_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
     // 4096 x 14336 at 256 rows, four of 128 x 128, 43.0 / 44.2, 5120 x 13824 at 129 rows, two of 64 x 128, 36.9 / 39.2)
     TilePartCost parts;
     parts.lead = 0.89;
+    // (in powers of two / three or six parts: 5120 x 13824 at 96 / 128 / 256 rows 33.8 / 30.9, 40.7 / 33.0, 49.1 / 46.4; 10240 x 8192 at 40 / 77 / 113 rows 26.0 / 27.6, 30.3 /
+    // 33.1, 34.3 / 36.1; 9000 x 6144 and 5120 x 5120 level)
+    parts.uneven = K >= 10240;
     return tile_plan(kFp6Shapes, (int)(sizeof(kFp6Shapes) / sizeof(kFp6Shapes[0])), M, N, K, max_parts, parts);
 }
 

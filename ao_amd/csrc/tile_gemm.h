@@ -355,31 +355,49 @@ struct TilePlan {
 struct TilePartCost {
     double launch = 1.5, doubling = 1.0, sums = 8.0;
     double lead = 1.0;   // K parts have to take less than this share of the whole K's estimate
+    bool uneven = true;  // part counts that are no power of two
 };
-// us of one shape with K in `z` parts
-inline double tile_us(const TileShape& s, int64_t M, int64_t N, int64_t K, int z, const TilePartCost& c = TilePartCost()) {
-    const int64_t per = (K / 64 + z - 1) / z, wgs = (M + s.bm - 1) / s.bm * ((N + s.bn - 1) / s.bn) * z;
-    const int64_t fit = s.two > 0 ? 512 : 256, full = wgs / fit, rest = wgs % fit;
+// us of one shape whose M x N has `tiles` tiles, with K in `z` parts of `per` steps
+inline double tile_us(const TileShape& s, int64_t tiles, int64_t per, int z, int64_t M, int64_t N, int64_t K, const TilePartCost& c) {
+    const int shift = s.two > 0 ? 9 : 8;   // two workgroups fit a CU, or one
+    const int64_t wgs = tiles * z, full = wgs >> shift, rest = wgs & (((int64_t)1 << shift) - 1);
     auto us = [&](double t) { return 6.0 + (t - 6.0) * (double)per / 64.0; };
     const double one = us(s.one), wave = s.two > 0 ? us(s.two) : one;
     // (CUs that read a large weight at once share the memory: 120 workgroups take 0.7 to 0.97 of the time of 224)
     const double alone = full == 0 && rest < 256 && N * K >= ((int64_t)1 << 25) ? 0.85 + 0.15 * (double)rest / 256.0 : 1.0;
     // (the first CU with two workgroups sets the time, and the more there are the more they slow each other down)
-    const double t = full * wave + (rest == 0 ? 0.0 : rest <= 256 ? one * alone : one + (wave - one) * (0.4 + 0.6 * (double)(rest - 256) / 256.0));
-    return z == 1 ? t : t + c.launch + (z == 2 ? 1.0 : z == 4 ? 2.0 : 3.0) * c.doubling + c.sums * 1e-6 * (double)(M * N * z) / 4.0;
+    const double t = (double)full * wave + (rest == 0 ? 0.0 : rest <= 256 ? one * alone : one + (wave - one) * (0.4 + 0.6 * (double)(rest - 256) / 256.0));
+    constexpr double LOG2[9] = {0.0, 0.0, 1.0, 1.585, 2.0, 2.322, 2.585, 2.807, 3.0};
+    return z == 1 ? t : t + c.launch + LOG2[z] * c.doubling + c.sums * 1e-6 * (double)(M * N * z) / 4.0;
 }
+// Part counts that are no power of two fill the chip where a weight has 48, 80 or 160 tiles, but the estimates do not rank them finely: of 154
+// calls (33 to 1000 rows, 21 weights) those with an estimate below 0.945 of the best power of two took 0.90 of its time on average and 1.03 at most, the others 1.02 (and
+// up to 1.19), and weights below 2^23 gained nothing (1024 x 4096 0.96 to 1.04).  us in powers of two / other parts: int8 10240 x 8192 at 77 / 128 rows 39.7 /
+// 31.0, 41.2 / 38.2, 9000 x 6144 at 48 rows 25.0 / 22.0, 5120 x 13824 at 200 rows 52.5 / 45.0; int4 5120 x 13824 at 256 rows 66.2 / 49.4, 5120 x 5120 at 40 rows
+// 15.3 / 14.2.  Not for shapes with few parts, whose sums are large (int4 5120 x 5120 at 420 rows in three of 256 x 128, 36.8 / 46.4).
 inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64_t N, int64_t K, int max_parts,
                           const TilePartCost& c = TilePartCost()) {
-    TilePlan best{-1, 1, 1e30}, whole = best;
+    TilePlan best{-1, 1, 1e30}, whole = best, uneven = best;
+    constexpr int MOST = 16;
+    int64_t tiles[MOST];   // (a call plans twice: the divisions stand outside the loop over the parts)
+    for (int i = 0; i < nshapes && i < MOST; ++i) tiles[i] = (M + shapes[i].bm - 1) / shapes[i].bm * ((N + shapes[i].bn - 1) / shapes[i].bn);
     const int64_t steps = K / 64;
-    for (int i = 0; i < nshapes; ++i)
-        for (int z = 1; z <= (max_parts < shapes[i].max_parts ? max_parts : shapes[i].max_parts); z *= 2) {
-            const int64_t per = (steps + z - 1) / z;
-            if (z > 1 && (per < 8 || (z - 1) * per >= steps)) break;
-            const double t = tile_us(shapes[i], M, N, K, z, c);
-            if (t < best.us) best = TilePlan{i, z, t};
+    const bool all = c.uneven && N * K >= ((int64_t)1 << 23);
+    for (int z = 1; z <= (max_parts < 8 ? max_parts : 8); ++z) {
+        const bool power = (z & (z - 1)) == 0;
+        if (!power && !all) continue;
+        const int64_t per = (steps + z - 1) / z;
+        if (z > 1 && per < 8) break;
+        if ((z - 1) * per >= steps) continue;   // the last part would be empty
+        for (int i = 0; i < nshapes && i < MOST; ++i) {
+            if (z > shapes[i].max_parts || (!power && shapes[i].max_parts < 8)) continue;
+            const double t = tile_us(shapes[i], tiles[i], per, z, M, N, K, c);
+            TilePlan& to = power ? best : uneven;
+            if (t < to.us) to = TilePlan{i, z, t};
             if (z == 1 && t < whole.us) whole = TilePlan{i, z, t};
         }
+    }
+    if (uneven.us < 0.945 * best.us) best = uneven;
     return best.us < c.lead * whole.us ? best : whole;
 }
 

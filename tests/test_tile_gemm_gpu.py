@@ -400,3 +400,19 @@ def test_every_tile_once(fmt, M, N, K, group, name):
         native = ops.fp6_repack(tc, 6)
         dq, y = ops.fp6_dequantize(tc, scale, 3, 2).half(), ops.fp6_linear_native(3, 2, x, native, scale)
     assert torch.equal(y, dq[:, at].t())
+
+
+# K parts that are no power of two: equal ones and a shorter last one, of pairs of steps (64 x 128 int8 tiles) too, rows and columns that end within a tile
+@pytest.mark.parametrize("fmt,M,N,K,plan", [
+    ("int8", 40, 5120, 13824, "tile 64x128 parts=6"), ("int8", 61, 10200, 8320, "tile 64x128 parts=3"), ("int8", 77, 10240, 8256, "tile 96x128 parts=3"),
+    ("int8", 100, 2300, 4160, "tile 64x64 parts=3"), ("int4wo", 40, 5120, 5120, "tile 64x64 parts=3"), ("int4wo", 90, 5110, 13888, "tile 96x128 parts=6"),
+    ("int4wo", 200, 5120, 13824, "tile 128x128 parts=3"), ("fp6", 113, 5120, 13824, "tile 64x128 parts=3"), ("fp6", 77, 5120, 13888, "tile 96x128 parts=6")])
+def test_parts_that_are_no_power_of_two(fmt, M, N, K, plan):
+    assert (_plan(M, N, K) if fmt == "int8" else _tiled_plan(fmt, M, N, K)) == plan
+    # (the bounds of the helpers: up to 13888 products a sum)
+    if fmt == "int8":
+        _run(M, N, K)
+    elif fmt == "int4wo":
+        _int4_tiles(M, N, K, 64)
+    else:
+        _fp6_tiles(M, N, K, 3, 2)
