@@ -137,4 +137,6 @@ void launch_int8wo_gemm(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
     tile_finish<Int8Tile<false>>(a, p.parts, st);
 }
 
+void int8wo_finish_parts(const TileGemmArgs& a, int parts, hipStream_t st) { tile_finish<Int8Tile<false>>(a, parts, st); }
+
 }  // namespace ao

@@ -69,6 +69,7 @@ struct Int8Args {
     const uint16_t* gate; int64_t ldgate;     // y = silu(gate) * bf16(result) (SwiGLU with the gate already computed), or null
     const uint16_t* norm_w; float norm_eps;   // STAGED only: RMSNorm weight [K] applied to x while staging, or null
     const int8_t* w_up; const uint16_t* scale_up;  // DUAL only: second weight (same shape and row stride) and its scales
+    int kb_per_part; float* parts;            // SPLIT only (int8wo_linear_rb4_kernel)
 };
 
 // sum of the squares of the 8 bf16 values of a 16-byte chunk
@@ -323,8 +324,9 @@ __global__ __launch_bounds__(WAVES * 64) void int8wo_linear_kernel(const Int8Arg
 // weights at 16 rows, and a CU's L1 fill rate (about 20 bytes per cycle), not memory, sets the time.  A wave loads the
 // activation fragments of a K tile once and runs them against the tiles of four row blocks; wave j finishes block j.
 // The next tile is requested ahead, under no condition: 14336 x 4096 at 7 / 16 rows 17.4 / 19.2 -> 16.7 / 18.5 us, 28672 x 8192 at 4 rows 56.6 -> 54.1.
-template <int WAVES, int MB>
+template <int WAVES, int MB, bool SPLIT = false>
 __global__ __launch_bounds__(WAVES * 64) void int8wo_linear_rb4_kernel(const Int8Args a) {
+    // SPLIT: the workgroup takes the blockIdx.z-th run of a.kb_per_part K tiles and leaves fp32 sums at a.parts + (z * M + m) * N + n
     // MB 16-row blocks of activations per workgroup (MB = 2 from 17 rows on): a converted weight fragment feeds MB
     // matrix instructions and the weight is streamed once per 16 MB rows
     constexpr int RBW = 4;
@@ -334,7 +336,7 @@ __global__ __launch_bounds__(WAVES * 64) void int8wo_linear_rb4_kernel(const Int
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, qd = lane >> 4;
     const int64_t rb0 = (int64_t)blockIdx.x * RBW, m0 = (int64_t)blockIdx.y * (16 * MB);
-    const int KB = (int)(a.K / 128);
+    const int KA = (int)(a.K / 128), kb0 = SPLIT ? (int)blockIdx.z * a.kb_per_part : 0, KB = SPLIT && kb0 + a.kb_per_part < KA ? kb0 + a.kb_per_part : KA;
     const int8_t* wp[RBW];
 #pragma unroll
     for (int j = 0; j < RBW; ++j) {
@@ -386,7 +388,7 @@ __global__ __launch_bounds__(WAVES * 64) void int8wo_linear_rb4_kernel(const Int
             }
         }
     };
-    tiles_ahead<Buf>(wave, KB, WAVES, load_tile, compute_tile);
+    tiles_ahead<Buf>(kb0 + wave, KB, WAVES, load_tile, compute_tile);
     // acc[j][mb][i] = C[m = m0 + 16 mb + 4*qd + i][n = 16 (rb0 + j) + r]; one pass of the reduction buffer per
     // activation block
 #pragma unroll
@@ -400,15 +402,17 @@ __global__ __launch_bounds__(WAVES * 64) void int8wo_linear_rb4_kernel(const Int
         if (wave < RBW) {
             const int64_t n = (rb0 + wave) * 16 + r;
             if (n < a.N) {
-                const float sc = bf16_bits_to_f32(a.scale[n]);
-                const float bv = a.bias ? bf16_bits_to_f32(a.bias[n]) : 0.f;
+                const float sc = SPLIT ? 0.f : bf16_bits_to_f32(a.scale[n]);
+                const float bv = !SPLIT && a.bias ? bf16_bits_to_f32(a.bias[n]) : 0.f;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     float s = 0.f;
 #pragma unroll
                     for (int w = 0; w < WAVES; ++w) s += red[wave][w][i][lane];
                     const int64_t m = m0 + 16 * mb + 4 * qd + i;
-                    if (m < a.M) {
+                    if (SPLIT) {
+                        if (m < a.M) a.parts[((int64_t)blockIdx.z * a.M + m) * a.N + n] = s;
+                    } else if (m < a.M) {
                         // the epilogue of int8wo_linear_kernel: mm result rounded to bf16, times scale, plus bias, then
                         // the fused residual or gate
                         float v = hw_rne_bf16(s) * sc;
@@ -581,6 +585,46 @@ static bool tiled(int64_t M, int64_t N, int64_t K, bool workspace) {
     return M > (workspace && K >= 8192 && (N <= 8192 || N >= 24576) ? 8 : 16);
 }
 
+// 2 to 32 rows of weights with fewer than 768 row blocks: one row block a workgroup, which reads all of x per 16 weight rows and runs in rounds of 256
+// row blocks, from 17 rows on for each 16 (streaming); four blocks a workgroup with K in parts (four_parts, up to 16 rows); or the tiles with K in parts (int8wo_gemm.hip).  us streaming / four_parts /
+// tiles: 5120 x 13824 at 2 / 8 / 16 rows 23.8 / 20.3 / 23.1, 33.3 / 21.8 / 23.6, 42.4 / 23.9 / 24.0; 4096 x 14336 at 4 / 8 / 16 rows 15.7 / 18.2 / 22.0, 19.5 / 18.7 / 22.1, 24.4 /
+// 20.1 / 22.5; 2048 x 16384 at 4 / 12 rows 15.4 / 14.3 / 16.9, 22.7 / 15.1 / 17.7; 8192 x 8192 at 12 rows 23.7 / 20.8 / 23.9; 5120 x 5120 at 8 rows 15.3 / 13.4 / 15.2;
+// 4096 x 11008 at 12 rows 17.7 / 17.0 / 20.5; 1024 x 14336 at 8 rows 18.4 / 13.6 / 13.8; 10240 x 8192 at 8 / 16 rows 29.3 / - / 25.2, 36.8 / - / 25.8; 4096 x 4096 at 16
+// rows 8.8 / 10.6 / 11.6; streaming / tiles at 20 rows: 1024 x 14336 22.7 / 13.9, 4096 x 4096 12.9 / 11.9, 1024 x 4096 8.5 / 11.5.  (Weight and row count each had a line of their own before, which sent 5120 x 13824 at 8 rows and 10240 x 8192 at 16 to streaming and 4096 x
+// 11008 at 12 to the tiles.)  The estimates are within some 6 % of these calls.
+struct Int8Rows {
+    enum Kind { other, streaming, four_parts, tiles };   // other: not one of these calls
+    int kind, parts;
+};
+static Int8Rows int8_rows_plan(int64_t M, int64_t K, int64_t N) {
+    static const bool forced = knob("AO_AMD_INT8_TILED") != nullptr;
+    const int64_t KB = K / 128, RB = (N + 15) / 16, groups = (RB + 3) / 4;
+    if (M < 2 || M > 32 || K % 128 != 0 || KB < 8 || groups >= 192 || forced) return Int8Rows{Int8Rows::other, 1};
+    // (row blocks that are no multiple of four keep their route up to 8 rows, which callers rely on: 4104 x 8320 at 8 rows takes 19.1 us and would take 15.7 in parts)
+    if (M <= 8 && RB % 4 != 0) return Int8Rows{Int8Rows::other, 1};
+    const double m = (double)M, kb = (double)KB;
+    // (rows that fit LDS are staged there, with one workgroup to a CU)
+    const bool staged = RB <= 256 && KB >= 64 && M * K * 2 <= 140 * 1024;
+    const double streaming = 4.0 + (double)((RB * ((M + 15) / 16) + 255) / 256) * kb * ((staged ? 0.07 : 0.09) + 0.0055 * (M < 16 ? m : 16.0));
+    Int8Rows best{Int8Rows::streaming, 1};
+    double us = (M <= 16 ? 0.96 : 1.0) * streaming;
+    for (int z = 2; M <= 16 && z <= 8; ++z) {
+        const int64_t per = (KB + z - 1) / z;
+        if (per < 4 || (z - 1) * per >= KB || groups * z > 256) continue;
+        const double t = 7.0 + 0.03 * m + (0.365 + 0.0053 * m) * (double)per + 0.08 * z;
+        if (t < us) {
+            us = t;
+            best = Int8Rows{Int8Rows::four_parts, z};
+        }
+    }
+    if (streaming > 12.0) {   // (no tiles take less)
+        const TilePlan p = int8wo_gemm_plan(M, N, K, 8);
+        // (their estimates are of 33 and more rows and 10 % low at the fewest)
+        if (p.us < (M <= 16 ? 0.9 : 1.0) * us) best = Int8Rows{Int8Rows::tiles, p.parts};
+    }
+    return best;
+}
+
 // Per-lane offsets within a tile are 32 bits wide: rows further apart than that keep the streaming kernels.
 static bool tiles_reach(int64_t M, int64_t N, int64_t ldx, int64_t ldw) {
     return 192 * ldx * 2 < ((int64_t)1 << 32) && 256 * ldw < ((int64_t)1 << 32) && M * N < ((int64_t)1 << 40);
@@ -608,10 +652,37 @@ static int int8wo_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, c
     return 0;
 }
 
+static int int8wo_four_parts(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* w_int8, int64_t ldw, const void* scale_bf16, int64_t N,
+                             const void* bias_bf16, void* y, int64_t ldy, int parts, float* workspace, void* stream) {
+    AO_REQUIRE(x_bf16 && w_int8 && scale_bf16 && y, "null pointer argument");
+    AO_REQUIRE(ldx >= K && ldw >= K && ldy >= N, "row strides (ldx=%lld, ldw=%lld, ldy=%lld) smaller than the rows", (long long)ldx, (long long)ldw,
+               (long long)ldy);
+    AO_REQUIRE((((uintptr_t)x_bf16) & 15) == 0 && (ldx & 7) == 0 && (((uintptr_t)w_int8) & 15) == 0 && (ldw & 15) == 0,
+               "activation and weight rows must be 16-byte aligned");
+    Int8Args a{};
+    a.x = (const uint16_t*)x_bf16; a.M = M; a.K = K; a.ldx = ldx;
+    a.w = (const int8_t*)w_int8; a.ldw = ldw; a.N = N;
+    a.kb_per_part = (int)((K / 128 + parts - 1) / parts);
+    a.parts = workspace;
+    hipStream_t st = (hipStream_t)stream;
+    hipEvent_t ev0 = g_prof_start, ev1 = g_prof_stop;
+    g_prof_start = g_prof_stop = nullptr;
+    hipExtLaunchKernelGGL((int8wo_linear_rb4_kernel<4, 1, true>), dim3((unsigned)((N + 63) / 64), 1, (unsigned)parts), dim3(256), 0, st, ev0, ev1, 0, a);
+    int8wo_finish_parts(TileGemmArgs{a.x, M, K, ldx, (const uint8_t*)w_int8, ldw, scale_bf16, (const uint16_t*)bias_bf16, N, (uint16_t*)y, ldy, TileOrder(),
+                                     nullptr, 0, nullptr, 0, 0, workspace}, parts, st);
+    AO_LAUNCH_CHECK();
+    return 0;
+}
+
 extern "C" int ao_amd_int8wo_linear_ws_bytes(int64_t M, int64_t K, int64_t N, int64_t* bytes) {
     AO_REQUIRE(bytes, "null pointer argument");
     AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
     *bytes = 0;
+    const Int8Rows rows = int8_rows_plan(M, K, N);
+    if (rows.kind != Int8Rows::other) {
+        if (rows.parts > 1) *bytes = rows.parts * M * N * (int64_t)sizeof(float);
+        return 0;
+    }
     if (M > 0 && K % 64 == 0 && tiled(M, N, K, true)) {
         const TilePlan p = int8wo_gemm_plan(M, N, K, 8);
         if (p.parts > 1) *bytes = p.parts * M * N * (int64_t)sizeof(float);
@@ -621,7 +692,12 @@ extern "C" int ao_amd_int8wo_linear_ws_bytes(int64_t M, int64_t K, int64_t N, in
 
 extern "C" int ao_amd_int8wo_linear_plan(int64_t M, int64_t K, int64_t N, char* out, int64_t out_cap) {
     AO_REQUIRE(out && out_cap > 0 && M > 0 && N > 0 && K > 0 && K % 64 == 0, "need positive M and N, K a multiple of 64, and a buffer");
-    if (!tiled(M, N, K, true)) {
+    const Int8Rows rows = int8_rows_plan(M, K, N);
+    if (rows.kind == Int8Rows::four_parts) {
+        snprintf(out, (size_t)out_cap, "streaming parts=%d", rows.parts);
+        return 0;
+    }
+    if (rows.kind == Int8Rows::other ? !tiled(M, N, K, true) : rows.kind == Int8Rows::streaming) {
         snprintf(out, (size_t)out_cap, "streaming");
         return 0;
     }
@@ -633,8 +709,14 @@ extern "C" int ao_amd_int8wo_linear_ws(const void* x_bf16, int64_t M, int64_t K,
                                        const void* scale_bf16, int64_t N, const void* bias_bf16, void* y, int y_dtype, int64_t ldy,
                                        void* workspace, int64_t workspace_bytes, void* stream) {
     AO_REQUIRE(!workspace || (((uintptr_t)workspace) & 15) == 0, "the workspace must be 16-byte aligned");
+    // (rows whose workspace is not there take the routes of a call without one)
+    Int8Rows rows = y_dtype == AO_BF16 ? int8_rows_plan(M, K, N) : Int8Rows{Int8Rows::other, 1};
+    if (rows.parts > 1 && (!workspace || workspace_bytes < rows.parts * M * N * (int64_t)sizeof(float))) rows.kind = Int8Rows::other;
+    if (rows.kind == Int8Rows::four_parts)
+        return int8wo_four_parts(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, ldy, rows.parts, (float*)workspace, stream);
+    const bool tiles = rows.kind == Int8Rows::other ? tiled(M, N, K, workspace != nullptr) : rows.kind == Int8Rows::tiles;
     // (in_features that are an odd multiple of 64 have no other kernel)
-    if (y_dtype == AO_BF16 && K % 64 == 0 && tiled(M, N, K, workspace != nullptr) && (K % 128 != 0 || tiles_reach(M, N, ldx, ldw)))
+    if (y_dtype == AO_BF16 && K % 64 == 0 && tiles && (K % 128 != 0 || tiles_reach(M, N, ldx, ldw)))
         return int8wo_tiled(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, ldy, nullptr, 0, nullptr, 0, (float*)workspace, workspace_bytes, stream);
     return int8wo_dispatch(x_bf16, M, K, ldx, w_int8, ldw, scale_bf16, N, bias_bf16, y, y_dtype, ldy, nullptr, 0, nullptr, 0, stream);
 }

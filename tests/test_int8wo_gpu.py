@@ -370,3 +370,38 @@ def test_rows_that_are_far_apart():
     # each side sums exact products in fp32 and rounds twice to bf16: within a step (2^-8) each
     for got, ref in ((ops.int8wo_linear(x, w, scale), want), (ops.int8wo_linear_residual(x, w, scale, other), want + other)):
         assert (got.float() - ref.float()).norm() <= 2 ** -7 * ref.float().norm()
+
+
+# 2 to 16 rows with K in parts: the first and last row counts, a shorter last part, row blocks that are no multiple of four and rows that end within one, a
+# bias, and the same call without a workspace
+@pytest.mark.parametrize("N,K,M,parts", [(5120, 13824, 2, 3), (5120, 13824, 16, 3), (4096, 14336, 11, 4), (2048, 16384, 7, 8), (1000, 14336, 16, 8),
+                                         (2069, 16256, 13, 7), (5160, 5120, 12, 3)])
+def test_few_rows_in_parts(N, K, M, parts):
+    import ctypes
+
+    from ao_amd import _lib, ops
+
+    L, plan, need = _lib.lib(), ctypes.create_string_buffer(64), ctypes.c_int64(-1)
+    _lib.check(L.ao_amd_int8wo_linear_plan(M, K, N, plan, 64))
+    assert plan.value.decode() == f"streaming parts={parts}"
+    _lib.check(L.ao_amd_int8wo_linear_ws_bytes(M, K, N, ctypes.byref(need)))
+    assert need.value == 4 * parts * M * N
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    w = torch.randint(-128, 128, (N, K), device="cuda", dtype=torch.int8, generator=g)
+    x, b = torch.randn(M, K, device="cuda", generator=g).bfloat16(), torch.randn(N, device="cuda", generator=g).bfloat16()
+    s = (torch.rand(N, device="cuda", generator=g) * 0.01 + 0.001).bfloat16()
+    scaled = ((x.float() @ w.float().t()).bfloat16().float() * s.float()).bfloat16()
+    for bias, want in ((None, scaled), (b, (scaled.float() + b.float()).bfloat16())):
+        y, plain = ops.int8wo_linear(x, w, s, bias), torch.empty_like(scaled)
+        _lib.check(L.ao_amd_int8wo_linear(x.data_ptr(), M, K, K, w.data_ptr(), K, s.data_ptr(), N, None if bias is None else bias.data_ptr(), plain.data_ptr(),
+                                          _lib.BF16, N, torch.cuda.current_stream().cuda_stream))
+        # exact products; fp32 sums of K of them in another order move a rounding now and then, by one step of the result
+        for got in (y, plain):
+            assert (got != want).float().mean() <= 0.01 and ((got.float() - want.float()).norm() / want.float().norm()).item() <= 1e-3
+    # one-hot rows at both ends of K and of the parts read the weight back
+    per = -(-(K // 128) // parts) * 128
+    ends = [0, K - 1] + [k for z in range(1, parts) for k in (z * per - 1, z * per)]
+    ks = torch.tensor([ends[i % len(ends)] for i in range(M)], device="cuda")
+    xh = torch.zeros(M, K, device="cuda").bfloat16()
+    xh[torch.arange(M, device="cuda"), ks] = 1.0
+    assert torch.equal(ops.int8wo_linear(xh, w, s, None), (w[:, ks].float().t() * s.float()).bfloat16())
