@@ -79,13 +79,13 @@ static void launch_shape(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
     typedef Fp6Tile<E3M2> F;
     tile_grid(a, kFp6Shapes[p.shape], 48, p.parts);
     switch (p.shape) {
-        case 0: tile_launch<F, 2, 4, 2, 1>(a, p.parts, st); break;
-        case 1: tile_launch<F, 4, 2, 2, 1>(a, p.parts, st); break;
-        case 2: tile_launch<F, 4, 2, 3, 1>(a, p.parts, st); break;
-        case 3: tile_launch<F, 4, 2, 4, 1>(a, p.parts, st); break;
-        case 4: tile_launch<F, 4, 1, 3, 1, 2>(a, p.parts, st); break;
-        case 5: tile_launch<F, 4, 1, 4, 2>(a, p.parts, st); break;
-        default: tile_launch<F, 8, 1, 6, 1>(a, p.parts, st); break;
+        case 0: tile_launch<F, 2, 4, 2, 1>(a, st); break;
+        case 1: tile_launch<F, 4, 2, 2, 1>(a, st); break;
+        case 2: tile_launch<F, 4, 2, 3, 1>(a, st); break;
+        case 3: tile_launch<F, 4, 2, 4, 1>(a, st); break;
+        case 4: tile_launch<F, 4, 1, 3, 1, 2>(a, st); break;
+        case 5: tile_launch<F, 4, 1, 4, 2>(a, st); break;
+        default: tile_launch<F, 8, 1, 6, 1>(a, st); break;
     }
     tile_finish<F>(a, p.parts, st);
 }

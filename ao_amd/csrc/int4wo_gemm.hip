@@ -150,7 +150,7 @@ __device__ __forceinline__ const T* uniform_ptr(const T* p) {
 // registers, in the shadow of the matrix instructions.  The activation slice (256 x 64 bf16) is shared through LDS,
 // double buffered, one barrier per K step.
 //
-// K may be split over blockIdx.y (launch_int4wo_gemm_lds_parts) where the tiles of a narrow weight leave CUs idle: 4096 x 14336 at
+// K may be split over workgroups (launch_int4wo_gemm_lds_parts) where the tiles of a narrow weight leave CUs idle: 4096 x 14336 at
 // 1000 rows, 128 tiles of 256 x 128 in two parts each, 123 us against 137 of the 128-row kernel's 512 workgroups.
 //
 // One K step = 4 sub-steps ks of 16 slots; a slot is one matrix instruction followed by the work that runs in its
@@ -172,12 +172,12 @@ __global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int tile_m, tile_n;
-    if (!tile_at(TileOrder{tiles_m, tiles_n, panel}, (int)blockIdx.x, tile_m, tile_n)) return;
+    int tile_m, tile_n, part;
+    tile_at(TileOrder{tiles_m, tiles_n, panel, a.ksplit}, (int)blockIdx.x, tile_m, tile_n, part);
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
-    // the 64-wide K steps of this workgroup: all of them, or with a.ksplit > 1 the blockIdx.y-th run of an even number of them,
-    // whose fp32 products go to part blockIdx.y of a.y [ksplit][M][ldy]
-    const int KA = (int)(a.Kp / 64), per = ((KA + a.ksplit - 1) / a.ksplit + 1) & ~1, first = per * (int)blockIdx.y;
+    // the 64-wide K steps of this workgroup: all of them, or with a.ksplit > 1 the part-th run of an even number of them,
+    // whose fp32 products go to that part of a.y [ksplit][M][ldy]
+    const int KA = (int)(a.Kp / 64), per = ((KA + a.ksplit - 1) / a.ksplit + 1) & ~1, first = per * part;
     const int KS = KA - first < per ? KA - first : per;
     const int KB = (int)(a.Kp / 128);
     const int64_t nblocks = (a.N + 15) / 16;
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(256) void int4wo_gemm_lds_kernel(const LinearArgs a
                 const int64_t m = m0 + i * 32 + 8 * (e >> 2) + 4 * kq + (e & 3);
                 if (m < a.M) {
                     const float v = acc_read(acc[i][j][e]) + bv;
-                    if (a.y_is_f32) ((float*)a.y)[((int64_t)blockIdx.y * a.M + m) * a.ldy + n] = v;
+                    if (a.y_is_f32) ((float*)a.y)[((int64_t)part * a.M + m) * a.ldy + n] = v;
                     else ((uint16_t*)a.y)[m * a.ldy + n] = f32_to_bf16_bits(v);
                 }
             }
@@ -422,8 +422,8 @@ __device__ __forceinline__ void gemm_kwave(const LinearArgs& a, int tiles_m, int
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int tile_m, tile_n;
-    if (!tile_at(TileOrder{tiles_m, tiles_n, panel}, (int)blockIdx.x, tile_m, tile_n)) return;
+    int tile_m, tile_n, part;
+    tile_at(TileOrder{tiles_m, tiles_n, panel, 1}, (int)blockIdx.x, tile_m, tile_n, part);
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
     const int KS = (int)(a.Kp / 64);
     const int KB = (int)(a.Kp / 128);
@@ -718,7 +718,7 @@ bool int4wo_gemm_lds_plan(const LinearArgs& a, int64_t g, Int4Plan* plan) {
 static void launch_gemm_kwave(const LinearArgs& a, int64_t g, const GemmLdsPlan& p, hipStream_t st) {
     const bool three = (a.M + 95) / 96 == p.tiles_m;   // 96-row tiles where they are no more
     const TileOrder order = tile_order(p.tiles_m, p.tiles_n, (three ? 96 : 128) * 128, 64 * 32);
-    const dim3 grid((unsigned)(order.per_xcd() * 8)), block(256);
+    const dim3 grid(order.workgroups()), block(256);
     auto go = [&](auto kernel) {
         if (g_prof_start && g_prof_stop) {
             hipExtLaunchKernelGGL(kernel, grid, block, 0, st, g_prof_start, g_prof_stop, 0, a, order.tiles_m, order.tiles_n, order.panel);
@@ -745,8 +745,8 @@ static void launch_gemm_kwave(const LinearArgs& a, int64_t g, const GemmLdsPlan&
 // 105.1 / 103.0; level up to 1500 rows.
 template <int NT>
 static void launch_gemm_lds_nt(const LinearArgs& a, int64_t g, const GemmLdsPlan& p, hipStream_t st, bool copied = false) {
-    const TileOrder order{p.tiles_m, p.tiles_n, copied ? 1 : p.tiles_m <= 4 ? p.tiles_m : 2};
-    const dim3 grid((unsigned)(order.per_xcd() * 8), (unsigned)a.ksplit), block(256);
+    const TileOrder order{p.tiles_m, p.tiles_n, copied ? 1 : p.tiles_m <= 4 ? p.tiles_m : 2, a.ksplit};
+    const dim3 grid(order.workgroups()), block(256);
     auto go = [&](auto kernel) {
         if (g_prof_start && g_prof_stop) {
             hipExtLaunchKernelGGL(kernel, grid, block, 0, st, g_prof_start, g_prof_stop, 0, a, order.tiles_m, order.tiles_n, order.panel);

@@ -269,12 +269,12 @@ extern "C" int ao_amd_int4wo_linear_tiled(const void* x_bf16, int64_t M, int64_t
     hipStream_t st = (hipStream_t)stream;
     tile_grid(a, kInt4Shapes[p.shape], 32, p.parts);
     switch (p.shape) {
-        case 0: tile_launch<Int4Tile, 2, 4, 2, 1>(a, p.parts, st); break;
-        case 1: tile_launch<Int4Tile, 4, 2, 2, 1>(a, p.parts, st); break;
-        case 2: tile_launch<Int4Tile, 4, 2, 3, 1>(a, p.parts, st); break;
-        case 3: tile_launch<Int4Tile, 4, 2, 4, 1>(a, p.parts, st); break;
-        case 4: tile_launch<Int4Tile, 4, 1, 6, 1>(a, p.parts, st); break;
-        case 5: tile_launch<Int4Tile, 4, 1, 8, 1>(a, p.parts, st); break;
+        case 0: tile_launch<Int4Tile, 2, 4, 2, 1>(a, st); break;
+        case 1: tile_launch<Int4Tile, 4, 2, 2, 1>(a, st); break;
+        case 2: tile_launch<Int4Tile, 4, 2, 3, 1>(a, st); break;
+        case 3: tile_launch<Int4Tile, 4, 2, 4, 1>(a, st); break;
+        case 4: tile_launch<Int4Tile, 4, 1, 6, 1>(a, st); break;
+        case 5: tile_launch<Int4Tile, 4, 1, 8, 1>(a, st); break;
         default: {
             LinearArgs l{};
             l.x = a.x; l.M = M; l.K = l.Kp = K; l.ldx = ldx;

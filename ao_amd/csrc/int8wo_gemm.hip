@@ -117,8 +117,8 @@ template <bool PAIR>
 static bool launch_paired(const TileGemmArgs& a, const TilePlan& p, hipStream_t st) {
     typedef Int8Tile<PAIR> F;
     switch (p.shape) {
-        case 0: tile_launch<F, 4, 2, 2, 1>(a, p.parts, st); return true;
-        case 4: tile_launch<F, 8, 1, 4, 1>(a, p.parts, st); return true;
+        case 0: tile_launch<F, 4, 2, 2, 1>(a, st); return true;
+        case 4: tile_launch<F, 8, 1, 4, 1>(a, st); return true;
         default: return false;
     }
 }
@@ -127,11 +127,11 @@ void launch_int8wo_gemm(TileGemmArgs a, const TilePlan& p, hipStream_t st) {
     tile_grid(a, kInt8Shapes[p.shape], 64, p.parts);
     if (!(a.K % 128 == 0 ? launch_paired<true>(a, p, st) : launch_paired<false>(a, p, st))) {
         switch (p.shape) {
-            case 1: tile_launch<Int8Tile<false>, 4, 1, 3, 1>(a, p.parts, st); break;
-            case 2: tile_launch<Int8Tile<false>, 4, 2, 4, 1>(a, p.parts, st); break;
-            case 3: tile_launch<Int8Tile<false>, 4, 1, 3, 1, 2>(a, p.parts, st); break;
-            case 5: tile_launch<Int8Tile<false>, 2, 4, 2, 1>(a, p.parts, st); break;
-            default: tile_launch<Int8Tile<false>, 8, 1, 6, 1>(a, p.parts, st); break;
+            case 1: tile_launch<Int8Tile<false>, 4, 1, 3, 1>(a, st); break;
+            case 2: tile_launch<Int8Tile<false>, 4, 2, 4, 1>(a, st); break;
+            case 3: tile_launch<Int8Tile<false>, 4, 1, 3, 1, 2>(a, st); break;
+            case 5: tile_launch<Int8Tile<false>, 2, 4, 2, 1>(a, st); break;
+            default: tile_launch<Int8Tile<false>, 8, 1, 6, 1>(a, st); break;
         }
     }
     tile_finish<Int8Tile<false>>(a, p.parts, st);

@@ -46,7 +46,7 @@ struct TileGemmArgs {
     const uint16_t* residual; int64_t ldres;   // y += residual, or null
     const uint16_t* gate; int64_t ldgate;      // y = silu(gate) * y, or null
     int group_shift;                    // int4: log2 of the group size
-    float* parts;                       // K split over blockIdx.y: fp32 partial products [gridDim.y][M][N], or null
+    float* parts;                       // K in parts: fp32 partial products [order.parts][M][N], or null
 };
 
 template <int N>
@@ -85,13 +85,13 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void tile_gemm_kernel(const Tile
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int group = wave / G, gw = wave % G, wn = gw % WN, wm = WM == 1 ? 0 : gw / WN;
-    int tile_m, tile_n;
-    if (!tile_at(a.order, (int)blockIdx.x, tile_m, tile_n)) return;
+    int tile_m, tile_n, part;
+    tile_at(a.order, (int)blockIdx.x, tile_m, tile_n, part);
     const int64_t m0 = (int64_t)tile_m * BM, n0 = (int64_t)tile_n * BN;
-    // this workgroup's run of 64-wide K steps: all of them, or the blockIdx.y-th of gridDim.y equal parts
+    // this workgroup's run of 64-wide K steps: all of them, or the part-th of order.parts equal parts
     // (PAIR: whole pairs, and the groups take pairs; a last part may be left without any and stores zeros)
     constexpr int UNIT = PAIR ? 2 : 1;
-    const int all = (int)(a.K / 64), per = (all / UNIT + (int)gridDim.y - 1) / (int)gridDim.y * UNIT, first = per * (int)blockIdx.y;
+    const int all = (int)(a.K / 64), per = (all / UNIT + a.order.parts - 1) / a.order.parts * UNIT, first = per * part;
     const int KS = PAIR ? max(min(per, all - first), 0) : min(per, all - first);
     const int nst = PAIR ? KS / (2 * KW) * 2 + min(KS % (2 * KW), 2) : (KS + KW - 1) / KW;
 
@@ -282,7 +282,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void tile_gemm_kernel(const Tile
                 const int64_t m = m0 + (wm * MT + i) * 32 + r32;
                 if (m >= a.M) continue;
                 if (a.parts) {
-                    float* dst = a.parts + ((int64_t)blockIdx.y * a.M + m) * a.N + n;
+                    float* dst = a.parts + ((int64_t)part * a.M + m) * a.N + n;
                     if ((a.N & 3) == 0 && n + 3 < a.N)
                         *(float4*)dst = make_float4(acc[i][j][e], acc[i][j][e + 1], acc[i][j][e + 2], acc[i][j][e + 3]);
                     else
@@ -405,13 +405,14 @@ inline TilePlan tile_plan(const TileShape* shapes, int nshapes, int64_t M, int64
 // row_bytes: a weight row's bytes in a 64-wide step.
 inline void tile_grid(TileGemmArgs& a, const TileShape& s, int row_bytes, int parts) {
     a.order = tile_order((a.M + s.bm - 1) / s.bm, (a.N + s.bn - 1) / s.bn, s.bm * 128, s.bn * row_bytes);
+    a.order.parts = parts;
     if (parts == 1) a.parts = nullptr;
 }
 template <class F, int WN, int KW, int MT, int NT, int WM = 1>
-void tile_launch(const TileGemmArgs& a, int parts, hipStream_t st) {
+void tile_launch(const TileGemmArgs& a, hipStream_t st) {
     hipEvent_t ev0 = g_prof_start, ev1 = g_prof_stop;
     g_prof_start = g_prof_stop = nullptr;
-    hipExtLaunchKernelGGL((tile_gemm_kernel<F, WN, KW, MT, NT, WM>), dim3((unsigned)(a.order.per_xcd() * 8), (unsigned)parts), dim3(64 * WM * WN * KW), 0, st,
+    hipExtLaunchKernelGGL((tile_gemm_kernel<F, WN, KW, MT, NT, WM>), dim3(a.order.workgroups()), dim3(64 * WM * WN * KW), 0, st,
                           ev0, ev1, 0, a);
 }
 template <class F>

@@ -406,7 +406,9 @@ def test_every_tile_once(fmt, M, N, K, group, name):
 @pytest.mark.parametrize("fmt,M,N,K,plan", [
     ("int8", 40, 5120, 13824, "tile 64x128 parts=6"), ("int8", 61, 10200, 8320, "tile 64x128 parts=3"), ("int8", 77, 10240, 8256, "tile 96x128 parts=3"),
     ("int8", 100, 2300, 4160, "tile 64x64 parts=3"), ("int4wo", 40, 5120, 5120, "tile 64x64 parts=3"), ("int4wo", 90, 5110, 13888, "tile 96x128 parts=6"),
-    ("int4wo", 200, 5120, 13824, "tile 128x128 parts=3"), ("fp6", 113, 5120, 13824, "tile 64x128 parts=3"), ("fp6", 77, 5120, 13888, "tile 96x128 parts=6")])
+    ("int4wo", 200, 5120, 13824, "tile 128x128 parts=3"), ("fp6", 113, 5120, 13824, "tile 64x128 parts=3"), ("fp6", 77, 5120, 13888, "tile 96x128 parts=6"),
+    # tiles times parts that the XCDs cannot share evenly: 41 x 6, 33 x 7
+    ("int8", 40, 5128, 13824, "tile 64x128 parts=6"), ("int8", 24, 4104, 14336, "tile 64x128 parts=7"), ("int4wo", 130, 4110, 13888, "tile 192x128 parts=7")])
 def test_parts_that_are_no_power_of_two(fmt, M, N, K, plan):
     assert (_plan(M, N, K) if fmt == "int8" else _tiled_plan(fmt, M, N, K)) == plan
     # (the bounds of the helpers: up to 13888 products a sum)
