@@ -42,8 +42,12 @@ inline TileOrder tile_order(int64_t tiles_m, int64_t tiles_n, int64_t x_bytes, i
 __device__ __forceinline__ void tile_at(const TileOrder& o, int block, int& tile_m, int& tile_n, int& part) {
     const int tiles = o.tiles_m * o.tiles_n;
     int tile = xcd_run(block, tiles * o.parts);
-    // (a division of scalars runs on the vector unit and leaves its result there)
-    for (part = 0; tile >= tiles; ++part) tile -= tiles;
+    // at most eight parts: compared rather than divided, since a division of scalars runs on the vector unit and leaves its result there
+    part = 0;
+#pragma unroll
+    for (int z = 1; z < 8; ++z) part += tile >= z * tiles;
+    part = __builtin_amdgcn_readfirstlane(part);
+    tile -= part * tiles;
     const int per_panel = o.panel * o.tiles_n;
     int p = 0, in = tile;
     if (tile >= per_panel) p = tile / per_panel, in = tile - p * per_panel;
