@@ -115,6 +115,12 @@ static TilePlan int4wo_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts)
 static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
     Int4Kernel kernel;
     if (!int4wo_plain_kernel(M, K, N, g, &kernel)) return 0.0;
+    const int parts = ao_amd_int4wo_linear_ws_parts(M, K, N, g);
+    const int64_t per = (K / 128 + parts - 1) / parts;
+    // (33 to 64 rows, one tile row: the ws kernel's parts are powers of two and its 64 x 64 tiles without the tiled product's pipeline.  us there / tiled at 33, 64
+    // rows: 5120 x 13824 31.7 / 23.5, 32.8 / 24.3; 8192 x 8192 24.1 / 22.3, 24.8 / 23.0; 4096 x 14336 23.2 / 22.2, 22.6 / 22.1; up to 16 tiles a part it is level or ahead:
+    // 4096 x 4096 11.9 / 12.4, 13.0 / 13.2; 4096 x 6144 13.2 / 13.9, 14.5 / 14.5)
+    if (parts > 1 && M <= 64) return per >= 20 ? 8.0 + 0.46 * (double)per : 0.0;
     if (kernel == Int4Kernel::streaming) {
         // Four blocks of streamed rows (weights of 768 row blocks and up) are behind the tiles, except where the weight has very many rows and the batch
         // few.  us at 33 / 48 rows, streamed / tiled: 12288 x 1024 8.6 / 8.4, 9.1 / 8.3; 14336 x 4096 18.9 / 17.2, 19.3 / 17.3; 13824 x 5120 22.1 / 19.9, 23.8 / 20.2; 16384
@@ -123,7 +129,13 @@ static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
         // end early, 18837 x 1088 14.9 / 12.0, 16.1 / 12.8.  Up to 32 rows (two blocks) the streaming kernel is ahead: 14336 x 1024 at 32 rows 7.7 / 8.3,
         // 65536 x 4096 49.0 / 58.1.
         const int64_t blocks = (N + 15) / 16;
-        return blocks >= 768 && (blocks <= 4096 || M > 48) ? 1e9 : 0.0;
+        // (one block a workgroup, 16 rows at a time, up to 768 of them: XXX)
+        // Narrower ones are streamed 16 rows and one block a workgroup, or four blocks where K is long; an estimate of each.  us streamed / tiled at 33, 40 rows: 2048
+        // x 16384 25.1 / 16.1, 32.0 / 16.2; 3072 x 8192 22.0 / 14.7, 23.8 / 14.8; 1024 x 14336 17.8 / 14.3; 3584 x 18944 44.4 / 23.4; 256 x 28672 30.7 / 19.1 (40); ahead where K
+        // is short: 2048 x 4096 8.6 / 11.7 (33), 1024 x 8192 11.6 / 12.4 (33).
+        const double tiles = (double)(K / 128), full = (double)(blocks * ((M + 15) / 16)) / 256.0;
+        if (blocks < 768) return fmin(2.6 + 0.12 * tiles * fmax(1.0, full), 6.2 + 0.05 * (double)M + 0.35 * tiles);
+        return blocks <= 4096 || M > 48 ? 1e9 : 0.0;
     }
     const double k = (double)K / 4096.0;
     auto rounds = [&](int bm, int bn) { return (double)((M + bm - 1) / bm * ((N + bn - 1) / bn)) / 256.0; };
@@ -143,7 +155,7 @@ static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
     }
     // (short K: the sums of eight parts cost the tiles more than they save.  us in K parts there / tiled at 100 rows: 512 x 4096 10.7 / 11.4, 1024 x 4096
     // 11.1 / 12.6, 1536 x 4096 11.5 / 12.0, 1024 x 2048 10.3 / 10.4, 1024 x 6144 12.5 / 12.9; 512 x 8192 14.1 / 13.3, 1024 x 14336 20.0 / 16.5)
-    if (ao_amd_int4wo_linear_ws_parts(M, K, N, g) > 1) return M <= 64 || K < 7168 ? 0.0 : 4.0 + 8.0 * k;
+    if (parts > 1) return K < 7168 ? 0.0 : 4.0 + 8.0 * k;
     if (kernel == Int4Kernel::tiles_128x128) return 90.0 * k * rounds(128, 128) / 2.0;
     if (rounds(64, 64) >= 0.75) return 5.0 + (K >= 8192 ? 14.0 : 18.0) * k * up(rounds(64, 64));
     return 4.0 + 10.4 * k * up(rounds(32, 64));

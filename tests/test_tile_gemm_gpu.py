@@ -373,6 +373,24 @@ def test_int4_tiles_where_their_k_parts_pay():
         assert (_tiled_bytes("int4wo", M, N, K, 128) >= 0) == tiled, (M, N, K)
 
 
+@pytest.mark.parametrize("M,N,K,group,tiled", [
+    (33, 2048, 16384, 64, True), (40, 3080, 8320, 128, True), (64, 5120, 13824, 32, True), (47, 1030, 14336, 64, True), (33, 2048, 4096, 64, False),
+    (64, 4096, 4096, 64, False), (33, 1024, 8192, 128, False),
+])
+def test_int4_tiles_at_one_tile_row(M, N, K, group, tiled):
+    """33 to 64 rows of narrow weights: tiles in K parts where K is long (2048 x 16384 at 40 rows 32.0 -> 16.2 us), the streaming kernel or its parts where it
+    is short.  The tolerance is that of two bf16 roundings of one fp32 sum in another order."""
+    from ao_amd import ops
+
+    assert (_tiled_bytes("int4wo", M, N, K, group) >= 0) == tiled
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    packed, qp = ops.int4wo_quantize_pack((torch.randn(N, K, device="cuda", generator=g) * 0.02).bfloat16(), group)
+    x = torch.randn(M, K, device="cuda", generator=g).bfloat16()
+    y, want = ops.int4wo_linear(x, packed, qp, group, N), (x.float() @ ops.int4wo_dequantize(packed, qp, N, K, group).float().t()).bfloat16()
+    rel = ((y.float() - want.float()).norm() / want.float().norm()).item()
+    assert rel <= 1e-3 and (y != want).float().mean() <= 0.01, rel
+
+
 @pytest.mark.parametrize("fmt,M,N,K,group,name", [
     ("int4", 1700, 7000, 512, 64, "int4wo_gemm_lds_kernel<64,2>"), ("int4", 1000, 6400, 512, 128, "int4wo_gemm_lds_kernel<128,1>"),
     ("int4", 300, 4100, 1024, 32, "int4wo_gemm_kwave_kernel"), ("int4", 2750, 1024, 4096, 64, ""), ("int4", 5000, 64, 256, 64, ""),
