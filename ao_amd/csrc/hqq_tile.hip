@@ -20,7 +20,6 @@
 
 #include "hqq_format.h"
 #include "lds_dma.h"
-#include "tile_order.h"
 
 namespace ao {
 
@@ -32,9 +31,9 @@ struct HqqTileArgs {
     const uint8_t* packed;
     const uint16_t *scales, *zeros, *a;
     int64_t lda, M, K, N, group;
-    int tiles_m, tiles, parts;
+    int tiles_m, tiles, per_xcd;
     uint32_t per_group;   // forward: 2^32 / (group / 64) rounded up, exact for the steps that hqq_tile_plan admits, or 0 where a step is a group
-    float* part;      // [parts][M][columns], or null: y is written
+    float* part;      // [gridDim.y][M][columns], or null: y is written
     uint16_t* y;
 };
 
@@ -61,13 +60,13 @@ __global__ __launch_bounds__(256) void hqq_tile_kernel(const HqqTileArgs g) {
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int tile = xcd_run((int)blockIdx.x, g.tiles * g.parts), k_part = 0;
-    for (; tile >= g.tiles; ++k_part) tile -= g.tiles;
+    const int tile = (int)(blockIdx.x & 7) * g.per_xcd + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= g.per_xcd || tile >= g.tiles) return;
     // the row tiles of a weight tile are neighbours on one XCD, whose L2 then holds its codes
     const int tile_n = tile / g.tiles_m, tile_m = tile - tile_n * g.tiles_m;
     const int64_t m0 = (int64_t)tile_m * BM, c0 = (int64_t)tile_n * BN;   // first row, first output column
     const int64_t R = TR ? g.N : g.K, K2 = g.K / 2;
-    const int all = (int)((R + 63) / 64), per = (all + g.parts - 1) / g.parts, first = per * k_part;
+    const int all = (int)((R + 63) / 64), per = (all + (int)gridDim.y - 1) / (int)gridDim.y, first = per * (int)blockIdx.y;
     const int KS = min(per, all - first), nst = (KS - wave + W - 1) / W;   // this wave's steps: first + wave + 4 t
     const int r32 = lane & 31, half = lane >> 5;
 
@@ -371,7 +370,7 @@ __global__ __launch_bounds__(256) void hqq_tile_kernel(const HqqTileArgs g) {
                 }
                 if (col >= cols) continue;
                 if (g.part) {
-                    *(float4*)(g.part + ((int64_t)k_part * g.M + m) * cols + col) = quad[0];
+                    *(float4*)(g.part + ((int64_t)blockIdx.y * g.M + m) * cols + col) = quad[0];
                 } else {
                     uint16_t o[4];
                     const float f[4] = {quad[0].x, quad[0].y, quad[0].z, quad[0].w};
@@ -473,10 +472,10 @@ static void launch_direction(bool transposed, int rows, dim3 grid, const HqqTile
 void launch_hqq_tile(const HqqTilePlan& p, const uint8_t* packed, const uint16_t* scales, const uint16_t* zeros, const uint16_t* a, int64_t lda,
                      int64_t M, int64_t K, int64_t N, int64_t group, bool is_signed, bool bf16, bool transposed, float* part, uint16_t* y,
                      hipStream_t st) {
-    const int tiles = p.tiles_m * p.tiles_n;
-    const HqqTileArgs g{packed, scales, zeros, a, lda, M, K, N, group, p.tiles_m, tiles, p.parts,
+    const int tiles = p.tiles_m * p.tiles_n, per_xcd = (tiles + 7) / 8;
+    const HqqTileArgs g{packed, scales, zeros, a, lda, M, K, N, group, p.tiles_m, tiles, per_xcd,
                         group == 64 ? 0u : (uint32_t)((((uint64_t)1 << 32) + group / 64 - 1) / (uint64_t)(group / 64)), p.parts > 1 ? part : nullptr, y};
-    const dim3 grid((unsigned)tiles * (unsigned)p.parts);
+    const dim3 grid((unsigned)(per_xcd * 8), (unsigned)p.parts);
     if (bf16) is_signed ? launch_direction<true, true>(transposed, p.rows, grid, g, st) : launch_direction<true, false>(transposed, p.rows, grid, g, st);
     else is_signed ? launch_direction<false, true>(transposed, p.rows, grid, g, st) : launch_direction<false, false>(transposed, p.rows, grid, g, st);
     if (p.parts > 1) launch_hqq_finish(part, p.parts, M * (transposed ? K : N), bf16, y, st);
