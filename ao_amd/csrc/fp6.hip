@@ -1894,4 +1894,3 @@ extern "C" int ao_amd_fp6_native_to_f16(const void* weights_native, const void* 
     AO_LAUNCH_CHECK();
     return 0;
 }
-

@@ -1530,8 +1530,9 @@ static int ws_parts(int64_t M, int64_t K, int64_t N, int64_t g) {
 int ao::int4wo_stream_parts(int64_t M, int64_t K, int64_t N, int64_t g) {
     if (M < 4 || M > 32 || N % 4 != 0) return 1;
     int64_t Np, Kp;
-    if (ao_amd_int4wo_packed_shape(N, K, g, &Np, &Kp, nullptr, nullptr) || Kp != K) return 1;
-    const int64_t KB = Kp / 128, RB = Np / 16, groups = (RB + 3) / 4;
+    if (ao_amd_int4wo_packed_shape(N, K, g, &Np, &Kp, nullptr, nullptr)) return 1;
+    // (what K reaches, as the launch counts: with g = 256 the packed row may have a tile more, and 49 tiles are not 50 in eight parts, the last would be empty)
+    const int64_t KB = (K + 127) / 128, RB = Np / 16, groups = (RB + 3) / 4;
     if (groups >= 192 || KB < 8 || KB >= (1 << 21)) return 1;
     const double m = (double)M;
     auto whole = [&]() {   // one row block a workgroup, 16 rows at a time

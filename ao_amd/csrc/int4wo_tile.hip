@@ -129,7 +129,6 @@ static double int4wo_other_us(int64_t M, int64_t N, int64_t K, int64_t g) {
         // end early, 18837 x 1088 14.9 / 12.0, 16.1 / 12.8.  Up to 32 rows (two blocks) the streaming kernel is ahead: 14336 x 1024 at 32 rows 7.7 / 8.3,
         // 65536 x 4096 49.0 / 58.1.
         const int64_t blocks = (N + 15) / 16;
-        // (one block a workgroup, 16 rows at a time, up to 768 of them: XXX)
         // Narrower ones are streamed 16 rows and one block a workgroup, or four blocks where K is long; an estimate of each.  us streamed / tiled at 33, 40 rows: 2048
         // x 16384 25.1 / 16.1, 32.0 / 16.2; 3072 x 8192 22.0 / 14.7, 23.8 / 14.8; 1024 x 14336 17.8 / 14.3; 3584 x 18944 44.4 / 23.4; 256 x 28672 30.7 / 19.1 (40); ahead where K
         // is short: 2048 x 4096 8.6 / 11.7 (33), 1024 x 8192 11.6 / 12.4 (33).
@@ -233,7 +232,7 @@ static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t
         r->copy = M * Kp * 2;
         r->as_is = aligned && K % 8 == 0 && int4wo_takes_short_rows(M, N, g);
     }
-    r->stream_parts = (K == Kp && aligned) || r->Kp ? int4wo_stream_parts(M, Kp, N, g) : 1;
+    r->stream_parts = (K == Kp && aligned) || r->Kp ? int4wo_stream_parts(M, r->as_is ? K : Kp, N, g) : 1;
     if (r->stream_parts > 1) {
         r->parts = r->stream_parts * M * N * (int64_t)sizeof(float);
         return 0;

@@ -111,11 +111,11 @@ def test_workspace_linear_refusals_and_fallbacks():
 
 # (N, K, group, M, K parts): an even split and a last part that is shorter; row blocks that are no multiple of four, the last one with 4 rows;
 # more workgroups than CUs; rows that end before the packed width, read as they are (up to 15) and copied; g = 256 with a packed tile that no row
-# reaches; 4, 16, 17 and 32 rows; and neighbours of those calls that are not split
+# reaches (and which makes 50 tiles, eight parts, of 49, which have no eight of one length); 4, 16, 17 and 32 rows; and neighbours of those calls that are not split
 @pytest.mark.parametrize("N,K,g,M,parts", [
     (8192, 8192, 64, 16, 2), (5120, 13824, 64, 4, 1), (5120, 13824, 64, 6, 3), (5120, 13824, 32, 13, 3), (5120, 13824, 128, 17, 3),
     (5120, 13824, 64, 32, 3), (5120, 13824, 64, 33, 0), (10240, 8192, 64, 16, 3), (1000, 14336, 128, 16, 8), (2052, 16384, 256, 16, 7),
-    (5000, 8000, 256, 13, 3), (5000, 8000, 256, 20, 3), (5120, 13768, 128, 15, 3), (5120, 13768, 128, 18, 3), (4096, 4096, 64, 16, 1)])
+    (5000, 8000, 256, 13, 3), (5000, 8000, 256, 20, 3), (2048, 6272, 256, 15, 7), (5120, 13768, 128, 15, 3), (5120, 13768, 128, 18, 3), (4096, 4096, 64, 16, 1)])
 def test_few_rows_of_narrow_weights_in_parts(N, K, g, M, parts):
     from ao_amd import _lib, ops
 
