@@ -1744,7 +1744,7 @@ int ao::fp6_ws_parts(int64_t M, int64_t K, int64_t N) {
 //  * tiles: fp6_gemm_kernel's 64 columns in parts that are no power of two (5120 x 13824 at 32 rows 21.5 / 18.4) or of narrow weights (1024 x 14336 at 40 rows
 //    18.9 / 13.2), 48 rows a tile up to 48 (4096 x 4096 at 48 rows 11.0 / 10.4, the fourth block was padding);
 //  * wide: 128 columns a tile and twice the parts, from 33 rows on: x, at 48 rows twice the bytes of the codes, is read half as often.  5120 x 13824 at 48 / 64 rows
-//    30.4 / 20.9, 31.6 / 23.2; 8192 x 8192 23.1 / 19.7, 23.6 / 22.0; 4096 x 14336 20.1 / 19.2, 21.1 / 21.0; 7168 x 5120 at 48 rows 15.0 / 14.0.
+//    30.4 / 19.4, 31.6 / 22.6; 8192 x 8192 23.1 / 18.4, 23.6 / 21.3; 6144 x 16384 at 40 rows (four parts / five) 23.4 / 22.3; 7168 x 5120 at 33 rows 14.3 / 12.5.
 // The estimates (us; a part's K tiles, rows, weight bytes) are within some 8 % of those calls.
 struct Fp6Rows {
     enum Kind { none, rows, tiles, wide };
@@ -1756,13 +1756,18 @@ static Fp6Rows fp6_rows_plan(int64_t M, int64_t K, int64_t N) {
     const int64_t KB = K / 128, RB = N / 16, groups = (RB + 3) / 4, wide = (RB + 7) / 8;
     if (KB < 8 || groups >= 192) return best;
     const double m = (double)M, kb = (double)KB, mb = (double)(N * K) * 0.75e-6;
+    // 33 to 64 rows on tiles of 64 columns (48 rows at 33 / 48 rows, 64 at 64; us): 4096 x 4096 / 8192 / 11008 / 14336 in 4 parts 10.7 / 12.3 / 15.8 / 18.4, 10.7 / 12.8 / 16.2 /
+    // 19.1, 11.5 / 14.2 / 17.4 / 19.7; from some 17 K tiles a part on each costs twice as much up to 48 rows
+    auto tiles = [&](double per, int z) {
+        return M <= 48 ? 0.028 * (m - 48.0) + fmax(8.2 + 0.295 * per, 4.2 + 0.53 * per) : 7.35 + 0.345 * per + 0.058 * z + 0.062 * mb;
+    };
     const int z0 = fp6_ws_parts(M, K, N);
     static const bool forced = knob("AO_AMD_WS_PARTS") != nullptr;
     if (forced) return best;
     double other;
     if (z0 > 1) {
         const double per = (double)((KB + z0 - 1) / z0);
-        other = M <= 32 ? (groups < 64 ? 6.1 : 6.9) + 0.315 * per : M <= 48 ? 7.6 + 0.45 * per : 8.0 + 0.47 * per;
+        other = M <= 32 ? (groups < 64 ? 6.1 : 6.9) + 0.315 * per : M <= 48 ? 7.6 + 0.45 * per : tiles(per, z0);
     } else if (M > 32) {
         other = 4.0 + 0.25 * kb * (double)((groups * 2 + 255) / 256);
     } else if (M > 16) {
@@ -1782,7 +1787,7 @@ static Fp6Rows fp6_rows_plan(int64_t M, int64_t K, int64_t N) {
     for (int z = 2; z <= 8; ++z) {
         const int64_t per = (KB + z - 1) / z;
         if (per < 4 || (z - 1) * per >= KB) continue;
-        const double p = (double)per, launch = (M <= 16 ? 0.1 : M <= 32 ? 0.14 : M <= 48 ? 0.1 : 0.2) * z;
+        const double p = (double)per, launch = (M <= 16 ? 0.1 : 0.14) * z;
         if (M <= 16 && groups * z <= 512) offer(Fp6Rows::rows, z, 5.0 + 0.04 * m + (0.24 + 0.002 * m) * p * (groups * z > 256 ? 2.1 : 1.0) + launch);
         if (M > 16 && M <= 32 && groups * z <= 256) {
             offer(Fp6Rows::rows, z, 5.1 + 0.05 * m + (0.22 + 0.0044 * m) * p + launch);
@@ -1790,9 +1795,11 @@ static Fp6Rows fp6_rows_plan(int64_t M, int64_t K, int64_t N) {
         }
         // (short K that is split in four already gains by the 48-row tiles only)
         if (M > 32 && groups * z <= 256 && (z == z0 ? M <= 48 : z0 == 1 || KB >= 64))
-            offer(Fp6Rows::tiles, z, (M <= 48 ? 6.9 + 0.43 * p : 7.6 + 0.47 * p) + launch);
-        // (few workgroups do not bring the weight in at that rate)
-        if (M > 32 && wide * z >= 190 && wide * z <= 256) offer(Fp6Rows::wide, z, (M <= 48 ? 7.0 + 0.235 * mb : 8.0 + 0.27 * mb) + 0.25 * z);
+            offer(Fp6Rows::tiles, z, tiles(p, z) + (z0 == 1 ? 0.6 : 0.0));   // (5120 x 5120 at 48 rows in three parts 12.9, wide in six 12.7)
+        // (a workgroup a CU: parts up to 256 workgroups shorten each, one more part queues.  us in 4 / 6 / 8 / 9 parts at 48 rows: 4096 x 14336 20.8 / 17.8 / 16.6 / 20.3,
+        // 4096 x 11008 17.5 / 15.7 / 15.1 / 17.6; in 5 / 6 / 7: 5120 x 13824 19.5 / 18.5 / 23.6; in 3 / 4 / 5: 8192 x 8192 19.2 / 17.8 / 21.9)
+        if (M > 32 && wide * z >= 150 && wide * z <= 256)
+            offer(Fp6Rows::wide, z, M <= 48 ? 8.6 + 0.057 * (m - 48.0) + 0.28 * p + 0.16 * z + 0.067 * mb : 10.3 + 0.39 * p + 0.15 * z + 0.065 * mb);
     }
     return best;
 }

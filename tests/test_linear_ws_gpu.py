@@ -215,9 +215,9 @@ def test_fp6_workspace_linear(N, K, M, parts, ebits, mbits):
 # last row counts of its kernels, a shorter last part, more workgroups than CUs, row blocks that fill neither four nor eight
 @pytest.mark.parametrize("ebits,mbits", [(3, 2), (2, 3)])
 @pytest.mark.parametrize("N,K,M,parts", [
-    (5120, 13824, 4, 3), (5120, 13824, 16, 3), (5120, 13824, 17, 3), (5120, 13824, 32, 3), (5120, 13824, 33, 5), (5120, 13824, 48, 5), (5120, 13824, 49, 5),
-    (5120, 13824, 64, 5), (10240, 8192, 16, 3), (4096, 14336, 48, 6), (4096, 4096, 40, 4), (1024, 14336, 30, 8), (1024, 14336, 48, 8), (1024, 14336, 64, 8),
-    (2064, 16384, 16, 7), (2064, 16384, 30, 7), (2064, 16384, 64, 7), (5008, 13824, 24, 3), (5008, 13824, 60, 5)])
+    (5120, 13824, 4, 3), (5120, 13824, 16, 3), (5120, 13824, 17, 3), (5120, 13824, 32, 3), (5120, 13824, 33, 6), (5120, 13824, 48, 6), (5120, 13824, 49, 6),
+    (5120, 13824, 64, 6), (10240, 8192, 16, 3), (4096, 14336, 48, 8), (4096, 4096, 40, 4), (1024, 14336, 30, 8), (1024, 14336, 48, 8), (1024, 14336, 64, 8),
+    (2064, 16384, 16, 7), (2064, 16384, 30, 7), (2064, 16384, 64, 7), (5008, 13824, 24, 3), (5008, 13824, 60, 6)])
 def test_fp6_rows_in_parts(N, K, M, parts, ebits, mbits):
     from ao_amd import _lib, ops
 
