@@ -1837,6 +1837,7 @@ extern "C" int ao_amd_fp6_linear_ws_parts(int64_t M, int64_t K, int64_t N) {
 extern "C" int ao_amd_fp6_linear_ws(const void* x_f16, int64_t M, int64_t K, const void* weights_native, const void* scale_f16,
                                     int64_t N, int ebits, int mbits, void* out_f16, void* workspace, int64_t workspace_bytes,
                                     void* stream) {
+    AO_REQUIRE(N > 0 && N % 16 == 0, "out_features must be a positive multiple of 16, got %lld", (long long)N);   // (the plans below count row blocks)
     const Fp6Rows rows = fp6_rows_plan(M, K, N);
     const int z = rows.kind != Fp6Rows::none ? rows.parts : fp6_ws_parts(M, K, N);
     if (z <= 1)

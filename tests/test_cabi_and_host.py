@@ -48,6 +48,16 @@ def test_argument_errors_without_launch(cabi):
     assert L.ao_amd_choose_qparams_affine(None, 0, 4, 4, 4, 1, 4, 1, 0, 15, -1.0, 1, 0, 0, 0, None, None, None) != 0
 
 
+@pytest.mark.parametrize("M,K", [(4, 13824), (12, 14336), (24, 5760), (40, 5120), (64, 16384), (16, 14336), (100, 4096)])
+@pytest.mark.parametrize("N", [0, -16, -64, -8192])
+def test_fp6_workspace_linear_refuses_no_columns(cabi, M, K, N):
+    """Whatever way of splitting K the row count asks for, the width is looked at first: nothing is launched with a grid of none."""
+    L, p = cabi.lib(), 4096   # (an aligned address that nothing reads)
+    for ws, room in ((p, 1 << 40), (None, 0)):
+        assert L.ao_amd_fp6_linear_ws(p, M, K, p, p, N, 3, 2, p, ws, room, None) != 0
+        assert b"out_features must be a positive multiple of 16" in L.ao_amd_last_error(), L.ao_amd_last_error()
+
+
 def test_cpu_tensors_are_rejected():
     """There is no CPU fallback: a CPU tensor raises instead of silently computing somewhere else."""
     import ao_amd
