@@ -1355,7 +1355,12 @@ __global__ __launch_bounds__(256) void fp6_ws_finish_kernel(const float* __restr
     }
     const uint32_t lo = (uint32_t)f32_to_f16_bits(v.x) | ((uint32_t)f32_to_f16_bits(v.y) << 16);
     const uint32_t hi = (uint32_t)f32_to_f16_bits(v.z) | ((uint32_t)f32_to_f16_bits(v.w) << 16);
-    *reinterpret_cast<uint2*>(out + i) = uint2{lo, hi};
+    if ((((uintptr_t)out) & 7) == 0) {
+        *reinterpret_cast<uint2*>(out + i) = uint2{lo, hi};
+    } else {   // (any fp16 address is taken, as by the kernels that are not split)
+        out[i] = (uint16_t)lo; out[i + 1] = (uint16_t)(lo >> 16);
+        out[i + 2] = (uint16_t)hi; out[i + 3] = (uint16_t)(hi >> 16);
+    }
 }
 
 static int check_fp6_format(int ebits, int mbits) {

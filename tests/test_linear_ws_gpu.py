@@ -244,6 +244,31 @@ def test_fp6_rows_in_parts(N, K, M, parts, ebits, mbits):
     assert torch.equal(ops.fp6_linear_native(ebits, mbits, xh.cuda(), native, scale), w[:, ks.cuda()].t().contiguous())
 
 
+# outputs that begin at any fp16 element: every way of splitting K, and one row count of each that is not split, in the middle of a larger buffer
+@pytest.mark.parametrize("N,K,M", [(5120, 13824, 4), (5120, 13824, 12), (5120, 13824, 24), (5120, 13824, 48), (1024, 14336, 64), (4096, 4096, 8)])
+@pytest.mark.parametrize("at", [1, 2, 3])
+def test_fp6_output_at_any_element(N, K, M, at):
+    from ao_amd import _lib, ops
+
+    print(f"case fp6 output at {at} N={N} K={K} M={M}", flush=True)
+    L, need = _lib.lib(), ctypes.c_int64(-1)
+    data, scale = ops.fp6_quantize_pack((torch.randn(N, K, generator=torch.Generator().manual_seed(N)) * 0.02).half().cuda(), 3, 2)
+    native = ops.fp6_repack(data, 6)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).half().cuda()
+    _lib.check(L.ao_amd_fp6_linear_ws_bytes(M, K, N, ctypes.byref(need)))
+    ws = _empty_ws(need.value)
+
+    def run(out):
+        _lib.check(L.ao_amd_fp6_linear_ws(x.data_ptr(), M, K, native.data_ptr(), scale.data_ptr(), N, 3, 2, out.data_ptr(), ws.data_ptr(), need.value,
+                                          torch.cuda.current_stream().cuda_stream))
+
+    want, buf = torch.empty(M * N, dtype=torch.float16, device="cuda"), torch.full((M * N + 8,), 7.0, dtype=torch.float16, device="cuda")
+    run(want)
+    run(buf[at:])
+    assert torch.equal(buf[at:at + M * N], want)   # the same sums, stored in other pieces
+    assert bool((buf[:at] == 7.0).all()) and bool((buf[at + M * N:] == 7.0).all())
+
+
 def _empty_ws(nbytes):
     return torch.empty(max(nbytes, 16), dtype=torch.uint8, device="cuda")
 
