@@ -1843,14 +1843,16 @@ extern "C" int ao_amd_fp6_linear_ws(const void* x_f16, int64_t M, int64_t K, con
                                     int64_t N, int ebits, int mbits, void* out_f16, void* workspace, int64_t workspace_bytes,
                                     void* stream) {
     AO_REQUIRE(N > 0 && N % 16 == 0, "out_features must be a positive multiple of 16, got %lld", (long long)N);   // (the plans below count row blocks)
-    const Fp6Rows rows = fp6_rows_plan(M, K, N);
+    Fp6Rows rows = fp6_rows_plan(M, K, N);
+    const bool aligned = workspace && (((uintptr_t)workspace) & 15) == 0;
+    // (a call without that room takes the way of one that needs less or none, below 16 rows always none)
+    if (rows.kind != Fp6Rows::none && !(aligned && workspace_bytes >= rows.parts * M * N * (int64_t)sizeof(float))) rows.kind = Fp6Rows::none;
     const int z = rows.kind != Fp6Rows::none ? rows.parts : fp6_ws_parts(M, K, N);
     if (z <= 1)
         return fp6_linear_dispatch(x_f16, M, K, weights_native, scale_f16, N, ebits, mbits, nullptr, nullptr, out_f16, stream);
     const int64_t need = (int64_t)z * M * N * (int64_t)sizeof(float);
-    AO_REQUIRE(workspace && workspace_bytes >= need && (((uintptr_t)workspace) & 15) == 0,
-               "16-byte aligned workspace of %lld bytes needed (ao_amd_fp6_linear_ws_bytes), got %lld", (long long)need,
-               (long long)workspace_bytes);
+    AO_REQUIRE(aligned && workspace_bytes >= need, "16-byte aligned workspace of %lld bytes needed (ao_amd_fp6_linear_ws_bytes), got %lld",
+               (long long)need, (long long)workspace_bytes);
     if (rows.kind == Fp6Rows::none)
         return fp6_linear_dispatch(x_f16, M, K, weights_native, scale_f16, N, ebits, mbits, nullptr, nullptr, out_f16, stream, nullptr,
                                    0.f, nullptr, nullptr, nullptr, 0, z, (float*)workspace);

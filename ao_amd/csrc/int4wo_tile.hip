@@ -208,13 +208,14 @@ struct Int4Auto {
     int stream_parts;     // K parts of the streaming kernel with four row blocks, 1: not split
     int64_t copy, parts;  // bytes
 };
-static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t N, int64_t g, int y_dtype, Int4Auto* r) {
+// room: the workspace that the call has.  Up to 64 rows a call without room for the K parts takes the way of one that needs less or none.
+static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t N, int64_t g, int y_dtype, int64_t room, Int4Auto* r) {
     *r = Int4Auto{false, false, 0, 1, 0, 0};
     const bool aligned = (ldx & 7) == 0 && (((uintptr_t)x) & 15) == 0;
     if (M > 32 && y_dtype == AO_BF16 && aligned && 256 * ldx * 2 < ((int64_t)1 << 32)) {
         int64_t need = -1;
         if (int rc = ao_amd_int4wo_linear_tiled_bytes(M, K, N, g, &need)) return rc;
-        if (need >= 0) {
+        if (need >= 0 && (M > 64 || need <= room)) {
             r->tiled = true;
             r->parts = need;
             return 0;
@@ -235,7 +236,8 @@ static int int4wo_auto(const void* x, int64_t M, int64_t K, int64_t ldx, int64_t
     r->stream_parts = (K == Kp && aligned) || r->Kp ? int4wo_stream_parts(M, r->as_is ? K : Kp, N, g) : 1;
     if (r->stream_parts > 1) {
         r->parts = r->stream_parts * M * N * (int64_t)sizeof(float);
-        return 0;
+        if (r->copy + r->parts <= room) return 0;
+        r->stream_parts = 1;
     }
     return ao_amd_int4wo_linear_ws_bytes(M, r->Kp ? Kp : K, N, g, &r->parts);
 }
@@ -322,7 +324,7 @@ extern "C" int ao_amd_int4wo_linear_auto_bytes(const void* x_bf16, int64_t M, in
     AO_REQUIRE(bytes, "null pointer argument");
     AO_REQUIRE(M >= 0 && K > 0 && N > 0, "need M >= 0 and positive K, N");
     Int4Auto r;
-    if (int rc = int4wo_auto(x_bf16, M, K, ldx, N, g, y_dtype, &r)) return rc;
+    if (int rc = int4wo_auto(x_bf16, M, K, ldx, N, g, y_dtype, INT64_MAX, &r)) return rc;
     *bytes = r.copy + r.parts;
     return 0;
 }
@@ -334,8 +336,9 @@ extern "C" int ao_amd_int4wo_linear_auto(const void* x_bf16, int64_t M, int64_t 
     AO_REQUIRE(ldx >= K && ldy >= N, "row strides (ldx=%lld, ldy=%lld) smaller than the rows (K=%lld, N=%lld)", (long long)ldx, (long long)ldy,
                (long long)K, (long long)N);
     Int4Auto r;
-    if (int rc = int4wo_auto(x_bf16, M, K, ldx, N, g, y_dtype, &r)) return rc;
-    AO_REQUIRE(r.copy + r.parts == 0 || (workspace && workspace_bytes >= r.copy + r.parts && (((uintptr_t)workspace) & 15) == 0),
+    const int64_t room = workspace && (((uintptr_t)workspace) & 15) == 0 ? workspace_bytes : 0;
+    if (int rc = int4wo_auto(x_bf16, M, K, ldx, N, g, y_dtype, room, &r)) return rc;
+    AO_REQUIRE(r.copy + r.parts <= (room > 0 ? room : 0),
                "16-byte aligned workspace of %lld bytes needed (ao_amd_int4wo_linear_auto_bytes), got %lld", (long long)(r.copy + r.parts),
                (long long)workspace_bytes);
     if (r.tiled)

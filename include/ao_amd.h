@@ -173,7 +173,8 @@ int ao_amd_int4wo_linear_tiled(const void* x_bf16, int64_t M, int64_t K, int64_t
                                int64_t workspace_bytes, void* stream);
 /* The linear on whichever of the routes above is the fastest for the shape and for the alignment of the rows: one call for the
  * workspace (x is not read), one for the product.  The workspace holds the K parts and, where the rows are not 16-byte aligned or end
- * before the packed width and it pays, their copy; the second call needs all of it. */
+ * before the packed width and it pays, their copy; the second call needs all of it (up to 64 rows one with less takes, where there
+ * is one, a route that needs less or none). */
 int ao_amd_int4wo_linear_auto_bytes(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, int64_t N, int64_t g, int y_dtype,
                                     int64_t* bytes);
 int ao_amd_int4wo_linear_auto(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* packed, const void* qparams,
@@ -429,11 +430,13 @@ int ao_amd_fp6_repack(const void* tc, int64_t N, int64_t K, int nbits, void* nat
 int ao_amd_fp6_linear(const void* x_f16, int64_t M, int64_t K, const void* weights_native, const void* scale_f16,
                       int64_t N, int ebits, int mbits, void* out_f16, void* stream);
 
-/* ao_amd_fp6_linear with a caller-owned workspace (device memory, 16-byte aligned): for batches of 16 to 256 rows on
- * weights whose 32- / 64-row tiles leave most CUs idle (4096-row weights), the K range is split over 2 or 4 groups of
- * workgroups, fp32 partial outputs [parts][M][N] go to the workspace and a second small launch adds them and rounds once
+/* ao_amd_fp6_linear with a caller-owned workspace (device memory, 16-byte aligned): for batches of 4 to 256 rows on
+ * weights whose row blocks or tiles leave CUs idle (fewer than 768 row blocks up to 64 rows), the K range is split over 2 to 8
+ * groups of workgroups (four row blocks a workgroup, or tiles of 32, 48 or 64 rows and 64 or 128 columns; 2 or 4 groups beyond
+ * 64 rows), fp32 partial outputs [parts][M][N] go to the workspace and a second small launch adds them and rounds once
  * to fp16.  ao_amd_fp6_linear_ws_bytes gives the size for a shape (0 where the split is not used: the call is then
- * ao_amd_fp6_linear itself and `workspace` may be NULL); ao_amd_fp6_linear_ws_parts the number of parts.  Same product as
+ * ao_amd_fp6_linear itself and `workspace` may be NULL); ao_amd_fp6_linear_ws_parts the number of parts.  Up to 64 rows a call
+ * with less room takes a way that needs less: below 16 rows none, from there on what 2 or 4 groups need.  Same product as
  * torchao::quant_llm_linear (torchao/csrc/cuda/fp6_llm/fp6_linear.cu:139-200); it stands where the reference's operator
  * takes `splitK` and allocates its [splitK, M, N] fp32 reduction workspace (fp6_linear.cu:104-111, 167-168,
  * SplitK_Reduction in kernel_reduction.cuh:44), with the part count chosen by the library instead of the caller.

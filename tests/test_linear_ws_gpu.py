@@ -269,6 +269,43 @@ def test_fp6_output_at_any_element(N, K, M, at):
     assert bool((buf[:at] == 7.0).all()) and bool((buf[at + M * N:] == 7.0).all())
 
 
+# Calls with less workspace than the query says, down to what the way needs that they then take (none below 16 rows): int4 in streamed parts, in streamed parts
+# of rows that are copied first, and on tiles; FP6 on four row blocks and on tiles.  With less than that a call is refused.
+@pytest.mark.parametrize("fmt,N,K,M,less", [
+    ("int4", 5120, 13824, 10, 0), ("int4", 5120, 13768, 14, 0), ("int4", 2048, 16384, 40, 0), ("int4", 5120, 13824, 24, 2), ("int4", 5120, 13824, 48, 2),
+    ("fp6", 5120, 13824, 10, 0), ("fp6", 1024, 14336, 6, 0), ("fp6", 5120, 13824, 24, 2), ("fp6", 2064, 16384, 60, 4)])
+def test_few_rows_with_less_workspace(fmt, N, K, M, less):
+    from ao_amd import _lib, ops
+
+    print(f"case less workspace {fmt} N={N} K={K} M={M} less={less}", flush=True)
+    L, need, g = _lib.lib(), ctypes.c_int64(-1), 128
+    st = torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator().manual_seed(M + N)
+    if fmt == "int4":
+        packed, qp, w = _setup(N, K, g, seed=N + K)
+        x, w = torch.randn(M, K, generator=gen).bfloat16().cuda(), w.float()
+        query = lambda: L.ao_amd_int4wo_linear_auto_bytes(x.data_ptr(), M, K, K, N, g, _lib.BF16, ctypes.byref(need))
+        call = lambda y, ws, n: L.ao_amd_int4wo_linear_auto(x.data_ptr(), M, K, K, packed.data_ptr(), qp.data_ptr(), N, g, None, y.data_ptr(), _lib.BF16, N, ws, n, st)
+    else:
+        data, scale = ops.fp6_quantize_pack((torch.randn((N + 63) // 64 * 64, K, generator=gen) * 0.02).half().cuda(), 3, 2)
+        native, w = ops.fp6_repack(data, 6), ops.fp6_dequantize(data, scale, 3, 2)[:N].half().float()
+        x = torch.randn(M, K, generator=gen).half().cuda()
+        query = lambda: L.ao_amd_fp6_linear_ws_bytes(M, K, N, ctypes.byref(need))
+        call = lambda y, ws, n: L.ao_amd_fp6_linear_ws(x.data_ptr(), M, K, native.data_ptr(), scale.data_ptr(), N, 3, 2, y.data_ptr(), ws, n, st)
+    _lib.check(query())
+    copy = 2 * M * (-(-K // g) * g) if fmt == "int4" and K % g else 0
+    room = copy + 4 * less * M * N
+    assert need.value > room
+    ref = x.float() @ w.t()
+    ws = _empty_ws(need.value)
+    for ptr, n in ((ws.data_ptr(), need.value), (ws.data_ptr(), need.value - 16), (ws.data_ptr() if room else None, room)):
+        y = torch.full((M, N), float("nan"), device="cuda").to(x.dtype)
+        _lib.check(call(y, ptr, n))
+        assert float((y.float() - ref.to(x.dtype).float()).norm() / ref.norm()) <= 1e-3   # one rounding of fp32 sums in another order, as in the tests above
+    if room:
+        assert call(y, ws.data_ptr(), room - 16) != 0 and b"workspace" in L.ao_amd_last_error()
+
+
 def _empty_ws(nbytes):
     return torch.empty(max(nbytes, 16), dtype=torch.uint8, device="cuda")
 
