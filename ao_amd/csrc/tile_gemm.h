@@ -307,37 +307,39 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void tile_gemm_kernel(const Tile
         }
 }
 
-// Adds the K parts of a tile_gemm_kernel and finishes as that kernel does: 4 columns a thread.
-template <class F>
+// Adds the K parts of a tile_gemm_kernel and finishes as that kernel does: W columns a thread, 4 or, where rows of sums are not 16-byte aligned, 1.
+// (Latency bounds it.  Four columns a thread of such rows, one load after the other under a condition, cost 2 to 4 us more, which the estimates of K parts do not
+// have: int8 1093 x 6144 at 10 rows in eight parts 12.5 -> 9.9 us, 4098 x 14336 at 16 rows 24.3 -> 20.9; int4 695 x 4416 at 52 rows 14.2 -> 11.5.)
+template <class F, int W>
 __global__ __launch_bounds__(256) void tile_finish_kernel(const TileGemmArgs a, int nparts) {
-    const int64_t per_row = (a.N + 3) / 4, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t m = i / per_row, n = (i - m * per_row) * 4;
+    const int64_t per_row = a.N / W, i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t m = i / per_row, n = (i - m * per_row) * W;
     if (m >= a.M) return;
-    const bool quad = (a.N & 3) == 0;
-    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+    float sum[W];
+#pragma unroll
+    for (int v = 0; v < W; ++v) sum[v] = 0.f;
     for (int p = 0; p < nparts; ++p) {
         const float* src = a.parts + ((int64_t)p * a.M + m) * a.N + n;
-        if (quad) {
+        if constexpr (W == 4) {
             const float4 v = *(const float4*)src;
             sum[0] += v.x; sum[1] += v.y; sum[2] += v.z; sum[3] += v.w;
         } else {
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                if (n + v < a.N) sum[v] += src[v];
+            sum[0] += src[0];
         }
     }
     const typename F::Cols cols = F::columns(a, n);
-    uint16_t o[4];
+    uint16_t o[W];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) o[v] = F::finish(sum[v], cols, v);
+    for (int v = 0; v < W; ++v) o[v] = F::finish(sum[v], cols, v);
     uint16_t* dst = a.y + m * a.ldy + n;
-    if (quad && (a.ldy & 3) == 0 && ((uintptr_t)a.y & 7) == 0) {
-        *(uint2*)dst = make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
-    } else {
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            if (n + v < a.N) dst[v] = o[v];
+    if constexpr (W == 4) {
+        if ((a.ldy & 3) == 0 && ((uintptr_t)a.y & 7) == 0) {
+            *(uint2*)dst = make_uint2(o[0] | ((uint32_t)o[1] << 16), o[2] | ((uint32_t)o[3] << 16));
+            return;
+        }
     }
+#pragma unroll
+    for (int v = 0; v < W; ++v) dst[v] = o[v];
 }
 
 // Tile shape and K parts for M x N x K: the cheapest by a measured model.  A shape costs `one` us for a wave of workgroups
@@ -418,8 +420,10 @@ void tile_launch(const TileGemmArgs& a, hipStream_t st) {
 template <class F>
 void tile_finish(const TileGemmArgs& a, int parts, hipStream_t st) {
     if (parts == 1) return;
-    const int64_t n = a.M * ((a.N + 3) / 4);
-    hipLaunchKernelGGL(tile_finish_kernel<F>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, parts);
+    const bool quads = a.N % 4 == 0;
+    const dim3 grid((unsigned)((a.M * (quads ? a.N / 4 : a.N) + 255) / 256)), block(256);
+    if (quads) hipLaunchKernelGGL((tile_finish_kernel<F, 4>), grid, block, 0, st, a, parts);
+    else hipLaunchKernelGGL((tile_finish_kernel<F, 1>), grid, block, 0, st, a, parts);
 }
 
 }  // namespace ao

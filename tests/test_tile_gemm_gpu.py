@@ -436,3 +436,51 @@ def test_parts_that_are_no_power_of_two(fmt, M, N, K, plan):
         _int4_tiles(M, N, K, 64)
     else:
         _fp6_tiles(M, N, K, 3, 2)
+
+
+# Sums of K parts whose rows are 16-byte aligned (a multiple of four columns: four a thread add them) or not (one a thread), stored to rows of any stride:
+# streamed row blocks of int8 (up to 16 rows) and of int4 (up to 32), tiles of both.  Activations and int8 weights are views of wider rows with NaN or 127 behind
+# their ends; what lies between the rows of the output stays.
+@pytest.mark.parametrize("fmt,M,N,K,pad_y", [
+    ("int8", 11, 2301, 14336, 0), ("int8", 16, 2302, 14336, 3), ("int8", 9, 2303, 14336, 1), ("int8", 13, 2304, 14336, 1), ("int8", 12, 2304, 14336, 4),
+    ("int8", 40, 1021, 14336, 2), ("int8", 70, 1022, 8192, 0), ("int8", 24, 4100, 14336, 5), ("int8", 65, 513, 8192, 0),
+    ("int4", 40, 1021, 16384, 2), ("int4", 64, 2050, 14336, 1), ("int4", 47, 1028, 14336, 3), ("int4", 12, 5120, 13824, 5), ("int4", 30, 5124, 13824, 4),
+    ("int4", 13, 5000, 8000, 1)])
+def test_sums_of_parts_in_rows_of_any_stride(fmt, M, N, K, pad_y):
+    from ao_amd import _lib, ops
+
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    L, need, st = _lib.lib(), ctypes.c_int64(-1), torch.cuda.current_stream().cuda_stream
+    rows = torch.full((M, K + 24), float("nan"), device="cuda").bfloat16()
+    x = rows[:, :K]
+    x.copy_(torch.randn(M, K, device="cuda", generator=g))
+    x[0, 5], x[M // 2, K - 7] = float("inf"), float("-inf")   # in the first and in the last part of K
+    if M > 3:
+        x[M - 1, K // 2] = float("nan")
+    b = torch.randn(N, device="cuda", generator=g).bfloat16()
+    y = torch.full((M, N + pad_y), 7.0, device="cuda").bfloat16()
+    if fmt == "int8":
+        w = torch.full((N, K + 32), 127, device="cuda", dtype=torch.int8)[:, :K]
+        w.copy_(torch.randint(-128, 128, (N, K), device="cuda", dtype=torch.int8, generator=g))
+        s = (torch.rand(N, device="cuda", generator=g) * 0.01 + 0.001).bfloat16()
+        _lib.check(L.ao_amd_int8wo_linear_ws_bytes(M, K, N, ctypes.byref(need)))
+        ws = torch.full((need.value // 4,), float("nan"), device="cuda")
+        _lib.check(L.ao_amd_int8wo_linear_ws(x.data_ptr(), M, K, K + 24, w.data_ptr(), K + 32, s.data_ptr(), N, b.data_ptr(), y.data_ptr(), _lib.BF16, N + pad_y,
+                                             ws.data_ptr(), need.value, st))
+        scaled = ((x.float() @ w.float().t()).bfloat16().float() * s.float()).bfloat16()
+        want = (scaled.float() + b.float()).bfloat16()
+    else:
+        packed, qp = ops.int4wo_quantize_pack((torch.randn(N, K, device="cuda", generator=g) * 0.02).bfloat16(), 64)
+        _lib.check(L.ao_amd_int4wo_linear_auto_bytes(x.data_ptr(), M, K, K + 24, N, 64, _lib.BF16, ctypes.byref(need)))
+        ws = torch.full((need.value // 4,), float("nan"), device="cuda")
+        _lib.check(L.ao_amd_int4wo_linear_auto(x.data_ptr(), M, K, K + 24, packed.data_ptr(), qp.data_ptr(), N, 64, b.data_ptr(), y.data_ptr(), _lib.BF16, N + pad_y,
+                                               ws.data_ptr(), need.value, st))
+        want = (x.float() @ ops.int4wo_dequantize(packed, qp, N, K, 64).float().t() + b.float()).bfloat16()
+    assert need.value >= 2 * 4 * M * N   # (in parts)
+    assert bool((y[:, N:] == 7.0).all())
+    y = y[:, :N]
+    assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.isinf(), want.isinf()) and torch.equal(y[y.isinf()], want[want.isinf()])
+    ok = want.isfinite()
+    # the bounds of _run, for the rows without a special value (up to 16384 products a sum)
+    rel = ((y[ok].float() - want[ok].float()).norm() / want[ok].float().norm()).item()
+    assert rel <= 1e-3 and (y[ok] != want[ok]).float().mean() <= 0.01, rel
