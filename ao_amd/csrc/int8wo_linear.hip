@@ -590,8 +590,10 @@ static bool tiled(int64_t M, int64_t N, int64_t K, bool workspace) {
 // tiles: 5120 x 13824 at 2 / 8 / 16 rows 23.8 / 20.3 / 23.1, 33.3 / 21.8 / 23.6, 42.4 / 23.9 / 24.0; 4096 x 14336 at 4 / 8 / 16 rows 15.7 / 18.2 / 22.0, 19.5 / 18.7 / 22.1, 24.4 /
 // 20.1 / 22.5; 2048 x 16384 at 4 / 12 rows 15.4 / 14.3 / 16.9, 22.7 / 15.1 / 17.7; 8192 x 8192 at 12 rows 23.7 / 20.8 / 23.9; 5120 x 5120 at 8 rows 15.3 / 13.4 / 15.2;
 // 4096 x 11008 at 12 rows 17.7 / 17.0 / 20.5; 1024 x 14336 at 8 rows 18.4 / 13.6 / 13.8; 10240 x 8192 at 8 / 16 rows 29.3 / - / 25.2, 36.8 / - / 25.8; 4096 x 4096 at 16
-// rows 8.8 / 10.6 / 11.6; streaming / tiles at 20 rows: 1024 x 14336 22.7 / 13.9, 4096 x 4096 12.9 / 11.9, 1024 x 4096 8.5 / 11.5.  (Weight and row count each had a line of their own before, which sent 5120 x 13824 at 8 rows and 10240 x 8192 at 16 to streaming and 4096 x
-// 11008 at 12 to the tiles.)  The estimates are within some 6 % of these calls.
+// rows 8.8 / 10.6 / 11.6; streaming / tiles at 20 rows: 1024 x 14336 22.7 / 13.9, 4096 x 4096 12.9 / 11.9, 1024 x 4096 8.5 / 11.5, at 17 rows 2064 x 3584 8.4 / 10.8.  (Weight and row count each had
+// a line of their own before, which sent 5120 x 13824 at 8 rows and 10240 x 8192 at 16 to streaming and 4096 x 11008 at 12 to the tiles.)
+// 7135 calls of 2 to 32 rows, timed in every way with weights in turn (a quarter on weights of models, the others 256 to 12280 columns, 1024 to 29440 in_features), take 0.954 of
+// the time that those lines gave and 1.021 of the best way's; fifteen take 5 % more than by the lines, none 8 %.
 struct Int8Rows {
     enum Kind { other, streaming, four_parts, tiles };   // other: not one of these calls
     int kind, parts;
@@ -605,9 +607,10 @@ static Int8Rows int8_rows_plan(int64_t M, int64_t K, int64_t N) {
     const double m = (double)M, kb = (double)KB;
     // (rows that fit LDS are staged there, with one workgroup to a CU)
     const bool staged = RB <= 256 && KB >= 64 && M * K * 2 <= 140 * 1024;
-    const double streaming = 4.0 + (double)((RB * ((M + 15) / 16) + 255) / 256) * kb * ((staged ? 0.07 : 0.09) + 0.0055 * (M < 16 ? m : 16.0));
+    const double streaming = 4.0 + (double)((RB * ((M + 15) / 16) + 255) / 256) * kb * ((staged ? 0.07 : 0.09) + 0.0055 * (M <= 16 ? m : 0.5 * m));
+    const bool large = N * K >= 110000000;
     Int8Rows best{Int8Rows::streaming, 1};
-    double us = (M <= 16 ? 0.96 : 1.0) * streaming;
+    double us = (M > 16 || large ? 1.0 : 0.96) * streaming;
     for (int z = 2; M <= 16 && z <= 8; ++z) {
         const int64_t per = (KB + z - 1) / z;
         if (per < 4 || (z - 1) * per >= KB || groups * z > 256) continue;
@@ -619,8 +622,9 @@ static Int8Rows int8_rows_plan(int64_t M, int64_t K, int64_t N) {
     }
     if (streaming > 12.0) {   // (no tiles take less)
         const TilePlan p = int8wo_gemm_plan(M, N, K, 8);
-        // (their estimates are of 33 and more rows and 10 % low at the fewest)
-        if (p.us < (M <= 16 ? 0.9 : 1.0) * us) best = Int8Rows{Int8Rows::tiles, p.parts};
+        // (estimates of 33 and more rows: some 5 to 10 % low up to 16, 10 % high beyond.  Weights from 110 MB on come from memory as fast as it gives them, which all three
+        // estimates miss by as much: with the leads that smaller ones need 8192 x 28672 at 3 rows streamed in 56.4 us, 50.0 in tiles)
+        if (p.us < (M > 16 ? 1.15 : large ? 1.0 : 0.92) * us) best = Int8Rows{Int8Rows::tiles, p.parts};
     }
     return best;
 }

@@ -58,6 +58,18 @@ def test_fp6_workspace_linear_refuses_no_columns(cabi, M, K, N):
         assert b"out_features must be a positive multiple of 16" in L.ao_amd_last_error(), L.ao_amd_last_error()
 
 
+@pytest.mark.parametrize("M,N,K,plan", [
+    # large weights, timed streaming (or in two parts) / in tiles: 56.4 / 50.0, 56.0 / 48.4, 47.0 / 42.2 us
+    (3, 8192, 28672, "tile 64x128 parts=4"), (5, 11008, 17408, "tile 64x128 parts=2"), (4, 8192, 22016, "tile 64x128 parts=4"),
+    # a second chunk of one row costs what one row costs: 8.4 / 10.8
+    (17, 2064, 3584, "streaming"),
+    (4, 4104, 4096, "streaming")])
+def test_int8_plan_of_few_rows(cabi, M, N, K, plan):
+    out = ctypes.create_string_buffer(64)
+    cabi.check(cabi.lib().ao_amd_int8wo_linear_plan(M, K, N, out, 64))
+    assert out.value.decode() == plan
+
+
 def test_cpu_tensors_are_rejected():
     """There is no CPU fallback: a CPU tensor raises instead of silently computing somewhere else."""
     import ao_amd

@@ -87,13 +87,15 @@ def test_int8_tiles_bias_and_row_stride(case):
     _run(*case, bias=True, pad=72)
 
 
-@pytest.mark.parametrize("case,tiles", [
-    ((3, 4096, 14336), False), ((5, 4090, 14336), False), ((6, 2064, 11008), False), ((2, 4096, 28672), False),  # rows staged in 65 to 140 KB
-    ((6, 4096, 14336), False),                                                                                # just past that
-    ((3, 2048, 16512), True), ((9, 4104, 8320), True), ((8, 4104, 8320), False), ((9, 24592, 8192), True),
+@pytest.mark.parametrize("case,plan", [
+    ((3, 4096, 14336), "streaming"), ((5, 4090, 14336), "streaming"), ((6, 2064, 11008), "streaming"), ((2, 4096, 28672), "streaming"),  # rows staged in 65 to 140 KB
+    ((6, 4096, 14336), "streaming"),                                                                                                     # just past that
+    ((3, 2048, 16512), "streaming parts=8"), ((9, 4104, 8320), "streaming parts=3"), ((8, 4104, 8320), "streaming"),
+    ((9, 24592, 8192), "tile 64x128 parts=1"), ((8, 10240, 8192), "tile 64x128 parts=3"), ((12, 4104, 14336), "tile 64x128 parts=7"),
+    ((3, 8192, 28672), "tile 64x128 parts=4"), ((5, 11010, 17408), "tile 64x128 parts=2"),
 ])
-def test_int8_few_rows(case, tiles):
-    assert (_plan(*case) != "streaming") == tiles
+def test_int8_few_rows(case, plan):
+    assert _plan(*case) == plan
     # the bound of _run holds here too: the sums are at most 3.5 times as long, and their order moves them by about
     # sqrt(K) 2^-24 of their size, 1e-5 at most, against the 2^-8 steps of the result
     _run(*case)
