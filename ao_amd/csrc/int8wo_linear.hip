@@ -592,8 +592,8 @@ static bool tiled(int64_t M, int64_t N, int64_t K, bool workspace) {
 // 4096 x 11008 at 12 rows 17.7 / 17.0 / 20.5; 1024 x 14336 at 8 rows 18.4 / 13.6 / 13.8; 10240 x 8192 at 8 / 16 rows 29.3 / - / 25.2, 36.8 / - / 25.8; 4096 x 4096 at 16
 // rows 8.8 / 10.6 / 11.6; streaming / tiles at 20 rows: 1024 x 14336 22.7 / 13.9, 4096 x 4096 12.9 / 11.9, 1024 x 4096 8.5 / 11.5, at 17 rows 2064 x 3584 8.4 / 10.8.  (Weight and row count each had
 // a line of their own before, which sent 5120 x 13824 at 8 rows and 10240 x 8192 at 16 to streaming and 4096 x 11008 at 12 to the tiles.)
-// 7135 calls of 2 to 32 rows, timed in every way with weights in turn (a quarter on weights of models, the others 256 to 12280 columns, 1024 to 29440 in_features), take 0.954 of
-// the time that those lines gave and 1.021 of the best way's; fifteen take 5 % more than by the lines, none 8 %.
+// 7135 calls of 2 to 32 rows, timed in every way with weights in turn (a quarter on weights of models, the others 256 to 12280 columns, 1024 to 29440 in_features), take 0.945 of
+// the time that those lines gave and 1.008 of the best way's; sixteen take 5 % more than by the lines, none 8 %.
 struct Int8Rows {
     enum Kind { other, streaming, four_parts, tiles };   // other: not one of these calls
     int kind, parts;
@@ -602,8 +602,6 @@ static Int8Rows int8_rows_plan(int64_t M, int64_t K, int64_t N) {
     static const bool forced = knob("AO_AMD_INT8_TILED") != nullptr;
     const int64_t KB = K / 128, RB = (N + 15) / 16, groups = (RB + 3) / 4;
     if (M < 2 || M > 32 || K % 128 != 0 || KB < 8 || groups >= 192 || forced) return Int8Rows{Int8Rows::other, 1};
-    // (row blocks that are no multiple of four keep their route up to 8 rows, which callers rely on: 4104 x 8320 at 8 rows takes 19.1 us and would take 15.7 in parts)
-    if (M <= 8 && RB % 4 != 0) return Int8Rows{Int8Rows::other, 1};
     const double m = (double)M, kb = (double)KB;
     // (rows that fit LDS are staged there, with one workgroup to a CU)
     const bool staged = RB <= 256 && KB >= 64 && M * K * 2 <= 140 * 1024;

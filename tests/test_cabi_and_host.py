@@ -63,7 +63,9 @@ def test_fp6_workspace_linear_refuses_no_columns(cabi, M, K, N):
     (3, 8192, 28672, "tile 64x128 parts=4"), (5, 11008, 17408, "tile 64x128 parts=2"), (4, 8192, 22016, "tile 64x128 parts=4"),
     # a second chunk of one row costs what one row costs: 8.4 / 10.8
     (17, 2064, 3584, "streaming"),
-    (4, 4104, 4096, "streaming")])
+    # row blocks that are no multiple of four are planned as their neighbours are: 33.1 us streaming, 21 in parts
+    (8, 5120, 13824, "streaming parts=3"), (8, 5104, 13824, "streaming parts=3"), (8, 5128, 13824, "streaming parts=3"), (2, 5128, 13824, "streaming parts=3"),
+    (8, 10248, 8192, "tile 64x128 parts=3"), (8, 4104, 8320, "streaming parts=3"), (4, 4104, 4096, "streaming")])
 def test_int8_plan_of_few_rows(cabi, M, N, K, plan):
     out = ctypes.create_string_buffer(64)
     cabi.check(cabi.lib().ao_amd_int8wo_linear_plan(M, K, N, out, 64))

@@ -375,7 +375,7 @@ def test_rows_that_are_far_apart():
 # 2 to 16 rows with K in parts: the first and last row counts, a shorter last part, row blocks that are no multiple of four and rows that end within one, a
 # bias, and the same call without a workspace
 @pytest.mark.parametrize("N,K,M,parts", [(5120, 13824, 2, 3), (5120, 13824, 16, 3), (4096, 14336, 11, 4), (2048, 16384, 7, 8), (1000, 14336, 16, 8),
-                                         (2069, 16256, 13, 7), (5160, 5120, 12, 3)])
+                                         (2069, 16256, 13, 7), (5160, 5120, 12, 3), (5128, 13824, 8, 3), (4104, 8320, 8, 3), (2069, 16256, 5, 7), (290, 28032, 8, 8)])
 def test_few_rows_in_parts(N, K, M, parts):
     import ctypes
 

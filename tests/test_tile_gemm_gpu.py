@@ -90,7 +90,7 @@ def test_int8_tiles_bias_and_row_stride(case):
 @pytest.mark.parametrize("case,plan", [
     ((3, 4096, 14336), "streaming"), ((5, 4090, 14336), "streaming"), ((6, 2064, 11008), "streaming"), ((2, 4096, 28672), "streaming"),  # rows staged in 65 to 140 KB
     ((6, 4096, 14336), "streaming"),                                                                                                     # just past that
-    ((3, 2048, 16512), "streaming parts=8"), ((9, 4104, 8320), "streaming parts=3"), ((8, 4104, 8320), "streaming"),
+    ((3, 2048, 16512), "streaming parts=8"), ((9, 4104, 8320), "streaming parts=3"), ((8, 4104, 8320), "streaming parts=3"), ((8, 5128, 13824), "streaming parts=3"),
     ((9, 24592, 8192), "tile 64x128 parts=1"), ((8, 10240, 8192), "tile 64x128 parts=3"), ((12, 4104, 14336), "tile 64x128 parts=7"),
     ((3, 8192, 28672), "tile 64x128 parts=4"), ((5, 11010, 17408), "tile 64x128 parts=2"),
 ])
