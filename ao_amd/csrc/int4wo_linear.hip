@@ -1535,18 +1535,19 @@ int ao::int4wo_stream_parts(int64_t M, int64_t K, int64_t N, int64_t g) {
     const int64_t KB = (K + 127) / 128, RB = Np / 16, groups = (RB + 3) / 4;
     if (groups >= 192 || KB < 8 || KB >= (1 << 21)) return 1;
     const double m = (double)M;
-    auto whole = [&]() {   // one row block a workgroup, 16 rows at a time
-        const int64_t chunks = RB * ((M + 15) / 16);
-        return 4.0 + (double)((chunks + 255) / 256) * (double)KB * (0.029 + 0.0061 * (M < 16 ? m : 16.0));
-    };
-    double other = whole();
+    // one row block a workgroup, 16 rows at a time
+    double other = 4.0 + (double)((RB * ((M + 15) / 16) + 255) / 256) * (double)KB * (0.029 + 0.0061 * (M < 16 ? m : 16.0));
+    int z0 = 1;
     if (M > 16) {
-        const int z = ws_parts(M, K, N, g);
-        if (z > 1) other = 7.4 + 0.33 * (double)((KB + z - 1) / z);
+        z0 = ws_parts(M, K, N, g);
+        if (z0 > 1) other = 7.4 + 0.33 * (double)((KB + z0 - 1) / z0);
         else if (groups >= 128) other = 4.0 + 0.33 * (double)KB;   // 32 x 64 tiles
     }
     int best = 1;
     double us = (M > 16 ? 0.88 : 0.97) * other;
+    // Where the second 16 rows begin beside the first and end behind them they cost what rows there are: a full round charged for them took 2512 x 3584 at 19 rows
+    // from 8.6 us into six parts, 9.9 (fitted to 253 calls of 17 to 32 rows, nine of ten within 15 %; with 3 % more the splits that gained stay)
+    if (M > 16 && z0 == 1 && RB <= 256 && 2 * RB > 256) us = fmin(us, 4.0 + 1.03 * (double)KB * ((double)RB / 256.0 * (0.104 + 0.003 * m) + 0.0034 * m));
     for (int z = 2; z <= 8; ++z) {
         const int64_t per = (KB + z - 1) / z, wgs = groups * z;
         if (per < 4 || (z - 1) * per >= KB || wgs > (M > 16 ? 256 : 512)) continue;   // (105 registers a lane up to 16 rows: two workgroups share a CU)

@@ -72,6 +72,16 @@ def test_int8_plan_of_few_rows(cabi, M, N, K, plan):
     assert out.value.decode() == plan
 
 
+@pytest.mark.parametrize("M,N,K,group,parts", [
+    # one row block a workgroup / in parts, us: 8.6 / 9.9, 8.9 / 10.1, 8.9 / 9.8, 8.0 / 9.4
+    (19, 2512, 3584, 128, 1), (21, 2352, 3584, 64, 1), (18, 2060, 4352, 32, 1), (17, 2352, 3456, 32, 1),
+    (20, 2828, 6784, 128, 5), (18, 6596, 3456, 128, 2), (20, 2048, 16384, 64, 8), (17, 5120, 13824, 128, 3), (16, 5120, 13824, 64, 3)])
+def test_int4_parts_of_17_to_32_rows(cabi, M, N, K, group, parts):
+    need = ctypes.c_int64(-1)
+    cabi.check(cabi.lib().ao_amd_int4wo_linear_auto_bytes(4096, M, K, K, N, group, cabi.BF16, ctypes.byref(need)))   # (an aligned address that nothing reads)
+    assert need.value == (4 * parts * M * N if parts > 1 else 0)
+
+
 def test_cpu_tensors_are_rejected():
     """There is no CPU fallback: a CPU tensor raises instead of silently computing somewhere else."""
     import ao_amd
