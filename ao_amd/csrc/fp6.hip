@@ -1776,7 +1776,9 @@ static Fp6Rows fp6_rows_plan(int64_t M, int64_t K, int64_t N) {
     } else if (M > 32) {
         other = 4.0 + 0.25 * kb * (double)((groups * 2 + 255) / 256);
     } else if (M > 16) {
-        other = 4.5 + 0.31 * kb;
+        // (4.5 us and 0.31 a tile for short rows of wide weights too sent these into parts: 4928 x 1536 at 21 rows 6.6 / 7.2 us, 4304 x 1792 at 23 rows 7.1 / 7.6, 5440 x 1920 at
+        // 27 rows 7.4 / 8.1; narrow ones, whose sums are few, gain by them: 1552 x 1920 at 25 rows 7.2 / 6.4)
+        other = groups >= 48 ? fmin(4.5 + 0.31 * kb, 3.15 + 0.36 * kb) : 4.5 + 0.31 * kb;
     } else {
         const int rbw = fp6_row_blocks_per_wave(M, RB, 1);
         const double per_tile = rbw == 1 ? (double)((RB + 255) / 256) * (0.043 + 0.0048 * m)

@@ -82,6 +82,13 @@ def test_int4_parts_of_17_to_32_rows(cabi, M, N, K, group, parts):
     assert need.value == (4 * parts * M * N if parts > 1 else 0)
 
 
+@pytest.mark.parametrize("M,N,K,parts", [
+    (21, 4928, 1536, 1), (23, 4304, 1792, 1), (27, 5440, 1920, 1), (18, 4160, 1792, 1), (24, 3648, 1664, 1),   # 6.6 / 7.2, 7.1 / 7.6, 7.4 / 8.1, 6.9 / 7.3, 6.7 / 7.1 us
+    (25, 1552, 1920, 4), (24, 5120, 5120, 3), (17, 5120, 13824, 3), (24, 2048, 16384, 8), (32, 10240, 4096, 1)])
+def test_fp6_parts_of_17_to_32_rows(cabi, M, N, K, parts):
+    assert cabi.lib().ao_amd_fp6_linear_ws_parts(M, K, N) == parts
+
+
 def test_cpu_tensors_are_rejected():
     """There is no CPU fallback: a CPU tensor raises instead of silently computing somewhere else."""
     import ao_amd
