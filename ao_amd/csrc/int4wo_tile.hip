@@ -176,7 +176,11 @@ static bool int4wo_tiled(int64_t M, int64_t N, int64_t K, int64_t g) {
     if (plan.shape >= kInt4Own && plan.parts == 1 && int4wo_plain_kernel(M, Kp, N, g, &kernel) &&
         kernel == (plan.shape == kInt4Own ? Int4Kernel::lds_256x128 : Int4Kernel::lds_256x256))
         return false;
-    return plan.us < (Kp == K ? 0.95 * other : other + 4.0);
+    // (sums whose rows are not 16-byte aligned are stored one by one, which the estimates of K parts do not have.  Up to 64 rows, us in the other kernels / tiled:
+    // 4481 x 3584 at 56 rows 12.7 / 14.1, 667 x 4416 at 39 rows 10.4 / 11.3, 4277 x 3584 at 59 rows 13.2 / 14.2)
+    const double single = M <= 64 && plan.parts > 1 && N % 4 != 0 ? 0.8 : 0.0;
+    // (rows that end early are copied for the others: 4 us, up to 64 rows 2.5.  3400 x 1472 at 38 rows 9.2 copied and streamed / 10.1 tiled, 912 x 4672 at 57 rows 11.4 / 12.2)
+    return plan.us + single < (Kp == K ? 0.95 * other : other + (M <= 64 ? 2.5 : 4.0));
 }
 
 // x [M, K] with row stride ldx -> y [M, Kp], zeros beyond K, 8 elements a thread: activations whose rows are not 16-byte aligned

@@ -89,6 +89,16 @@ def test_fp6_parts_of_17_to_32_rows(cabi, M, N, K, parts):
     assert cabi.lib().ao_amd_fp6_linear_ws_parts(M, K, N) == parts
 
 
+@pytest.mark.parametrize("M,N,K,tiled", [
+    (56, 4481, 3584, False), (39, 667, 4416, False), (59, 4277, 3584, False),   # 12.7 / 14.1, 10.4 / 11.3, 13.2 / 14.2 us
+    (38, 3400, 1472, False), (57, 912, 4672, False),   # rows that end within a tile of K: 9.2 / 10.1, 11.4 / 12.2
+    (56, 4480, 3584, True), (50, 8163, 5888, True), (40, 2049, 16384, True), (42, 1519, 576, True), (44, 7736, 1600, True)])
+def test_int4_tiles_up_to_64_rows(cabi, M, N, K, tiled):
+    need = ctypes.c_int64(-1)
+    cabi.check(cabi.lib().ao_amd_int4wo_linear_tiled_bytes(M, K, N, 64, ctypes.byref(need)))
+    assert (need.value >= 0) == tiled
+
+
 def test_cpu_tensors_are_rejected():
     """There is no CPU fallback: a CPU tensor raises instead of silently computing somewhere else."""
     import ao_amd
