@@ -1802,7 +1802,7 @@ static Fp6Rows fp6_rows_plan(int64_t M, int64_t K, int64_t N) {
         }
         // (short K that is split in four already gains by the 48-row tiles only)
         if (M > 32 && groups * z <= 256 && (z == z0 ? M <= 48 : z0 == 1 || KB >= 64))
-            offer(Fp6Rows::tiles, z, tiles(p, z) + (z0 == 1 ? 0.6 : 0.0));   // (5120 x 5120 at 48 rows in three parts 12.9, wide in six 12.7)
+            offer(Fp6Rows::tiles, z, tiles(p, z) + (z0 == 1 ? 0.6 : 0.0));   // (5120 x 5120 at 48 rows in three parts 12.9, wide in six 12.7: by this entry; ao_amd_fp6_linear_auto takes fp6_tile.hip's tiles, 12.9)
         // (a workgroup a CU: parts up to 256 workgroups shorten each, one more part queues.  us in 4 / 6 / 8 / 9 parts at 48 rows: 4096 x 14336 20.8 / 17.8 / 16.6 / 20.3,
         // 4096 x 11008 17.5 / 15.7 / 15.1 / 17.6; in 5 / 6 / 7: 5120 x 13824 19.5 / 18.5 / 23.6; in 3 / 4 / 5: 8192 x 8192 19.2 / 17.8 / 21.9)
         if (M > 32 && wide * z >= 150 && wide * z <= 256)

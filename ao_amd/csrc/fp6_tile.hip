@@ -97,7 +97,8 @@ static TilePlan fp6_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
     TilePartCost parts;
     parts.lead = 0.89;
     // (in powers of two / three or six parts: 5120 x 13824 at 96 / 128 / 256 rows 33.8 / 30.9, 40.7 / 33.0, 49.1 / 46.4; 10240 x 8192 at 40 / 77 / 113 rows 26.0 / 27.6, 30.3 /
-    // 33.1, 34.3 / 36.1; 9000 x 6144 and 5120 x 5120 level)
+    // 33.1, 34.3 / 36.1; 9000 x 6144 and 5120 x 5120 level.  The line is drawn between these weights: a part has to be long enough to pay for its sums, and where
+    // between 8192 and 13824 that begins was not measured)
     parts.uneven = K >= 10240;
     return tile_plan(kFp6Shapes, (int)(sizeof(kFp6Shapes) / sizeof(kFp6Shapes[0])), M, N, K, max_parts, parts);
 }
@@ -113,6 +114,10 @@ static TilePlan fp6_tile_plan(int64_t M, int64_t N, int64_t K, int max_parts) {
 // 46); below it only where that round is long and its workgroups leave room for two K parts (5120 x 5120 14.0 / 12.4, 14.1 / 13.7; 6400 x
 // 7168 19.2 / 16.7, 19.6 / 18.9; but 8192 x 4096 12.2 / 13.1 at 33 and 12.5 / 13.6 at 56 rows, 7168 x 6144 16.8 / 15.7, 16.9 / 17.7, 8192 x 7168 20.0 / 20.4,
 // 20.6 / 22.3).  Weights below 26 M were not measured there.
+// Those lines for 33 to 64 rows were drawn against unsplit 32 x 64 tiles.  The parts that ao_amd_fp6_linear_ws has since (fp6.hip: fp6_rows_plan) are ahead of the tiles on
+// most of these weights, but ao_amd_fp6_linear_auto asks here first and does not compare the two.  us tiled / in parts at 40 and 64 rows: 10240 x 8192 24.0 / 19.7, 26.6 / 24.0; 9216 x
+// 8192 23.7 / 19.3, 26.4 / 23.7; 6400 x 7168 17.1 / 15.1, 18.7 / 19.5; 5376 x 7168 16.8 / 14.1, 18.3 / 16.2; 12032 x 8192 24.6 / 23.6, 27.2 / 29.8; level: 5120 x 5120 12.5 / 12.8, 13.0 /
+// 14.1; 8448 x 4096 14.0 / 14.1, 15.5 / 16.7.
 // Where the others split K over workgroups (fp6.hip: fp6_ws_parts) they are kept but for 65 to 96 rows of weights from 50 M on (4096 x
 // 14336 at 64 / 66 / 96 rows 20.9 / 20.9, 31.0 / 22.2, 32.3 / 24.1; 4096 x 4096 at 66 rows 11.9 / 13.4).
 static bool fp6_tiled(int64_t M, int64_t N, int64_t K) {

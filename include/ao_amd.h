@@ -270,7 +270,8 @@ int ao_amd_int8wo_linear(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, 
  * computed (F.silu(self.w1(x)) * self.w3(x), FeedForward.forward, model.py:209-214).  bf16 output, no bias. */
 /* The same with a caller's fp32 workspace, which lets the library split K over workgroups where the shape leaves CUs idle:
  * ao_amd_int8wo_linear_ws_bytes gives the size (0: not used); too small or null, and K is not split. */
-/* ... and ao_amd_int8wo_linear_plan writes which kernel a shape runs ("streaming" or "tile <rows>x<columns> parts=<K parts>"). */
+/* ... and ao_amd_int8wo_linear_plan writes which kernel a shape runs ("streaming", "streaming parts=<K parts>" or
+ * "tile <rows>x<columns> parts=<K parts>"). */
 int ao_amd_int8wo_linear_plan(int64_t M, int64_t K, int64_t N, char* out, int64_t out_cap);
 int ao_amd_int8wo_linear_ws_bytes(int64_t M, int64_t K, int64_t N, int64_t* bytes);
 int ao_amd_int8wo_linear_ws(const void* x_bf16, int64_t M, int64_t K, int64_t ldx, const void* w_int8, int64_t ldw,
