@@ -592,8 +592,8 @@ static bool tiled(int64_t M, int64_t N, int64_t K, bool workspace) {
 // 4096 x 11008 at 12 rows 17.7 / 17.0 / 20.5; 1024 x 14336 at 8 rows 18.4 / 13.6 / 13.8; 10240 x 8192 at 8 / 16 rows 29.3 / - / 25.2, 36.8 / - / 25.8; 4096 x 4096 at 16
 // rows 8.8 / 10.6 / 11.6; streaming / tiles at 20 rows: 1024 x 14336 22.7 / 13.9, 4096 x 4096 12.9 / 11.9, 1024 x 4096 8.5 / 11.5, at 17 rows 2064 x 3584 8.4 / 10.8.  (Weight and row count each had
 // a line of their own before, which sent 5120 x 13824 at 8 rows and 10240 x 8192 at 16 to streaming and 4096 x 11008 at 12 to the tiles.)
-// 7135 calls of 2 to 32 rows, timed in every way with weights in turn (a quarter on weights of models, the others 256 to 12280 columns, 1024 to 29440 in_features), take 0.945 of
-// the time that those lines gave and 1.008 of the best way's; sixteen take 5 % more than by the lines, none 8 %.
+// 7135 calls of 2 to 32 rows, timed in every way with weights in turn (a quarter on weights of models, the others 256 to 12280 columns, 1024 to 29440 in_features), take 0.943 of
+// the time that those lines gave and 1.007 of the best way's; twenty-two take 5 % more than by the lines, two 8 %.
 struct Int8Rows {
     enum Kind { other, streaming, four_parts, tiles };   // other: not one of these calls
     int kind, parts;
@@ -605,10 +605,13 @@ static Int8Rows int8_rows_plan(int64_t M, int64_t K, int64_t N) {
     const double m = (double)M, kb = (double)KB;
     // (rows that fit LDS are staged there, with one workgroup to a CU)
     const bool staged = RB <= 256 && KB >= 64 && M * K * 2 <= 140 * 1024;
-    const double streaming = 4.0 + (double)((RB * ((M + 15) / 16) + 255) / 256) * kb * ((staged ? 0.07 : 0.09) + 0.0055 * (M <= 16 ? m : 0.5 * m));
-    const bool large = N * K >= 110000000;
+    const double streaming = 4.0 + (double)((RB * ((M + 15) / 16) + 255) / 256) * kb * ((staged ? 0.07 : 0.09) + 0.0055 * (M < 16 ? m : 16.0));
+    const bool large = N * K >= 120000000;
     Int8Rows best{Int8Rows::streaming, 1};
     double us = (M > 16 || large ? 1.0 : 0.96) * streaming;
+    // Where the second 16 rows begin beside the first and end behind them they cost what rows there are: a full round charged for one row sent 2064 x 3584 at 17 rows to the
+    // tiles.  (Fitted to 452 such calls, nine of ten within 5 %; with 10 % more the tiles that gained stay)
+    if (M > 16 && RB <= 256 && 2 * RB > 256) us = fmin(us, 1.1 * (2.9 + kb * ((double)RB / 256.0 * (0.22 - 0.0075 * m) + 0.0122 * m)));
     for (int z = 2; M <= 16 && z <= 8; ++z) {
         const int64_t per = (KB + z - 1) / z;
         if (per < 4 || (z - 1) * per >= KB || groups * z > 256) continue;
@@ -620,9 +623,9 @@ static Int8Rows int8_rows_plan(int64_t M, int64_t K, int64_t N) {
     }
     if (streaming > 12.0) {   // (no tiles take less)
         const TilePlan p = int8wo_gemm_plan(M, N, K, 8);
-        // (estimates of 33 and more rows: some 5 to 10 % low up to 16, 10 % high beyond.  Weights from 110 MB on come from memory as fast as it gives them, which all three
+        // (estimates of 33 and more rows: some 5 to 10 % low up to 16, a little high beyond.  Weights from 120 MB on come from memory as fast as it gives them, which all three
         // estimates miss by as much: with the leads that smaller ones need 8192 x 28672 at 3 rows streamed in 56.4 us, 50.0 in tiles)
-        if (p.us < (M > 16 ? 1.15 : large ? 1.0 : 0.92) * us) best = Int8Rows{Int8Rows::tiles, p.parts};
+        if (p.us < (M > 16 ? 1.05 : large ? 1.0 : 0.9) * us) best = Int8Rows{Int8Rows::tiles, p.parts};
     }
     return best;
 }
