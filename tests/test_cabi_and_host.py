@@ -63,6 +63,8 @@ def test_fp6_workspace_linear_refuses_no_columns(cabi, M, K, N):
     (3, 8192, 28672, "tile 64x128 parts=4"), (5, 11008, 17408, "tile 64x128 parts=2"), (4, 8192, 22016, "tile 64x128 parts=4"),
     # a second chunk of one row costs what one row costs: 8.4 / 10.8
     (17, 2064, 3584, "streaming"),
+    # short rows of wide weights and rows of 117 MB keep what they gained: 14.3 us streaming / 8.2 in tiles, 36 in tiles / 30.7 in parts
+    (20, 12192, 1024, "tile 64x64 parts=1"), (6, 4096, 28672, "streaming parts=4"),
     # row blocks that are no multiple of four are planned as their neighbours are: 33.1 us streaming, 21 in parts
     (8, 5120, 13824, "streaming parts=3"), (8, 5104, 13824, "streaming parts=3"), (8, 5128, 13824, "streaming parts=3"), (2, 5128, 13824, "streaming parts=3"),
     (8, 10248, 8192, "tile 64x128 parts=3"), (8, 4104, 8320, "streaming parts=3"), (4, 4104, 4096, "streaming")])
